@@ -55,6 +55,12 @@ SIGNATURES = {
     "dmf_silu_bwd": (c_int, [_P] * 3 + [_L, _I, _I, _P]),
 }
 
+# the fused combinations of include/dmf_fused.h
+FUSED_SIGNATURES = {
+    "dmf_attn_bwd_qknorm_workspace_floats": (c_int64, [_I] * 5),
+    "dmf_attn_bwd_qknorm": (c_int, [_P] * 10 + [_F] + [_P] * 7 + [_S] + [_I] * 5 + [_F, _I, _P]),
+}
+
 _lib = None
 
 
@@ -68,7 +74,7 @@ def load() -> ctypes.CDLL:
                 "(the HIP kernels are the only implementation; there is no fallback)"
             )
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in (SIGNATURES | FUSED_SIGNATURES).items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
         _lib = lib
@@ -394,6 +400,35 @@ def bwd(dout, q, k, v, o, lse, scale: float, out=None):
             _strides(dout, q, k, v, o, dq, dk, dv), B, H, Lq, Lkv, D, float(scale), _dtype_code(q), _stream(q))
     _check(rc, "dmf_attn_bwd")
     return dq, dk, dv
+
+
+def bwd_qknorm(dout, q_hat, k_hat, v, o, lse, q, k, q_gain, k_gain, eps: float, scale: float, out):
+    """Backward of attention behind per-head RMS norms of q and k: fills ``out`` = (dq, dk, dv) with the gradients of the
+    raw rows ``q``, ``k`` and of v and returns the two gain gradients (D), in the gains' dtypes -- or None when no kernel
+    implements it for this shape / dtype (nothing has been launched then)."""
+    _check_inputs(q, dout, q_hat, k_hat, v, o, k)
+    dout, q_hat, k_hat, v, o, q, k = map(_prep, (dout, q_hat, k_hat, v, o, q, k))
+    if q.dtype != torch.bfloat16:
+        return None
+    gains = [_raw(_raw(g).float().contiguous()) for g in (q_gain, k_gain)]
+    lse = _raw(_raw(lse).contiguous())
+    dq, dk, dv = map(_raw, out)
+    _check_inputs(q, dq, dk, dv)
+    B, Lq, H, D = q.shape
+    Lkv = k.shape[1]
+    delta = _empty((B, H, Lq), torch.float32, q.device)
+    ws = _empty((int(load().dmf_attn_bwd_qknorm_workspace_floats(B, H, Lq, Lkv, D)),), torch.float32, q.device)
+    dgains = [_empty((D,), torch.float32, q.device) for _ in range(2)]
+    with _on(q.device):
+        rc = load().dmf_attn_bwd_qknorm(
+            dout.data_ptr(), q_hat.data_ptr(), k_hat.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), q.data_ptr(), k.data_ptr(),
+            gains[0].data_ptr(), gains[1].data_ptr(), float(eps), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+            dgains[0].data_ptr(), dgains[1].data_ptr(), delta.data_ptr(), ws.data_ptr(),
+            _strides(dout, q_hat, k_hat, v, o, dq, dk, dv, q, k), B, H, Lq, Lkv, D, float(scale), _dtype_code(q), _stream(q))
+    if rc == ENOKERNEL:
+        return None
+    _check(rc, "dmf_attn_bwd_qknorm")
+    return dgains[0].to(q_gain.dtype), dgains[1].to(k_gain.dtype)
 
 
 # ---- fused block glue (include/dmf_block.h) -----------------------------------------------------------------------

@@ -13,6 +13,7 @@
 #include "attn_kernels.h"
 #include <algorithm>
 #include <cstdio>
+#include <type_traits>
 
 // Nothing is scheduled across a pin, and a block that holds one is not turned into selects.
 #define DMF_PIN() __builtin_amdgcn_sched_barrier(0)
@@ -111,10 +112,81 @@ __device__ __forceinline__ uint32_t lds_read32_issue(uint32_t addr) {
   return r;
 }
 
+// ------------------------------------------------------------- RMS-norm backward in the store epilogue
+// With q and k normalised per head in front of the attention (q_hat = q r gain, r = rsqrt(mean q^2 + eps)), the gradient the
+// caller wants is that of the RAW rows, gx = (g gain) r - x r^3 mean(x g gain), and of the gain, sum over rows of g x r.  Both
+// need one whole row of g = dq_hat (dk_hat), which the store epilogue already has in LDS, so it is applied there: the
+// stand-alone pass (44 us each for q and k at B16 H16 N1024 D72: reads g and x, writes gx) and the round trip of dq_hat, dk_hat
+// through HBM go away for one extra read of the raw rows.  16 lanes own a row (8 columns each), like rmsnorm_bwd_kernel, whose
+// arithmetic this repeats on the same bf16-rounded g.  Every call leaves one row of gain-gradient partial sums.
+template <int D, int NW>
+__device__ __forceinline__ void store_rows_norm_bwd(const NormSide& n, int b, int h, float eps, const __bf16* stage, char* red,
+                                                    __bf16* gdst, int64_t dst_stride, int row0, int rows, int nrows,
+                                                    float* partial, int tid) {
+  using C = Cfg<__bf16, D>;
+  constexpr int GROUPS = 4 * NW;
+  const int sub = tid & 15, grp = tid >> 4, lane = tid & 63, wave = tid >> 6;
+  const bool col_live = sub < C::VPR;
+  const __bf16* gx = static_cast<const __bf16*>(n.x) + (int64_t)b * n.st[0] + (int64_t)h * n.st[2] + 8 * sub;
+  float gain[8], acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    gain[e] = col_live ? n.gain[8 * sub + e] : 0.f;
+    acc[e] = 0.f;
+  }
+  for (int r = grp; r < rows; r += GROUPS) {
+    const bool live = col_live && row0 + r < nrows;
+    const u32x4 xv = live ? *reinterpret_cast<const u32x4*>(gx + (int64_t)(row0 + r) * n.st[1]) : u32x4{0, 0, 0, 0};
+    const u32x4 gv = live ? *reinterpret_cast<const u32x4*>(stage + r * C::OSTRIDE + 8 * sub) : u32x4{0, 0, 0, 0};
+    float x[8], g[8], ss = 0.f, sg = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[2 * e] = __uint_as_float(xv[e] << 16);
+      x[2 * e + 1] = __uint_as_float(xv[e] & 0xffff0000u);
+      g[2 * e] = __uint_as_float(gv[e] << 16);
+      g[2 * e + 1] = __uint_as_float(gv[e] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      ss = fmaf(x[e], x[e], ss);
+      sg = fmaf(x[e], g[e] * gain[e], sg);
+    }
+    const float rs = 1.f / sqrtf(group16_sum(ss) * (1.f / D) + eps);
+    const float c = rs * rs * rs * group16_sum(sg) * (1.f / D);
+    if (live) {
+      u32x4 out;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(g[e], x[e] * rs, acc[e]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[e] = pack_bf16x2(fmaf(g[2 * e] * gain[2 * e], rs, -x[2 * e] * c), fmaf(g[2 * e + 1] * gain[2 * e + 1], rs, -x[2 * e + 1] * c));
+      *reinterpret_cast<u32x4*>(gdst + (int64_t)(row0 + r) * dst_stride + 8 * sub) = out;
+    }
+  }
+  // gain gradient: the four row groups of a wave, then the waves through `red` (NW x 512 bytes that nobody else uses)
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    acc[e] += __shfl_xor(acc[e], 16);
+    acc[e] += __shfl_xor(acc[e], 32);
+  }
+  float* rf = reinterpret_cast<float*>(red);
+  if (lane < 16) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) rf[wave * 128 + 8 * sub + e] = acc[e];
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if (tid < D) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) s += rf[w * 128 + tid];
+    partial[tid] = s;
+  }
+}
+
 // ------------------------------------------------------------------ dQ kernel
 // SUB = 32-key tiles per stage (and per work-group barrier).
-template <int D, int SUB>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const BwdParams p) {
+template <int D, int SUB, bool NORM>
+__device__ __forceinline__ void bwd_dq_body(const BwdParams& p, const BwdNorm& nrm) {
   using F = BwdFastCfg<D, true>;
   using T = __bf16;
   constexpr int VPR = F::VPR, NCHUNK = F::NCHUNK, NMT = F::NMT, P = F::P, STR = F::STR;
@@ -286,17 +358,36 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const BwdParam
     });
    }
   }
-  store_rows_transposed<T, D, 4, NMT>(reinterpret_cast<T*>(smem), reinterpret_cast<T*>(p.dq) + base(5), p.st[5][1], q0, p.Lq, tid,
-                                      [&](int t, int i) { return dQ[t][i] * p.scale; },
-                                      [&](void* ws) {
-                                        if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dQ16[hq][e] * p.scale; });
-                                      });
+  T* stage = reinterpret_cast<T*>(smem);
+  auto value = [&](int t, int i) { return dQ[t][i] * p.scale; };
+  auto tail_value = [&](void* ws) {
+    if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dQ16[hq][e] * p.scale; });
+  };
+  T* gdq = reinterpret_cast<T*>(p.dq) + base(5);
+  if constexpr (NORM) {
+    lds_barrier();
+    stage_rows<T, D, NMT>(stage, tid, value, tail_value);
+    lds_barrier();
+    store_rows_norm_bwd<D, 4>(nrm.q, b, h, nrm.eps, stage, smem + 128 * Cfg<T, D>::OROWV * 16, gdq, p.st[5][1], q0, 128, p.Lq,
+                              nrm.q.partial + (int64_t)wg * D, tid);
+  } else {
+    store_rows_transposed<T, D, 4, NMT>(stage, gdq, p.st[5][1], q0, p.Lq, tid, value, tail_value);
+  }
+}
+
+template <int D, int SUB>
+__global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const BwdParams p) {
+  bwd_dq_body<D, SUB, false>(p, BwdNorm{});
+}
+template <int D, int SUB>
+__global__ __launch_bounds__(256, 2) void attn_bwd_dq_norm_bf16_kernel(const BwdNormParams p) {
+  bwd_dq_body<D, SUB, true>(p.b, p.n);
 }
 
 // --------------------------------------------------------------- dK/dV kernel
 // NW waves of 32 keys each per work-group.
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_bwd_dkv_bf16_kernel(const BwdParams p) {
+template <int D, int NW, bool NORM>
+__device__ __forceinline__ void bwd_dkv_body(const BwdParams& p, const BwdNorm& nrm) {
   using F = BwdFastCfg<D, true>;
   using T = __bf16;
   constexpr int VPR = F::VPR, NCHUNK = F::NCHUNK, NMT = F::NMT, P = F::P, STR = F::STR;
@@ -527,16 +618,34 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_bwd_dkv_bf16_kernel(cons
     }
   }
   T* stage = reinterpret_cast<T*>(smem);
-  store_rows_transposed<T, D, NW, NMT>(stage, reinterpret_cast<T*>(p.dk) + base(6), p.st[6][1], k0, p.Lkv, tid,
-                                      [&](int t, int i) { return dK[t][i] * p.scale; },
-                                      [&](void* ws) {
-                                        if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dK16[hq][e] * p.scale; });
-                                      });
+  auto k_value = [&](int t, int i) { return dK[t][i] * p.scale; };
+  auto k_tail = [&](void* ws) {
+    if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dK16[hq][e] * p.scale; });
+  };
+  T* gdk = reinterpret_cast<T*>(p.dk) + base(6);
+  if constexpr (NORM) {
+    lds_barrier();
+    stage_rows<T, D, NMT>(stage, tid, k_value, k_tail);
+    lds_barrier();
+    store_rows_norm_bwd<D, NW>(nrm.k, b, h, nrm.eps, stage, smem + 32 * NW * Cfg<T, D>::OROWV * 16, gdk, p.st[6][1], k0, 32 * NW,
+                               p.Lkv, nrm.k.partial + (int64_t)wg * D, tid);
+  } else {
+    store_rows_transposed<T, D, NW, NMT>(stage, gdk, p.st[6][1], k0, p.Lkv, tid, k_value, k_tail);
+  }
   store_rows_transposed<T, D, NW, NMT>(stage, reinterpret_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid,
                                       [&](int t, int i) { return dV[t][i]; },
                                       [&](void* ws) {
                                         if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dV16[hq][e]; });
                                       });
+}
+
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_bwd_dkv_bf16_kernel(const BwdParams p) {
+  bwd_dkv_body<D, NW, false>(p, BwdNorm{});
+}
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_bwd_dkv_norm_bf16_kernel(const BwdNormParams p) {
+  bwd_dkv_body<D, NW, true>(p.b, p.n);
 }
 
 // ------------------------------------------------ single-pass backward, whole (batch, head) unit per work-group
@@ -571,8 +680,8 @@ struct BwdFusedCfg {
   static_assert(256 * Cfg<__bf16, D>::OROWV * 16 <= XBYTES, "store staging must fit the exchange area");
 };
 
-template <int D>
-__global__ __launch_bounds__(512, 1) void attn_bwd_fused_bf16_kernel(const BwdParams p) {
+template <int D, bool NORM>
+__device__ __forceinline__ void bwd_fused_body(const BwdParams& p, const BwdNorm& nrm) {
   using F = BwdFastCfg<D, true>;
   using FC = BwdFusedCfg<D>;
   using T = __bf16;
@@ -1097,23 +1206,41 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_fused_bf16_kernel(const BwdPa
       }
       bare_barrier();   // (no fence: tiles of the next half are in flight)
       T* gdq = reinterpret_cast<T*>(p.dq) + base(5);
-      for (int v = tid; v < 128 * VPR; v += 512) {
-        const int row = v / VPR, cv = v % VPR, qrow = half * 128 + row;
-        if (qrow < p.Lq)
-          *reinterpret_cast<u32x4*>(gdq + (int64_t)qrow * p.st[5][1] + cv * C::VEC) =
-              *reinterpret_cast<const u32x4*>(stage + row * C::OSTRIDE + cv * C::VEC);
+      if constexpr (NORM) {
+        // (one row of gain partial sums per 128 queries; the reduction area sits behind the 128 staged rows)
+        store_rows_norm_bwd<D, 8>(nrm.q, b, h, nrm.eps, stage, smem + FC::X_OFF + 128 * C::OROWV * 16, gdq, p.st[5][1], half * 128, 128,
+                                  p.Lq, nrm.q.partial + ((int64_t)bh * ((p.Lq + 127) / 128) + half) * D, tid);
+      } else {
+        for (int v = tid; v < 128 * VPR; v += 512) {
+          const int row = v / VPR, cv = v % VPR, qrow = half * 128 + row;
+          if (qrow < p.Lq)
+            *reinterpret_cast<u32x4*>(gdq + (int64_t)qrow * p.st[5][1] + cv * C::VEC) =
+                *reinterpret_cast<const u32x4*>(stage + row * C::OSTRIDE + cv * C::VEC);
+        }
+        // The first tile of the next half has no barrier of its own and writes X: every wave's staging reads come first.
+        // (The norm epilogue ends in a barrier.)
+        if (4 * (half + 1) < nqt) bare_barrier();
       }
-      // (the next half's first barrier orders these staging reads before X is written again)
     }
   }
 
   // ---- dK, dV of this wave's 32 keys
   T* stage = reinterpret_cast<T*>(smem + FC::X_OFF);
-  store_rows_transposed<T, D, 8, NMT>(stage, reinterpret_cast<T*>(p.dk) + base(6), p.st[6][1], 0, p.Lkv, tid,
-                                      [&](int t, int i) { return dK[t][i] * p.scale; },
-                                      [&](void* ws) {
-                                        if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dK16[hq][e] * p.scale; });
-                                      });
+  auto k_value = [&](int t, int i) { return dK[t][i] * p.scale; };
+  auto k_tail = [&](void* ws) {
+    if constexpr (TAIL) store_tail16<T, D, NMT>(ws, lane, [&](int hq, int e) { return dK16[hq][e] * p.scale; });
+  };
+  T* gdk = reinterpret_cast<T*>(p.dk) + base(6);
+  if constexpr (NORM) {
+    lds_barrier();
+    stage_rows<T, D, NMT>(stage, tid, k_value, k_tail);
+    lds_barrier();
+    // (reduction area: the K tiles, which nobody reads any more)
+    store_rows_norm_bwd<D, 8>(nrm.k, b, h, nrm.eps, stage, smem + FC::K_OFF, gdk, p.st[6][1], 0, 256, p.Lkv,
+                              nrm.k.partial + (int64_t)bh * D, tid);
+  } else {
+    store_rows_transposed<T, D, 8, NMT>(stage, gdk, p.st[6][1], 0, p.Lkv, tid, k_value, k_tail);
+  }
   store_rows_transposed<T, D, 8, NMT>(stage, reinterpret_cast<T*>(p.dv) + base(7), p.st[7][1], 0, p.Lkv, tid,
                                       [&](int t, int i) { return dV[t][i]; },
                                       [&](void* ws) {
@@ -1122,29 +1249,58 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_fused_bf16_kernel(const BwdPa
 }
 
 template <int D>
-static int launch_bwd_fused_t(const BwdParams& p, int BH, hipStream_t stream) {
-  auto kern = attn_bwd_fused_bf16_kernel<D>;
-  static bool lds_ok[64] = {};
-  if (!ensure_dynamic_lds(kern, BwdFusedCfg<D>::LDS_BYTES, lds_ok)) return -7;
-  return launch_kernel(kern, dim3((uint32_t)BH), dim3(512), BwdFusedCfg<D>::LDS_BYTES, stream, p);
+__global__ __launch_bounds__(512, 1) void attn_bwd_fused_bf16_kernel(const BwdParams p) {
+  bwd_fused_body<D, false>(p, BwdNorm{});
+}
+template <int D>
+__global__ __launch_bounds__(512, 1) void attn_bwd_fused_norm_bf16_kernel(const BwdNormParams p) {
+  bwd_fused_body<D, true>(p.b, p.n);
 }
 
-template <int D>
-static int launch_bwd_fast_t(const BwdParams& p, int BH, hipStream_t stream) {
+// Norm variants: the same kernels with store_rows_norm_bwd behind them.
+struct NoNorm {};
+
+template <int D, typename N>
+static int launch_bwd_fused_t(const BwdParams& p, const N& norm, int BH, hipStream_t stream) {
+  static bool lds_ok[64] = {};
+  const dim3 grid((uint32_t)BH), block(512);
+  if constexpr (std::is_same<N, BwdNorm>::value) {
+    auto kern = attn_bwd_fused_norm_bf16_kernel<D>;
+    if (!ensure_dynamic_lds(kern, BwdFusedCfg<D>::LDS_BYTES, lds_ok)) return -7;
+    return launch_kernel(kern, grid, block, BwdFusedCfg<D>::LDS_BYTES, stream, BwdNormParams{p, norm});
+  } else {
+    auto kern = attn_bwd_fused_bf16_kernel<D>;
+    if (!ensure_dynamic_lds(kern, BwdFusedCfg<D>::LDS_BYTES, lds_ok)) return -7;
+    return launch_kernel(kern, grid, block, BwdFusedCfg<D>::LDS_BYTES, stream, p);
+  }
+}
+
+template <int D, typename N>
+static int launch_bwd_fast_t(const BwdParams& p, const N& norm, int BH, hipStream_t stream) {
   using F = BwdFastCfg<D, true>;
+  constexpr bool NORM = std::is_same<N, BwdNorm>::value;
   constexpr int tiles = 2 * (2 * F::TBYTES + F::STAT) + 512;
-  constexpr int stage = 128 * Cfg<__bf16, D>::OROWV * 16;
-  constexpr int stage2 = 32 * kKvWaves * Cfg<__bf16, D>::OROWV * 16;
+  constexpr int stage = 128 * Cfg<__bf16, D>::OROWV * 16 + (NORM ? 4 * 512 : 0);
+  constexpr int stage2 = 32 * kKvWaves * Cfg<__bf16, D>::OROWV * 16 + (NORM ? kKvWaves * 512 : 0);
   constexpr int smem = tiles > stage2 ? tiles : stage2;
   constexpr int tiles1 = 2 * kDqSub * 2 * F::TBYTES + 512;
   constexpr int smem1 = tiles1 > stage ? tiles1 : stage;
-  auto k1 = attn_bwd_dq_bf16_kernel<D, kDqSub>;
-  auto k2 = attn_bwd_dkv_bf16_kernel<D, kKvWaves>;
+  const dim3 grid1((p.Lq + 127) / 128 * (uint32_t)BH), grid2((p.Lkv + 32 * kKvWaves - 1) / (32 * kKvWaves) * (uint32_t)BH);
   static bool lds_ok1[64] = {}, lds_ok2[64] = {};
-  if (!ensure_dynamic_lds(k1, smem1, lds_ok1) || !ensure_dynamic_lds(k2, smem, lds_ok2)) return -7;
-  const uint32_t nqb = (p.Lq + 127) / 128, nkb = (p.Lkv + 32 * kKvWaves - 1) / (32 * kKvWaves);
-  if (int rc = launch_kernel(k1, dim3(nqb * (uint32_t)BH), dim3(256), smem1, stream, p)) return rc;
-  return launch_kernel(k2, dim3(nkb * (uint32_t)BH), dim3(64 * kKvWaves), smem, stream, p);
+  if constexpr (NORM) {
+    auto k1 = attn_bwd_dq_norm_bf16_kernel<D, kDqSub>;
+    auto k2 = attn_bwd_dkv_norm_bf16_kernel<D, kKvWaves>;
+    if (!ensure_dynamic_lds(k1, smem1, lds_ok1) || !ensure_dynamic_lds(k2, smem, lds_ok2)) return -7;
+    const BwdNormParams np{p, norm};
+    if (int rc = launch_kernel(k1, grid1, dim3(256), smem1, stream, np)) return rc;
+    return launch_kernel(k2, grid2, dim3(64 * kKvWaves), smem, stream, np);
+  } else {
+    auto k1 = attn_bwd_dq_bf16_kernel<D, kDqSub>;
+    auto k2 = attn_bwd_dkv_bf16_kernel<D, kKvWaves>;
+    if (!ensure_dynamic_lds(k1, smem1, lds_ok1) || !ensure_dynamic_lds(k2, smem, lds_ok2)) return -7;
+    if (int rc = launch_kernel(k1, grid1, dim3(256), smem1, stream, p)) return rc;
+    return launch_kernel(k2, grid2, dim3(64 * kKvWaves), smem, stream, p);
+  }
 }
 
 // Policy: does the single-pass kernel take this case?  Whole (batch, head) units per work-group, every score tile formed
@@ -1166,28 +1322,40 @@ bool plan_bwd_bf16_fast(int Lq, int Lkv, int D, int BH, char* buf, size_t n) {
   return true;
 }
 
-// Returns 1 if there is no tuned kernel for the case (caller uses the generic ones).
-int launch_bwd_bf16_fast(const BwdParams& p, int BH, int D, hipStream_t stream) {
+template <typename N>
+static int launch_bwd_any(const BwdParams& p, const N& norm, int BH, int D, hipStream_t stream) {
   // 32-bit buffer addressing: every (batch, head) slab of rows must span < 2 GiB
   const int64_t max_row = std::max(std::max(std::max(p.st[0][1], p.st[1][1]), std::max(p.st[2][1], p.st[3][1])), p.st[4][1]);
   if (max_row * 2 * (int64_t)(std::max(p.Lq, p.Lkv) + 256) >= (int64_t)1 << 31) return 1;
   if (bwd_single_pass(p.Lq, p.Lkv, D, BH)) {
     switch (D) {
-      case 64: return launch_bwd_fused_t<64>(p, BH, stream);
-      case 72: return launch_bwd_fused_t<72>(p, BH, stream);
-      case 80: return launch_bwd_fused_t<80>(p, BH, stream);
-      case 96: return launch_bwd_fused_t<96>(p, BH, stream);
+      case 64: return launch_bwd_fused_t<64>(p, norm, BH, stream);
+      case 72: return launch_bwd_fused_t<72>(p, norm, BH, stream);
+      case 80: return launch_bwd_fused_t<80>(p, norm, BH, stream);
+      case 96: return launch_bwd_fused_t<96>(p, norm, BH, stream);
       default: break;
     }
   }
   switch (D) {
-    case 64: return launch_bwd_fast_t<64>(p, BH, stream);
-    case 72: return launch_bwd_fast_t<72>(p, BH, stream);
-    case 80: return launch_bwd_fast_t<80>(p, BH, stream);
-    case 96: return launch_bwd_fast_t<96>(p, BH, stream);
-    case 128: return launch_bwd_fast_t<128>(p, BH, stream);
+    case 64: return launch_bwd_fast_t<64>(p, norm, BH, stream);
+    case 72: return launch_bwd_fast_t<72>(p, norm, BH, stream);
+    case 80: return launch_bwd_fast_t<80>(p, norm, BH, stream);
+    case 96: return launch_bwd_fast_t<96>(p, norm, BH, stream);
+    case 128: return launch_bwd_fast_t<128>(p, norm, BH, stream);
     default: return 1;
   }
+}
+
+// Both return 1 if there is no tuned kernel for the case (caller uses the generic ones).
+int launch_bwd_bf16_fast(const BwdParams& p, int BH, int D, hipStream_t stream) { return launch_bwd_any(p, NoNorm{}, BH, D, stream); }
+int launch_bwd_norm_bf16_fast(const BwdParams& p, const BwdNorm& norm, int BH, int D, hipStream_t stream) {
+  return launch_bwd_any(p, norm, BH, D, stream);
+}
+
+// Rows of gain-gradient partial sums that launch_bwd_norm_bf16_fast leaves for q and for k.
+void bwd_norm_partials(int Lq, int Lkv, int D, int BH, int64_t& nq, int64_t& nk) {
+  nq = (int64_t)BH * ((Lq + 127) / 128);
+  nk = bwd_single_pass(Lq, Lkv, D, BH) ? (int64_t)BH : (int64_t)BH * ((Lkv + 32 * kKvWaves - 1) / (32 * kKvWaves));
 }
 
 }  // namespace dmf

@@ -39,6 +39,23 @@ struct BwdParams {
   float scale, scale_log2;
 };
 
+// Per-head RMS norm of q and of k in front of the attention whose gradient is wanted: dq, dk are then the gradients of the raw
+// rows x, and `partial` receives rows of partial sums (D floats each, bwd_norm_partials of them) of the gain gradient.
+struct NormSide {
+  const void* x;            // raw rows (B, L, H, D), strides st = {stride_B, stride_L, stride_H} in elements
+  const float* gain;        // (D)
+  float* partial;
+  int64_t st[3];
+};
+struct BwdNorm {
+  NormSide q, k;
+  float eps;
+};
+struct BwdNormParams {
+  BwdParams b;
+  BwdNorm n;
+};
+
 // Opt a kernel in to `bytes` of dynamic LDS on the current device.  The attribute is per device, so the
 // "already done" flag is kept per (kernel instantiation, device); a race between two host threads at worst
 // repeats the idempotent call.
@@ -88,6 +105,10 @@ int launch_fwd_bf16_fast(const FwdParams& p, int BH, int D, bool jvp, hipStream_
 int launch_bwd_generic(const BwdParams& p, int BH, int D, bool bf16, hipStream_t stream);
 int launch_bwd_bf16_fast(const BwdParams& p, int BH, int D, hipStream_t stream);
 int launch_bwd(const BwdParams& p, int BH, int D, bool bf16, hipStream_t stream);
+int launch_bwd_norm_bf16_fast(const BwdParams& p, const BwdNorm& norm, int BH, int D, hipStream_t stream);
+void bwd_norm_partials(int Lq, int Lkv, int D, int BH, int64_t& nq, int64_t& nk);
+// out_q[d] = sum over nq rows of part_q, the same for k (fp32, fixed order; block_ops.hip)
+int launch_gain_reduce(const float* part_q, int64_t nq, float* out_q, const float* part_k, int64_t nk, float* out_k, int D, hipStream_t stream);
 
 // Host-only: the tuned kernel(s) the two *_bf16_fast launchers pick for a case, written to buf as profilers spell them
 // ("dmf::attn_fwd_bf16_kernel<72, true, 8, false, false>", the backward pair joined by " + "), for rows less than

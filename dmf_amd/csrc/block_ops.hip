@@ -293,47 +293,55 @@ __global__ __launch_bounds__(kThreads) void ln_modulate_bwd_kernel(LnBwdParams p
   reduce_waves_to_partial<NV, 2>(acc, lds, p.partial + static_cast<int64_t>(blockIdx.x) * 2 * p.C, p.C, lane, wave);
 }
 
-// out[k][b][c] = sum_chunk partial[b][chunk][k][c]; out[k] dense (B, C) of the given element type.
+// out[k][b][c] = sum over chunks of part[k][(b * nchunk[k] + chunk) * stride + c]; out[k] dense (B, C) of the given element type.
 struct ReduceParams {
-  const float* partial;
+  const float* part[2];
   void* out[2];
-  int64_t total;  // B * K * C / 8 vectors
-  int nchunk, K, C;
+  int64_t total;  // B * C / 8 vectors per k
+  int64_t stride;
+  int nchunk[2], C;
   int obf;
 };
 
-// Work-group: 64 output vectors (8 columns each); wave w adds chunks w, w+4, ...; the four waves meet in LDS.
-__global__ __launch_bounds__(kThreads) void reduce_partials_kernel(ReduceParams p) {
-  __shared__ float lds[kWaves - 1][64 * 8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t v = static_cast<int64_t>(blockIdx.x) * 64 + lane;
+// Work-group (x, k): NVEC output vectors (8 columns each) of output k; the NT / NVEC thread groups add every (NT / NVEC)-th
+// chunk, four loads in flight, and meet in LDS.  Which shape: see reduce_partials().
+template <int NT, int NVEC>
+__global__ __launch_bounds__(NT) void reduce_partials_kernel(ReduceParams p) {
+  constexpr int G = NT / NVEC;
+  __shared__ float lds[G][NVEC * 8];
+  const int k = blockIdx.y, lv = threadIdx.x % NVEC, grp = threadIdx.x / NVEC;
+  const int64_t v = static_cast<int64_t>(blockIdx.x) * NVEC + lv;
   const bool live = v < p.total;
   const int vec_per_row = p.C / 8;
   const int col = static_cast<int>(v % vec_per_row) * 8;
-  const int64_t bk = v / vec_per_row;
-  const int k = static_cast<int>(bk % p.K);
-  const int64_t b = bk / p.K;
+  const int64_t b = v / vec_per_row;
+  const int n = p.nchunk[k];
   float s[8];
   zero8(s);
   if (live) {
+    const float* src = p.part[k] + b * n * p.stride + col;
 #pragma unroll 4
-    for (int c = wave; c < p.nchunk; c += kWaves) {
+    for (int c = grp; c < n; c += G) {
       float t[8];
-      load8(p.partial, 0, ((b * p.nchunk + c) * p.K + k) * p.C + col, t);
+      load8(src, 0, c * p.stride, t);
 #pragma unroll
       for (int e = 0; e < 8; ++e) s[e] += t[e];
     }
   }
-  if (wave > 0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) lds[wave - 1][lane * 8 + e] = s[e];
-  }
+  for (int e = 0; e < 8; ++e) lds[grp][lv * 8 + e] = s[e];
   __syncthreads();
-  if (wave == 0 && live) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      for (int w = 0; w < kWaves - 1; ++w) s[e] += lds[w][lane * 8 + e];
-    store8(p.out[k], p.obf, b * p.C + col, s);
+  constexpr int NE = NVEC * 8;                    // columns of this work-group
+  if (threadIdx.x < NE) {
+    const int64_t ve = static_cast<int64_t>(blockIdx.x) * NVEC + threadIdx.x / 8;
+    float a = 0.f;
+#pragma unroll 8
+    for (int w = 0; w < G; ++w) a += lds[w][threadIdx.x];
+    if (ve < p.total) {
+      const int64_t idx = (ve / vec_per_row) * p.C + (ve % vec_per_row) * 8 + threadIdx.x % 8;
+      if (p.obf) static_cast<uint16_t*>(p.out[k])[idx] = static_cast<uint16_t>(pack_bf16x2(a, 0.f));
+      else static_cast<float*>(p.out[k])[idx] = a;
+    }
   }
 }
 
@@ -721,19 +729,28 @@ inline int dispatch_nv(int C, F&& f) {
   }
 }
 
+// The reduction is a chain of dependent loads per thread with next to no work, so the shape that shortens the chain wins as
+// long as a row is read in whole 128-byte lines: 8 vectors (256 bytes) per work-group of 256 threads = 32 chunk groups, and
+// 1024 threads = 128 groups from 256 chunks on (the gain gradients: 1024 partial rows of 72 columns, one work-group).
+inline int launch_reduce(ReduceParams& r, int K, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>((r.total + 7) / 8), K);
+  if (std::max(r.nchunk[0], r.nchunk[1]) >= 256) return launch_kernel(reduce_partials_kernel<1024, 8>, grid, dim3(1024), 0, s, r);
+  return launch_kernel(reduce_partials_kernel<256, 8>, grid, dim3(256), 0, s, r);
+}
+
 inline int reduce_partials(const float* partial, void* out0, void* out1, int B, int nchunk, int K, int C, int obf,
                            hipStream_t s) {
   ReduceParams r{};
-  r.partial = partial;
+  r.part[0] = partial;
+  r.part[1] = partial + C;
   r.out[0] = out0;
   r.out[1] = out1;
-  r.total = static_cast<int64_t>(B) * K * (C / 8);
-  r.nchunk = nchunk;
-  r.K = K;
+  r.total = static_cast<int64_t>(B) * (C / 8);
+  r.stride = static_cast<int64_t>(K) * C;
+  r.nchunk[0] = r.nchunk[1] = nchunk;
   r.C = C;
   r.obf = obf;
-  const unsigned grid = static_cast<unsigned>((r.total + 63) / 64);
-  return launch_kernel(reduce_partials_kernel, dim3(grid), dim3(kThreads), 0, s, r);
+  return launch_reduce(r, K, s);
 }
 
 template <int ACT>
@@ -754,6 +771,18 @@ inline int act_impl(const void* x, const void* t, void* y, void* ty, int64_t n, 
 }
 
 }  // namespace blk
+
+int launch_gain_reduce(const float* part_q, int64_t nq, float* out_q, const float* part_k, int64_t nk, float* out_k, int D, hipStream_t stream) {
+  blk::ReduceParams r{};
+  r.part[0] = part_q; r.part[1] = part_k;
+  r.out[0] = out_q; r.out[1] = out_k;
+  r.total = D / 8;
+  r.stride = D;
+  r.nchunk[0] = static_cast<int>(nq); r.nchunk[1] = static_cast<int>(nk);
+  r.C = D;
+  return blk::launch_reduce(r, 2, stream);
+}
+
 }  // namespace dmf
 
 using namespace dmf::blk;

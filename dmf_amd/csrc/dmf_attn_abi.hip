@@ -2,6 +2,7 @@
 // validation and marshalling into the kernel parameter blocks.  Nothing here
 // allocates, frees or synchronises.
 #include "../../include/dmf_attn.h"
+#include "../../include/dmf_fused.h"
 #include "attn_kernels.h"
 #include <algorithm>
 #include <cstdio>
@@ -160,6 +161,43 @@ int dmf_attn_bwd(const void* dout, const void* q, const void* k, const void* v, 
   p.H = H; p.Lq = Lq; p.Lkv = Lkv;
   p.scale = scale; p.scale_log2 = scale * 1.4426950408889634f;
   return dmf::launch_bwd(p, B * H, D, dtype == DMF_ATTN_BF16, static_cast<hipStream_t>(stream));
+}
+
+int64_t dmf_attn_bwd_qknorm_workspace_floats(int B, int H, int Lq, int Lkv, int D) {
+  if (B < 1 || H < 1 || Lq < 1 || Lkv < 1 || !head_dim_ok(D)) return 0;
+  int64_t nq, nk;
+  dmf::bwd_norm_partials(Lq, Lkv, D, B * H, nq, nk);
+  return (nq + nk) * D;
+}
+
+int dmf_attn_bwd_qknorm(const void* dout, const void* q_hat, const void* k_hat, const void* v, const void* o, const float* lse,
+                        const void* q, const void* k, const float* q_gain, const float* k_gain, float eps,
+                        void* dq, void* dk, void* dv, float* dq_gain, float* dk_gain, float* delta, float* workspace,
+                        const int64_t* strides, int B, int H, int Lq, int Lkv, int D, float scale, int dtype, void* stream) {
+  if (int rc = check_common(B, H, Lq, Lkv, D, dtype)) return rc;
+  if (dtype != DMF_ATTN_BF16) return DMF_ATTN_ENOKERNEL;
+  if (strides == nullptr || lse == nullptr || delta == nullptr || q_gain == nullptr || k_gain == nullptr || dq_gain == nullptr ||
+      dk_gain == nullptr || workspace == nullptr)
+    return DMF_ATTN_ENULL;
+  dmf::BwdParams p{};
+  dmf::BwdNorm n{};
+  const void* ptrs[10] = {dout, q_hat, k_hat, v, o, dq, dk, dv, q, k};
+  for (int i = 0; i < 10; ++i)
+    if (int rc = check_tensor(ptrs[i], strides + 4 * i, 2, i < 8 ? p.st[i] : (i == 8 ? n.q.st : n.k.st))) return rc;
+  p.dout = dout; p.q = q_hat; p.k = k_hat; p.v = v; p.o = o; p.lse = lse;
+  p.dq = dq; p.dk = dk; p.dv = dv; p.delta = delta;
+  p.H = H; p.Lq = Lq; p.Lkv = Lkv;
+  p.scale = scale; p.scale_log2 = scale * 1.4426950408889634f;
+  int64_t nq, nk;
+  dmf::bwd_norm_partials(Lq, Lkv, D, B * H, nq, nk);
+  n.q.x = q; n.k.x = k;
+  n.q.gain = q_gain; n.k.gain = k_gain;
+  n.q.partial = workspace; n.k.partial = workspace + nq * D;
+  n.eps = eps;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = dmf::launch_bwd_norm_bf16_fast(p, n, B * H, D, s);
+  if (rc) return rc == 1 ? DMF_ATTN_ENOKERNEL : rc;
+  return dmf::launch_gain_reduce(n.q.partial, nq, dq_gain, n.k.partial, nk, dk_gain, D, s);
 }
 
 }  // extern "C"

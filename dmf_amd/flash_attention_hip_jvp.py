@@ -250,7 +250,8 @@ def flash_attn_qkvpacked_func(qkv, softmax_scale=None):
     return out if tg is None else fwAD.make_dual(out, t_out)
 
 
-# Normalise q / q and k inside the attention kernel where a kernel offers it (module switches for A/B timing and tests).
+# Normalise q / q and k inside the attention kernel where a kernel offers it, and run the norms' backward in the store epilogue of
+# the attention backward (module switches for A/B timing and tests).
 IN_KERNEL_Q_NORM = True
 IN_KERNEL_K_NORM = True
 # A work-group of the tuned kernels covers 256 query rows and normalises the key tiles it consumes, so beyond that
@@ -320,6 +321,10 @@ class QKNormAttnQKVPackedFunc(torch.autograd.Function):
             kn, _ = _lib.rmsnorm_fwd(k, k_gain, None, ctx.eps, False)
         gqkv = torch.empty(qkv.shape, dtype=qkv.dtype, device=qkv.device)
         gq, gk, gv = gqkv.unbind(2)
+        if IN_KERNEL_Q_NORM:   # the norms' backward rides in the kernels' store epilogue
+            fused = _lib.bwd_qknorm(dout, qn, kn, v, o, lse, q, k, q_gain, k_gain, ctx.eps, ctx.softmax_scale, (gq, gk, gv))
+            if fused is not None:
+                return gqkv, None, *fused, None, None
         dqn = torch.empty(qn.shape, dtype=qn.dtype, device=qn.device)
         dkn = torch.empty(kn.shape, dtype=kn.dtype, device=kn.device)
         _lib.bwd(dout, qn, kn, v, o, lse, ctx.softmax_scale, out=(dqn, dkn, gv))

@@ -1,0 +1,34 @@
+/*
+ * Fused entry points beyond the operator boundary of dmf_attn.h / dmf_block.h: combinations of those operators that run as
+ * fewer passes.  Same conventions as there (plain pointers, element strides, return codes, a hipStream_t as void*; nothing
+ * allocates, frees or synchronises); each is optional for a caller, who can always compose the basic entry points.
+ */
+#ifndef DMF_FUSED_H
+#define DMF_FUSED_H
+
+#include "dmf_attn.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/*
+ * dmf_attn_bwd behind per-head RMS norms of q and k (dmf_attn_fwd_qknorm): q_hat, k_hat are the normalised rows the forward
+ * handed out, q, k the raw ones; dq, dk are the gradients of the RAW rows and dq_gain, dk_gain (D) fp32 those of the gains --
+ * dmf_attn_bwd followed by dmf_rmsnorm_bwd for q and for k, with the norm's backward applied where the rows of dq_hat,
+ * dk_hat are stored.  strides: 10 tensors {dout, q_hat, k_hat, v, o, dq, dk, dv, q, k}.  workspace:
+ * dmf_attn_bwd_qknorm_workspace_floats() floats.  Deterministic (no atomics).  bf16 shapes the tuned kernels cover;
+ * DMF_ATTN_ENOKERNEL otherwise (nothing launched).
+ */
+DMF_ATTN_API int64_t dmf_attn_bwd_qknorm_workspace_floats(int B, int H, int Lq, int Lkv, int D);
+DMF_ATTN_API int dmf_attn_bwd_qknorm(const void* dout, const void* q_hat, const void* k_hat, const void* v,
+                        const void* o, const float* lse, const void* q, const void* k,
+                        const float* q_gain, const float* k_gain, float eps,
+                        void* dq, void* dk, void* dv, float* dq_gain, float* dk_gain,
+                        float* delta, float* workspace, const int64_t* strides,
+                        int B, int H, int Lq, int Lkv, int D, float scale, int dtype, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* DMF_FUSED_H */

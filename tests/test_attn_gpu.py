@@ -753,3 +753,29 @@ def test_registered_operators_pass_opcheck():
     assert set(res.values()) == {"SUCCESS"}, res
     o2, lse2 = _lib.fwd(q.detach(), k.detach(), v.detach(), 0.125)
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
+
+
+@pytest.mark.parametrize("L,D", [(1, 64), (33, 72), (128, 80), (129, 72), (160, 64), (256, 72), (256, 96), (257, 72), (300, 128), (512, 64)])
+def test_bwd_qknorm_matches_backward_followed_by_the_stand_alone_norm_backward(L, D):
+    """The norm backward in the store epilogue repeats the stand-alone kernel's arithmetic on the same bf16-rounded
+    gradient rows: raw-row gradients agree to one bf16 rounding (2^-9 each side), gain gradients to the order of an fp32 sum."""
+    B, H, scale, eps = 2, 3, D ** -0.5, 1e-6
+    g = torch.Generator().manual_seed(L * 131 + D)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    qkv, dout = rnd(B, L, 3, H, D), rnd(B, L, H, D)
+    gq, gk = (1 + 0.1 * torch.randn(D, generator=g)).to(DEV), (1 + 0.1 * torch.randn(D, generator=g)).to(DEV)
+    q, k, v = qkv.unbind(2)
+    qn, kn = _lib.rmsnorm_fwd(q, gq, None, eps)[0], _lib.rmsnorm_fwd(k, gk, None, eps)[0]
+    o, lse = _lib.fwd(qn, kn, v, scale)
+    out, ref = torch.empty_like(qkv), torch.empty_like(qkv)
+    gains = _lib.bwd_qknorm(dout, qn, kn, v, o, lse, q, k, gq, gk, eps, scale, out.unbind(2))
+    assert gains is not None
+    dqn, dkn, _ = _lib.bwd(dout, qn, kn, v, o, lse, scale, out=(torch.empty_like(qn), torch.empty_like(kn), ref[:, :, 2]))
+    _, rq = _lib.rmsnorm_bwd(dqn, q, gq, eps, out=ref[:, :, 0])
+    _, rk = _lib.rmsnorm_bwd(dkn, k, gk, eps, out=ref[:, :, 1])
+    assert torch.equal(out[:, :, 2], ref[:, :, 2])
+    for i in (0, 1):   # (L == 1: a single key, so dq and dk are exactly zero)
+        d = (out[:, :, i].float() - ref[:, :, i].float()).norm()
+        assert float(d) <= 2 ** -8 * float(ref[:, :, i].float().norm()), (i, float(d))
+    for a, r in zip(gains, (rq, rk)):
+        assert float((a - r).norm()) <= 1e-5 * float(r.norm()) + 1e-12
