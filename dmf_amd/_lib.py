@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p, POINTER
@@ -24,7 +25,7 @@ except ImportError:
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdmf_attn.so")
 
-DMF_ATTN_F32, DMF_ATTN_BF16 = 0, 1
+DMF_ATTN_F32, DMF_ATTN_BF16, DMF_ATTN_F16 = 0, 1, 2
 SUPPORTED_HEAD_DIMS = (32, 64, 72, 80, 96, 128)
 
 # name -> (restype, argtypes): the complete exported surface of include/dmf_attn.h and include/dmf_block.h
@@ -252,9 +253,10 @@ def _check_inputs(ref: torch.Tensor, *others: torch.Tensor) -> None:
             raise ValueError("all attention operands must share device and dtype")
 
 
-def fwd_jvp(q, k, v, tq, tk, tv, scale: float, need_dlse: bool = False):
+def fwd_jvp(q, k, v, tq, tk, tv, scale: float, need_dlse: bool = False, dtype_code=None):
     """Fused forward + JVP.  Returns (o, to, lse) -- or (o, to, lse, dlse) with
-    ``need_dlse`` -- o/to contiguous (B, Lq, H, D), lse/dlse (B, H, Lq) fp32."""
+    ``need_dlse`` -- o/to contiguous (B, Lq, H, D), lse/dlse (B, H, Lq) fp32.
+    ``dtype_code``: the operands' type where it is not one the whole package takes (see ``fwd_jvp_half``)."""
     _check_inputs(q, k, v, tq, tk, tv)
     q, k, v, tq, tk, tv = map(_prep, (q, k, v, tq, tk, tv))
     B, Lq, H, D = q.shape
@@ -268,12 +270,12 @@ def fwd_jvp(q, k, v, tq, tk, tv, scale: float, need_dlse: bool = False):
             q.data_ptr(), k.data_ptr(), v.data_ptr(), tq.data_ptr(), tk.data_ptr(), tv.data_ptr(),
             o.data_ptr(), to.data_ptr(), lse.data_ptr(), dlse.data_ptr() if need_dlse else None,
             _strides(q, k, v, tq, tk, tv, o, to),
-            B, H, Lq, Lkv, D, float(scale), _dtype_code(q), _stream(q))
+            B, H, Lq, Lkv, D, float(scale), _dtype_code(q) if dtype_code is None else dtype_code, _stream(q))
     _check(rc, "dmf_attn_fwd_jvp")
     return (o, to, lse, dlse) if need_dlse else (o, to, lse)
 
 
-def fwd(q, k, v, scale: float, need_lse: bool = True):
+def fwd(q, k, v, scale: float, need_lse: bool = True, dtype_code=None):
     """Primal-only forward.  Returns (o, lse) (lse is None when not requested)."""
     _check_inputs(q, k, v)
     q, k, v = map(_prep, (q, k, v))
@@ -284,7 +286,7 @@ def fwd(q, k, v, scale: float, need_lse: bool = True):
     with _on(q.device):
         rc = load().dmf_attn_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if need_lse else None,
-            _strides(q, k, v, o), B, H, Lq, Lkv, D, float(scale), _dtype_code(q), _stream(q))
+            _strides(q, k, v, o), B, H, Lq, Lkv, D, float(scale), _dtype_code(q) if dtype_code is None else dtype_code, _stream(q))
     _check(rc, "dmf_attn_fwd")
     return o, lse
 
@@ -373,7 +375,7 @@ def fwd_qknorm(q, k, v, tq, tk, tv, q_gain, k_gain, eps: float, scale: float, ne
     return o, to, lse, qh, kh
 
 
-def bwd(dout, q, k, v, o, lse, scale: float, out=None):
+def bwd(dout, q, k, v, o, lse, scale: float, out=None, dtype_code=None):
     """Backward on the primal output.  Returns (dq, dk, dv): freshly allocated
     contiguous tensors, or the three tensors given as ``out`` (any (B, L, H, D)
     views with unit last-dim stride and 16-byte aligned rows, e.g. the three slots
@@ -397,9 +399,15 @@ def bwd(dout, q, k, v, o, lse, scale: float, out=None):
         rc = load().dmf_attn_bwd(
             dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr(),
-            _strides(dout, q, k, v, o, dq, dk, dv), B, H, Lq, Lkv, D, float(scale), _dtype_code(q), _stream(q))
+            _strides(dout, q, k, v, o, dq, dk, dv), B, H, Lq, Lkv, D, float(scale), _dtype_code(q) if dtype_code is None else dtype_code,
+            _stream(q))
     _check(rc, "dmf_attn_bwd")
     return dq, dk, dv
+
+
+# fp16 operands exist for the attention operator alone (the block kernels and the in-kernel norms take fp32 and bf16), so the
+# functions above keep refusing them and the operator asks for them by name.
+fwd_half, fwd_jvp_half, bwd_half = (functools.partial(f, dtype_code=DMF_ATTN_F16) for f in (fwd, fwd_jvp, bwd))
 
 
 def bwd_qknorm(dout, q_hat, k_hat, v, o, lse, q, k, q_gain, k_gain, eps: float, scale: float, out):

@@ -14,14 +14,17 @@
 // This is the computation the reference hands to the third-party
 // flash-attention backward (models/flash_attention_2_jvp.py:260-276); P is
 // recomputed from the saved logsumexp as exp(s*QK^T - lse).
+#include <type_traits>
+
 #include "attn_common.h"
 #include "attn_kernels.h"
+#include "attn_split.h"
 
 namespace dmf {
 
 // ------------------------------------------------------------------ dQ kernel
 template <typename T, int D>
-__global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const BwdParams p) {
+__device__ __forceinline__ void generic_bwd_dq_body(const BwdParams& p) {
   using C = Cfg<T, D>;
   constexpr int VEC = C::VEC, VPR = C::VPR, NCHUNK = C::NCHUNK, NDT = C::NDT;
   constexpr int STRIDE = C::STRIDE, BKV = C::BKV, NSUB = C::NSUB, PV_STEPS = C::PV_STEPS;
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const BwdParams p) {
 
 // --------------------------------------------------------------- dK/dV kernel
 template <typename T, int D>
-__global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const BwdParams p) {
+__device__ __forceinline__ void generic_bwd_dkv_body(const BwdParams& p) {
   using C = Cfg<T, D>;
   constexpr int VEC = C::VEC, VPR = C::VPR, NCHUNK = C::NCHUNK, NDT = C::NDT;
   constexpr int STRIDE = C::STRIDE, BQ = C::BKV, NSUB = C::NSUB, PV_STEPS = C::PV_STEPS;
@@ -243,12 +246,35 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(const BwdParams p) {
                               [&](int t, int i) { return dV[t][i]; });
 }
 
+// fp32 and fp16 take the split-operand bodies (attn_split.h); two fp32 rows per lane in three planes plus the accumulators need
+// the register file of one wave per SIMD.
+template <typename T, int D>
+constexpr int bwd_waves_per_simd() { return std::is_same<T, _Float16>::value && D <= 96 ? 2 : 1; }
+
+template <typename T, int D>
+__global__ __launch_bounds__(256, (bwd_waves_per_simd<T, D>())) void attn_bwd_dq_kernel(const BwdParams p) {
+  if constexpr (std::is_same<T, __bf16>::value) generic_bwd_dq_body<T, D>(p);
+  else split_bwd_dq_body<T, D, 4>(p);
+}
+template <typename T, int D>
+__global__ __launch_bounds__(256, (bwd_waves_per_simd<T, D>())) void attn_bwd_dkv_kernel(const BwdParams p) {
+  if constexpr (std::is_same<T, __bf16>::value) generic_bwd_dkv_body<T, D>(p);
+  else split_bwd_dkv_body<T, D, 4>(p);
+}
+
 template <typename T, int D>
 static int launch_bwd_t(const BwdParams& p, int BH, hipStream_t stream) {
-  using C = Cfg<T, D>;
-  constexpr int tiles = 2 * C::TILE_BYTES + 512 + 2 * C::BKV * 4;
-  constexpr int stage = 128 * C::OROWV * 16;
-  constexpr int smem = tiles > stage ? tiles : stage;
+  constexpr int smem = [] {
+    if constexpr (std::is_same<T, __bf16>::value) {
+      using C = Cfg<T, D>;
+      constexpr int tiles = 2 * C::TILE_BYTES + 512 + 2 * C::BKV * 4;
+      constexpr int stage = 128 * C::OROWV * 16;
+      return tiles > stage ? tiles : stage;
+    } else {
+      return SplitStages<T, D, 4, 2>::BYTES + 512;   // + lse, delta of two tiles (dK/dV kernel)
+    }
+  }();
+  static_assert(smem <= 160 * 1024, "LDS budget");
   auto k1 = attn_bwd_dq_kernel<T, D>;
   auto k2 = attn_bwd_dkv_kernel<T, D>;
   static bool lds_ok1[64] = {}, lds_ok2[64] = {};
@@ -271,16 +297,20 @@ static int launch_bwd_d(const BwdParams& p, int BH, int D, hipStream_t stream) {
   }
 }
 
-int launch_bwd_generic(const BwdParams& p, int BH, int D, bool bf16, hipStream_t stream) {
-  return bf16 ? launch_bwd_d<__bf16>(p, BH, D, stream) : launch_bwd_d<float>(p, BH, D, stream);
+int launch_bwd_generic(const BwdParams& p, int BH, int D, ElemType type, hipStream_t stream) {
+  switch (type) {
+    case ElemType::bf16: return launch_bwd_d<__bf16>(p, BH, D, stream);
+    case ElemType::f16: return launch_bwd_d<_Float16>(p, BH, D, stream);
+    default: return launch_bwd_d<float>(p, BH, D, stream);
+  }
 }
 
-int launch_bwd(const BwdParams& p, int BH, int D, bool bf16, hipStream_t stream) {
-  if (bf16) {
+int launch_bwd(const BwdParams& p, int BH, int D, ElemType type, hipStream_t stream) {
+  if (type == ElemType::bf16) {
     const int rc = launch_bwd_bf16_fast(p, BH, D, stream);
     if (rc != 1) return rc;   // 1 = no tuned kernel for this shape
   }
-  return launch_bwd_generic(p, BH, D, bf16, stream);
+  return launch_bwd_generic(p, BH, D, type, stream);
 }
 
 }  // namespace dmf

@@ -14,13 +14,16 @@
 // Quantities follow models/triton_utils.py:92-118 of the reference (S, dS,
 // P*dS, mu = rowsum(P*dS), lse = m + log l) but the accumulators are kept
 // unnormalised and divided once in the epilogue.
+#include <type_traits>
+
 #include "attn_common.h"
 #include "attn_kernels.h"
+#include "attn_split.h"
 
 namespace dmf {
 
 template <typename T, int D, bool JVP>
-__global__ __launch_bounds__(256) void attn_fwd_kernel(const FwdParams p) {
+__device__ __forceinline__ void generic_fwd_body(const FwdParams& p) {
   using C = Cfg<T, D>;
   constexpr int VEC = C::VEC, VPR = C::VPR, NCHUNK = C::NCHUNK, NDT = C::NDT;
   constexpr int STRIDE = C::STRIDE, BKV = C::BKV, NSUB = C::NSUB, PV_STEPS = C::PV_STEPS;
@@ -192,12 +195,32 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(const FwdParams p) {
                                 [&](int t, int i) { return fmaf(-mu_n, O[t][i] * inv_l, dO[t][i] * inv_l); });
 }
 
+// fp32 and fp16 take the split-operand body (attn_split.h).  Waves per SIMD: with fp32 tangents the operand planes alone are
+// 96 .. 192 registers, so those kernels run one wave per SIMD with the whole register file instead of spilling.
+template <typename T, int D, bool JVP>
+constexpr int fwd_waves_per_simd() {
+  if constexpr (std::is_same<T, float>::value) return JVP || D > 96 ? 1 : 2;
+  return std::is_same<T, _Float16>::value && D <= 96 ? 2 : 1;
+}
+
+template <typename T, int D, bool JVP>
+__global__ __launch_bounds__(256, (fwd_waves_per_simd<T, D, JVP>())) void attn_fwd_kernel(const FwdParams p) {
+  if constexpr (std::is_same<T, __bf16>::value) generic_fwd_body<T, D, JVP>(p);
+  else split_fwd_body<T, D, JVP, 4>(p);
+}
+
 template <typename T, int D, bool JVP>
 static int launch_fwd_t(const FwdParams& p, int BH, hipStream_t stream) {
-  using C = Cfg<T, D>;
-  constexpr int tiles = (JVP ? 4 : 2) * C::TILE_BYTES + 512;   // + slack: P*V operands read a few columns past the last row
-  constexpr int stage = 128 * C::OROWV * 16;
-  constexpr int smem = tiles > stage ? tiles : stage;
+  constexpr int smem = [] {
+    if constexpr (std::is_same<T, __bf16>::value) {
+      using C = Cfg<T, D>;
+      constexpr int tiles = (JVP ? 4 : 2) * C::TILE_BYTES + 512;   // + slack: P*V operands read a few columns past the last row
+      constexpr int stage = 128 * C::OROWV * 16;
+      return tiles > stage ? tiles : stage;
+    } else {
+      return SplitStages<T, D, 4, JVP ? 4 : 2>::BYTES;
+    }
+  }();
   auto kern = attn_fwd_kernel<T, D, JVP>;
   static bool lds_ok[64] = {};
   if (!ensure_dynamic_lds(kern, smem, lds_ok)) return -7;
@@ -218,18 +241,21 @@ static int launch_fwd_d(const FwdParams& p, int BH, int D, hipStream_t stream) {
   }
 }
 
-int launch_fwd_generic(const FwdParams& p, int BH, int D, bool bf16, bool jvp, hipStream_t stream) {
-  if (bf16) return jvp ? launch_fwd_d<__bf16, true>(p, BH, D, stream) : launch_fwd_d<__bf16, false>(p, BH, D, stream);
-  return jvp ? launch_fwd_d<float, true>(p, BH, D, stream) : launch_fwd_d<float, false>(p, BH, D, stream);
+int launch_fwd_generic(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream) {
+  switch (type) {
+    case ElemType::bf16: return jvp ? launch_fwd_d<__bf16, true>(p, BH, D, stream) : launch_fwd_d<__bf16, false>(p, BH, D, stream);
+    case ElemType::f16: return jvp ? launch_fwd_d<_Float16, true>(p, BH, D, stream) : launch_fwd_d<_Float16, false>(p, BH, D, stream);
+    default: return jvp ? launch_fwd_d<float, true>(p, BH, D, stream) : launch_fwd_d<float, false>(p, BH, D, stream);
+  }
 }
 
-int launch_fwd(const FwdParams& p, int BH, int D, bool bf16, bool jvp, hipStream_t stream) {
-  if (bf16) {
+int launch_fwd(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream) {
+  if (type == ElemType::bf16) {
     const int rc = launch_fwd_bf16_fast(p, BH, D, jvp, stream);
     if (rc != 1) return rc;   // 1 = no tuned kernel for this shape
   }
   if (p.q_gain != nullptr) return kNoQNormKernel;   // the generic kernels take already-normalised q
-  return launch_fwd_generic(p, BH, D, bf16, jvp, stream);
+  return launch_fwd_generic(p, BH, D, type, jvp, stream);
 }
 
 }  // namespace dmf

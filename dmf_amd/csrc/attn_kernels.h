@@ -6,6 +6,9 @@
 
 namespace dmf {
 
+// Element types of the attention operands; values of the C ABI's dtype argument.
+enum class ElemType { f32 = 0, bf16 = 1, f16 = 2 };
+
 // Strides are in elements: st[t] = {stride_B, stride_L, stride_H}; the head-dim
 // stride is 1 by contract.
 struct FwdParams {
@@ -97,14 +100,14 @@ inline int launch_kernel(void (*kernel)(P), dim3 grid, dim3 block, size_t lds_by
 }
 
 // Return 0 or a negative DMF_ATTN_E* code.
-int launch_fwd(const FwdParams& p, int BH, int D, bool bf16, bool jvp, hipStream_t stream);
-// Building blocks of launch_fwd: the generic kernels (fp32 and bf16, any length)
+int launch_fwd(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream);
+// Building blocks of launch_fwd: the generic kernels (any element type, any length)
 // and the tuned bf16 kernels (returns 1 when it has no kernel for the case).
-int launch_fwd_generic(const FwdParams& p, int BH, int D, bool bf16, bool jvp, hipStream_t stream);
+int launch_fwd_generic(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream);
 int launch_fwd_bf16_fast(const FwdParams& p, int BH, int D, bool jvp, hipStream_t stream);
-int launch_bwd_generic(const BwdParams& p, int BH, int D, bool bf16, hipStream_t stream);
+int launch_bwd_generic(const BwdParams& p, int BH, int D, ElemType type, hipStream_t stream);
 int launch_bwd_bf16_fast(const BwdParams& p, int BH, int D, hipStream_t stream);
-int launch_bwd(const BwdParams& p, int BH, int D, bool bf16, hipStream_t stream);
+int launch_bwd(const BwdParams& p, int BH, int D, ElemType type, hipStream_t stream);
 int launch_bwd_norm_bf16_fast(const BwdParams& p, const BwdNorm& norm, int BH, int D, hipStream_t stream);
 void bwd_norm_partials(int Lq, int Lkv, int D, int BH, int64_t& nq, int64_t& nk);
 // out_q[d] = sum over nq rows of part_q, the same for k (fp32, fixed order; block_ops.hip)

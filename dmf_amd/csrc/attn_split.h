@@ -1,0 +1,690 @@
+// Attention kernel bodies for fp32 and fp16 operands on the 16-bit matrix pipes.
+//
+// What bounds the fp32 mode is the matrix pipe: v_mfma_f32_32x32x2_f32 runs at 1/16 of the bf16 rate (157 TFLOP/s nominal,
+// 137 reached by a large library product).  A product of fp32 operands is formed here from bf16 MFMAs instead, without giving
+// up fp32 precision: every operand is the sum of three bf16 numbers (8 + 8 + 8 significant bits, each the rounded remainder
+// of the one before: x = x0 + x1 + x2 up to 2^-27 |x|), and of the nine plane products the six with i + j <= 2 are
+// accumulated in fp32, smallest first; the three left out are below 2^-26 of the product, a quarter of the rounding of an
+// fp32 multiplication.  Six MFMAs of 32x32x16 take 192 cycles where eight of 32x32x2 take 512.
+//
+// fp16 operands are exact in one f16 plane, so the score-like products are single f16 MFMAs; the probability-like operand
+// W (P, P*dS, dS: fp32 values) is split into two f16 planes (21 significant bits) so that nothing is rounded to 11 bits
+// before the final store.  P lies in [0, 2^6]; operands that carry a tangent or gradient factor have no such bound and are
+// kept in range by a per-row power of two (RowScale), raised lazily like the running maximum.
+//
+// Layouts are those of attn_common.h (transposed scores, per-lane softmax state, accumulator tile = next B operand).
+// A work-group of NW waves owns 32 NW rows of one (batch, head); tiles of 32 streamed rows travel HBM -> registers -> planes
+// -> LDS, each element being split once per work-group, and every plane chunk read from LDS feeds up to three MFMAs.
+#pragma once
+#include "attn_common.h"
+#include "attn_kernels.h"
+
+namespace dmf {
+
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(2))) __fp16 fp16x2;
+
+// NI planes of a loaded operand, NWT of a probability-like one.
+template <typename T> struct SplitType;
+template <> struct SplitType<float> { static constexpr int NI = 3, NWT = 3; static constexpr bool F16 = false; };
+template <> struct SplitType<_Float16> { static constexpr int NI = 1, NWT = 2; static constexpr bool F16 = true; };
+
+template <>
+__device__ __forceinline__ void store4<_Float16>(_Float16* dst, float a, float b, float c, float d) {
+  typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+  *reinterpret_cast<f16x4*>(dst) = f16x4{(_Float16)a, (_Float16)b, (_Float16)c, (_Float16)d};
+}
+
+template <typename T>
+__device__ __forceinline__ void mma_one(f32x16& acc, const u32x4& a, const u32x4& b) {
+  if constexpr (SplitType<T>::F16)
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
+  else
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+}
+template <typename T>
+__device__ __forceinline__ void mma_one16(f32x4& acc, const u32x4& a, const u32x4& b) {
+  if constexpr (SplitType<T>::F16)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
+  else
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+}
+
+// acc += sum of a_i b_j over i + j < max(NA, NB), smallest products first.
+template <int NA, int NB, typename F>
+__device__ __forceinline__ void for_plane_pairs(F&& f) {
+  constexpr int MX = (NA > NB ? NA : NB) - 1;
+#pragma unroll
+  for (int s = MX; s >= 0; --s)
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if (s - i >= 0 && s - i < NB) f(i, s - i);
+}
+template <typename T, int NA, int NB>
+__device__ __forceinline__ void mma_planes(f32x16& acc, const u32x4 (&a)[NA], const u32x4 (&b)[NB]) {
+  for_plane_pairs<NA, NB>([&](int i, int j) { mma_one<T>(acc, a[i], b[j]); });
+}
+template <typename T, int NA, int NB>
+__device__ __forceinline__ void mma_planes16(f32x4& acc, const u32x4 (&a)[NA], const u32x4 (&b)[NB]) {
+  for_plane_pairs<NA, NB>([&](int i, int j) { mma_one16<T>(acc, a[i], b[j]); });
+}
+
+// Eight fp32 values as NP planes of eight 16-bit ones.
+template <typename T, int NP>
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      if constexpr (SplitType<T>::F16) {
+        const fp16x2 h = __builtin_amdgcn_cvt_pkrtz(a, b);
+        pl[k][i] = __builtin_bit_cast(uint32_t, h);
+        if (k + 1 < NP) {
+          a -= (float)h[0];
+          b -= (float)h[1];
+        }
+      } else {
+        const uint32_t h = pack_bf16x2(a, b);
+        pl[k][i] = h;
+        if (k + 1 < NP) {
+          a -= __uint_as_float(h << 16);
+          b -= __uint_as_float(h & 0xffff0000u);
+        }
+      }
+    }
+  }
+}
+
+// Odd, and rows 0 .. 3 apart modulo 16 vectors: free of bank conflicts for row and for transposed reads.
+constexpr int split_pitch(int min_vectors) {
+  for (int p = min_vectors | 1;; p += 2) {
+    const int m = p % 16;
+    if (m == 3 || m == 7 || m == 9 || m == 13) return p;
+  }
+}
+
+template <typename T, int D, int NW>
+struct SplitCfg {
+  using S = SplitType<T>;
+  static constexpr int VPR = D / 8, NCHUNK = (D + 15) / 16;          // 8-element vectors per row; contraction chunks over the head dim
+  static constexpr int P = split_pitch(2 * NCHUNK), STR = P * 8;     // tile row pitch in vectors / elements
+  static constexpr int PLANE = 32 * P * 16, TILE = S::NI * PLANE;    // bytes
+  static constexpr bool TAIL = (D % 32) != 0 && (D % 32) <= 16;      // 16-wide remainder by 16x16x32 MFMAs (72, 80)
+  static constexpr int NMT = TAIL ? D / 32 : (D + 31) / 32;
+  static constexpr int ITERS = (32 * VPR + 64 * NW - 1) / (64 * NW); // vectors of a tile per thread
+  static constexpr int RAW = sizeof(T) / 2;                          // 16-byte registers quads per vector
+  static constexpr int STAGE_ROWS_BYTES = 32 * NW * Cfg<T, D>::OROWV * 16;
+};
+
+// One streamed tensor tile of 32 rows: load() requests this thread's vectors (rows at or past nrows read as zero), commit()
+// splits them and writes the planes.
+template <typename T, int D, int NW>
+struct TileLoad {
+  using C = SplitCfg<T, D, NW>;
+  u32x4 r[C::ITERS][C::RAW];
+  __device__ __forceinline__ void load(const T* src, int64_t row_stride, int row0, int nrows, int tid) {
+#pragma unroll
+    for (int it = 0; it < C::ITERS; ++it) {
+      const int v = tid + it * 64 * NW, row = v / C::VPR, cv = v % C::VPR;
+      const bool ok = v < 32 * C::VPR && row0 + row < nrows;
+      const u32x4* g = reinterpret_cast<const u32x4*>(src + (int64_t)(row0 + row) * row_stride + cv * 8);
+#pragma unroll
+      for (int k = 0; k < C::RAW; ++k) r[it][k] = ok ? g[k] : u32x4{0, 0, 0, 0};
+    }
+  }
+  __device__ __forceinline__ void commit(char* tile, int tid) const {
+#pragma unroll
+    for (int it = 0; it < C::ITERS; ++it) {
+      const int v = tid + it * 64 * NW, row = v / C::VPR, cv = v % C::VPR;
+      if (v < 32 * C::VPR) {
+        char* dst = tile + (row * C::P + cv) * 16;
+        if constexpr (SplitType<T>::F16) {
+          *reinterpret_cast<u32x4*>(dst) = r[it][0];
+        } else {
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[e] = __uint_as_float(r[it][0][e]);
+            x[4 + e] = __uint_as_float(r[it][C::RAW - 1][e]);
+          }
+          u32x4 pl[SplitType<T>::NI];
+          split8<T>(x, pl);
+#pragma unroll
+          for (int k = 0; k < SplitType<T>::NI; ++k) *reinterpret_cast<u32x4*>(dst + k * C::PLANE) = pl[k];
+        }
+      }
+    }
+  }
+};
+
+// Operand planes of this lane's own row (register resident): chunk c = elements 16c + 8g .. +7; zero past the head dim or the end.
+template <typename T, int D, int NW>
+__device__ __forceinline__ void load_own_row(const T* base, int64_t row_stride, int row, int nrows, int g,
+                                             u32x4 (&out)[SplitCfg<T, D, NW>::NCHUNK][SplitType<T>::NI]) {
+  using C = SplitCfg<T, D, NW>;
+#pragma unroll
+  for (int c = 0; c < C::NCHUNK; ++c) {
+    const bool in = row < nrows && 2 * c + g < C::VPR;
+    const u32x4* p = reinterpret_cast<const u32x4*>(base + (int64_t)row * row_stride + 16 * c + 8 * g);
+    const u32x4 a = in ? p[0] : u32x4{0, 0, 0, 0};
+    if constexpr (SplitType<T>::F16) {
+      out[c][0] = a;
+    } else {
+      const u32x4 b = in ? p[1] : u32x4{0, 0, 0, 0};
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = __uint_as_float(a[e]);
+        x[4 + e] = __uint_as_float(b[e]);
+      }
+      split8<T>(x, out[c]);
+    }
+  }
+}
+
+// Planes of operand chunk c of row `row` of a tile (contraction along the row) ...
+template <typename T, int D, int NW>
+__device__ __forceinline__ void row_planes(const char* tile, int row, int c, int g, u32x4 (&out)[SplitType<T>::NI]) {
+  using C = SplitCfg<T, D, NW>;
+#pragma unroll
+  for (int k = 0; k < SplitType<T>::NI; ++k)
+    out[k] = *reinterpret_cast<const u32x4*>(tile + k * C::PLANE + (row * C::P + 2 * c + g) * 16);
+}
+// ... and of the transposed one: 16 tile rows (step s) at columns col0 .. col0 + 31,
+template <typename T, int D, int NW>
+__device__ __forceinline__ void col_planes(const char* tile, int col0, int s, int lane, u32x4 (&out)[SplitType<T>::NI]) {
+  using C = SplitCfg<T, D, NW>;
+#pragma unroll
+  for (int k = 0; k < SplitType<T>::NI; ++k)
+    out[k] = lds_col_operand<__bf16, C::STR>(reinterpret_cast<const __bf16*>(tile + k * C::PLANE), 0, col0, s, lane).v;
+}
+// or all 32 tile rows at the 16 remainder columns.
+template <typename T, int D, int NW>
+__device__ __forceinline__ void tail_planes(const char* tile, int lane, u32x4 (&out)[SplitType<T>::NI]) {
+  using C = SplitCfg<T, D, NW>;
+#pragma unroll
+  for (int k = 0; k < SplitType<T>::NI; ++k) {
+    const __bf16* p = reinterpret_cast<const __bf16*>(tile + k * C::PLANE) + tail_lane_offset(lane, C::STR, 32 * C::NMT);
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p)));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p + 8 * C::STR)));
+    out[k] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  }
+}
+
+// Transposed accumulators of 32 output rows: NMT full 32-wide tiles and, with a remainder, two 16x16 ones (one per half of the
+// wave's 32 rows).
+template <typename T, int D, int NW>
+struct OutAcc {
+  using C = SplitCfg<T, D, NW>;
+  f32x16 t[C::NMT];
+  f32x4 tail[2];
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < C::NMT; ++i) t[i] = f32x16{0};
+    tail[0] = tail[1] = f32x4{0, 0, 0, 0};
+  }
+  // by a factor per row (= lane % 32)
+  __device__ __forceinline__ void scale(float f) {
+#pragma unroll
+    for (int i = 0; i < C::NMT; ++i) t[i] *= f;
+    if constexpr (C::TAIL) {
+      float f0, f1;
+      swap16f(f, f0, f1);
+      tail[0] *= f0;
+      tail[1] *= f1;
+    }
+  }
+};
+
+// W operand of a 32x32 tile: planes of steps 0 and 1, and their re-distribution for the remainder products.
+template <typename T>
+struct WOperand {
+  u32x4 s[2][SplitType<T>::NWT];
+  __device__ __forceinline__ void form(const f32x16& e) {
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = e[8 * st + i];
+      split8<T>(x, s[st]);
+    }
+  }
+  __device__ __forceinline__ void tail(u32x4 (&h0)[SplitType<T>::NWT], u32x4 (&h1)[SplitType<T>::NWT]) const {
+#pragma unroll
+    for (int k = 0; k < SplitType<T>::NWT; ++k) {
+      ColOperand a, b, x, y;
+      a.v = s[0][k];
+      b.v = s[1][k];
+      tail_operands(a, b, x, y);
+      h0[k] = x.v;
+      h1[k] = y.v;
+    }
+  }
+};
+
+// acc^T += tile^T W over the 32 rows of a tile, for one or two (acc, W) pairs that share the tile.
+template <typename T, int D, int NW>
+__device__ __forceinline__ void contract_rows(const char* tile, int lane, OutAcc<T, D, NW>& a0, const WOperand<T>& w0) {
+  using C = SplitCfg<T, D, NW>;
+  constexpr int NI = SplitType<T>::NI, NWT = SplitType<T>::NWT;
+#pragma unroll
+  for (int st = 0; st < 2; ++st)
+#pragma unroll
+    for (int t = 0; t < C::NMT; ++t) {
+      u32x4 v[NI];
+      col_planes<T, D, NW>(tile, 32 * t, st, lane, v);
+      mma_planes<T>(a0.t[t], v, w0.s[st]);
+    }
+  if constexpr (C::TAIL) {
+    u32x4 v[NI], h0[NWT], h1[NWT];
+    tail_planes<T, D, NW>(tile, lane, v);
+    w0.tail(h0, h1);
+    mma_planes16<T>(a0.tail[0], v, h0);
+    mma_planes16<T>(a0.tail[1], v, h1);
+  }
+}
+template <typename T, int D, int NW>
+__device__ __forceinline__ void contract_rows(const char* tile, int lane, OutAcc<T, D, NW>& a0, const WOperand<T>& w0,
+                                              OutAcc<T, D, NW>& a1, const WOperand<T>& w1) {
+  using C = SplitCfg<T, D, NW>;
+  constexpr int NI = SplitType<T>::NI, NWT = SplitType<T>::NWT;
+#pragma unroll
+  for (int st = 0; st < 2; ++st)
+#pragma unroll
+    for (int t = 0; t < C::NMT; ++t) {
+      u32x4 v[NI];
+      col_planes<T, D, NW>(tile, 32 * t, st, lane, v);
+      mma_planes<T>(a0.t[t], v, w0.s[st]);
+      mma_planes<T>(a1.t[t], v, w1.s[st]);
+    }
+  if constexpr (C::TAIL) {
+    u32x4 v[NI], h0[NWT], h1[NWT];
+    tail_planes<T, D, NW>(tile, lane, v);
+    w0.tail(h0, h1);
+    mma_planes16<T>(a0.tail[0], v, h0);
+    mma_planes16<T>(a0.tail[1], v, h1);
+    w1.tail(h0, h1);
+    mma_planes16<T>(a1.tail[0], v, h0);
+    mma_planes16<T>(a1.tail[1], v, h1);
+  }
+}
+
+// Power of two per output row that keeps an unbounded W operand inside the f16 range (fp16 operands only): W is multiplied by
+// `mul` before it is split and the accumulator it feeds carries the same factor until the epilogue divides it out.  mul = 2^-e
+// for the largest magnitude 2^e seen when it was last set; raised when a magnitude exceeds 32 times that.
+template <typename T>
+struct RowScale {
+  float mul = 1.f, limit = 0.f;
+  template <typename A>
+  __device__ __forceinline__ void update(const f32x16& w, A& acc) {
+    if constexpr (SplitType<T>::F16) {
+      float mx = fmaxf(fabsf(w[0]), fabsf(w[1]));
+#pragma unroll
+      for (int i = 2; i < 16; ++i) mx = fmaxf(mx, fabsf(w[i]));
+      mx = xhalf_max(mx);
+      if (__builtin_amdgcn_ballot_w64(mx > limit) != 0) {
+        const uint32_t e = __float_as_uint(mx) & 0x7f800000u;
+        const bool up = mx > limit && e > 0 && e < 0x7f000000u;
+        const float m2 = up ? __uint_as_float(0x7f000000u - e) : mul;
+        limit = up ? 32.f * __uint_as_float(e) : limit;
+        acc.scale(m2 / mul);
+        mul = m2;
+      }
+    }
+  }
+  __device__ __forceinline__ float inverse() const { return SplitType<T>::F16 ? 1.f / mul : 1.f; }
+};
+
+// Zero the vectors past the head dim of NT tile planes once; commits never touch them.
+template <typename T, int D, int NW>
+__device__ __forceinline__ void zero_plane_pads(char* planes, int nplanes, int tid) {
+  using C = SplitCfg<T, D, NW>;
+  constexpr int PADV = C::P - C::VPR;
+  for (int i = tid; i < nplanes * 32 * PADV; i += 64 * NW)
+    *reinterpret_cast<u32x4*>(planes + (i / PADV) * C::P * 16 + (C::VPR + i % PADV) * 16) = u32x4{0, 0, 0, 0};
+}
+
+// Epilogue: rows of a transposed accumulator, times a factor per row, staged through LDS and stored.
+template <typename T, int D, int NW>
+__device__ __forceinline__ void store_out(char* smem, T* dst, int64_t row_stride, int row0, int nrows, int tid, const OutAcc<T, D, NW>& a,
+                                          float f) {
+  using C = SplitCfg<T, D, NW>;
+  float f16[2] = {f, f};
+  if constexpr (C::TAIL) swap16f(f, f16[0], f16[1]);
+  store_rows_transposed<T, D, NW, C::NMT>(reinterpret_cast<T*>(smem), dst, row_stride, row0, nrows, tid,
+                                          [&](int t, int i) { return a.t[t][i] * f; },
+                                          [&](void* ws) {
+                                            if constexpr (C::TAIL)
+                                              store_tail16<T, D, C::NMT>(ws, tid & 63, [&](int hq, int e) { return a.tail[hq][e] * f16[hq]; });
+                                          });
+}
+
+// ------------------------------------------------------------------------------------------------- forward (+ JVP)
+// Stages of K, V [, dK, dV] planes in LDS: two when they fit beside each other (one barrier per tile), else one.
+template <typename T, int D, int NW, int NT>
+struct SplitStages {
+  static constexpr int STAGE = NT * SplitCfg<T, D, NW>::TILE;
+  static constexpr int N = 2 * STAGE <= 160 * 1024 ? 2 : 1;
+  static constexpr int BYTES = N * STAGE > SplitCfg<T, D, NW>::STAGE_ROWS_BYTES ? N * STAGE : SplitCfg<T, D, NW>::STAGE_ROWS_BYTES;
+  static_assert(STAGE <= 160 * 1024 && BYTES <= 160 * 1024, "LDS budget");
+};
+
+constexpr float kSplitLazyLog2 = 6.0f;   // the running maximum is raised when exceeded by more than 2^6 (exact: normalised once at the end)
+
+template <typename T, int D, bool JVP, int NW>
+__device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
+  using C = SplitCfg<T, D, NW>;
+  constexpr int NI = SplitType<T>::NI, NCHUNK = C::NCHUNK, NT = JVP ? 4 : 2, BQ = 32 * NW;
+  using ST = SplitStages<T, D, NW, NT>;
+  constexpr bool F16 = SplitType<T>::F16;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c32 = lane & 31, g = lane >> 5;
+  const uint32_t nqb = (p.Lq + BQ - 1) / BQ;
+  const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int bh = wg / nqb, q0 = (wg % nqb) * BQ, b = bh / p.H, h = bh % p.H;
+  auto base = [&](int t) { return (int64_t)b * p.st[t][0] + (int64_t)h * p.st[t][2]; };
+  const int qrow = q0 + wave * 32 + c32;
+
+  zero_plane_pads<T, D, NW>(smem, ST::N * NT * NI, tid);
+
+  const T* src[4] = {static_cast<const T*>(p.k) + base(1), static_cast<const T*>(p.v) + base(2), JVP ? static_cast<const T*>(p.tk) + base(4) : nullptr,
+                     JVP ? static_cast<const T*>(p.tv) + base(5) : nullptr};
+  const int64_t rs[4] = {p.st[1][1], p.st[2][1], p.st[4][1], p.st[5][1]};
+  TileLoad<T, D, NW> ld[NT];
+  auto load = [&](int it) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) ld[t].load(src[t], rs[t], it * 32, p.Lkv, tid);
+  };
+  auto tile = [&](int it, int t) { return smem + (ST::N == 2 ? (it & 1) * ST::STAGE : 0) + t * C::TILE; };
+  auto commit = [&](int it) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) ld[t].commit(tile(it, t), tid);
+  };
+  load(0);
+
+  u32x4 Q[NCHUNK][NI], dQ[JVP ? NCHUNK : 1][NI];
+  load_own_row<T, D, NW>(static_cast<const T*>(p.q) + base(0), p.st[0][1], qrow, p.Lq, g, Q);
+  if constexpr (JVP) load_own_row<T, D, NW>(static_cast<const T*>(p.tq) + base(3), p.st[3][1], qrow, p.Lq, g, dQ);
+
+  OutAcc<T, D, NW> O, dO, dOv;   // dOv (fp16 tangents only): dV^T P, apart because dO carries the row scale of P*dS
+  O.zero();
+  if constexpr (JVP) {
+    dO.zero();
+    if constexpr (F16) dOv.zero();
+  }
+  RowScale<T> gs;
+  float m_run = -INFINITY, l_run = 0.f, mu_run = 0.f;
+  const float c2 = p.scale_log2;
+
+  const int ntiles = (p.Lkv + 31) / 32;
+  commit(0);
+  for (int it = 0; it < ntiles; ++it) {
+    __syncthreads();                     // tile `it` is in LDS
+    if (it + 1 < ntiles) load(it + 1);   // in flight during the math
+    const char *Kt = tile(it, 0), *Vt = tile(it, 1), *dKt = tile(it, 2), *dVt = tile(it, 3);
+    f32x16 S = {0}, dS = {0};
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c) {
+      u32x4 k[NI];
+      row_planes<T, D, NW>(Kt, c32, c, g, k);
+      mma_planes<T>(S, k, Q[c]);
+      if constexpr (JVP) {
+        u32x4 dk[NI];
+        row_planes<T, D, NW>(dKt, c32, c, g, dk);
+        mma_planes<T>(dS, k, dQ[c]);
+        mma_planes<T>(dS, dk, Q[c]);
+      }
+    }
+    if ((it + 1) * 32 > p.Lkv) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (it * 32 + acc_row(i, g) >= p.Lkv) S[i] = -INFINITY;
+    }
+    float mx = fmaxf(S[0], S[1]);
+#pragma unroll
+    for (int i = 2; i < 16; ++i) mx = fmaxf(mx, S[i]);
+    mx = xhalf_max(mx) * c2;
+    if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
+      const float m_new = fmaxf(m_run, mx), alpha = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+      O.scale(alpha);
+      if constexpr (JVP) {
+        mu_run *= alpha;
+        dO.scale(alpha);
+        if constexpr (F16) dOv.scale(alpha);
+      }
+    }
+    f32x16 E, G;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      E[i] = fast_exp2(fmaf(S[i], c2, -m_run));
+      l_run += E[i];
+      if constexpr (JVP) {
+        G[i] = E[i] * (dS[i] * p.scale);
+        mu_run += G[i];
+      }
+    }
+    WOperand<T> we;
+    we.form(E);
+    if constexpr (JVP) {
+      gs.update(G, dO);
+      if constexpr (F16) G *= gs.mul;
+      WOperand<T> wg_;
+      wg_.form(G);
+      contract_rows<T, D, NW>(Vt, lane, O, we, dO, wg_);
+      if constexpr (F16) contract_rows<T, D, NW>(dVt, lane, dOv, we);
+      else contract_rows<T, D, NW>(dVt, lane, dO, we);
+    } else {
+      contract_rows<T, D, NW>(Vt, lane, O, we);
+    }
+    if constexpr (ST::N == 1) __syncthreads();   // every wave is done with the stage
+    if (it + 1 < ntiles) commit(it + 1);
+  }
+
+  const float l_tot = xhalf_sum(l_run), inv_l = 1.0f / l_tot;
+  const float mu_n = JVP ? xhalf_sum(mu_run) * inv_l : 0.f;
+  if (g == 0 && qrow < p.Lq) {
+    if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + qrow] = (m_run + log2f(l_tot)) * kLn2;
+    if constexpr (JVP)
+      if (p.dlse != nullptr) p.dlse[(int64_t)bh * p.Lq + qrow] = mu_n;
+  }
+  store_out<T, D, NW>(smem, static_cast<T*>(p.o) + base(6), p.st[6][1], q0, p.Lq, tid, O, inv_l);
+  if constexpr (JVP) {
+    // dO/l - (mu/l) O, in place
+    const float gi = gs.inverse();
+#pragma unroll
+    for (int t = 0; t < C::NMT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float d = F16 ? fmaf(dO.t[t][i], gi, dOv.t[t][i]) : dO.t[t][i];
+        dO.t[t][i] = fmaf(-mu_n, O.t[t][i], d);
+      }
+    if constexpr (C::TAIL) {
+      float mu16[2], gi16[2];
+      swap16f(mu_n, mu16[0], mu16[1]);
+      swap16f(gi, gi16[0], gi16[1]);
+#pragma unroll
+      for (int hq = 0; hq < 2; ++hq)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float d = F16 ? fmaf(dO.tail[hq][e], gi16[hq], dOv.tail[hq][e]) : dO.tail[hq][e];
+          dO.tail[hq][e] = fmaf(-mu16[hq], O.tail[hq][e], d);
+        }
+    }
+    store_out<T, D, NW>(smem, static_cast<T*>(p.to) + base(7), p.st[7][1], q0, p.Lq, tid, dO, inv_l);
+  }
+}
+
+// --------------------------------------------------------------------------------------------------------- backward
+template <typename T, int D, int NW>
+__device__ __forceinline__ void split_bwd_dq_body(const BwdParams& p) {
+  using C = SplitCfg<T, D, NW>;
+  constexpr int NI = SplitType<T>::NI, NCHUNK = C::NCHUNK, BQ = 32 * NW;
+  using ST = SplitStages<T, D, NW, 2>;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c32 = lane & 31, g = lane >> 5;
+  const uint32_t nqb = (p.Lq + BQ - 1) / BQ;
+  const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int bh = wg / nqb, q0 = (wg % nqb) * BQ, b = bh / p.H, h = bh % p.H;
+  auto base = [&](int t) { return (int64_t)b * p.st[t][0] + (int64_t)h * p.st[t][2]; };
+  const int qrow = q0 + wave * 32 + c32;
+  const bool qok = qrow < p.Lq;
+
+  zero_plane_pads<T, D, NW>(smem, ST::N * 2 * NI, tid);
+  TileLoad<T, D, NW> lk, lv;
+  auto load = [&](int it) {
+    lk.load(static_cast<const T*>(p.k) + base(2), p.st[2][1], it * 32, p.Lkv, tid);
+    lv.load(static_cast<const T*>(p.v) + base(3), p.st[3][1], it * 32, p.Lkv, tid);
+  };
+  auto tile = [&](int it) { return smem + (ST::N == 2 ? (it & 1) * ST::STAGE : 0); };
+  auto commit = [&](int it) {
+    lk.commit(tile(it), tid);
+    lv.commit(tile(it) + C::TILE, tid);
+  };
+  load(0);
+
+  u32x4 Q[NCHUNK][NI], dO[NCHUNK][NI];
+  load_own_row<T, D, NW>(static_cast<const T*>(p.q) + base(1), p.st[1][1], qrow, p.Lq, g, Q);
+  load_own_row<T, D, NW>(static_cast<const T*>(p.dout) + base(0), p.st[0][1], qrow, p.Lq, g, dO);
+  float dpart = 0.f;   // delta = rowsum(dout * o)
+  if (qok) {
+    const T* gdo = static_cast<const T*>(p.dout) + base(0) + (int64_t)qrow * p.st[0][1] + 8 * g;
+    const T* go = static_cast<const T*>(p.o) + base(4) + (int64_t)qrow * p.st[4][1] + 8 * g;
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c)
+      if (2 * c + g < C::VPR)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dpart = fmaf((float)gdo[16 * c + e], (float)go[16 * c + e], dpart);
+  }
+  const float delta = xhalf_sum(dpart);
+  float lse2 = INFINITY;   // +inf switches padded rows off
+  if (qok) {
+    lse2 = p.lse[(int64_t)bh * p.Lq + qrow] * kLog2e;
+    if (g == 0) p.delta[(int64_t)bh * p.Lq + qrow] = delta;
+  }
+  OutAcc<T, D, NW> acc;
+  acc.zero();
+  RowScale<T> gs;
+  const float c2 = p.scale_log2;
+  const int ntiles = (p.Lkv + 31) / 32;
+  commit(0);
+  for (int it = 0; it < ntiles; ++it) {
+    __syncthreads();
+    if (it + 1 < ntiles) load(it + 1);
+    const char *Kt = tile(it), *Vt = Kt + C::TILE;
+    f32x16 S = {0}, dP = {0}, dS;
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c) {
+      u32x4 x[NI];
+      row_planes<T, D, NW>(Kt, c32, c, g, x);
+      mma_planes<T>(S, x, Q[c]);
+      row_planes<T, D, NW>(Vt, c32, c, g, x);
+      mma_planes<T>(dP, x, dO[c]);
+    }
+    const bool last = (it + 1) * 32 > p.Lkv;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float pr = fast_exp2(fmaf(S[i], c2, -lse2));
+      if (last && it * 32 + acc_row(i, g) >= p.Lkv) pr = 0.f;
+      dS[i] = pr * (dP[i] - delta);
+    }
+    gs.update(dS, acc);
+    if constexpr (SplitType<T>::F16) dS *= gs.mul;
+    WOperand<T> w;
+    w.form(dS);
+    contract_rows<T, D, NW>(Kt, lane, acc, w);
+    if constexpr (ST::N == 1) __syncthreads();
+    if (it + 1 < ntiles) commit(it + 1);
+  }
+  store_out<T, D, NW>(smem, static_cast<T*>(p.dq) + base(5), p.st[5][1], q0, p.Lq, tid, acc, p.scale * gs.inverse());
+}
+
+template <typename T, int D, int NW>
+__device__ __forceinline__ void split_bwd_dkv_body(const BwdParams& p) {
+  using C = SplitCfg<T, D, NW>;
+  constexpr int NI = SplitType<T>::NI, NCHUNK = C::NCHUNK, BK = 32 * NW;
+  using ST = SplitStages<T, D, NW, 2>;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c32 = lane & 31, g = lane >> 5;
+  const uint32_t nkb = (p.Lkv + BK - 1) / BK;
+  const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int bh = wg / nkb, k0 = (wg % nkb) * BK, b = bh / p.H, h = bh % p.H;
+  auto base = [&](int t) { return (int64_t)b * p.st[t][0] + (int64_t)h * p.st[t][2]; };
+  const int krow = k0 + wave * 32 + c32;
+
+  zero_plane_pads<T, D, NW>(smem, ST::N * 2 * NI, tid);
+  TileLoad<T, D, NW> lq, lo;
+  // lse (log2 units; +inf for rows past the end: P = 0) and delta of the tile's 32 queries, one per lane: rows acc_row order
+  // is read back with bpermute-free broadcasts from LDS
+  float* stat = reinterpret_cast<float*>(smem + ST::BYTES);   // [stage][2][32]
+  float st_pre = 0.f;
+  auto load = [&](int it) {
+    lq.load(static_cast<const T*>(p.q) + base(1), p.st[1][1], it * 32, p.Lq, tid);
+    lo.load(static_cast<const T*>(p.dout) + base(0), p.st[0][1], it * 32, p.Lq, tid);
+    if (tid < 64) {
+      const int r = it * 32 + (tid & 31);
+      const bool ok = r < p.Lq;
+      if (tid < 32) st_pre = ok ? p.lse[(int64_t)bh * p.Lq + r] * kLog2e : INFINITY;
+      else st_pre = ok ? p.delta[(int64_t)bh * p.Lq + r] : 0.f;
+    }
+  };
+  auto tile = [&](int it) { return smem + (ST::N == 2 ? (it & 1) * ST::STAGE : 0); };
+  auto commit = [&](int it) {
+    lq.commit(tile(it), tid);
+    lo.commit(tile(it) + C::TILE, tid);
+    if (tid < 64) stat[(it & 1) * 64 + tid] = st_pre;
+  };
+  load(0);
+  u32x4 K[NCHUNK][NI], V[NCHUNK][NI];
+  load_own_row<T, D, NW>(static_cast<const T*>(p.k) + base(2), p.st[2][1], krow, p.Lkv, g, K);
+  load_own_row<T, D, NW>(static_cast<const T*>(p.v) + base(3), p.st[3][1], krow, p.Lkv, g, V);
+  OutAcc<T, D, NW> dK, dV;
+  dK.zero();
+  dV.zero();
+  RowScale<T> gs;
+  const float c2 = p.scale_log2;
+  const int ntiles = (p.Lq + 31) / 32;
+  commit(0);
+  for (int it = 0; it < ntiles; ++it) {
+    __syncthreads();
+    if (it + 1 < ntiles) load(it + 1);
+    const char *Qt = tile(it), *dOt = Qt + C::TILE;
+    const float* ls = stat + (it & 1) * 64 + 4 * g;
+    f32x16 S = {0}, dP = {0}, Pm, dS;
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c) {
+      u32x4 x[NI];
+      row_planes<T, D, NW>(Qt, c32, c, g, x);
+      mma_planes<T>(S, x, K[c]);
+      row_planes<T, D, NW>(dOt, c32, c, g, x);
+      mma_planes<T>(dP, x, V[c]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 l4 = *reinterpret_cast<const f32x4*>(ls + 8 * j), d4 = *reinterpret_cast<const f32x4*>(ls + 32 + 8 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * j + e;
+        Pm[i] = fast_exp2(fmaf(S[i], c2, -l4[e]));
+        dS[i] = Pm[i] * (dP[i] - d4[e]);
+      }
+    }
+    WOperand<T> wp;
+    wp.form(Pm);
+    contract_rows<T, D, NW>(dOt, lane, dV, wp);
+    gs.update(dS, dK);
+    if constexpr (SplitType<T>::F16) dS *= gs.mul;
+    WOperand<T> ws;
+    ws.form(dS);
+    contract_rows<T, D, NW>(Qt, lane, dK, ws);
+    if constexpr (ST::N == 1) __syncthreads();
+    if (it + 1 < ntiles) commit(it + 1);
+  }
+  store_out<T, D, NW>(smem, static_cast<T*>(p.dk) + base(6), p.st[6][1], k0, p.Lkv, tid, dK, p.scale * gs.inverse());
+  store_out<T, D, NW>(smem, static_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid, dV, 1.f);
+}
+
+}  // namespace dmf

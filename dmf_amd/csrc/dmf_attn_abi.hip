@@ -26,7 +26,7 @@ int check_tensor(const void* ptr, const int64_t* st4, int elem_bytes, int64_t (&
 }
 
 int check_common(int B, int H, int Lq, int Lkv, int D, int dtype) {
-  if (dtype != DMF_ATTN_F32 && dtype != DMF_ATTN_BF16) return DMF_ATTN_EDTYPE;
+  if (dtype != DMF_ATTN_F32 && dtype != DMF_ATTN_BF16 && dtype != DMF_ATTN_F16) return DMF_ATTN_EDTYPE;
   if (!head_dim_ok(D)) return DMF_ATTN_EHEADDIM;
   if (B < 1 || H < 1 || Lq < 1 || Lkv < 1) return DMF_ATTN_ESHAPE;
   const int64_t blocks = (int64_t)B * H * ((std::max(Lq, Lkv) + 127) / 128);
@@ -43,7 +43,7 @@ int dmf_attn_version(void) { return kVersion; }
 const char* dmf_attn_strerror(int code) {
   switch (code) {
     case DMF_ATTN_OK: return "ok";
-    case DMF_ATTN_EDTYPE: return "unsupported dtype (expected DMF_ATTN_F32 or DMF_ATTN_BF16)";
+    case DMF_ATTN_EDTYPE: return "unsupported dtype (expected DMF_ATTN_F32, DMF_ATTN_BF16 or, for attention, DMF_ATTN_F16)";
     case DMF_ATTN_EHEADDIM: return "unsupported head dim (supported: 32, 64, 72, 80, 96, 128)";
     case DMF_ATTN_ESHAPE: return "bad shape (a dimension is < 1 or the grid would overflow)";
     case DMF_ATTN_ESTRIDE: return "bad stride (last-dim stride must be 1, other strides non-negative multiples of 16 bytes)";
@@ -65,13 +65,14 @@ static int fwd_impl(const void* q, const void* k, const void* v, const void* tq,
                     void* k_hat = nullptr) {
   if (int rc = check_common(B, H, Lq, Lkv, D, dtype)) return rc;
   if (strides == nullptr) return DMF_ATTN_ENULL;
-  const int eb = dtype == DMF_ATTN_BF16 ? 2 : 4;
+  const int eb = dtype == DMF_ATTN_F32 ? 4 : 2;
   dmf::FwdParams p{};
   // parameter-block slots: q k v tq tk tv o to
   const void* ptrs[8] = {q, k, v, tq, tk, tv, o, to};
   const int slots_jvp[8] = {0, 1, 2, 3, 4, 5, 6, 7};
   const int slots_fwd[4] = {0, 1, 2, 6};
   const int n = jvp ? 8 : 4;
+  if (dtype == DMF_ATTN_F16 && q_gain != nullptr) return DMF_ATTN_ENOKERNEL;
   // the q-norm entry point always passes the 8-tensor stride table
   const bool wide = jvp || q_gain != nullptr;
   for (int i = 0; i < n; ++i) {
@@ -85,7 +86,7 @@ static int fwd_impl(const void* q, const void* k, const void* v, const void* tq,
   p.scale = scale; p.scale_log2 = scale * 1.4426950408889634f;
   p.q_gain = q_gain; p.q_eps = q_eps;
   p.k_gain = k_gain; p.q_hat = q_hat; p.k_hat = k_hat;
-  return dmf::launch_fwd(p, B * H, D, dtype == DMF_ATTN_BF16, jvp, static_cast<hipStream_t>(stream));
+  return dmf::launch_fwd(p, B * H, D, static_cast<dmf::ElemType>(dtype), jvp, static_cast<hipStream_t>(stream));
 }
 
 int dmf_attn_fwd_qnorm(const void* q, const void* k, const void* v, const void* tq, const void* tk, const void* tv,
@@ -131,7 +132,7 @@ int dmf_attn_plan(int entry, int B, int H, int Lq, int Lkv, int D, int dtype, ch
   if (buf == nullptr || buflen < 1) return DMF_ATTN_ENULL;
   if (entry < DMF_ATTN_PLAN_FWD || entry > DMF_ATTN_PLAN_FWD_QKNORM_JVP) return DMF_ATTN_ESHAPE;
   const bool bf16 = dtype == DMF_ATTN_BF16;
-  const char* t = bf16 ? "__bf16" : "float";
+  const char* t = bf16 ? "__bf16" : (dtype == DMF_ATTN_F16 ? "_Float16" : "float");
   const size_t n = (size_t)buflen;
   if (entry == DMF_ATTN_PLAN_BWD) {
     if (!(bf16 && dmf::plan_bwd_bf16_fast(Lq, Lkv, D, B * H, buf, n)))
@@ -151,7 +152,7 @@ int dmf_attn_bwd(const void* dout, const void* q, const void* k, const void* v, 
                  int B, int H, int Lq, int Lkv, int D, float scale, int dtype, void* stream) {
   if (int rc = check_common(B, H, Lq, Lkv, D, dtype)) return rc;
   if (strides == nullptr || lse == nullptr || delta == nullptr) return DMF_ATTN_ENULL;
-  const int eb = dtype == DMF_ATTN_BF16 ? 2 : 4;
+  const int eb = dtype == DMF_ATTN_F32 ? 4 : 2;
   dmf::BwdParams p{};
   const void* ptrs[8] = {dout, q, k, v, o, dq, dk, dv};
   for (int i = 0; i < 8; ++i)
@@ -160,7 +161,7 @@ int dmf_attn_bwd(const void* dout, const void* q, const void* k, const void* v, 
   p.dq = dq; p.dk = dk; p.dv = dv; p.delta = delta;
   p.H = H; p.Lq = Lq; p.Lkv = Lkv;
   p.scale = scale; p.scale_log2 = scale * 1.4426950408889634f;
-  return dmf::launch_bwd(p, B * H, D, dtype == DMF_ATTN_BF16, static_cast<hipStream_t>(stream));
+  return dmf::launch_bwd(p, B * H, D, static_cast<dmf::ElemType>(dtype), static_cast<hipStream_t>(stream));
 }
 
 int64_t dmf_attn_bwd_qknorm_workspace_floats(int B, int H, int Lq, int Lkv, int D) {

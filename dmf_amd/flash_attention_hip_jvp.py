@@ -19,8 +19,6 @@ a second pass of the fused kernel over the saved primals.
 """
 from __future__ import annotations
 
-import warnings
-
 import torch
 import torch.autograd.forward_ad as fwAD
 
@@ -42,10 +40,11 @@ class FlashAttnFunc(torch.autograd.Function):
     def forward(q, k, v, tq, tk, tv, softmax_scale):
         scale = _default_scale(q, softmax_scale)
         enable_jvp = (tq is not None) and (tk is not None) and (tv is not None)
+        half = q.dtype == torch.float16
         if enable_jvp:
-            o, to, lse = _lib.fwd_jvp(q, k, v, tq, tk, tv, scale)
+            o, to, lse = (_lib.fwd_jvp_half if half else _lib.fwd_jvp)(q, k, v, tq, tk, tv, scale)
         else:
-            o, lse = _lib.fwd(q, k, v, scale, need_lse=True)
+            o, lse = (_lib.fwd_half if half else _lib.fwd)(q, k, v, scale, need_lse=True)
             to = None
         return o, lse, to
 
@@ -67,7 +66,7 @@ class FlashAttnFunc(torch.autograd.Function):
         q, k, v, o, lse = ctx.saved_tensors
         if dout is None:
             return None, None, None, None, None, None, None
-        dq, dk, dv = _lib.bwd(dout, q, k, v, o, lse, ctx.softmax_scale)
+        dq, dk, dv = (_lib.bwd_half if q.dtype == torch.float16 else _lib.bwd)(dout, q, k, v, o, lse, ctx.softmax_scale)
         return dq, dk, dv, None, None, None, None
 
     @staticmethod
@@ -82,7 +81,8 @@ class FlashAttnFunc(torch.autograd.Function):
         gq = torch.zeros_like(q) if gq is None else gq
         gk = torch.zeros_like(k) if gk is None else gk
         gv = torch.zeros_like(v) if gv is None else gv
-        _, to, _, dlse = _lib.fwd_jvp(q, k, v, gq, gk, gv, ctx.softmax_scale, need_dlse=True)
+        fwd_jvp = _lib.fwd_jvp_half if _lib._raw(q).dtype == torch.float16 else _lib.fwd_jvp
+        _, to, _, dlse = fwd_jvp(q, k, v, gq, gk, gv, ctx.softmax_scale, need_dlse=True)
         return to, dlse, None
 
 
@@ -97,7 +97,7 @@ def _is_dual_mode(*tensors) -> bool:
 
 @torch.library.custom_op("dmf_amd::attn_fwd", mutates_args=())
 def _attn_fwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> tuple[torch.Tensor, torch.Tensor]:
-    return _lib.fwd(q, k, v, scale, need_lse=True)
+    return (_lib.fwd_half if q.dtype == torch.float16 else _lib.fwd)(q, k, v, scale, need_lse=True)
 
 
 @_attn_fwd_op.register_fake
@@ -109,7 +109,7 @@ def _(q, k, v, scale):
 @torch.library.custom_op("dmf_amd::attn_bwd", mutates_args=())
 def _attn_bwd_op(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor,
                  scale: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    return _lib.bwd(dout, q, k, v, o, lse, scale)
+    return (_lib.bwd_half if q.dtype == torch.float16 else _lib.bwd)(dout, q, k, v, o, lse, scale)
 
 
 @_attn_bwd_op.register_fake
@@ -133,9 +133,6 @@ def _attn_op_backward(ctx, dout, dlse_unused):
 _attn_fwd_op.register_autograd(_attn_op_backward, setup_context=_attn_op_setup)
 
 
-_warned_fp16 = False
-
-
 def _padded_head_dim(d: int) -> int:
     """The kernels' head dim that serves head dim ``d``: itself, or the next larger one."""
     for n in _lib.SUPPORTED_HEAD_DIMS:
@@ -155,16 +152,11 @@ def flash_attn_func(q, k, v, softmax_scale=None):
     and masking, models/triton_utils.py:22-45) are zero-padded to the next one that
     has -- exact, since zero columns add nothing to the scores and give zero output
     columns -- at the price of a padded copy of every operand.  fp16 operands (the
-    reference's ``--mixed-precision fp16`` / ``--dtype fp16``) have no kernels of their
-    own either: they are computed by the fp32 kernels and rounded back to fp16, which
-    is exact to fp16 rounding but an order of magnitude slower than bf16 (warned once).
+    reference's ``--mixed-precision fp16`` / ``--dtype fp16``) have kernels of their own
+    (fp32 accumulation and softmax, nothing rounded to fp16 before the result); with
+    k, v of another type next to an fp16 q everything is computed in fp32 and rounded back.
     """
-    if q.dtype == torch.float16:
-        global _warned_fp16
-        if not _warned_fp16:
-            _warned_fp16 = True
-            warnings.warn("dmf_amd attention: fp16 operands are computed by the fp32 kernels (correct, but about ten times "
-                          "slower than bf16 on this device); use bf16 for speed", stacklevel=2)
+    if q.dtype == torch.float16 and not (k.dtype == v.dtype == torch.float16):
         return flash_attn_func(q.float(), k.float(), v.float(), _default_scale(q, softmax_scale)).to(torch.float16)
     d = q.shape[-1]
     dp = _padded_head_dim(d)
@@ -184,7 +176,7 @@ def flash_attn_func(q, k, v, softmax_scale=None):
         out, _, t_out = _lib.run_function(FlashAttnFunc, *primals, *tangents, softmax_scale)
         return fwAD.make_dual(out, t_out)
     if _lib.plain_inference(q, k, v):
-        return _lib.fwd(q, k, v, _default_scale(q, softmax_scale), need_lse=False)[0]
+        return (_lib.fwd_half if q.dtype == torch.float16 else _lib.fwd)(q, k, v, _default_scale(q, softmax_scale), need_lse=False)[0]
     out, _, _ = _lib.run_function(FlashAttnFunc, q, k, v, None, None, None, softmax_scale)
     return out
 

@@ -20,8 +20,11 @@
  *   - `strides` is a flat int64 array of n_tensors*4 entries in the order the
  *     tensor pointers appear in the signature (outputs included, lse/delta
  *     excluded: those are dense (B, H, Lq) fp32).
- *   - `dtype`: DMF_ATTN_F32 (fp32 in/out, fp32 MFMA products) or
- *     DMF_ATTN_BF16 (bf16 in/out, bf16 MFMA, fp32 accumulation and softmax).
+ *   - `dtype`: DMF_ATTN_F32 (fp32 in/out; products accurate to fp32, formed
+ *     from bf16 MFMAs over operands split into three bf16 parts),
+ *     DMF_ATTN_BF16 (bf16 in/out, bf16 MFMA, fp32 accumulation and softmax)
+ *     or DMF_ATTN_F16 (fp16 in/out, f16 MFMA, probabilities as two f16 parts,
+ *     fp32 accumulation and softmax; not in the q-norm entry points).
  *   - `lse` is the natural-log logsumexp of the scaled scores
  *     (models/triton_utils.py:347).
  *   - Ownership: the caller allocates every buffer; the library neither
@@ -47,11 +50,11 @@
 extern "C" {
 #endif
 
-enum { DMF_ATTN_F32 = 0, DMF_ATTN_BF16 = 1 };
+enum { DMF_ATTN_F32 = 0, DMF_ATTN_BF16 = 1, DMF_ATTN_F16 = 2 };
 
 enum {
   DMF_ATTN_OK = 0,
-  DMF_ATTN_EDTYPE = -1,    /* dtype is not DMF_ATTN_F32 / DMF_ATTN_BF16        */
+  DMF_ATTN_EDTYPE = -1,    /* dtype is not one of DMF_ATTN_F32 / _BF16 / _F16     */
   DMF_ATTN_EHEADDIM = -2,  /* head dim not in the supported set                 */
   DMF_ATTN_ESHAPE = -3,    /* a dimension is < 1 or B*H exceeds the grid limit  */
   DMF_ATTN_ESTRIDE = -4,   /* last-dim stride != 1 or a stride breaks alignment */

@@ -779,3 +779,50 @@ def test_bwd_qknorm_matches_backward_followed_by_the_stand_alone_norm_backward(L
         assert float(d) <= 2 ** -8 * float(ref[:, :, i].float().norm()), (i, float(d))
     for a, r in zip(gains, (rq, rk)):
         assert float((a - r).norm()) <= 1e-5 * float(r.norm()) + 1e-12
+
+
+# Sizes at the edges of the split-operand kernels' 32-row tiles and 128-row work-groups.
+SPLIT_SHAPES = [(1, 1, 64), (31, 33, 72), (128, 129, 32), (97, 64, 80), (257, 200, 72), (130, 300, 96), (65, 40, 128)]
+
+
+def _split_reference(q, k, v, tq, tk, tv, do):
+    d = lambda t: t.detach().double().cpu()
+    q, k, v, tq, tk, tv, do = map(d, (q, k, v, tq, tk, tv, do))
+    o, to = ao.base_attn_jvp(q, k, v, tq, tk, tv)
+    return (o, to, *ao.base_attn_grads(q, k, v, do))
+
+
+@pytest.mark.parametrize("tangent", [1e-5, 1.0, 3e2])
+@pytest.mark.parametrize("Lq,Lkv,D", SPLIT_SHAPES)
+def test_fp16_kernels_round_only_the_result(Lq, Lkv, D, tangent):
+    """fp16 operands against the fp64 oracle on the same values.  Everything before the final store carries at least 20
+    significant bits, so a result is off by its own fp16 rounding: 2^-11 of its value where it is a normal fp16 number, half
+    a subnormal step (2^-25) below, whatever the size of tangents and gradients (1e-5 ... 300; a per-row power of two keeps
+    the products inside the fp16 range)."""
+    g = torch.Generator().manual_seed(Lq * 7 + Lkv + D)
+    rnd = lambda L, s: (torch.randn(2, L, 3, D, generator=g) * s).to(torch.float16).to(DEV)
+    q, k, v = rnd(Lq, 1), rnd(Lkv, 1), rnd(Lkv, 1)
+    tq, tk, tv, do = rnd(Lq, tangent), rnd(Lkv, tangent), rnd(Lkv, tangent), rnd(Lq, tangent)
+    scale = D ** -0.5
+    o, to, lse = _lib.fwd_jvp_half(q, k, v, tq, tk, tv, scale)
+    got = (o, to, *_lib.bwd_half(do, q, k, v, o, lse, scale))
+    o2, _ = _lib.fwd_half(q, k, v, scale)
+    for name, a, r in zip(("o", "to", "dq", "dk", "dv", "o primal-only"), (*got, o2), (*(ref := _split_reference(q, k, v, tq, tk, tv, do)), ref[0])):
+        err, bound = (a.double().cpu() - r).norm(), 2.0 ** -11 * r.norm() + 2.0 ** -25 * r.numel() ** 0.5
+        if name in ("dq", "dk", "dv"):   # delta = rowsum(dout o) takes the rounded o: the same relative size again, on the terms of dS
+            bound = 2 * bound + 2.0 ** -11 * tangent * scale * r.numel() ** 0.5
+        assert a.dtype == torch.float16 and float(err) <= float(bound), (name, float(err), float(bound))
+
+
+@pytest.mark.parametrize("Lq,Lkv,D", SPLIT_SHAPES)
+def test_fp32_kernels_keep_fp32_products(Lq, Lkv, D):
+    """fp32 operands whose magnitudes span 2^20 within a row, against the fp64 oracle: dropping any of the six plane products
+    that the kernels form would show as 2^-16 of the result; fp32 arithmetic leaves a few times 2^-24 sqrt(terms)."""
+    g = torch.Generator().manual_seed(Lq * 5 + Lkv + D)
+    rnd = lambda L: (torch.randn(2, L, 3, D, generator=g) * 2.0 ** torch.randint(-18, 2, (2, L, 3, D), generator=g)).to(DEV)
+    q, k, v, tq, tk, tv, do = rnd(Lq), rnd(Lkv), rnd(Lkv), rnd(Lq), rnd(Lkv), rnd(Lkv), rnd(Lq)
+    scale = D ** -0.5
+    o, to, lse = _lib.fwd_jvp(q, k, v, tq, tk, tv, scale)
+    got = (o, to, *_lib.bwd(do, q, k, v, o, lse, scale))
+    for name, a, r in zip(("o", "to", "dq", "dk", "dv"), got, _split_reference(q, k, v, tq, tk, tv, do)):
+        assert ao.rel_l2(a.double().cpu(), r) <= 4e-6 or float(r.norm()) < 1e-9, (name, ao.rel_l2(a.double().cpu(), r))
