@@ -246,10 +246,11 @@ __device__ __forceinline__ void generic_bwd_dkv_body(const BwdParams& p) {
                               [&](int t, int i) { return dV[t][i]; });
 }
 
-// fp32 and fp16 take the split-operand bodies (attn_split.h); two fp32 rows per lane in three planes plus the accumulators need
-// the register file of one wave per SIMD.
+// fp32 and fp16 take the split-operand bodies (attn_split.h).  From head dim 72 on two fp32 rows per lane in three planes plus the
+// accumulators need the register file of one wave per SIMD; at head dim 64 two waves win although the dK/dV kernel then spills
+// 19 registers (B16 H12 N256: 111 -> 98 us for the pair).
 template <typename T, int D>
-constexpr int bwd_waves_per_simd() { return std::is_same<T, _Float16>::value && D <= 96 ? 2 : 1; }
+constexpr int bwd_waves_per_simd() { return D <= 64 || (std::is_same<T, _Float16>::value && D <= 96) ? 2 : 1; }
 
 template <typename T, int D>
 __global__ __launch_bounds__(256, (bwd_waves_per_simd<T, D>())) void attn_bwd_dq_kernel(const BwdParams p) {

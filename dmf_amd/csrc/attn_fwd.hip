@@ -196,11 +196,13 @@ __device__ __forceinline__ void generic_fwd_body(const FwdParams& p) {
 }
 
 // fp32 and fp16 take the split-operand body (attn_split.h).  Waves per SIMD: with fp32 tangents the operand planes alone are
-// 96 .. 192 registers, so those kernels run one wave per SIMD with the whole register file instead of spilling.
+// 96 .. 192 registers, and with fp16 ones the third accumulator set needs 437 at head dim 72, so those kernels run one wave per
+// SIMD with the whole register file instead of spilling (fp16 with tangents at B8 H16 N1024 D72: 636 us held to 256 registers,
+// 165 of them spilled, 315 us without; fp32 at head dim 64 fits neither way better: 78 us with 47 spills, 80 without).
 template <typename T, int D, bool JVP>
 constexpr int fwd_waves_per_simd() {
   if constexpr (std::is_same<T, float>::value) return JVP || D > 96 ? 1 : 2;
-  return std::is_same<T, _Float16>::value && D <= 96 ? 2 : 1;
+  return std::is_same<T, _Float16>::value && D <= (JVP ? 64 : 96) ? 2 : 1;
 }
 
 template <typename T, int D, bool JVP>
