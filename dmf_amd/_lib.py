@@ -10,6 +10,7 @@ import contextlib
 import ctypes
 import functools
 import os
+import sys
 import warnings
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p, POINTER
 
@@ -80,6 +81,30 @@ def load() -> ctypes.CDLL:
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+_host_module = None
+
+
+def host():
+    """The native host path (dmf_amd/_host*.so, built together with the kernel library): each function does a whole operator
+    call -- forward-AD duals, one torch.func.jvp level, autograd node, launch -- or returns None where the general route
+    below has to be taken."""
+    global _host_module
+    if _host_module is None:
+        load()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError("dmf_amd/_host*.so is missing or does not fit the installed torch: build it with `python -m dmf_amd.build`") from e
+        _host.bind(sys.modules[__name__])
+        _host_module = _host
+    return _host_module
+
+
+def native(t) -> bool:
+    """True where an operator call on ``t`` may try the native host path: a GPU tensor outside of torch.compile's tracing."""
+    return t.is_cuda and not torch.compiler.is_compiling()
 
 
 def _check(rc: int, what: str) -> None:

@@ -289,6 +289,10 @@ def dual_linear(x, weight, bias=None, w_lp=None, b_lp=None):
     (weight and bias are constants of the tangent map).  ``w_lp`` / ``b_lp``: optional
     copies of the parameters in the autocast dtype, used instead of casting per call
     (the caller guarantees they are current)."""
+    if _lib.native(x):
+        out = _lib.host().linear(x, weight, bias, w_lp, b_lp)
+        if out is not None:
+            return out
     (xp,), (tx,), dual = _unpack(x)
     y, ty, _ = _lib.run_function(DualLinearFunc, xp, tx, weight, bias, w_lp, b_lp)
     return fwAD.make_dual(y, ty) if dual else y
@@ -300,6 +304,10 @@ def linear_gelu_tanh(x, weight, bias, w_lp=None, b_lp=None):
     the activation rides in the GEMM's epilogue (one library call, the pre-activation
     never reaches HBM); otherwise the pre-activation is needed for the tangent and for
     the backward pass and this is ``dual_linear`` followed by ``gelu_tanh``."""
+    if bias is not None and not torch.is_grad_enabled() and _lib.native(x):
+        out = _lib.host().linear_gelu_inference(x, weight, bias, w_lp, b_lp)
+        if out is not None:
+            return out
     if torch.is_grad_enabled() or bias is None or not x.is_cuda or fwAD.unpack_dual(x).tangent is not None:
         return gelu_tanh(dual_linear(x, weight, bias, w_lp, b_lp))
     dt = _autocast_dtype(x)
@@ -321,6 +329,10 @@ def ln_modulate(x, shift, scale, eps: float = 1e-6):
     (B, C) or (B, 1, C); LayerNorm over C without affine parameters.  Under
     autocast the result is produced directly in the autocast dtype (it only ever
     feeds a Linear, which would cast it)."""
+    if _lib.native(x):
+        out = _lib.host().ln_modulate(x, shift, scale, eps)
+        if out is not None:
+            return out
     (xp, shp, scp), (tx, tsh, tsc), dual = _unpack(x, shift, scale)
     y, ty = _lib.run_function(LNModulateFunc, xp, shp, scp, tx, tsh, tsc, eps, _autocast_dtype(xp), dual)
     return fwAD.make_dual(y, ty) if dual else y
@@ -329,6 +341,10 @@ def ln_modulate(x, shift, scale, eps: float = 1e-6):
 def gate_residual(x, gate, h):
     """``x + gate * h`` for x, h (B, L, C) and gate (B, C) or (B, 1, C); the result
     has the promoted dtype of x and h (the fp32 residual stream under autocast)."""
+    if _lib.native(x):
+        out = _lib.host().gate_residual(x, gate, h)
+        if out is not None:
+            return out
     (xp, gp, hp), (tx, tg, th), dual = _unpack(x, gate, h)
     dt = torch.promote_types(xp.dtype, hp.dtype)
     if xp.dtype != dt:
@@ -340,6 +356,10 @@ def gate_residual(x, gate, h):
 def residual_ln_modulate(x, gate, h, shift, scale, eps: float = 1e-6):
     """``y = x + gate * h`` and ``z = LayerNorm(y) * (1 + scale) + shift`` in one pass;
     returns ``(y, z)`` with the dtypes ``gate_residual`` and ``ln_modulate`` would give."""
+    if _lib.native(x):
+        out = _lib.host().residual_ln_modulate(x, gate, h, shift, scale, eps)
+        if out is not None:
+            return out
     (xp, gp, hp, shp, scp), (tx, tg, th, tsh, tsc), dual = _unpack(x, gate, h, shift, scale)
     dt = torch.promote_types(xp.dtype, hp.dtype)
     if xp.dtype != dt:
@@ -350,6 +370,10 @@ def residual_ln_modulate(x, gate, h, shift, scale, eps: float = 1e-6):
 
 def gelu_tanh(x):
     """tanh-approximated GELU."""
+    if _lib.native(x):
+        out = _lib.host().gelu_tanh(x)
+        if out is not None:
+            return out
     (xp,), (tx,), dual = _unpack(x)
     y, ty = _lib.run_function(GeluTanhFunc, xp, tx)
     return fwAD.make_dual(y, ty) if dual else y
@@ -358,6 +382,10 @@ def gelu_tanh(x):
 def silu(x):
     """``x * sigmoid(x)``; under autocast the result is produced in the autocast
     dtype (it feeds the adaLN projection, which would cast it)."""
+    if _lib.native(x):
+        out = _lib.host().silu(x)
+        if out is not None:
+            return out
     (xp,), (tx,), dual = _unpack(x)
     y, ty = _lib.run_function(SiluFunc, xp, tx, _autocast_dtype(xp))
     return fwAD.make_dual(y, ty) if dual else y
@@ -370,3 +398,12 @@ def rms_norm(x, gain, eps: float = 1e-6):
     (xp,), (tx,), dual = _unpack(x)
     y, ty = _lib.run_function(RMSNormFunc, xp, gain, tx, eps, dual)
     return fwAD.make_dual(y, ty) if dual else y
+
+
+def chunk_last(x, n: int):
+    """``x.chunk(n, dim=-1)`` for a modulation tensor whose width ``n`` divides."""
+    if _lib.native(x):
+        out = _lib.host().chunk_last(x, n)
+        if out is not None:
+            return out
+    return x.chunk(n, dim=-1)

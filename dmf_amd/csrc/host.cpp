@@ -1,0 +1,906 @@
+// Native host path of the operators: what the Python wrappers of this package did around a kernel launch -- unpack forward-AD
+// duals, check operands, allocate outputs, launch, build the autograd node, re-pack the dual -- in C++.
+//
+// Why: a fused operator call costs a few microseconds of GPU work at the sizes of one model layer, and Python's share of it
+// (custom autograd.Function, functorch's dispatch of make_dual / unpack_dual, ctypes) was 16 us for the plainest call and about
+// 100 us for a differentiated one, so eager steps and small calls were paced by the host.
+//
+// How forward-mode AD is handled: under torch.autograd.forward_ad a tangent hangs on the tensor itself; under one torch.func.jvp
+// level it hangs on the level's wrapper tensor.  In both cases it is read here without dispatching anything, the kernels
+// receive primals and tangents as plain buffers, the autograd node (a KernelNode over the primal's variables) is built below the
+// level exactly like a built-in operator's, and the outputs are wrapped for the level and given their tangents.  Everything
+// else -- several levels, vmap, torch.func.grad, tensor subclasses, CPU tensors, operands a kernel cannot read in place --
+// returns None, and the caller takes the general Python route.
+//
+// The kernels are reached through the C ABI of libdmf_attn.so, which this module links against.
+#include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+#include <torch/extension.h>
+
+#include <ATen/autocast_mode.h>
+#include <ATen/functorch/DynamicLayer.h>
+#include <ATen/functorch/TensorWrapper.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/Event.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
+#include <c10/hip/HIPStream.h>
+
+#include <functional>
+
+#include "../../include/dmf_attn.h"
+#include "../../include/dmf_block.h"
+#include "../../include/dmf_fused.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::edge_list;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+void check(int rc, const char* what) {
+  TORCH_CHECK(rc == 0, what, " failed: ", dmf_attn_strerror(rc), " (code ", rc, ")");
+}
+
+// ---- dispatch state ------------------------------------------------------------------------------------------------------
+
+// Below autograd, autocast and functorch: at:: calls go straight to their device kernels.
+struct Below {
+  c10::impl::ExcludeDispatchKeyGuard functorch{c10::DispatchKeySet(
+      {c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchDynamicLayerBackMode})};
+  c10::impl::ExcludeDispatchKeyGuard autocast{c10::autocast_dispatch_keyset};
+  at::AutoDispatchBelowADInplaceOrView autograd;
+};
+
+constexpr int64_t kNoLevel = -1, kUnsupported = -2;
+
+// The one torch.func.jvp level that is active, kNoLevel, or kUnsupported.
+int64_t current_level() {
+  const auto& stack = at::functorch::getDynamicLayerStack();
+  if (stack.empty()) return kNoLevel;
+  if (stack.size() == 1 && stack[0].key() == at::functorch::TransformType::Jvp) return stack[0].layerId();
+  return kUnsupported;
+}
+
+Tensor unwrap(Tensor t) {
+  while (t.defined() && t.key_set().has(c10::DispatchKey::FuncTorchGradWrapper)) {
+    auto* w = at::functorch::maybeGetTensorWrapper(t);
+    if (w == nullptr) break;
+    t = w->value();
+  }
+  return t;
+}
+
+// The buffer of a variable: same storage and version counter, no autograd metadata.
+Tensor data_of(const Tensor& v) { return v.defined() ? Tensor(v.tensor_data()) : v; }
+
+struct Arg {
+  Tensor var;    // the variable below the level: its gradient edge
+  Tensor data;   // its buffer
+  Tensor tan;    // tangent buffer or undefined
+  bool defined() const { return data.defined(); }
+  bool grad() const { return var.defined() && var.requires_grad(); }
+};
+
+Arg unpack(const Tensor& x) {
+  Arg a;
+  if (!x.defined()) return a;
+  const Tensor& t = x._fw_grad(0);
+  if (t.defined()) a.tan = data_of(unwrap(t));
+  a.var = unwrap(x);
+  a.data = data_of(a.var);
+  return a;
+}
+Arg unpack(const OptTensor& x) { return x.has_value() ? unpack(*x) : Arg{}; }
+
+bool plain_gpu(const Arg& a) {
+  return a.data.is_cuda() && a.data.layout() == at::kStrided && !a.data.key_set().has(c10::DispatchKey::Python) &&
+         (!a.tan.defined() || (a.tan.is_cuda() && a.tan.scalar_type() == a.data.scalar_type() && a.tan.sizes() == a.data.sizes()));
+}
+
+template <typename... A>
+bool any_grad(const A&... a) {
+  return c10::GradMode::is_enabled() && (a.grad() || ...);
+}
+
+int code_of(const Tensor& t) {   // -1: none
+  switch (t.scalar_type()) {
+    case at::kFloat: return DMF_ATTN_F32;
+    case at::kBFloat16: return DMF_ATTN_BF16;
+    case at::kHalf: return DMF_ATTN_F16;
+    default: return -1;
+  }
+}
+bool block_dtype(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+const void* ptr(const Tensor& t) { return t.defined() ? t.const_data_ptr() : nullptr; }
+void* mptr(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
+
+Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, const Tensor& like) {
+  return Tensor(at::detail::empty_cuda(sizes, dt, like.device(), std::nullopt));
+}
+Tensor dense_like(const Tensor& t) { return empty(t.sizes(), t.scalar_type(), t); }
+Tensor workspace(int64_t floats, const Tensor& like) { return empty({std::max<int64_t>(floats, 1)}, at::kFloat, like); }
+Tensor dense(const Tensor& t) { return !t.defined() || t.is_contiguous() ? t : t.contiguous(); }
+
+at::ScalarType autocast_type(const Tensor& x) {
+  return at::autocast::is_autocast_enabled(at::kCUDA) ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
+}
+
+// ---- autograd ------------------------------------------------------------------------------------------------------------
+
+// One operator call in the graph: saved tensors and a function (saved, output gradients, node) -> input gradients.
+struct KernelNode : Node {
+  using Fn = std::function<variable_list(KernelNode&, const std::vector<Tensor>&, const variable_list&)>;
+  const char* label;
+  std::vector<SavedVariable> saved;
+  Fn fn;
+  bool released = false;
+
+  explicit KernelNode(const char* l) : label(l) {}
+  std::string name() const override { return label; }
+  bool wants(size_t i) { return task_should_compute_output(i); }
+  variable_list apply(variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    TORCH_CHECK(!released, torch::autograd::ERR_BACKWARD_TWICE);
+    std::vector<Tensor> s;
+    s.reserve(saved.size());
+    for (auto& v : saved) s.push_back(v.unpack(shared_from_this()));
+    const size_t n = num_outputs();
+    bool any = false;
+    for (const auto& g : grads) any = any || g.defined();
+    if (!any) return variable_list(n);
+    c10::OptionalDeviceGuard device(s[0].device());
+    Below below;
+    variable_list out = fn(*this, s, grads);
+    out.resize(n);
+    return out;
+  }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto& v : saved) v.reset_data();
+    released = true;
+  }
+};
+
+std::shared_ptr<KernelNode> make_node(const char* name, std::initializer_list<Arg> inputs, std::initializer_list<Tensor> save) {
+  std::shared_ptr<KernelNode> node(new KernelNode(name), torch::autograd::deleteNode);
+  edge_list edges;
+  edges.reserve(inputs.size());
+  for (const Arg& a : inputs) edges.push_back(a.grad() ? torch::autograd::impl::gradient_edge(a.var) : torch::autograd::Edge());
+  node->set_next_edges(std::move(edges));
+  node->saved.reserve(save.size());
+  for (const Tensor& t : save) node->saved.emplace_back(t, false);
+  return node;
+}
+
+// Output for the caller: history, level wrapper, tangent.
+Tensor finish(Tensor out, const Tensor& tan, const std::shared_ptr<KernelNode>& node, int64_t level) {
+  if (node) torch::autograd::set_history(out, node);
+  Tensor res = level >= 0 ? at::functorch::makeTensorWrapper(out, level) : out;
+  if (tan.defined()) {
+    auto* meta = torch::autograd::impl::materialize_autograd_meta(res);
+    meta->fw_grad_ = std::make_shared<torch::autograd::ForwardGrad>();
+    meta->fw_grad_->set_value(level >= 0 ? at::functorch::makeTensorWrapper(tan, level) : tan, 0);
+  }
+  return res;
+}
+
+// The functions below run with the GIL held; what they call back into Python for is rare.
+py::handle g_lib;   // dmf_amd._lib
+
+// Operands the kernels cannot read in place are copied, counted and warned about by dmf_amd._lib._prep.
+Tensor prep_counted(const Tensor& t) {
+  py::gil_scoped_acquire gil;
+  return g_lib.attr("_prep")(t).cast<Tensor>();
+}
+
+// ---- (B, L, H, D) operands -----------------------------------------------------------------------------------------------
+
+bool readable(const Tensor& t) {   // unit last-dim stride, 16-byte aligned rows
+  const int64_t eb = t.element_size();
+  const auto st = t.strides();
+  if (st.back() != 1 || reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16) return false;
+  for (size_t i = 0; i + 1 < st.size(); ++i)
+    if ((st[i] * eb) % 16) return false;
+  return true;
+}
+Tensor prepared(const Tensor& t) { return readable(t) ? t : prep_counted(t); }
+
+// A tensor's address and strides, or those of one of the three slots of a packed (B, L, 3, H, D) one.
+struct Operand {
+  const void* p = nullptr;
+  int64_t st[4] = {0, 0, 0, 1};
+  Operand() = default;
+  explicit Operand(const Tensor& t) : p(t.const_data_ptr()) {
+    for (int i = 0; i < 4; ++i) st[i] = t.stride(i);
+  }
+  Operand(const Tensor& packed, int slot)
+      : p(static_cast<const char*>(packed.const_data_ptr()) + slot * packed.stride(2) * packed.element_size()),
+        st{packed.stride(0), packed.stride(1), packed.stride(3), 1} {}
+};
+
+struct Strides {
+  std::vector<int64_t> v;
+  Strides(std::initializer_list<const Operand*> ops) {
+    v.reserve(4 * ops.size());
+    for (const Operand* o : ops) v.insert(v.end(), o->st, o->st + 4);
+  }
+  const int64_t* data() const { return v.data(); }
+};
+
+bool head_dim_ok(int64_t d) { return d == 32 || d == 64 || d == 72 || d == 80 || d == 96 || d == 128; }
+
+struct AttnShape {
+  int B, H, Lq, Lkv, D, code;
+  float scale;
+};
+
+struct QKV {
+  Operand q, k, v;
+};
+
+// o [, to], lse of one call; `tan` null: primal only, without lse unless asked for.
+struct AttnOut {
+  Tensor o, to, lse;
+};
+AttnOut attn_forward(const AttnShape& s, const QKV& x, const QKV* tan, bool need_lse, const Tensor& like) {
+  AttnOut r;
+  r.o = empty({s.B, s.Lq, s.H, s.D}, like.scalar_type(), like);
+  if (tan) r.to = empty({s.B, s.Lq, s.H, s.D}, like.scalar_type(), like);
+  if (tan || need_lse) r.lse = empty({s.B, s.H, s.Lq}, at::kFloat, like);
+  const Operand oo(r.o);
+  if (tan) {
+    const Operand oto(r.to);
+    const Strides st{&x.q, &x.k, &x.v, &tan->q, &tan->k, &tan->v, &oo, &oto};
+    check(dmf_attn_fwd_jvp(x.q.p, x.k.p, x.v.p, tan->q.p, tan->k.p, tan->v.p, mptr(r.o), mptr(r.to), static_cast<float*>(mptr(r.lse)), nullptr,
+                           st.data(), s.B, s.H, s.Lq, s.Lkv, s.D, s.scale, s.code, stream_of(like)),
+          "dmf_attn_fwd_jvp");
+  } else {
+    const Strides st{&x.q, &x.k, &x.v, &oo};
+    check(dmf_attn_fwd(x.q.p, x.k.p, x.v.p, mptr(r.o), static_cast<float*>(mptr(r.lse)), st.data(), s.B, s.H, s.Lq, s.Lkv, s.D, s.scale,
+                       s.code, stream_of(like)),
+          "dmf_attn_fwd");
+  }
+  return r;
+}
+
+void attn_backward(const AttnShape& s, const Tensor& dout, const QKV& x, const Tensor& o, const Tensor& lse, const QKV& grad) {
+  const Tensor delta = empty({s.B, s.H, s.Lq}, at::kFloat, o);
+  const Operand od(dout), oo(o);
+  const Strides st{&od, &x.q, &x.k, &x.v, &oo, &grad.q, &grad.k, &grad.v};
+  check(dmf_attn_bwd(od.p, x.q.p, x.k.p, x.v.p, oo.p, static_cast<const float*>(ptr(lse)), const_cast<void*>(grad.q.p), const_cast<void*>(grad.k.p),
+                     const_cast<void*>(grad.v.p), static_cast<float*>(mptr(delta)), st.data(), s.B, s.H, s.Lq, s.Lkv, s.D, s.scale, s.code,
+                     stream_of(o)),
+        "dmf_attn_bwd");
+}
+
+py::object none() { return py::none(); }
+
+// flash_attn_func
+py::object attention(const Tensor& q_, const Tensor& k_, const Tensor& v_, std::optional<double> scale) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg q = unpack(q_), k = unpack(k_), v = unpack(v_);
+  if (!plain_gpu(q) || !plain_gpu(k) || !plain_gpu(v) || q.data.dim() != 4 || k.data.dim() != 4 || v.data.dim() != 4) return none();
+  const int code = code_of(q.data);
+  const int64_t D = q.data.size(3);
+  if (code < 0 || code_of(k.data) != code || code_of(v.data) != code || !head_dim_ok(D) || k.data.sizes() != v.data.sizes() ||
+      k.data.size(3) != D || k.data.size(2) != q.data.size(2) || k.data.size(0) != q.data.size(0) || q.data.numel() == 0 ||
+      k.data.numel() == 0 || k.data.device() != q.data.device() || v.data.device() != q.data.device())
+    return none();
+  for (const Arg* a : {&q, &k, &v})
+    if (!readable(a->data) || (a->tan.defined() && !readable(a->tan))) return none();
+  c10::OptionalDeviceGuard device(q.data.device());
+  AttnShape s{(int)q.data.size(0), (int)q.data.size(2), (int)q.data.size(1), (int)k.data.size(1), (int)D, code,
+              (float)(scale ? *scale : 1.0 / std::sqrt((double)D))};
+  const bool dual = q.tan.defined() || k.tan.defined() || v.tan.defined(), grad = any_grad(q, k, v);
+  AttnOut r;
+  {
+    Below below;
+    const QKV x{Operand(q.data), Operand(k.data), Operand(v.data)};
+    if (dual) {
+      auto tangent = [](const Arg& a) { return a.tan.defined() ? a.tan : at::zeros_like(a.data, at::MemoryFormat::Contiguous); };
+      const Tensor tq = tangent(q), tk = tangent(k), tv = tangent(v);
+      const QKV t{Operand(tq), Operand(tk), Operand(tv)};
+      r = attn_forward(s, x, &t, true, q.data);
+    } else {
+      r = attn_forward(s, x, nullptr, grad, q.data);
+    }
+  }
+  std::shared_ptr<KernelNode> node;
+  if (grad) {
+    node = make_node("FlashAttnBackward", {q, k, v}, {q.data, k.data, v.data, data_of(r.o), r.lse});
+    node->fn = [s](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      const Tensor dout = prepared(g[0]);
+      variable_list out{dense_like(sv[0]), dense_like(sv[1]), dense_like(sv[2])};
+      attn_backward(s, dout, {Operand(sv[0]), Operand(sv[1]), Operand(sv[2])}, sv[3], sv[4], {Operand(out[0]), Operand(out[1]), Operand(out[2])});
+      return out;
+    };
+  }
+  return py::cast(finish(r.o, r.to, node, level));
+}
+
+// A packed projection output: (B, L, 3, H, D), or (B, L, 3 H D) with the head count given (the result is then (B, L, H D)).
+struct Packed {
+  Arg a;
+  Tensor qkv, tan;   // 5-d views
+  bool flat = false;
+  AttnShape s{};
+};
+bool unpack_packed(const Tensor& x, int64_t heads, Packed& p) {
+  p.a = unpack(x);
+  if (!plain_gpu(p.a)) return false;
+  p.qkv = p.a.data;
+  p.tan = p.a.tan;
+  p.flat = heads > 0;
+  if (p.flat) {
+    if (p.qkv.dim() != 3 || p.qkv.size(2) % (3 * heads)) return false;
+    Below below;
+    const std::array<int64_t, 5> sz{p.qkv.size(0), p.qkv.size(1), 3, heads, p.qkv.size(2) / (3 * heads)};
+    if (p.qkv.stride(2) != 1 || (p.tan.defined() && p.tan.stride(2) != 1)) return false;
+    p.qkv = p.qkv.view(sz);
+    if (p.tan.defined()) p.tan = p.tan.view(sz);
+  }
+  if (p.qkv.dim() != 5 || p.qkv.size(2) != 3 || p.qkv.numel() == 0) return false;
+  const int code = code_of(p.qkv);
+  if ((code != DMF_ATTN_F32 && code != DMF_ATTN_BF16) || !head_dim_ok(p.qkv.size(4))) return false;
+  if (!readable(p.qkv) || (p.tan.defined() && !readable(p.tan))) return false;
+  p.s = AttnShape{(int)p.qkv.size(0), (int)p.qkv.size(3), (int)p.qkv.size(1), (int)p.qkv.size(1), (int)p.qkv.size(4), code, 0.f};
+  return true;
+}
+QKV slots(const Tensor& t) { return {Operand(t, 0), Operand(t, 1), Operand(t, 2)}; }
+
+Tensor flat_view(const Tensor& o, bool flat) {   // (B, L, H, D) -> (B, L, H D)
+  return flat && o.defined() ? o.view({o.size(0), o.size(1), o.size(2) * o.size(3)}) : o;
+}
+
+Tensor heads_of(const Tensor& dout, const AttnShape& s) {   // the gradient of the (possibly flat) output as (B, L, H, D)
+  return prepared(dout.dim() == 4 ? dout : dout.reshape({s.B, s.Lq, s.H, s.D}));
+}
+
+// flash_attn_qkvpacked_func
+py::object attention_packed(const Tensor& qkv, int64_t heads, std::optional<double> scale) {
+  const int64_t level = current_level();
+  Packed p;
+  if (level == kUnsupported || !unpack_packed(qkv, heads, p)) return none();
+  c10::OptionalDeviceGuard device(p.qkv.device());
+  p.s.scale = (float)(scale ? *scale : 1.0 / std::sqrt((double)p.s.D));
+  const bool grad = any_grad(p.a);
+  AttnOut r;
+  {
+    Below below;
+    const QKV x = slots(p.qkv);
+    if (p.tan.defined()) {
+      const QKV t = slots(p.tan);
+      r = attn_forward(p.s, x, &t, true, p.qkv);
+    } else {
+      r = attn_forward(p.s, x, nullptr, grad, p.qkv);
+    }
+    r.o = flat_view(r.o, p.flat);
+    r.to = flat_view(r.to, p.flat);
+  }
+  std::shared_ptr<KernelNode> node;
+  if (grad) {
+    node = make_node("FlashAttnQKVPackedBackward", {p.a}, {p.qkv, data_of(r.o), r.lse});
+    node->fn = [s = p.s, shape = p.a.data.sizes().vec()](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      const Tensor dout = heads_of(g[0], s), o = sv[1].view({s.B, s.Lq, s.H, s.D});
+      const Tensor gqkv = empty({s.B, s.Lq, 3, s.H, s.D}, sv[0].scalar_type(), sv[0]);
+      attn_backward(s, dout, slots(sv[0]), o, sv[2], slots(gqkv));
+      return {gqkv.view(shape)};
+    };
+  }
+  return py::cast(finish(r.o, r.to, node, level));
+}
+
+// flash_attn_qknorm_qkvpacked_func where a tuned kernel normalises in place (bf16); k_max_len: longest sequence whose keys are
+// normalised inside the kernel.
+py::object attention_qknorm_packed(const Tensor& qkv, const Tensor& qg_, const Tensor& kg_, int64_t heads, double eps, std::optional<double> scale,
+                                   int64_t k_max_len) {
+  const int64_t level = current_level();
+  Packed p;
+  if (level == kUnsupported || !unpack_packed(qkv, heads, p)) return none();
+  const Arg qg = unpack(qg_), kg = unpack(kg_);
+  const int D = p.s.D;
+  // (rows 2 GiB apart have no tuned kernel)
+  if (p.s.code != DMF_ATTN_BF16 || D == 32 || p.qkv.stride(1) * 2 * (int64_t)(p.s.Lq + 256) >= (int64_t)1 << 31 ||
+      (p.tan.defined() && p.tan.stride(1) * 2 * (int64_t)(p.s.Lq + 256) >= (int64_t)1 << 31))
+    return none();
+  for (const Arg* g : {&qg, &kg})
+    if (!plain_gpu(*g) || g->tan.defined() || g->data.dim() != 1 || g->data.size(0) != D || !block_dtype(g->data) || g->data.device() != p.qkv.device())
+      return none();
+  c10::OptionalDeviceGuard device(p.qkv.device());
+  p.s.scale = (float)(scale ? *scale : 1.0 / std::sqrt((double)D));
+  const AttnShape& s = p.s;
+  const bool grad = any_grad(p.a, qg, kg), dual = p.tan.defined();
+  AttnOut r;
+  Tensor qh, kh, tkh, gq, gk;
+  {
+    Below below;
+    gq = dense(qg.data.to(at::kFloat));
+    gk = dense(kg.data.to(at::kFloat));
+    if (reinterpret_cast<uintptr_t>(gq.const_data_ptr()) % 16 || reinterpret_cast<uintptr_t>(gk.const_data_ptr()) % 16) return none();
+    QKV x = slots(p.qkv), t;
+    if (dual) t = slots(p.tan);
+    const bool k_inside = s.Lq <= k_max_len;
+    if (!k_inside) {
+      const py::tuple n = g_lib.attr("rmsnorm_fwd")(p.qkv.select(2, 1), kg.data, dual ? py::cast(p.tan.select(2, 1)) : none(), eps, dual);
+      kh = n[0].cast<Tensor>();
+      if (dual) tkh = n[1].cast<Tensor>();
+      x.k = Operand(kh);
+      if (dual) t.k = Operand(tkh);
+    } else if (grad) {
+      kh = empty({s.B, s.Lkv, s.H, D}, p.qkv.scalar_type(), p.qkv);
+    }
+    if (grad) qh = empty({s.B, s.Lq, s.H, D}, p.qkv.scalar_type(), p.qkv);
+    r.o = empty({s.B, s.Lq, s.H, D}, p.qkv.scalar_type(), p.qkv);
+    if (dual) r.to = empty({s.B, s.Lq, s.H, D}, p.qkv.scalar_type(), p.qkv);
+    if (dual || grad) r.lse = empty({s.B, s.H, s.Lq}, at::kFloat, p.qkv);
+    const Operand oo(r.o), oto(dual ? r.to : r.o);
+    const QKV& tt = dual ? t : x;
+    const Strides st{&x.q, &x.k, &x.v, &tt.q, &tt.k, &tt.v, &oo, &oto};
+    check(dmf_attn_fwd_qknorm(x.q.p, x.k.p, x.v.p, dual ? t.q.p : nullptr, dual ? t.k.p : nullptr, dual ? t.v.p : nullptr,
+                              static_cast<const float*>(ptr(gq)), k_inside ? static_cast<const float*>(ptr(gk)) : nullptr, (float)eps, mptr(r.o),
+                              mptr(r.to), static_cast<float*>(mptr(r.lse)), nullptr, mptr(qh), k_inside ? mptr(kh) : nullptr, st.data(), s.B, s.H,
+                              s.Lq, s.Lkv, D, s.scale, s.code, stream_of(p.qkv)),
+          "dmf_attn_fwd_qknorm");
+    r.o = flat_view(r.o, p.flat);
+    r.to = flat_view(r.to, p.flat);
+  }
+  std::shared_ptr<KernelNode> node;
+  if (grad) {
+    node = make_node("QKNormAttnQKVPackedBackward", {p.a, qg, kg}, {p.qkv, gq, gk, qh, kh, data_of(r.o), r.lse});
+    node->fn = [s, eps, shape = p.a.data.sizes().vec(), tq = qg.data.scalar_type(), tk = kg.data.scalar_type()](
+                   KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      const Tensor dout = heads_of(g[0], s), o = sv[5].view({s.B, s.Lq, s.H, s.D});
+      const Tensor gqkv = empty({s.B, s.Lq, 3, s.H, s.D}, sv[0].scalar_type(), sv[0]);
+      const Tensor dgq = empty({s.D}, at::kFloat, o), dgk = empty({s.D}, at::kFloat, o), delta = empty({s.B, s.H, s.Lq}, at::kFloat, o);
+      const Tensor ws = workspace(dmf_attn_bwd_qknorm_workspace_floats(s.B, s.H, s.Lq, s.Lkv, s.D), o);
+      const QKV raw = slots(sv[0]), grad = slots(gqkv);
+      const Operand od(dout), oqh(sv[3]), okh(sv[4]), oo(o);
+      const Strides st{&od, &oqh, &okh, &raw.v, &oo, &grad.q, &grad.k, &grad.v, &raw.q, &raw.k};
+      check(dmf_attn_bwd_qknorm(od.p, oqh.p, okh.p, raw.v.p, oo.p, static_cast<const float*>(ptr(sv[6])), raw.q.p, raw.k.p,
+                                static_cast<const float*>(ptr(sv[1])), static_cast<const float*>(ptr(sv[2])), (float)eps,
+                                const_cast<void*>(grad.q.p), const_cast<void*>(grad.k.p), const_cast<void*>(grad.v.p),
+                                static_cast<float*>(mptr(dgq)), static_cast<float*>(mptr(dgk)), static_cast<float*>(mptr(delta)),
+                                static_cast<float*>(mptr(ws)), st.data(), s.B, s.H, s.Lq, s.Lkv, s.D, s.scale, s.code, stream_of(o)),
+            "dmf_attn_bwd_qknorm");
+      return {gqkv.view(shape), dgq.to(tq), dgk.to(tk)};
+    };
+  }
+  return py::cast(finish(r.o, r.to, node, level));
+}
+
+// ---- block glue ----------------------------------------------------------------------------------------------------------
+
+// A (B, C) / (B, 1, C) modulation operand; its tangent if any.  Chunks of a wider adaLN output are read in place.
+struct Mod {
+  Tensor t, tan;
+  int64_t st = 0, tst = 0;
+};
+bool mod_shape_ok(const Arg& a, int64_t B, int64_t C) {
+  return a.data.numel() == B * C && a.data.dim() >= 2 && a.data.size(0) == B && a.data.size(-1) == C && block_dtype(a.data);
+}
+void mod_operand(const Tensor& x, int64_t B, int64_t C, Tensor& t, int64_t& st) {
+  if (!x.defined()) return;
+  t = x;
+  const int64_t eb = t.element_size();
+  if (t.stride(-1) != 1 || reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 || (t.stride(0) * eb) % 16) t = t.contiguous();
+  st = B > 1 ? t.stride(0) : C;
+}
+Mod mod(const Arg& a, int64_t B, int64_t C) {
+  Mod m;
+  mod_operand(a.data, B, C, m.t, m.st);
+  mod_operand(a.tan, B, C, m.tan, m.tst);
+  return m;
+}
+
+bool blc_ok(const Arg& x) {
+  return plain_gpu(x) && x.data.dim() == 3 && block_dtype(x.data) && x.data.size(2) % 8 == 0 && x.data.size(2) <= 2048 && x.data.numel() > 0;
+}
+template <typename... A>
+bool mods_ok(int64_t B, int64_t C, const Arg& first, const A&... rest) {
+  auto ok = [&](const Arg& a) { return plain_gpu(a) && mod_shape_ok(a, B, C) && a.data.scalar_type() == first.data.scalar_type() && a.data.device() == first.data.device(); };
+  return ok(first) && (ok(rest) && ...);
+}
+
+struct Blc {
+  int B, L, C;
+  explicit Blc(const Tensor& t) : B((int)t.size(0)), L((int)t.size(1)), C((int)t.size(2)) {}
+};
+
+// gx, gshift, gscale of LayerNorm + modulate
+variable_list ln_backward(const Tensor& gy_, const Tensor& x, const Tensor& scale_, float eps, const Tensor& gres) {
+  const Blc n(x);
+  const Tensor gy = dense(gy_), res = dense(gres);
+  Tensor scale;
+  int64_t ss = 0;
+  mod_operand(scale_, n.B, n.C, scale, ss);
+  const Tensor gx = dense_like(x), gsh = empty({n.B, n.C}, scale.scalar_type(), x), gsc = empty({n.B, n.C}, scale.scalar_type(), x);
+  const Tensor ws = workspace(dmf_block_workspace_floats(0, n.B, n.L, n.C), x);
+  check(dmf_ln_modulate_bwd(ptr(gy), ptr(x), ptr(scale), ptr(res), mptr(gx), mptr(gsh), mptr(gsc), static_cast<float*>(mptr(ws)), ss, n.B, n.L, n.C,
+                            eps, code_of(x), code_of(scale), code_of(gy), stream_of(x)),
+        "dmf_ln_modulate_bwd");
+  return {gx, gsh, gsc};
+}
+// gh, ggate of the gated residual
+variable_list gate_backward(const Tensor& gy_, const Tensor& gate_, const Tensor& h) {
+  const Blc n(h);
+  const Tensor gy = dense(gy_);
+  Tensor gate;
+  int64_t gs = 0;
+  mod_operand(gate_, n.B, n.C, gate, gs);
+  const Tensor gh = dense_like(h), gg = empty({n.B, n.C}, gate.scalar_type(), h);
+  const Tensor ws = workspace(dmf_block_workspace_floats(1, n.B, n.L, n.C), h);
+  check(dmf_gate_residual_bwd(ptr(gy), ptr(gate), ptr(h), mptr(gh), mptr(gg), static_cast<float*>(mptr(ws)), gs, n.B, n.L, n.C, code_of(gy),
+                              code_of(gate), code_of(h), stream_of(h)),
+        "dmf_gate_residual_bwd");
+  return {gh, gg};
+}
+
+[[noreturn]] void tangent_cotangent() {
+  C10_THROW_ERROR(NotImplementedError,
+                  "dmf_amd.block_ops: a gradient arrived at the tangent (JVP) output of a fused block operator; these operators back-propagate "
+                  "through the primal output only -- detach the JVP output (as DMFLoss does) or build the model with block_ops='torch'");
+}
+
+py::object ln_modulate(const Tensor& x_, const Tensor& shift_, const Tensor& scale_, double eps) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg x = unpack(x_), sh = unpack(shift_), sc = unpack(scale_);
+  if (!blc_ok(x)) return none();
+  const Blc n(x.data);
+  const auto out_t = autocast_type(x.data);
+  if (!mods_ok(n.B, n.C, sh, sc) || sh.data.device() != x.data.device() || (out_t != at::kFloat && out_t != at::kBFloat16)) return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  const bool dual = x.tan.defined() || sh.tan.defined() || sc.tan.defined();
+  Tensor y, ty, xd;
+  {
+    Below below;
+    xd = dense(x.data);
+    const Tensor tx = dense(x.tan);
+    const Mod msh = mod(sh, n.B, n.C), msc = mod(sc, n.B, n.C);
+    y = empty({n.B, n.L, n.C}, out_t, xd);
+    if (dual) ty = empty({n.B, n.L, n.C}, out_t, xd);
+    const int64_t st[4] = {msh.st, msc.st, msh.tst, msc.tst};
+    check(dmf_ln_modulate_fwd(ptr(xd), ptr(tx), ptr(msh.t), ptr(msc.t), ptr(msh.tan), ptr(msc.tan), mptr(y), mptr(ty), st, n.B, n.L, n.C, (float)eps,
+                              code_of(xd), code_of(msh.t), code_of(y), stream_of(xd)),
+          "dmf_ln_modulate_fwd");
+  }
+  std::shared_ptr<KernelNode> node;
+  if (any_grad(x, sh, sc)) {
+    node = make_node("LNModulateBackward", {x, sh, sc}, {xd, sc.data});
+    node->fn = [eps, shs = sh.data.sizes().vec(), scs = sc.data.sizes().vec()](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) {
+      variable_list r = ln_backward(g[0], sv[0], sv[1], (float)eps, Tensor());
+      r[1] = r[1].view(shs);
+      r[2] = r[2].view(scs);
+      return r;
+    };
+  }
+  return py::cast(finish(y, ty, node, level));
+}
+
+// x (and its tangent) in the promoted type of x and h
+bool promote(Arg& x, const Arg& h) {
+  const auto dt = c10::promoteTypes(x.data.scalar_type(), h.data.scalar_type());
+  if (x.data.scalar_type() == dt) return true;
+  return false;   // rare (a low-precision residual stream next to fp32 branches): the general route casts
+}
+
+py::object gate_residual(const Tensor& x_, const Tensor& gate_, const Tensor& h_) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  Arg x = unpack(x_);
+  const Arg gate = unpack(gate_), h = unpack(h_);
+  if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !promote(x, h)) return none();
+  const Blc n(x.data);
+  if (!mods_ok(n.B, n.C, gate) || gate.data.device() != x.data.device() || h.data.device() != x.data.device()) return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  const bool dual = x.tan.defined() || gate.tan.defined() || h.tan.defined();
+  Tensor y, ty, hd;
+  {
+    Below below;
+    const Tensor xd = dense(x.data), tx = dense(x.tan), th = dense(h.tan);
+    hd = dense(h.data);
+    const Mod mg = mod(gate, n.B, n.C);
+    y = dense_like(xd);
+    if (dual) ty = dense_like(xd);
+    const int64_t st[2] = {mg.st, mg.tst};
+    check(dmf_gate_residual_fwd(ptr(xd), ptr(tx), ptr(mg.t), ptr(mg.tan), ptr(hd), ptr(th), mptr(y), mptr(ty), st, n.B, n.L, n.C, code_of(xd),
+                                code_of(mg.t), code_of(hd), stream_of(xd)),
+          "dmf_gate_residual_fwd");
+  }
+  std::shared_ptr<KernelNode> node;
+  if (any_grad(x, gate, h)) {
+    node = make_node("GateResidualBackward", {x, gate, h}, {hd, gate.data});
+    node->fn = [gs = gate.data.sizes().vec()](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      const variable_list r = gate_backward(g[0], sv[1], sv[0]);
+      return {g[0], r[1].view(gs), r[0]};
+    };
+  }
+  return py::cast(finish(y, ty, node, level));
+}
+
+py::object residual_ln_modulate(const Tensor& x_, const Tensor& gate_, const Tensor& h_, const Tensor& shift_, const Tensor& scale_, double eps) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  Arg x = unpack(x_);
+  const Arg gate = unpack(gate_), h = unpack(h_), sh = unpack(shift_), sc = unpack(scale_);
+  if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !promote(x, h)) return none();
+  const Blc n(x.data);
+  const auto out_t = autocast_type(x.data);
+  if (!mods_ok(n.B, n.C, gate, sh, sc) || gate.data.device() != x.data.device() || h.data.device() != x.data.device() ||
+      (out_t != at::kFloat && out_t != at::kBFloat16))
+    return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  const bool dual = x.tan.defined() || gate.tan.defined() || h.tan.defined() || sh.tan.defined() || sc.tan.defined();
+  Tensor y, ty, z, tz, hd;
+  {
+    Below below;
+    const Tensor xd = dense(x.data), tx = dense(x.tan), th = dense(h.tan);
+    hd = dense(h.data);
+    const Mod mg = mod(gate, n.B, n.C), msh = mod(sh, n.B, n.C), msc = mod(sc, n.B, n.C);
+    y = dense_like(xd);
+    z = empty(xd.sizes(), out_t, xd);
+    if (dual) {
+      ty = dense_like(xd);
+      tz = empty(xd.sizes(), out_t, xd);
+    }
+    const int64_t st[6] = {mg.st, mg.tst, msh.st, msc.st, msh.tst, msc.tst};
+    check(dmf_residual_ln_modulate_fwd(ptr(xd), ptr(tx), ptr(mg.t), ptr(mg.tan), ptr(hd), ptr(th), ptr(msh.t), ptr(msc.t), ptr(msh.tan), ptr(msc.tan),
+                                       mptr(y), mptr(ty), mptr(z), mptr(tz), st, n.B, n.L, n.C, (float)eps, code_of(xd), code_of(mg.t), code_of(hd),
+                                       code_of(z), stream_of(xd)),
+          "dmf_residual_ln_modulate_fwd");
+  }
+  std::shared_ptr<KernelNode> node;
+  if (any_grad(x, gate, h, sh, sc)) {
+    node = make_node("ResidualLNModulateBackward", {x, gate, h, sh, sc}, {data_of(y), hd, gate.data, sc.data});
+    node->fn = [eps, gs = gate.data.sizes().vec(), shs = sh.data.sizes().vec(), scs = sc.data.sizes().vec()](
+                   KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      const Tensor &gy = g[0], &gz = g[1];
+      if (!gz.defined()) {   // only the residual output was used
+        const variable_list r = gate_backward(gy, sv[2], sv[1]);
+        return {gy, r[1].view(gs), r[0]};
+      }
+      const variable_list ln = ln_backward(gz, sv[0], sv[3], (float)eps, gy);
+      const variable_list r = gate_backward(ln[0], sv[2], sv[1]);
+      return {ln[0], r[1].view(gs), r[0], ln[1].view(shs), ln[2].view(scs)};
+    };
+  }
+  const Tensor yo = finish(y, ty, node, level), zo = finish(z, tz, node, level);
+  return py::make_tuple(yo, zo);
+}
+
+enum class Act { gelu, silu };
+py::object activation(const Tensor& x_, Act act) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg x = unpack(x_);
+  if (!plain_gpu(x) || !block_dtype(x.data) || x.data.numel() == 0 || x.data.numel() % 8) return none();
+  const auto out_t = act == Act::silu ? autocast_type(x.data) : x.data.scalar_type();
+  if (out_t != at::kFloat && out_t != at::kBFloat16) return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  Tensor xd, y, ty;
+  {
+    Below below;
+    xd = dense(x.data);
+    const Tensor tx = dense(x.tan);
+    y = empty(xd.sizes(), out_t, xd);
+    if (tx.defined()) ty = empty(xd.sizes(), out_t, xd);
+    const int64_t n = xd.numel();
+    if (act == Act::gelu)
+      check(dmf_gelu_tanh_fwd(ptr(xd), ptr(tx), mptr(y), mptr(ty), n, code_of(xd), stream_of(xd)), "dmf_gelu_tanh_fwd");
+    else
+      check(dmf_silu_fwd(ptr(xd), ptr(tx), mptr(y), mptr(ty), n, code_of(xd), code_of(y), stream_of(xd)), "dmf_silu_fwd");
+  }
+  std::shared_ptr<KernelNode> node;
+  if (any_grad(x)) {
+    node = make_node(act == Act::gelu ? "GeluTanhBackward" : "SiluBackward", {x}, {xd});
+    node->fn = [act](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      const Tensor& x = sv[0];
+      const Tensor gx = dense_like(x);
+      if (act == Act::gelu) {
+        const Tensor gy = dense(g[0].to(x.scalar_type()));
+        check(dmf_gelu_tanh_bwd(ptr(gy), ptr(x), mptr(gx), x.numel(), code_of(x), stream_of(x)), "dmf_gelu_tanh_bwd");
+      } else {
+        const Tensor gy = dense(g[0]);
+        check(dmf_silu_bwd(ptr(gy), ptr(x), mptr(gx), x.numel(), code_of(x), code_of(gy), stream_of(x)), "dmf_silu_bwd");
+      }
+      return {gx};
+    };
+  }
+  return py::cast(finish(y, ty, node, level));
+}
+
+// ---- linear --------------------------------------------------------------------------------------------------------------
+
+// One extra stream per device for the weight-gradient half of a layer's backward (the one dmf_amd._lib.side_stream hands out).
+c10::Stream side_stream(const Tensor& t) {
+  static std::array<std::optional<c10::Stream>, 64> streams;
+  static std::mutex m;
+  std::lock_guard<std::mutex> lock(m);
+  auto& s = streams.at(t.get_device());
+  if (!s) {
+    py::gil_scoped_acquire gil;
+    const py::object st = g_lib.attr("side_stream")(t.get_device());
+    s = c10::Stream::unpack3(st.attr("stream_id").cast<int64_t>(), st.attr("device_index").cast<int>(), at::kCUDA);
+  }
+  return *s;
+}
+
+Tensor column_sum(const Tensor& x, at::ScalarType dt) {
+  const int64_t rows = x.size(0), C = x.size(1);
+  const Tensor out = empty({C}, dt, x), ws = workspace(dmf_block_workspace_floats(3, 1, (int)std::min<int64_t>(rows, INT32_MAX), (int)C), x);
+  check(dmf_colsum(ptr(x), mptr(out), static_cast<float*>(mptr(ws)), rows, (int)C, code_of(x), code_of(out), stream_of(x)), "dmf_colsum");
+  return out;
+}
+
+// DualLinearFunc.backward: the parameter gradients on the side stream next to the input gradient.
+variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w, const Tensor& gy, at::ScalarType x_type, at::ScalarType w_type,
+                              at::ScalarType b_type, bool has_bias, const std::vector<int64_t>& x_shape) {
+  Tensor g2 = gy.reshape({-1, gy.size(-1)}).to(w.scalar_type());
+  const bool want_gx = node.wants(0), want_gw = node.wants(1), want_gb = has_bias && node.wants(2), fork = want_gx && (want_gw || want_gb);
+  Tensor gx, gw, gb;
+  auto parameters = [&] {
+    if (want_gw) {
+      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = at::mm(g2.t(), x, at::kFloat);   // the GEMM stores its fp32 accumulators
+      else gw = at::mm(g2.t(), x).to(w_type);
+    }
+    if (want_gb) gb = column_sum(dense(g2), b_type);
+  };
+  if (fork) {
+    const c10::impl::VirtualGuardImpl impl(at::kCUDA);
+    const c10::Stream main = impl.getStream(g2.device()), side = side_stream(g2);
+    c10::Event forked(at::kCUDA), joined(at::kCUDA);
+    forked.record(main);
+    side.wait(forked);
+    impl.exchangeStream(side);
+    try {
+      parameters();
+    } catch (...) {
+      impl.exchangeStream(main);
+      throw;
+    }
+    joined.record(side);
+    impl.exchangeStream(main);
+    gx = at::mm(g2, w).reshape(x_shape).to(x_type);
+    main.wait(joined);
+    for (const Tensor* t : {&gw, &gb})   // allocated on the side stream, consumed (and later freed) on the main one
+      if (t->defined()) t->record_stream(main);
+  } else {
+    parameters();
+    if (want_gx) gx = at::mm(g2, w).reshape(x_shape).to(x_type);
+  }
+  return {gx, gw, gb};
+}
+
+struct LinearOperands {
+  Tensor w, b;
+  at::ScalarType dt;
+  bool ok = false;
+};
+// (autocast state is read by the caller: a Below guard hides it)
+LinearOperands linear_operands(bool autocast, at::ScalarType dt, const Arg& weight, const Arg& bias, const OptTensor& w_lp, const OptTensor& b_lp) {
+  LinearOperands o;
+  o.dt = dt;
+  if (o.dt != at::kFloat && o.dt != at::kBFloat16) return o;
+  if (o.dt == weight.data.scalar_type() || !autocast) {
+    if (weight.data.scalar_type() != o.dt || (bias.defined() && bias.data.scalar_type() != o.dt)) return o;
+    o.w = weight.data;
+    o.b = bias.data;
+  } else {
+    const bool cached = w_lp && w_lp->defined() && w_lp->scalar_type() == o.dt;
+    o.w = cached ? data_of(unwrap(*w_lp)) : weight.data.to(o.dt);
+    if (bias.defined()) o.b = cached && b_lp && b_lp->defined() ? data_of(unwrap(*b_lp)) : bias.data.to(o.dt);
+  }
+  o.ok = true;
+  return o;
+}
+bool linear_ok(const Arg& x, const Arg& weight, const Arg& bias) {
+  return plain_gpu(x) && plain_gpu(weight) && (!bias.defined() || plain_gpu(bias)) && block_dtype(x.data) && block_dtype(weight.data) &&
+         weight.data.dim() == 2 && x.data.dim() >= 2 && x.data.size(-1) == weight.data.size(1) && x.data.numel() > 0 && !weight.tan.defined() &&
+         !bias.tan.defined() && weight.data.device() == x.data.device();
+}
+
+py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg x = unpack(x_), weight = unpack(weight_), bias = unpack(bias_);
+  if (!linear_ok(x, weight, bias)) return none();
+  const bool grad = any_grad(x, weight, bias);
+  // (a bias gradient of another width goes through torch's column sum, whose replay from a captured graph the general route refuses)
+  if (grad && bias.grad() && weight.data.size(0) % 8) return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  Tensor y, ty, x2;
+  LinearOperands o;
+  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+  const at::ScalarType dt = autocast_type(x.data);
+  {
+    Below below;
+    o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp);
+    if (!o.ok) return none();
+    const int64_t K = x.data.size(-1);
+    auto sizes = x.data.sizes().vec();
+    sizes.back() = o.w.size(0);
+    x2 = x.data.reshape({-1, K}).to(o.dt);
+    y = (o.b.defined() ? at::addmm(o.b, x2, o.w.t()) : at::mm(x2, o.w.t())).view(sizes);
+    if (x.tan.defined()) ty = at::mm(x.tan.reshape({-1, K}).to(o.dt), o.w.t()).view(sizes);
+  }
+  std::shared_ptr<KernelNode> node;
+  if (grad) {
+    node = make_node("DualLinearBackward", {x, weight, bias}, {x2, o.w});
+    node->fn = [xs = x.data.sizes().vec(), xt = x.data.scalar_type(), wt = weight.data.scalar_type(), has_bias = bias.defined(),
+                bt = bias.defined() ? bias.data.scalar_type() : at::kFloat](KernelNode& node, const std::vector<Tensor>& sv, const variable_list& g) {
+      return linear_backward(node, sv[0], sv[1], g[0], xt, wt, bt, has_bias, xs);
+    };
+  }
+  return py::cast(finish(y, ty, node, level));
+}
+
+// gelu_tanh(linear(x)) with nothing differentiated: the activation rides in the GEMM's epilogue.
+py::object linear_gelu_inference(const Tensor& x_, const Tensor& weight_, const Tensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
+  const int64_t level = current_level();
+  if (level != kNoLevel || c10::GradMode::is_enabled()) return none();
+  const Arg x = unpack(x_), weight = unpack(weight_), bias = unpack(bias_);
+  if (!linear_ok(x, weight, bias) || x.tan.defined()) return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+  const at::ScalarType dt = autocast_type(x.data);
+  Below below;
+  const LinearOperands o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp);
+  if (!o.ok) return none();
+  auto sizes = x.data.sizes().vec();
+  sizes.back() = o.w.size(0);
+  return py::cast(at::_addmm_activation(o.b, x.data.reshape({-1, x.data.size(-1)}).to(o.dt), o.w.t(), 1, 1, true).view(sizes));
+}
+
+// x.chunk(n, -1) of a modulation tensor, tangent included
+py::object chunk_last(const Tensor& x_, int64_t n) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg x = unpack(x_);
+  if (!plain_gpu(x) || x.data.dim() < 1 || x.data.size(-1) % n) return none();
+  std::vector<Tensor> parts, tparts;
+  const int64_t w = x.data.size(-1) / n;
+  {
+    Below below;
+    parts = x.data.split(w, -1);
+    if (x.tan.defined()) tparts = x.tan.split(w, -1);
+  }
+  std::shared_ptr<KernelNode> node;
+  if (any_grad(x)) {
+    node = make_node("ChunkBackward", {x}, {parts[0]});
+    node->fn = [n](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+      std::vector<Tensor> parts;
+      for (int64_t i = 0; i < n; ++i) parts.push_back(g[i].defined() ? g[i] : at::zeros_like(sv[0], at::MemoryFormat::Contiguous));
+      return {at::cat(parts, -1)};
+    };
+  }
+  py::list out;
+  for (int64_t i = 0; i < n; ++i) out.append(finish(parts[i], tparts.empty() ? Tensor() : tparts[i], node, level));
+  return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.doc() = "native host path of dmf_amd's operators (None: take the general route)";
+  m.def("bind", [](py::object lib) { g_lib = lib.release(); });
+  m.def("attention", &attention);
+  m.def("attention_packed", &attention_packed);
+  m.def("attention_qknorm_packed", &attention_qknorm_packed);
+  m.def("ln_modulate", &ln_modulate);
+  m.def("gate_residual", &gate_residual);
+  m.def("residual_ln_modulate", &residual_ln_modulate);
+  m.def("gelu_tanh", [](const Tensor& x) { return activation(x, Act::gelu); });
+  m.def("silu", [](const Tensor& x) { return activation(x, Act::silu); });
+  m.def("linear", &linear);
+  m.def("linear_gelu_inference", &linear_gelu_inference);
+  m.def("chunk_last", &chunk_last);
+}

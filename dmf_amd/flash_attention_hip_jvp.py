@@ -156,6 +156,10 @@ def flash_attn_func(q, k, v, softmax_scale=None):
     (fp32 accumulation and softmax, nothing rounded to fp16 before the result); with
     k, v of another type next to an fp16 q everything is computed in fp32 and rounded back.
     """
+    if _lib.native(q):
+        out = _lib.host().attention(q, k, v, softmax_scale)
+        if out is not None:
+            return out
     if q.dtype == torch.float16 and not (k.dtype == v.dtype == torch.float16):
         return flash_attn_func(q.float(), k.float(), v.float(), _default_scale(q, softmax_scale)).to(torch.float16)
     d = q.shape[-1]
@@ -234,6 +238,10 @@ def flash_attn_qkvpacked_func(qkv, softmax_scale=None):
     -> dual out, like ``flash_attn_func``."""
     if qkv.dim() != 5 or qkv.shape[2] != 3:
         raise ValueError(f"expected a packed (B, L, 3, H, D) tensor, got shape {tuple(qkv.shape)}")
+    if _lib.native(qkv):
+        out = _lib.host().attention_packed(qkv, 0, softmax_scale)
+        if out is not None:
+            return out
     p, tg = fwAD.unpack_dual(qkv)
     if tg is None and _lib.plain_inference(p):
         q, k, v = p.unbind(2)
@@ -331,6 +339,10 @@ def flash_attn_qknorm_qkvpacked_func(qkv, q_gain, k_gain, eps: float = 1e-6, sof
     Dual in -> dual out; the gains are constants of the tangent map."""
     if qkv.dim() != 5 or qkv.shape[2] != 3:
         raise ValueError(f"expected a packed (B, L, 3, H, D) tensor, got shape {tuple(qkv.shape)}")
+    if IN_KERNEL_Q_NORM and _lib.native(qkv):
+        out = _lib.host().attention_qknorm_packed(qkv, q_gain, k_gain, 0, eps, softmax_scale, K_NORM_IN_KERNEL_MAX_LQ if IN_KERNEL_K_NORM else 0)
+        if out is not None:
+            return out
     p, tg = fwAD.unpack_dual(qkv)
     if tg is None and _lib.plain_inference(p, q_gain, k_gain):
         q, k, v = p.unbind(2)
@@ -347,3 +359,21 @@ def flash_attn_qknorm_qkvpacked_func(qkv, q_gain, k_gain, eps: float = 1e-6, sof
         return _lib.fwd(qn, kn, v, scale, need_lse=False)[0]
     out, _, t_out, _, _ = _lib.run_function(QKNormAttnQKVPackedFunc, p, tg, q_gain, k_gain, eps, softmax_scale)
     return out if tg is None else fwAD.make_dual(out, t_out)
+
+
+def flash_attn_projection(qkv, num_heads: int, q_gain=None, k_gain=None, eps: float = 1e-6):
+    """Attention on a projection output (B, L, 3 C) with ``num_heads`` heads, returns (B, L, C): the packed operators above
+    (with gains: the q/k-norm one) without a reshape on either side."""
+    if _lib.native(qkv):
+        if q_gain is None:
+            out = _lib.host().attention_packed(qkv, num_heads, None)
+        elif IN_KERNEL_Q_NORM:
+            out = _lib.host().attention_qknorm_packed(qkv, q_gain, k_gain, num_heads, eps, None, K_NORM_IN_KERNEL_MAX_LQ if IN_KERNEL_K_NORM else 0)
+        else:
+            out = None
+        if out is not None:
+            return out
+    B, L, C3 = qkv.shape
+    packed = qkv.reshape(B, L, 3, num_heads, C3 // (3 * num_heads))
+    out = flash_attn_qkvpacked_func(packed) if q_gain is None else flash_attn_qknorm_qkvpacked_func(packed, q_gain, k_gain, eps)
+    return out.reshape(B, L, C3 // 3)

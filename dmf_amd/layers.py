@@ -19,8 +19,7 @@ from torch import Tensor
 from . import block_ops as fused
 from ._lib import SUPPORTED_HEAD_DIMS
 from .flash_attention_hip_jvp import flash_attn_func as hip_func
-from .flash_attention_hip_jvp import flash_attn_qknorm_qkvpacked_func as hip_qknorm_qkvpacked_func
-from .flash_attention_hip_jvp import flash_attn_qkvpacked_func as hip_qkvpacked_func
+from .flash_attention_hip_jvp import flash_attn_projection as hip_projection
 
 # values accepted by --attn-func; "hip" is the one this package adds
 ATTN_FUNCS = ("base", "torch_sdpa", "hip")
@@ -189,12 +188,9 @@ class Attention(nn.Module):
     def forward(self, x: Tensor) -> Tensor:
         B, L, C = x.shape
         if self.packed:
-            qkv = self.qkv(x).reshape(B, L, 3, self.num_heads, self.head_dim)
             if self.qk_norm:
-                x = hip_qknorm_qkvpacked_func(qkv, self.q_norm.scale, self.k_norm.scale, self.q_norm.eps)
-            else:
-                x = hip_qkvpacked_func(qkv)
-            return self.proj(x.reshape(B, L, C))
+                return self.proj(hip_projection(self.qkv(x), self.num_heads, self.q_norm.scale, self.k_norm.scale, self.q_norm.eps))
+            return self.proj(hip_projection(self.qkv(x), self.num_heads))
         qkv = self.qkv(x).reshape(B, L, 3, self.num_heads, self.head_dim).permute(2, 0, 1, 3, 4)
         q, k, v = qkv.unbind(0)  # each (B, L, H, D), strides (3LHD, 3HD, D, 1)
         q, k = self.q_norm(q), self.k_norm(k)
@@ -232,8 +228,13 @@ class DiTBlock(nn.Module):
         self.mlp = Mlp(hidden_size, int(hidden_size * mlp_ratio), block_ops=block_ops)
         self.adaLN_modulation = nn.Sequential(SiLU(block_ops), Linear(hidden_size, 6 * hidden_size, block_ops=block_ops))
 
+    def modulation(self, c: Tensor):
+        """The six (B, 1, C) chunks of the adaLN output: shift, scale, gate of the attention branch, then of the MLP branch."""
+        m = self.adaLN_modulation(c)
+        return fused.chunk_last(m, 6) if self.fused else m.chunk(6, dim=-1)
+
     def forward(self, x: Tensor, c: Tensor) -> Tensor:
-        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = self.adaLN_modulation(c).chunk(6, dim=-1)
+        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = self.modulation(c)
         if self.fused:   # same expressions; the first residual is fused with the norm+modulate that follows it
             x, z = fused.residual_ln_modulate(x, gate_msa, self.attn(fused.ln_modulate(x, shift_msa, scale_msa, self.norm1.eps)),
                                               shift_mlp, scale_mlp, self.norm2.eps)
@@ -265,8 +266,12 @@ class FinalLayer(nn.Module):
         self.linear = Linear(hidden_size, patch_size * patch_size * out_channels, block_ops=block_ops)
         self.adaLN_modulation = nn.Sequential(SiLU(block_ops), Linear(hidden_size, 2 * hidden_size, block_ops=block_ops))
 
+    def modulation(self, c: Tensor):
+        m = self.adaLN_modulation(c)
+        return fused.chunk_last(m, 2) if self.fused else m.chunk(2, dim=-1)
+
     def forward(self, x: Tensor, c: Tensor) -> Tensor:
-        shift, scale = self.adaLN_modulation(c).chunk(2, dim=-1)
+        shift, scale = self.modulation(c)
         if self.fused:
             return self.linear(fused.ln_modulate(x, shift, scale, self.norm_final.eps))
         return self.linear(modulate(self.norm_final(x), shift, scale))

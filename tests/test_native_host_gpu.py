@@ -1,0 +1,113 @@
+"""The native host path against the general Python route: same kernels, same operands, so the same bits -- outputs, tangents,
+gradients -- in every way an operator is differentiated; and the cases it hands back to the general route."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwAD
+
+import dmf_amd
+from dmf_amd import _lib, block_ops, harness
+from dmf_amd.dmft import DMFT
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _general(fn):
+    """``fn()`` with the native path switched off."""
+    native, _lib.native = _lib.native, lambda t: False
+    try:
+        return fn()
+    finally:
+        _lib.native = native
+
+
+def _attn_case(kind, dtype):
+    g = torch.Generator().manual_seed(9)
+    B, L, H, D = 2, 40, 3, 64
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)
+    if kind == "separate":
+        return dmf_amd.flash_attn_func, [rnd(B, L, H, D) for _ in range(3)]
+    if kind == "views":
+        return dmf_amd.flash_attn_func, list(rnd(B, L, 3, H, D).unbind(2))
+    if kind == "packed":
+        return dmf_amd.flash_attn_qkvpacked_func, [rnd(B, L, 3, H, D)]
+    gains = [torch.rand(D, generator=g).to(DEV) + 0.5 for _ in range(2)]
+    return dmf_amd.flash_attn_qknorm_qkvpacked_func, [rnd(B, L, 3, H, D), *gains]
+
+
+def _all_modes(fn, args, moving):
+    """Plain, no-grad, torch.func.jvp and dual-level calls, the last two with a gradient through the primal output; the first
+    ``moving`` arguments carry tangents."""
+    outs = []
+    with torch.no_grad():
+        outs.append(fn(*args))
+    leaves = [a.detach().clone().requires_grad_() for a in args]
+    o = fn(*leaves)
+    gy = torch.linspace(-1, 1, o.numel(), device=DEV).reshape(o.shape).to(o.dtype)
+    outs += [o.detach(), *torch.autograd.grad(o, leaves, gy)]
+    tangents = [a.detach().flip(0) for a in args[:moving]]
+    o, to = torch.func.jvp(lambda *m: fn(*m, *leaves[moving:]), tuple(leaves[:moving]), tuple(tangents))
+    outs += [o.detach(), to.detach(), *torch.autograd.grad(o, leaves, gy)]
+    with fwAD.dual_level():
+        o, to = fwAD.unpack_dual(fn(*(fwAD.make_dual(a, t) for a, t in zip(leaves, tangents)), *leaves[moving:]))
+    outs += [o.detach(), to.detach(), *torch.autograd.grad(o, leaves, gy)]
+    # only one operand moves: the others' tangents are zeros
+    o, to = torch.func.jvp(lambda m: fn(m, *args[1:]), (args[0],), (tangents[0],))
+    return outs + [o, to]
+
+
+@pytest.mark.parametrize("kind,dtype", [("separate", torch.float32), ("separate", torch.float16), ("views", torch.bfloat16),
+                                        ("packed", torch.bfloat16), ("packed", torch.float32), ("qknorm", torch.bfloat16)])
+def test_attention_operators_give_the_same_bits(kind, dtype):
+    fn, args = _attn_case(kind, dtype)
+    moving = len(args) if kind in ("separate", "views") else 1
+    if kind in ("separate", "views"):
+        assert _lib.host().attention(*args, None) is not None
+    new, old = _all_modes(fn, args, moving), _general(lambda: _all_modes(fn, args, moving))
+    assert len(new) == len(old)
+    for i, (a, b) in enumerate(zip(new, old)):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("qk_norm", [False, True])
+@pytest.mark.parametrize("functorch", [True, False])
+@pytest.mark.parametrize("autocast", [True, False])
+def test_training_step_gives_the_same_bits(autocast, functorch, qk_norm):
+    """Every block operator, forward-mode and backward, through a small model."""
+    torch.manual_seed(3)
+    model = DMFT(input_size=16, hidden_size=256, depth=3, num_heads=4, dmf_depth=2, qk_norm=qk_norm, attn_func="hip", block_ops="hip")
+    model = model.to(DEV).init_trunc_normal_()
+    batch = harness.synthetic_batch(3, DEV, input_size=16)
+
+    def step():
+        model.zero_grad(set_to_none=True)
+        loss = harness.train_step(model, batch, autocast=autocast, functorch=functorch)
+        return [loss.detach()] + [p.grad for p in model.parameters() if p.requires_grad]
+
+    for i, (a, b) in enumerate(zip(step(), _general(step))):
+        assert torch.equal(a, b), i
+
+
+def test_what_the_native_path_hands_back():
+    q = torch.randn(2, 16, 2, 64, device=DEV)
+    host = _lib.host()
+    assert host.attention(q, q, q, None) is not None
+    assert host.attention(q.cpu(), q.cpu(), q.cpu(), None) is None                      # not on the GPU
+    assert host.attention(q[..., :40], q[..., :40], q[..., :40], None) is None           # head dim without a kernel
+    assert host.attention(q.transpose(2, 3), q.transpose(2, 3), q.transpose(2, 3), None) is None
+    assert host.attention(q.double(), q.double(), q.double(), None) is None
+    seen = []
+    torch.func.jvp(lambda x: torch.func.jvp(lambda y: (seen.append(host.attention(y, y, y, None)), y)[1], (x,), (x,))[0], (q,), (q,))
+    assert seen == [None]                                                                # two levels
+    x = torch.randn(2, 8, 64, device=DEV)
+    m = torch.randn(2, 64, device=DEV)
+    with torch.enable_grad():   # saved tensors are freed with the first backward, as for any node
+        y = block_ops.ln_modulate(x.requires_grad_(), m, m)
+        y.sum().backward()
+        with pytest.raises(RuntimeError, match="second time"):
+            y.sum().backward()
+        z = x * 1.0
+        y = block_ops.ln_modulate(z, m, m)
+        z.mul_(2.0)             # and modifying one in place is caught
+        with pytest.raises(RuntimeError, match="inplace"):
+            y.sum().backward()
