@@ -80,6 +80,35 @@ __device__ __forceinline__ float wave_sum(float v) {
   return xhalf_sum(even + odd);
 }
 
+// The same in two steps with the element type known at compile time: RawVec holds the loaded registers, so that a kernel can
+// request everything it reads before it converts (and thereby waits for) the first of it.  A run-time type puts each load and
+// its conversion into a branch of its own, one memory latency after the other: B64 L256 C768, fp32 stream and
+// bf16 branches, residual + LayerNorm with tangents 75 -> 56 us = 5.4 TB/s (a 1 GiB copy: 5.0), LayerNorm 33 -> 27 us.
+template <bool BF>
+struct RawVec {
+  u32x4 r[BF ? 1 : 2];
+  __device__ __forceinline__ void load(const void* p, int64_t idx) {   // p == nullptr reads as zeros
+    const u32x4* q = reinterpret_cast<const u32x4*>(static_cast<const char*>(p) + idx * (BF ? 2 : 4));
+#pragma unroll
+    for (int i = 0; i < (BF ? 1 : 2); ++i) r[i] = p != nullptr ? q[i] : u32x4{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ void get(float (&o)[8]) const {
+    if constexpr (BF) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o[2 * i] = __uint_as_float(r[0][i] << 16);
+        o[2 * i + 1] = __uint_as_float(r[0][i] & 0xffff0000u);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o[i] = __uint_as_float(r[0][i]);
+        o[4 + i] = __uint_as_float(r[1][i]);
+      }
+    }
+  }
+};
+
 // ---- a row of C elements held by one wave: lane owns columns (j*64 + lane)*8 .. +8, j < NV -------------------------
 
 template <int NV>
@@ -87,15 +116,25 @@ struct Row {
   float v[NV][8];
 };
 
-template <int NV>
-__device__ __forceinline__ void load_row(const void* p, int bf16, int64_t base, int C, int lane, Row<NV>& r) {
+// Columns past C: the address is clamped into the row (no branch around the load) and the values read as zeros.
+template <int NV, bool BF>
+struct RawRow {
+  RawVec<BF> v[NV];
+  __device__ __forceinline__ void load(const void* p, int64_t base, int C, int lane) {
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    const int col = (j * 64 + lane) * 8;
-    if (col < C) load8(p, bf16, base + col, r.v[j]);
-    else zero8(r.v[j]);
+    for (int j = 0; j < NV; ++j) {
+      const int col = (j * 64 + lane) * 8;
+      v[j].load(p, base + (col < C ? col : 0));
+    }
   }
-}
+  __device__ __forceinline__ void get(Row<NV>& o, int C, int lane) const {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      v[j].get(o.v[j]);
+      if ((j * 64 + lane) * 8 >= C) zero8(o.v[j]);
+    }
+  }
+};
 
 template <int NV>
 __device__ __forceinline__ void store_row(void* p, int bf16, int64_t base, int C, int lane, const Row<NV>& r) {
@@ -163,6 +202,32 @@ __device__ __forceinline__ void project_row(Row<NV>& t, const Row<NV>& xh, float
   }
 }
 
+// y = xh (1 + scale) + shift and, with JVP, ty = t (1 + scale) + xh tscale + tshift, stored.
+template <int NV, bool JVP, bool MB>
+__device__ __forceinline__ void modulate_row(const Row<NV>& xh, const Row<NV>& t, const RawRow<NV, MB>& rsh, const RawRow<NV, MB>& rsc,
+                                             const RawRow<NV, MB>& rtsh, const RawRow<NV, MB>& rtsc, void* y, void* ty, int ybf, int64_t base,
+                                             int C, int lane) {
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int col = (j * 64 + lane) * 8;
+    if (col >= C) continue;
+    float sh[8], sc[8], out[8];
+    rsh.v[j].get(sh);
+    rsc.v[j].get(sc);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = fmaf(xh.v[j][e], 1.f + sc[e], sh[e]);
+    store8(y, ybf, base + col, out);
+    if (JVP) {
+      float tsh[8], tsc[8];
+      rtsh.v[j].get(tsh);
+      rtsc.v[j].get(tsc);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out[e] = fmaf(t.v[j][e], 1.f + sc[e], fmaf(xh.v[j][e], tsc[e], tsh[e]));
+      store8(ty, ybf, base + col, out);
+    }
+  }
+}
+
 // ---- LayerNorm + modulate -----------------------------------------------------------------------------------------
 
 struct LnFwdParams {
@@ -174,36 +239,30 @@ struct LnFwdParams {
   int xbf, mbf, ybf;
 };
 
-template <int NV, bool JVP>
+template <int NV, bool JVP, bool XB, bool MB, bool YB>
 __global__ __launch_bounds__(kThreads) void ln_modulate_fwd_kernel(LnFwdParams p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
   if (row >= p.rows) return;  // no work-group barrier in this kernel
   const int64_t b = row / p.L, base = row * p.C;
-  Row<NV> xh, t;
-  load_row(p.x, p.xbf, base, p.C, lane, xh);
-  if (JVP) load_row(p.tx, p.xbf, base, p.C, lane, t);
-  const float rstd = normalize_row(xh, p.C, lane, p.eps);
-  if (JVP) project_row(t, xh, rstd, p.C, lane);
-#pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    const int col = (j * 64 + lane) * 8;
-    if (col >= p.C) continue;
-    float sh[8], sc[8], out[8];
-    load8(p.shift, p.mbf, b * p.ms[0] + col, sh);
-    load8(p.scale, p.mbf, b * p.ms[1] + col, sc);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = fmaf(xh.v[j][e], 1.f + sc[e], sh[e]);
-    store8(p.y, p.ybf, base + col, out);
-    if (JVP) {
-      float tsh[8], tsc[8];
-      load8(p.tshift, p.mbf, b * p.ms[2] + col, tsh);
-      load8(p.tscale, p.mbf, b * p.ms[3] + col, tsc);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] = fmaf(t.v[j][e], 1.f + sc[e], fmaf(xh.v[j][e], tsc[e], tsh[e]));
-      store8(p.ty, p.ybf, base + col, out);
-    }
+  RawRow<NV, XB> rx, rt;
+  RawRow<NV, MB> rsh, rsc, rtsh, rtsc;
+  rx.load(p.x, base, p.C, lane);
+  if (JVP) rt.load(p.tx, base, p.C, lane);
+  rsh.load(p.shift, b * p.ms[0], p.C, lane);
+  rsc.load(p.scale, b * p.ms[1], p.C, lane);
+  if (JVP) {
+    rtsh.load(p.tshift, b * p.ms[2], p.C, lane);
+    rtsc.load(p.tscale, b * p.ms[3], p.C, lane);
   }
+  Row<NV> xh, t;
+  rx.get(xh, p.C, lane);
+  const float rstd = normalize_row(xh, p.C, lane, p.eps);
+  if (JVP) {
+    rt.get(t, p.C, lane);
+    project_row(t, xh, rstd, p.C, lane);
+  }
+  modulate_row<NV, JVP>(xh, t, rsh, rsc, rtsh, rtsc, p.y, p.ty, YB, base, p.C, lane);
 }
 
 // Adds the per-wave column accumulators of a work-group and writes them as one partial-sum row.
@@ -250,15 +309,29 @@ struct LnBwdParams {
   int xbf, mbf, gbf;
 };
 
-template <int NV>
+template <int NV, bool XB, bool MB, bool GB>
 __global__ __launch_bounds__(kThreads) void ln_modulate_bwd_kernel(LnBwdParams p) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t b = blockIdx.x / p.nchunk;
   const int chunk = blockIdx.x % p.nchunk;
   const int r1 = min(p.L, (chunk + 1) * kChunkRows);
+  RawRow<NV, MB> rsc;
+  rsc.load(p.scale, b * p.ss, p.C, lane);
+  // The next row's operands are requested before this row's arithmetic; the residual gradient, wanted last, with this row's
+  // (requested a row ahead it costs 24 registers and, at C > 1024, the second wave per SIMD: 37 us against 32 at B32 L256
+  // C1152, 4.1 TB/s).
+  RawRow<NV, XB> rx, rres;
+  RawRow<NV, GB> rg;
+  auto request = [&](int r) {
+    const int64_t base = (b * p.L + min(r, p.L - 1)) * p.C;
+    rx.load(p.x, base, p.C, lane);
+    rg.load(p.gy, base, p.C, lane);
+  };
+  int r = chunk * kChunkRows + wave;
+  request(r);
   Row<NV> one_plus_scale, acc[2];
-  load_row(p.scale, p.mbf, b * p.ss, p.C, lane, one_plus_scale);
+  rsc.get(one_plus_scale, p.C, lane);
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     zero8(acc[0].v[j]);
@@ -266,11 +339,13 @@ __global__ __launch_bounds__(kThreads) void ln_modulate_bwd_kernel(LnBwdParams p
 #pragma unroll
     for (int e = 0; e < 8; ++e) one_plus_scale.v[j][e] += 1.f;
   }
-  for (int r = chunk * kChunkRows + wave; r < r1; r += kWaves) {
+  for (; r < r1; r += kWaves) {
     const int64_t base = (b * p.L + r) * p.C;
-    Row<NV> xh, g;
-    load_row(p.x, p.xbf, base, p.C, lane, xh);
-    load_row(p.gy, p.gbf, base, p.C, lane, g);
+    Row<NV> xh, g, res;
+    rx.get(xh, p.C, lane);
+    rg.get(g, p.C, lane);
+    rres.load(p.gres, base, p.C, lane);
+    if (r + kWaves < r1) request(r + kWaves);
     const float rstd = normalize_row(xh, p.C, lane, p.eps);
 #pragma unroll
     for (int j = 0; j < NV; ++j)
@@ -281,14 +356,12 @@ __global__ __launch_bounds__(kThreads) void ln_modulate_bwd_kernel(LnBwdParams p
         g.v[j][e] *= one_plus_scale.v[j][e];
       }
     project_row(g, xh, rstd, p.C, lane);
-    if (p.gres != nullptr) {
-      load_row(p.gres, p.xbf, base, p.C, lane, xh);
+    rres.get(res, p.C, lane);
 #pragma unroll
-      for (int j = 0; j < NV; ++j)
+    for (int j = 0; j < NV; ++j)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) g.v[j][e] += xh.v[j][e];
-    }
-    store_row(p.gx, p.xbf, base, p.C, lane, g);
+      for (int e = 0; e < 8; ++e) g.v[j][e] += res.v[j][e];
+    store_row(p.gx, XB, base, p.C, lane, g);
   }
   reduce_waves_to_partial<NV, 2>(acc, lds, p.partial + static_cast<int64_t>(blockIdx.x) * 2 * p.C, p.C, lane, wave);
 }
@@ -355,28 +428,39 @@ struct GateFwdParams {
   int xbf, mbf, hbf;
 };
 
-template <bool JVP>
+template <bool JVP, bool XB, bool MB, bool HB>
 __global__ __launch_bounds__(kThreads) void gate_residual_fwd_kernel(GateFwdParams p) {
   const int64_t v = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (v >= p.total) return;
   const int vec_per_row = p.C / 8;
   const int col = static_cast<int>(v % vec_per_row) * 8;
   const int64_t row = v / vec_per_row, b = row / p.L, idx = v * 8;
+  RawVec<XB> rx, rtx;
+  RawVec<MB> rg, rtg;
+  RawVec<HB> rh, rth;
+  rx.load(p.x, idx);
+  rh.load(p.h, idx);
+  rg.load(p.gate, b * p.gs[0] + col);
+  if (JVP) {
+    rtx.load(p.tx, idx);
+    rth.load(p.th, idx);
+    rtg.load(p.tgate, b * p.gs[1] + col);
+  }
   float x[8], g[8], h[8], out[8];
-  load8(p.x, p.xbf, idx, x);
-  load8(p.h, p.hbf, idx, h);
-  load8(p.gate, p.mbf, b * p.gs[0] + col, g);
+  rx.get(x);
+  rh.get(h);
+  rg.get(g);
 #pragma unroll
   for (int e = 0; e < 8; ++e) out[e] = fmaf(g[e], h[e], x[e]);
-  store8(p.y, p.xbf, idx, out);
+  store8(p.y, XB, idx, out);
   if (JVP) {
     float tx[8], tg[8], th[8];
-    load8(p.tx, p.xbf, idx, tx);
-    load8(p.th, p.hbf, idx, th);
-    load8(p.tgate, p.mbf, b * p.gs[1] + col, tg);
+    rtx.get(tx);
+    rtg.get(tg);
+    rth.get(th);
 #pragma unroll
     for (int e = 0; e < 8; ++e) out[e] = fmaf(tg[e], h[e], fmaf(g[e], th[e], tx[e]));
-    store8(p.ty, p.xbf, idx, out);
+    store8(p.ty, XB, idx, out);
   }
 }
 
@@ -389,22 +473,34 @@ struct GateBwdParams {
   int gbf, mbf, hbf;
 };
 
-template <int NV>
+template <int NV, bool GB, bool MB, bool HB>
 __global__ __launch_bounds__(kThreads) void gate_residual_bwd_kernel(GateBwdParams p) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t b = blockIdx.x / p.nchunk;
   const int chunk = blockIdx.x % p.nchunk;
   const int r1 = min(p.L, (chunk + 1) * kChunkRows);
+  RawRow<NV, MB> rgate;
+  rgate.load(p.gate, b * p.gs, p.C, lane);
+  RawRow<NV, GB> rg;
+  RawRow<NV, HB> rh;
+  auto request = [&](int r) {
+    const int64_t base = (b * p.L + min(r, p.L - 1)) * p.C;
+    rg.load(p.gy, base, p.C, lane);
+    rh.load(p.h, base, p.C, lane);
+  };
+  int r = chunk * kChunkRows + wave;
+  request(r);
   Row<NV> gate, acc[1];
-  load_row(p.gate, p.mbf, b * p.gs, p.C, lane, gate);
+  rgate.get(gate, p.C, lane);
 #pragma unroll
   for (int j = 0; j < NV; ++j) zero8(acc[0].v[j]);
-  for (int r = chunk * kChunkRows + wave; r < r1; r += kWaves) {
+  for (; r < r1; r += kWaves) {
     const int64_t base = (b * p.L + r) * p.C;
     Row<NV> g, h;
-    load_row(p.gy, p.gbf, base, p.C, lane, g);
-    load_row(p.h, p.hbf, base, p.C, lane, h);
+    rg.get(g, p.C, lane);
+    rh.get(h, p.C, lane);
+    if (r + kWaves < r1) request(r + kWaves);
 #pragma unroll
     for (int j = 0; j < NV; ++j)
 #pragma unroll
@@ -412,7 +508,7 @@ __global__ __launch_bounds__(kThreads) void gate_residual_bwd_kernel(GateBwdPara
         acc[0].v[j][e] = fmaf(g.v[j][e], h.v[j][e], acc[0].v[j][e]);
         g.v[j][e] *= gate.v[j][e];
       }
-    store_row(p.gh, p.hbf, base, p.C, lane, g);
+    store_row(p.gh, HB, base, p.C, lane, g);
   }
   reduce_waves_to_partial<NV, 1>(acc, lds, p.partial + static_cast<int64_t>(blockIdx.x) * p.C, p.C, lane, wave);
 }
@@ -430,55 +526,54 @@ struct ResLnFwdParams {
   int xbf, mbf, hbf, zbf;
 };
 
-template <int NV, bool JVP>
+template <int NV, bool JVP, bool XB, bool MB, bool HB, bool ZB>
 __global__ __launch_bounds__(kThreads) void residual_ln_modulate_fwd_kernel(ResLnFwdParams p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
   if (row >= p.rows) return;  // no work-group barrier in this kernel
   const int64_t b = row / p.L, base = row * p.C;
-  Row<NV> y, t, h;
-  load_row(p.x, p.xbf, base, p.C, lane, y);
-  load_row(p.h, p.hbf, base, p.C, lane, h);
-  if (JVP) load_row(p.tx, p.xbf, base, p.C, lane, t);
+  RawRow<NV, XB> rx, rt;
+  RawRow<NV, HB> rh, rth;
+  RawRow<NV, MB> rg, rtg, rsh, rsc, rtsh, rtsc;
+  rx.load(p.x, base, p.C, lane);
+  rh.load(p.h, base, p.C, lane);
+  if (JVP) {
+    rt.load(p.tx, base, p.C, lane);
+    rth.load(p.th, base, p.C, lane);
+  }
+  rg.load(p.gate, b * p.ms[0], p.C, lane);
+  if (JVP) rtg.load(p.tgate, b * p.ms[1], p.C, lane);
+  rsh.load(p.shift, b * p.ms[2], p.C, lane);
+  rsc.load(p.scale, b * p.ms[3], p.C, lane);
+  if (JVP) {
+    rtsh.load(p.tshift, b * p.ms[4], p.C, lane);
+    rtsc.load(p.tscale, b * p.ms[5], p.C, lane);
+  }
+  Row<NV> y, t;
+  rx.get(y, p.C, lane);
+  if (JVP) rt.get(t, p.C, lane);
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int col = (j * 64 + lane) * 8;
     if (col >= p.C) continue;
-    float g[8];
-    load8(p.gate, p.mbf, b * p.ms[0] + col, g);
+    float g[8], h[8];
+    rg.v[j].get(g);
+    rh.v[j].get(h);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) y.v[j][e] = fmaf(g[e], h.v[j][e], y.v[j][e]);
-    store8(p.y, p.xbf, base + col, y.v[j]);
+    for (int e = 0; e < 8; ++e) y.v[j][e] = fmaf(g[e], h[e], y.v[j][e]);
+    store8(p.y, XB, base + col, y.v[j]);
     if (JVP) {
       float tg[8], th[8];
-      load8(p.tgate, p.mbf, b * p.ms[1] + col, tg);
-      load8(p.th, p.hbf, base + col, th);
+      rtg.v[j].get(tg);
+      rth.v[j].get(th);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) t.v[j][e] = fmaf(tg[e], h.v[j][e], fmaf(g[e], th[e], t.v[j][e]));
-      store8(p.ty, p.xbf, base + col, t.v[j]);
+      for (int e = 0; e < 8; ++e) t.v[j][e] = fmaf(tg[e], h[e], fmaf(g[e], th[e], t.v[j][e]));
+      store8(p.ty, XB, base + col, t.v[j]);
     }
   }
   const float rstd = normalize_row(y, p.C, lane, p.eps);
   if (JVP) project_row(t, y, rstd, p.C, lane);
-#pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    const int col = (j * 64 + lane) * 8;
-    if (col >= p.C) continue;
-    float sh[8], sc[8], out[8];
-    load8(p.shift, p.mbf, b * p.ms[2] + col, sh);
-    load8(p.scale, p.mbf, b * p.ms[3] + col, sc);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = fmaf(y.v[j][e], 1.f + sc[e], sh[e]);
-    store8(p.z, p.zbf, base + col, out);
-    if (JVP) {
-      float tsh[8], tsc[8];
-      load8(p.tshift, p.mbf, b * p.ms[4] + col, tsh);
-      load8(p.tscale, p.mbf, b * p.ms[5] + col, tsc);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] = fmaf(t.v[j][e], 1.f + sc[e], fmaf(y.v[j][e], tsc[e], tsh[e]));
-      store8(p.tz, p.zbf, base + col, out);
-    }
-  }
+  modulate_row<NV, JVP>(y, t, rsh, rsc, rtsh, rtsc, p.z, p.tz, ZB, base, p.C, lane);
 }
 
 // ---- pointwise activations: GELU (tanh approximation) and SiLU ------------------------------------------------------
@@ -729,6 +824,14 @@ inline int dispatch_nv(int C, F&& f) {
   }
 }
 
+// f(integral constants of three element types)
+template <typename F>
+inline int dispatch_types(bool a, bool b, bool c, F&& f) {
+  const auto with = [&](auto x, auto y) { return c ? f(x, y, std::true_type{}) : f(x, y, std::false_type{}); };
+  const auto with_a = [&](auto x) { return b ? with(x, std::true_type{}) : with(x, std::false_type{}); };
+  return a ? with_a(std::true_type{}) : with_a(std::false_type{});
+}
+
 // The reduction is a chain of dependent loads per thread with next to no work, so the shape that shortens the chain wins as
 // long as a row is read in whole 128-byte lines: 8 vectors (256 bytes) per work-group of 256 threads = 32 chunk groups, and
 // 1024 threads = 128 groups from 256 chunks on (the gain gradients: 1024 partial rows of 72 columns, one work-group).
@@ -822,8 +925,11 @@ int dmf_ln_modulate_fwd(const void* x, const void* tx, const void* shift, const 
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dispatch_nv(C, [&](auto nv) {
     constexpr int NV = decltype(nv)::value;
-    if (ty) return launch_kernel(ln_modulate_fwd_kernel<NV, true>, dim3(grid), dim3(kThreads), 0, s, p);
-    return launch_kernel(ln_modulate_fwd_kernel<NV, false>, dim3(grid), dim3(kThreads), 0, s, p);
+    return dispatch_types(p.xbf, p.mbf, p.ybf, [&](auto xb, auto mb, auto yb) {
+      constexpr bool X = decltype(xb)::value, M = decltype(mb)::value, Y = decltype(yb)::value;
+      if (ty) return launch_kernel(ln_modulate_fwd_kernel<NV, true, X, M, Y>, dim3(grid), dim3(kThreads), 0, s, p);
+      return launch_kernel(ln_modulate_fwd_kernel<NV, false, X, M, Y>, dim3(grid), dim3(kThreads), 0, s, p);
+    });
   });
 }
 
@@ -846,7 +952,9 @@ int dmf_ln_modulate_bwd(const void* gy, const void* x, const void* scale, const 
   const int rc = dispatch_nv(C, [&](auto nv) {
     constexpr int NV = decltype(nv)::value;
     constexpr size_t lds = (kWaves - 1) * 2 * NV * 512 * sizeof(float);
-    return launch_kernel(ln_modulate_bwd_kernel<NV>, dim3(grid), dim3(kThreads), lds, s, p);
+    return dispatch_types(p.xbf, p.mbf, p.gbf, [&](auto xb, auto mb, auto gb) {
+      return launch_kernel(ln_modulate_bwd_kernel<NV, decltype(xb)::value, decltype(mb)::value, decltype(gb)::value>, dim3(grid), dim3(kThreads), lds, s, p);
+    });
   });
   if (rc) return rc;
   return reduce_partials(workspace, gshift, gscale, B, p.nchunk, 2, C, p.mbf, s);
@@ -870,8 +978,11 @@ int dmf_gate_residual_fwd(const void* x, const void* tx, const void* gate, const
   p.xbf = x_dtype == DMF_ATTN_BF16; p.mbf = mod_dtype == DMF_ATTN_BF16; p.hbf = h_dtype == DMF_ATTN_BF16;
   const unsigned grid = static_cast<unsigned>((p.total + kThreads - 1) / kThreads);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (ty) return launch_kernel(gate_residual_fwd_kernel<true>, dim3(grid), dim3(kThreads), 0, s, p);
-  return launch_kernel(gate_residual_fwd_kernel<false>, dim3(grid), dim3(kThreads), 0, s, p);
+  return dispatch_types(p.xbf, p.mbf, p.hbf, [&](auto xb, auto mb, auto hb) {
+    constexpr bool X = decltype(xb)::value, M = decltype(mb)::value, H = decltype(hb)::value;
+    if (ty) return launch_kernel(gate_residual_fwd_kernel<true, X, M, H>, dim3(grid), dim3(kThreads), 0, s, p);
+    return launch_kernel(gate_residual_fwd_kernel<false, X, M, H>, dim3(grid), dim3(kThreads), 0, s, p);
+  });
 }
 
 int dmf_gate_residual_bwd(const void* gy, const void* gate, const void* h, void* gh, void* ggate, float* workspace,
@@ -892,7 +1003,9 @@ int dmf_gate_residual_bwd(const void* gy, const void* gate, const void* h, void*
   const int rc = dispatch_nv(C, [&](auto nv) {
     constexpr int NV = decltype(nv)::value;
     constexpr size_t lds = (kWaves - 1) * NV * 512 * sizeof(float);
-    return launch_kernel(gate_residual_bwd_kernel<NV>, dim3(grid), dim3(kThreads), lds, s, p);
+    return dispatch_types(p.gbf, p.mbf, p.hbf, [&](auto gb, auto mb, auto hb) {
+      return launch_kernel(gate_residual_bwd_kernel<NV, decltype(gb)::value, decltype(mb)::value, decltype(hb)::value>, dim3(grid), dim3(kThreads), lds, s, p);
+    });
   });
   if (rc) return rc;
   return reduce_partials(workspace, ggate, nullptr, B, p.nchunk, 1, C, p.mbf, s);
@@ -928,8 +1041,14 @@ int dmf_residual_ln_modulate_fwd(const void* x, const void* tx, const void* gate
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dispatch_nv(C, [&](auto nv) {
     constexpr int NV = decltype(nv)::value;
-    if (jvp) return launch_kernel(residual_ln_modulate_fwd_kernel<NV, true>, dim3(grid), dim3(kThreads), 0, s, p);
-    return launch_kernel(residual_ln_modulate_fwd_kernel<NV, false>, dim3(grid), dim3(kThreads), 0, s, p);
+    return dispatch_types(p.xbf, p.mbf, p.hbf, [&](auto xb, auto mb, auto hb) {
+      const auto launch = [&](auto zb) {
+        constexpr bool X = decltype(xb)::value, M = decltype(mb)::value, H = decltype(hb)::value, Z = decltype(zb)::value;
+        if (jvp) return launch_kernel(residual_ln_modulate_fwd_kernel<NV, true, X, M, H, Z>, dim3(grid), dim3(kThreads), 0, s, p);
+        return launch_kernel(residual_ln_modulate_fwd_kernel<NV, false, X, M, H, Z>, dim3(grid), dim3(kThreads), 0, s, p);
+      };
+      return p.zbf ? launch(std::true_type{}) : launch(std::false_type{});
+    });
   });
 }
 
