@@ -252,6 +252,7 @@ int launch_fwd_generic(const FwdParams& p, int BH, int D, ElemType type, bool jv
 }
 
 int launch_fwd(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream) {
+  if (fwd_small_grid(p.Lq, p.Lkv, D, BH, type, jvp)) return launch_fwd_small(p, BH, D, type, jvp, stream);
   if (type == ElemType::bf16) {
     const int rc = launch_fwd_bf16_fast(p, BH, D, jvp, stream);
     if (rc != 1) return rc;   // 1 = no tuned kernel for this shape

@@ -627,9 +627,26 @@ static int launch_fast_t(const FwdParams& p, int BH, hipStream_t stream) {
 //   * other head dims, N <= 256: 4 waves win only where 8-wave work-groups would run in two or three rounds
 //     (B32 H16: 0.0438 -> 0.0413 ms, B48: 0.070 -> 0.062) and lose 2-3 % from four rounds on;
 //   * without tangents the 8-wave kernel fits twice per CU and is slower only at head dim 64 on large grids.
+// and, whatever the head dim up to 80 and with or without tangents, from the number of work-groups:
+//   * 128-row work-groups that get a CU each win (a wave has its SIMD to itself): N256 BH64 D72 15.8 -> 14.1 us with tangents,
+//     N512 BH64 D64 13.9 -> 12.4 / 23.7 -> 21.4;
+//   * so they do where 256-row ones pad the sequence more or leave a last round nearly empty.  With W the time of one 256-row
+//     work-group on a CU, n of them take ceil(n / CUs) W; 128-row ones take about W per two on a CU, 0.88 W for a lone one, and
+//     5 % more throughout: N333 BH320 D72 28.1 -> 23.2 / 61.5 -> 48.0, N333 BH768 56.2 -> 45.4 / 137.5 -> 118.8, N768 BH96
+//     29.9 -> 27.7 / 70.1 -> 64.8, N256 BH320 D64 15.1 -> 13.9 / 30.7 -> 26.5; the comparison leaves the 256-row ones where they
+//     win (N333 BH96 D72 11.3 against 12.1, N1024 BH64 54.4 against 59.1 with tangents).
+static bool narrow_fills_better(int Lq, int BH, int cus) {
+  const int64_t wide = (int64_t)BH * ((Lq + 255) / 256), narrow = (int64_t)BH * ((Lq + 127) / 128), slots = 2 * (int64_t)cus;
+  if (narrow <= cus) return true;
+  const int64_t rest = narrow % slots;
+  const double narrow_cost = 1.05 * ((double)(narrow / slots) + (rest == 0 ? 0. : 2 * rest <= slots ? 0.88 : 1.));
+  return narrow_cost < (double)((wide + cus - 1) / cus);
+}
+
 static bool fwd_wide_workgroups(int Lq, int D, bool jvp, int BH) {
   if (Lq <= 128) return false;
   const int cus = compute_units();
+  if (D <= 80 && narrow_fills_better(Lq, BH, cus)) return false;
   // (without tangents only head dim 64 on a grid of at least eight narrow work-groups per CU prefers them:
   //  B256 H16 N256 0.129 -> 0.123 ms, B64 N1024 0.331 -> 0.326; the DMFT-B/2 call B64 H12 N256 is equal either way)
   if (!jvp) return !(D == 64 && (int64_t)BH * ((Lq + 127) / 128) >= 8 * (int64_t)cus);

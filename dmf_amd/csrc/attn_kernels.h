@@ -105,6 +105,11 @@ int launch_fwd(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipSt
 // and the tuned bf16 kernels (returns 1 when it has no kernel for the case).
 int launch_fwd_generic(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream);
 int launch_fwd_bf16_fast(const FwdParams& p, int BH, int D, bool jvp, hipStream_t stream);
+// Forward for grids that do not fill the device (bf16, with or without the in-kernel norms, and fp16): the policy, the launch,
+// and the kernel's name as profilers print it.
+bool fwd_small_grid(int Lq, int Lkv, int D, int BH, ElemType type, bool jvp);
+int launch_fwd_small(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream);
+void plan_fwd_small(int D, bool jvp, bool norm, ElemType type, char* buf, size_t n);
 int launch_bwd_generic(const BwdParams& p, int BH, int D, ElemType type, hipStream_t stream);
 int launch_bwd_bf16_fast(const BwdParams& p, int BH, int D, hipStream_t stream);
 int launch_bwd(const BwdParams& p, int BH, int D, ElemType type, hipStream_t stream);

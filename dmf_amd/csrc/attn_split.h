@@ -139,7 +139,7 @@ struct TileLoad {
       const int v = tid + it * 64 * NW, row = v / C::VPR, cv = v % C::VPR;
       if (v < 32 * C::VPR) {
         char* dst = tile + (row * C::P + cv) * 16;
-        if constexpr (SplitType<T>::F16) {
+        if constexpr (sizeof(T) == 2) {   // one plane, as it is
           *reinterpret_cast<u32x4*>(dst) = r[it][0];
         } else {
           float x[8];
@@ -168,7 +168,7 @@ __device__ __forceinline__ void load_own_row(const T* base, int64_t row_stride, 
     const bool in = row < nrows && 2 * c + g < C::VPR;
     const u32x4* p = reinterpret_cast<const u32x4*>(base + (int64_t)row * row_stride + 16 * c + 8 * g);
     const u32x4 a = in ? p[0] : u32x4{0, 0, 0, 0};
-    if constexpr (SplitType<T>::F16) {
+    if constexpr (sizeof(T) == 2) {   // one plane, as it is (16 bytes of the row per chunk and half)
       out[c][0] = a;
     } else {
       const u32x4 b = in ? p[1] : u32x4{0, 0, 0, 0};

@@ -141,6 +141,11 @@ int dmf_attn_plan(int entry, int B, int H, int Lq, int Lkv, int D, int dtype, ch
   }
   const bool jvp = entry == DMF_ATTN_PLAN_FWD_JVP || entry == DMF_ATTN_PLAN_FWD_QNORM_JVP || entry == DMF_ATTN_PLAN_FWD_QKNORM_JVP;
   const bool qn = entry >= DMF_ATTN_PLAN_FWD_QNORM_JVP, kn = entry == DMF_ATTN_PLAN_FWD_QKNORM_JVP;
+  if (qn && !bf16) return DMF_ATTN_ENOKERNEL;
+  if (dmf::fwd_small_grid(Lq, Lkv, D, B * H, static_cast<dmf::ElemType>(dtype), jvp)) {
+    dmf::plan_fwd_small(D, jvp, qn, static_cast<dmf::ElemType>(dtype), buf, n);
+    return DMF_ATTN_OK;
+  }
   if (bf16 && dmf::plan_fwd_bf16_fast(Lq, D, jvp, B * H, qn, kn, buf, n)) return DMF_ATTN_OK;
   if (qn) return DMF_ATTN_ENOKERNEL;
   snprintf(buf, n, "dmf::attn_fwd_kernel<%s, %d, %s>", t, D, jvp ? "true" : "false");

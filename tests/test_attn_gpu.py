@@ -826,3 +826,30 @@ def test_fp32_kernels_keep_fp32_products(Lq, Lkv, D):
     got = (o, to, *_lib.bwd(do, q, k, v, o, lse, scale))
     for name, a, r in zip(("o", "to", "dq", "dk", "dv"), got, _split_reference(q, k, v, tq, tk, tv, do)):
         assert ao.rel_l2(a.double().cpu(), r) <= 4e-6 or float(r.norm()) < 1e-9, (name, ao.rel_l2(a.double().cpu(), r))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L,D", [(97, 72), (128, 64), (129, 80), (160, 72), (255, 64), (333, 72), (512, 64), (130, 96), (200, 128)])
+def test_small_grid_and_tuned_forward_against_the_oracle(L, D, dtype):
+    """The same two batch elements once alone (few work-groups: the kernel that splits the keys over its waves) and once at the head of a
+    batch that fills the device (the tuned kernels, in the work-group width their policy picks), each against the fp32 oracle: lengths at the
+    edges of 32-row blocks and of 128- / 256-row work-groups."""
+    H, big = 2, 340
+    g = torch.Generator(device=DEV).manual_seed(L + D)
+    x = [torch.randn(big, L, H, D, generator=g, device=DEV).to(dtype) for _ in range(6)]
+    scale = D ** -0.5
+    half = dtype == torch.float16
+    fwd_jvp, fwd = (_lib.fwd_jvp_half, _lib.fwd_half) if half else (_lib.fwd_jvp, _lib.fwd)
+    if not half:
+        assert "small" in _lib.plan("fwd", 2, H, L, L, D) and "small" not in _lib.plan("fwd", big, H, L, L, D)
+    f = lambda t: t[:2].float().cpu()
+    o_ref, to_ref = ao.base_attn_jvp(*map(f, x))
+    lse_ref = ao.lse_ref(f(x[0]), f(x[1]), scale)
+    tol, lse_tol = (1e-3, 1e-5) if half else (2e-2, 2e-3)
+    for batch in (2, big):
+        a = [t[:batch] for t in x]
+        o, to, lse = fwd_jvp(*a, scale)
+        o2, lse2 = fwd(*a[:3], scale)
+        for name, got, ref, t in (("o", o, o_ref, tol), ("to", to, to_ref, tol), ("o primal", o2, o_ref, tol), ("lse", lse, lse_ref, lse_tol),
+                                  ("lse primal", lse2, lse_ref, lse_tol)):
+            assert ao.rel_l2(f(got), ref) <= t, (batch, name, ao.rel_l2(f(got), ref))
