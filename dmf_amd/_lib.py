@@ -102,9 +102,10 @@ def host():
     return _host_module
 
 
-def native(t) -> bool:
-    """True where an operator call on ``t`` may try the native host path: a GPU tensor outside of torch.compile's tracing."""
-    return t.is_cuda and not torch.compiler.is_compiling()
+def native(t, *others) -> bool:
+    """True where an operator call on these operands may try the native host path: GPU tensors, none of a class with a
+    ``__torch_function__`` of its own, outside of torch.compile's tracing."""
+    return t.is_cuda and not torch.compiler.is_compiling() and not torch.overrides.has_torch_function((t, *others))
 
 
 def _check(rc: int, what: str) -> None:

@@ -289,7 +289,7 @@ def dual_linear(x, weight, bias=None, w_lp=None, b_lp=None):
     (weight and bias are constants of the tangent map).  ``w_lp`` / ``b_lp``: optional
     copies of the parameters in the autocast dtype, used instead of casting per call
     (the caller guarantees they are current)."""
-    if _lib.native(x):
+    if _lib.native(x, weight, bias):
         out = _lib.host().linear(x, weight, bias, w_lp, b_lp)
         if out is not None:
             return out
@@ -304,7 +304,7 @@ def linear_gelu_tanh(x, weight, bias, w_lp=None, b_lp=None):
     the activation rides in the GEMM's epilogue (one library call, the pre-activation
     never reaches HBM); otherwise the pre-activation is needed for the tangent and for
     the backward pass and this is ``dual_linear`` followed by ``gelu_tanh``."""
-    if bias is not None and not torch.is_grad_enabled() and _lib.native(x):
+    if bias is not None and not torch.is_grad_enabled() and _lib.native(x, weight, bias):
         out = _lib.host().linear_gelu_inference(x, weight, bias, w_lp, b_lp)
         if out is not None:
             return out
@@ -329,7 +329,7 @@ def ln_modulate(x, shift, scale, eps: float = 1e-6):
     (B, C) or (B, 1, C); LayerNorm over C without affine parameters.  Under
     autocast the result is produced directly in the autocast dtype (it only ever
     feeds a Linear, which would cast it)."""
-    if _lib.native(x):
+    if _lib.native(x, shift, scale):
         out = _lib.host().ln_modulate(x, shift, scale, eps)
         if out is not None:
             return out
@@ -341,7 +341,7 @@ def ln_modulate(x, shift, scale, eps: float = 1e-6):
 def gate_residual(x, gate, h):
     """``x + gate * h`` for x, h (B, L, C) and gate (B, C) or (B, 1, C); the result
     has the promoted dtype of x and h (the fp32 residual stream under autocast)."""
-    if _lib.native(x):
+    if _lib.native(x, gate, h):
         out = _lib.host().gate_residual(x, gate, h)
         if out is not None:
             return out
@@ -356,7 +356,7 @@ def gate_residual(x, gate, h):
 def residual_ln_modulate(x, gate, h, shift, scale, eps: float = 1e-6):
     """``y = x + gate * h`` and ``z = LayerNorm(y) * (1 + scale) + shift`` in one pass;
     returns ``(y, z)`` with the dtypes ``gate_residual`` and ``ln_modulate`` would give."""
-    if _lib.native(x):
+    if _lib.native(x, gate, h, shift, scale):
         out = _lib.host().residual_ln_modulate(x, gate, h, shift, scale, eps)
         if out is not None:
             return out

@@ -9,8 +9,8 @@
 // level it hangs on the level's wrapper tensor.  In both cases it is read here without dispatching anything, the kernels
 // receive primals and tangents as plain buffers, the autograd node (a KernelNode over the primal's variables) is built below the
 // level exactly like a built-in operator's, and the outputs are wrapped for the level and given their tangents.  Everything
-// else -- several levels, vmap, torch.func.grad, tensor subclasses, CPU tensors, operands a kernel cannot read in place --
-// returns None, and the caller takes the general Python route.
+// else -- several levels, vmap, torch.func.grad, tensor subclasses, dispatch and function modes, tracing, CPU tensors, operands a
+// kernel cannot read in place -- returns None, and the caller takes the general Python route.
 //
 // The kernels are reached through the C ABI of libdmf_attn.so, which this module links against.
 #include <torch/csrc/autograd/forward_grad.h>
@@ -20,11 +20,13 @@
 #include <torch/csrc/autograd/variable.h>
 #include <torch/extension.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/functorch/DynamicLayer.h>
 #include <ATen/functorch/TensorWrapper.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/Event.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 
@@ -61,6 +63,10 @@ constexpr int64_t kNoLevel = -1, kUnsupported = -2;
 
 // The one torch.func.jvp level that is active, kNoLevel, or kUnsupported.
 int64_t current_level() {
+  // whoever watches the calls (dispatch and function modes, torch.jit.trace) sees those of the general route
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
+      c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer))
+    return kUnsupported;
   const auto& stack = at::functorch::getDynamicLayerStack();
   if (stack.empty()) return kNoLevel;
   if (stack.size() == 1 && stack[0].key() == at::functorch::TransformType::Jvp) return stack[0].layerId();
@@ -83,6 +89,7 @@ struct Arg {
   Tensor var;    // the variable below the level: its gradient edge
   Tensor data;   // its buffer
   Tensor tan;    // tangent buffer or undefined
+  bool tan_grad = false;   // the tangent has history or is a leaf that asks for a gradient
   bool defined() const { return data.defined(); }
   bool grad() const { return var.defined() && var.requires_grad(); }
 };
@@ -91,7 +98,11 @@ Arg unpack(const Tensor& x) {
   Arg a;
   if (!x.defined()) return a;
   const Tensor& t = x._fw_grad(0);
-  if (t.defined()) a.tan = data_of(unwrap(t));
+  if (t.defined()) {
+    const Tensor tv = unwrap(t);
+    a.tan = data_of(tv);
+    a.tan_grad = tv.requires_grad();
+  }
   a.var = unwrap(x);
   a.data = data_of(a.var);
   return a;
@@ -106,6 +117,12 @@ bool plain_gpu(const Arg& a) {
 template <typename... A>
 bool any_grad(const A&... a) {
   return c10::GradMode::is_enabled() && (a.grad() || ...);
+}
+
+// Only tangents ask for a gradient (the operators have none for them): left to the general route.
+template <typename... A>
+bool only_tangents_want(const A&... a) {
+  return c10::GradMode::is_enabled() && !(a.grad() || ...) && (a.tan_grad || ...);
 }
 
 int code_of(const Tensor& t) {   // -1: none
@@ -135,12 +152,22 @@ at::ScalarType autocast_type(const Tensor& x) {
 
 // ---- autograd ------------------------------------------------------------------------------------------------------------
 
-// One operator call in the graph: saved tensors and a function (saved, output gradients, node) -> input gradients.
+[[noreturn]] void tangent_cotangent() {
+  C10_THROW_ERROR(NotImplementedError,
+                  "dmf_amd.block_ops: a gradient arrived at the tangent (JVP) output of a fused block operator; these operators back-propagate "
+                  "through the primal output only -- detach the JVP output (as DMFLoss does) or build the model with block_ops='torch'");
+}
+
+// One operator call in the graph: saved tensors and a function (saved, gradients of the primal outputs, node) -> input gradients.
+// Of a call with tangents, each output is followed by its tangent, which belongs to the node as well: a gradient that arrives
+// there is dropped by the attention operators and refused by the block operators, whose callers would miss its second-order terms.
 struct KernelNode : Node {
   using Fn = std::function<variable_list(KernelNode&, const std::vector<Tensor>&, const variable_list&)>;
   const char* label;
   std::vector<SavedVariable> saved;
   Fn fn;
+  bool dual = false, refuse_tangent_gradient = true;
+  bool torch_ops = false;   // fn can be made of differentiable, batchable calls (see plain_call)
   bool released = false;
 
   explicit KernelNode(const char* l) : label(l) {}
@@ -153,14 +180,33 @@ struct KernelNode : Node {
     s.reserve(saved.size());
     for (auto& v : saved) s.push_back(v.unpack(shared_from_this()));
     const size_t n = num_outputs();
+    variable_list primal;
     bool any = false;
-    for (const auto& g : grads) any = any || g.defined();
+    for (size_t i = 0; i < grads.size(); ++i) {
+      if (dual && i % 2) {
+        if (refuse_tangent_gradient && grads[i].defined()) tangent_cotangent();
+        continue;
+      }
+      any = any || grads[i].defined();
+      primal.push_back(std::move(grads[i]));
+    }
     if (!any) return variable_list(n);
     c10::OptionalDeviceGuard device(s[0].device());
-    Below below;
-    variable_list out = fn(*this, s, grads);
+    std::optional<Below> below;
+    if (!torch_ops || plain_call(primal)) below.emplace();
+    variable_list out = fn(*this, s, primal);
     out.resize(n);
     return out;
+  }
+  // False under create_graph=True and for batched gradients: there, what consists of torch operators stays differentiable and
+  // mapped, as autograd.Function's backward is.
+  static bool plain_call(const variable_list& grads) {
+    if (c10::GradMode::is_enabled()) return false;
+    for (const Tensor& g : grads)
+      if (g.defined() && g.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                                                 c10::DispatchKey::Batched, c10::DispatchKey::Python})))
+        return false;
+    return true;
   }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -183,6 +229,10 @@ std::shared_ptr<KernelNode> make_node(const char* name, std::initializer_list<Ar
 // Output for the caller: history, level wrapper, tangent.
 Tensor finish(Tensor out, const Tensor& tan, const std::shared_ptr<KernelNode>& node, int64_t level) {
   if (node) torch::autograd::set_history(out, node);
+  if (node && tan.defined()) {
+    node->dual = true;
+    torch::autograd::set_history(tan, node);
+  }
   Tensor res = level >= 0 ? at::functorch::makeTensorWrapper(out, level) : out;
   if (tan.defined()) {
     auto* meta = torch::autograd::impl::materialize_autograd_meta(res);
@@ -297,6 +347,7 @@ py::object attention(const Tensor& q_, const Tensor& k_, const Tensor& v_, std::
     return none();
   for (const Arg* a : {&q, &k, &v})
     if (!readable(a->data) || (a->tan.defined() && !readable(a->tan))) return none();
+  if (only_tangents_want(q, k, v)) return none();
   c10::OptionalDeviceGuard device(q.data.device());
   AttnShape s{(int)q.data.size(0), (int)q.data.size(2), (int)q.data.size(1), (int)k.data.size(1), (int)D, code,
               (float)(scale ? *scale : 1.0 / std::sqrt((double)D))};
@@ -317,6 +368,7 @@ py::object attention(const Tensor& q_, const Tensor& k_, const Tensor& v_, std::
   std::shared_ptr<KernelNode> node;
   if (grad) {
     node = make_node("FlashAttnBackward", {q, k, v}, {q.data, k.data, v.data, data_of(r.o), r.lse});
+    node->refuse_tangent_gradient = false;
     node->fn = [s](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
       const Tensor dout = prepared(g[0]);
       variable_list out{dense_like(sv[0]), dense_like(sv[1]), dense_like(sv[2])};
@@ -369,7 +421,7 @@ Tensor heads_of(const Tensor& dout, const AttnShape& s) {   // the gradient of t
 py::object attention_packed(const Tensor& qkv, int64_t heads, std::optional<double> scale) {
   const int64_t level = current_level();
   Packed p;
-  if (level == kUnsupported || !unpack_packed(qkv, heads, p)) return none();
+  if (level == kUnsupported || !unpack_packed(qkv, heads, p) || only_tangents_want(p.a)) return none();
   c10::OptionalDeviceGuard device(p.qkv.device());
   p.s.scale = (float)(scale ? *scale : 1.0 / std::sqrt((double)p.s.D));
   const bool grad = any_grad(p.a);
@@ -388,11 +440,13 @@ py::object attention_packed(const Tensor& qkv, int64_t heads, std::optional<doub
   }
   std::shared_ptr<KernelNode> node;
   if (grad) {
-    node = make_node("FlashAttnQKVPackedBackward", {p.a}, {p.qkv, data_of(r.o), r.lse});
+    // (the argument itself is saved, not a view of it: in-place changes to it are noticed)
+    node = make_node("FlashAttnQKVPackedBackward", {p.a}, {p.a.data, data_of(r.o), r.lse});
+    node->refuse_tangent_gradient = false;
     node->fn = [s = p.s, shape = p.a.data.sizes().vec()](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
       const Tensor dout = heads_of(g[0], s), o = sv[1].view({s.B, s.Lq, s.H, s.D});
       const Tensor gqkv = empty({s.B, s.Lq, 3, s.H, s.D}, sv[0].scalar_type(), sv[0]);
-      attn_backward(s, dout, slots(sv[0]), o, sv[2], slots(gqkv));
+      attn_backward(s, dout, slots(sv[0].view(gqkv.sizes())), o, sv[2], slots(gqkv));
       return {gqkv.view(shape)};
     };
   }
@@ -415,6 +469,7 @@ py::object attention_qknorm_packed(const Tensor& qkv, const Tensor& qg_, const T
   for (const Arg* g : {&qg, &kg})
     if (!plain_gpu(*g) || g->tan.defined() || g->data.dim() != 1 || g->data.size(0) != D || !block_dtype(g->data) || g->data.device() != p.qkv.device())
       return none();
+  if (only_tangents_want(p.a, qg, kg)) return none();
   c10::OptionalDeviceGuard device(p.qkv.device());
   p.s.scale = (float)(scale ? *scale : 1.0 / std::sqrt((double)D));
   const AttnShape& s = p.s;
@@ -455,14 +510,15 @@ py::object attention_qknorm_packed(const Tensor& qkv, const Tensor& qg_, const T
   }
   std::shared_ptr<KernelNode> node;
   if (grad) {
-    node = make_node("QKNormAttnQKVPackedBackward", {p.a, qg, kg}, {p.qkv, gq, gk, qh, kh, data_of(r.o), r.lse});
+    node = make_node("QKNormAttnQKVPackedBackward", {p.a, qg, kg}, {p.a.data, gq, gk, qh, kh, data_of(r.o), r.lse});
+    node->refuse_tangent_gradient = false;
     node->fn = [s, eps, shape = p.a.data.sizes().vec(), tq = qg.data.scalar_type(), tk = kg.data.scalar_type()](
                    KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
       const Tensor dout = heads_of(g[0], s), o = sv[5].view({s.B, s.Lq, s.H, s.D});
       const Tensor gqkv = empty({s.B, s.Lq, 3, s.H, s.D}, sv[0].scalar_type(), sv[0]);
       const Tensor dgq = empty({s.D}, at::kFloat, o), dgk = empty({s.D}, at::kFloat, o), delta = empty({s.B, s.H, s.Lq}, at::kFloat, o);
       const Tensor ws = workspace(dmf_attn_bwd_qknorm_workspace_floats(s.B, s.H, s.Lq, s.Lkv, s.D), o);
-      const QKV raw = slots(sv[0]), grad = slots(gqkv);
+      const QKV raw = slots(sv[0].view(gqkv.sizes())), grad = slots(gqkv);
       const Operand od(dout), oqh(sv[3]), okh(sv[4]), oo(o);
       const Strides st{&od, &oqh, &okh, &raw.v, &oo, &grad.q, &grad.k, &grad.v, &raw.q, &raw.k};
       check(dmf_attn_bwd_qknorm(od.p, oqh.p, okh.p, raw.v.p, oo.p, static_cast<const float*>(ptr(sv[6])), raw.q.p, raw.k.p,
@@ -544,12 +600,6 @@ variable_list gate_backward(const Tensor& gy_, const Tensor& gate_, const Tensor
   return {gh, gg};
 }
 
-[[noreturn]] void tangent_cotangent() {
-  C10_THROW_ERROR(NotImplementedError,
-                  "dmf_amd.block_ops: a gradient arrived at the tangent (JVP) output of a fused block operator; these operators back-propagate "
-                  "through the primal output only -- detach the JVP output (as DMFLoss does) or build the model with block_ops='torch'");
-}
-
 py::object ln_modulate(const Tensor& x_, const Tensor& shift_, const Tensor& scale_, double eps) {
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
@@ -558,6 +608,7 @@ py::object ln_modulate(const Tensor& x_, const Tensor& shift_, const Tensor& sca
   const Blc n(x.data);
   const auto out_t = autocast_type(x.data);
   if (!mods_ok(n.B, n.C, sh, sc) || sh.data.device() != x.data.device() || (out_t != at::kFloat && out_t != at::kBFloat16)) return none();
+  if (only_tangents_want(x, sh, sc)) return none();
   c10::OptionalDeviceGuard device(x.data.device());
   const bool dual = x.tan.defined() || sh.tan.defined() || sc.tan.defined();
   Tensor y, ty, xd;
@@ -601,6 +652,7 @@ py::object gate_residual(const Tensor& x_, const Tensor& gate_, const Tensor& h_
   if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !promote(x, h)) return none();
   const Blc n(x.data);
   if (!mods_ok(n.B, n.C, gate) || gate.data.device() != x.data.device() || h.data.device() != x.data.device()) return none();
+  if (only_tangents_want(x, gate, h)) return none();
   c10::OptionalDeviceGuard device(x.data.device());
   const bool dual = x.tan.defined() || gate.tan.defined() || h.tan.defined();
   Tensor y, ty, hd;
@@ -636,7 +688,7 @@ py::object residual_ln_modulate(const Tensor& x_, const Tensor& gate_, const Ten
   const Blc n(x.data);
   const auto out_t = autocast_type(x.data);
   if (!mods_ok(n.B, n.C, gate, sh, sc) || gate.data.device() != x.data.device() || h.data.device() != x.data.device() ||
-      (out_t != at::kFloat && out_t != at::kBFloat16))
+      (out_t != at::kFloat && out_t != at::kBFloat16) || only_tangents_want(x, gate, h, sh, sc))
     return none();
   c10::OptionalDeviceGuard device(x.data.device());
   const bool dual = x.tan.defined() || gate.tan.defined() || h.tan.defined() || sh.tan.defined() || sc.tan.defined();
@@ -684,7 +736,7 @@ py::object activation(const Tensor& x_, Act act) {
   const Arg x = unpack(x_);
   if (!plain_gpu(x) || !block_dtype(x.data) || x.data.numel() == 0 || x.data.numel() % 8) return none();
   const auto out_t = act == Act::silu ? autocast_type(x.data) : x.data.scalar_type();
-  if (out_t != at::kFloat && out_t != at::kBFloat16) return none();
+  if ((out_t != at::kFloat && out_t != at::kBFloat16) || only_tangents_want(x)) return none();
   c10::OptionalDeviceGuard device(x.data.device());
   Tensor xd, y, ty;
   {
@@ -742,15 +794,24 @@ Tensor column_sum(const Tensor& x, at::ScalarType dt) {
 }
 
 // DualLinearFunc.backward: the parameter gradients on the side stream next to the input gradient.
-variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w, const Tensor& gy, at::ScalarType x_type, at::ScalarType w_type,
-                              at::ScalarType b_type, bool has_bias, const std::vector<int64_t>& x_shape) {
-  Tensor g2 = gy.reshape({-1, gy.size(-1)}).to(w.scalar_type());
+variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w, const Tensor& gy, at::ScalarType w_type, at::ScalarType b_type,
+                              bool has_bias) {
+  const Tensor g2 = gy.reshape({-1, gy.size(-1)}).to(w.scalar_type()), x2 = x.reshape({-1, x.size(-1)}).to(w.scalar_type());
   const bool want_gx = node.wants(0), want_gw = node.wants(1), want_gb = has_bias && node.wants(2), fork = want_gx && (want_gw || want_gb);
   Tensor gx, gw, gb;
+  if (!KernelNode::plain_call({gy})) {   // differentiated again or mapped over: operators that can be
+    if (want_gx) gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
+    if (want_gw) {
+      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = at::mm(g2.t().to(at::kFloat), x2.to(at::kFloat));
+      else gw = at::mm(g2.t(), x2).to(w_type);
+    }
+    if (want_gb) gb = g2.sum(at::IntArrayRef{0}, false, at::kFloat).to(b_type);
+    return {gx, gw, gb};
+  }
   auto parameters = [&] {
     if (want_gw) {
-      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = at::mm(g2.t(), x, at::kFloat);   // the GEMM stores its fp32 accumulators
-      else gw = at::mm(g2.t(), x).to(w_type);
+      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = at::mm(g2.t(), x2, at::kFloat);   // the GEMM stores its fp32 accumulators
+      else gw = at::mm(g2.t(), x2).to(w_type);
     }
     if (want_gb) gb = column_sum(dense(g2), b_type);
   };
@@ -769,13 +830,13 @@ variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w
     }
     joined.record(side);
     impl.exchangeStream(main);
-    gx = at::mm(g2, w).reshape(x_shape).to(x_type);
+    gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
     main.wait(joined);
     for (const Tensor* t : {&gw, &gb})   // allocated on the side stream, consumed (and later freed) on the main one
       if (t->defined()) t->record_stream(main);
   } else {
     parameters();
-    if (want_gx) gx = at::mm(g2, w).reshape(x_shape).to(x_type);
+    if (want_gx) gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
   }
   return {gx, gw, gb};
 }
@@ -812,12 +873,12 @@ py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
   const Arg x = unpack(x_), weight = unpack(weight_), bias = unpack(bias_);
-  if (!linear_ok(x, weight, bias)) return none();
+  if (!linear_ok(x, weight, bias) || only_tangents_want(x, weight, bias)) return none();
   const bool grad = any_grad(x, weight, bias);
   // (a bias gradient of another width goes through torch's column sum, whose replay from a captured graph the general route refuses)
   if (grad && bias.grad() && weight.data.size(0) % 8) return none();
   c10::OptionalDeviceGuard device(x.data.device());
-  Tensor y, ty, x2;
+  Tensor y, ty;
   LinearOperands o;
   const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
   const at::ScalarType dt = autocast_type(x.data);
@@ -828,16 +889,18 @@ py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias
     const int64_t K = x.data.size(-1);
     auto sizes = x.data.sizes().vec();
     sizes.back() = o.w.size(0);
-    x2 = x.data.reshape({-1, K}).to(o.dt);
+    const Tensor x2 = x.data.reshape({-1, K}).to(o.dt);
     y = (o.b.defined() ? at::addmm(o.b, x2, o.w.t()) : at::mm(x2, o.w.t())).view(sizes);
     if (x.tan.defined()) ty = at::mm(x.tan.reshape({-1, K}).to(o.dt), o.w.t()).view(sizes);
   }
   std::shared_ptr<KernelNode> node;
   if (grad) {
-    node = make_node("DualLinearBackward", {x, weight, bias}, {x2, o.w});
-    node->fn = [xs = x.data.sizes().vec(), xt = x.data.scalar_type(), wt = weight.data.scalar_type(), has_bias = bias.defined(),
-                bt = bias.defined() ? bias.data.scalar_type() : at::kFloat](KernelNode& node, const std::vector<Tensor>& sv, const variable_list& g) {
-      return linear_backward(node, sv[0], sv[1], g[0], xt, wt, bt, has_bias, xs);
+    // the variables themselves, for create_graph=True; a low-precision copy of the weight is a constant
+    node = make_node("DualLinearBackward", {x, weight, bias}, {x.var, o.w.is_same(weight.data) ? weight.var : o.w});
+    node->torch_ops = true;
+    node->fn = [wt = weight.data.scalar_type(), has_bias = bias.defined(), bt = bias.defined() ? bias.data.scalar_type() : at::kFloat](
+                   KernelNode& node, const std::vector<Tensor>& sv, const variable_list& g) {
+      return linear_backward(node, sv[0], sv[1], g[0], wt, bt, has_bias);
     };
   }
   return py::cast(finish(y, ty, node, level));
@@ -865,7 +928,7 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
   const Arg x = unpack(x_);
-  if (!plain_gpu(x) || x.data.dim() < 1 || x.data.size(-1) % n) return none();
+  if (!plain_gpu(x) || x.data.dim() < 1 || x.data.size(-1) % n || only_tangents_want(x)) return none();
   std::vector<Tensor> parts, tparts;
   const int64_t w = x.data.size(-1) / n;
   {
@@ -876,6 +939,7 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
   std::shared_ptr<KernelNode> node;
   if (any_grad(x)) {
     node = make_node("ChunkBackward", {x}, {parts[0]});
+    node->torch_ops = true;
     node->fn = [n](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
       std::vector<Tensor> parts;
       for (int64_t i = 0; i < n; ++i) parts.push_back(g[i].defined() ? g[i] : at::zeros_like(sv[0], at::MemoryFormat::Contiguous));

@@ -156,7 +156,7 @@ def flash_attn_func(q, k, v, softmax_scale=None):
     (fp32 accumulation and softmax, nothing rounded to fp16 before the result); with
     k, v of another type next to an fp16 q everything is computed in fp32 and rounded back.
     """
-    if _lib.native(q):
+    if _lib.native(q, k, v):
         out = _lib.host().attention(q, k, v, softmax_scale)
         if out is not None:
             return out
@@ -339,7 +339,7 @@ def flash_attn_qknorm_qkvpacked_func(qkv, q_gain, k_gain, eps: float = 1e-6, sof
     Dual in -> dual out; the gains are constants of the tangent map."""
     if qkv.dim() != 5 or qkv.shape[2] != 3:
         raise ValueError(f"expected a packed (B, L, 3, H, D) tensor, got shape {tuple(qkv.shape)}")
-    if IN_KERNEL_Q_NORM and _lib.native(qkv):
+    if IN_KERNEL_Q_NORM and _lib.native(qkv, q_gain, k_gain):
         out = _lib.host().attention_qknorm_packed(qkv, q_gain, k_gain, 0, eps, softmax_scale, K_NORM_IN_KERNEL_MAX_LQ if IN_KERNEL_K_NORM else 0)
         if out is not None:
             return out
@@ -364,7 +364,7 @@ def flash_attn_qknorm_qkvpacked_func(qkv, q_gain, k_gain, eps: float = 1e-6, sof
 def flash_attn_projection(qkv, num_heads: int, q_gain=None, k_gain=None, eps: float = 1e-6):
     """Attention on a projection output (B, L, 3 C) with ``num_heads`` heads, returns (B, L, C): the packed operators above
     (with gains: the q/k-norm one) without a reshape on either side."""
-    if _lib.native(qkv):
+    if _lib.native(qkv, q_gain, k_gain):
         if q_gain is None:
             out = _lib.host().attention_packed(qkv, num_heads, None)
         elif IN_KERNEL_Q_NORM:

@@ -3,10 +3,12 @@ gradients -- in every way an operator is differentiated; and the cases it hands 
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import dmf_amd
 from dmf_amd import _lib, block_ops, harness
 from dmf_amd.dmft import DMFT
+from dmf_amd.flash_attention_hip_jvp import flash_attn_projection
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -14,7 +16,7 @@ DEV = "cuda:0"
 
 def _general(fn):
     """``fn()`` with the native path switched off."""
-    native, _lib.native = _lib.native, lambda t: False
+    native, _lib.native = _lib.native, lambda *t: False
     try:
         return fn()
     finally:
@@ -111,3 +113,73 @@ def test_what_the_native_path_hands_back():
         z.mul_(2.0)             # and modifying one in place is caught
         with pytest.raises(RuntimeError, match="inplace"):
             y.sum().backward()
+
+
+def test_gradients_at_tangent_outputs():
+    """Attention drops them, the block operators refuse them -- attached to a loss together with the primal output or alone."""
+    q, t = torch.randn(2, 16, 2, 64, device=DEV, requires_grad=True), torch.randn(2, 16, 2, 64, device=DEV)
+    o, to = torch.func.jvp(lambda x: dmf_amd.flash_attn_func(x, x, x), (q,), (t,))
+    assert to.requires_grad
+    both, alone = torch.autograd.grad((o.sum() + to.sum()), q, retain_graph=True)[0], torch.autograd.grad(o.sum(), q)[0]
+    assert torch.equal(both, alone)
+    x, tx = torch.randn(2, 8, 64, device=DEV, requires_grad=True), torch.randn(2, 8, 64, device=DEV)
+    m, w = torch.randn(2, 64, device=DEV), torch.randn(128, 64, device=DEV)
+    for fn in (lambda x: block_ops.ln_modulate(x, m, m), lambda x: block_ops.gate_residual(x, m, x), block_ops.gelu_tanh, block_ops.silu,
+               lambda x: block_ops.residual_ln_modulate(x, m, x, m, m)[0], lambda x: block_ops.residual_ln_modulate(x, m, x, m, m)[1],
+               lambda x: block_ops.dual_linear(x, w), lambda x: block_ops.chunk_last(x, 2)[1]):
+        y, ty = torch.func.jvp(fn, (x,), (tx,))
+        torch.autograd.grad(y.sum(), x, retain_graph=True)
+        with pytest.raises(NotImplementedError, match="primal output only"):
+            (y.sum() + ty.sum()).backward()
+        # only the tangent asks for a gradient: none, and no error, as on the general route
+        _, ty = torch.func.jvp(fn, (x.detach(),), (tx.clone().requires_grad_(),))
+        assert ty.requires_grad
+
+
+@pytest.mark.parametrize("op", ["packed", "qknorm", "linear"])
+def test_in_place_changes_of_reshaped_operands_are_noticed(op):
+    gains = torch.ones(64, device=DEV)
+    x = torch.randn(2, 16, 3 * 128, device=DEV, requires_grad=True)
+    z = (x * 1.0).to(torch.bfloat16)
+    if op == "linear":
+        y = block_ops.dual_linear(z, torch.randn(64, 384, device=DEV, dtype=torch.bfloat16, requires_grad=True))
+    else:
+        y = flash_attn_projection(z, 2, *((gains, gains) if op == "qknorm" else ()))
+    z.mul_(2.0)
+    with pytest.raises(RuntimeError, match="inplace"):
+        y.sum().backward()
+
+
+def test_linear_and_chunk_stay_twice_differentiable():
+    torch.manual_seed(1)
+    x = torch.randn(3, 5, 64, device=DEV, requires_grad=True)
+    w, b = torch.randn(32, 64, device=DEV, requires_grad=True), torch.randn(32, device=DEV, requires_grad=True)
+
+    def second(linear, chunk):
+        a, c = chunk(linear(x, w, b), 2)
+        gx, gw, gb = torch.autograd.grad((a * c).sum(), (x, w, b), create_graph=True)
+        return torch.autograd.grad(gx.square().sum() + gw.square().sum() + gb.square().sum(), (x, w))
+
+    for got, exp in zip(second(block_ops.dual_linear, block_ops.chunk_last), second(torch.nn.functional.linear, lambda t, n: t.chunk(n, -1))):
+        # two library products of 64 to 480 terms in fp32, in another order
+        assert (got - exp).norm() <= 1e-5 * exp.norm()
+    g = torch.randn(4, 3, 5, 32, device=DEV)
+    batched = torch.autograd.grad(block_ops.dual_linear(x, w), (x, w), g, is_grads_batched=True)
+    for i in range(4):
+        for got, exp in zip(batched, torch.autograd.grad(block_ops.dual_linear(x, w), (x, w), g[i])):
+            assert (got[i] - exp).norm() <= 1e-5 * exp.norm()
+
+
+def test_watched_calls_take_the_general_route():
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Tagged(torch.Tensor):
+        pass
+
+    q = torch.randn(2, 16, 2, 64, device=DEV)
+    host = _lib.host()
+    with Watch():
+        assert host.attention(q, q, q, None) is None
+    assert _lib.native(q, None) and not _lib.native(q, q.as_subclass(Tagged)) and host.attention(q, q, q, None) is not None
