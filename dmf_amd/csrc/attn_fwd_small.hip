@@ -137,7 +137,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     if constexpr (F16) dOv.zero();
   }
   RowScale<T> gs;
-  float m_run = -INFINITY, l_run = 0.f, mu_run = 0.f;
+  float m_run = kLowestMax, l_run = 0.f, mu_run = 0.f;
   const float c2 = p.scale_log2;
   for (int it = wave; it < ntiles; it += NW) {
     if constexpr (NORM) {
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     }
   }
 
-  // ---- merge: every wave's state is brought to the largest maximum of the row (a wave without keys has m = -inf, l = 0)
+  // ---- merge: every wave's state is brought to the largest maximum of the row (a wave without keys has m = kLowestMax, l = 0)
   float* stat = reinterpret_cast<float*>(smem + S::STAT_OFF);   // [m | l | mu][wave][row]
   const float l_w = xhalf_sum(l_run), mu_w = JVP ? xhalf_sum(mu_run) : 0.f;
   if (g == 0) stat[wave * 32 + c32] = m_run;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
   float m = stat[c32];
 #pragma unroll
   for (int w = 1; w < NW; ++w) m = fmaxf(m, stat[w * 32 + c32]);
-  const float f = fast_exp2(m_run - m);   // m is finite: wave 0 always has a key
+  const float f = fast_exp2(m_run - m); 
   if (g == 0) {
     stat[(NW + wave) * 32 + c32] = l_w * f;
     stat[(2 * NW + wave) * 32 + c32] = mu_w * f;

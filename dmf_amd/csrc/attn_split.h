@@ -69,9 +69,13 @@ __device__ __forceinline__ void mma_planes16(f32x4& acc, const u32x4 (&a)[NA], c
   for_plane_pairs<NA, NB>([&](int i, int j) { mma_one16<T>(acc, a[i], b[j]); });
 }
 
-// Eight fp32 values as NP planes of eight 16-bit ones.
-template <typename T, int NP>
+// Eight fp32 values as NP planes of eight 16-bit ones.  ANY (operands as the caller gave them, in bf16 planes): all but the last
+// plane are held within the finite range, so that a value above the largest bf16 number does not round to infinity and an
+// infinity or NaN ends up in the last plane alone -- it then meets only the first plane of the other operand, whose sign is the
+// value's.
+template <typename T, bool ANY = false, int NP>
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
+  constexpr float kMax = 3.38953139e38f;   // the largest bf16 number
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float a = x[2 * i], b = x[2 * i + 1];
@@ -85,7 +89,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
           b -= (float)h[1];
         }
       } else {
-        const uint32_t h = pack_bf16x2(a, b);
+        const bool hold = ANY && k + 1 < NP;
+        const uint32_t h = hold ? pack_bf16x2(__builtin_amdgcn_fmed3f(a, -kMax, kMax), __builtin_amdgcn_fmed3f(b, -kMax, kMax)) : pack_bf16x2(a, b);
         pl[k][i] = h;
         if (k + 1 < NP) {
           a -= __uint_as_float(h << 16);
@@ -149,7 +154,7 @@ struct TileLoad {
             x[4 + e] = __uint_as_float(r[it][C::RAW - 1][e]);
           }
           u32x4 pl[SplitType<T>::NI];
-          split8<T>(x, pl);
+          split8<T, true>(x, pl);
 #pragma unroll
           for (int k = 0; k < SplitType<T>::NI; ++k) *reinterpret_cast<u32x4*>(dst + k * C::PLANE) = pl[k];
         }
@@ -178,7 +183,7 @@ __device__ __forceinline__ void load_own_row(const T* base, int64_t row_stride, 
         x[e] = __uint_as_float(a[e]);
         x[4 + e] = __uint_as_float(b[e]);
       }
-      split8<T>(x, out[c]);
+      split8<T, true>(x, out[c]);
     }
   }
 }
@@ -370,6 +375,10 @@ struct SplitStages {
   static_assert(STAGE <= 160 * 1024 && BYTES <= 160 * 1024, "LDS budget");
 };
 
+// Start of the running maximum (log2 units).  Finite, and above what keys masked by the lowest number of their type give, so that
+// a tile of nothing but such keys or of -inf scores weighs nothing: with its own maximum m subtracted, fma(S, c2, -m) would be the
+// rounding error of m, which is large where m is.
+constexpr float kLowestMax = -1e30f;
 constexpr float kSplitLazyLog2 = 6.0f;   // the running maximum is raised when exceeded by more than 2^6 (exact: normalised once at the end)
 
 template <typename T, int D, bool JVP, int NW>
@@ -415,7 +424,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     if constexpr (F16) dOv.zero();
   }
   RowScale<T> gs;
-  float m_run = -INFINITY, l_run = 0.f, mu_run = 0.f;
+  float m_run = kLowestMax, l_run = 0.f, mu_run = 0.f;
   const float c2 = p.scale_log2;
 
   const int ntiles = (p.Lkv + 31) / 32;

@@ -853,3 +853,26 @@ def test_small_grid_and_tuned_forward_against_the_oracle(L, D, dtype):
         for name, got, ref, t in (("o", o, o_ref, tol), ("to", to, to_ref, tol), ("o primal", o2, o_ref, tol), ("lse", lse, lse_ref, lse_tol),
                                   ("lse primal", lse2, lse_ref, lse_tol)):
             assert ao.rel_l2(f(got), ref) <= t, (batch, name, ao.rel_l2(f(got), ref))
+
+
+@pytest.mark.parametrize("dtype,L", [(torch.float32, 70), (torch.float16, 70), (torch.float16, 200), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("value", ["lowest", "-inf"])
+def test_keys_masked_by_extreme_values(dtype, L, value):
+    """Keys switched off through a feature of the type's lowest value or -inf (against a query feature of one), among them every key of the
+    first tile and so of one wave; values with an infinity and a NaN reach exactly the columns they stand in (fp16: an infinity meets
+    both parts of the probability, and the second is zero where the first is exact -- 0 inf = NaN -- so either may come out)."""
+    H, D = 2, 64
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(1, L, H, D, generator=g).to(dtype) for _ in range(3))
+    q[..., -1] = 1
+    off = torch.arange(L) < 40
+    k[:, off, :, -1] = torch.finfo(dtype).min if value == "lowest" else -float("inf")
+    v[0, 50, 0, 3], v[0, 51, 1, 5] = float("inf"), float("nan")
+    got = flash_attn_func(*(t.to(DEV) for t in (q, k, v))).double().cpu()
+    q64, k64, v64 = (t.double().transpose(1, 2) for t in (q, k, v))
+    ref = (torch.softmax(q64 @ k64.transpose(-1, -2) * D ** -0.5, -1) @ v64).transpose(1, 2)
+    assert torch.equal(torch.isfinite(got), torch.isfinite(ref)) and not torch.isinf(got[torch.isnan(ref)]).any()
+    assert dtype == torch.float16 or torch.equal(torch.isnan(got), torch.isnan(ref))
+    # (bf16: probabilities rounded to 8 bits before the second product)
+    tol = {torch.float32: 1e-5, torch.float16: 1e-3, torch.bfloat16: 2e-2}[dtype]
+    assert ao.rel_l2(got[torch.isfinite(ref)], ref[torch.isfinite(ref)]) <= tol
