@@ -120,7 +120,7 @@ def plan(entry: str, B: int, H: int, Lq: int, Lkv: int, D: int, dtype=torch.bflo
     """Name(s) of the kernel(s) the entry point ``entry`` launches for this shape on the current
     device, as profilers print them (``dmf_attn_plan``; host-only, launches nothing)."""
     buf = ctypes.create_string_buffer(256)
-    code = DMF_ATTN_BF16 if dtype == torch.bfloat16 else DMF_ATTN_F32
+    code = {torch.bfloat16: DMF_ATTN_BF16, torch.float16: DMF_ATTN_F16}.get(dtype, DMF_ATTN_F32)
     _check(load().dmf_attn_plan(PLAN_ENTRIES[entry], B, H, Lq, Lkv, D, code, buf, len(buf)), "dmf_attn_plan")
     return buf.value.decode()
 

@@ -14,6 +14,7 @@
 // Quantities follow models/triton_utils.py:92-118 of the reference (S, dS,
 // P*dS, mu = rowsum(P*dS), lse = m + log l) but the accumulators are kept
 // unnormalised and divided once in the epilogue.
+#include <cstdio>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -210,9 +211,35 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<T, D, JVP>())) void attn_f
   if constexpr (std::is_same<T, __bf16>::value) generic_fwd_body<T, D, JVP>(p);
   else split_fwd_body<T, D, JVP, 4>(p);
 }
-
+// The 8-wave form (SplitFwdPlan) exists where it was measured to win: 128 registers (two work-groups per CU) without tangents.
 template <typename T, int D, bool JVP>
-static int launch_fwd_t(const FwdParams& p, int BH, hipStream_t stream) {
+constexpr bool has_wide_split() {
+  return std::is_same<T, _Float16>::value ? (JVP ? D == 72 || D == 80 : D == 72) : std::is_same<T, float>::value && JVP && D == 64;
+}
+template <typename T, int D, bool JVP>
+__global__ __launch_bounds__(512, (JVP ? 2 : 4)) void attn_fwd_wide_kernel(const FwdParams p) {
+  split_fwd_body<T, D, JVP, 8>(p);
+}
+
+// Policy between the two forms, by the rounds their grids take: the 4-wave form has one (fp16 with tangents, fp32) or three (fp16
+// without) work-groups of 128 rows per CU, the 8-wave form one or two of 256 rows.  A round of the 8-wave form takes 1.1 to 1.2
+// (fp16) or 1.72 times (fp32 with tangents) one of the 4-wave form.  us, 4 -> 8 waves:
+//   fp16 + tangents D72, 16 heads: B4 N1024 156 -> 99, B32 N256 96 -> 62, B20 N256 71 -> 55, B16 N333 91 -> 70, B6 N512 84 -> 48;
+//     equal rounds lose: B2 N1024 84 -> 88, B8 N256 25 -> 28;
+//   fp32 + tangents D64: B4 N1024 270 -> 236, B32 N256 162 -> 138, B6 N512 134 -> 105; left alone: B20 N256 115 -> 119,
+//     B2 N1024 138 -> 185, B16 N333 150 -> 158;
+//   fp16 D72: B16 N512 48 -> 40, B16 N1024 153 -> 140, B32 N256 29.9 -> 28.5; left alone: B16 N333 26 -> 29, B6 N1024 62 -> 65.
+static bool wide_split(int Lq, int D, int BH, ElemType type, bool jvp) {
+  const int64_t cus = compute_units(), narrow = (int64_t)BH * ((Lq + 127) / 128), wide = (int64_t)BH * ((Lq + 255) / 256);
+  auto rounds = [](int64_t n, int64_t slots) { return (n + slots - 1) / slots; };
+  if (type == ElemType::f16 && jvp && (D == 72 || D == 80)) return rounds(wide, cus) < rounds(narrow, cus);
+  if (type == ElemType::f32 && jvp && D == 64) return 172 * rounds(wide, cus) < 100 * rounds(narrow, cus);
+  if (type == ElemType::f16 && !jvp && D == 72 && Lq >= 256) return rounds(wide, 2 * cus) < rounds(narrow, 3 * cus);
+  return false;
+}
+
+template <typename T, int D, bool JVP, int NW>
+static int launch_fwd_nw(const FwdParams& p, int BH, hipStream_t stream) {
   constexpr int smem = [] {
     if constexpr (std::is_same<T, __bf16>::value) {
       using C = Cfg<T, D>;
@@ -220,14 +247,24 @@ static int launch_fwd_t(const FwdParams& p, int BH, hipStream_t stream) {
       constexpr int stage = 128 * C::OROWV * 16;
       return tiles > stage ? tiles : stage;
     } else {
-      return SplitStages<T, D, 4, JVP ? 4 : 2>::BYTES;
+      return SplitFwdPlan<T, D, JVP, NW>::BYTES;
     }
   }();
-  auto kern = attn_fwd_kernel<T, D, JVP>;
+  auto kern = [] {
+    if constexpr (NW == 8) return attn_fwd_wide_kernel<T, D, JVP>;
+    else return attn_fwd_kernel<T, D, JVP>;
+  }();
   static bool lds_ok[64] = {};
   if (!ensure_dynamic_lds(kern, smem, lds_ok)) return -7;
-  const uint32_t nqb = (p.Lq + 127) / 128;
-  return launch_kernel(kern, dim3(nqb * (uint32_t)BH), dim3(256), smem, stream, p);
+  const uint32_t nqb = (p.Lq + 32 * NW - 1) / (32 * NW);
+  return launch_kernel(kern, dim3(nqb * (uint32_t)BH), dim3(64 * NW), smem, stream, p);
+}
+template <typename T, int D, bool JVP>
+static int launch_fwd_t(const FwdParams& p, int BH, hipStream_t stream) {
+  if constexpr (has_wide_split<T, D, JVP>()) {
+    if (wide_split(p.Lq, D, BH, std::is_same<T, float>::value ? ElemType::f32 : ElemType::f16, JVP)) return launch_fwd_nw<T, D, JVP, 8>(p, BH, stream);
+  }
+  return launch_fwd_nw<T, D, JVP, 4>(p, BH, stream);
 }
 
 template <typename T, bool JVP>
@@ -249,6 +286,11 @@ int launch_fwd_generic(const FwdParams& p, int BH, int D, ElemType type, bool jv
     case ElemType::f16: return jvp ? launch_fwd_d<_Float16, true>(p, BH, D, stream) : launch_fwd_d<_Float16, false>(p, BH, D, stream);
     default: return jvp ? launch_fwd_d<float, true>(p, BH, D, stream) : launch_fwd_d<float, false>(p, BH, D, stream);
   }
+}
+
+void plan_fwd_generic(int Lq, int D, int BH, ElemType type, bool jvp, char* buf, size_t n) {
+  const char* t = type == ElemType::bf16 ? "__bf16" : (type == ElemType::f16 ? "_Float16" : "float");
+  snprintf(buf, n, "dmf::attn_fwd_%skernel<%s, %d, %s>", wide_split(Lq, D, BH, type, jvp) ? "wide_" : "", t, D, jvp ? "true" : "false");
 }
 
 int launch_fwd(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream) {

@@ -104,6 +104,7 @@ int launch_fwd(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipSt
 // Building blocks of launch_fwd: the generic kernels (any element type, any length)
 // and the tuned bf16 kernels (returns 1 when it has no kernel for the case).
 int launch_fwd_generic(const FwdParams& p, int BH, int D, ElemType type, bool jvp, hipStream_t stream);
+void plan_fwd_generic(int Lq, int D, int BH, ElemType type, bool jvp, char* buf, size_t n);
 int launch_fwd_bf16_fast(const FwdParams& p, int BH, int D, bool jvp, hipStream_t stream);
 // Forward for grids that do not fill the device (bf16, with or without the in-kernel norms, and fp16): the policy, the launch,
 // and the kernel's name as profilers print it.

@@ -69,6 +69,16 @@ __device__ __forceinline__ void mma_planes16(f32x4& acc, const u32x4 (&a)[NA], c
   for_plane_pairs<NA, NB>([&](int i, int j) { mma_one16<T>(acc, a[i], b[j]); });
 }
 
+// x minus the low (0) / high (1) f16 half of w: one mixed-precision instruction where conversion and subtraction take two
+// (exact either way: the difference is).
+template <int HALF>
+__device__ __forceinline__ float sub_half(float x, uint32_t w) {
+  float r;
+  if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
+  else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
+  return r;
+}
+
 // Eight fp32 values as NP planes of eight 16-bit ones.  ANY (operands as the caller gave them, in bf16 planes): all but the last
 // plane are held within the finite range, so that a value above the largest bf16 number does not round to infinity and an
 // infinity or NaN ends up in the last plane alone -- it then meets only the first plane of the other operand, whose sign is the
@@ -85,8 +95,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
         const fp16x2 h = __builtin_amdgcn_cvt_pkrtz(a, b);
         pl[k][i] = __builtin_bit_cast(uint32_t, h);
         if (k + 1 < NP) {
-          a -= (float)h[0];
-          b -= (float)h[1];
+          a = sub_half<0>(a, pl[k][i]);
+          b = sub_half<1>(b, pl[k][i]);
         }
       } else {
         const bool hold = ANY && k + 1 < NP;
@@ -117,22 +127,48 @@ struct SplitCfg {
   static constexpr int PLANE = 32 * P * 16, TILE = S::NI * PLANE;    // bytes
   static constexpr bool TAIL = (D % 32) != 0 && (D % 32) <= 16;      // 16-wide remainder by 16x16x32 MFMAs (72, 80)
   static constexpr int NMT = TAIL ? D / 32 : (D + 31) / 32;
-  static constexpr int ITERS = (32 * VPR + 64 * NW - 1) / (64 * NW); // vectors of a tile per thread
   static constexpr int RAW = sizeof(T) / 2;                          // 16-byte registers quads per vector
   static constexpr int STAGE_ROWS_BYTES = 32 * NW * Cfg<T, D>::OROWV * 16;
 };
 
 // One streamed tensor tile of 32 rows: load() requests this thread's vectors (rows at or past nrows read as zero), commit()
-// splits them and writes the planes.
-template <typename T, int D, int NW>
+// splits them and writes the planes.  FAST: full tiles are read through a buffer descriptor and 32-bit offsets kept from tile to
+// tile (the per-lane 64-bit addresses and row checks are a tenth of the vector instructions of an fp16 tile); the ragged last one,
+// and rows 2^26 bytes or more apart, take the general addresses.  In kernels of one wave per SIMD the branch between the two costs
+// more than it saves (it ends the block in which loads are scheduled among the products).
+template <typename T, int D, int NW, bool FAST = false>
 struct TileLoad {
   using C = SplitCfg<T, D, NW>;
-  u32x4 r[C::ITERS][C::RAW];
-  __device__ __forceinline__ void load(const T* src, int64_t row_stride, int row0, int nrows, int tid) {
+  static constexpr int NVEC = 32 * C::VPR, ITERS = (NVEC + 64 * NW - 1) / (64 * NW);   // vectors of a tile; per thread
+  u32x4 r[ITERS][C::RAW];
+  uint32_t off[FAST ? ITERS : 1];
+  bool near;
+  __device__ __forceinline__ void init(int64_t row_stride, int tid) {
+    if constexpr (FAST) {
+      near = row_stride < (int64_t)(1 << 26) / (int64_t)sizeof(T);
 #pragma unroll
-    for (int it = 0; it < C::ITERS; ++it) {
+      for (int it = 0; it < ITERS; ++it) {
+        const int v = tid + it * 64 * NW, row = v / C::VPR, cv = v % C::VPR;
+        // (threads without a vector in the last round read the tile's first one)
+        off[it] = v < NVEC ? static_cast<uint32_t>(row) * static_cast<uint32_t>(row_stride * (int64_t)sizeof(T)) + cv * (uint32_t)sizeof(T) * 8 : 0u;
+      }
+    }
+  }
+  __device__ __forceinline__ void load(const T* src, int64_t row_stride, int row0, int nrows, int tid) {
+    if constexpr (FAST) {
+      if (near && row0 + 32 <= nrows) {
+        const __amdgpu_buffer_rsrc_t rsrc = make_rows_rsrc(src + (int64_t)row0 * row_stride, (uint32_t)row_stride * (uint32_t)sizeof(T), 32, D * (int)sizeof(T));
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+          for (int k = 0; k < C::RAW; ++k) r[it][k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[it] + 16 * k, 0, 0));
+        return;
+      }
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
       const int v = tid + it * 64 * NW, row = v / C::VPR, cv = v % C::VPR;
-      const bool ok = v < 32 * C::VPR && row0 + row < nrows;
+      const bool ok = v < NVEC && row0 + row < nrows;
       const u32x4* g = reinterpret_cast<const u32x4*>(src + (int64_t)(row0 + row) * row_stride + cv * 8);
 #pragma unroll
       for (int k = 0; k < C::RAW; ++k) r[it][k] = ok ? g[k] : u32x4{0, 0, 0, 0};
@@ -140,9 +176,9 @@ struct TileLoad {
   }
   __device__ __forceinline__ void commit(char* tile, int tid) const {
 #pragma unroll
-    for (int it = 0; it < C::ITERS; ++it) {
+    for (int it = 0; it < ITERS; ++it) {
       const int v = tid + it * 64 * NW, row = v / C::VPR, cv = v % C::VPR;
-      if (v < 32 * C::VPR) {
+      if (v < NVEC) {
         char* dst = tile + (row * C::P + cv) * 16;
         if constexpr (sizeof(T) == 2) {   // one plane, as it is
           *reinterpret_cast<u32x4*>(dst) = r[it][0];
@@ -366,56 +402,92 @@ __device__ __forceinline__ void store_out(char* smem, T* dst, int64_t row_stride
 }
 
 // ------------------------------------------------------------------------------------------------- forward (+ JVP)
-// Stages of K, V [, dK, dV] planes in LDS: two when they fit beside each other (one barrier per tile), else one.
-template <typename T, int D, int NW, int NT>
-struct SplitStages {
-  static constexpr int STAGE = NT * SplitCfg<T, D, NW>::TILE;
-  static constexpr int N = 2 * STAGE <= 160 * 1024 ? 2 : 1;
-  static constexpr int BYTES = N * STAGE > SplitCfg<T, D, NW>::STAGE_ROWS_BYTES ? N * STAGE : SplitCfg<T, D, NW>::STAGE_ROWS_BYTES;
-  static_assert(STAGE <= 160 * 1024 && BYTES <= 160 * 1024, "LDS budget");
-};
-
 // Start of the running maximum (log2 units).  Finite, and above what keys masked by the lowest number of their type give, so that
 // a tile of nothing but such keys or of -inf scores weighs nothing: with its own maximum m subtracted, fma(S, c2, -m) would be the
 // rounding error of m, which is large where m is.
 constexpr float kLowestMax = -1e30f;
 constexpr float kSplitLazyLog2 = 6.0f;   // the running maximum is raised when exceeded by more than 2^6 (exact: normalised once at the end)
 
+// Two forms of the forward.  NW = 4 (128 rows): the tiles of the next step are requested before a step's products and committed
+// after them, into the other of two LDS stages where two fit (one barrier per step).  NW = 8 (256 rows): what bounds the 4-wave
+// form with tangents is that a wave has a SIMD's register file to itself (422 of 512 registers at fp16 D72, 352 at fp32 D64), so
+// nothing runs beside its softmax and its splitting (matrix pipe 37 % busy).  Here a wave stays within 256: one LDS stage, K and V
+// requested and committed a phase apart (half as many loads in flight), the planes of dQ in LDS; and with twice as many rows to a
+// tile the splitting of fp32 elements, a third of the vector instructions, is shared by twice as many waves -- with tangents four
+// of them bring the primal tile of a pair and four the tangent's.  us (4 -> 8 waves): fp16 + tangents B8 H16 N1024 D72 311 -> 188,
+// fp32 + tangents B4 H16 N1024 D64 267 -> 233, fp16 B8 H16 N1024 D72 97 -> 78 (four waves per SIMD instead of three).
+template <typename T, int D, bool JVP, int NW>
+struct SplitFwdPlan {
+  using C = SplitCfg<T, D, NW>;
+  static constexpr bool WIDE = NW == 8, PAIR = JVP && WIDE;
+  static constexpr int NT = JVP ? 4 : 2, STAGE = NT * C::TILE;
+  static constexpr int STAGES = !WIDE && 2 * STAGE <= 160 * 1024 ? 2 : 1;
+  static constexpr bool DQ_LDS = PAIR && (sizeof(T) == 4 || D > 64);
+  static constexpr int DQ_OFF = STAGES * STAGE, DQ_BYTES = DQ_LDS ? NW * C::NCHUNK * SplitType<T>::NI * 64 * 16 : 0;
+  static constexpr int BYTES = DQ_OFF + DQ_BYTES > C::STAGE_ROWS_BYTES ? DQ_OFF + DQ_BYTES : C::STAGE_ROWS_BYTES;
+  static_assert(BYTES <= 160 * 1024, "LDS budget");
+};
+
 template <typename T, int D, bool JVP, int NW>
 __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   using C = SplitCfg<T, D, NW>;
-  constexpr int NI = SplitType<T>::NI, NCHUNK = C::NCHUNK, NT = JVP ? 4 : 2, BQ = 32 * NW;
-  using ST = SplitStages<T, D, NW, NT>;
+  using Plan = SplitFwdPlan<T, D, JVP, NW>;
+  constexpr int NI = SplitType<T>::NI, NCHUNK = C::NCHUNK, BQ = 32 * NW;
   constexpr bool F16 = SplitType<T>::F16;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c32 = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c32 = lane & 31, g = lane >> 5;
   const uint32_t nqb = (p.Lq + BQ - 1) / BQ;
   const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
   const int bh = wg / nqb, q0 = (wg % nqb) * BQ, b = bh / p.H, h = bh % p.H;
   auto base = [&](int t) { return (int64_t)b * p.st[t][0] + (int64_t)h * p.st[t][2]; };
   const int qrow = q0 + wave * 32 + c32;
 
-  zero_plane_pads<T, D, NW>(smem, ST::N * NT * NI, tid);
+  zero_plane_pads<T, D, NW>(smem, Plan::STAGES * Plan::NT * NI, tid);
 
-  const T* src[4] = {static_cast<const T*>(p.k) + base(1), static_cast<const T*>(p.v) + base(2), JVP ? static_cast<const T*>(p.tk) + base(4) : nullptr,
-                     JVP ? static_cast<const T*>(p.tv) + base(5) : nullptr};
-  const int64_t rs[4] = {p.st[1][1], p.st[2][1], p.st[4][1], p.st[5][1]};
-  TileLoad<T, D, NW> ld[NT];
-  auto load = [&](int it) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) ld[t].load(src[t], rs[t], it * 32, p.Lkv, tid);
+  // K [, dK] and V [, dV] tiles
+  constexpr int LW = Plan::PAIR ? NW / 2 : NW;
+  const bool second = Plan::PAIR && wave >= LW;
+  const int ltid = Plan::PAIR ? tid & (64 * LW - 1) : tid;
+  const int tk = second ? 4 : 1, tv = second ? 5 : 2;
+  const T *gk = static_cast<const T*>(second ? p.tk : p.k) + base(tk), *gv = static_cast<const T*>(second ? p.tv : p.v) + base(tv);
+  auto tile = [&](int it, int t) { return smem + (Plan::STAGES == 2 ? (it & 1) * Plan::STAGE : 0) + t * C::TILE; };
+  TileLoad<T, D, LW, Plan::WIDE> lk, lv, ldk, ldv;
+  lk.init(p.st[tk][1], ltid);
+  lv.init(p.st[tv][1], ltid);
+  auto load_k = [&](int it) {
+    lk.load(gk, p.st[tk][1], it * 32, p.Lkv, ltid);
+    if constexpr (JVP && !Plan::PAIR) ldk.load(static_cast<const T*>(p.tk) + base(4), p.st[4][1], it * 32, p.Lkv, tid);
   };
-  auto tile = [&](int it, int t) { return smem + (ST::N == 2 ? (it & 1) * ST::STAGE : 0) + t * C::TILE; };
-  auto commit = [&](int it) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) ld[t].commit(tile(it, t), tid);
+  auto load_v = [&](int it) {
+    lv.load(gv, p.st[tv][1], it * 32, p.Lkv, ltid);
+    if constexpr (JVP && !Plan::PAIR) ldv.load(static_cast<const T*>(p.tv) + base(5), p.st[5][1], it * 32, p.Lkv, tid);
   };
-  load(0);
+  auto commit_k = [&](int it) {
+    lk.commit(tile(it, second ? 2 : 0), ltid);
+    if constexpr (JVP && !Plan::PAIR) ldk.commit(tile(it, 2), tid);
+  };
+  auto commit_v = [&](int it) {
+    lv.commit(tile(it, second ? 3 : 1), ltid);
+    if constexpr (JVP && !Plan::PAIR) ldv.commit(tile(it, 3), tid);
+  };
+  load_k(0);
+  load_v(0);
 
-  u32x4 Q[NCHUNK][NI], dQ[JVP ? NCHUNK : 1][NI];
+  // dQ planes beside Q's in registers, or where that would spill in LDS, in the order in which this wave reads them back
+  u32x4 Q[NCHUNK][NI], dQ[JVP && !Plan::DQ_LDS ? NCHUNK : 1][NI];
+  u32x4* const dQl = reinterpret_cast<u32x4*>(smem + Plan::DQ_OFF) + wave * (NCHUNK * NI * 64) + lane;
   load_own_row<T, D, NW>(static_cast<const T*>(p.q) + base(0), p.st[0][1], qrow, p.Lq, g, Q);
-  if constexpr (JVP) load_own_row<T, D, NW>(static_cast<const T*>(p.tq) + base(3), p.st[3][1], qrow, p.Lq, g, dQ);
+  if constexpr (Plan::DQ_LDS) {
+    u32x4 x[NCHUNK][NI];
+    load_own_row<T, D, NW>(static_cast<const T*>(p.tq) + base(3), p.st[3][1], qrow, p.Lq, g, x);
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c)
+#pragma unroll
+      for (int k = 0; k < NI; ++k) dQl[(c * NI + k) * 64] = x[c][k];
+  } else if constexpr (JVP) {
+    load_own_row<T, D, NW>(static_cast<const T*>(p.tq) + base(3), p.st[3][1], qrow, p.Lq, g, dQ);
+  }
 
   OutAcc<T, D, NW> O, dO, dOv;   // dOv (fp16 tangents only): dV^T P, apart because dO carries the row scale of P*dS
   O.zero();
@@ -428,10 +500,15 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   const float c2 = p.scale_log2;
 
   const int ntiles = (p.Lkv + 31) / 32;
-  commit(0);
+  commit_k(0);
+  if constexpr (!Plan::WIDE) commit_v(0);
   for (int it = 0; it < ntiles; ++it) {
-    __syncthreads();                     // tile `it` is in LDS
-    if (it + 1 < ntiles) load(it + 1);   // in flight during the math
+    __syncthreads();   // the tile (wide: its K half) is in LDS; wide: every wave is done with V of the tile before
+    if constexpr (Plan::WIDE) commit_v(it);
+    if (it + 1 < ntiles) {   // in flight during the math
+      load_k(it + 1);
+      if constexpr (!Plan::WIDE) load_v(it + 1);
+    }
     const char *Kt = tile(it, 0), *Vt = tile(it, 1), *dKt = tile(it, 2), *dVt = tile(it, 3);
     f32x16 S = {0}, dS = {0};
 #pragma unroll
@@ -442,8 +519,16 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
       if constexpr (JVP) {
         u32x4 dk[NI];
         row_planes<T, D, NW>(dKt, c32, c, g, dk);
-        mma_planes<T>(dS, k, dQ[c]);
-        mma_planes<T>(dS, dk, Q[c]);
+        if constexpr (Plan::DQ_LDS) {
+          mma_planes<T>(dS, dk, Q[c]);
+          u32x4 dq[NI];
+#pragma unroll
+          for (int i = 0; i < NI; ++i) dq[i] = dQl[(c * NI + i) * 64];
+          mma_planes<T>(dS, k, dq);
+        } else {
+          mma_planes<T>(dS, k, dQ[c]);
+          mma_planes<T>(dS, dk, Q[c]);
+        }
       }
     }
     if ((it + 1) * 32 > p.Lkv) {
@@ -478,6 +563,13 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     }
     WOperand<T> we;
     we.form(E);
+    if constexpr (Plan::WIDE) {
+      __syncthreads();   // V is in LDS; every wave is done with K
+      if (it + 1 < ntiles) {
+        commit_k(it + 1);
+        load_v(it + 1);
+      }
+    }
     if constexpr (JVP) {
       gs.update(G, dO);
       if constexpr (F16) G *= gs.mul;
@@ -489,8 +581,13 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     } else {
       contract_rows<T, D, NW>(Vt, lane, O, we);
     }
-    if constexpr (ST::N == 1) __syncthreads();   // every wave is done with the stage
-    if (it + 1 < ntiles) commit(it + 1);
+    if constexpr (!Plan::WIDE) {
+      if constexpr (Plan::STAGES == 1) __syncthreads();   // every wave is done with the stage
+      if (it + 1 < ntiles) {
+        commit_k(it + 1);
+        commit_v(it + 1);
+      }
+    }
   }
 
   const float l_tot = xhalf_sum(l_run), inv_l = 1.0f / l_tot;
@@ -528,6 +625,15 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
 }
 
 // --------------------------------------------------------------------------------------------------------- backward
+// Stages of the backward's two tensors in LDS: two when they fit beside each other (one barrier per tile), else one.
+template <typename T, int D, int NW, int NT>
+struct SplitStages {
+  static constexpr int STAGE = NT * SplitCfg<T, D, NW>::TILE;
+  static constexpr int N = 2 * STAGE <= 160 * 1024 ? 2 : 1;
+  static constexpr int BYTES = N * STAGE > SplitCfg<T, D, NW>::STAGE_ROWS_BYTES ? N * STAGE : SplitCfg<T, D, NW>::STAGE_ROWS_BYTES;
+  static_assert(STAGE <= 160 * 1024 && BYTES <= 160 * 1024, "LDS budget");
+};
+
 template <typename T, int D, int NW>
 __device__ __forceinline__ void split_bwd_dq_body(const BwdParams& p) {
   using C = SplitCfg<T, D, NW>;

@@ -148,7 +148,7 @@ int dmf_attn_plan(int entry, int B, int H, int Lq, int Lkv, int D, int dtype, ch
   }
   if (bf16 && dmf::plan_fwd_bf16_fast(Lq, D, jvp, B * H, qn, kn, buf, n)) return DMF_ATTN_OK;
   if (qn) return DMF_ATTN_ENOKERNEL;
-  snprintf(buf, n, "dmf::attn_fwd_kernel<%s, %d, %s>", t, D, jvp ? "true" : "false");
+  dmf::plan_fwd_generic(Lq, D, B * H, static_cast<dmf::ElemType>(dtype), jvp, buf, n);
   return DMF_ATTN_OK;
 }
 

@@ -876,3 +876,50 @@ def test_keys_masked_by_extreme_values(dtype, L, value):
     # (bf16: probabilities rounded to 8 bits before the second product)
     tol = {torch.float32: 1e-5, torch.float16: 1e-3, torch.bfloat16: 2e-2}[dtype]
     assert ao.rel_l2(got[torch.isfinite(ref)], ref[torch.isfinite(ref)]) <= tol
+
+
+@pytest.mark.parametrize("dtype,D,jvp,B,H,L,wide", [
+    (torch.float16, 72, True, 65, 4, 257, True), (torch.float16, 72, True, 32, 4, 333, True), (torch.float16, 80, True, 65, 4, 256, True),
+    (torch.float16, 72, True, 64, 4, 256, True), (torch.float16, 72, True, 32, 4, 256, False), (torch.float16, 72, False, 200, 4, 256, True),
+    (torch.float16, 72, False, 256, 4, 300, False), (torch.float32, 64, True, 64, 4, 256, True), (torch.float32, 64, True, 64, 4, 225, True),
+    (torch.float32, 64, True, 65, 4, 256, False)])
+@pytest.mark.parametrize("Lkv", [None, 1, 31, 65])
+def test_wide_split_forward_against_the_oracle(dtype, D, jvp, B, H, L, wide, Lkv):
+    """The fp16 / fp32 forward in 256-row work-groups and its neighbours on either side of the policy: ragged and single key tiles, a
+    ragged last query block."""
+    Lkv = Lkv or L
+    plan = _lib.plan("fwd_jvp" if jvp else "fwd", B, H, L, Lkv, D, dtype)
+    assert ("wide" in plan) == wide, plan
+    g = torch.Generator(device=DEV).manual_seed(L + D)
+    rnd = lambda n: torch.randn(B, n, H, D, generator=g, device=DEV).to(dtype)
+    q, k, v, tq, tk, tv = rnd(L), rnd(Lkv), rnd(Lkv), rnd(L), rnd(Lkv), rnd(Lkv)
+    half, scale = dtype == torch.float16, D ** -0.5
+    if jvp:
+        o, to, lse = (_lib.fwd_jvp_half if half else _lib.fwd_jvp)(q, k, v, tq, tk, tv, scale)
+    else:
+        o, lse = (_lib.fwd_half if half else _lib.fwd)(q, k, v, scale)
+    pick = [0, B // 2, B - 1]
+    f = lambda t: t[pick].float().cpu()
+    o_ref, to_ref = ao.base_attn_jvp(*map(f, (q, k, v, tq, tk, tv)))
+    tol = 1e-3 if half else 1e-5
+    _check("o", f(o), o_ref, tol)
+    assert ao.rel_l2(f(lse), ao.lse_ref(f(q), f(k), scale)) <= 1e-5
+    if jvp:
+        _check("to", f(to), to_ref, tol)
+
+
+def test_wide_split_forward_reads_rows_far_apart():
+    """Key rows 2^26 bytes apart (beyond the 32-bit offsets of the fast tile loads), values in a transposed (L, B, H, D) buffer, the batch of
+    both expanded: the same bits as from dense copies."""
+    B, H, L, Lkv, D = 64, 4, 256, 33, 64
+    g = torch.Generator(device=DEV).manual_seed(8)
+    q, tq = (torch.randn(B, L, H, D, generator=g, device=DEV) for _ in range(2))
+    far = torch.empty(Lkv << 24, device=DEV)
+    k = far.as_strided((B, Lkv, H, D), (0, 1 << 24, D, 1))
+    k[0].copy_(torch.randn(Lkv, H, D, generator=g, device=DEV))
+    v = torch.randn(Lkv, 1, H, D, generator=g, device=DEV).transpose(0, 1).expand(B, Lkv, H, D)
+    assert "wide" in _lib.plan("fwd_jvp", B, H, L, Lkv, D, torch.float32)
+    got = _lib.fwd_jvp(q, k, v, tq, k, v, D ** -0.5)
+    exp = _lib.fwd_jvp(q, k.contiguous(), v.contiguous(), tq, k.contiguous(), v.contiguous(), D ** -0.5)
+    for a, b in zip(got, exp):
+        assert torch.equal(a, b)
