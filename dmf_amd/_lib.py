@@ -61,6 +61,7 @@ SIGNATURES = {
 FUSED_SIGNATURES = {
     "dmf_attn_bwd_qknorm_workspace_floats": (c_int64, [_I] * 5),
     "dmf_attn_bwd_qknorm": (c_int, [_P] * 10 + [_F] + [_P] * 7 + [_S] + [_I] * 5 + [_F, _I, _P]),
+    "dmf_modulation_fwd": (c_int, [_P] * 5 + [_I] * 6 + [_P]),
 }
 
 _lib = None

@@ -951,6 +951,100 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
   return out;
 }
 
+// ---- adaLN modulations ---------------------------------------------------------------------------------------------------
+
+// A (B, 1, C) column block of a dense (B, n) region of `whole`, without the dispatcher.
+Tensor column_block(const Tensor& whole, int64_t offset, int64_t B, int64_t n, int64_t C) {
+  auto impl = c10::make_intrusive<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
+  impl->set_storage_offset(offset);
+  const std::array<int64_t, 3> sizes{B, 1, C}, strides{n, n, 1};
+  impl->set_sizes_and_strides(sizes, strides);
+  return Tensor(std::move(impl));
+}
+
+// Every block's silu -> Linear -> chunk(chunks) and the final layer's (the last weight, chunk(chunks_last)) with nothing to
+// differentiate: one silu per conditioning vector and one launch for all products.  cond[g]: the conditioning vector of group g.
+// Weights the kernel does not read as they are (a cast per call, other types, widths or batches) go to the general route.
+py::object modulations(const std::vector<Tensor>& conds_, const std::vector<int>& cond, const std::vector<Tensor>& weights,
+                       const std::vector<OptTensor>& biases, const std::vector<OptTensor>& w_lp, const std::vector<OptTensor>& b_lp, int64_t chunks,
+                       int64_t chunks_last) {
+  const int64_t level = current_level();
+  const size_t G = weights.size();
+  if (level == kUnsupported || conds_.empty() || conds_.size() > 2 || G < 1 || G > 64 || cond.size() != G || biases.size() != G || w_lp.size() != G ||
+      b_lp.size() != G)
+    return none();
+  std::vector<Arg> c;
+  for (const Tensor& t : conds_) c.push_back(unpack(t));
+  const int64_t K = c[0].data.size(-1), B = c[0].data.size(0);
+  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+  bool dual = false;
+  for (const Arg& a : c) {
+    if (!plain_gpu(a) || !block_dtype(a.data) || (a.data.dim() != 3 && a.data.dim() != 2) || a.data.size(-1) != K || a.data.size(0) != B ||
+        a.data.numel() != B * K || a.data.device() != c[0].data.device() || autocast_type(a.data) != at::kBFloat16 || any_grad(a) || only_tangents_want(a))
+      return none();
+    dual = dual || a.tan.defined();
+  }
+  if (B < 1 || B > 128 || K % 128 || K < 128) return none();
+  const int64_t n = weights[0].size(0), n_last = weights[G - 1].size(0);
+  if (n % 32 || n_last % 32 || n % chunks || n_last % chunks_last || n < 32 || n_last < 32) return none();
+  std::vector<Tensor> keep;   // the operands, alive until the launch
+  std::vector<const void*> w(G), b(G);
+  for (size_t g = 0; g < G; ++g) {
+    const Arg weight = unpack(weights[g]), bias = unpack(biases[g]);
+    if (!plain_gpu(weight) || (bias.defined() && !plain_gpu(bias)) || weight.tan.defined() || bias.tan.defined() || any_grad(weight, bias) ||
+        weight.data.dim() != 2 || weight.data.size(1) != K || weight.data.size(0) != (g + 1 < G ? n : n_last) ||
+        weight.data.device() != c[0].data.device())
+      return none();
+    const auto as_is = [&](const Arg& own, const OptTensor& lp) {
+      if (own.data.scalar_type() == at::kBFloat16) return own.data;
+      return autocast && lp && lp->defined() && lp->scalar_type() == at::kBFloat16 && lp->is_cuda() ? data_of(unwrap(*lp)) : Tensor();
+    };
+    const Tensor wt = as_is(weight, w_lp[g]), bt = bias.defined() ? as_is(bias, b_lp[g]) : Tensor();
+    if (!wt.defined() || !wt.is_contiguous() || wt.sizes() != weight.data.sizes() || reinterpret_cast<uintptr_t>(wt.const_data_ptr()) % 16) return none();
+    if (bias.defined() && (!bt.defined() || !bt.is_contiguous() || bt.numel() != weight.data.size(0) || reinterpret_cast<uintptr_t>(bt.const_data_ptr()) % 8))
+      return none();
+    w[g] = wt.const_data_ptr();
+    b[g] = ptr(bt);
+    keep.push_back(wt);
+    if (bt.defined()) keep.push_back(bt);
+  }
+  c10::OptionalDeviceGuard device(c[0].data.device());
+  Tensor whole;
+  std::vector<int64_t> at_(G);   // element offset of each group's primal rows
+  const int64_t rows = dual ? 2 * B : B;
+  {
+    Below below;
+    std::array<const void*, 2> s{nullptr, nullptr};
+    for (size_t i = 0; i < c.size(); ++i) {
+      const Tensor x = dense(c[i].data), tx = dual ? (c[i].tan.defined() ? dense(c[i].tan) : at::zeros_like(x)) : Tensor();
+      const Tensor y = empty({rows, K}, at::kBFloat16, x);
+      check(dmf_silu_fwd(ptr(x), ptr(tx), mptr(y), dual ? static_cast<char*>(mptr(y)) + B * K * 2 : nullptr, B * K, code_of(x), DMF_ATTN_BF16,
+                         stream_of(x)),
+            "dmf_silu_fwd");
+      s[i] = ptr(y);
+      keep.push_back(y);
+    }
+    whole = empty({rows * ((int64_t)(G - 1) * n + n_last)}, at::kBFloat16, c[0].data);
+    std::vector<void*> out(G);
+    for (size_t g = 0; g < G; ++g) {
+      at_[g] = (int64_t)g * rows * n;
+      out[g] = static_cast<char*>(mptr(whole)) + at_[g] * 2;
+    }
+    check(dmf_modulation_fwd(s.data(), w.data(), b.data(), out.data(), cond.data(), (int)G, (int)B, (int)K, (int)n, (int)n_last, dual, stream_of(whole)),
+          "dmf_modulation_fwd");
+  }
+  py::list result;
+  for (size_t g = 0; g < G; ++g) {
+    const int64_t width = g + 1 < G ? n : n_last, parts = g + 1 < G ? chunks : chunks_last, C = width / parts;
+    py::list of_group;
+    for (int64_t i = 0; i < parts; ++i)
+      of_group.append(finish(column_block(whole, at_[g] + i * C, B, width, C),
+                             dual ? column_block(whole, at_[g] + B * width + i * C, B, width, C) : Tensor(), nullptr, level));
+    result.append(of_group);
+  }
+  return result;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -967,4 +1061,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("linear", &linear);
   m.def("linear_gelu_inference", &linear_gelu_inference);
   m.def("chunk_last", &chunk_last);
+  m.def("modulations", &modulations);
 }

@@ -17,6 +17,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import block_ops as fused
+from . import _lib
 from ._lib import SUPPORTED_HEAD_DIMS
 from .flash_attention_hip_jvp import flash_attn_func as hip_func
 from .flash_attention_hip_jvp import flash_attn_projection as hip_projection
@@ -275,6 +276,41 @@ class FinalLayer(nn.Module):
         if self.fused:
             return self.linear(fused.ln_modulate(x, shift, scale, self.norm_final.eps))
         return self.linear(modulate(self.norm_final(x), shift, scale))
+
+
+def _plain(module: nn.Module, cls: type) -> bool:
+    return type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
+
+
+def _projection(owner: nn.Module, cls: type):
+    """The adaLN projection of a block or final layer that computes it the way this file does: no subclass, no hook, no replaced
+    method on the path from the conditioning vector to the chunks.  None otherwise."""
+    if type(owner).modulation is not cls.modulation or "modulation" in owner.__dict__ or not owner.fused:
+        return None
+    seq = owner.adaLN_modulation
+    if not _plain(seq, nn.Sequential) or len(seq._modules) != 2:
+        return None
+    act, proj = seq._modules.values()
+    return proj if _plain(act, SiLU) and act.fused and _plain(proj, Linear) and proj.fused else None
+
+
+def stacked_modulations(blocks, conds, final_layer: FinalLayer, c_final: Tensor):
+    """``([blk.modulation(c) for blk, c in zip(blocks, conds)], final_layer.modulation(c_final))``.  Where nothing is differentiated
+    in reverse and the weights are in the compute dtype (a low-precision model, or under ``frozen_low_precision_params``), all
+    projections are one launch."""
+    # one condition per object: the two conditioning vectors of a stack
+    distinct = list({id(c): c for c in (*conds, c_final)}.values())
+    first = _projection(final_layer, FinalLayer)
+    if (first is not None and len(distinct) <= 2 and not (torch.is_grad_enabled() and first.weight.requires_grad)
+            and _lib.native(*distinct) and not torch.nn.modules.module._has_any_global_hook()):
+        projs = [_projection(blk, DiTBlock) for blk in blocks] + [first]
+        if all(p is not None for p in projs) and not torch.overrides.has_torch_function([p.weight for p in projs]):
+            index = {id(c): i for i, c in enumerate(distinct)}
+            out = _lib.host().modulations(distinct, [index[id(c)] for c in (*conds, c_final)], [p.weight for p in projs], [p.bias for p in projs],
+                                          [p.lp_weight for p in projs], [p.lp_bias for p in projs], 6, 2)
+            if out is not None:
+                return out[:-1], out[-1]
+    return [blk.modulation(c) for blk, c in zip(blocks, conds)], final_layer.modulation(c_final)
 
 
 def get_2d_sincos_pos_embed(embed_dim: int, grid_size: int) -> np.ndarray:

@@ -28,6 +28,15 @@ DMF_ATTN_API int dmf_attn_bwd_qknorm(const void* dout, const void* q_hat, const 
                         float* delta, float* workspace, const int64_t* strides,
                         int B, int H, int Lq, int Lkv, int D, float scale, int dtype, void* stream);
 
+/*
+ * The adaLN projections of a stack in one launch, bf16: out[g] = s[cond[g]] w[g]^T + bias[g] for `groups` (1 .. 64) groups, w[g]
+ * (n, K) row-major -- (n_last, K) for the last one --, bias[g] (n) or NULL, s[0 .. 1] the (B, K) activated conditioning vectors
+ * (s[1] may be NULL if no group uses it).  jvp: s[.] holds B more rows, the tangents, and out[g] takes B more rows, t w^T.  B up
+ * to 128, K a multiple of 128, n a multiple of 32; w and s 16-byte, bias and out 8-byte aligned.
+ */
+DMF_ATTN_API int dmf_modulation_fwd(const void* const* s, const void* const* w, const void* const* bias, void* const* out, const int* cond,
+                        int groups, int B, int K, int n, int n_last, int jvp, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

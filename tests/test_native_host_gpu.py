@@ -1,5 +1,7 @@
 """The native host path against the general Python route: same kernels, same operands, so the same bits -- outputs, tangents,
 gradients -- in every way an operator is differentiated; and the cases it hands back to the general route."""
+import contextlib
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -9,6 +11,7 @@ import dmf_amd
 from dmf_amd import _lib, block_ops, harness
 from dmf_amd.dmft import DMFT
 from dmf_amd.flash_attention_hip_jvp import flash_attn_projection
+from dmf_amd.layers import DiTBlock, FinalLayer, frozen_low_precision_params, stacked_modulations
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -183,3 +186,86 @@ def test_watched_calls_take_the_general_route():
     with Watch():
         assert host.attention(q, q, q, None) is None
     assert _lib.native(q, None) and not _lib.native(q, q.as_subclass(Tagged)) and host.attention(q, q, q, None) is not None
+
+
+@pytest.mark.parametrize("dual", [False, True])
+@pytest.mark.parametrize("B,C,depth", [(1, 128, 1), (2, 384, 3), (31, 768, 2), (32, 640, 2), (33, 1152, 2), (64, 768, 2), (65, 1024, 1), (128, 384, 2)])
+def test_stacked_modulations_against_the_blocks_own(B, C, depth, dual):
+    """All adaLN projections in one launch: batches around the 32-row tiles, widths around the 128-column work-groups, one and two
+    conditioning vectors, weights in bf16 and as low-precision copies under autocast.  Both sides round the same fp32 sums of products
+    of bf16 numbers to bf16, so elements differ by one unit in the last place (2^-8) where the sums straddle a boundary: few."""
+    torch.manual_seed(B + C)
+    blocks = [DiTBlock(C, C // 64, attn_func="hip", block_ops="hip").to(DEV) for _ in range(depth)]
+    final = FinalLayer(C, 2, 4, block_ops="hip").to(DEV)
+    stack = torch.nn.ModuleList([*blocks, final]).requires_grad_(False)
+    for p in stack.parameters():
+        torch.nn.init.normal_(p, std=0.05)
+    cs = [torch.randn(B, 1, C, device=DEV) for _ in range(2)]
+    ts = [torch.randn(B, 1, C, device=DEV) for _ in range(2)]
+
+    def call(c, c2):
+        mods, last = stacked_modulations(blocks, [c] + [c2] * (depth - 1), final, c2)
+        return [m for group in (*mods, last) for m in group]
+
+    def run(c, c2):
+        if not dual:
+            return call(c, c2)
+        o, to = torch.func.jvp(lambda a, b: tuple(call(a, b)), (c, c2), (ts[0].to(c.dtype), ts[1].to(c.dtype)))
+        return [*o, *to]
+
+    seen = []
+    native = _lib.host().modulations
+    for low in (False, True):
+        if low:
+            stack.bfloat16()
+        args = [c.bfloat16() if low else c for c in cs]
+        with contextlib.ExitStack() as ctx:
+            if not low:
+                ctx.enter_context(torch.autocast("cuda", dtype=torch.bfloat16))
+                ctx.enter_context(frozen_low_precision_params(stack))
+            new, old = run(*args), _general(lambda: run(*args))
+            seen.append(native([args[0]], [0, 0], [blocks[0].adaLN_modulation[1].weight, final.adaLN_modulation[1].weight], [None, None],
+                               *([m.adaLN_modulation[1].lp_weight for m in (blocks[0], final)], [None, None]), 6, 2) is not None)
+        assert len(new) == len(old) == (6 * depth + 2) * (2 if dual else 1)
+        for a, b in zip(new, old):
+            assert a.dtype == b.dtype == torch.bfloat16 and a.shape == b.shape and a.stride() == b.stride()
+            assert (a.float() - b.float()).abs().max() <= 2 ** -7 * b.float().abs().max() and (a != b).float().mean() <= 0.02
+    assert seen == [True, True]
+
+
+def test_stacked_modulations_leave_to_the_blocks():
+    C = 256
+    blk, final = DiTBlock(C, 4, attn_func="hip", block_ops="hip").to(DEV).bfloat16(), FinalLayer(C, 2, 4, block_ops="hip").to(DEV).bfloat16()
+    host, taken = _lib.host(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            return getattr(host, name)
+
+        def modulations(self, *a):
+            taken.append(host.modulations(*a) is not None)
+            return host.modulations(*a)
+
+    def tries(c):
+        taken.clear()
+        real, _lib.host = _lib.host, Spy
+        try:
+            stacked_modulations([blk], [c], final, c)
+        finally:
+            _lib.host = real
+        return list(taken)
+
+    c = torch.randn(4, 1, C, device=DEV, dtype=torch.bfloat16)
+    assert tries(c) == []                       # parameters ask for gradients
+    with torch.no_grad():
+        assert tries(c) == [True]
+        with pytest.raises(RuntimeError, match="dtype"):   # fp32 outside of autocast is refused as ever
+            tries(c.float())
+        assert taken == [False]
+        assert tries(torch.randn(129, 1, C, device=DEV, dtype=torch.bfloat16)) == [False]
+        calls = []
+        handle = blk.adaLN_modulation[0].register_forward_hook(lambda *a: calls.append(1))
+        assert tries(c) == [] and calls == [1]  # hooks see their module's call
+        handle.remove()
+    blk.requires_grad_(False), final.requires_grad_(False)
+    assert tries(c) == [True] and tries(c.requires_grad_()) == [False]
