@@ -62,6 +62,8 @@ FUSED_SIGNATURES = {
     "dmf_attn_bwd_qknorm_workspace_floats": (c_int64, [_I] * 5),
     "dmf_attn_bwd_qknorm": (c_int, [_P] * 10 + [_F] + [_P] * 7 + [_S] + [_I] * 5 + [_F, _I, _P]),
     "dmf_modulation_fwd": (c_int, [_P] * 5 + [_I] * 6 + [_P]),
+    "dmf_linear_plan": (c_int, [_L] + [_I] * 4),
+    "dmf_linear_fwd": (c_int, [_P] * 6 + [_I] * 4 + [_P]),
 }
 
 _lib = None
@@ -651,6 +653,28 @@ def rmsnorm_bwd(gy, x, gain, eps: float = 1e-6, out=None):
             B, L, H, D, float(eps), _dtype_code(x), _dtype_code(gain), _stream(x))
     _check(rc, "dmf_rmsnorm_bwd")
     return gx, ggain
+
+
+def linear_fwd(x, tx, w, bias, gelu: bool = False):
+    """``(x w^T + bias, tx w^T or None)`` for (M, K) x and tx, (N, K) w, by the package's own product kernel (``gelu``: activated, the
+    tangent through the derivative); None where a library product is the better choice or the operands are not plain dense bf16
+    tensors on the GPU (other types and strides, subclasses, traced or watched calls)."""
+    ops = [_raw(t) for t in (x, tx, w, bias)]
+    x, tx, w, bias = ops
+    present = [t for t in ops if t is not None]
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous()
+                   for t in present) or any(t.data_ptr() % 16 for t in present)):
+        return None
+    M, K, N = x.shape[0], x.shape[1], w.shape[0]
+    if w.dim() != 2 or w.shape[1] != K or (bias is not None and bias.shape != (N,)) or max(M, N, K) > 0x7fffffff or not load().dmf_linear_plan(
+            M, N, K, tx is not None, gelu):
+        return None
+    with torch.cuda.device(x.device):
+        y = _empty((M, N), x.dtype, x.device)
+        ty = None if tx is None else _empty((M, N), x.dtype, x.device)
+        _check(load().dmf_linear_fwd(_ptr(x), _ptr(tx), _ptr(w), _ptr(bias), _ptr(y), _ptr(ty), M, N, K, gelu, _stream(x)), "dmf_linear_fwd")
+    return y, ty
 
 
 def colsum(x, out_dtype=None):

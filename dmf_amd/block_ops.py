@@ -196,9 +196,21 @@ class RMSNormFunc(torch.autograd.Function):
         return gx, ggain, None, None, None
 
 
+def _products(x, tx, w, b):
+    """``x w^T + b`` and ``tx w^T`` (None without a tangent): one launch of the package's own product kernel where that is the
+    faster one, library products elsewhere."""
+    x2 = x.reshape(-1, x.shape[-1])
+    own = None if torch.compiler.is_compiling() else _lib.linear_fwd(x2, None if tx is None else tx.reshape(-1, tx.shape[-1]), w, b)
+    if own is not None:
+        shape = (*x.shape[:-1], w.shape[0])
+        return own[0].reshape(shape), (None if tx is None else own[1].reshape(shape))
+    linear = torch.nn.functional.linear
+    return linear(x, w, b), (None if tx is None else linear(tx, w))
+
+
 class DualLinearFunc(torch.autograd.Function):
     """(x, tx, weight, bias, w_lp, b_lp) -> (y, ty, w) with y = x W^T + b, ty = tx W^T: exactly
-    one library GEMM per stream.  torch's own forward-mode rule for ``linear``
+    one product per stream.  torch's own forward-mode rule for ``linear``
     also multiplies the primal input by a materialised all-zero weight tangent
     and adds the two products (three GEMMs, two fills, a copy and an add per
     layer); parameters carry no tangent in the MeanFlow JVP (loss.py:165-170), so
@@ -207,18 +219,16 @@ class DualLinearFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(x, tx, weight, bias, w_lp, b_lp):
-        linear = torch.nn.functional.linear
         if x.is_cuda and torch.is_autocast_enabled("cuda"):
             dt = torch.get_autocast_dtype("cuda")
             cached = w_lp is not None and w_lp.dtype == dt
             w = w_lp if cached else weight.to(dt)
             b = None if bias is None else (b_lp if cached and b_lp is not None else bias.to(dt))
             with torch.autocast("cuda", enabled=False):
-                y = linear(x.to(dt), w, b)
-                ty = None if tx is None else linear(tx.to(dt), w)
+                y, ty = _products(x.to(dt), None if tx is None else tx.to(dt), w, b)
             # (an input is never handed back as an output: a cached copy reaches backward through the inputs)
             return y, ty, (w if not cached and w is not weight else None)
-        return linear(x, weight, bias), (None if tx is None else linear(tx, weight)), None
+        return *_products(x, tx, weight, bias), None
 
     @staticmethod
     def setup_context(ctx, inputs, outputs):
@@ -300,12 +310,12 @@ def dual_linear(x, weight, bias=None, w_lp=None, b_lp=None):
 
 def linear_gelu_tanh(x, weight, bias, w_lp=None, b_lp=None):
     """``gelu_tanh(F.linear(x, weight, bias))`` -- the first half of the MLP
-    (reference models/layers.py:161-166).  Without gradients and without a tangent
-    the activation rides in the GEMM's epilogue (one library call, the pre-activation
-    never reaches HBM); otherwise the pre-activation is needed for the tangent and for
+    (reference models/layers.py:161-166).  With nothing to differentiate in reverse the
+    activation -- and its derivative on the tangent -- rides in the product's epilogue
+    (the pre-activation never reaches HBM); otherwise the pre-activation is needed for
     the backward pass and this is ``dual_linear`` followed by ``gelu_tanh``."""
-    if bias is not None and not torch.is_grad_enabled() and _lib.native(x, weight, bias):
-        out = _lib.host().linear_gelu_inference(x, weight, bias, w_lp, b_lp)
+    if bias is not None and not (torch.is_grad_enabled() and weight.requires_grad) and _lib.native(x, weight, bias):
+        out = _lib.host().linear_gelu(x, weight, bias, w_lp, b_lp)
         if out is not None:
             return out
     if torch.is_grad_enabled() or bias is None or not x.is_cuda or fwAD.unpack_dual(x).tangent is not None:
@@ -315,6 +325,9 @@ def linear_gelu_tanh(x, weight, bias, w_lp=None, b_lp=None):
     w = w_lp if cached else weight.to(dt)
     b = b_lp if cached and b_lp is not None else bias.to(dt)
     x2 = _lib._raw(x).reshape(-1, x.shape[-1]).to(dt)
+    own = _lib.linear_fwd(x2, None, w, b, gelu=True)
+    if own is not None:
+        return own[0].reshape(*x.shape[:-1], w.shape[0])
     return torch._addmm_activation(b, x2, _lib._raw(w).t(), use_gelu=True).reshape(*x.shape[:-1], w.shape[0])
 
 

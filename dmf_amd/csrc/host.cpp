@@ -869,6 +869,22 @@ bool linear_ok(const Arg& x, const Arg& weight, const Arg& bias) {
          !bias.tan.defined() && weight.data.device() == x.data.device();
 }
 
+// The package's own product kernel (dmf_linear_fwd) where it reads the operands as they are and is the faster one: y, and ty with a
+// tangent.  False: nothing done.
+bool own_linear(const Tensor& x2, const Tensor& tx2, const Tensor& w, const Tensor& b, bool gelu, Tensor& y, Tensor& ty) {
+  const auto readable16 = [](const Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+  };
+  const int64_t M = x2.size(0), N = w.size(0), K = w.size(1);
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !dmf_linear_plan(M, (int)N, (int)K, tx2.defined(), gelu) || !readable16(x2) || !readable16(w) ||
+      (tx2.defined() && !readable16(tx2)) || (b.defined() && (!readable16(b) || b.numel() != N)))
+    return false;
+  y = empty({M, N}, at::kBFloat16, x2);
+  if (tx2.defined()) ty = empty({M, N}, at::kBFloat16, x2);
+  check(dmf_linear_fwd(ptr(x2), ptr(tx2), ptr(w), ptr(b), mptr(y), mptr(ty), (int)M, (int)N, (int)K, gelu, stream_of(x2)), "dmf_linear_fwd");
+  return true;
+}
+
 py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
@@ -889,9 +905,13 @@ py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias
     const int64_t K = x.data.size(-1);
     auto sizes = x.data.sizes().vec();
     sizes.back() = o.w.size(0);
-    const Tensor x2 = x.data.reshape({-1, K}).to(o.dt);
-    y = (o.b.defined() ? at::addmm(o.b, x2, o.w.t()) : at::mm(x2, o.w.t())).view(sizes);
-    if (x.tan.defined()) ty = at::mm(x.tan.reshape({-1, K}).to(o.dt), o.w.t()).view(sizes);
+    const Tensor x2 = x.data.reshape({-1, K}).to(o.dt), tx2 = x.tan.defined() ? x.tan.reshape({-1, K}).to(o.dt) : Tensor();
+    if (!own_linear(x2, tx2, o.w, o.b, false, y, ty)) {
+      y = o.b.defined() ? at::addmm(o.b, x2, o.w.t()) : at::mm(x2, o.w.t());
+      if (tx2.defined()) ty = at::mm(tx2, o.w.t());
+    }
+    y = y.view(sizes);
+    if (ty.defined()) ty = ty.view(sizes);
   }
   std::shared_ptr<KernelNode> node;
   if (grad) {
@@ -906,21 +926,33 @@ py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias
   return py::cast(finish(y, ty, node, level));
 }
 
-// gelu_tanh(linear(x)) with nothing differentiated: the activation rides in the GEMM's epilogue.
-py::object linear_gelu_inference(const Tensor& x_, const Tensor& weight_, const Tensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
+// gelu_tanh(linear(x)) with nothing differentiated in reverse: the activation, and its derivative on the tangent, ride in the product's
+// epilogue.
+py::object linear_gelu(const Tensor& x_, const Tensor& weight_, const Tensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
   const int64_t level = current_level();
-  if (level != kNoLevel || c10::GradMode::is_enabled()) return none();
+  if (level == kUnsupported) return none();
   const Arg x = unpack(x_), weight = unpack(weight_), bias = unpack(bias_);
-  if (!linear_ok(x, weight, bias) || x.tan.defined()) return none();
+  if (!linear_ok(x, weight, bias) || any_grad(x, weight, bias) || only_tangents_want(x)) return none();
   c10::OptionalDeviceGuard device(x.data.device());
   const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
   const at::ScalarType dt = autocast_type(x.data);
-  Below below;
-  const LinearOperands o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp);
-  if (!o.ok) return none();
-  auto sizes = x.data.sizes().vec();
-  sizes.back() = o.w.size(0);
-  return py::cast(at::_addmm_activation(o.b, x.data.reshape({-1, x.data.size(-1)}).to(o.dt), o.w.t(), 1, 1, true).view(sizes));
+  Tensor y, ty;
+  {
+    Below below;
+    const LinearOperands o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp);
+    if (!o.ok) return none();
+    const int64_t K = x.data.size(-1);
+    auto sizes = x.data.sizes().vec();
+    sizes.back() = o.w.size(0);
+    const Tensor x2 = x.data.reshape({-1, K}).to(o.dt), tx2 = x.tan.defined() ? x.tan.reshape({-1, K}).to(o.dt) : Tensor();
+    if (!own_linear(x2, tx2, o.w, o.b, true, y, ty)) {
+      if (tx2.defined()) return none();
+      y = at::_addmm_activation(o.b, x2, o.w.t(), 1, 1, true);
+    }
+    y = y.view(sizes);
+    if (ty.defined()) ty = ty.view(sizes);
+  }
+  return py::cast(finish(y, ty, nullptr, level));
 }
 
 // x.chunk(n, -1) of a modulation tensor, tangent included
@@ -1059,7 +1091,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("gelu_tanh", [](const Tensor& x) { return activation(x, Act::gelu); });
   m.def("silu", [](const Tensor& x) { return activation(x, Act::silu); });
   m.def("linear", &linear);
-  m.def("linear_gelu_inference", &linear_gelu_inference);
+  m.def("linear_gelu", &linear_gelu);
   m.def("chunk_last", &chunk_last);
   m.def("modulations", &modulations);
 }

@@ -1,0 +1,89 @@
+"""The package's own product kernel (dmf_linear_fwd) against fp32 products of the same bf16 operands."""
+import pytest
+import torch
+
+from dmf_amd import _lib, block_ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# operands are exact and sums in fp32 (up to 4608 terms: below 1e-5); what is left is the rounding of the result to bf16, at most 2^-9 of
+# an element, and for gelu an exp2 and a reciprocal good to 2^-21
+TOL = 2 ** -9 * 1.05
+
+
+def _operands(M, N, K, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    return r(M, K).bfloat16(), r(M, K).bfloat16(), (r(N, K) * K ** -0.5).bfloat16(), r(N).bfloat16()
+
+
+def _call(x, tx, w, b, gelu):
+    lib, (M, K), N = _lib.load(), x.shape, w.shape[0]
+    # (one row more than the result: what is written past it shows)
+    y = torch.full((M + 1, N), 7.0, device=DEV, dtype=torch.bfloat16)
+    ty = torch.full_like(y, 7.0) if tx is not None else None
+    p = lambda t: None if t is None else t.data_ptr()
+    rc = lib.dmf_linear_fwd(p(x), p(tx), p(w), p(b), p(y), p(ty), M, N, K, gelu, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    for t in (y, ty):
+        assert t is None or (t[M] == 7.0).all()
+    return y[:M], None if ty is None else ty[:M]
+
+
+def _check(got, ref):
+    assert (got.float() - ref).norm() <= TOL * ref.norm()
+    assert ((got.float() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all()
+
+
+# the four tiles (64 x 64; 128 x 64; 128 x 128; 128 x 192) and their edges: one row, a row past a tile, columns that fill none, one step
+SIZES = [(1, 8, 64), (63, 64, 64), (65, 72, 128), (129, 200, 192), (333, 1152, 384), (4096, 768, 768), (4097, 712, 640), (2048, 2304, 768),
+         (2000, 3456, 128), (8192, 2304, 768), (16384, 2304, 64), (16389, 2296, 320), (256, 768, 3072)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_products(M, N, K):
+    x, tx, w, b = _operands(M, N, K)
+    ref, tref = torch.nn.functional.linear(x.float(), w.float(), b.float()), tx.float() @ w.float().t()
+    _check(_call(x, None, w, b, 0)[0], ref)
+    _check(_call(x, None, w, None, 0)[0], ref - b.float())
+    y, ty = _call(x, tx, w, b, 0)
+    _check(y, ref)
+    _check(ty, tref)
+    gelu = lambda t: torch.nn.functional.gelu(t, approximate="tanh")
+    act, tact = torch.func.jvp(gelu, (ref.double(),), (tref.double(),))
+    for tangent in (None, tx):
+        y, ty = _call(x, tangent, w, b, 1)
+        assert (y.float() - act).norm() <= TOL * act.norm()
+        if tangent is not None:
+            assert (ty.float() - tact).norm() <= TOL * tact.norm()
+
+
+def test_what_the_entry_refuses():
+    x, tx, w, b = _operands(64, 64, 64)
+    lib, p = _lib.load(), lambda t: t.data_ptr()
+    y = torch.empty(64, 64, device=DEV, dtype=torch.bfloat16)
+    for (M, N, K), rc in (((64, 64, 32), -3), ((64, 60, 64), -3), ((0, 64, 64), -3)):
+        assert lib.dmf_linear_fwd(p(x), None, p(w), p(b), p(y), None, M, N, K, 0, None) == rc
+    assert lib.dmf_linear_fwd(p(x), p(tx), p(w), p(b), p(y), None, 64, 64, 64, 0, None) == -5
+    assert lib.dmf_linear_fwd(p(x) + 2, None, p(w), p(b), p(y), None, 64, 64, 64, 0, None) == -6
+
+
+@pytest.mark.parametrize("dual", [False, True])
+def test_layers_take_it_for_what_it_covers(dual):
+    """dual_linear and linear_gelu_tanh on dense, strided, misaligned and other-typed operands: the same values as library products (two
+    roundings apart at most: their pre-activation is rounded, the fused one's is not)."""
+    x, tx, w, b = _operands(130, 256, 128)
+    wide = torch.randn(130, 256, device=DEV).bfloat16()
+    cases = [(x, tx), (wide[:, ::2], tx), (wide[:, 1:129], tx), (x.float(), tx.float()), (x.reshape(2, 65, 128), tx.reshape(2, 65, 128))]
+    for i, (a, ta) in enumerate(cases):
+        wt, bias = (w.float(), b.float()) if a.dtype == torch.float32 else (w, b)
+        for fn, ref in ((block_ops.dual_linear, torch.nn.functional.linear),
+                        (block_ops.linear_gelu_tanh, lambda t, w, b: torch.nn.functional.gelu(torch.nn.functional.linear(t, w, b), approximate="tanh"))):
+            if dual:
+                got = torch.func.jvp(lambda t: fn(t, wt, bias), (a,), (ta,))
+                exp = torch.func.jvp(lambda t: ref(t, wt.float(), bias.float()), (a.float(),), (ta.float(),))
+            else:
+                with torch.no_grad():
+                    got, exp = (fn(a, wt, bias),), (ref(a.float(), wt.float(), bias.float()),)
+            for g, e in zip(got, exp):
+                assert g.shape == e.shape and (g.float() - e).norm() <= 2 * TOL * e.norm(), (i, fn)
