@@ -7,7 +7,9 @@
 // operands as they lie in memory (16 bytes of a row per lane), each is loaded once and used for every 32-row tile of S and dS,
 // which the waves of a work-group share through the first-level cache.  No LDS, no barrier: with all groups in one grid some 1700
 // waves are resident, four weight steps in flight each.
-//   MODULATION_FIGURES
+// us, both silu launches included, against a library product per group (and stream): C = 768, 12 blocks, B = 16 33 (the kernel 29, 3.0 TB/s)
+// against 89, B = 64 with tangents 85 against 201, B = 128 with tangents 144 against 227; C = 1152, 28 blocks, B = 16 125 (3.6 TB/s) against
+// 251, B = 32 with tangents 221 against 404.  From 64 rows up the operand reads of S and dS, not the weights, take the time.
 #include "attn_common.h"
 #include "attn_kernels.h"
 #include "../../include/dmf_fused.h"
