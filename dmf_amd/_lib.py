@@ -64,6 +64,9 @@ FUSED_SIGNATURES = {
     "dmf_modulation_fwd": (c_int, [_P] * 5 + [_I] * 6 + [_P]),
     "dmf_linear_plan": (c_int, [_L] + [_I] * 4),
     "dmf_linear_fwd": (c_int, [_P] * 6 + [_I] * 4 + [_P]),
+    "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
+    "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
+    "dmf_linear_wgrad": (c_int, [_P] * 4 + [_I] * 3 + [_P]),
 }
 
 _lib = None
@@ -675,6 +678,24 @@ def linear_fwd(x, tx, w, bias, gelu: bool = False):
         ty = None if tx is None else _empty((M, N), x.dtype, x.device)
         _check(load().dmf_linear_fwd(_ptr(x), _ptr(tx), _ptr(w), _ptr(bias), _ptr(y), _ptr(ty), M, N, K, gelu, _stream(x)), "dmf_linear_fwd")
     return y, ty
+
+
+def linear_wgrad(g, x):
+    """``g^T x`` in fp32 for (M, N) g and (M, K) x by the package's own kernel; None where a library product is the better choice or
+    the operands are not plain dense bf16 tensors on the GPU."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or any(type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16
+                   for t in (g, x)) or torch._C._functorch.peek_interpreter_stack() is not None):
+        return None
+    (M, N), K = g.shape, x.shape[1]
+    if max(M, N, K) > 0x7fffffff or not load().dmf_linear_wgrad_plan(M, N, K):
+        return None
+    with torch.cuda.device(g.device):
+        gw = _empty((N, K), torch.float32, g.device)
+        need = load().dmf_linear_wgrad_workspace_floats(M, N, K)
+        ws = _empty((need,), torch.float32, g.device) if need else None
+        _check(load().dmf_linear_wgrad(_ptr(g), _ptr(x), _ptr(gw), _ptr(ws), M, N, K, _stream(g)), "dmf_linear_wgrad")
+    return gw
 
 
 def colsum(x, out_dtype=None):

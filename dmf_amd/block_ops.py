@@ -268,7 +268,9 @@ class DualLinearFunc(torch.autograd.Function):
             if want_gw:
                 x2 = x.reshape(-1, x.shape[-1]).to(w.dtype)
                 if g2.is_cuda and g2.dtype != ctx.weight_dtype and ctx.weight_dtype == torch.float32:
-                    gw = torch.mm(g2.t(), x2, out_dtype=torch.float32)   # the GEMM stores its fp32 accumulators: no cast kernel
+                    gw = None if torch.is_grad_enabled() else _lib.linear_wgrad(g2, x2)
+                    if gw is None:
+                        gw = torch.mm(g2.t(), x2, out_dtype=torch.float32)   # the GEMM stores its fp32 accumulators: no cast kernel
                 else:
                     gw = (g2.t() @ x2).to(ctx.weight_dtype)
             if want_gb:

@@ -267,3 +267,207 @@ extern "C" int dmf_linear_fwd(const void* x, const void* tx, const void* w, cons
   const int tile = dmf::linear_tile(M, N, K, jvp);
   return gelu ? dmf::launch_linear_tile<dmf::kLinGelu>(tile, p, false, stm) : dmf::launch_linear_tile<dmf::kLinPlain>(tile, p, jvp, stm);
 }
+
+namespace dmf {
+
+// ---- weight gradient: gw = g^T x, contracted over the rows of both ----------------------------------------------------------
+//
+// The result is small (4608 x 1152 at most in the models) and the contraction thousands of rows deep, so that output tiles alone leave
+// most CUs idle: the library's products reached 160 to 400 TFLOP/s here.  The rows are split over work-groups until the grid fills the
+// chip; each writes its fp32 sums to the workspace and a second kernel adds them in a fixed order.
+// Both tiles lie in LDS as they lie in memory, 64 rows of 64-column panels (128-byte lines); the transposed reads give operands that
+// contract over rows.  The 64-byte halves of rows 4 i + 2 and 4 i + 3 are exchanged, so that the 32 lanes of a pass, which read 64 bytes
+// of four consecutive rows, meet all 64 banks.  Step, stages and register plan are linear_kernel's.
+struct WgradParams {
+  const __bf16 *g, *x;   // (M, N), (M, K)
+  float* out;            // gw, or with splits the partial sums, N * K apart
+  int M, N, K, ntiles, ktiles, splits, per;   // per: steps of 64 rows per split
+};
+constexpr int kWgN = 128, kWgK = 192, kWgStage = (kWgN + kWgK) * 128;
+
+__global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5, i16 = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // the tiles of one split are neighbours, in bands of six k tiles: the work-groups of an XCD share few columns of either operand in its L2
+  const uint32_t per = (uint32_t)p.ntiles * p.ktiles, id = xcd_remap(blockIdx.x, gridDim.x), split = id / per, tile = id - split * per;
+  const uint32_t band = tile / (6 * p.ntiles), in = tile - band * 6 * p.ntiles, wide = min((uint32_t)p.ktiles - 6 * band, 6u);
+  const int n0 = (int)(in / wide) * kWgN, k0 = (int)(6 * band + in % wide) * kWgK;
+  const int first = (int)split * p.per, steps = max(0, min(p.per, (p.M + 63) / 64 - first));
+
+  // the whole operands from the tile's first column on: rows past the last read as zeros, columns past the last are not stored
+  const uint32_t gb = (uint32_t)p.N * 2, xb = (uint32_t)p.K * 2;
+  const __amdgpu_buffer_rsrc_t rg = make_rows_rsrc(p.g + n0, gb, p.M, (int)(gb - n0 * 2));
+  const __amdgpu_buffer_rsrc_t rx = make_rows_rsrc(p.x + k0, xb, p.M, (int)(xb - k0 * 2));
+  const uint32_t vec = ((lane & 7) ^ (((lane >> 4) & 1) * 4)) * 16, gvoff = (lane >> 3) * gb + vec, xvoff = (lane >> 3) * xb + vec;
+  auto issue = [&](int step) {
+    char* st = smem + (step & 1) * kWgStage;
+    const uint32_t row0 = (uint32_t)(first + step) * 64;
+#pragma unroll
+    for (int j = 0; j < kWgN / 32; ++j) {   // block b: rows 8 (b % 8) .. + 7 of panel b / 8
+      const int b = 4 * j + wave;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)(st + b * 1024), 16, gvoff,
+                                               (row0 + (b & 7) * 8) * gb + (b >> 3) * 128, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < kWgK / 32; ++j) {
+      const int b = 4 * j + wave;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(st + kWgN * 128 + b * 1024), 16, xvoff,
+                                               (row0 + (b & 7) * 8) * xb + (b >> 3) * 128, 0, 0);
+    }
+  };
+
+  // lane address of 32-column group c of either tile (see lds_col_operand); rows 16 s + 8 h on: + 2048 s + 1024 h
+  const uint32_t in_panel = (4 * g + (i16 >> 2)) * 128 + ((lane >> 4) & 1) * 32 + (i16 & 3) * 8, swap = (i16 >> 3) & 1;
+  auto group = [&](uint32_t base, int c) { return base + (c >> 1) * 8192 + in_panel + (((uint32_t)c & 1) ^ swap) * 64; };
+  uint32_t gaddr[2], xaddr[3];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) gaddr[m] = group(lds_addr(smem), 2 * wm + m);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) xaddr[n] = group(lds_addr(smem) + kWgN * 128, 3 * wn + n);
+
+  f32x16 acc[3][2];
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+#pragma unroll
+    for (int m = 0; m < 2; ++m) acc[n][m] = f32x16{0};
+  issue(0);
+  for (int s = 0; s < steps; ++s) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's share of step s is in LDS
+    asm volatile("s_barrier" ::: "memory");   // everybody's is, and everybody has its operands of step s - 1
+    const uint32_t st = (s & 1) * kWgStage;
+    TrPair G[4][2], X[4][3];
+    auto read = [&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+#pragma unroll
+      for (int m = 0; m < 2; ++m) G[c][m] = lds_tr16_issue<c * 2048, c * 2048 + 1024>(gaddr[m] + st);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) X[c][n] = lds_tr16_issue<c * 2048, c * 2048 + 1024>(xaddr[n] + st);
+    };
+    read(std::integral_constant<int, 0>{});
+    read(std::integral_constant<int, 1>{});
+    read(std::integral_constant<int, 2>{});
+    read(std::integral_constant<int, 3>{});
+    issue(s + 1);   // (past the last step too: rows of the next split, or zeros; nothing reads them, the end waits for them)
+    auto chunk = [&](auto cc) {
+      constexpr int c = decltype(cc)::value, LATER = (3 - c) * 10 < 15 ? (3 - c) * 10 : 15;
+      lds_tr16_wait<LATER>(G[c][0], G[c][1]);
+      lds_tr16_wait<LATER>(X[c][0], X[c][1]);
+      lds_tr16_wait<LATER>(X[c][2]);
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tr_operand(X[c][n]).v),
+                                                              __builtin_bit_cast(bf16x8, tr_operand(G[c][m]).v), acc[n][m], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    chunk(std::integral_constant<int, 0>{});
+    chunk(std::integral_constant<int, 1>{});
+    chunk(std::integral_constant<int, 2>{});
+    chunk(std::integral_constant<int, 3>{});
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // (no DMA may outlive the work-group's LDS)
+  float* out = p.out + (int64_t)split * p.N * p.K;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int row = n0 + 64 * wm + 32 * m + c32;
+#pragma unroll
+    for (int n = 0; n < 3; ++n)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int col = k0 + 96 * wn + 32 * n + 8 * q + 4 * g;
+        const f32x16& a = acc[n][m];
+        if (row < p.N && col < p.K)
+          *reinterpret_cast<f32x4*>(out + (int64_t)row * p.K + col) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+      }
+  }
+}
+
+// out = the sum of `splits` arrays of 4 n4 floats, in order
+struct SumSplitsParams { const f32x4* part; f32x4* out; int64_t n4; int splits; };
+__global__ __launch_bounds__(256) void sum_splits_kernel(const SumSplitsParams p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.n4) return;
+  f32x4 s = p.part[i];
+  for (int j = 1; j < p.splits; j += 4) {
+    f32x4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = j + k < p.splits ? p.part[i + (j + k) * p.n4] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s += v[k];
+  }
+  p.out[i] = s;
+}
+
+// Splits of the rows: the least of the estimated times, a step and a work-group's start and end fitted to M = 8192 .. 32768, plus the
+// partial sums' way through memory (written once, read once, at some 5 TB/s) and a launch.
+static int wgrad_splits(int64_t M, int64_t N, int64_t K) {
+  const int64_t cus = compute_units(), tiles = ((N + kWgN - 1) / kWgN) * ((K + kWgK - 1) / kWgK), total = (M + 63) / 64;
+  int best = 1;
+  int64_t cost_best = INT64_MAX;
+  for (int s = 1; s <= 64 && s <= total; ++s) {
+    const int64_t per = (total + s - 1) / s, wgs = tiles * s, rounds = wgs / (2 * cus), rest = wgs % (2 * cus);
+    const int64_t one = 95 * per + 350, two = 125 * per + 450;   // one, two work-groups on a CU, in 10 ns
+    int64_t cost = rounds * two + (rest == 0 ? 0 : rest <= cus ? one : one + (two - one) * (35 * cus + 65 * (rest - cus)) / (100 * cus));
+    if (s > 1) cost += N * K * 4 * (2 * s + 1) / 50000 + 300;
+    if (cost < cost_best) {
+      cost_best = cost;
+      best = s;
+    }
+  }
+  return best;
+}
+
+static bool wgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
+  return M >= 1 && N >= 8 && N % 8 == 0 && K >= 8 && K % 8 == 0 && M * K < (int64_t)1 << 30 && N * K < (int64_t)1 << 30 && M * N < (int64_t)1 << 30;
+}
+
+}  // namespace dmf
+
+extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
+  if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return -1;
+  const int s = dmf::wgrad_splits(M, N, K);
+  return s > 1 ? (int64_t)s * N * K : 0;
+}
+
+// Which weight gradients this kernel is the faster one for (us, library -> here; the library's launch alone takes 20 us of host time):
+//   M 1000: 768 x 768 20.5 -> 15.6, 4608 x 1152 29 -> 20;  M 2048: 1536 x 384 20.0 -> 18.4, but 2304 x 768 21 against 23, 3456 x 1152 28 against 34;
+//   M 4096: 3072 x 768 42 -> 36, 1152 x 1152 33 -> 25, but 3456 x 1152 46 against 51;  M 8192: 3456 x 1152 83 -> 81, 4608 x 1152 119 -> 101,
+//   1152 x 4608 118 -> 97, 1152 x 1152 61 -> 36, 768 x 768 48 -> 24;  M 16384: 3072 x 768 172 -> 94, 4608 x 1152 327 -> 183 (948 TFLOP/s);
+//   widths that 192 columns do not divide lose on large results: 4096 x 1024 M 8192 86 against 89.  Results beyond 8 M elements are not measured.
+extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
+  if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return 0;
+  const int64_t result = (int64_t)N * K;
+  if (result > 8000000) return 0;
+  if (M < 1536) return 1;
+  if (M < 4096) return result <= 600000;
+  if (M < 8192) return result <= 2400000;
+  return K % dmf::kWgK == 0 || result <= 3200000;
+}
+
+extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* workspace, int M, int N, int K, void* stream) {
+  if (g == nullptr || x == nullptr || gw == nullptr) return DMF_ATTN_ENULL;
+  if (!dmf::wgrad_shape_ok(M, N, K)) return DMF_ATTN_ESHAPE;
+  const int splits = dmf::wgrad_splits(M, N, K);
+  if (splits > 1 && workspace == nullptr) return DMF_ATTN_ENULL;
+  for (const void* q : {g, x, (const void*)gw, (const void*)workspace})
+    if (reinterpret_cast<uintptr_t>(q) % 16) return DMF_ATTN_EALIGN;
+  dmf::WgradParams p{};
+  p.g = static_cast<const __bf16*>(g);
+  p.x = static_cast<const __bf16*>(x);
+  p.out = splits > 1 ? workspace : gw;
+  p.M = M; p.N = N; p.K = K;
+  p.ntiles = (N + dmf::kWgN - 1) / dmf::kWgN;
+  p.ktiles = (K + dmf::kWgK - 1) / dmf::kWgK;
+  p.splits = splits;
+  p.per = ((M + 63) / 64 + splits - 1) / splits;
+  static bool lds_ok[64] = {};
+  if (!dmf::ensure_dynamic_lds(dmf::linear_wgrad_kernel, 2 * dmf::kWgStage, lds_ok)) return -7;
+  auto stm = static_cast<hipStream_t>(stream);
+  const int rc = dmf::launch_kernel(dmf::linear_wgrad_kernel, dim3((uint32_t)p.ntiles * p.ktiles * splits), dim3(256), 2 * dmf::kWgStage, stm, p);
+  if (rc != 0 || splits == 1) return rc;
+  const int64_t n4 = (int64_t)N * K / 4;
+  const dmf::SumSplitsParams q{reinterpret_cast<const f32x4*>(workspace), reinterpret_cast<f32x4*>(gw), n4, splits};
+  return dmf::launch_kernel(dmf::sum_splits_kernel, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, stm, q);
+}

@@ -87,3 +87,49 @@ def test_layers_take_it_for_what_it_covers(dual):
                     got, exp = (fn(a, wt, bias),), (ref(a.float(), wt.float(), bias.float()),)
             for g, e in zip(got, exp):
                 assert g.shape == e.shape and (g.float() - e).norm() <= 2 * TOL * e.norm(), (i, fn)
+
+
+# ---- weight gradient (dmf_linear_wgrad): products exact in fp32, sums in fp32 -- M terms in some order, error below sqrt(M) 2^-24 of the
+# sum of magnitudes on random data; 2e-6 covers M = 16389 (7.6e-6 of a worst single element, checked against the largest)
+WGRAD = [(1, 8, 8), (63, 64, 64), (64, 128, 192), (65, 136, 200), (129, 120, 184), (333, 1152, 1152), (2048, 384, 1536), (4097, 712, 328),
+         (8192, 1152, 1152), (8192, 3456, 1152), (4096, 4608, 1152), (4096, 1152, 4608), (16389, 768, 768), (32768, 96, 200), (20001, 384, 384)]
+
+
+@pytest.mark.parametrize("M,N,K", WGRAD)
+def test_weight_gradient(M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    # (rows past the last hold values that would show if they were summed)
+    g, x = (torch.randn(M + 64, C, generator=gen, device=DEV).bfloat16() for C in (N, K))
+    g[M:], x[M:] = 1e4, 1e4
+    lib = _lib.load()
+    need = lib.dmf_linear_wgrad_workspace_floats(M, N, K)
+    out, ws = torch.full((N + 1, K), 7.0, device=DEV), torch.full((max(need, 4) + 4,), float("nan"), device=DEV)
+    assert lib.dmf_linear_wgrad(g.data_ptr(), x.data_ptr(), out.data_ptr(), ws.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+    ref = g[:M].double().t() @ x[:M].double()
+    assert (out[N] == 7.0).all() and ws[need:].isnan().all()
+    assert (out[:N] - ref).norm() <= 2e-6 * ref.norm() and (out[:N] - ref).abs().max() <= 1e-5 * ref.abs().max()
+
+
+def test_weight_gradient_routes():
+    """Layer backward under autocast with dense and strided gradients, native and Python route: the fp32 product of the bf16 operands."""
+    x, _, w, b = _operands(130, 256, 128)
+    weight, bias, dense = w.float().requires_grad_(), b.float().requires_grad_(), torch.randn(130, 256, device=DEV).bfloat16()
+    for gy in (dense, torch.randn(256, 130, device=DEV).bfloat16().t(), dense[:1].expand(130, 256)):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = block_ops.dual_linear(x, weight, bias)
+        (gw,) = torch.autograd.grad(y, weight, gy)
+        ref = gy.double().t() @ x.double()
+        assert gw.dtype == torch.float32 and (gw - ref).norm() <= 2e-6 * ref.norm()
+    own = _lib.linear_wgrad(dense, x)
+    assert own is None or (own - dense.double().t() @ x.double()).norm() <= 2e-6 * own.norm()
+    assert _lib.linear_wgrad(dense[:, ::2], x) is None and _lib.linear_wgrad(dense.float(), x.float()) is None
+
+
+def test_weight_gradient_refuses():
+    g, x = torch.randn(64, 64, device=DEV).bfloat16(), torch.randn(64, 64, device=DEV).bfloat16()
+    out, lib = torch.empty(64, 64, device=DEV), _lib.load()
+    call = lambda g, x, o, M, N, K: lib.dmf_linear_wgrad(g, x, o, None, M, N, K, None)
+    p, q, o = g.data_ptr(), x.data_ptr(), out.data_ptr()
+    assert call(p, q, o, 0, 64, 64) == -3 and call(p, q, o, 64, 60, 64) == -3 and call(p, q, o, 64, 64, 12) == -3
+    assert call(None, q, o, 64, 64, 64) == -5 and call(p + 2, q, o, 64, 64, 64) == -6
+    assert lib.dmf_linear_wgrad_workspace_floats(64, 60, 64) == -1
