@@ -66,7 +66,7 @@ FUSED_SIGNATURES = {
     "dmf_linear_fwd": (c_int, [_P] * 6 + [_I] * 4 + [_P]),
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
     "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
-    "dmf_linear_wgrad": (c_int, [_P] * 4 + [_I] * 3 + [_P]),
+    "dmf_linear_wgrad": (c_int, [_P] * 5 + [_I] * 3 + [_P]),
 }
 
 _lib = None
@@ -680,8 +680,8 @@ def linear_fwd(x, tx, w, bias, gelu: bool = False):
     return y, ty
 
 
-def linear_wgrad(g, x):
-    """``g^T x`` in fp32 for (M, N) g and (M, K) x by the package's own kernel; None where a library product is the better choice or
+def linear_wgrad(g, x, bias: bool = False):
+    """``(g^T x, column sums of g or None)`` in fp32 for (M, N) g and (M, K) x by the package's own kernel; None where a library product is the better choice or
     the operands are not plain dense bf16 tensors on the GPU."""
     if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
             or any(type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16
@@ -692,10 +692,11 @@ def linear_wgrad(g, x):
         return None
     with torch.cuda.device(g.device):
         gw = _empty((N, K), torch.float32, g.device)
+        gb = _empty((N,), torch.float32, g.device) if bias else None
         need = load().dmf_linear_wgrad_workspace_floats(M, N, K)
         ws = _empty((need,), torch.float32, g.device) if need else None
-        _check(load().dmf_linear_wgrad(_ptr(g), _ptr(x), _ptr(gw), _ptr(ws), M, N, K, _stream(g)), "dmf_linear_wgrad")
-    return gw
+        _check(load().dmf_linear_wgrad(_ptr(g), _ptr(x), _ptr(gw), _ptr(gb), _ptr(ws), M, N, K, _stream(g)), "dmf_linear_wgrad")
+    return gw, gb
 
 
 def colsum(x, out_dtype=None):

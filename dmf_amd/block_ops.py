@@ -268,12 +268,14 @@ class DualLinearFunc(torch.autograd.Function):
             if want_gw:
                 x2 = x.reshape(-1, x.shape[-1]).to(w.dtype)
                 if g2.is_cuda and g2.dtype != ctx.weight_dtype and ctx.weight_dtype == torch.float32:
-                    gw = None if torch.is_grad_enabled() else _lib.linear_wgrad(g2, x2)
-                    if gw is None:
+                    own = None if torch.is_grad_enabled() else _lib.linear_wgrad(g2, x2, want_gb and ctx.bias_dtype == torch.float32)
+                    if own is not None:
+                        gw, gb = own
+                    else:
                         gw = torch.mm(g2.t(), x2, out_dtype=torch.float32)   # the GEMM stores its fp32 accumulators: no cast kernel
                 else:
                     gw = (g2.t() @ x2).to(ctx.weight_dtype)
-            if want_gb:
+            if want_gb and gb is None:
                 # torch's multi-block column reduction clears its scratch with a memset node, which does not survive
                 # HIP-graph replay; the library's two-stage sum has no such node
                 if g2.is_cuda and g2.shape[1] % 8 == 0:

@@ -793,8 +793,9 @@ Tensor column_sum(const Tensor& x, at::ScalarType dt) {
   return out;
 }
 
-// g^T x in fp32: the package's own kernel where it reads the operands as they are, else a library product that stores its accumulators.
-Tensor weight_gradient(const Tensor& g, const Tensor& x) {
+// g^T x in fp32 and, with `gb`, the column sums of g: the package's own kernel where it reads the operands as they are, else a library
+// product that stores its accumulators (and no sums).
+Tensor weight_gradient(const Tensor& g, const Tensor& x, Tensor* gb) {
   const auto readable16 = [](const Tensor& t) {
     return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
   };
@@ -802,8 +803,9 @@ Tensor weight_gradient(const Tensor& g, const Tensor& x) {
   if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !readable16(g) || !readable16(x) || !dmf_linear_wgrad_plan(M, (int)N, (int)K))
     return at::mm(g.t(), x, at::kFloat);
   const int64_t need = dmf_linear_wgrad_workspace_floats(M, (int)N, (int)K);
+  if (gb) *gb = empty({N}, at::kFloat, x);
   const Tensor gw = empty({N, K}, at::kFloat, x), ws = need > 0 ? workspace(need, x) : Tensor();
-  check(dmf_linear_wgrad(ptr(g), ptr(x), static_cast<float*>(mptr(gw)), need > 0 ? static_cast<float*>(mptr(ws)) : nullptr, (int)M, (int)N, (int)K,
+  check(dmf_linear_wgrad(ptr(g), ptr(x), static_cast<float*>(mptr(gw)), gb ? static_cast<float*>(mptr(*gb)) : nullptr, need > 0 ? static_cast<float*>(mptr(ws)) : nullptr, (int)M, (int)N, (int)K,
                          stream_of(x)),
         "dmf_linear_wgrad");
   return gw;
@@ -826,10 +828,10 @@ variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w
   }
   auto parameters = [&] {
     if (want_gw) {
-      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = weight_gradient(g2, x2);
+      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = weight_gradient(g2, x2, want_gb && b_type == at::kFloat ? &gb : nullptr);
       else gw = at::mm(g2.t(), x2).to(w_type);
     }
-    if (want_gb) gb = column_sum(dense(g2), b_type);
+    if (want_gb && !gb.defined()) gb = column_sum(dense(g2), b_type);
   };
   if (fork) {
     const c10::impl::VirtualGuardImpl impl(at::kCUDA);

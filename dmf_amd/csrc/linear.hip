@@ -281,6 +281,7 @@ namespace dmf {
 struct WgradParams {
   const __bf16 *g, *x;   // (M, N), (M, K)
   float* out;            // gw, or with splits the partial sums, N * K apart
+  float* bias;           // the column sums of g (partial ones: N apart), or null
   int M, N, K, ntiles, ktiles, splits, per;   // per: steps of 64 rows per split
 };
 constexpr int kWgN = 128, kWgK = 192, kWgStage = (kWgN + kWgK) * 128;
@@ -331,6 +332,11 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
   for (int n = 0; n < 3; ++n)
 #pragma unroll
     for (int m = 0; m < 2; ++m) acc[n][m] = f32x16{0};
+  // column sums of g, the bias gradient: the first k tile's work-groups have every element in registers; a step's 64 rows are summed by
+  // themselves, then added to the others' (a separate column sum read g again, 11 us and a 4 us reduction a layer: four-block XL/2-width
+  // training step 8.59 -> 8.42 ms)
+  const bool sums = p.bias != nullptr && k0 == 0 && wn == 0;
+  float total[2] = {0.f, 0.f};
   issue(0);
   for (int s = 0; s < steps; ++s) {
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's share of step s is in LDS
@@ -366,12 +372,30 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
     chunk(std::integral_constant<int, 1>{});
     chunk(std::integral_constant<int, 2>{});
     chunk(std::integral_constant<int, 3>{});
+    if (sums) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        float t = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t pair = tr_operand(G[c][m]).v[e];
+            t += __uint_as_float(pair << 16) + __uint_as_float(pair & 0xffff0000u);
+          }
+        total[m] += t;
+      }
+    }
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // (no DMA may outlive the work-group's LDS)
   float* out = p.out + (int64_t)split * p.N * p.K;
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     const int row = n0 + 64 * wm + 32 * m + c32;
+    if (sums) {
+      const float both = total[m] + __shfl_xor(total[m], 32);   // the halves of a wave hold different rows
+      if (g == 0 && row < p.N) p.bias[(int64_t)split * p.N + row] = both;
+    }
 #pragma unroll
     for (int n = 0; n < 3; ++n)
 #pragma unroll
@@ -384,20 +408,24 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
   }
 }
 
-// out = the sum of `splits` arrays of 4 n4 floats, in order
-struct SumSplitsParams { const f32x4* part; f32x4* out; int64_t n4; int splits; };
+// out = the sum of `splits` arrays of 4 n4 floats, in order; behind them, arrays of 4 b4 floats into bias
+struct SumSplitsParams { const f32x4* part; f32x4 *out, *bias; int64_t n4, b4; int splits; };
 __global__ __launch_bounds__(256) void sum_splits_kernel(const SumSplitsParams p) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n4) return;
-  f32x4 s = p.part[i];
+  if (i >= p.n4 + p.b4) return;
+  const bool weight = i < p.n4;
+  const int64_t stride = weight ? p.n4 : p.b4;
+  const f32x4* part = weight ? p.part + i : p.part + p.splits * p.n4 + (i - p.n4);
+  f32x4 s = part[0];
   for (int j = 1; j < p.splits; j += 4) {
     f32x4 v[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = j + k < p.splits ? p.part[i + (j + k) * p.n4] : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < 4; ++k) v[k] = j + k < p.splits ? part[(j + k) * stride] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < 4; ++k) s += v[k];
   }
-  p.out[i] = s;
+  if (weight) p.out[i] = s;
+  else p.bias[i - p.n4] = s;
 }
 
 // Splits of the rows: the least of the estimated times, a step and a work-group's start and end fitted to M = 8192 .. 32768, plus the
@@ -428,7 +456,7 @@ static bool wgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
 extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
   if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return -1;
   const int s = dmf::wgrad_splits(M, N, K);
-  return s > 1 ? (int64_t)s * N * K : 0;
+  return s > 1 ? (int64_t)s * N * (K + 1) : 0;
 }
 
 // Which weight gradients this kernel is the faster one for (us, library -> here; the library's launch alone takes 20 us of host time):
@@ -446,17 +474,18 @@ extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   return K % dmf::kWgK == 0 || result <= 3200000;
 }
 
-extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* workspace, int M, int N, int K, void* stream) {
+extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream) {
   if (g == nullptr || x == nullptr || gw == nullptr) return DMF_ATTN_ENULL;
   if (!dmf::wgrad_shape_ok(M, N, K)) return DMF_ATTN_ESHAPE;
   const int splits = dmf::wgrad_splits(M, N, K);
   if (splits > 1 && workspace == nullptr) return DMF_ATTN_ENULL;
-  for (const void* q : {g, x, (const void*)gw, (const void*)workspace})
+  for (const void* q : {g, x, (const void*)gw, (const void*)gbias, (const void*)workspace})
     if (reinterpret_cast<uintptr_t>(q) % 16) return DMF_ATTN_EALIGN;
   dmf::WgradParams p{};
   p.g = static_cast<const __bf16*>(g);
   p.x = static_cast<const __bf16*>(x);
   p.out = splits > 1 ? workspace : gw;
+  p.bias = gbias == nullptr ? nullptr : splits > 1 ? workspace + (int64_t)splits * N * K : gbias;
   p.M = M; p.N = N; p.K = K;
   p.ntiles = (N + dmf::kWgN - 1) / dmf::kWgN;
   p.ktiles = (K + dmf::kWgK - 1) / dmf::kWgK;
@@ -467,7 +496,7 @@ extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* 
   auto stm = static_cast<hipStream_t>(stream);
   const int rc = dmf::launch_kernel(dmf::linear_wgrad_kernel, dim3((uint32_t)p.ntiles * p.ktiles * splits), dim3(256), 2 * dmf::kWgStage, stm, p);
   if (rc != 0 || splits == 1) return rc;
-  const int64_t n4 = (int64_t)N * K / 4;
-  const dmf::SumSplitsParams q{reinterpret_cast<const f32x4*>(workspace), reinterpret_cast<f32x4*>(gw), n4, splits};
-  return dmf::launch_kernel(dmf::sum_splits_kernel, dim3((uint32_t)((n4 + 255) / 256)), dim3(256), 0, stm, q);
+  const int64_t n4 = (int64_t)N * K / 4, b4 = gbias == nullptr ? 0 : N / 4;
+  const dmf::SumSplitsParams q{reinterpret_cast<const f32x4*>(workspace), reinterpret_cast<f32x4*>(gw), reinterpret_cast<f32x4*>(gbias), n4, b4, splits};
+  return dmf::launch_kernel(dmf::sum_splits_kernel, dim3((uint32_t)((n4 + b4 + 255) / 256)), dim3(256), 0, stm, q);
 }

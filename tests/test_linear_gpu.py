@@ -103,9 +103,12 @@ def test_weight_gradient(M, N, K):
     g[M:], x[M:] = 1e4, 1e4
     lib = _lib.load()
     need = lib.dmf_linear_wgrad_workspace_floats(M, N, K)
+    gb = torch.full((N + 4,), 7.0, device=DEV)
     out, ws = torch.full((N + 1, K), 7.0, device=DEV), torch.full((max(need, 4) + 4,), float("nan"), device=DEV)
-    assert lib.dmf_linear_wgrad(g.data_ptr(), x.data_ptr(), out.data_ptr(), ws.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+    assert lib.dmf_linear_wgrad(g.data_ptr(), x.data_ptr(), out.data_ptr(), gb.data_ptr(), ws.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream) == 0
     ref = g[:M].double().t() @ x[:M].double()
+    sums = g[:M].double().sum(0)
+    assert (gb[:N] - sums).norm() <= 2e-6 * sums.norm() and (gb[N:] == 7.0).all()
     assert (out[N] == 7.0).all() and ws[need:].isnan().all()
     assert (out[:N] - ref).norm() <= 2e-6 * ref.norm() and (out[:N] - ref).abs().max() <= 1e-5 * ref.abs().max()
 
@@ -117,18 +120,19 @@ def test_weight_gradient_routes():
     for gy in (dense, torch.randn(256, 130, device=DEV).bfloat16().t(), dense[:1].expand(130, 256)):
         with torch.autocast("cuda", dtype=torch.bfloat16):
             y = block_ops.dual_linear(x, weight, bias)
-        (gw,) = torch.autograd.grad(y, weight, gy)
+        gw, gb = torch.autograd.grad(y, (weight, bias), gy)
+        assert (gb - gy.double().sum(0)).norm() <= 2e-6 * gy.double().sum(0).norm()
         ref = gy.double().t() @ x.double()
         assert gw.dtype == torch.float32 and (gw - ref).norm() <= 2e-6 * ref.norm()
-    own = _lib.linear_wgrad(dense, x)
-    assert own is None or (own - dense.double().t() @ x.double()).norm() <= 2e-6 * own.norm()
+    own = _lib.linear_wgrad(dense, x)[0]
+    assert (own - dense.double().t() @ x.double()).norm() <= 2e-6 * own.norm()
     assert _lib.linear_wgrad(dense[:, ::2], x) is None and _lib.linear_wgrad(dense.float(), x.float()) is None
 
 
 def test_weight_gradient_refuses():
     g, x = torch.randn(64, 64, device=DEV).bfloat16(), torch.randn(64, 64, device=DEV).bfloat16()
     out, lib = torch.empty(64, 64, device=DEV), _lib.load()
-    call = lambda g, x, o, M, N, K: lib.dmf_linear_wgrad(g, x, o, None, M, N, K, None)
+    call = lambda g, x, o, M, N, K: lib.dmf_linear_wgrad(g, x, o, None, None, M, N, K, None)
     p, q, o = g.data_ptr(), x.data_ptr(), out.data_ptr()
     assert call(p, q, o, 0, 64, 64) == -3 and call(p, q, o, 64, 60, 64) == -3 and call(p, q, o, 64, 64, 12) == -3
     assert call(None, q, o, 64, 64, 64) == -5 and call(p + 2, q, o, 64, 64, 64) == -6
