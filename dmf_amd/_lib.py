@@ -661,11 +661,12 @@ def rmsnorm_bwd(gy, x, gain, eps: float = 1e-6, out=None):
 def linear_fwd(x, tx, w, bias, gelu: bool = False):
     """``(x w^T + bias, tx w^T or None)`` for (M, K) x and tx, (N, K) w, by the package's own product kernel (``gelu``: activated, the
     tangent through the derivative); None where a library product is the better choice or the operands are not plain dense bf16
-    tensors on the GPU (other types and strides, subclasses, traced or watched calls)."""
+    tensors on the GPU (other types and strides, subclasses, traced or watched calls) -- or belong to several functorch levels: of
+    those only the innermost one's tangents were unpacked, and stripping the wrappers would drop the others'."""
     ops = [_raw(t) for t in (x, tx, w, bias)]
     x, tx, w, bias = ops
     present = [t for t in ops if t is not None]
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or len(_interpreters()) > 1
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous()
                    for t in present) or any(t.data_ptr() % 16 for t in present)):
         return None

@@ -173,6 +173,29 @@ def test_linear_and_chunk_stay_twice_differentiable():
             assert (got[i] - exp).norm() <= 1e-5 * exp.norm()
 
 
+@pytest.mark.parametrize("autocast", [False, True])
+def test_linear_under_two_jvp_levels(autocast):
+    """The second directional derivative of linear(x * x) and the mixed parts, against the same nesting of torch's own linear: bf16 operands
+    in the sizes that the package's product kernel takes (the values of x are small integers, so x * x and its derivatives are exact in bf16
+    and both sides round the same fp32 sums once: 2^-8 of an element apart at most)."""
+    M, N, K = 64, 128, 64
+    assert _lib.load().dmf_linear_plan(M, N, K, 1, 0) == 1
+    g = torch.Generator(device=DEV).manual_seed(2)
+    x, t = (torch.randint(-4, 5, (M, K), generator=g, device=DEV).to(torch.float32 if autocast else torch.bfloat16) for _ in range(2))
+    w, b = torch.randn(N, K, generator=g, device=DEV).bfloat16(), torch.randn(N, generator=g, device=DEV).bfloat16()
+    if autocast:
+        w, b = w.float(), b.float()
+
+    def twice(linear):
+        inner = lambda x: torch.func.jvp(lambda y: linear(y * y, w, b), (x,), (t,))
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            (o, to), (o2, to2) = torch.func.jvp(inner, (x,), (t,))
+        return o, to, o2, to2
+
+    for got, exp in zip(twice(block_ops.dual_linear), twice(torch.nn.functional.linear)):
+        assert float(exp.float().norm()) > 0 and float((got.float() - exp.float()).norm()) <= 2 ** -8 * float(exp.float().norm())
+
+
 def test_watched_calls_take_the_general_route():
     class Watch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
