@@ -164,6 +164,8 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     lv.commit(Vt, lane);
     if constexpr (JVP) ldv.commit(dVt, lane);
     if (it + NW < ntiles) request(it + NW);   // in flight during the softmax and the output products
+    // Scaled before anything is masked or compared: c2 may be negative (the order of the scores is reversed) or zero.
+    Sc *= c2;
     if ((it + 1) * 32 > p.Lkv) {
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -172,7 +174,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     float mx = fmaxf(Sc[0], Sc[1]);
 #pragma unroll
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, Sc[i]);
-    mx = xhalf_max(mx) * c2;
+    mx = xhalf_max(mx);
     if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
       const float m_new = fmaxf(m_run, mx), alpha = fast_exp2(m_run - m_new);
       m_run = m_new;
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     f32x16 E, G;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      E[i] = fast_exp2(fmaf(Sc[i], c2, -m_run));
+      E[i] = fast_exp2(Sc[i] - m_run);
       l_run += E[i];
       if constexpr (JVP) {
         G[i] = E[i] * (dS[i] * p.scale);

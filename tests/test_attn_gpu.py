@@ -923,3 +923,28 @@ def test_wide_split_forward_reads_rows_far_apart():
     exp = _lib.fwd_jvp(q, k.contiguous(), v.contiguous(), tq, k.contiguous(), v.contiguous(), D ** -0.5)
     for a, b in zip(got, exp):
         assert torch.equal(a, b)
+
+
+def _softmax_attention(q, k, v, scale):
+    q, k, v = (t.transpose(1, 2) for t in (q, k, v))
+    return (torch.softmax(q @ k.transpose(-1, -2).contiguous() * scale, -1) @ v).transpose(1, 2)
+
+
+@pytest.mark.parametrize("batch,dtype,D", [(b, torch.bfloat16, d) for b in (2, 340) for d in (64, 72, 128)] + [(2, torch.float16, d) for d in (64, 72, 80)])
+@pytest.mark.parametrize("scale", [-2.0, -0.125, 0.0])
+def test_softmax_scale_of_any_sign(scale, dtype, D, batch):
+    """Scales that turn the order of the scores around or make them all equal, with a ragged last key tile (whose absent keys must stay out) and
+    without, on grids that fill the device and on those that do not, against the fp64 formula.  bf16: the operands' own rounding, times the
+    scale; fp16: the result's."""
+    half, tol = dtype == torch.float16, {torch.bfloat16: 2e-2, torch.float16: 1e-3}[dtype]
+    for L in (100, 128):
+        g = torch.Generator(device=DEV).manual_seed(L + D)
+        x = [torch.randn(batch, L, 2, D, generator=g, device=DEV).to(dtype) for _ in range(6)]
+        o, to, _ = (_lib.fwd_jvp_half if half else _lib.fwd_jvp)(*x, scale)
+        o2, _ = (_lib.fwd_half if half else _lib.fwd)(*x[:3], scale)
+        x64 = [t[:2].double().cpu() for t in x]
+        o_ref, to_ref = torch.func.jvp(lambda q, k, v: _softmax_attention(q, k, v, scale), tuple(x64[:3]), tuple(x64[3:]))
+        for name, got, ref in (("o", o, o_ref), ("o primal", o2, o_ref), ("to", to, to_ref)):
+            # (the tangent's terms are scale * log of a probability's range larger than the result where they cancel)
+            t = tol * max(1.0, abs(scale) * D ** 0.5) if name == "to" else tol
+            assert ao.rel_l2(got[:2].double().cpu(), ref) <= t, (name, L, ao.rel_l2(got[:2].double().cpu(), ref))
