@@ -137,7 +137,9 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     if constexpr (F16) dOv.zero();
   }
   RowScale<T> gs;
-  float m_run = kLowestMax, l_run = 0.f, mu_run = 0.f;
+  // Start of the running maximum (log2 units): finite, so that a tile of nothing but keys masked by -inf weighs nothing, and no higher
+  // than any score, so that a row whose keys all carry the lowest number still has its maximum (which is subtracted exactly: weights of one).
+  float m_run = -3.40282347e38f, l_run = 0.f, mu_run = 0.f;
   const float c2 = p.scale_log2;
   for (int it = wave; it < ntiles; it += NW) {
     if constexpr (NORM) {
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     }
   }
 
-  // ---- merge: every wave's state is brought to the largest maximum of the row (a wave without keys has m = kLowestMax, l = 0)
+  // ---- merge: every wave's state is brought to the largest maximum of the row (a wave without keys has l = 0)
   float* stat = reinterpret_cast<float*>(smem + S::STAT_OFF);   // [m | l | mu][wave][row]
   const float l_w = xhalf_sum(l_run), mu_w = JVP ? xhalf_sum(mu_run) : 0.f;
   if (g == 0) stat[wave * 32 + c32] = m_run;

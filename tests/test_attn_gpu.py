@@ -948,3 +948,19 @@ def test_softmax_scale_of_any_sign(scale, dtype, D, batch):
             # (the tangent's terms are scale * log of a probability's range larger than the result where they cancel)
             t = tol * max(1.0, abs(scale) * D ** 0.5) if name == "to" else tol
             assert ao.rel_l2(got[:2].double().cpu(), ref) <= t, (name, L, ao.rel_l2(got[:2].double().cpu(), ref))
+
+
+@pytest.mark.parametrize("L,D", [(128, 72), (100, 72), (128, 64), (128, 80), (129, 96)])
+def test_rows_whose_keys_are_all_masked(L, D):
+    """bf16 on a small grid: queries for which every key carries the lowest number (a padded row) weigh the keys by what is left of the scores
+    at that magnitude -- nothing: the plain average --, next to rows that see no mask."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(2, L, 2, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    q[..., -1] = 0
+    q[:, ::2, :, -1] = 1
+    k[..., -1] = torch.finfo(torch.bfloat16).min
+    assert "small" in _lib.plan("fwd", 2, 2, L, L, D)
+    got = flash_attn_func(*(t.to(DEV) for t in (q, k, v))).double().cpu()
+    ref = _softmax_attention(q.double(), k.double(), v.double(), D ** -0.5)
+    for rows in (slice(0, None, 2), slice(1, None, 2)):
+        assert ao.rel_l2(got[:, rows], ref[:, rows]) <= TOL[torch.bfloat16]
