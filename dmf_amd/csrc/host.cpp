@@ -198,13 +198,14 @@ struct KernelNode : Node {
     out.resize(n);
     return out;
   }
-  // False under create_graph=True and for batched gradients: there, what consists of torch operators stays differentiable and
-  // mapped, as autograd.Function's backward is.
+  // False under create_graph=True, for batched gradients and for gradients that carry a tangent (forward over reverse at a dual
+  // level): there, what consists of torch operators stays differentiable and mapped, as autograd.Function's backward is.
   static bool plain_call(const variable_list& grads) {
     if (c10::GradMode::is_enabled()) return false;
     for (const Tensor& g : grads)
-      if (g.defined() && g.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
-                                                                 c10::DispatchKey::Batched, c10::DispatchKey::Python})))
+      if (g.defined() && (g._fw_grad(0).defined() ||
+                          g.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                                                   c10::DispatchKey::Batched, c10::DispatchKey::Python}))))
         return false;
     return true;
   }

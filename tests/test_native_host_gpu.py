@@ -196,6 +196,21 @@ def test_linear_under_two_jvp_levels(autocast):
         assert float(exp.float().norm()) > 0 and float((got.float() - exp.float()).norm()) <= 2 ** -8 * float(exp.float().norm())
 
 
+def test_tangents_of_incoming_gradients():
+    """Forward over reverse: a gradient that carries a tangent at a dual level gives input gradients that carry theirs."""
+    torch.manual_seed(5)
+    x, w, b = torch.randn(6, 64, device=DEV, requires_grad=True), torch.randn(32, 64, device=DEV, requires_grad=True), torch.randn(32, device=DEV, requires_grad=True)
+    g, tg = torch.randn(6, 32, device=DEV), torch.randn(6, 32, device=DEV)
+    with fwAD.dual_level():
+        grads = torch.autograd.grad(block_ops.dual_linear(x, w, b), (x, w, b), fwAD.make_dual(g, tg))
+        for got, exp in zip(grads, (tg @ w, tg.t() @ x, tg.sum(0))):
+            tangent = fwAD.unpack_dual(got).tangent
+            assert tangent is not None and (tangent - exp).norm() <= 1e-5 * exp.norm()   # up to 64 terms in fp32
+        parts = block_ops.chunk_last(x, 2)
+        gx, = torch.autograd.grad(parts[1], x, fwAD.make_dual(g, tg))
+        assert torch.equal(fwAD.unpack_dual(gx).tangent, torch.cat([torch.zeros_like(tg), tg], -1))
+
+
 def test_watched_calls_take_the_general_route():
     class Watch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
