@@ -30,6 +30,7 @@
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <functional>
 
 #include "../../include/dmf_attn.h"
@@ -191,7 +192,8 @@ struct KernelNode : Node {
       primal.push_back(std::move(grads[i]));
     }
     if (!any) return variable_list(n);
-    c10::OptionalDeviceGuard device(s[0].device());
+    const auto first = std::find_if(primal.begin(), primal.end(), [](const Tensor& g) { return g.defined(); });
+    c10::OptionalDeviceGuard device(first->device());
     std::optional<Below> below;
     if (!torch_ops || plain_call(primal)) below.emplace();
     variable_list out = fn(*this, s, primal);
@@ -989,11 +991,13 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
   }
   std::shared_ptr<KernelNode> node;
   if (any_grad(x)) {
-    node = make_node("ChunkBackward", {x}, {parts[0]});
+    // (nothing is saved: a part that the node saves and that belongs to the node would keep both alive)
+    node = make_node("ChunkBackward", {x}, {});
     node->torch_ops = true;
-    node->fn = [n](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+    node->fn = [n, shape = parts[0].sizes().vec(), options = parts[0].options()](KernelNode&, const std::vector<Tensor>&,
+                                                                                const variable_list& g) -> variable_list {
       std::vector<Tensor> parts;
-      for (int64_t i = 0; i < n; ++i) parts.push_back(g[i].defined() ? g[i] : at::zeros_like(sv[0], at::MemoryFormat::Contiguous));
+      for (int64_t i = 0; i < n; ++i) parts.push_back(g[i].defined() ? g[i] : at::zeros(shape, options));
       return {at::cat(parts, -1)};
     };
   }

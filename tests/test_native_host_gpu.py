@@ -173,6 +173,25 @@ def test_linear_and_chunk_stay_twice_differentiable():
             assert (got[i] - exp).norm() <= 1e-5 * exp.norm()
 
 
+def test_graphs_that_never_run_backward_are_freed():
+    """A gradient-enabled call whose results are dropped without a backward pass leaves nothing behind: a node that holds its own output
+    would keep the graph above it."""
+    torch.manual_seed(6)
+    model = DMFT(input_size=16, hidden_size=256, depth=2, num_heads=4, dmf_depth=1, attn_func="hip", block_ops="hip").to(DEV).init_trunc_normal_()
+    x, c = torch.randn(2, 4, 16, 16, device=DEV), torch.randn(2, 1, 3 * 64, device=DEV, requires_grad=True)
+    t, y = torch.rand(2, device=DEV), torch.zeros(2, dtype=torch.long, device=DEV)
+    calls = (lambda: block_ops.chunk_last(c * 1.0, 3), lambda: model(x, t, t, y), lambda: block_ops.dual_linear(c * 1.0, torch.randn(64, 192, device=DEV)),
+             lambda: torch.func.jvp(lambda v: block_ops.chunk_last(v * 1.0, 3)[0], (c,), (c.detach(),)),
+             lambda: dmf_amd.flash_attn_qkvpacked_func((c * torch.ones(2, 40, 1, device=DEV)).view(2, 40, 3, 1, 64)))
+    for i, call in enumerate(calls):
+        call()
+        held = []
+        for _ in range(3):
+            call()
+            held.append(torch.cuda.memory_allocated())
+        assert held[0] == held[-1], (i, held)
+
+
 @pytest.mark.parametrize("autocast", [False, True])
 def test_linear_under_two_jvp_levels(autocast):
     """The second directional derivative of linear(x * x) and the mixed parts, against the same nesting of torch's own linear: bf16 operands
