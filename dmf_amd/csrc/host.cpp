@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 #include <torch/extension.h>
@@ -1001,6 +1002,14 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
       return {at::cat(parts, -1)};
     };
   }
+  // Views of x as those of torch's chunk: writing into one in place is refused where it has a gradient to keep right, and counts as a change
+  // of x elsewhere.
+  for (Tensor& t : parts) {
+    if (node) t = torch::autograd::as_view(x.var, t, /*is_bw_differentiable=*/true, /*is_fw_differentiable=*/false, nullptr, nullptr,
+                                           torch::autograd::CreationMeta::MULTI_OUTPUT_NODE);
+    else torch::autograd::impl::set_version_counter(t, torch::autograd::impl::version_counter(x.data));
+  }
+  for (Tensor& t : tparts) torch::autograd::impl::set_version_counter(t, torch::autograd::impl::version_counter(x.tan));
   py::list out;
   for (int64_t i = 0; i < n; ++i) out.append(finish(parts[i], tparts.empty() ? Tensor() : tparts[i], node, level));
   return out;

@@ -153,6 +153,22 @@ def test_in_place_changes_of_reshaped_operands_are_noticed(op):
         y.sum().backward()
 
 
+def test_chunks_are_views():
+    """In-place writes to a chunk: refused where the chunk has history, a change of the whole tensor elsewhere."""
+    x = torch.randn(2, 1, 192, device=DEV, requires_grad=True)
+    z = x * 1.0
+    part = block_ops.chunk_last(z, 3)[1]
+    assert part._is_view() and part._base is z
+    with pytest.raises(RuntimeError, match="view"):
+        part.mul_(2.0)
+    y = z.square()   # saves z
+    with torch.no_grad():
+        block_ops.chunk_last(z, 3)[0].zero_()
+    assert z._version == 1
+    with pytest.raises(RuntimeError, match="inplace"):
+        y.sum().backward()
+
+
 def test_linear_and_chunk_stay_twice_differentiable():
     torch.manual_seed(1)
     x = torch.randn(3, 5, 64, device=DEV, requires_grad=True)
