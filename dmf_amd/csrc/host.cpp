@@ -525,12 +525,20 @@ py::object attention_qknorm_packed(const Tensor& qkv, const Tensor& qg_, const T
       const QKV raw = slots(sv[0].view(gqkv.sizes())), grad = slots(gqkv);
       const Operand od(dout), oqh(sv[3]), okh(sv[4]), oo(o);
       const Strides st{&od, &oqh, &okh, &raw.v, &oo, &grad.q, &grad.k, &grad.v, &raw.q, &raw.k};
-      check(dmf_attn_bwd_qknorm(od.p, oqh.p, okh.p, raw.v.p, oo.p, static_cast<const float*>(ptr(sv[6])), raw.q.p, raw.k.p,
+      const int rc = dmf_attn_bwd_qknorm(od.p, oqh.p, okh.p, raw.v.p, oo.p, static_cast<const float*>(ptr(sv[6])), raw.q.p, raw.k.p,
                                 static_cast<const float*>(ptr(sv[1])), static_cast<const float*>(ptr(sv[2])), (float)eps,
                                 const_cast<void*>(grad.q.p), const_cast<void*>(grad.k.p), const_cast<void*>(grad.v.p),
                                 static_cast<float*>(mptr(dgq)), static_cast<float*>(mptr(dgk)), static_cast<float*>(mptr(delta)),
-                                static_cast<float*>(mptr(ws)), st.data(), s.B, s.H, s.Lq, s.Lkv, s.D, s.scale, s.code, stream_of(o)),
-            "dmf_attn_bwd_qknorm");
+                                static_cast<float*>(mptr(ws)), st.data(), s.B, s.H, s.Lq, s.Lkv, s.D, s.scale, s.code, stream_of(o));
+      if (rc == DMF_ATTN_ENOKERNEL) {   // rows of the output gradient too far apart: attention and norms one after the other
+        py::gil_scoped_acquire gil;
+        const Tensor dqh = dense_like(sv[3]), dkh = dense_like(sv[4]), five = sv[0].view(gqkv.sizes());
+        g_lib.attr("bwd")(dout, sv[3], sv[4], five.select(2, 2), o, sv[6], (double)s.scale, py::make_tuple(dqh, dkh, gqkv.select(2, 2)));
+        const py::tuple nq = g_lib.attr("rmsnorm_bwd")(dqh, five.select(2, 0), sv[1], eps, gqkv.select(2, 0));
+        const py::tuple nk = g_lib.attr("rmsnorm_bwd")(dkh, five.select(2, 1), sv[2], eps, gqkv.select(2, 1));
+        return {gqkv.view(shape), nq[1].cast<Tensor>().to(tq), nk[1].cast<Tensor>().to(tk)};
+      }
+      check(rc, "dmf_attn_bwd_qknorm");
       return {gqkv.view(shape), dgq.to(tq), dgk.to(tk)};
     };
   }

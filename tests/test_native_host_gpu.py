@@ -118,6 +118,23 @@ def test_what_the_native_path_hands_back():
             y.sum().backward()
 
 
+def test_qknorm_backward_of_far_apart_gradient_rows():
+    """Rows of the output gradient 2 GiB / (L + 256) or more apart (time-major, a very large batch): no kernel has the norms' backward in its
+    epilogue there, so attention and norms run one after the other, as on the general route, whose bits these are."""
+    fn, (qkv, qg, kg) = _attn_case("qknorm", torch.bfloat16)
+    B, L, _, H, D = qkv.shape
+    row = (1 << 31) // (2 * (L + 256)) // 8 * 8 + 8
+    gy = torch.empty(L * row, device=DEV, dtype=torch.bfloat16).as_strided((B, L, H, D), (H * D, row, D, 1))
+    gy.copy_(torch.linspace(-1, 1, B * L * H * D, device=DEV).view(B, L, H, D))
+
+    def grads():
+        leaves = [t.detach().clone().requires_grad_() for t in (qkv, qg, kg)]
+        return torch.autograd.grad(fn(*leaves), leaves, gy)
+
+    for got, exp in zip(grads(), _general(grads)):
+        assert got.dtype == exp.dtype and torch.equal(got, exp)
+
+
 def test_gradients_at_tangent_outputs():
     """Attention drops them, the block operators refuse them -- attached to a loss together with the primal output or alone."""
     q, t = torch.randn(2, 16, 2, 64, device=DEV, requires_grad=True), torch.randn(2, 16, 2, 64, device=DEV)
