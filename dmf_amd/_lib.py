@@ -666,7 +666,8 @@ def linear_fwd(x, tx, w, bias, gelu: bool = False):
     ops = [_raw(t) for t in (x, tx, w, bias)]
     x, tx, w, bias = ops
     present = [t for t in ops if t is not None]
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or len(_interpreters()) > 1
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0
+            or len(_interpreters()) > 1
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous()
                    for t in present) or any(t.data_ptr() % 16 for t in present)):
         return None

@@ -263,6 +263,16 @@ def test_tangents_of_incoming_gradients():
         assert torch.equal(fwAD.unpack_dual(gx).tangent, torch.cat([torch.zeros_like(tg), tg], -1))
 
 
+def test_traced_linear_gelu_computes():
+    """torch.jit.trace records operators, not the buffers that a launch of the package's own filled while it was recorded.  Both sides round
+    fp32 values once to bf16 (the library's after rounding the pre-activation as well)."""
+    x, x2, w, b = (torch.randn(*s, device=DEV).bfloat16() for s in ((64, 64), (64, 64), (128, 64), (128,)))
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda x: block_ops.linear_gelu_tanh(x, w, b), (x,), check_trace=False)
+        got, exp = traced(x2).float(), block_ops.linear_gelu_tanh(x2, w, b).float()
+    assert (got - exp).norm() <= 2 ** -7 * exp.norm()
+
+
 def test_watched_calls_take_the_general_route():
     class Watch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
