@@ -178,13 +178,13 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, Sc[i]);
     mx = xhalf_max(mx);
     if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
-      const float m_new = fmaxf(m_run, mx), alpha = fast_exp2(m_run - m_new);
+      const float m_new = fmaxf(m_run, mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
       if constexpr (JVP) {
         mu_run *= alpha;
-        dO.scale(alpha);
+        dO.scale(gs.decay(alpha, drop));
         if constexpr (F16) dOv.scale(alpha);
       }
     }

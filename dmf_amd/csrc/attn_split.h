@@ -353,10 +353,24 @@ __device__ __forceinline__ void contract_rows(const char* tile, int lane, OutAcc
 
 // Power of two per output row that keeps an unbounded W operand inside the f16 range (fp16 operands only): W is multiplied by
 // `mul` before it is split and the accumulator it feeds carries the same factor until the epilogue divides it out.  mul = 2^-e
-// for the largest magnitude 2^e seen when it was last set; raised when a magnitude exceeds 32 times that.
+// for the largest magnitude 2^e seen when it was last set; raised when a magnitude exceeds 32 times that, and lowered together
+// with the accumulator where a larger maximum scales what was summed so far away.
 template <typename T>
 struct RowScale {
   float mul = 1.f, limit = 0.f;
+  // The accumulator's factor where its row is to be scaled by alpha = 2^-drop, drop >= 0.  The reference magnitude shrinks with the row:
+  // left where an early tile put it, the f16 steps of later, smaller W would be as coarse as that tile's (dO behind a step of the scores
+  // by 30 nats, tangent scores 10^5 times larger in front of it: 2.6e-2 off; fp16 rounding 5e-4).
+  __device__ __forceinline__ float decay(float alpha, float drop) {
+    if constexpr (!SplitType<T>::F16) return alpha;
+    const uint32_t k = static_cast<uint32_t>(fminf(drop, 120.f));
+    const float m2 = mul * __uint_as_float((127u + k) << 23);
+    const bool ok = k < 120u && m2 < 0x1p120f;   // beyond: back to the start, with what is left of the row in its own units
+    const float f = alpha * (ok ? __uint_as_float((127u + k) << 23) : 1.f / mul);
+    limit = ok ? limit * __uint_as_float((127u - k) << 23) : 0.f;
+    mul = ok ? m2 : 1.f;
+    return f;
+  }
   template <typename A>
   __device__ __forceinline__ void update(const f32x16& w, A& acc) {
     if constexpr (SplitType<T>::F16) {
@@ -541,13 +555,13 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, S[i]);
     mx = xhalf_max(mx) * c2;
     if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
-      const float m_new = fmaxf(m_run, mx), alpha = fast_exp2(m_run - m_new);
+      const float m_new = fmaxf(m_run, mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
       if constexpr (JVP) {
         mu_run *= alpha;
-        dO.scale(alpha);
+        dO.scale(gs.decay(alpha, drop));
         if constexpr (F16) dOv.scale(alpha);
       }
     }

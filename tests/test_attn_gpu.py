@@ -964,3 +964,29 @@ def test_rows_whose_keys_are_all_masked(L, D):
     ref = _softmax_attention(q.double(), k.double(), v.double(), D ** -0.5)
     for rows in (slice(0, None, 2), slice(1, None, 2)):
         assert ao.rel_l2(got[:, rows], ref[:, rows]) <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("B,H,L,D,kind", [(2, 2, 100, 72, "small"), (64, 4, 130, 64, "kernel"), (64, 4, 256, 72, "wide")])
+@pytest.mark.parametrize("step", [8, 20, 30, 90, 400])
+def test_half_tangent_behind_a_step_of_the_scores(step, B, H, L, D, kind):
+    """fp16, the second half of the keys scoring `step` nats above the first, whose tangent scores are some 10^5 times larger: what the first
+    half sums up fades with the maximum, and the second half's small products keep their digits (fp64 formula of the same operands)."""
+    assert kind in _lib.plan("fwd_jvp", B, H, L, L, D, torch.float16)
+    g = torch.Generator(device=DEV).manual_seed(L + step)
+    q, k, v, tq, tk, tv = (0.5 * torch.randn(B, L, H, D, generator=g, device=DEV) for _ in range(6))
+    first = torch.arange(L, device=DEV) < L // 2
+    scale = D ** -0.5
+    q[..., 0], q[..., 1] = 8.0, 0.0
+    k[..., 0] = torch.where(first, 0.0, step / (8.0 * scale))[None, :, None]
+    tq[..., 0], tq[..., 1] = 0.0, 1e3
+    k[..., 1] = torch.where(first, torch.linspace(1e3, 2e3, L, device=DEV), torch.zeros((), device=DEV))[None, :, None]
+    tk[..., :2] = 0
+    x = [t.half() for t in (q, k, v, tq, tk, tv)]
+    o, to, _ = _lib.fwd_jvp_half(*x, scale)
+    x64 = [t[:2].double().cpu() for t in x]
+    o_ref, to_ref = torch.func.jvp(lambda q, k, v: _softmax_attention(q, k, v, scale), tuple(x64[:3]), tuple(x64[3:]))
+    # Half-precision results: 2^-12 of an element on average.  The scores' fp32 sums carry 2^-24 of their magnitude into the probabilities, and
+    # the first half's weight, exp(-step), times its tangent scores is of order one and more where the step is small.
+    tol = 1e-3
+    assert ao.rel_l2(o[:2].double().cpu(), o_ref) <= tol
+    assert ao.rel_l2(to[:2].double().cpu(), to_ref) <= tol, ao.rel_l2(to[:2].double().cpu(), to_ref)
