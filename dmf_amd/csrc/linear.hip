@@ -5,6 +5,7 @@
 // The library ran the two products of a layer one after the other (two partly empty last rounds), in tiles that fit these widths
 // badly, and spent 18 us of host time on each.  Here both are one grid; 192 columns divide every layer width of the models, so the
 // 128 x 192 tile fills whole rounds.
+#include <algorithm>
 #include <type_traits>
 #include "attn_common.h"
 #include "attn_kernels.h"
@@ -450,7 +451,9 @@ static int wgrad_splits(int64_t M, int64_t N, int64_t K) {
 }
 
 static bool wgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
-  return M >= 1 && N >= 8 && N % 8 == 0 && K >= 8 && K % 8 == 0 && M * K < (int64_t)1 << 30 && N * K < (int64_t)1 << 30 && M * N < (int64_t)1 << 30;
+  if (M < 1 || N < 8 || N % 8 || K < 8 || K % 8 || M * K >= (int64_t)1 << 30 || N * K >= (int64_t)1 << 30 || M * N >= (int64_t)1 << 30) return false;
+  // rows up to the end of the last step are addressed too, in 32 bits: wrapped around, one past the last would be read, not be zero
+  return (M + 63) / 64 * 64 * std::max(N, K) < (int64_t)1 << 31;
 }
 
 }  // namespace dmf

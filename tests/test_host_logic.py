@@ -348,3 +348,15 @@ def test_stale_gradient_accumulator_probe():
     assert stale_grad_accumulator(p)          # the graph's nodes live as long as `loss` does
     del loss
     assert not stale_grad_accumulator(p)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1 << 26, 8), (1, 1 << 25, 8), (31, 8, 1 << 25), (3, 8, 1 << 25)])
+def test_weight_gradient_keeps_padded_rows_within_32_bits(M, N, K):
+    """The weight-gradient kernel reads whole steps of 64 rows and counts on zeros past the last: shapes whose 64th row lies 4 GiB or more
+    from the first (where the 32-bit offset would come back to row 0) are refused, those just below are not."""
+    lib = _lib.load()
+    assert lib.dmf_linear_wgrad_workspace_floats(M, N, K) == -1 and lib.dmf_linear_wgrad_plan(M, N, K) == 0
+    assert lib.dmf_linear_wgrad(16, 16, 16, None, None, M, N, K, None) == -3
+    narrower = (M, N - 8, K) if (1 << 25) == N else None
+    if narrower:
+        assert lib.dmf_linear_wgrad_workspace_floats(*narrower) >= 0
