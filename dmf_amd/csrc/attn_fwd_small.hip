@@ -25,8 +25,7 @@ struct SmallCfg {
   using C = SplitCfg<T, D, 1>;
   static constexpr int VTILES = JVP ? 2 : 1;
   static constexpr int WAVE_BYTES = VTILES * C::TILE;
-  static constexpr int MERGE_OFF = 0;                                              // the fp32 rows of the four waves reuse the tiles
-  static constexpr int ROWS_BYTES = 32 * kSmallWaves * Cfg<float, D>::OROWV * 16;
+  static constexpr int ROWS_BYTES = 32 * kSmallWaves * Cfg<float, D>::OROWV * 16;   // the fp32 rows of the four waves, over the tiles
   static constexpr int TILES_BYTES = kSmallWaves * WAVE_BYTES;
   static constexpr int STAT_OFF = ROWS_BYTES > TILES_BYTES ? ROWS_BYTES : TILES_BYTES;   // m, l, mu of every wave and row
   static constexpr int LDS_BYTES = STAT_OFF + 3 * kSmallWaves * 32 * 4;
@@ -178,7 +177,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, Sc[i]);
     mx = xhalf_max(mx);
     if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
-      const float m_new = fmaxf(m_run, mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
+      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
@@ -189,9 +188,10 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
       }
     }
     f32x16 E, G;
+    const float m_off = m_run - kFwdBias<T>;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      E[i] = fast_exp2(Sc[i] - m_run);
+      E[i] = fast_exp2(Sc[i] - m_off);
       l_run += E[i];
       if constexpr (JVP) {
         G[i] = E[i] * (dS[i] * p.scale);
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     const float l = row_stats(tid);
     const int row = q0 + tid;
     if (row < p.Lq) {
-      if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + row] = (m + log2f(l)) * kLn2;
+      if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + row] = (m - kFwdBias<T> + log2f(l)) * kLn2;
       if constexpr (JVP)
         if (p.dlse != nullptr) p.dlse[(int64_t)bh * p.Lq + row] = mu_n;
     }

@@ -8,9 +8,12 @@
 // fp32 multiplication.  Six MFMAs of 32x32x16 take 192 cycles where eight of 32x32x2 take 512.
 //
 // fp16 operands are exact in one f16 plane, so the score-like products are single f16 MFMAs; the probability-like operand
-// W (P, P*dS, dS: fp32 values) is split into two f16 planes (21 significant bits) so that nothing is rounded to 11 bits
-// before the final store.  P lies in [0, 2^6]; operands that carry a tangent or gradient factor have no such bound and are
-// kept in range by a per-row power of two (RowScale), raised lazily like the running maximum.
+// W (P, P*dS, dS: fp32 values) is split into two f16 planes (23 significant bits) so that nothing is rounded to
+// 11 bits before the final store.  f16 has no digits below 2^-24, so P is formed times a power of two that puts its largest value near the
+// top of the range (kFwdBias, kBwdBias: part of the exponent, hence free): formed as it is, a weight of e^-10 kept 10 bits and one of e^-14
+// four, which the rows of a key with nearly all of the weight and a zero value are made of (N1024: results 6.8e-4 and 3.6e-2 off where
+// fp16 rounds to 2e-4).  Operands that carry a tangent or gradient factor have no bound and are kept in range by a power of two per row
+// (RowScale), raised lazily like the running maximum.
 //
 // Layouts are those of attn_common.h (transposed scores, per-lane softmax state, accumulator tile = next B operand).
 // A work-group of NW waves owns 32 NW rows of one (batch, head); tiles of 32 streamed rows travel HBM -> registers -> planes
@@ -22,12 +25,16 @@
 namespace dmf {
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) __fp16 fp16x2;
 
 // NI planes of a loaded operand, NWT of a probability-like one.
 template <typename T> struct SplitType;
 template <> struct SplitType<float> { static constexpr int NI = 3, NWT = 3; static constexpr bool F16 = false; };
 template <> struct SplitType<_Float16> { static constexpr int NI = 1, NWT = 2; static constexpr bool F16 = true; };
+
+// log2 of the factor on P in the f16 kernels: P reaches 2^6 in the forward (kSplitLazyLog2), 1 in the backward, the range 2^16.
+template <typename T> constexpr float kFwdBias = SplitType<T>::F16 ? 9.f : 0.f;
+template <typename T> constexpr float kBwdBias = SplitType<T>::F16 ? 14.f : 0.f;
+constexpr uint32_t kRowScaleBias = 9;   // and of RowScale's largest value before it is raised: 2^5 times that
 
 template <>
 __device__ __forceinline__ void store4<_Float16>(_Float16* dst, float a, float b, float c, float d) {
@@ -79,6 +86,13 @@ __device__ __forceinline__ float sub_half(float x, uint32_t w) {
   return r;
 }
 
+// two fp32 values to f16, rounded to nearest
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), f16x2));
+}
+
 // Eight fp32 values as NP planes of eight 16-bit ones.  ANY (operands as the caller gave them, in bf16 planes): all but the last
 // plane are held within the finite range, so that a value above the largest bf16 number does not round to infinity and an
 // infinity or NaN ends up in the last plane alone -- it then meets only the first plane of the other operand, whose sign is the
@@ -92,8 +106,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       if constexpr (SplitType<T>::F16) {
-        const fp16x2 h = __builtin_amdgcn_cvt_pkrtz(a, b);
-        pl[k][i] = __builtin_bit_cast(uint32_t, h);
+        pl[k][i] = pack_f16x2(a, b);
         if (k + 1 < NP) {
           a = sub_half<0>(a, pl[k][i]);
           b = sub_half<1>(b, pl[k][i]);
@@ -352,8 +365,9 @@ __device__ __forceinline__ void contract_rows(const char* tile, int lane, OutAcc
 }
 
 // Power of two per output row that keeps an unbounded W operand inside the f16 range (fp16 operands only): W is multiplied by
-// `mul` before it is split and the accumulator it feeds carries the same factor until the epilogue divides it out.  mul = 2^-e
-// for the largest magnitude 2^e seen when it was last set; raised when a magnitude exceeds 32 times that, and lowered together
+// `mul` before it is split and the accumulator it feeds carries the same factor until the epilogue divides it out.  mul = 2^(9-e)
+// for the largest magnitude 2^e seen when it was last set (2^14 is the most that W then reaches, and its small elements lie as
+// far above the end of the f16 range as they can); raised when a magnitude exceeds 32 times that, and lowered together
 // with the accumulator where a larger maximum scales what was summed so far away.
 template <typename T>
 struct RowScale {
@@ -381,7 +395,8 @@ struct RowScale {
       if (__builtin_amdgcn_ballot_w64(mx > limit) != 0) {
         const uint32_t e = __float_as_uint(mx) & 0x7f800000u;
         const bool up = mx > limit && e > 0 && e < 0x7f000000u;
-        const float m2 = up ? __uint_as_float(0x7f000000u - e) : mul;
+        const uint32_t scaled = 0x7f000000u + (kRowScaleBias << 23) - e;
+        const float m2 = up ? __uint_as_float(scaled < 0x7e800000u ? scaled : 0x7e800000u) : mul;
         limit = up ? 32.f * __uint_as_float(e) : limit;
         acc.scale(m2 / mul);
         mul = m2;
@@ -555,7 +570,8 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, S[i]);
     mx = xhalf_max(mx) * c2;
     if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
-      const float m_new = fmaxf(m_run, mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
+      // (a whole number in the f16 kernels: nothing is rounded when kFwdBias is taken off)
+      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
@@ -566,9 +582,10 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
       }
     }
     f32x16 E, G;
+    const float m_off = m_run - kFwdBias<T>;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      E[i] = fast_exp2(fmaf(S[i], c2, -m_run));
+      E[i] = fast_exp2(fmaf(S[i], c2, -m_off));
       l_run += E[i];
       if constexpr (JVP) {
         G[i] = E[i] * (dS[i] * p.scale);
@@ -607,7 +624,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   const float l_tot = xhalf_sum(l_run), inv_l = 1.0f / l_tot;
   const float mu_n = JVP ? xhalf_sum(mu_run) * inv_l : 0.f;
   if (g == 0 && qrow < p.Lq) {
-    if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + qrow] = (m_run + log2f(l_tot)) * kLn2;
+    if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + qrow] = (m_run - kFwdBias<T> + log2f(l_tot)) * kLn2;
     if constexpr (JVP)
       if (p.dlse != nullptr) p.dlse[(int64_t)bh * p.Lq + qrow] = mu_n;
   }
@@ -756,7 +773,7 @@ __device__ __forceinline__ void split_bwd_dkv_body(const BwdParams& p) {
     if (tid < 64) {
       const int r = it * 32 + (tid & 31);
       const bool ok = r < p.Lq;
-      if (tid < 32) st_pre = ok ? p.lse[(int64_t)bh * p.Lq + r] * kLog2e : INFINITY;
+      if (tid < 32) st_pre = ok ? fmaf(p.lse[(int64_t)bh * p.Lq + r], kLog2e, -kBwdBias<T>) : INFINITY;   // P, and dS with it, times 2^kBwdBias
       else st_pre = ok ? p.delta[(int64_t)bh * p.Lq + r] : 0.f;
     }
   };
@@ -812,8 +829,9 @@ __device__ __forceinline__ void split_bwd_dkv_body(const BwdParams& p) {
     if constexpr (ST::N == 1) __syncthreads();
     if (it + 1 < ntiles) commit(it + 1);
   }
-  store_out<T, D, NW>(smem, static_cast<T*>(p.dk) + base(6), p.st[6][1], k0, p.Lkv, tid, dK, p.scale * gs.inverse());
-  store_out<T, D, NW>(smem, static_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid, dV, 1.f);
+  constexpr float kUnbias = SplitType<T>::F16 ? 1.f / 16384.f : 1.f;   // 2^-kBwdBias
+  store_out<T, D, NW>(smem, static_cast<T*>(p.dk) + base(6), p.st[6][1], k0, p.Lkv, tid, dK, p.scale * kUnbias * gs.inverse());
+  store_out<T, D, NW>(smem, static_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid, dV, kUnbias);
 }
 
 }  // namespace dmf

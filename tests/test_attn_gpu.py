@@ -8,6 +8,8 @@ Tolerances (relative L2 over the whole tensor), from the contract of this build:
 for O, dO and for dQ, dK, dV.  In bf16 mode the oracle sees the bf16-rounded
 inputs (the values the kernel sees), computed in fp32.
 """
+import math
+
 import pytest
 import torch
 
@@ -990,3 +992,38 @@ def test_half_tangent_behind_a_step_of_the_scores(step, B, H, L, D, kind):
     tol = 1e-3
     assert ao.rel_l2(o[:2].double().cpu(), o_ref) <= tol
     assert ao.rel_l2(to[:2].double().cpu(), to_ref) <= tol, ao.rel_l2(to[:2].double().cpu(), to_ref)
+
+
+@pytest.mark.parametrize("B,H,L,D,kind", [(1, 2, 256, 64, "small"), (1, 2, 300, 72, "small"), (12, 16, 260, 64, "kernel"), (16, 16, 512, 72, "wide"),
+                                          (3, 16, 384, 128, "kernel")])
+@pytest.mark.parametrize("nats", [0, 10, 14])
+def test_half_rows_made_of_small_weights(nats, B, H, L, D, kind):
+    """fp16, the first key scoring `nats` above all others with a value of zero, so that the result is what the small weights contribute: these
+    keep their digits in the forward, its tangent and the gradients (fp64 formula of the same operands)."""
+    assert kind in _lib.plan("fwd", B, H, L, L, D, torch.float16)
+    g = torch.Generator(device=DEV).manual_seed(L + nats)
+    rnd = lambda: torch.randn(B, L, H, D, generator=g, device=DEV)
+    q, k, v, tq, tk, tv, do = rnd(), 0.1 * rnd(), rnd() + 1, rnd(), rnd(), rnd(), rnd() + 1
+    q[..., 0], k[..., 0], tq[..., 0] = D ** 0.5, 0.0, 0.0
+    if nats:
+        k[:, 0], v[:, 0], tv[:, 0] = 0.0, 0.0, 0.0
+        k[:, 0, :, 0] = nats
+    x = [t.half() for t in (q, k, v, tq, tk, tv, do)]
+    o, to, lse = _lib.fwd_jvp_half(*x[:6], D ** -0.5)
+    o2, _ = _lib.fwd_half(*x[:3], D ** -0.5)
+    grads = _lib.bwd_half(x[6], *x[:3], o, lse, D ** -0.5)
+    x64 = [t[:1].double().cpu() for t in x]
+    attn = lambda q, k, v: _softmax_attention(q, k, v, D ** -0.5)
+    o_ref, to_ref = torch.func.jvp(attn, tuple(x64[:3]), tuple(x64[3:6]))
+    # Results in half precision: at most 2^-11, 2^-12 to 2^-11.5 of an array.  Weights: half of 2^-24 after the factor of 2^9, against e^-nats.
+    # Gradients of q and k besides: differences of two terms with the rounded result in one of them, 2^-12 of sums that partly cancel.
+    tol = 3e-4 + 2.0 ** -34 * math.exp(nats)
+    got = {"o": (o, o_ref), "o primal": (o2, o_ref), "to": (to, to_ref)}
+    ref = torch.autograd.grad(attn(*(t.requires_grad_() for t in x64[:3])), x64[:3], x64[6])
+    got |= {n: (a, b) for n, a, b in zip(("dq", "dk", "dv"), grads, ref)}
+    s = torch.einsum("blhd,bmhd->bhlm", x64[0].detach(), x64[1].detach()) * D ** -0.5
+    assert (lse[:1].double().cpu() - s.logsumexp(-1)).abs().max() <= 1e-5 * (1 + nats)
+    for name, (a, b) in got.items():
+        err = ao.rel_l2(a[:1].double().cpu(), b.detach())
+        print(f"{name} {err:.2e}", flush=True)
+        assert err <= tol * (2 if name in ("dq", "dk") else 1), (name, err)
