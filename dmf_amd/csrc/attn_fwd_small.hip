@@ -199,7 +199,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
       }
     }
     WOperand<T> we;
-    we.form(E);
+    we.template form<true>(E);
     if constexpr (JVP) {
       gs.update(G, dO);
       if constexpr (F16) G *= gs.mul;

@@ -8,7 +8,7 @@
 // fp32 multiplication.  Six MFMAs of 32x32x16 take 192 cycles where eight of 32x32x2 take 512.
 //
 // fp16 operands are exact in one f16 plane, so the score-like products are single f16 MFMAs; the probability-like operand
-// W (P, P*dS, dS: fp32 values) is split into two f16 planes (23 significant bits) so that nothing is rounded to
+// W (P, P*dS, dS: fp32 values) is split into two f16 planes (21 significant bits of P, 23 of the others) so that nothing is rounded to
 // 11 bits before the final store.  f16 has no digits below 2^-24, so P is formed times a power of two that puts its largest value near the
 // top of the range (kFwdBias, kBwdBias: part of the exponent, hence free): formed as it is, a weight of e^-10 kept 10 bits and one of e^-14
 // four, which the rows of a key with nearly all of the weight and a zero value are made of (N1024: results 6.8e-4 and 3.6e-2 off where
@@ -25,6 +25,7 @@
 namespace dmf {
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
 
 // NI planes of a loaded operand, NWT of a probability-like one.
 template <typename T> struct SplitType;
@@ -96,8 +97,9 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
 // Eight fp32 values as NP planes of eight 16-bit ones.  ANY (operands as the caller gave them, in bf16 planes): all but the last
 // plane are held within the finite range, so that a value above the largest bf16 number does not round to infinity and an
 // infinity or NaN ends up in the last plane alone -- it then meets only the first plane of the other operand, whose sign is the
-// value's.
-template <typename T, bool ANY = false, int NP>
+// value's.  WEIGHT (probabilities, in f16 planes): the first plane is one step below the truncated value, so that the second is
+// positive wherever the value is, and an infinity among the elements it weighs stays one (next to an exact first plane it met a zero).
+template <typename T, bool ANY = false, bool WEIGHT = false, int NP>
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
   constexpr float kMax = 3.38953139e38f;   // the largest bf16 number
 #pragma unroll
@@ -106,7 +108,14 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       if constexpr (SplitType<T>::F16) {
-        pl[k][i] = pack_f16x2(a, b);
+        if constexpr (WEIGHT && NP > 1) {
+          if (k + 1 < NP)
+            pl[k][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, __builtin_amdgcn_cvt_pkrtz(a, b)), u16x2{1, 1}));
+          else
+            pl[k][i] = pack_f16x2(a, b);
+        } else {
+          pl[k][i] = pack_f16x2(a, b);
+        }
         if (k + 1 < NP) {
           a = sub_half<0>(a, pl[k][i]);
           b = sub_half<1>(b, pl[k][i]);
@@ -295,13 +304,14 @@ struct OutAcc {
 template <typename T>
 struct WOperand {
   u32x4 s[2][SplitType<T>::NWT];
+  template <bool WEIGHT = false>
   __device__ __forceinline__ void form(const f32x16& e) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       float x[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] = e[8 * st + i];
-      split8<T>(x, s[st]);
+      split8<T, false, WEIGHT>(x, s[st]);
     }
   }
   __device__ __forceinline__ void tail(u32x4 (&h0)[SplitType<T>::NWT], u32x4 (&h1)[SplitType<T>::NWT]) const {
@@ -593,7 +603,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
       }
     }
     WOperand<T> we;
-    we.form(E);
+    we.template form<true>(E);
     if constexpr (Plan::WIDE) {
       __syncthreads();   // V is in LDS; every wave is done with K
       if (it + 1 < ntiles) {
@@ -819,7 +829,7 @@ __device__ __forceinline__ void split_bwd_dkv_body(const BwdParams& p) {
       }
     }
     WOperand<T> wp;
-    wp.form(Pm);
+    wp.template form<true>(Pm);
     contract_rows<T, D, NW>(dOt, lane, dV, wp);
     gs.update(dS, dK);
     if constexpr (SplitType<T>::F16) dS *= gs.mul;

@@ -1027,3 +1027,24 @@ def test_half_rows_made_of_small_weights(nats, B, H, L, D, kind):
         err = ao.rel_l2(a[:1].double().cpu(), b.detach())
         print(f"{name} {err:.2e}", flush=True)
         assert err <= tol * (2 if name in ("dq", "dk") else 1), (name, err)
+
+
+@pytest.mark.parametrize("B,H,L,D", [(1, 2, 64, 64), (1, 2, 130, 72), (12, 16, 260, 64), (16, 16, 512, 72), (2, 4, 100, 128)])
+@pytest.mark.parametrize("spread", [0.0, 1.0])
+def test_half_infinite_values_stay_infinite(spread, B, H, L, D):
+    """fp16: an infinite value element makes that element of every row infinite, whatever the weight (with equal scores it is a power of two),
+    and leaves the others alone; an infinite element of the output gradient likewise reaches the value gradients."""
+    g = torch.Generator(device=DEV).manual_seed(L)
+    q, k, v = (torch.randn(B, L, H, D, generator=g, device=DEV).half() for _ in range(3))
+    q *= spread
+    v[:, L // 2, :, 3] = math.inf
+    v[:, L // 3, :, 5] = -math.inf
+    o, lse = _lib.fwd_half(q, k, v, D ** -0.5)
+    assert (o[..., 3] == math.inf).all() and (o[..., 5] == -math.inf).all()
+    rest = [i for i in range(D) if i not in (3, 5)]
+    assert o[..., rest].isfinite().all()
+    v[:, L // 2, :, 3] = v[:, L // 3, :, 5] = 0
+    do = torch.randn(B, L, H, D, generator=g, device=DEV).half()
+    do[:, L // 2, :, 3] = math.inf
+    _, _, dv = _lib.bwd_half(do, q, k, v, torch.zeros_like(o), lse, D ** -0.5)
+    assert (dv[..., 3] == math.inf).all() and dv[..., rest].isfinite().all()
