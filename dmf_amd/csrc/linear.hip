@@ -199,11 +199,18 @@ constexpr LinTile kLinTiles[4] = {
     {128, 192, 2, {90, 140, 0}, {350, 450, 0}}, {128, 128, 2, {77, 95, 0}, {120, 400, 0}},
     {128, 64, 3, {61, 63, 93}, {60, 200, 250}}, {64, 64, 2, {20, 36, 0}, {320, 320, 0}}};
 
-static int linear_tile(int64_t M, int N, int K, bool jvp) {
+// A gelu pair holds an element of x and its tangent in one wave, BM / 2 rows of each: it has as many work-groups as a single product of twice
+// the rows, and takes the tiles with two row tiles per wave.
+static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
   const int64_t cus = compute_units(), steps = K / kLinK;
+  const bool both = jvp && gelu;
+  if (both) {
+    M *= 2;
+    jvp = false;
+  }
   int best = 0;
   int64_t cost_best = INT64_MAX;
-  for (int t = 0; t < 4; ++t) {
+  for (int t = 0; t < (both ? 3 : 4); ++t) {
     const LinTile& c = kLinTiles[t];
     const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * (jvp ? 2 : 1), slots = cus * c.per_cu, rest = wgs % slots;
     auto full = [&](int64_t occ) { return c.a[occ] * steps + c.b[occ]; };
@@ -226,8 +233,10 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
     case 0: return launch_linear<128, 192, 2, MODE>(p, jvp, stream);
     case 1: return launch_linear<128, 128, 2, MODE>(p, jvp, stream);
     case 2: return launch_linear<128, 64, 2, MODE>(p, jvp, stream);
-    default: return launch_linear<64, 64, 4, MODE>(p, jvp, stream);
+    default: break;
   }
+  if constexpr (MODE == kLinGeluJvp) return DMF_ATTN_ESHAPE;   // (linear_tile does not answer this)
+  else return launch_linear<64, 64, 4, MODE>(p, jvp, stream);
 }
 
 }  // namespace dmf
@@ -264,8 +273,8 @@ extern "C" int dmf_linear_fwd(const void* x, const void* tx, const void* w, cons
   p.M = M; p.N = N; p.K = K;
   auto stm = static_cast<hipStream_t>(stream);
   const bool jvp = tx != nullptr;
-  if (jvp && gelu) return dmf::launch_linear<128, 192, 2, dmf::kLinGeluJvp>(p, true, stm);
-  const int tile = dmf::linear_tile(M, N, K, jvp);
+  const int tile = dmf::linear_tile(M, N, K, jvp, gelu != 0);
+  if (jvp && gelu) return dmf::launch_linear_tile<dmf::kLinGeluJvp>(tile, p, true, stm);
   return gelu ? dmf::launch_linear_tile<dmf::kLinGelu>(tile, p, false, stm) : dmf::launch_linear_tile<dmf::kLinPlain>(tile, p, jvp, stm);
 }
 
