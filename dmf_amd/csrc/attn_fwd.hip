@@ -211,11 +211,10 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<T, D, JVP>())) void attn_f
   if constexpr (std::is_same<T, __bf16>::value) generic_fwd_body<T, D, JVP>(p);
   else split_fwd_body<T, D, JVP, 4>(p);
 }
-// The 8-wave form (SplitFwdPlan) exists where it was measured to win: 128 registers (two work-groups per CU) without tangents.
-template <typename T, int D, bool JVP>
-constexpr bool has_wide_split() {
-  return std::is_same<T, _Float16>::value ? (JVP ? D == 72 || D == 80 : D == 72) : std::is_same<T, float>::value && JVP && D == 64;
-}
+// The 8-wave form (SplitFwdPlan) exists where it fits and wins: fp16 at head dims 72 and 80 (64 gains nothing, whether or not with
+// tangents: B16 H16 N512 37.9 -> 37.8 us, 83.8 -> 83.0, B32 N256 22.9 -> 22.6, 51.7 -> 53.0; 96 and 128 spill 21 and 65 of the 128
+// registers that two work-groups per CU leave without tangents), fp32 with tangents up to head dim 64 (72 and more do not fit the LDS).
+constexpr bool has_wide_split(bool f16, int D, bool jvp) { return f16 ? D == 72 || D == 80 : jvp && D <= 64; }
 template <typename T, int D, bool JVP>
 __global__ __launch_bounds__(512, (JVP ? 2 : 4)) void attn_fwd_wide_kernel(const FwdParams p) {
   split_fwd_body<T, D, JVP, 8>(p);
@@ -228,14 +227,16 @@ __global__ __launch_bounds__(512, (JVP ? 2 : 4)) void attn_fwd_wide_kernel(const
 //     equal rounds lose: B2 N1024 84 -> 88, B8 N256 25 -> 28;
 //   fp32 + tangents D64: B4 N1024 270 -> 236, B32 N256 162 -> 138, B6 N512 134 -> 105; left alone: B20 N256 115 -> 119,
 //     B2 N1024 138 -> 185, B16 N333 150 -> 158;
-//   fp16 D72: B16 N512 48 -> 40, B16 N1024 153 -> 140, B32 N256 29.9 -> 28.5; left alone: B16 N333 26 -> 29, B6 N1024 62 -> 65.
+//   fp32 + tangents D32: B16 N512 180 -> 138, B32 N256 100 -> 77, B64 H12 N256 150 -> 114, B6 N1024 257 -> 230; left alone: B20 N256 75 -> 68;
+//   fp16 D72: B16 N512 47 -> 39, B16 N1024 150 -> 134, B32 N256 28.9 -> 25.4; left alone: B16 N333 26 -> 29, B6 N1024 60 -> 64;
+//   fp16 D80: B16 N512 47.6 -> 39.4, B16 N1024 152 -> 134, B32 N256 29.5 -> 25.6; left alone: B6 N1024 60 -> 64, B20 N256 20.6 -> 22.1.
 static bool wide_split(int Lq, int D, int BH, ElemType type, bool jvp) {
   const int64_t cus = compute_units(), narrow = (int64_t)BH * ((Lq + 127) / 128), wide = (int64_t)BH * ((Lq + 255) / 256);
   auto rounds = [](int64_t n, int64_t slots) { return (n + slots - 1) / slots; };
-  if (type == ElemType::f16 && jvp && (D == 72 || D == 80)) return rounds(wide, cus) < rounds(narrow, cus);
-  if (type == ElemType::f32 && jvp && D == 64) return 172 * rounds(wide, cus) < 100 * rounds(narrow, cus);
-  if (type == ElemType::f16 && !jvp && D == 72 && Lq >= 256) return rounds(wide, 2 * cus) < rounds(narrow, 3 * cus);
-  return false;
+  if (type == ElemType::bf16 || !has_wide_split(type == ElemType::f16, D, jvp)) return false;
+  if (type == ElemType::f32) return 172 * rounds(wide, cus) < 100 * rounds(narrow, cus);
+  if (jvp) return rounds(wide, cus) < rounds(narrow, cus);
+  return Lq >= 256 && rounds(wide, 2 * cus) < rounds(narrow, 3 * cus);
 }
 
 template <typename T, int D, bool JVP, int NW>
@@ -261,7 +262,7 @@ static int launch_fwd_nw(const FwdParams& p, int BH, hipStream_t stream) {
 }
 template <typename T, int D, bool JVP>
 static int launch_fwd_t(const FwdParams& p, int BH, hipStream_t stream) {
-  if constexpr (has_wide_split<T, D, JVP>()) {
+  if constexpr (!std::is_same<T, __bf16>::value && has_wide_split(std::is_same<T, _Float16>::value, D, JVP)) {
     if (wide_split(p.Lq, D, BH, std::is_same<T, float>::value ? ElemType::f32 : ElemType::f16, JVP)) return launch_fwd_nw<T, D, JVP, 8>(p, BH, stream);
   }
   return launch_fwd_nw<T, D, JVP, 4>(p, BH, stream);

@@ -884,7 +884,8 @@ def test_keys_masked_by_extreme_values(dtype, L, value):
     (torch.float16, 72, True, 65, 4, 257, True), (torch.float16, 72, True, 32, 4, 333, True), (torch.float16, 80, True, 65, 4, 256, True),
     (torch.float16, 72, True, 64, 4, 256, True), (torch.float16, 72, True, 32, 4, 256, False), (torch.float16, 72, False, 200, 4, 256, True),
     (torch.float16, 72, False, 256, 4, 300, False), (torch.float32, 64, True, 64, 4, 256, True), (torch.float32, 64, True, 64, 4, 225, True),
-    (torch.float32, 64, True, 65, 4, 256, False)])
+    (torch.float32, 64, True, 65, 4, 256, False), (torch.float16, 80, False, 200, 4, 256, True), (torch.float16, 80, False, 256, 4, 300, False),
+    (torch.float32, 32, True, 64, 4, 256, True), (torch.float32, 32, True, 64, 4, 225, True), (torch.float32, 32, True, 65, 4, 256, False)])
 @pytest.mark.parametrize("Lkv", [None, 1, 31, 65])
 def test_wide_split_forward_against_the_oracle(dtype, D, jvp, B, H, L, wide, Lkv):
     """The fp16 / fp32 forward in 256-row work-groups and its neighbours on either side of the policy: ragged and single key tiles, a
