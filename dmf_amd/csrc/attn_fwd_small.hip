@@ -237,7 +237,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
                                      store_tail16<float, D, C::NMT>(ws, lane, [&](int hq, int e) { return a.tail[hq][e] * s16[hq]; });
                                  });
   };
-  stage(O, f);
+  stage(O, f * kWeightUnit<T>);
   __syncthreads();
   float inv_l, mu_n = 0.f;
   auto row_stats = [&](int r) {
@@ -296,11 +296,11 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
 #pragma unroll
       for (int t = 0; t < C::NMT; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dO.t[t][i] = fmaf(dO.t[t][i], gi, dOv.t[t][i]);
+        for (int i = 0; i < 16; ++i) dO.t[t][i] = fmaf(dO.t[t][i], gi, dOv.t[t][i] * kWeightUnit<T>);
 #pragma unroll
       for (int hq = 0; hq < 2; ++hq)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dO.tail[hq][e] = fmaf(dO.tail[hq][e], gi16[hq], dOv.tail[hq][e]);
+        for (int e = 0; e < 4; ++e) dO.tail[hq][e] = fmaf(dO.tail[hq][e], gi16[hq], dOv.tail[hq][e] * kWeightUnit<T>);
     }
     stage(dO, f);
     __syncthreads();

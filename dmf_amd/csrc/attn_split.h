@@ -25,7 +25,6 @@
 namespace dmf {
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
 
 // NI planes of a loaded operand, NWT of a probability-like one.
 template <typename T> struct SplitType;
@@ -35,6 +34,8 @@ template <> struct SplitType<_Float16> { static constexpr int NI = 1, NWT = 2; s
 // log2 of the factor on P in the f16 kernels: P reaches 2^6 in the forward (kSplitLazyLog2), 1 in the backward, the range 2^16.
 template <typename T> constexpr float kFwdBias = SplitType<T>::F16 ? 9.f : 0.f;
 template <typename T> constexpr float kBwdBias = SplitType<T>::F16 ? 14.f : 0.f;
+// What an accumulator of P (its planes' sum: split8) is multiplied by at the end.
+template <typename T> constexpr float kWeightUnit = SplitType<T>::F16 ? 1.f / (1.f + 1.f / 1024.f) : 1.f;
 constexpr uint32_t kRowScaleBias = 9;   // and of RowScale's largest value before it is raised: 2^5 times that
 
 template <>
@@ -78,11 +79,15 @@ __device__ __forceinline__ void mma_planes16(f32x4& acc, const u32x4 (&a)[NA], c
 }
 
 // x minus the low (0) / high (1) f16 half of w: one mixed-precision instruction where conversion and subtraction take two
-// (exact either way: the difference is).
-template <int HALF>
+// (exact either way: the difference is).  WEIGHT: minus 1 - 2^-10 times it.
+template <int HALF, bool WEIGHT = false>
 __device__ __forceinline__ float sub_half(float x, uint32_t w) {
   float r;
-  if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
+  if constexpr (WEIGHT) {
+    const float m = -1.f + 1.f / 1024.f;
+    if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, %3, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x), "s"(m));
+    else asm("v_fma_mix_f32 %0, %1, %3, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x), "s"(m));
+  } else if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
   else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
   return r;
 }
@@ -97,8 +102,9 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
 // Eight fp32 values as NP planes of eight 16-bit ones.  ANY (operands as the caller gave them, in bf16 planes): all but the last
 // plane are held within the finite range, so that a value above the largest bf16 number does not round to infinity and an
 // infinity or NaN ends up in the last plane alone -- it then meets only the first plane of the other operand, whose sign is the
-// value's.  WEIGHT (probabilities, in f16 planes): the first plane is one step below the truncated value, so that the second is
-// positive wherever the value is, and an infinity among the elements it weighs stays one (next to an exact first plane it met a zero).
+// value's.  WEIGHT (probabilities, in f16 planes): the second plane is the remainder plus 2^-10 of the first, which is at least twice the
+// rounding and makes it positive wherever the value is, so that an infinity among the elements it weighs stays one (next to an exact first
+// plane it met a zero).  The planes' sum is then 1 + 2^-10 times the value, up to 2^-21 of it: kWeightUnit takes that off the accumulator.
 template <typename T, bool ANY = false, bool WEIGHT = false, int NP>
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
   constexpr float kMax = 3.38953139e38f;   // the largest bf16 number
@@ -108,17 +114,10 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&pl)[NP]) {
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       if constexpr (SplitType<T>::F16) {
-        if constexpr (WEIGHT && NP > 1) {
-          if (k + 1 < NP)
-            pl[k][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, __builtin_amdgcn_cvt_pkrtz(a, b)), u16x2{1, 1}));
-          else
-            pl[k][i] = pack_f16x2(a, b);
-        } else {
-          pl[k][i] = pack_f16x2(a, b);
-        }
+        pl[k][i] = pack_f16x2(a, b);
         if (k + 1 < NP) {
-          a = sub_half<0>(a, pl[k][i]);
-          b = sub_half<1>(b, pl[k][i]);
+          a = sub_half<0, WEIGHT>(a, pl[k][i]);
+          b = sub_half<1, WEIGHT>(b, pl[k][i]);
         }
       } else {
         const bool hold = ANY && k + 1 < NP;
@@ -638,26 +637,26 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     if constexpr (JVP)
       if (p.dlse != nullptr) p.dlse[(int64_t)bh * p.Lq + qrow] = mu_n;
   }
-  store_out<T, D, NW>(smem, static_cast<T*>(p.o) + base(6), p.st[6][1], q0, p.Lq, tid, O, inv_l);
+  store_out<T, D, NW>(smem, static_cast<T*>(p.o) + base(6), p.st[6][1], q0, p.Lq, tid, O, inv_l * kWeightUnit<T>);
   if constexpr (JVP) {
     // dO/l - (mu/l) O, in place
-    const float gi = gs.inverse();
+    const float gi = gs.inverse(), mu_o = mu_n * kWeightUnit<T>;
 #pragma unroll
     for (int t = 0; t < C::NMT; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const float d = F16 ? fmaf(dO.t[t][i], gi, dOv.t[t][i]) : dO.t[t][i];
-        dO.t[t][i] = fmaf(-mu_n, O.t[t][i], d);
+        const float d = F16 ? fmaf(dO.t[t][i], gi, dOv.t[t][i] * kWeightUnit<T>) : dO.t[t][i];
+        dO.t[t][i] = fmaf(-mu_o, O.t[t][i], d);
       }
     if constexpr (C::TAIL) {
       float mu16[2], gi16[2];
-      swap16f(mu_n, mu16[0], mu16[1]);
+      swap16f(mu_o, mu16[0], mu16[1]);
       swap16f(gi, gi16[0], gi16[1]);
 #pragma unroll
       for (int hq = 0; hq < 2; ++hq)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float d = F16 ? fmaf(dO.tail[hq][e], gi16[hq], dOv.tail[hq][e]) : dO.tail[hq][e];
+          const float d = F16 ? fmaf(dO.tail[hq][e], gi16[hq], dOv.tail[hq][e] * kWeightUnit<T>) : dO.tail[hq][e];
           dO.tail[hq][e] = fmaf(-mu16[hq], O.tail[hq][e], d);
         }
     }
@@ -841,7 +840,7 @@ __device__ __forceinline__ void split_bwd_dkv_body(const BwdParams& p) {
   }
   constexpr float kUnbias = SplitType<T>::F16 ? 1.f / 16384.f : 1.f;   // 2^-kBwdBias
   store_out<T, D, NW>(smem, static_cast<T*>(p.dk) + base(6), p.st[6][1], k0, p.Lkv, tid, dK, p.scale * kUnbias * gs.inverse());
-  store_out<T, D, NW>(smem, static_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid, dV, kUnbias);
+  store_out<T, D, NW>(smem, static_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid, dV, kUnbias * kWeightUnit<T>);
 }
 
 }  // namespace dmf
