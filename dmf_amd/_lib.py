@@ -90,28 +90,42 @@ def load() -> ctypes.CDLL:
 
 
 _host_module = None
+_host_error = None   # why there is none
+
+
+def _load_host():
+    """The native host path, or None with the reason in ``_host_error``: it is built against one torch and one Python."""
+    global _host_module, _host_error
+    if _host_module is None and _host_error is None:
+        load()
+        try:
+            from . import _host
+            if _host.torch_version != torch.__version__.partition("+")[0]:
+                raise ImportError(f"built for torch {_host.torch_version}, torch {torch.__version__} is installed")
+            _host.bind(sys.modules[__name__])
+            _host_module = _host
+        except ImportError as e:
+            _host_error = e
+            warnings.warn(f"dmf_amd/_host*.so is missing or does not fit the installed torch ({e}): operators take the Python route around the "
+                          "same kernels, at some 10 to 100 us of host time more per call; `python -m dmf_amd.build` builds it", RuntimeWarning,
+                          stacklevel=3)
+    return _host_module
 
 
 def host():
     """The native host path (dmf_amd/_host*.so, built together with the kernel library): each function does a whole operator
     call -- forward-AD duals, one torch.func.jvp level, autograd node, launch -- or returns None where the general route
     below has to be taken."""
-    global _host_module
-    if _host_module is None:
-        load()
-        try:
-            from . import _host
-        except ImportError as e:
-            raise RuntimeError("dmf_amd/_host*.so is missing or does not fit the installed torch: build it with `python -m dmf_amd.build`") from e
-        _host.bind(sys.modules[__name__])
-        _host_module = _host
+    if _load_host() is None:
+        raise RuntimeError("dmf_amd/_host*.so is missing or does not fit the installed torch: build it with `python -m dmf_amd.build`") from _host_error
     return _host_module
 
 
 def native(t, *others) -> bool:
     """True where an operator call on these operands may try the native host path: GPU tensors, none of a class with a
-    ``__torch_function__`` of its own, outside of torch.compile's tracing."""
-    return t.is_cuda and not torch.compiler.is_compiling() and not torch.overrides.has_torch_function((t, *others))
+    ``__torch_function__`` of its own, outside of torch.compile's tracing, and the path is there."""
+    return (t.is_cuda and not torch.compiler.is_compiling() and not torch.overrides.has_torch_function((t, *others))
+            and (_host_module is not None or _load_host() is not None))
 
 
 def _check(rc: int, what: str) -> None:

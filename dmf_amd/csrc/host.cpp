@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 #include <torch/extension.h>
+#include <torch/version.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/autocast_mode.h>
@@ -649,19 +650,15 @@ py::object ln_modulate(const Tensor& x_, const Tensor& shift_, const Tensor& sca
   return py::cast(finish(y, ty, node, level));
 }
 
-// x (and its tangent) in the promoted type of x and h
-bool promote(Arg& x, const Arg& h) {
-  const auto dt = c10::promoteTypes(x.data.scalar_type(), h.data.scalar_type());
-  if (x.data.scalar_type() == dt) return true;
-  return false;   // rare (a low-precision residual stream next to fp32 branches): the general route casts
-}
+// The result has the promoted type of x and h.  Where that is not x's own (a low-precision residual stream next to fp32 branches: rare) the
+// general route casts.
+bool keeps_type(const Arg& x, const Arg& h) { return c10::promoteTypes(x.data.scalar_type(), h.data.scalar_type()) == x.data.scalar_type(); }
 
 py::object gate_residual(const Tensor& x_, const Tensor& gate_, const Tensor& h_) {
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
-  Arg x = unpack(x_);
-  const Arg gate = unpack(gate_), h = unpack(h_);
-  if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !promote(x, h)) return none();
+  const Arg x = unpack(x_), gate = unpack(gate_), h = unpack(h_);
+  if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !keeps_type(x, h)) return none();
   const Blc n(x.data);
   if (!mods_ok(n.B, n.C, gate) || gate.data.device() != x.data.device() || h.data.device() != x.data.device()) return none();
   if (only_tangents_want(x, gate, h)) return none();
@@ -694,9 +691,8 @@ py::object gate_residual(const Tensor& x_, const Tensor& gate_, const Tensor& h_
 py::object residual_ln_modulate(const Tensor& x_, const Tensor& gate_, const Tensor& h_, const Tensor& shift_, const Tensor& scale_, double eps) {
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
-  Arg x = unpack(x_);
-  const Arg gate = unpack(gate_), h = unpack(h_), sh = unpack(shift_), sc = unpack(scale_);
-  if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !promote(x, h)) return none();
+  const Arg x = unpack(x_), gate = unpack(gate_), h = unpack(h_), sh = unpack(shift_), sc = unpack(scale_);
+  if (!blc_ok(x) || !blc_ok(h) || h.data.sizes() != x.data.sizes() || !keeps_type(x, h)) return none();
   const Blc n(x.data);
   const auto out_t = autocast_type(x.data);
   if (!mods_ok(n.B, n.C, gate, sh, sc) || gate.data.device() != x.data.device() || h.data.device() != x.data.device() ||
@@ -1121,6 +1117,7 @@ py::object modulations(const std::vector<Tensor>& conds_, const std::vector<int>
 
 PYBIND11_MODULE(_host, m) {
   m.doc() = "native host path of dmf_amd's operators (None: take the general route)";
+  m.attr("torch_version") = TORCH_VERSION;
   m.def("bind", [](py::object lib) { g_lib = lib.release(); });
   m.def("attention", &attention);
   m.def("attention_packed", &attention_packed);

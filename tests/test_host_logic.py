@@ -360,3 +360,27 @@ def test_weight_gradient_keeps_padded_rows_within_32_bits(M, N, K):
     narrower = (M, N - 8, K) if (1 << 25) == N else None
     if narrower:
         assert lib.dmf_linear_wgrad_workspace_floats(*narrower) >= 0
+
+
+@pytest.mark.parametrize("built_for", [None, "0.0.1"])
+def test_operators_do_without_the_native_host_path(monkeypatch, built_for):
+    """Where the extension is missing or was built for another torch, operator calls take the Python route and say so once."""
+    import sys
+    import types
+    import warnings
+
+    fake = None if built_for is None else types.SimpleNamespace(torch_version=built_for, bind=lambda lib: pytest.fail("bound"))
+    monkeypatch.setattr(_lib, "_host_module", None)
+    monkeypatch.setattr(_lib, "_host_error", None, raising=False)
+    monkeypatch.setitem(sys.modules, "dmf_amd._host", fake)
+    monkeypatch.delattr(dmf_amd, "_host", raising=False)
+    if fake is not None:
+        monkeypatch.setattr(dmf_amd, "_host", fake, raising=False)
+    on_gpu = types.SimpleNamespace(is_cuda=True)
+    with pytest.warns(RuntimeWarning, match="Python route"):
+        assert not _lib.native(on_gpu)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert not _lib.native(on_gpu)
+    with pytest.raises(RuntimeError, match="dmf_amd.build"):
+        _lib.host()
