@@ -100,8 +100,8 @@ def _load_host():
         load()
         try:
             from . import _host
-            if _host.torch_version != torch.__version__.partition("+")[0]:
-                raise ImportError(f"built for torch {_host.torch_version}, torch {torch.__version__} is installed")
+            if getattr(_host, "torch_version", None) != torch.__version__.partition("+")[0]:
+                raise ImportError(f"built for torch {getattr(_host, 'torch_version', '(unknown)')}, torch {torch.__version__} is installed")
             _host.bind(sys.modules[__name__])
             _host_module = _host
         except ImportError as e:
