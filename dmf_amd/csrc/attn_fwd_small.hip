@@ -136,7 +136,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     if constexpr (F16) dOv.zero();
   }
   RowScale<T> gs;
-  // Start of the running maximum (log2 units): finite, so that a tile of nothing but keys masked by -inf weighs nothing, and no higher
+  // Start of the running maximum (log2 units; less kFwdBias, as in split_fwd_body): finite, so that a tile of nothing but keys masked by -inf weighs nothing, and no higher
   // than any score, so that a row whose keys all carry the lowest number still has its maximum (which is subtracted exactly: weights of one).
   float m_run = -3.40282347e38f, l_run = 0.f, mu_run = 0.f;
   const float c2 = p.scale_log2;
@@ -176,8 +176,8 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
 #pragma unroll
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, Sc[i]);
     mx = xhalf_max(mx);
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
-      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
+    if (__builtin_amdgcn_ballot_w64(mx > m_run + (kSplitLazyLog2 + kFwdBias<T>)) != 0) {
+      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) - kFwdBias<T> : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
@@ -188,10 +188,9 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
       }
     }
     f32x16 E, G;
-    const float m_off = m_run - kFwdBias<T>;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      E[i] = fast_exp2(Sc[i] - m_off);
+      E[i] = fast_exp2(Sc[i] - m_run);
       l_run += E[i];
       if constexpr (JVP) {
         G[i] = E[i] * (dS[i] * p.scale);
@@ -255,7 +254,7 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
     const float l = row_stats(tid);
     const int row = q0 + tid;
     if (row < p.Lq) {
-      if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + row] = (m - kFwdBias<T> + log2f(l)) * kLn2;
+      if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + row] = (m + log2f(l)) * kLn2;
       if constexpr (JVP)
         if (p.dlse != nullptr) p.dlse[(int64_t)bh * p.Lq + row] = mu_n;
     }

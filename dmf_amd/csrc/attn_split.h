@@ -534,7 +534,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     if constexpr (F16) dOv.zero();
   }
   RowScale<T> gs;
-  float m_run = kLowestMax, l_run = 0.f, mu_run = 0.f;
+  float m_run = kLowestMax, l_run = 0.f, mu_run = 0.f;   // m_run: the running maximum less kFwdBias
   const float c2 = p.scale_log2;
 
   const int ntiles = (p.Lkv + 31) / 32;
@@ -578,9 +578,9 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
 #pragma unroll
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, S[i]);
     mx = xhalf_max(mx) * c2;
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + kSplitLazyLog2) != 0) {
-      // (a whole number in the f16 kernels: nothing is rounded when kFwdBias is taken off)
-      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
+    if (__builtin_amdgcn_ballot_w64(mx > m_run + (kSplitLazyLog2 + kFwdBias<T>)) != 0) {
+      // (whole numbers in the f16 kernels: alpha is a power of two, and nothing is rounded when kFwdBias is taken off)
+      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) - kFwdBias<T> : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
@@ -591,10 +591,9 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
       }
     }
     f32x16 E, G;
-    const float m_off = m_run - kFwdBias<T>;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      E[i] = fast_exp2(fmaf(S[i], c2, -m_off));
+      E[i] = fast_exp2(fmaf(S[i], c2, -m_run));
       l_run += E[i];
       if constexpr (JVP) {
         G[i] = E[i] * (dS[i] * p.scale);
@@ -633,7 +632,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   const float l_tot = xhalf_sum(l_run), inv_l = 1.0f / l_tot;
   const float mu_n = JVP ? xhalf_sum(mu_run) * inv_l : 0.f;
   if (g == 0 && qrow < p.Lq) {
-    if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + qrow] = (m_run - kFwdBias<T> + log2f(l_tot)) * kLn2;
+    if (p.lse != nullptr) p.lse[(int64_t)bh * p.Lq + qrow] = (m_run + log2f(l_tot)) * kLn2;
     if constexpr (JVP)
       if (p.dlse != nullptr) p.dlse[(int64_t)bh * p.Lq + qrow] = mu_n;
   }
