@@ -63,13 +63,9 @@ __device__ __forceinline__ void generic_bwd_dq_body(const BwdParams& p) {
       const u32x4 ov = in ? *reinterpret_cast<const u32x4*>(go + cv * VEC) : u32x4{0, 0, 0, 0};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        if constexpr (C::BF) {
-          // bf16 -> fp32 is a 16-bit shift
-          dpart += __uint_as_float(dOr[c][e] << 16) * __uint_as_float(ov[e] << 16);
-          dpart += __uint_as_float(dOr[c][e] & 0xffff0000u) * __uint_as_float(ov[e] & 0xffff0000u);
-        } else {
-          dpart += __uint_as_float(dOr[c][e]) * __uint_as_float(ov[e]);
-        }
+        // bf16 -> fp32 is a 16-bit shift
+        dpart += __uint_as_float(dOr[c][e] << 16) * __uint_as_float(ov[e] << 16);
+        dpart += __uint_as_float(dOr[c][e] & 0xffff0000u) * __uint_as_float(ov[e] & 0xffff0000u);
       }
     }
   }
@@ -248,7 +244,7 @@ __device__ __forceinline__ void generic_bwd_dkv_body(const BwdParams& p) {
 
 // fp32 and fp16 take the split-operand bodies (attn_split.h).  From head dim 72 on two fp32 rows per lane in three planes plus the
 // accumulators need the register file of one wave per SIMD; at head dim 64 two waves win although the dK/dV kernel then spills
-// 19 registers (B16 H12 N256: 111 -> 98 us for the pair).
+// 12 registers (B16 H12 N256: 111 -> 98 us for the pair).
 template <typename T, int D>
 constexpr int bwd_waves_per_simd() { return D <= 64 || (std::is_same<T, _Float16>::value && D <= 96) ? 2 : 1; }
 

@@ -4,15 +4,16 @@
 //   lane = threadIdx.x & 63,  c32 = lane & 31,  g = lane >> 5.
 //   A 32x32 fp32 accumulator tile `acc[16]` of a lane holds
 //       row(i) = (i/4)*8 + 4*g + (i%4),   col = c32.
-//   An MFMA operand "chunk" is one 16-byte vector per lane:
-//     bf16: 8 elements = contraction slots of ONE v_mfma_f32_32x32x16_bf16,
-//     fp32: 4 elements = the operand of FOUR v_mfma_f32_32x32x2_f32.
+//   An MFMA operand "chunk" is one 16-byte vector per lane: 8 bf16 elements, the
+//   contraction slots of one v_mfma_f32_32x32x16_bf16 (fp32 and fp16 operands:
+//   attn_split.h).
 //   Both operands of a product always use the same slot->index mapping, so
 //   any consistent permutation of the contraction index is legal; the kernels
 //   exploit that to feed accumulator tiles straight back in as operands.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include <utility>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -84,36 +85,30 @@ __device__ __forceinline__ u32x4 split3_bf16(float x) {
   return u32x4{h | (m << 16), pack_bf16x2(r2, 0.f), 0u, 0u};
 }
 
-// Static configuration for element type T (float or __bf16) and head dim D.
+// Static configuration for element type T and head dim D: vectors and staging rows of any type, operand chunks and tiles of bf16.
 template <typename T, int D>
 struct Cfg {
   static_assert(D % 8 == 0 && D >= 16 && D <= 128, "head dim must be a multiple of 8 in [16,128]");
-  static constexpr bool BF = sizeof(T) == 2;
   static constexpr int VEC = 16 / (int)sizeof(T);              // elements per 16-byte vector
   static constexpr int VPR = D / VEC;                          // valid vectors per row
-  static constexpr int NCHUNK = BF ? (D + 15) / 16 : D / 8;    // operand chunks over the head dim
+  static constexpr int NCHUNK = (D + 15) / 16;                 // operand chunks over the head dim
   static constexpr int NDT = (D + 31) / 32;                    // 32-wide output tiles over the head dim
   static constexpr int ROWV0 = (2 * NCHUNK > VPR ? 2 * NCHUNK : VPR);
   static constexpr int ROWV = ROWV0 + 1 + (ROWV0 & 1);         // LDS row pitch in vectors, odd => conflict-free b128 reads
   static constexpr int STRIDE = ROWV * VEC;                    // LDS row pitch in elements
   static constexpr int OROWV = NDT * 32 / VEC + 1;             // epilogue staging pitch (vectors, odd)
   static constexpr int OSTRIDE = OROWV * VEC;
-  static constexpr int NSUB = BF ? 2 : 1;                      // 32-row sub-tiles per KV tile
+  static constexpr int NSUB = 2;                               // 32-row sub-tiles per KV tile
   static constexpr int BKV = 32 * NSUB;
   static constexpr int TILE_BYTES = BKV * ROWV * 16;
-  static constexpr int PV_STEPS = BF ? 2 : 16;                 // operand steps per 32-row sub-tile in P*V-like products
+  static constexpr int PV_STEPS = 2;                           // operand steps per 32-row sub-tile in P*V-like products
 };
 
 // acc += A_chunk * B_chunk  (one 16-byte operand chunk per lane each).
 template <typename T>
 __device__ __forceinline__ void mma_chunk(f32x16& acc, const u32x4& a, const u32x4& b) {
-  if constexpr (sizeof(T) == 2) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[e]), __uint_as_float(b[e]), acc, 0, 0, 0);
-  }
+  static_assert(std::is_same<T, __bf16>::value, "operand chunks are bf16");
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
 }
 
 // Operand chunk c of row `row` of a row-major LDS tile (contraction along the row).
@@ -126,26 +121,20 @@ __device__ __forceinline__ u32x4 lds_row_chunk(const T* tile, int row, int c, in
 // tile (P*V-like): the lane's M index is column col0 + c32 and the contraction
 // slots follow the accumulator row order of the lane (see header comment), so
 // an accumulator tile converted with acc_operand() is the matching B operand.
-//   bf16: step s in {0,1} covers rows r0+16s .. r0+16s+15 (two ds_read_b64_tr_b16).
-//   fp32: step s in 0..15 covers row r0 + (s/4)*8 + 4g + s%4.
+// Step s in {0,1} covers rows r0+16s .. r0+16s+15 (two ds_read_b64_tr_b16).
 struct ColOperand { u32x4 v; };
 
 template <typename T, int STRIDE>
 __device__ __forceinline__ ColOperand lds_col_operand(const T* tile, int r0, int col0, int s, int lane) {
+  static_assert(std::is_same<T, __bf16>::value, "operand chunks are bf16");
   ColOperand r;
-  if constexpr (sizeof(T) == 2) {
-    const int g = lane >> 5, i = lane & 15, half = (lane >> 4) & 1;
-    // 16 lanes cooperatively fetch a 4(row) x 16(col) block; lane i supplies row i/4, cols 4*(i%4)..+3
-    const T* p = tile + (r0 + 16 * s + 4 * g + (i >> 2)) * STRIDE + col0 + 16 * half + 4 * (i & 3);
-    s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p));
-    s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p + 8 * STRIDE));
-    u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
-    r.v = u32x4{a[0], a[1], b[0], b[1]};
-  } else {
-    const int g = lane >> 5, c32 = lane & 31;
-    const int row = r0 + (s >> 2) * 8 + 4 * g + (s & 3);
-    r.v = u32x4{__float_as_uint(tile[row * STRIDE + col0 + c32]), 0u, 0u, 0u};
-  }
+  const int g = lane >> 5, i = lane & 15, half = (lane >> 4) & 1;
+  // 16 lanes cooperatively fetch a 4(row) x 16(col) block; lane i supplies row i/4, cols 4*(i%4)..+3
+  const T* p = tile + (r0 + 16 * s + 4 * g + (i >> 2)) * STRIDE + col0 + 16 * half + 4 * (i & 3);
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p));
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p + 8 * STRIDE));
+  u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
+  r.v = u32x4{a[0], a[1], b[0], b[1]};
   return r;
 }
 
@@ -231,23 +220,17 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // the probabilities / weights to be contracted).
 template <typename T>
 __device__ __forceinline__ ColOperand acc_operand(const f32x16& e, int s) {
+  static_assert(std::is_same<T, __bf16>::value, "operand chunks are bf16");
   ColOperand r;
-  if constexpr (sizeof(T) == 2) {
-    r.v = u32x4{pack_bf16x2(e[8 * s + 0], e[8 * s + 1]), pack_bf16x2(e[8 * s + 2], e[8 * s + 3]),
-                pack_bf16x2(e[8 * s + 4], e[8 * s + 5]), pack_bf16x2(e[8 * s + 6], e[8 * s + 7])};
-  } else {
-    r.v = u32x4{__float_as_uint(e[s]), 0u, 0u, 0u};
-  }
+  r.v = u32x4{pack_bf16x2(e[8 * s + 0], e[8 * s + 1]), pack_bf16x2(e[8 * s + 2], e[8 * s + 3]),
+              pack_bf16x2(e[8 * s + 4], e[8 * s + 5]), pack_bf16x2(e[8 * s + 6], e[8 * s + 7])};
   return r;
 }
 
 template <typename T>
 __device__ __forceinline__ void mma_col(f32x16& acc, const ColOperand& a, const ColOperand& b) {
-  if constexpr (sizeof(T) == 2) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a.v), __builtin_bit_cast(bf16x8, b.v), acc, 0, 0, 0);
-  } else {
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.v[0]), __uint_as_float(b.v[0]), acc, 0, 0, 0);
-  }
+  static_assert(std::is_same<T, __bf16>::value, "operand chunks are bf16");
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a.v), __builtin_bit_cast(bf16x8, b.v), acc, 0, 0, 0);
 }
 
 // Row index inside a 32-row tile held by accumulator element i of a lane in half g.
