@@ -515,16 +515,28 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   // dQ planes beside Q's in registers, or where that would spill in LDS, in the order in which this wave reads them back
   u32x4 Q[NCHUNK][NI], dQ[JVP && !Plan::DQ_LDS ? NCHUNK : 1][NI];
   u32x4* const dQl = reinterpret_cast<u32x4*>(smem + Plan::DQ_OFF) + wave * (NCHUNK * NI * 64) + lane;
+  // The sign of the softmax scale goes into Q and dQ, and one of zero makes them zero, so that the scores keep their order: keys are masked and
+  // the maximum is taken of the unscaled ones.
+  const uint32_t keep = p.scale_log2 == 0.f ? 0u : ~0u, flip = p.scale_log2 < 0.f ? 0x80008000u : 0u;
+  auto signed_rows = [&](u32x4 (&x)[NCHUNK][NI]) {
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c)
+#pragma unroll
+      for (int k = 0; k < NI; ++k) x[c][k] = (x[c][k] & keep) ^ flip;
+  };
   load_own_row<T, D, NW>(static_cast<const T*>(p.q) + base(0), p.st[0][1], qrow, p.Lq, g, Q);
+  signed_rows(Q);
   if constexpr (Plan::DQ_LDS) {
     u32x4 x[NCHUNK][NI];
     load_own_row<T, D, NW>(static_cast<const T*>(p.tq) + base(3), p.st[3][1], qrow, p.Lq, g, x);
+    signed_rows(x);
 #pragma unroll
     for (int c = 0; c < NCHUNK; ++c)
 #pragma unroll
       for (int k = 0; k < NI; ++k) dQl[(c * NI + k) * 64] = x[c][k];
   } else if constexpr (JVP) {
     load_own_row<T, D, NW>(static_cast<const T*>(p.tq) + base(3), p.st[3][1], qrow, p.Lq, g, dQ);
+    signed_rows(dQ);
   }
 
   OutAcc<T, D, NW> O, dO, dOv;   // dOv (fp16 tangents only): dV^T P, apart because dO carries the row scale of P*dS
@@ -535,7 +547,8 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   }
   RowScale<T> gs;
   float m_run = kLowestMax, l_run = 0.f, mu_run = 0.f;   // m_run: the running maximum less kFwdBias
-  const float c2 = p.scale_log2;
+  auto uniform = [](float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); };   // (else in a vector register)
+  const float c2 = uniform(p.scale_log2 == 0.f ? 1.f : fabsf(p.scale_log2)), scale = uniform(fabsf(p.scale));
 
   const int ntiles = (p.Lkv + 31) / 32;
   commit_k(0);
@@ -596,7 +609,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
       E[i] = fast_exp2(fmaf(S[i], c2, -m_run));
       l_run += E[i];
       if constexpr (JVP) {
-        G[i] = E[i] * (dS[i] * p.scale);
+        G[i] = E[i] * (dS[i] * scale);
         mu_run += G[i];
       }
     }

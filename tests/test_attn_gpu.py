@@ -1049,3 +1049,36 @@ def test_half_infinite_values_stay_infinite(spread, B, H, L, D):
     do[:, L // 2, :, 3] = math.inf
     _, _, dv = _lib.bwd_half(do, q, k, v, torch.zeros_like(o), lse, D ** -0.5)
     assert (dv[..., 3] == math.inf).all() and dv[..., rest].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype,B,H,D", [(torch.float16, 340, 2, 64), (torch.float16, 340, 2, 72), (torch.float16, 200, 4, 72), (torch.float16, 340, 2, 128),
+                                         (torch.float32, 2, 2, 64), (torch.float32, 64, 4, 64), (torch.float32, 2, 2, 72)])
+@pytest.mark.parametrize("scale", [-2.0, -0.125, 0.0])
+def test_softmax_scale_of_any_sign_in_the_split_operand_kernels(scale, dtype, B, H, D):
+    """As test_softmax_scale_of_any_sign, for the fp16 and fp32 kernels on grids of every size, with their gradients: fp16 spreads of scores far
+    beyond the 2^16 of a probability's range."""
+    half = dtype == torch.float16
+    for L in (100, 256):
+        assert "small" not in _lib.plan("fwd", B, H, L, L, D, dtype)
+        g = torch.Generator(device=DEV).manual_seed(L + D)
+        x = [torch.randn(B, L, H, D, generator=g, device=DEV).to(dtype) for _ in range(7)]
+        o, to, lse = (_lib.fwd_jvp_half if half else _lib.fwd_jvp)(*x[:6], scale)
+        o2, _ = (_lib.fwd_half if half else _lib.fwd)(*x[:3], scale)
+        grads = (_lib.bwd_half if half else _lib.bwd)(x[6], *x[:3], o, lse, scale)
+        x64 = [t[:2].double().cpu() for t in x]
+        fn = lambda q, k, v: _softmax_attention(q, k, v, scale)
+        o_ref, to_ref = torch.func.jvp(fn, tuple(x64[:3]), tuple(x64[3:6]))
+        ref = torch.autograd.grad(fn(*(t.requires_grad_() for t in x64[:3])), x64[:3], x64[6])
+        # fp16: the result's rounding (5e-4 at most).  fp32: 1e-5, and scores of magnitude |scale| D, whose fp32 sums are 2^-24 of that off,
+        # in the exponent; tangents and q / k gradients cancel to a part of their terms
+        tol = 1e-3 if half else 1e-5 * max(1.0, abs(scale))
+        pairs = [("o", o, o_ref), ("o primal", o2, o_ref), ("to", to, to_ref), ("dv", grads[2], ref[2])]
+        if scale != 0:
+            pairs += [("dq", grads[0], ref[0]), ("dk", grads[1], ref[1])]
+        else:
+            assert not grads[0].any() and not grads[1].any()
+        for name, got, exp in pairs:
+            err = ao.rel_l2(got[:2].double().cpu(), exp.detach())
+            print(f"{name} L{L} {err:.2e}", flush=True)
+            # (a rounded fp16 output next to a nearly one-hot row: its error is what dq and dk consist of there)
+            assert err <= tol * (10 if name in ("to", "dq", "dk") and abs(scale) > 1 else 1), (name, L, err)
