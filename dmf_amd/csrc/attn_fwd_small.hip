@@ -328,7 +328,7 @@ static int launch_small_t(const FwdParams& p, int BH, hipStream_t stream) {
   return launch_kernel(kern, dim3((uint32_t)((p.Lq + 31) / 32) * (uint32_t)BH), dim3(64 * kSmallWaves), smem, stream, p);
 }
 
-// With tangents a wave keeps K, dK, Q, dQ and two accumulator sets: 324 .. 480 registers up to head dim 80, and beyond that
+// With tangents a wave keeps K, dK, Q, dQ and two accumulator sets: 336 .. 492 registers up to head dim 80, and beyond that
 // more than there are (head dim 128: 86 .. 534 spilled), so those stay with the tuned kernel.
 constexpr int kSmallMaxDimJvp = 80;
 

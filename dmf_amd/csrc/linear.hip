@@ -247,7 +247,10 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
 //   single: C768 M2048 N 3C 16.4 -> 13.1, M4096 N 3C 19.9 -> 20.5, N C 12.0 -> 9.4, gelu N 4C 29.5 -> 26.0; C1152 M8192 N 3C 79 -> 70;
 //   the library keeps single products with few columns for their depth (K 4C: M4096 C768 26.9 against 31.3, C1152 48 against 56), pairs
 //   that spread a short K over a large result (N 4C M16384: C768 141 against 155, C1152 296 against 317; C768 with gelu 86 against 90)
-//   and outputs narrower than a tile.
+//   and outputs narrower than a tile;
+//   pairs with gelu (library pair and activation kernel; this kernel's pair and the activation kernel -> here), N 4C, wins from one row up:
+//     M16 C384 10.4; 7.7 -> 5.3, C768 11.3; 8.1 -> 7.1, C1152 12.7; 9.2 -> 8.9;  M512 C768 23.4; 15.5 -> 10.6, C1152 34.0; 24.1 -> 18.3;
+//     M4096 C768 61.7; 58.2 -> 44.1, C1152 131; 104 -> 85;  M8192 C384 63.8; 43.6 -> 30.1, C1024 152; 182 -> 142, C1152 212; 212 -> 169.
 extern "C" int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu) {
   if (M < 1 || N < 64 || N % 8 || K < 64 || K % 64 || M * K > (int64_t)1 << 30 || (int64_t)N * K > (int64_t)1 << 30 || M * N > (int64_t)1 << 30) return 0;
   if (jvp && gelu) return 1;
@@ -474,10 +477,14 @@ extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
 }
 
 // Which weight gradients this kernel is the faster one for (us, library -> here; the library's launch alone takes 20 us of host time):
-//   M 1000: 768 x 768 20.5 -> 15.6, 4608 x 1152 29 -> 20;  M 2048: 1536 x 384 20.0 -> 18.4, but 2304 x 768 21 against 23, 3456 x 1152 28 against 34;
+//   up to M 1472 on every result of the models (column sums included on both sides): M 1 .. 128, the adaLN layers' batches: 2304 x 384
+//   9.3 .. 12.4 -> 6.3 .. 7.1, 4608 x 768 12.5 .. 15.3 -> 8.0 .. 8.8, 6912 x 1152 16.3 .. 22.0 -> 12.3 .. 14.1;  M 512: 768 x 768 15.2 -> 12.4,
+//   4608 x 1152 27.1 -> 15.5;  M 1000: 768 x 768 20.5 -> 15.9, 4608 x 1152 38.9 -> 23.3;  M 1472: 3072 x 768 30.5 -> 27.7, 3456 x 1152 32.8 -> 29.0;
+//   M 2048: 1536 x 384 20.0 -> 18.4, but 2304 x 768 21 against 23, 3456 x 1152 28 against 34;
 //   M 4096: 3072 x 768 42 -> 36, 1152 x 1152 33 -> 25, but 3456 x 1152 46 against 51;  M 8192: 3456 x 1152 83 -> 81, 4608 x 1152 119 -> 101,
 //   1152 x 4608 118 -> 97, 1152 x 1152 61 -> 36, 768 x 768 48 -> 24;  M 16384: 3072 x 768 172 -> 94, 4608 x 1152 327 -> 183 (948 TFLOP/s);
-//   widths that 192 columns do not divide lose on large results: 4096 x 1024 M 8192 86 against 89.  Results beyond 8 M elements are not measured.
+//   widths that 192 columns do not divide lose on large results: 4096 x 1024 M 8192 86 against 89.  The largest result
+//   measured is 6912 x 1152 (8 M elements); beyond it the library's products are kept.
 extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return 0;
   const int64_t result = (int64_t)N * K;

@@ -153,7 +153,8 @@ def flash_attn_func(q, k, v, softmax_scale=None):
     has -- exact, since zero columns add nothing to the scores and give zero output
     columns -- at the price of a padded copy of every operand.  fp16 operands (the
     reference's ``--mixed-precision fp16`` / ``--dtype fp16``) have kernels of their own
-    (fp32 accumulation and softmax, nothing rounded to fp16 before the result); with
+    (fp32 accumulation and softmax, nothing rounded to fp16 before the result; weights
+    below some 2**-33 of a row's largest are dropped, also in front of an infinite value); with
     k, v of another type next to an fp16 q everything is computed in fp32 and rounded back.
     """
     if _lib.native(q, k, v):

@@ -90,3 +90,24 @@ def test_lds_budgets(kernels):
     declares more than the 160 KB of a CU."""
     for n, k in kernels.items():
         assert k.get("group_segment_fixed_size", 0) <= 160 * 1024, (n, k)
+
+
+# (pattern of the mangled name, most vector registers, most spilled ones): what the launch bounds of the other kernels with a register
+# plan allow -- 256 where two waves share a SIMD, 128 where four do -- and the few spills that were measured to cost less than they save
+BUDGETS = [
+    (r"13linear_kernelI", 256, 0), (r"19linear_wgrad_kernelE", 256, 0), (r"17modulation_kernelI", 512, 0),
+    (r"21attn_fwd_small_kernelIDF16_Li(64|72|80|96)ELb0E", 256, 0), (r"21attn_fwd_small_kernelIDF16bLi(64|72|80|96)ELb0ELb0E", 256, 0),
+    (r"21attn_fwd_small_kernelI", 512, 0),
+    (r"20attn_fwd_wide_kernelIDF16_Li(72|80)ELb0E", 128, 4), (r"20attn_fwd_wide_kernelI(DF16_Li(72|80)|fLi(32|64))ELb1E", 256, 0),
+    (r"18attn_bwd_dq_kernelI(f|DF16_)Li64E", 256, 0), (r"19attn_bwd_dkv_kernelIDF16_Li(64|72|80)E", 256, 0), (r"19attn_bwd_dkv_kernelIfLi64E", 256, 12),
+    (r"18attn_bwd_dq_kernelI(f|DF16_)Li72E", 512, 0), (r"19attn_bwd_dkv_kernelIfLi72E", 512, 0),
+]
+
+
+@pytest.mark.parametrize("pattern,registers,spills", BUDGETS)
+def test_products_and_split_operand_kernels_stay_within_their_launch_bounds(kernels, pattern, registers, spills):
+    names = [n for n in kernels if re.search(pattern, n)]
+    assert names, pattern
+    for n in names:
+        k = kernels[n]
+        assert k["vgpr_count"] <= registers and k["vgpr_spill_count"] <= spills, (n, k)
