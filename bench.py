@@ -41,17 +41,17 @@ HBM_PEAK_GBS = 8000.0
 # q, k, v, dout twice.
 OFFLINE_COUNTERS = {
     ("fwd_jvp", "xl2_512px"): {"traffic": 1.2125e+09, "mfma_busy": 0.598, "kernel": "dmf::attn_fwd_bf16_kernel<72, true, 8, false, false>",
-                               "src": ("attn_fwd_bf16.hip", "7e3d2d2a31c113f8")},
+                               "src": ("attn_fwd_bf16.hip", "84019e6eea585528")},
     ("fwd_jvp", "xl2_256px"): {"traffic": 1.2124e+09, "mfma_busy": 0.351, "kernel": "dmf::attn_fwd_bf16_kernel<72, true, 8, false, false>",
-                               "src": ("attn_fwd_bf16.hip", "7e3d2d2a31c113f8")},
+                               "src": ("attn_fwd_bf16.hip", "84019e6eea585528")},
     ("fwd", "xl2_512px"): {"traffic": 6.0847e+08, "mfma_busy": 0.530, "kernel": "dmf::attn_fwd_bf16_kernel<72, false, 8, false, false>",
-                           "src": ("attn_fwd_bf16.hip", "7e3d2d2a31c113f8")},
+                           "src": ("attn_fwd_bf16.hip", "84019e6eea585528")},
     ("fwd", "xl2_256px"): {"traffic": 6.0897e+08, "mfma_busy": 0.301, "kernel": "dmf::attn_fwd_bf16_kernel<72, false, 8, false, false>",
-                           "src": ("attn_fwd_bf16.hip", "7e3d2d2a31c113f8")},
+                           "src": ("attn_fwd_bf16.hip", "84019e6eea585528")},
     ("bwd", "xl2_512px"): {"traffic": 1.8710e+09, "mfma_busy": 0.514,
-                           "kernel": "dmf::attn_bwd_dq_bf16_kernel<72, 2> + dmf::attn_bwd_dkv_bf16_kernel<72, 4>", "src": ("attn_bwd_bf16.hip", "499e8cb752b49fb2")},
+                           "kernel": "dmf::attn_bwd_dq_bf16_kernel<72, 2> + dmf::attn_bwd_dkv_bf16_kernel<72, 4>", "src": ("attn_bwd_bf16.hip", "03652ae92e25ff31")},
     ("bwd", "xl2_256px"): {"traffic": 1.2167e+09, "mfma_busy": 0.230, "kernel": "dmf::attn_bwd_fused_bf16_kernel<72>",
-                           "src": ("attn_bwd_bf16.hip", "499e8cb752b49fb2")},
+                           "src": ("attn_bwd_bf16.hip", "03652ae92e25ff31")},
 }
 
 
