@@ -176,8 +176,8 @@ __global__ __launch_bounds__(64 * kSmallWaves, 1) void attn_fwd_small_kernel(con
 #pragma unroll
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, Sc[i]);
     mx = xhalf_max(mx);
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + (kSplitLazyLog2 + kFwdBias<T>)) != 0) {
-      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) - kFwdBias<T> : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
+    if (__builtin_amdgcn_ballot_w64(mx - m_run > kSplitLazyLog2 + kFwdBias<T>) != 0) {
+      const float m_new = fmaxf(m_run, running_max<T>(mx)), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);

@@ -31,11 +31,19 @@ template <typename T> struct SplitType;
 template <> struct SplitType<float> { static constexpr int NI = 3, NWT = 3; static constexpr bool F16 = false; };
 template <> struct SplitType<_Float16> { static constexpr int NI = 1, NWT = 2; static constexpr bool F16 = true; };
 
-// log2 of the factor on P in the f16 kernels: P reaches 2^6 in the forward (kSplitLazyLog2), 1 in the backward, the range 2^16.
+// log2 of the factor on P in the f16 kernels: P reaches 2^6 in the forward (kSplitLazyLog2), the range 2^16; in the backward P reaches 1, and
+// more by what lse is rounded (2^5.8 at scores of 10^8).  Scores from 2^24 on (log2 units), whose last digit is a whole number, go without
+// the factor: it would be rounded to a larger one.
 template <typename T> constexpr float kFwdBias = SplitType<T>::F16 ? 9.f : 0.f;
-template <typename T> constexpr float kBwdBias = SplitType<T>::F16 ? 14.f : 0.f;
+template <typename T> constexpr float kBwdBias = SplitType<T>::F16 ? 10.f : 0.f;
 // What an accumulator of P (its planes' sum: split8) is multiplied by at the end.
 template <typename T> constexpr float kWeightUnit = SplitType<T>::F16 ? 1.f / (1.f + 1.f / 1024.f) : 1.f;
+constexpr float kBiasedScores = 0x1p24f;
+template <typename T>
+__device__ __forceinline__ float running_max(float mx) {   // what is kept of it: a whole number in the f16 kernels, less kFwdBias
+  if constexpr (!SplitType<T>::F16) return mx;
+  return ceilf(mx) - (fabsf(mx) < kBiasedScores ? kFwdBias<T> : 0.f);
+}
 constexpr uint32_t kRowScaleBias = 9;   // and of RowScale's largest value before it is raised: 2^5 times that
 
 template <>
@@ -550,6 +558,11 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
   auto uniform = [](float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); };   // (else in a vector register)
   const float c2 = uniform(p.scale_log2 == 0.f ? 1.f : fabsf(p.scale_log2)), scale = uniform(fabsf(p.scale));
 
+  // The fused product less m leaves m's own rounding error in the exponent, the same for every key of a row: harmless until it leaves the f16
+  // range.  From kBiasedScores on (a wave with such rows takes the branch below for every tile) the scores are rounded like m.
+  uint64_t large = 0;
+  float c2_fma = c2;
+
   const int ntiles = (p.Lkv + 31) / 32;
   commit_k(0);
   if constexpr (!Plan::WIDE) commit_v(0);
@@ -591,9 +604,9 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
 #pragma unroll
     for (int i = 2; i < 16; ++i) mx = fmaxf(mx, S[i]);
     mx = xhalf_max(mx) * c2;
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + (kSplitLazyLog2 + kFwdBias<T>)) != 0) {
+    if ((__builtin_amdgcn_ballot_w64(mx - m_run > kSplitLazyLog2 + kFwdBias<T>) | large) != 0) {
       // (whole numbers in the f16 kernels: alpha is a power of two, and nothing is rounded when kFwdBias is taken off)
-      const float m_new = fmaxf(m_run, F16 ? ceilf(mx) - kFwdBias<T> : mx), drop = m_new - m_run, alpha = fast_exp2(-drop);
+      const float m_new = fmaxf(m_run, running_max<T>(mx)), drop = m_new - m_run, alpha = fast_exp2(-drop);
       m_run = m_new;
       l_run *= alpha;
       O.scale(alpha);
@@ -602,11 +615,16 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
         dO.scale(gs.decay(alpha, drop));
         if constexpr (F16) dOv.scale(alpha);
       }
+      if constexpr (F16) {
+        large = __builtin_amdgcn_ballot_w64(fabsf(m_run) >= kBiasedScores);
+        c2_fma = uniform(large != 0 ? 1.f : c2);
+        if (large != 0) S *= c2;
+      }
     }
     f32x16 E, G;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      E[i] = fast_exp2(fmaf(S[i], c2, -m_run));
+      E[i] = fast_exp2(fmaf(S[i], c2_fma, -m_run));
       l_run += E[i];
       if constexpr (JVP) {
         G[i] = E[i] * (dS[i] * scale);
@@ -850,7 +868,7 @@ __device__ __forceinline__ void split_bwd_dkv_body(const BwdParams& p) {
     if constexpr (ST::N == 1) __syncthreads();
     if (it + 1 < ntiles) commit(it + 1);
   }
-  constexpr float kUnbias = SplitType<T>::F16 ? 1.f / 16384.f : 1.f;   // 2^-kBwdBias
+  constexpr float kUnbias = SplitType<T>::F16 ? 1.f / 1024.f : 1.f;   // 2^-kBwdBias
   store_out<T, D, NW>(smem, static_cast<T*>(p.dk) + base(6), p.st[6][1], k0, p.Lkv, tid, dK, p.scale * kUnbias * gs.inverse());
   store_out<T, D, NW>(smem, static_cast<T*>(p.dv) + base(7), p.st[7][1], k0, p.Lkv, tid, dV, kUnbias * kWeightUnit<T>);
 }

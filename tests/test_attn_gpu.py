@@ -1081,3 +1081,23 @@ def test_softmax_scale_of_any_sign_in_the_split_operand_kernels(scale, dtype, B,
             print(f"{name} L{L} {err:.2e}", flush=True)
             # (a rounded fp16 output next to a nearly one-hot row: its error is what dq and dk consist of there)
             assert err <= tol * (10 if name in ("to", "dq", "dk") and abs(scale) > 1 else 1), (name, L, err)
+
+
+@pytest.mark.parametrize("B,H,L,D", [(1, 2, 100, 64), (1, 2, 256, 72), (160, 2, 260, 64), (16, 16, 512, 72), (65, 4, 257, 72)])
+@pytest.mark.parametrize("magnitude", [1200.0, 3000.0, 4000.0, 5600.0, 11300.0])
+def test_half_scores_of_any_magnitude(magnitude, B, H, L, D):
+    """fp16, scores from 10^7 to 10^9: equal keys are averaged, and where one key stands out its value is the result -- the running maximum has a
+    last digit of 1 to 128 there, and neither its rounding nor the factor on the probabilities may leave the f16 range."""
+    g = torch.Generator(device=DEV).manual_seed(L)
+    q = torch.full((B, L, H, D), magnitude, device=DEV).half()
+    k, v = q.clone(), torch.randn(B, L, H, D, generator=g, device=DEV).half()
+    tq, tk = torch.zeros_like(q), torch.zeros_like(k)
+    for one in (False, True):
+        if one:
+            k[:, : L - 7] *= 0.5   # the last seven weigh everything
+        rows = slice(L - 7, L) if one else slice(0, L)
+        o, _ = _lib.fwd_half(q, k, v, D ** -0.5)
+        o2, to, _ = _lib.fwd_jvp_half(q, k, v, tq, tk, v, D ** -0.5)
+        ref = v[:, rows].double().mean(1, keepdim=True).expand(B, L, H, D)
+        for got in (o, o2, to):   # (fp16 rounding of the result, 21 bits of each probability)
+            assert ao.rel_l2(got.double(), ref) <= 4e-4, (one, ao.rel_l2(got.double(), ref))
