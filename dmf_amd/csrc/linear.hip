@@ -3,10 +3,10 @@
 // travels to HBM and back.
 //
 // The library ran the two products of a layer one after the other (two partly empty last rounds), in tiles that fit these widths
-// badly, and spent 18 us of host time on each.  Here both are one grid; 192 columns divide every layer width of the models, so the
-// 128 x 192 tile fills whole rounds.
+// badly, and spent 18 us of host time on each.  Here both are one grid; 192 columns divide most layer widths of the models.
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 #include "attn_common.h"
 #include "attn_kernels.h"
 #include "../../include/dmf_fused.h"
@@ -191,16 +191,358 @@ static int launch_linear(LinearParams& p, bool jvp, hipStream_t stream) {
   return launch_kernel(kern, dim3((uint32_t)p.mtiles * p.ntiles * (jvp && MODE == kLinPlain ? 2 : 1)), dim3(256), smem, stream, p);
 }
 
-// Tile policy: the shortest of four estimates, a K step (64) and a work-group's start and end taking `a` and `b` (in 10 ns) with one, two,
-// three work-groups on a CU -- fitted to K = 384 .. 4608 on MI355X (us: 128 x 192, 768 columns, 48 steps: 43.6 for 128 work-groups, 47 for 256,
-// 68.4 for 512; 12 steps, 1536 work-groups: 63.9):
-struct LinTile { int bm, bn, per_cu, a[3], b[3]; };
-constexpr LinTile kLinTiles[4] = {
-    {128, 192, 2, {90, 140, 0}, {350, 450, 0}}, {128, 128, 2, {77, 95, 0}, {120, 400, 0}},
-    {128, 64, 3, {61, 63, 93}, {60, 200, 250}}, {64, 64, 2, {20, 36, 0}, {320, 320, 0}}};
+// ---- products with many tiles ------------------------------------------------------------------------------------------------
+//
+// linear_kernel's 128 x 192 tile needs 29 bytes per clock and CU from the L2 at the matrix pipes' pace, which is what it gets: C768 M16384 N 3C
+// (pair) 145 us, 800 TFLOP/s.  Here one work-group of four waves has the CU to itself, one wave per SIMD with 512 registers and MT x NT accumulator
+// tiles: 256 x 192 takes 30 % fewer bytes and a third fewer LDS reads per product.  The work-groups stay and walk through the tiles, so that a
+// tile's first stages arrive during the last ones of the tile before and its stores drain behind the next one's products: 113 us, 1026 TFLOP/s; C768
+// M16384 K 4C 153 -> 125, gelu pair N 4C 195 -> 162; C1152 M8192 N 3C 126 -> 115, K 4C 170 -> 148, gelu pair 176 -> 163.  Without its DMA the loop runs at
+// 1560 TFLOP/s: what is left is the waves' wait at the CU's one address unit, four requests at a time (letting the waves take turns by branches cost
+// more than it gave: 8192 cubed 819 -> 927 us), and a tile's end (3 us of 19 at 12 steps).
+// Stages are 64 contraction elements, whole 128-byte lines (stages of 32 with twice the depth: 8192 x 3 unchanged, but 12 % more time in light
+// grids, where each half line is a request of its own); three of x and two of w fill the LDS, x being the operand that comes from HBM.  Slot v of
+// row r holds vector v ^ r / 2 % 8: 16 rows read at one vector meet all sixteen 16-byte bank groups.  While the products of one 16-deep chunk issue,
+// the operands of the next are read, one LDS read behind each product.
+// Results are stored past the caches (nt): C768 M16384 N 3C 122 -> 117, 256 x 128 tiles 140 -> 116.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N <= 63, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 
-// A gelu pair holds an element of x and its tangent in one wave, BM / 2 rows of each: it has as many work-groups as a single product of twice
-// the rows, and takes the tiles with two row tiles per wave.
+// one element of a product's sums
+__device__ __forceinline__ float sum(float a) {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
+  return v;
+}
+__device__ __forceinline__ void lds_write64(uint32_t addr, u32x2 v) { asm volatile("ds_write_b64 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
+
+// (after a wait: keeps uses of what has been read behind it)
+__device__ __forceinline__ void landed_in(u32x4& v) { asm volatile("" : "+v"(v)); }
+
+template <class F, int... I>
+__device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int MT_, int NT_, int WM_, int NSX_, int NSW_>
+struct WalkTile {
+  static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = 4 / WM, NSX = NSX_, NSW = NSW_, BM = 32 * MT * WM, BN = 32 * NT * WN;
+  static constexpr int XS = BM * 128, WS = BN * 128, LDS = NSX * XS + NSW * WS + 4 * 4096;
+  static constexpr int PX = XS / 4096, PW = WS / 4096, STORES = MT * NT * 2;
+  // requests of a wave that may be in flight behind the stage that is waited for
+  static constexpr int BEHIND = NSX > NSW ? (NSW - 2) * (PX + PW) + PX : (NSW - 2) * (PX + PW);
+  static constexpr int BEFORE = NSX > NSW ? NSW - 2 : NSW - 3;   // last stage of a tile whose last chunk waits for requests from before the stores
+  static_assert(NSW >= 2 && (NSX == NSW || NSX == NSW + 1) && LDS <= 160 * 1024 && MT % 2 == 0 && BEHIND + STORES <= 63);
+  // two accumulator tiles leave together, side by side where the row allows: a pass' tile h (0, 1)
+  static constexpr int row_of(int pass, int h) { return NT == 3 ? 2 * (pass / 3) + (pass % 3 == 2 ? h : pass % 3) : pass / (NT / 2); }
+  static constexpr int col_of(int pass, int h) { return NT == 3 ? (pass % 3 == 2 ? 2 : h) : 2 * (pass % (NT / 2)) + h; }
+};
+
+constexpr int kNonTemporal = 2;   // (buffer instructions' aux bits)
+
+template <class T, int MODE>
+__device__ __forceinline__ void linear_walk(const LinearParams& p) {
+  constexpr int MT = T::MT, NT = T::NT, BM = T::BM, BN = T::BN;
+  constexpr bool BOTH = MODE == kLinGeluJvp;
+  static_assert(!BOTH || MT % 2 == 0, "as many row tiles of x as of tx");
+  constexpr int ROWS = BOTH ? BM / 2 : BM, MX = BOTH ? MT / 2 : MT;   // of y: a tile's rows, a wave's row tiles (WM * 32 rows apart)
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  const uint32_t per = (uint32_t)p.mtiles * p.ntiles, total = MODE == kLinPlain && p.x[1] != nullptr ? 2 * per : per, G = gridDim.x;
+  // The n-th tile of this work-group.  The work-groups of an XCD take neighbours; where the last round has tiles for half of them at most,
+  // every tile of it is two of half the rows.
+  constexpr bool HALVES = !BOTH;
+  constexpr uint32_t END = ~0u;
+  struct Place { int second, m0, n0, rows; };   // rows: of the tile (ROWS, or half of it, or what is left of M; none is possible in the second half)
+  auto nth_tile = [&](uint32_t n) -> uint32_t {   // 4 * tile + (0: whole; 1, 2: a half)
+    if (n * G >= total) return END;
+    const uint32_t left = total - n * G, halves = HALVES && 2 * left <= G, take = left >= G ? G : left << halves;
+    if (blockIdx.x >= take) return END;
+    const uint32_t i = xcd_remap(blockIdx.x, take);
+    return halves ? 4 * (n * G + i / 2) + 1 + i % 2 : 4 * (n * G + i);
+  };
+  // groups of eight row blocks, column blocks within (as linear_kernel)
+  auto place = [&](uint32_t tile) {
+    Place t;
+    uint32_t id = tile >> 2;
+    t.second = id >= per;
+    if (t.second) id -= per;
+    const uint32_t grp = id / (8 * p.ntiles), first = grp * 8, rows_in = min((uint32_t)p.mtiles - first, 8u), in = id - grp * 8 * p.ntiles;
+    t.m0 = (int)(first + in % rows_in) * ROWS + (tile % 4 == 2 ? ROWS / 2 : 0);
+    t.n0 = (int)(in / rows_in) * BN;
+    t.rows = max(0, min(tile % 4 ? ROWS / 2 : ROWS, p.M - t.m0));
+    t.second = __builtin_amdgcn_readfirstlane(t.second);
+    t.m0 = __builtin_amdgcn_readfirstlane(t.m0);
+    t.n0 = __builtin_amdgcn_readfirstlane(t.n0);
+    t.rows = __builtin_amdgcn_readfirstlane(t.rows);
+    return t;
+  };
+
+  const uint32_t kb = (uint32_t)p.K * 2;
+  const int steps = p.K / kLinK;
+  const uint32_t drow = lane >> 3;
+  uint32_t voff[T::PX > T::PW ? T::PX : T::PW];   // rows 32 j + 8 wave on
+#pragma unroll
+  for (int j = 0; j < (T::PX > T::PW ? T::PX : T::PW); ++j)
+    voff[j] = (32 * j + 8 * wave + drow) * kb + (((lane & 7) ^ ((4 * (wave & 1) + (drow >> 1)) & 7)) * 16);
+  // the stages being requested, of x (with tx) and of w: tile, step, slot
+  struct Cursor { uint32_t nth, slot; int step; };
+  Cursor cx{0, 0, 0}, cw{0, 0, 0};
+  __amdgpu_buffer_rsrc_t rx, rtx, rw;
+  auto aim_x = [&](uint32_t id) {
+    const Place t = place(id);
+    rx = make_rows_rsrc(p.x[t.second] + (int64_t)t.m0 * p.K, kb, t.rows, (int)kb);
+    rtx = BOTH ? make_rows_rsrc(p.x[1] + (int64_t)t.m0 * p.K, kb, t.rows, (int)kb) : rx;
+  };
+  auto aim_w = [&](uint32_t id) {
+    const Place t = place(id);
+    rw = make_rows_rsrc(p.w + (int64_t)t.n0 * p.K, kb, min(BN, p.N - t.n0), (int)kb);
+  };
+  auto request_x = [&](int j) {   // a wave's j-th KB of the stage
+    char* dst = smem + cx.slot * T::XS + (4 * j + wave) * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(BOTH && j >= ROWS / 32 ? rtx : rx, (__attribute__((address_space(3))) void*)dst, 16, voff[j % (ROWS / 32)],
+                                             cx.step * 128, 0, 0);
+  };
+  auto request_w = [&](int j) {
+    char* dst = smem + T::NSX * T::XS + cw.slot * T::WS + (4 * j + wave) * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)dst, 16, voff[j], cw.step * 128, 0, 0);
+  };
+  // (past the last tile's last step the requests go on -- bytes of other rows, or zeros -- so that the number in flight is constant; nothing
+  //  reads them, and the kernel's end waits for them)
+  auto advance = [&](Cursor& c, uint32_t ring, auto&& aim) {
+    c.slot = c.slot + 1 == ring ? 0 : c.slot + 1;
+    if (++c.step == steps) {
+      const uint32_t next = nth_tile(c.nth + 1);
+      if (next != END) {
+        ++c.nth;
+        c.step = 0;
+        aim(next);
+      }
+    }
+  };
+
+  // this lane's vector of chunk c in its row of either tile
+  uint32_t xaddr[4], waddr[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t k = ((2 * c + g) ^ ((c32 >> 1) & 7)) * 16;
+    xaddr[c] = lds_addr(smem) + (wm * 32 + c32) * 128 + k;
+    waddr[c] = lds_addr(smem) + T::NSX * T::XS + (wn * 32 * NT + c32) * 128 + k;
+  }
+  u32x4 X[2][MT], W[2][NT];
+  uint32_t xslot = 0, wslot = 0;   // of the stage being read
+  auto read = [&](auto cc, auto ii) {   // operand ii of chunk cc
+    constexpr int c = decltype(cc)::value, i = decltype(ii)::value, b = c & 1;
+    if constexpr (i < NT) W[b][i] = lds_read128_issue<i * 4096>(waddr[c] + wslot * T::WS);
+    else X[b][i - NT] = lds_read128_issue<((i - NT) % MX * 32 * T::WM + (i - NT) / MX * ROWS) * 128>(xaddr[c] + xslot * T::XS);
+  };
+  auto landed = [&](auto bb, auto rows) {
+    constexpr int b = decltype(bb)::value;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NT; ++i) landed_in(W[b][i]);
+#pragma unroll
+    for (int i = 0; i < decltype(rows)::value; ++i) landed_in(X[b][i]);
+  };
+  f32x16 acc[NT][MT];
+
+  // One stage's products.  Between the last chunk's and the next stage's, the emptied slots are requested again: w's at once, x's over the three
+  // chunks that follow (all together the requests queue up in the CU's one address unit, and the waves with them).  `stores`: those of the
+  // tile before may be in flight behind the stage that the last chunk waits for.
+  auto stage = [&](auto first_, auto rows_, bool stores) {
+    constexpr bool FIRST = decltype(first_)::value;
+    constexpr int MA = decltype(rows_)::value;   // row tiles: all, or in half a tile the first half
+    for_each(std::make_integer_sequence<int, 4>{}, [&](auto cc) {
+      constexpr int c = decltype(cc)::value, NEXT = (c + 1) % 4, NM = MA * NT, R = MA + NT;
+      landed(std::integral_constant<int, c & 1>{}, rows_);
+      if constexpr (c == 3) {
+        if (stores) wait_vm<T::BEHIND + T::STORES>();
+        else wait_vm<T::BEHIND>();
+        asm volatile("s_barrier" ::: "memory");   // the next stage is in LDS and everybody has taken its operands of this one
+        xslot = xslot + 1 == T::NSX ? 0 : xslot + 1;
+        wslot = wslot + 1 == T::NSW ? 0 : wslot + 1;
+      }
+      for_each(std::make_integer_sequence<int, NM>{}, [&](auto ii) {
+        constexpr int i = decltype(ii)::value, n = i / MA, m = i % MA;
+        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, W[c & 1][n]), __builtin_bit_cast(bf16x8, X[c & 1][m]),
+                                                            FIRST && c == 0 ? f32x16{0} : acc[n][m], 0, 0, 0);
+        constexpr int SLOTS = NM < R ? NM : R, r0 = i < SLOTS ? i * R / SLOTS : R, r1 = i < SLOTS ? (i + 1) * R / SLOTS : R;
+        for_each(std::make_integer_sequence<int, r1 - r0>{}, [&](auto rr) {
+          read(std::integral_constant<int, NEXT>{}, std::integral_constant<int, r0 + decltype(rr)::value>{});
+        });
+        if constexpr (c == 3) {
+#pragma unroll
+          for (int j = i * T::PW / NM; j < (i + 1) * T::PW / NM; ++j) request_w(j);
+        } else {
+          constexpr int at = c * NM + i;
+#pragma unroll
+          for (int j = at * T::PX / (3 * NM); j < (at + 1) * T::PX / (3 * NM); ++j) request_x(j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (c == 3) advance(cw, T::NSW, aim_w);
+      if constexpr (c == 2) advance(cx, T::NSX, aim_x);
+    });
+  };
+
+  aim_x(nth_tile(0));
+  aim_w(nth_tile(0));
+#pragma unroll
+  for (int s = 0; s < T::NSW; ++s) {
+#pragma unroll
+    for (int j = 0; j < T::PW; ++j) request_w(j);
+    advance(cw, T::NSW, aim_w);
+    if (s < T::NSX - 1) {
+#pragma unroll
+      for (int j = 0; j < T::PX; ++j) request_x(j);
+      advance(cx, T::NSX, aim_x);
+    }
+  }
+  wait_vm<(T::NSW - 1) * T::PW + (T::NSX - 2) * T::PX>();
+  asm volatile("s_barrier" ::: "memory");
+  for_each(std::make_integer_sequence<int, MT + NT>{}, [&](auto ii) { read(std::integral_constant<int, 0>{}, ii); });
+
+  // Output rows leave two accumulator tiles at a time through this wave's 4 KB of LDS (32 rows of 128 bytes, slot v of row r holding vector
+  // v ^ r / 2 % 8), in whole 16-byte vectors; while one pass is on its way through LDS the next one is computed.
+  const uint32_t nb = (uint32_t)p.N * 2;
+  const uint32_t own = lds_addr(smem) + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
+  const uint32_t put = own + c32 * 128 + ((c32 >> 1) & 7) * 16 + g * 8;
+  const uint32_t get = own + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 4)) * 16);   // rows + 8 i: slot ^ 4 i % 8
+  const int half = (lane >> 2) & 1;
+  auto finish = [&](uint32_t id, auto rows_) {
+    constexpr int MA = decltype(rows_)::value;
+    const Place at = place(id);
+    // bias of columns 8 v + 4 g .. + 3: wave-uniform vectors of eight by scalar loads (vector loads would wait for the DMA in flight)
+    typedef const __attribute__((address_space(4))) uint32_t* ScalarPtr;
+    const bool biased = p.bias != nullptr && !at.second;
+    const __bf16* bias = biased ? p.bias : p.w;   // (something readable)
+    const uint32_t keep = biased ? ~0u : 0u;
+    u32x2 braw[NT * 4];
+    for_each(std::make_integer_sequence<int, NT * 4>{}, [&](auto vv) {
+      constexpr int v = decltype(vv)::value;
+      const ScalarPtr s = (ScalarPtr)(uintptr_t)(bias + min(at.n0 + wn * 32 * NT + v * 8, p.N - 8));
+      uint32_t w0 = s[0], w1 = s[1], w2 = s[2], w3 = s[3];
+      asm("" : "+s"(w0), "+s"(w1), "+s"(w2), "+s"(w3));   // (or the selection is made of addresses, and the loads are vector loads)
+      braw[v] = u32x2{(g ? w2 : w0) & keep, (g ? w3 : w1) & keep};
+    });
+    // (sums are taken out of their registers one quad at a time: left to itself the compiler copies all of them at once, and spills; the wait
+    //  states between the last product and the first of these reads are written out, as it does not look into assembly)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+    const int ncols = min(BN, p.N - at.n0);
+    __amdgpu_buffer_rsrc_t ry[2];
+    for (int h = 0; h < (BOTH ? 2 : 1); ++h)
+      ry[h] = make_rows_rsrc(p.y[BOTH ? h : at.second] + (int64_t)at.m0 * p.N + at.n0, nb, at.rows, at.rows > 0 ? ncols * 2 : (int)nb);
+    constexpr int PASSES = MA * NT / 2;   // with tangents: of x, then of tx, by turns
+    u32x4 out[2][4];
+    auto pass_row = [](int pass, int h) constexpr { return T::row_of(BOTH ? pass / 2 : pass, h) + (BOTH && pass % 2 ? MX : 0); };
+    auto pass_col = [](int pass, int h) constexpr { return T::col_of(BOTH ? pass / 2 : pass, h); };
+    auto store = [&](auto pp) {
+      constexpr int pass = decltype(pp)::value, m0 = pass_row(pass, 0), m1 = pass_row(pass, 1), n0 = pass_col(pass, 0), n1 = pass_col(pass, 1);
+      static_assert(m0 / MX == m1 / MX, "both of x, or both of tx");
+      const int col = (wn * NT + (half ? n1 : n0)) * 32 + (lane & 3) * 8, row = ((half ? m1 % MX : m0 % MX) * T::WM + wm) * 32 + (lane >> 3);
+      const uint32_t off = (row * nb + col * 2) | (col < ncols ? 0u : 0x80000000u);   // (past the end: dropped)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        landed_in(out[pass & 1][i]);
+        __builtin_amdgcn_raw_buffer_store_b128(out[pass & 1][i], ry[m0 / MX], off, 8 * i * nb, kNonTemporal);
+      }
+    };
+    float slope[BOTH ? 2 : 1][16];   // d gelu of the pass' elements, for their tangents
+    for_each(std::make_integer_sequence<int, PASSES>{}, [&](auto pp) {
+      constexpr int pass = decltype(pp)::value;
+      for_each(std::make_integer_sequence<int, 8>{}, [&](auto vv) {
+        constexpr int v = decltype(vv)::value, h = v / 4, m = pass_row(pass, h), n = pass_col(pass, h), q = v % 4;
+        const u32x2 raw = braw[4 * n + q];
+        const float bb[4] = {__uint_as_float(raw[0] << 16), __uint_as_float(raw[0] & 0xffff0000u), __uint_as_float(raw[1] << 16),
+                             __uint_as_float(raw[1] & 0xffff0000u)};
+        float o[4];
+        for_each(std::make_integer_sequence<int, 4>{}, [&](auto ee) {
+          constexpr int e = decltype(ee)::value;
+          o[e] = sum(acc[n][m][4 * q + e]);
+          if constexpr (BOTH && pass % 2) {
+            o[e] *= slope[h][4 * q + e];
+          } else {
+            o[e] += bb[e];
+            if constexpr (MODE != kLinPlain) {
+              const float x = o[e], sg = gelu_sigma(x);
+              o[e] = x * sg;
+              if constexpr (BOTH) slope[h][4 * q + e] = sg * fmaf(x * (1.f - sg), 1.5957691216057308f * fmaf(3.f * 0.044715f, x * x, 1.f), 1.f);
+            }
+          }
+        });
+        lds_write64(put ^ (v * 16), u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (pass > 0) {
+        asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");   // (what was read before these writes)
+        store(std::integral_constant<int, pass - 1>{});
+      }
+      for_each(std::make_integer_sequence<int, 4>{}, [&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        out[pass & 1][i] = lds_read128_issue<i * 1024>(i & 1 ? get ^ 64 : get);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    store(std::integral_constant<int, PASSES - 1>{});
+    asm volatile("s_nop 1" ::: "memory");   // (before assembly may write these registers again)
+  };
+
+  using Whole = std::integral_constant<int, MT>;
+  using Half = std::integral_constant<int, MT / 2>;
+  for (uint32_t n = 0;; ++n) {
+    const uint32_t id = nth_tile(n);
+    if (id == END) break;
+    const bool stores = n > 0 && T::BEFORE >= 0;
+    if (!HALVES || id % 4 == 0) {
+      stage(std::true_type{}, Whole{}, stores);
+      for (int t = 1; t < steps; ++t) stage(std::false_type{}, Whole{}, stores && t <= T::BEFORE);
+      finish(id, Whole{});
+    } else {
+      if constexpr (HALVES) {
+        stage(std::true_type{}, Half{}, stores);
+        for (int t = 1; t < steps; ++t) stage(std::false_type{}, Half{}, stores && t <= T::BEFORE);
+        finish(id, Half{});
+      }
+    }
+  }
+  wait_vm<0>();   // (no DMA may outlive the work-group's LDS)
+}
+
+template <class T, int MODE>
+__global__ __launch_bounds__(256, 1) void linear_walk_kernel(const LinearParams p) {
+  linear_walk<T, MODE>(p);
+}
+
+template <class T, int MODE>
+static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
+  constexpr int rows = MODE == kLinGeluJvp ? T::BM / 2 : T::BM;
+  auto kern = linear_walk_kernel<T, MODE>;
+  static bool lds_ok[64] = {};
+  if (!ensure_dynamic_lds(kern, T::LDS, lds_ok)) return -7;
+  p.mtiles = (p.M + rows - 1) / rows;
+  p.ntiles = (p.N + T::BN - 1) / T::BN;
+  const int64_t tiles = (int64_t)p.mtiles * p.ntiles * (jvp && MODE == kLinPlain ? 2 : 1);
+  const int64_t cus = compute_units(), grid = tiles >= cus ? cus : MODE != kLinGeluJvp && 2 * tiles <= cus ? 2 * tiles : tiles;
+  return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
+}
+
+// Tile policy: the shortest of the estimates, in 10 ns, of five kernels.  Fitted to 268 products of the models' widths (384, 768, 1024, 1152), 512
+// to 32768 rows, single and in pairs, with and without gelu; standard error 8 to 11 %, and the tile taken is within 1 % of the fastest one in the
+// mean.  linear_kernel: a K step (64) and a work-group's start and end with one, two, three work-groups on a CU; linear_walk_kernel: a step of a
+// whole and of half a tile, a tile's end, and the launch's.
+struct LinTile { int bm, bn, per_cu, a[3], b[3]; };
+constexpr LinTile kLinTiles[3] = {{128, 192, 2, {76, 121, 0}, {508, 750, 0}}, {128, 64, 3, {50, 60, 85}, {337, 437, 340}}, {64, 64, 2, {15, 37, 0}, {480, 170, 0}}};
+struct LinWalk { int bm, bn, a, b, a_half, b_half, launch; };
+constexpr LinWalk kLinWalks[2] = {{256, 192, 100, 700, 52, 540, 40}, {256, 128, 76, 460, 43, 430, 80}};
+
+// A gelu pair holds an element of x and its tangent in one wave, half of the rows of each: it has as many work-groups as a single product of twice
+// the rows, takes the tiles with two row tiles per wave, and whole ones.
 static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
   const int64_t cus = compute_units(), steps = K / kLinK;
   const bool both = jvp && gelu;
@@ -210,7 +552,13 @@ static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
   }
   int best = 0;
   int64_t cost_best = INT64_MAX;
-  for (int t = 0; t < (both ? 3 : 4); ++t) {
+  auto take = [&](int tile, int64_t cost) {
+    if (cost < cost_best) {
+      cost_best = cost;
+      best = tile;
+    }
+  };
+  for (int t = 0; t < (both ? 2 : 3); ++t) {
     const LinTile& c = kLinTiles[t];
     const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * (jvp ? 2 : 1), slots = cus * c.per_cu, rest = wgs % slots;
     auto full = [&](int64_t occ) { return c.a[occ] * steps + c.b[occ]; };
@@ -218,11 +566,14 @@ static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
       const int64_t o = (n + cus - 1) / cus - 1, over = n - o * cus;
       return o == 0 || over == cus ? full(o) : full(o - 1) + (full(o) - full(o - 1)) * (35 * cus + 65 * over) / (100 * cus);
     };
-    const int64_t cost = wgs / slots * round(slots) + (rest ? round(rest) : 0);
-    if (cost < cost_best) {
-      cost_best = cost;
-      best = t;
-    }
+    take(t, wgs / slots * round(slots) + (rest ? round(rest) : 0));
+  }
+  // (the walking kernel's row offsets within a tile are 32-bit)
+  for (int t = 0; t < 2 && N <= 65536 && K <= 65536; ++t) {
+    const LinWalk& c = kLinWalks[t];
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * (jvp ? 2 : 1), rest = tiles % cus;
+    const bool half = !both && 2 * rest <= cus;
+    take(3 + t, c.launch + tiles / cus * (c.a * steps + c.b) + (rest == 0 ? 0 : half ? c.a_half * steps + c.b_half : c.a * steps + c.b));
   }
   return best;
 }
@@ -231,8 +582,9 @@ template <int MODE>
 static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t stream) {
   switch (tile) {
     case 0: return launch_linear<128, 192, 2, MODE>(p, jvp, stream);
-    case 1: return launch_linear<128, 128, 2, MODE>(p, jvp, stream);
-    case 2: return launch_linear<128, 64, 2, MODE>(p, jvp, stream);
+    case 1: return launch_linear<128, 64, 2, MODE>(p, jvp, stream);
+    case 3: return launch_walk<WalkTile<4, 3, 2, 3, 2>, MODE>(p, jvp, stream);
+    case 4: return launch_walk<WalkTile<4, 2, 2, 3, 3>, MODE>(p, jvp, stream);
     default: break;
   }
   if constexpr (MODE == kLinGeluJvp) return DMF_ATTN_ESHAPE;   // (linear_tile does not answer this)
@@ -241,21 +593,24 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
 
 }  // namespace dmf
 
-// Which calls this kernel is the faster one for (us, library -> here; C: model width, M rows):
-//   pairs: C768 M16384 N 3C 133 -> 120, N C 48 -> 43, K 4C 130 -> 130; C1152 M8192 158 -> 124, 64 -> 47, N 4C 171 -> 161, K 4C 166 -> 160;
-//     M4096 82 -> 69, 40 -> 26, 114 -> 82, 94 -> 80;
-//   single: C768 M2048 N 3C 16.4 -> 13.1, M4096 N 3C 19.9 -> 20.5, N C 12.0 -> 9.4, gelu N 4C 29.5 -> 26.0; C1152 M8192 N 3C 79 -> 70;
-//   the library keeps single products with few columns for their depth (K 4C: M4096 C768 26.9 against 31.3, C1152 48 against 56), pairs
-//   that spread a short K over a large result (N 4C M16384: C768 141 against 155, C1152 296 against 317; C768 with gelu 86 against 90)
-//   and outputs narrower than a tile;
+// Which calls these kernels are the faster ones for (us, library -> here; C: model width, M rows):
+//   pairs: C768 M16384 N 3C 137 -> 113, N C 48 -> 40, K 4C 129 -> 125; C1152 M8192 161 -> 115, 65 -> 43, N 4C 169 -> 149, K 4C 167 -> 148;
+//     M4096 84 -> 66, 40 -> 24, K 4C 98 -> 73;
+//   single: C768 M2048 N 3C 20 -> 12.3, M4096 N 3C 20.8 -> 19.1; C1152 M8192 N 3C 83 -> 63, K 4C 80 -> 75, M16384 K 4C 157 -> 148;
+//     K 4C: M1024 C768 22 -> 13, M2048 C768 20.7 -> 19.6 (C384 22.7 -> 8.1), M8192 C768 37.3 -> 36.9;
+//   the library keeps single products with few columns for their depth between two and four million results (K 4C: M3000 C768 24.2 against 27.0,
+//   M4096 26.2 against 27.3, M2048 C1152 31.9 against 37.2), those that spread a short K over a large result (N 4C M16384: C768 pairs 137 against
+//   144, 32768 rows 130 against 136 single), rows of 2 or 8 KB on large results (C1024: M16384 K 4C 183 against 234, N C 60 against 63,
+//   M8192 N 4C 106 against 122) and outputs narrower than a tile;
 //   pairs with gelu (library pair and activation kernel; this kernel's pair and the activation kernel -> here), N 4C, wins from one row up:
 //     M16 C384 10.4; 7.7 -> 5.3, C768 11.3; 8.1 -> 7.1, C1152 12.7; 9.2 -> 8.9;  M512 C768 23.4; 15.5 -> 10.6, C1152 34.0; 24.1 -> 18.3;
-//     M4096 C768 61.7; 58.2 -> 44.1, C1152 131; 104 -> 85;  M8192 C384 63.8; 43.6 -> 30.1, C1024 152; 182 -> 142, C1152 212; 212 -> 169.
+//     M4096 C768 61.7; 58.2 -> 40.3, C1152 131; 104 -> 80;  M8192 C384 63.8; 43.6 -> 30.1, C1024 152; 182 -> 142, C1152 212; 212 -> 163.
 extern "C" int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu) {
   if (M < 1 || N < 64 || N % 8 || K < 64 || K % 64 || M * K > (int64_t)1 << 30 || (int64_t)N * K > (int64_t)1 << 30 || M * N > (int64_t)1 << 30) return 0;
   if (jvp && gelu) return 1;
-  if (!jvp && K >= 2 * N) return 0;
-  if (M * N > 40000000 && N > 3 * K && (jvp || K < 1024)) return 0;
+  if (!jvp && K >= 2 * N && K > 2048 && M * N > 2000000 && M * N < 4000000) return 0;
+  if (K >= 1024 && (K & (K - 1)) == 0 && (M >= 16384 || (N >= 4 * K && M >= 4096))) return 0;
+  if (M * N > 40000000 && N > 3 * K && N > 2048 && (jvp || K < 1024)) return 0;
   return 1;
 }
 

@@ -137,3 +137,25 @@ def test_weight_gradient_refuses():
     assert call(p, q, o, 0, 64, 64) == -3 and call(p, q, o, 64, 60, 64) == -3 and call(p, q, o, 64, 64, 12) == -3
     assert call(None, q, o, 64, 64, 64) == -5 and call(p + 2, q, o, 64, 64, 64) == -6
     assert lib.dmf_linear_wgrad_workspace_floats(64, 60, 64) == -1
+
+
+# the kernel whose work-groups walk through the tiles (256 x 192, 256 x 128; with tangents and gelu 128 rows of each): whole rounds and half
+# tiles behind them, only half tiles, a row and a column block that fill neither, one step per tile and fewer steps than stages; outputs whole
+WALK = [(2049, 2296, 768), (8193, 1152, 1152), (4100, 1016, 1024), (12345, 1016, 192), (16384, 2304, 64), (2300, 3064, 448)]
+
+
+@pytest.mark.parametrize("M,N,K", WALK)
+def test_products_of_many_tiles(M, N, K):
+    x, tx, w, b = _operands(M, N, K)
+    ref, tref = torch.nn.functional.linear(x.float(), w.float(), b.float()), tx.float() @ w.float().t()
+    gelu = lambda t: torch.nn.functional.gelu(t, approximate="tanh")
+    for _ in range(2):   # (a second launch finds its work-groups' LDS as the first left it)
+        _check(_call(x, None, w, None, 0)[0], ref - b.float())
+        y, ty = _call(x, tx, w, b, 0)
+        _check(y, ref)
+        _check(ty, tref)
+    act, tact = torch.func.jvp(gelu, (ref.double(),), (tref.double(),))
+    _check(_call(x, None, w, b, 1)[0], act)
+    y, ty = _call(x, tx, w, b, 1)
+    _check(y, act)
+    _check(ty, tact)
