@@ -204,6 +204,9 @@ static int launch_linear(LinearParams& p, bool jvp, hipStream_t stream) {
 // grids, where each half line is a request of its own); three of x and two of w fill the LDS, x being the operand that comes from HBM.  Slot v of
 // row r holds vector v ^ r / 2 % 8: 16 rows read at one vector meet all sixteen 16-byte bank groups.  While the products of one 16-deep chunk issue,
 // the operands of the next are read, one LDS read behind each product.
+// 128 x 96, one row tile per wave: products of at most 256 such tiles, deep or flat, filled half of the CUs or took the 64 x 64 kernel's bytes.  Five stages
+// of both operands; its LDS is what bounds it (a step writes 28 KB and reads 64, W once per wave: 736 clocks of 768 with few work-groups, 920 with 256):
+// C768 M4096 K 4C library 26.5 -> 24.0 us, K C 10.7 -> 9.5; C1152 M2048 K 4C 31.9 -> 28.6, K C 13.1 -> 10.9; C768 M1024 N 3C 10.2 -> 9.0.
 // Results are stored past the caches (nt): C768 M16384 N 3C 122 -> 117, 256 x 128 tiles 140 -> 116.
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -231,14 +234,16 @@ template <int MT_, int NT_, int WM_, int NSX_, int NSW_>
 struct WalkTile {
   static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = 4 / WM, NSX = NSX_, NSW = NSW_, BM = 32 * MT * WM, BN = 32 * NT * WN;
   static constexpr int XS = BM * 128, WS = BN * 128, LDS = NSX * XS + NSW * WS + 4 * 4096;
-  static constexpr int PX = XS / 4096, PW = WS / 4096, STORES = MT * NT * 2;
+  static constexpr int PX = XS / 4096, PW = WS / 4096, STORES = (MT * NT + 1) / 2 * 4;
+  // chunks whose operands are read ahead: with one row tile the products of one chunk are too short to hide its reads
+  static constexpr int AHEAD = MT == 1 ? 2 : 1, LAST = 3 - AHEAD;   // LAST: the chunk before the one that changes stages
   // requests of a wave that may be in flight behind the stage that is waited for
   static constexpr int BEHIND = NSX > NSW ? (NSW - 2) * (PX + PW) + PX : (NSW - 2) * (PX + PW);
   static constexpr int BEFORE = NSX > NSW ? NSW - 2 : NSW - 3;   // last stage of a tile whose last chunk waits for requests from before the stores
-  static_assert(NSW >= 2 && (NSX == NSW || NSX == NSW + 1) && LDS <= 160 * 1024 && MT % 2 == 0 && BEHIND + STORES <= 63);
+  static_assert(NSW >= 2 && (NSX == NSW || NSX == NSW + 1) && LDS <= 160 * 1024 && (MT % 2 == 0 || MT == 1 && NT == 3) && BEHIND + STORES <= 63);
   // two accumulator tiles leave together, side by side where the row allows: a pass' tile h (0, 1)
-  static constexpr int row_of(int pass, int h) { return NT == 3 ? 2 * (pass / 3) + (pass % 3 == 2 ? h : pass % 3) : pass / (NT / 2); }
-  static constexpr int col_of(int pass, int h) { return NT == 3 ? (pass % 3 == 2 ? 2 : h) : 2 * (pass % (NT / 2)) + h; }
+  static constexpr int row_of(int pass, int h) { return MT == 1 ? 0 : NT == 3 ? 2 * (pass / 3) + (pass % 3 == 2 ? h : pass % 3) : pass / (NT / 2); }
+  static constexpr int col_of(int pass, int h) { return MT == 1 ? 2 * pass + h : NT == 3 ? (pass % 3 == 2 ? 2 : h) : 2 * (pass % (NT / 2)) + h; }
 };
 
 constexpr int kNonTemporal = 2;   // (buffer instructions' aux bits)
@@ -255,7 +260,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   const uint32_t per = (uint32_t)p.mtiles * p.ntiles, total = MODE == kLinPlain && p.x[1] != nullptr ? 2 * per : per, G = gridDim.x;
   // The n-th tile of this work-group.  The work-groups of an XCD take neighbours; where the last round has tiles for half of them at most,
   // every tile of it is two of half the rows.
-  constexpr bool HALVES = !BOTH;
+  constexpr bool HALVES = !BOTH && MT % 2 == 0;
   constexpr uint32_t END = ~0u;
   struct Place { int second, m0, n0, rows; };   // rows: of the tile (ROWS, or half of it, or what is left of M; none is possible in the second half)
   auto nth_tile = [&](uint32_t n) -> uint32_t {   // 4 * tile + (0: whole; 1, 2: a half)
@@ -333,16 +338,18 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     xaddr[c] = lds_addr(smem) + (wm * 32 + c32) * 128 + k;
     waddr[c] = lds_addr(smem) + T::NSX * T::XS + (wn * 32 * NT + c32) * 128 + k;
   }
-  u32x4 X[2][MT], W[2][NT];
+  constexpr int AHEAD = T::AHEAD, BUFS = 2 * AHEAD;
+  u32x4 X[BUFS][MT], W[BUFS][NT];
   uint32_t xslot = 0, wslot = 0;   // of the stage being read
   auto read = [&](auto cc, auto ii) {   // operand ii of chunk cc
-    constexpr int c = decltype(cc)::value, i = decltype(ii)::value, b = c & 1;
+    constexpr int c = decltype(cc)::value, i = decltype(ii)::value, b = c % BUFS;
     if constexpr (i < NT) W[b][i] = lds_read128_issue<i * 4096>(waddr[c] + wslot * T::WS);
     else X[b][i - NT] = lds_read128_issue<((i - NT) % MX * 32 * T::WM + (i - NT) / MX * ROWS) * 128>(xaddr[c] + xslot * T::XS);
   };
-  auto landed = [&](auto bb, auto rows) {
-    constexpr int b = decltype(bb)::value;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  auto landed = [&](auto cc, auto rows) {   // chunk cc's operands; where stages change, all that are read
+    constexpr int c = decltype(cc)::value, b = c % BUFS;
+    if constexpr (AHEAD == 1 || c == T::LAST + 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MT + NT) : "memory");
 #pragma unroll
     for (int i = 0; i < NT; ++i) landed_in(W[b][i]);
 #pragma unroll
@@ -357,9 +364,9 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     constexpr bool FIRST = decltype(first_)::value;
     constexpr int MA = decltype(rows_)::value;   // row tiles: all, or in half a tile the first half
     for_each(std::make_integer_sequence<int, 4>{}, [&](auto cc) {
-      constexpr int c = decltype(cc)::value, NEXT = (c + 1) % 4, NM = MA * NT, R = MA + NT;
-      landed(std::integral_constant<int, c & 1>{}, rows_);
-      if constexpr (c == 3) {
+      constexpr int c = decltype(cc)::value, NEXT = (c + AHEAD) % 4, NM = MA * NT, R = MA + NT, CHANGE = T::LAST + 1;
+      landed(cc, rows_);
+      if constexpr (c == CHANGE) {
         if (stores) wait_vm<T::BEHIND + T::STORES>();
         else wait_vm<T::BEHIND>();
         asm volatile("s_barrier" ::: "memory");   // the next stage is in LDS and everybody has taken its operands of this one
@@ -368,24 +375,24 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       }
       for_each(std::make_integer_sequence<int, NM>{}, [&](auto ii) {
         constexpr int i = decltype(ii)::value, n = i / MA, m = i % MA;
-        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, W[c & 1][n]), __builtin_bit_cast(bf16x8, X[c & 1][m]),
+        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, W[c % BUFS][n]), __builtin_bit_cast(bf16x8, X[c % BUFS][m]),
                                                             FIRST && c == 0 ? f32x16{0} : acc[n][m], 0, 0, 0);
         constexpr int SLOTS = NM < R ? NM : R, r0 = i < SLOTS ? i * R / SLOTS : R, r1 = i < SLOTS ? (i + 1) * R / SLOTS : R;
         for_each(std::make_integer_sequence<int, r1 - r0>{}, [&](auto rr) {
           read(std::integral_constant<int, NEXT>{}, std::integral_constant<int, r0 + decltype(rr)::value>{});
         });
-        if constexpr (c == 3) {
+        if constexpr (c == CHANGE) {
 #pragma unroll
           for (int j = i * T::PW / NM; j < (i + 1) * T::PW / NM; ++j) request_w(j);
         } else {
-          constexpr int at = c * NM + i;
+          constexpr int at = (c + 3 - CHANGE) % 4 * NM + i;
 #pragma unroll
           for (int j = at * T::PX / (3 * NM); j < (at + 1) * T::PX / (3 * NM); ++j) request_x(j);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
-      if constexpr (c == 3) advance(cw, T::NSW, aim_w);
-      if constexpr (c == 2) advance(cx, T::NSX, aim_x);
+      if constexpr (c == CHANGE) advance(cw, T::NSW, aim_w);
+      if constexpr (c == T::LAST) advance(cx, T::NSX, aim_x);
     });
   };
 
@@ -405,6 +412,11 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   wait_vm<(T::NSW - 1) * T::PW + (T::NSX - 2) * T::PX>();
   asm volatile("s_barrier" ::: "memory");
   for_each(std::make_integer_sequence<int, MT + NT>{}, [&](auto ii) { read(std::integral_constant<int, 0>{}, ii); });
+  if constexpr (AHEAD == 2) {   // (what the chunk before would have read and requested)
+    for_each(std::make_integer_sequence<int, MT + NT>{}, [&](auto ii) { read(std::integral_constant<int, 1>{}, ii); });
+#pragma unroll
+    for (int j = 0; j < T::PX / 3; ++j) request_x(j);
+  }
 
   // Output rows leave two accumulator tiles at a time through this wave's 4 KB of LDS (32 rows of 128 bytes, slot v of row r holding vector
   // v ^ r / 2 % 8), in whole 16-byte vectors; while one pass is on its way through LDS the next one is computed.
@@ -437,15 +449,15 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     __amdgpu_buffer_rsrc_t ry[2];
     for (int h = 0; h < (BOTH ? 2 : 1); ++h)
       ry[h] = make_rows_rsrc(p.y[BOTH ? h : at.second] + (int64_t)at.m0 * p.N + at.n0, nb, at.rows, at.rows > 0 ? ncols * 2 : (int)nb);
-    constexpr int PASSES = MA * NT / 2;   // with tangents: of x, then of tx, by turns
+    constexpr int PASSES = (MA * NT + 1) / 2;   // with tangents: of x, then of tx, by turns
     u32x4 out[2][4];
     auto pass_row = [](int pass, int h) constexpr { return T::row_of(BOTH ? pass / 2 : pass, h) + (BOTH && pass % 2 ? MX : 0); };
     auto pass_col = [](int pass, int h) constexpr { return T::col_of(BOTH ? pass / 2 : pass, h); };
     auto store = [&](auto pp) {
       constexpr int pass = decltype(pp)::value, m0 = pass_row(pass, 0), m1 = pass_row(pass, 1), n0 = pass_col(pass, 0), n1 = pass_col(pass, 1);
       static_assert(m0 / MX == m1 / MX, "both of x, or both of tx");
-      const int col = (wn * NT + (half ? n1 : n0)) * 32 + (lane & 3) * 8, row = ((half ? m1 % MX : m0 % MX) * T::WM + wm) * 32 + (lane >> 3);
-      const uint32_t off = (row * nb + col * 2) | (col < ncols ? 0u : 0x80000000u);   // (past the end: dropped)
+      const int tile = half ? n1 : n0, col = (wn * NT + tile) * 32 + (lane & 3) * 8, row = ((half ? m1 % MX : m0 % MX) * T::WM + wm) * 32 + (lane >> 3);
+      const uint32_t off = (row * nb + col * 2) | (col < ncols && tile < NT ? 0u : 0x80000000u);   // (past the end: dropped)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         landed_in(out[pass & 1][i]);
@@ -455,7 +467,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     float slope[BOTH ? 2 : 1][16];   // d gelu of the pass' elements, for their tangents
     for_each(std::make_integer_sequence<int, PASSES>{}, [&](auto pp) {
       constexpr int pass = decltype(pp)::value;
-      for_each(std::make_integer_sequence<int, 8>{}, [&](auto vv) {
+      for_each(std::make_integer_sequence<int, pass_col(pass, 1) < NT ? 8 : 4>{}, [&](auto vv) {   // (a last tile by itself: half the rows' bytes)
         constexpr int v = decltype(vv)::value, h = v / 4, m = pass_row(pass, h), n = pass_col(pass, h), q = v % 4;
         const u32x2 raw = braw[4 * n + q];
         const float bb[4] = {__uint_as_float(raw[0] << 16), __uint_as_float(raw[0] & 0xffff0000u), __uint_as_float(raw[1] << 16),
@@ -479,7 +491,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
         __builtin_amdgcn_sched_barrier(0);
       });
       if constexpr (pass > 0) {
-        asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");   // (what was read before these writes)
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(pass_col(pass, 1) < NT ? 8 : 4) : "memory");   // (what was read before these writes)
         store(std::integral_constant<int, pass - 1>{});
       }
       for_each(std::make_integer_sequence<int, 4>{}, [&](auto ii) {
@@ -494,7 +506,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   };
 
   using Whole = std::integral_constant<int, MT>;
-  using Half = std::integral_constant<int, MT / 2>;
+  using Half = std::integral_constant<int, HALVES ? MT / 2 : MT>;
   for (uint32_t n = 0;; ++n) {
     const uint32_t id = nth_tile(n);
     if (id == END) break;
@@ -528,13 +540,13 @@ static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
   p.mtiles = (p.M + rows - 1) / rows;
   p.ntiles = (p.N + T::BN - 1) / T::BN;
   const int64_t tiles = (int64_t)p.mtiles * p.ntiles * (jvp && MODE == kLinPlain ? 2 : 1);
-  const int64_t cus = compute_units(), grid = tiles >= cus ? cus : MODE != kLinGeluJvp && 2 * tiles <= cus ? 2 * tiles : tiles;
+  const int64_t cus = compute_units(), grid = tiles >= cus ? cus : MODE != kLinGeluJvp && T::MT % 2 == 0 && 2 * tiles <= cus ? 2 * tiles : tiles;
   return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
 }
 
-// Tile policy: the shortest of the estimates, in 10 ns, of five kernels.  Fitted to 268 products of the models' widths (384, 768, 1024, 1152), 512
+// Tile policy: the shortest of the estimates, in 10 ns, of six kernels.  Fitted to 268 products of the models' widths (384, 768, 1024, 1152), 512
 // to 32768 rows, single and in pairs, with and without gelu; standard error 8 to 11 %, and the tile taken is within 1 % of the fastest one in the
-// mean.  linear_kernel: a K step (64) and a work-group's start and end with one, two, three work-groups on a CU; linear_walk_kernel: a step of a
+// mean.  (Refitted for the 128 x 96 tile alone, 110 products of which it takes 20.)  linear_kernel: a K step (64) and a work-group's start and end with one, two, three work-groups on a CU; linear_walk_kernel: a step of a
 // whole and of half a tile, a tile's end, and the launch's.
 struct LinTile { int bm, bn, per_cu, a[3], b[3]; };
 constexpr LinTile kLinTiles[3] = {{128, 192, 2, {76, 121, 0}, {508, 750, 0}}, {128, 64, 3, {50, 60, 85}, {337, 437, 340}}, {64, 64, 2, {15, 37, 0}, {480, 170, 0}}};
@@ -568,6 +580,11 @@ static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
     };
     take(t, wgs / slots * round(slots) + (rest ? round(rest) : 0));
   }
+  // 128 x 96, where all tiles run at once: an L2 shared by more than half of the CUs lengthens the step
+  if (!both && N <= 65536 && K <= 65536) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 95) / 96) * (jvp ? 2 : 1);
+    if (tiles <= cus) take(5, 480 + (30 * cus + 20 * std::max<int64_t>(0, tiles - cus / 2)) * steps / cus);
+  }
   // (the walking kernel's row offsets within a tile are 32-bit)
   for (int t = 0; t < 2 && N <= 65536 && K <= 65536; ++t) {
     const LinWalk& c = kLinWalks[t];
@@ -585,6 +602,9 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
     case 1: return launch_linear<128, 64, 2, MODE>(p, jvp, stream);
     case 3: return launch_walk<WalkTile<4, 3, 2, 3, 2>, MODE>(p, jvp, stream);
     case 4: return launch_walk<WalkTile<4, 2, 2, 3, 3>, MODE>(p, jvp, stream);
+    case 5:
+      if constexpr (MODE != kLinGeluJvp) return launch_walk<WalkTile<1, 3, 4, 5, 5>, MODE>(p, jvp, stream);
+      break;
     default: break;
   }
   if constexpr (MODE == kLinGeluJvp) return DMF_ATTN_ESHAPE;   // (linear_tile does not answer this)
@@ -597,9 +617,10 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
 //   pairs: C768 M16384 N 3C 137 -> 113, N C 48 -> 40, K 4C 129 -> 125; C1152 M8192 161 -> 115, 65 -> 43, N 4C 169 -> 149, K 4C 167 -> 148;
 //     M4096 84 -> 66, 40 -> 24, K 4C 98 -> 73;
 //   single: C768 M2048 N 3C 20 -> 12.3, M4096 N 3C 20.8 -> 19.1; C1152 M8192 N 3C 83 -> 63, K 4C 80 -> 75, M16384 K 4C 157 -> 148;
-//     K 4C: M1024 C768 22 -> 13, M2048 C768 20.7 -> 19.6 (C384 22.7 -> 8.1), M8192 C768 37.3 -> 36.9;
-//   the library keeps single products with few columns for their depth between two and four million results (K 4C: M3000 C768 24.2 against 27.0,
-//   M4096 26.2 against 27.3, M2048 C1152 31.9 against 37.2), those that spread a short K over a large result (N 4C M16384: C768 pairs 137 against
+//     K 4C: M1024 C768 22 -> 13, M2048 C768 20.7 -> 19.6 (C384 22.7 -> 8.1), M3000 C768 23.7 -> 21.2, M4096 C768 26.5 -> 24.0,
+//     M2048 C1152 32.0 -> 28.6, M8192 C768 37.3 -> 36.9;
+//   the library keeps single products with few columns for their depth up to four million results where the 128 x 96 tiles need a second round
+//   (K 4C: C768 M4500 28.3 against 29.1, M5000 30.4 against 35.7; C1024 M3072 30.0 against 31.7), those that spread a short K over a large result (N 4C M16384: C768 pairs 137 against
 //   144, 32768 rows 130 against 136 single), rows of 2 or 8 KB on large results (C1024: M16384 K 4C 183 against 234, N C 60 against 63,
 //   M8192 N 4C 106 against 122) and outputs narrower than a tile;
 //   pairs with gelu (library pair and activation kernel; this kernel's pair and the activation kernel -> here), N 4C, wins from one row up:
@@ -608,7 +629,7 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
 extern "C" int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu) {
   if (M < 1 || N < 64 || N % 8 || K < 64 || K % 64 || M * K > (int64_t)1 << 30 || (int64_t)N * K > (int64_t)1 << 30 || M * N > (int64_t)1 << 30) return 0;
   if (jvp && gelu) return 1;
-  if (!jvp && K >= 2 * N && K > 2048 && M * N > 2000000 && M * N < 4000000) return 0;
+  if (!jvp && K >= 2 * N && K > 2048 && M * N > 2000000 && M * N < 4000000 && ((M + 127) / 128) * ((N + 95) / 96) > dmf::compute_units()) return 0;
   if (K >= 1024 && (K & (K - 1)) == 0 && (M >= 16384 || (N >= 4 * K && M >= 4096))) return 0;
   if (M * N > 40000000 && N > 3 * K && N > 2048 && (jvp || K < 1024)) return 0;
   return 1;

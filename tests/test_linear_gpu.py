@@ -159,3 +159,22 @@ def test_products_of_many_tiles(M, N, K):
     y, ty = _call(x, tx, w, b, 1)
     _check(y, act)
     _check(ty, tact)
+
+
+# the same kernel's 128 x 96 tiles, up to one per CU: a row past a tile, a last column block of 8 and of 88 columns, fewer steps than stages' ring
+# and many; single products, and pairs of half the rows
+ONE_ROUND = [(2433, 776, 448), (2561, 1144, 576), (1025, 2296, 448), (2047, 1528, 768), (897, 3064, 768), (4096, 768, 3072)]
+
+
+@pytest.mark.parametrize("M,N,K", ONE_ROUND)
+def test_products_of_one_round(M, N, K):
+    x, tx, w, b = _operands(M, N, K)
+    ref, tref = torch.nn.functional.linear(x.float(), w.float(), b.float()), tx.float() @ w.float().t()
+    half = M // 2 + 1
+    for _ in range(2):
+        _check(_call(x, None, w, b, 0)[0], ref)
+        y, ty = _call(x[:half], tx[:half], w, b, 0)
+        _check(y, ref[:half])
+        _check(ty, tref[:half])
+    act = torch.nn.functional.gelu(ref, approximate="tanh")
+    assert (_call(x, None, w, b, 1)[0].float() - act).norm() <= TOL * act.norm()
