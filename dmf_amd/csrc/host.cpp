@@ -1019,6 +1019,58 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
   return out;
 }
 
+// ---- a block ---------------------------------------------------------------------------------------------------------------
+
+// weight, bias and their low-precision copies
+using Layer = std::tuple<Tensor, OptTensor, OptTensor, OptTensor>;
+
+// The operators of a transformer block in the order of DiTBlock.forward_chained, as one call: each is the function above, or where that
+// declines the package's general route, so that nothing is computed twice.  DMFT-B/2's four-step sampling loop of 8 images: 5.30 -> 4.24 ms of
+// host time (22 us a block), which now runs ahead of the kernels: 6.04 -> 5.92 ms in all.
+py::object block(const Tensor& x, const Tensor& z, const Tensor& gate_msa, const Tensor& shift, const Tensor& scale, const Tensor& gate_mlp,
+                 const Tensor& next_shift, const Tensor& next_scale, double eps, double next_eps, int64_t heads, const Layer& qkv, const Layer& proj,
+                 const Layer& fc1, const Layer& fc2, const OptTensor& q_gain, const OptTensor& k_gain, double qk_eps) {
+  if (current_level() == kUnsupported) return none();
+  const auto ops = [](const char* name) { return py::module_::import("dmf_amd.block_ops").attr(name); };
+  const auto project = [&](const py::object& in, const Layer& l) {
+    const auto& [w, b, w_lp, b_lp] = l;
+    const Tensor t = in.cast<Tensor>();
+    py::object out = linear(t, w, b, w_lp, b_lp);
+    return out.is_none() ? py::object(ops("dual_linear")(t, w, b, w_lp, b_lp)) : out;
+  };
+  const auto attend = [&](const py::object& in) {
+    py::object out = q_gain ? none() : attention_packed(in.cast<Tensor>(), heads, std::nullopt);
+    if (!out.is_none()) return out;
+    const py::object op = py::module_::import("dmf_amd.flash_attention_hip_jvp").attr("flash_attn_projection");
+    return q_gain ? op(in, heads, *q_gain, *k_gain, qk_eps) : op(in, heads);
+  };
+  const auto residual = [&](const Tensor& x, const Tensor& gate, const py::object& in, const Tensor& shift, const Tensor& scale, double eps) {
+    const Tensor h = in.cast<Tensor>();
+    py::object out = residual_ln_modulate(x, gate, h, shift, scale, eps);
+    if (out.is_none()) out = ops("residual_ln_modulate")(x, gate, h, shift, scale, eps);
+    return py::tuple(std::move(out));
+  };
+  const auto mlp_in = [&](const py::object& in) {   // (as block_ops.linear_gelu_tanh)
+    const auto& [w, b, w_lp, b_lp] = fc1;
+    const bool grad = c10::GradMode::is_enabled();
+    if (b && !(grad && w.requires_grad())) {
+      py::object out = linear_gelu(in.cast<Tensor>(), w, *b, w_lp, b_lp);
+      if (!out.is_none()) return out;
+    }
+    if (b && !grad) return py::object(ops("linear_gelu_tanh")(in, w, *b, w_lp, b_lp));
+    const py::object h = project(in, fc1);
+    py::object out = activation(h.cast<Tensor>(), Act::gelu);
+    return out.is_none() ? py::object(ops("gelu_tanh")(h)) : out;
+  };
+  py::object h = project(py::cast(z), qkv);
+  h = attend(h);
+  h = project(h, proj);
+  const py::tuple mid = residual(x, gate_msa, h, shift, scale, eps);
+  h = mlp_in(mid[1]);
+  h = project(h, fc2);
+  return residual(mid[0].cast<Tensor>(), gate_mlp, h, next_shift, next_scale, next_eps);
+}
+
 // ---- adaLN modulations ---------------------------------------------------------------------------------------------------
 
 // A (B, 1, C) column block of a dense (B, n) region of `whole`, without the dispatcher.
@@ -1131,4 +1183,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("linear_gelu", &linear_gelu);
   m.def("chunk_last", &chunk_last);
   m.def("modulations", &modulations);
+  m.def("block", &block);
 }

@@ -244,6 +244,23 @@ class DiTBlock(nn.Module):
         x = x + gate_mlp * self.mlp(modulate(self.norm2(x), shift_mlp, scale_mlp))
         return x
 
+    def _one_call(self, x: Tensor, z: Tensor):
+        """What the native host path needs to run the block in one call: heads, the four linear layers' tensors, the q / k norms.  None
+        where a module on the way is not this file's own, has a hook or a replaced forward, or anything watches the calls."""
+        if not _lib.native(x, z) or torch.nn.modules.module._has_any_global_hook():
+            return None
+        attn, mlp = self.attn, self.mlp
+        if not (_quiet(attn, Attention) and attn.packed and _quiet(mlp, Mlp)):
+            return None
+        linears = (attn.qkv, attn.proj, mlp.fc1, mlp.fc2)
+        if not all(_quiet(m, Linear) and m.fused for m in linears):
+            return None
+        tensors = [(m.weight, m.bias, m.lp_weight, m.lp_bias) for m in linears]
+        norms = (attn.q_norm.scale, attn.k_norm.scale, attn.q_norm.eps) if attn.qk_norm else (None, None, 0.0)
+        if torch.overrides.has_torch_function([t for layer in tensors for t in layer] + list(norms[:2])):
+            return None
+        return attn.num_heads, *tensors, *norms
+
     def forward_chained(self, x: Tensor, z: Tensor, mods, next_shift: Tensor, next_scale: Tensor, next_eps: float):
         """Fused-mode variant for a stack of blocks.  ``z`` is this block's already
         normalised and modulated input (``modulate(norm1(x), shift_msa, scale_msa)``,
@@ -253,6 +270,11 @@ class DiTBlock(nn.Module):
         block's msa pair, or the final layer's).  Returns ``(x_out, z_next)``; same
         values as ``forward``."""
         _, _, gate_msa, shift_mlp, scale_mlp, gate_mlp = mods
+        layers = self._one_call(x, z)
+        if layers is not None:
+            out = _lib.host().block(x, z, gate_msa, shift_mlp, scale_mlp, gate_mlp, next_shift, next_scale, self.norm2.eps, next_eps, *layers)
+            if out is not None:
+                return out
         x, z = fused.residual_ln_modulate(x, gate_msa, self.attn(z), shift_mlp, scale_mlp, self.norm2.eps)
         return fused.residual_ln_modulate(x, gate_mlp, self.mlp(z), next_shift, next_scale, next_eps)
 
@@ -276,6 +298,12 @@ class FinalLayer(nn.Module):
         if self.fused:
             return self.linear(fused.ln_modulate(x, shift, scale, self.norm_final.eps))
         return self.linear(modulate(self.norm_final(x), shift, scale))
+
+
+def _quiet(module: nn.Module, cls: type) -> bool:
+    """Calling the module is calling ``cls.forward``: no subclass, no replaced method, no hook of any direction."""
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks))
 
 
 def _plain(module: nn.Module, cls: type) -> bool:

@@ -369,3 +369,56 @@ def test_stacked_modulations_leave_to_the_blocks():
         handle.remove()
     blk.requires_grad_(False), final.requires_grad_(False)
     assert tries(c) == [True] and tries(c.requires_grad_()) == [False]
+
+
+@pytest.mark.parametrize("dtype,qk_norm,autocast", [(torch.float32, False, True), (torch.float32, True, True), (torch.float32, True, False),
+                                                   (torch.bfloat16, False, False)])
+def test_block_in_one_call(dtype, qk_norm, autocast):
+    """A block as one native call and as its modules one by one: the same bits in every way it is differentiated, with frozen weights too."""
+    torch.manual_seed(3)
+    blk = DiTBlock(128, 2, qk_norm=qk_norm, attn_func="hip", block_ops="hip").to(DEV, dtype)
+    rnd = lambda *s: torch.randn(*s, device=DEV).to(dtype)
+    x, z, mods, nxt = rnd(2, 24, 128), rnd(2, 24, 128), [rnd(2, 1, 128) for _ in range(6)], [rnd(2, 1, 128) for _ in range(2)]
+    params = list(blk.parameters())[:-2]   # (the modulation's own layer is not part of it)
+
+    def every_mode():
+        call = lambda x, z, *m: blk.forward_chained(x, z, m, *nxt, 1e-6)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            with torch.no_grad():
+                outs = [*call(x, z, *mods)]
+            leaves = [t.clone().requires_grad_() for t in (x, z, *mods)]
+            y = call(*leaves)
+            for weights in (True, False):
+                blk.requires_grad_(weights)
+                y, ty = torch.func.jvp(call, tuple(leaves), tuple(t.detach().flip(-1) for t in leaves))
+                outs += [*y, *ty]
+                grads = torch.autograd.grad([t.float().square().sum() for t in y], leaves + (params if weights else []), allow_unused=True)
+                outs += [g for g in grads if g is not None]
+            blk.requires_grad_(True)
+        return outs
+
+    layers, one_call = [], DiTBlock._one_call
+    try:
+        DiTBlock._one_call = lambda self, *a: layers.append(one_call(self, *a)) or layers[-1]
+        got = every_mode()
+        assert len(layers) == 4 and all(l is not None for l in layers)
+        DiTBlock._one_call = lambda self, *a: None
+        ref = every_mode()
+    finally:
+        DiTBlock._one_call = one_call
+    assert len(got) == len(ref) and all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+def test_block_with_hooks_or_replaced_parts_is_not_one_call():
+    blk = DiTBlock(128, 2, attn_func="hip", block_ops="hip").to(DEV)
+    x = torch.randn(2, 24, 128, device=DEV)
+    assert blk._one_call(x, x) is not None
+    for module in (blk.attn, blk.attn.qkv, blk.attn.proj, blk.mlp, blk.mlp.fc1, blk.mlp.fc2):
+        for hook in (module.register_forward_hook, module.register_forward_pre_hook, module.register_full_backward_hook):
+            handle = hook(lambda *a: None)
+            assert blk._one_call(x, x) is None
+            handle.remove()
+        module.forward = type(module).forward.__get__(module)
+        assert blk._one_call(x, x) is None
+        del module.forward
+    assert blk._one_call(x, x) is not None
