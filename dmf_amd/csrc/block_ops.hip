@@ -621,6 +621,48 @@ __global__ __launch_bounds__(kThreads) void act_kernel(ActParams p) {
   if (MODE) store8(p.ty, MODE == 2 ? p.xbf : p.ybf, v * 8, d);
 }
 
+// ---- timestep embedding --------------------------------------------------------------------------------------------
+// One thread per time and frequency.  A few KB: what it takes is the launch (2.5 us), and it stands for eleven of them, and for some
+// thirty with tangents.
+
+struct TimestepParams {
+  const void *t, *tt;
+  void *y, *ty;
+  int64_t total;   // times * (frequencies, and one more where dim is odd: the zero)
+  int dim, bf;
+  float neg_log_period;
+};
+
+__device__ __forceinline__ float load1(const void* p, int bf, int64_t i) {
+  return bf ? __uint_as_float((uint32_t)static_cast<const uint16_t*>(p)[i] << 16) : static_cast<const float*>(p)[i];
+}
+__device__ __forceinline__ void store1(void* p, int bf, int64_t i, float v) {
+  if (bf) static_cast<uint16_t*>(p)[i] = static_cast<uint16_t>(pack_bf16x2(v, 0.f));
+  else static_cast<float*>(p)[i] = v;
+}
+
+__global__ __launch_bounds__(kThreads) void timestep_embedding_kernel(TimestepParams p) {
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (id >= p.total) return;
+  const int half = p.dim / 2, cols = p.dim - half;
+  const int64_t row = id / cols, at = row * p.dim;
+  const int i = static_cast<int>(id - row * cols);
+  if (i == half) {
+    store1(p.y, p.bf, at + 2 * half, 0.f);
+    if (p.ty) store1(p.ty, p.bf, at + 2 * half, 0.f);
+    return;
+  }
+  const float f = expf(p.neg_log_period * static_cast<float>(i) / static_cast<float>(half)), a = load1(p.t, p.bf, row) * f;
+  const float c = cosf(a), s = sinf(a);
+  store1(p.y, p.bf, at + i, c);
+  store1(p.y, p.bf, at + half + i, s);
+  if (p.ty) {
+    const float da = load1(p.tt, p.bf, row) * f;
+    store1(p.ty, p.bf, at + i, -s * da);
+    store1(p.ty, p.bf, at + half + i, c * da);
+  }
+}
+
 // ---- per-head RMS norm --------------------------------------------------------------------------------------------
 // A 16-lane group owns one (b, l, h) row (lane i of the group holds elements 8i..8i+7, lanes past D/8 idle), so a
 // wave covers 4 rows and a work-group 16.
@@ -1069,6 +1111,17 @@ int dmf_silu_fwd(const void* x, const void* tx, void* y, void* ty, int64_t n, in
 
 int dmf_silu_bwd(const void* gy, const void* x, void* gx, int64_t n, int x_dtype, int gy_dtype, void* stream) {
   return act_impl<kActSilu>(x, gy, nullptr, gx, n, x_dtype, gy_dtype, 2, stream);
+}
+
+int dmf_timestep_embedding_fwd(const void* t, const void* tt, void* y, void* ty, int64_t n, int dim, float neg_log_period,
+                               int dtype, void* stream) {
+  if (!dtype_ok(dtype)) return DMF_ATTN_EDTYPE;
+  if (n < 1 || dim < 2 || dim > 65536 || n > (int64_t)1 << 30) return DMF_ATTN_ESHAPE;
+  if (!t || !y || (ty && !tt)) return DMF_ATTN_ENULL;
+  TimestepParams p{t, tt, y, ty, n * (dim - dim / 2), dim, dtype == DMF_ATTN_BF16, neg_log_period};
+  const int64_t blocks = (p.total + kThreads - 1) / kThreads;
+  if (blocks > 0x7fffffffLL) return DMF_ATTN_ESHAPE;
+  return launch_kernel(timestep_embedding_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, static_cast<hipStream_t>(stream), p);
 }
 
 int dmf_colsum(const void* x, void* out, float* workspace, int64_t rows, int C, int x_dtype, int out_dtype,

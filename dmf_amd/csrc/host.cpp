@@ -778,6 +778,30 @@ py::object activation(const Tensor& x_, Act act) {
   return py::cast(finish(y, ty, node, level));
 }
 
+// layers.timestep_embedding in the type of `t`, of which nothing asks for a gradient
+py::object timestep_embedding(const Tensor& t_, int64_t dim, double max_period) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg t = unpack(t_);
+  // (the zero of an odd width: refused by the expressions for anything but a vector)
+  if (!plain_gpu(t) || !block_dtype(t.data) || t.data.numel() == 0 || t.data.numel() > (int64_t)1 << 30 || dim < 2 || dim > 65536 ||
+      (dim % 2 && t.data.dim() != 1) || any_grad(t) || only_tangents_want(t))
+    return none();
+  c10::OptionalDeviceGuard device(t.data.device());
+  Tensor y, ty;
+  {
+    Below below;
+    const Tensor td = dense(t.data), tt = dense(t.tan);
+    auto sizes = td.sizes().vec();
+    sizes.push_back(dim);
+    y = empty(sizes, td.scalar_type(), td);
+    if (tt.defined()) ty = empty(sizes, td.scalar_type(), td);
+    check(dmf_timestep_embedding_fwd(ptr(td), ptr(tt), mptr(y), mptr(ty), td.numel(), (int)dim, (float)-std::log(max_period), code_of(td), stream_of(td)),
+          "dmf_timestep_embedding_fwd");
+  }
+  return py::cast(finish(y, ty, nullptr, level));
+}
+
 // ---- linear --------------------------------------------------------------------------------------------------------------
 
 // One extra stream per device for the weight-gradient half of a layer's backward (the one dmf_amd._lib.side_stream hands out).
@@ -1184,4 +1208,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("chunk_last", &chunk_last);
   m.def("modulations", &modulations);
   m.def("block", &block);
+  m.def("timestep_embedding", &timestep_embedding);
 }

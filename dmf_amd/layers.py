@@ -144,12 +144,18 @@ def timestep_embedding(t: Tensor, dim: int, max_period: int = 10000) -> Tensor:
 class TimestepEmbedder(nn.Module):
     """Reference models/layers.py:59-71."""
 
-    def __init__(self, hidden_size: int, emb_size: int = 256):
+    def __init__(self, hidden_size: int, emb_size: int = 256, block_ops: str = "torch"):
         super().__init__()
         self.emb_size = emb_size
-        self.mlp = nn.Sequential(nn.Linear(emb_size, hidden_size), nn.SiLU(), nn.Linear(hidden_size, hidden_size))
+        self.fused = _check_block_ops(block_ops)
+        self.mlp = nn.Sequential(Linear(emb_size, hidden_size, block_ops=block_ops), SiLU(block_ops),
+                                 Linear(hidden_size, hidden_size, block_ops=block_ops))
 
     def forward(self, t: Tensor) -> Tensor:
+        if self.fused and _lib.native(t):   # embedding and cast in one launch
+            emb = _lib.host().timestep_embedding(t, self.emb_size, 10000.0)
+            if emb is not None:
+                return self.mlp(emb)
         return self.mlp(timestep_embedding(t, self.emb_size).to(t.dtype))
 
 

@@ -5,6 +5,8 @@ Tolerances (relative L2): 1e-5 when everything is fp32; 6e-3 when the result is
 stored in bf16 (one rounding of an fp32 result, 2^-9 relative per element, so
 about 2.3e-3 in L2).  The oracle is always evaluated in fp32 on the values the
 kernel was given (bf16 inputs are rounded first, then widened)."""
+import math
+
 import pytest
 import torch
 
@@ -367,3 +369,35 @@ def test_linear_gelu_tanh_epilogue_path(mode):
     assert ao.rel_l2(tyd.float().cpu(), t_ref) <= tol
     y2.float().sum().backward()
     assert w.grad is not None and float(w.grad.abs().max()) > 0
+
+
+@pytest.mark.parametrize("shape,dim", [((1,), 2), ((1,), 256), ((64,), 256), ((15,), 7), ((3, 5), 64), ((333,), 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_timestep_embedding(shape, dim, dtype):
+    """One launch against the reference's expressions in fp64.  fp32: an exponential, a product and a sine or cosine of an angle up to
+    4, each good to 2 ulp, so 8 2^-23 of the angle (of the tangent's factor) in all; bf16: its rounding on top."""
+    from dmf_amd import _lib
+    from dmf_amd.layers import timestep_embedding
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    t, tt = ((torch.rand(*shape, generator=g, device=DEV) * 4).to(dtype) for _ in range(2))
+    half = dim // 2
+    f = torch.exp(-math.log(10000) * torch.arange(half, device=DEV, dtype=torch.float64) / half)
+    a, da = t.double()[..., None] * f, tt.double()[..., None] * f
+    pad = lambda *parts: torch.nn.functional.pad(torch.cat(parts, -1), (0, dim % 2))
+    ref, tref = pad(a.cos(), a.sin()), pad(-a.sin() * da, a.cos() * da)
+    embed = lambda t: _lib.host().timestep_embedding(t, dim, 10000.0)
+    y, ty = torch.func.jvp(embed, (t,), (tt,))
+    rel = 2 ** -8 if dtype == torch.bfloat16 else 0
+    assert y.dtype == dtype and torch.equal(embed(t), y)
+    assert ((y - ref).abs() <= 32 * 2 ** -23 + rel * ref.abs()).all()
+    assert ((ty - tref).abs() <= 4 * 32 * 2 ** -23 + rel * tref.abs()).all()
+    if dtype == torch.float32:
+        assert (y - timestep_embedding(t, dim)).abs().max() <= 32 * 2 ** -23
+    assert _lib.host().timestep_embedding(t.detach().requires_grad_(), dim, 10000.0) is None
+
+
+def test_timestep_embedding_refuses():
+    from dmf_amd import _lib
+    call, p = _lib.load().dmf_timestep_embedding_fwd, torch.zeros(8, device=DEV).data_ptr()
+    assert call(p, None, p, None, 1, 1, 0.0, 0, None) == -3 and call(p, None, p, None, 0, 4, 0.0, 0, None) == -3
+    assert call(p, None, p, p, 1, 4, 0.0, 0, None) == -5 and call(None, None, p, None, 1, 4, 0.0, 0, None) == -5
