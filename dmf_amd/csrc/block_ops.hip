@@ -621,6 +621,34 @@ __global__ __launch_bounds__(kThreads) void act_kernel(ActParams p) {
   if (MODE) store8(p.ty, MODE == 2 ? p.xbf : p.ybf, v * 8, d);
 }
 
+// ---- fp32 -> bf16 --------------------------------------------------------------------------------------------------
+// Eight elements per thread; the arrays follow each other in the grid.  A cast of its own for each of weight, bias, rows and their
+// tangents cost 4.5 us at least, back to back: 23 launches fewer in a four-block XL/2-width training step, 8.02 -> 7.83 ms.
+
+struct CastParams {
+  const float* src[4];
+  uint16_t* dst[4];
+  int64_t end[4];   // in threads, running
+};
+
+__global__ __launch_bounds__(kThreads) void cast_bf16_kernel(CastParams p) {
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (id >= p.end[3]) return;
+  const float* src = p.src[0];
+  uint16_t* dst = p.dst[0];
+  int64_t first = 0;
+#pragma unroll
+  for (int k = 1; k < 4; ++k)
+    if (id >= p.end[k - 1]) {
+      src = p.src[k];
+      dst = p.dst[k];
+      first = p.end[k - 1];
+    }
+  float v[8];
+  load8(src, 0, (id - first) * 8, v);
+  store8(dst, 1, (id - first) * 8, v);
+}
+
 // ---- timestep embedding --------------------------------------------------------------------------------------------
 // One thread per time and frequency.  A few KB: what it takes is the launch (2.5 us), and it stands for eleven of them, and for some
 // thirty with tangents.
@@ -1111,6 +1139,27 @@ int dmf_silu_fwd(const void* x, const void* tx, void* y, void* ty, int64_t n, in
 
 int dmf_silu_bwd(const void* gy, const void* x, void* gx, int64_t n, int x_dtype, int gy_dtype, void* stream) {
   return act_impl<kActSilu>(x, gy, nullptr, gx, n, x_dtype, gy_dtype, 2, stream);
+}
+
+int dmf_cast_bf16(const void* const* src, void* const* dst, const int64_t* n, int count, void* stream) {
+  if (!src || !dst || !n) return DMF_ATTN_ENULL;
+  if (count < 1 || count > 4) return DMF_ATTN_ESHAPE;
+  CastParams p{};
+  int64_t total = 0;
+  for (int k = 0; k < 4; ++k) {
+    if (k < count) {
+      if (n[k] < 8 || n[k] % 8 || n[k] > (int64_t)1 << 36) return DMF_ATTN_ESHAPE;
+      if (!src[k] || !dst[k]) return DMF_ATTN_ENULL;
+      if (!aligned16(src[k]) || !aligned16(dst[k])) return DMF_ATTN_EALIGN;
+      p.src[k] = static_cast<const float*>(src[k]);
+      p.dst[k] = static_cast<uint16_t*>(dst[k]);
+      total += n[k] / 8;
+    }
+    p.end[k] = total;
+  }
+  const int64_t blocks = (total + kThreads - 1) / kThreads;
+  if (blocks > 0x7fffffffLL) return DMF_ATTN_ESHAPE;
+  return launch_kernel(cast_bf16_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, static_cast<hipStream_t>(stream), p);
 }
 
 int dmf_timestep_embedding_fwd(const void* t, const void* tt, void* y, void* ty, int64_t n, int dim, float neg_log_period,

@@ -891,13 +891,37 @@ variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w
   return {gx, gw, gb};
 }
 
+// The casts in front of a product: those that are fp32 -> bf16 of dense arrays are one launch, made by run().
+struct Casts {
+  const void* src[4];
+  void* dst[4];
+  int64_t n[4];
+  int count = 0;
+  Tensor like;
+  Tensor add(const Tensor& t, at::ScalarType dt) {
+    if (t.scalar_type() == dt) return t;
+    if (dt != at::kBFloat16 || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.numel() < 8 || t.numel() % 8 ||
+        reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 || count == 4 || (like.defined() && like.device() != t.device()))
+      return t.to(dt);
+    like = empty(t.sizes(), dt, t);
+    src[count] = ptr(t);
+    dst[count] = mptr(like);
+    n[count++] = t.numel();
+    return like;
+  }
+  void run() const {
+    if (count) check(dmf_cast_bf16(src, dst, n, count, stream_of(like)), "dmf_cast_bf16");
+  }
+};
+
 struct LinearOperands {
   Tensor w, b;
   at::ScalarType dt;
   bool ok = false;
 };
 // (autocast state is read by the caller: a Below guard hides it)
-LinearOperands linear_operands(bool autocast, at::ScalarType dt, const Arg& weight, const Arg& bias, const OptTensor& w_lp, const OptTensor& b_lp) {
+LinearOperands linear_operands(bool autocast, at::ScalarType dt, const Arg& weight, const Arg& bias, const OptTensor& w_lp, const OptTensor& b_lp,
+                               Casts& casts) {
   LinearOperands o;
   o.dt = dt;
   if (o.dt != at::kFloat && o.dt != at::kBFloat16) return o;
@@ -907,8 +931,8 @@ LinearOperands linear_operands(bool autocast, at::ScalarType dt, const Arg& weig
     o.b = bias.data;
   } else {
     const bool cached = w_lp && w_lp->defined() && w_lp->scalar_type() == o.dt;
-    o.w = cached ? data_of(unwrap(*w_lp)) : weight.data.to(o.dt);
-    if (bias.defined()) o.b = cached && b_lp && b_lp->defined() ? data_of(unwrap(*b_lp)) : bias.data.to(o.dt);
+    o.w = cached ? data_of(unwrap(*w_lp)) : casts.add(weight.data, o.dt);
+    if (bias.defined()) o.b = cached && b_lp && b_lp->defined() ? data_of(unwrap(*b_lp)) : casts.add(bias.data, o.dt);
   }
   o.ok = true;
   return o;
@@ -950,12 +974,14 @@ py::object linear(const Tensor& x_, const Tensor& weight_, const OptTensor& bias
   const at::ScalarType dt = autocast_type(x.data);
   {
     Below below;
-    o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp);
+    Casts casts;
+    o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp, casts);
     if (!o.ok) return none();
     const int64_t K = x.data.size(-1);
     auto sizes = x.data.sizes().vec();
     sizes.back() = o.w.size(0);
-    const Tensor x2 = x.data.reshape({-1, K}).to(o.dt), tx2 = x.tan.defined() ? x.tan.reshape({-1, K}).to(o.dt) : Tensor();
+    const Tensor x2 = casts.add(x.data.reshape({-1, K}), o.dt), tx2 = x.tan.defined() ? casts.add(x.tan.reshape({-1, K}), o.dt) : Tensor();
+    casts.run();
     if (!own_linear(x2, tx2, o.w, o.b, false, y, ty)) {
       y = o.b.defined() ? at::addmm(o.b, x2, o.w.t()) : at::mm(x2, o.w.t());
       if (tx2.defined()) ty = at::mm(tx2, o.w.t());
@@ -989,12 +1015,14 @@ py::object linear_gelu(const Tensor& x_, const Tensor& weight_, const Tensor& bi
   Tensor y, ty;
   {
     Below below;
-    const LinearOperands o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp);
+    Casts casts;
+    const LinearOperands o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp, casts);
     if (!o.ok) return none();
     const int64_t K = x.data.size(-1);
     auto sizes = x.data.sizes().vec();
     sizes.back() = o.w.size(0);
-    const Tensor x2 = x.data.reshape({-1, K}).to(o.dt), tx2 = x.tan.defined() ? x.tan.reshape({-1, K}).to(o.dt) : Tensor();
+    const Tensor x2 = casts.add(x.data.reshape({-1, K}), o.dt), tx2 = x.tan.defined() ? casts.add(x.tan.reshape({-1, K}), o.dt) : Tensor();
+    casts.run();
     if (!own_linear(x2, tx2, o.w, o.b, true, y, ty)) {
       if (tx2.defined()) return none();
       y = at::_addmm_activation(o.b, x2, o.w.t(), 1, 1, true);

@@ -141,6 +141,12 @@ DMF_ATTN_API int dmf_silu_bwd(const void* gy, const void* x, void* gx, int64_t n
                               void* stream);
 
 /*
+ * dst[k] = src[k] rounded to bf16 (nearest, ties to even), k < count <= 4: dense fp32 arrays of n[k] elements, a multiple of 8.
+ * The casts of a linear layer's operands under autocast.
+ */
+DMF_ATTN_API int dmf_cast_bf16(const void* const* src, void* const* dst, const int64_t* n, int count, void* stream);
+
+/*
  * Sinusoidal embedding of n times: y[b] = [cos(t[b] f) | sin(t[b] f)] over the frequencies f[i] = exp(neg_log_period i / (dim / 2)),
  * i < dim / 2, a zero behind them where dim is odd, and when `ty` is given its tangent, [-sin(t f) f tt | cos(t f) f tt].
  * Replaces timestep_embedding (models/layers.py:46-55) and the cast behind it (:71).  t, tt: (n) of dtype; y, ty: (n, dim) of dtype;

@@ -401,3 +401,19 @@ def test_timestep_embedding_refuses():
     call, p = _lib.load().dmf_timestep_embedding_fwd, torch.zeros(8, device=DEV).data_ptr()
     assert call(p, None, p, None, 1, 1, 0.0, 0, None) == -3 and call(p, None, p, None, 0, 4, 0.0, 0, None) == -3
     assert call(p, None, p, p, 1, 4, 0.0, 0, None) == -5 and call(None, None, p, None, 1, 4, 0.0, 0, None) == -5
+
+
+@pytest.mark.parametrize("sizes", [(8,), (2048,), (2056, 8), (8, 4096, 24, 2040), (1152 * 64, 1152)])
+def test_cast_to_bf16(sizes):
+    """Arrays behind each other in one launch: the bits of torch's casts, nothing written past an end."""
+    import ctypes
+    from dmf_amd import _lib
+    src = [torch.randn(n, device=DEV) * 10.0 ** (i - 1) for i, n in enumerate(sizes)]
+    src[0][:6] = torch.tensor([float("inf"), -float("inf"), 0.0, -0.0, 3.4e38, 1e-40], device=DEV)
+    dst = [torch.full((n + 8,), 7.0, device=DEV, dtype=torch.bfloat16) for n in sizes]
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    call = lambda count, n: _lib.load().dmf_cast_bf16(ptrs(src), ptrs(dst), (ctypes.c_int64 * len(n))(*n), count, torch.cuda.current_stream().cuda_stream)
+    assert call(len(sizes), sizes) == 0
+    for s, d in zip(src, dst):
+        assert torch.equal(d[:-8].view(torch.int16), s.bfloat16().view(torch.int16)) and (d[-8:] == 7.0).all()
+    assert call(1, [12]) == -3 and call(5, sizes) == -3 and call(0, sizes) == -3
