@@ -783,8 +783,8 @@ py::object timestep_embedding(const Tensor& t_, int64_t dim, double max_period) 
   const int64_t level = current_level();
   if (level == kUnsupported) return none();
   const Arg t = unpack(t_);
-  // (the zero of an odd width: refused by the expressions for anything but a vector)
-  if (!plain_gpu(t) || !block_dtype(t.data) || t.data.numel() == 0 || t.data.numel() > (int64_t)1 << 30 || dim < 2 || dim > 65536 ||
+  // (a single time has a row of its own in the expressions; the zero of an odd width: refused by them for anything but a vector)
+  if (t.data.dim() == 0 || !plain_gpu(t) || !block_dtype(t.data) || t.data.numel() == 0 || t.data.numel() > (int64_t)1 << 30 || dim < 2 || dim > 65536 ||
       (dim % 2 && t.data.dim() != 1) || any_grad(t) || only_tangents_want(t))
     return none();
   c10::OptionalDeviceGuard device(t.data.device());

@@ -396,6 +396,14 @@ def test_timestep_embedding(shape, dim, dtype):
     assert _lib.host().timestep_embedding(t.detach().requires_grad_(), dim, 10000.0) is None
 
 
+def test_timestep_embedder_of_a_single_time():
+    """A time without a dimension is a row, as in the expressions, with the native path as without it."""
+    from dmf_amd.layers import TimestepEmbedder
+    emb, t = TimestepEmbedder(128, block_ops="hip").to(DEV), torch.tensor(0.5, device=DEV)
+    assert emb(t).shape == (1, 128)
+    assert torch.equal(emb(t), emb(t[None]))
+
+
 def test_timestep_embedding_refuses():
     from dmf_amd import _lib
     call, p = _lib.load().dmf_timestep_embedding_fwd, torch.zeros(8, device=DEV).data_ptr()
