@@ -900,7 +900,7 @@ struct Casts {
   Tensor like;
   Tensor add(const Tensor& t, at::ScalarType dt) {
     if (t.scalar_type() == dt) return t;
-    if (dt != at::kBFloat16 || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.numel() < 8 || t.numel() % 8 ||
+    if (dt != at::kBFloat16 || t.scalar_type() != at::kFloat || t._is_zerotensor() || !t.is_contiguous() || t.numel() < 8 || t.numel() % 8 ||
         reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 || count == 4 || (like.defined() && like.device() != t.device()))
       return t.to(dt);
     like = empty(t.sizes(), dt, t);
