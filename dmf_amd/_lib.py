@@ -53,8 +53,6 @@ SIGNATURES = {
     "dmf_colsum": (c_int, [_P] * 3 + [_L, _I, _I, _I, _P]),
     "dmf_colsum_static": (c_int, [_P] * 2 + [_L, _I, _I, _I, _P]),
     "dmf_residual_ln_modulate_fwd": (c_int, [_P] * 14 + [_S] + [_I] * 3 + [_F] + [_I] * 4 + [_P]),
-    "dmf_cast_bf16": (c_int, [_P] * 3 + [_I, _P]),
-    "dmf_timestep_embedding_fwd": (c_int, [_P] * 4 + [_L, _I, _F, _I, _P]),
     "dmf_silu_fwd": (c_int, [_P] * 4 + [_L, _I, _I, _P]),
     "dmf_silu_bwd": (c_int, [_P] * 3 + [_L, _I, _I, _P]),
 }
@@ -69,6 +67,8 @@ FUSED_SIGNATURES = {
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
     "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
     "dmf_linear_wgrad": (c_int, [_P] * 5 + [_I] * 3 + [_P]),
+    "dmf_cast_bf16": (c_int, [_P] * 3 + [_I, _P]),
+    "dmf_timestep_embedding_fwd": (c_int, [_P] * 4 + [_L, _I, _F, _I, _P]),
 }
 
 _lib = None

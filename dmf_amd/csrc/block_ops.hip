@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "../../include/dmf_block.h"
+#include "../../include/dmf_fused.h"
 #include "attn_common.h"
 #include "attn_kernels.h"
 

@@ -141,21 +141,6 @@ DMF_ATTN_API int dmf_silu_bwd(const void* gy, const void* x, void* gx, int64_t n
                               void* stream);
 
 /*
- * dst[k] = src[k] rounded to bf16 (nearest, ties to even), k < count <= 4: dense fp32 arrays of n[k] elements, a multiple of 8.
- * The casts of a linear layer's operands under autocast.
- */
-DMF_ATTN_API int dmf_cast_bf16(const void* const* src, void* const* dst, const int64_t* n, int count, void* stream);
-
-/*
- * Sinusoidal embedding of n times: y[b] = [cos(t[b] f) | sin(t[b] f)] over the frequencies f[i] = exp(neg_log_period i / (dim / 2)),
- * i < dim / 2, a zero behind them where dim is odd, and when `ty` is given its tangent, [-sin(t f) f tt | cos(t f) f tt].
- * Replaces timestep_embedding (models/layers.py:46-55) and the cast behind it (:71).  t, tt: (n) of dtype; y, ty: (n, dim) of dtype;
- * computed in fp32.
- */
-DMF_ATTN_API int dmf_timestep_embedding_fwd(const void* t, const void* tt, void* y, void* ty, int64_t n, int dim,
-                                            float neg_log_period, int dtype, void* stream);
-
-/*
  * Per-head RMS norm over D of a logical (B, L, H, D) tensor:
  *   r = rsqrt(mean(x^2) + eps),  y = x * r * gain,
  *   ty = (tx * r + x * dr) * gain,  dr = -r^3 * mean(x * tx)   (when `ty` is given).

@@ -57,6 +57,21 @@ DMF_ATTN_API int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K);
 DMF_ATTN_API int dmf_linear_wgrad_plan(int64_t M, int N, int K);
 DMF_ATTN_API int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream);
 
+/*
+ * dst[k] = src[k] rounded to bf16 (nearest, ties to even), k < count <= 4: dense fp32 arrays of n[k] elements, a multiple of 8.
+ * The casts of a linear layer's operands under autocast.
+ */
+DMF_ATTN_API int dmf_cast_bf16(const void* const* src, void* const* dst, const int64_t* n, int count, void* stream);
+
+/*
+ * Sinusoidal embedding of n times: y[b] = [cos(t[b] f) | sin(t[b] f)] over the frequencies f[i] = exp(neg_log_period i / (dim / 2)),
+ * i < dim / 2, a zero behind them where dim is odd, and when `ty` is given its tangent, [-sin(t f) f tt | cos(t f) f tt].
+ * Replaces timestep_embedding (models/layers.py:46-55) and the cast behind it (:71).  t, tt: (n) of dtype; y, ty: (n, dim) of dtype;
+ * computed in fp32.
+ */
+DMF_ATTN_API int dmf_timestep_embedding_fwd(const void* t, const void* tt, void* y, void* ty, int64_t n, int dim,
+                                            float neg_log_period, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
