@@ -255,46 +255,29 @@ class DualLinearFunc(torch.autograd.Function):
         want_gx, want_gw = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
         want_gb = ctx.bias_dtype is not None and ctx.needs_input_grad[3]
         gx = gw = gb = None
-        # The input gradient and the parameter gradients are independent and the weight-gradient GEMM (small
-        # output, long contraction) does not fill the device, so on the GPU they are issued on two streams: a
-        # fork/join that a stream capture records as two parallel branches (-4 % on the XL/2 train step; the same
-        # trick for the primal / tangent GEMMs of the forward pass measured neutral to negative and is not used).
-        fork = g2.is_cuda and want_gx and (want_gw or want_gb)
-        if fork:
-            main, side = torch.cuda.current_stream(g2.device), _lib.side_stream(g2.device)
-            side.wait_stream(main)
-            torch.cuda.set_stream(side)
-        try:
-            if want_gw:
-                x2 = x.reshape(-1, x.shape[-1]).to(w.dtype)
-                if g2.is_cuda and g2.dtype != ctx.weight_dtype and ctx.weight_dtype == torch.float32:
-                    own = None if torch.is_grad_enabled() else _lib.linear_wgrad(g2, x2, want_gb and ctx.bias_dtype == torch.float32)
-                    if own is not None:
-                        gw, gb = own
-                    else:
-                        gw = torch.mm(g2.t(), x2, out_dtype=torch.float32)   # the GEMM stores its fp32 accumulators: no cast kernel
+        # (in one stream: next to each other in two, the products slow one another down and each fork and join idles the GPU)
+        if want_gw:
+            x2 = x.reshape(-1, x.shape[-1]).to(w.dtype)
+            if g2.is_cuda and g2.dtype != ctx.weight_dtype and ctx.weight_dtype == torch.float32:
+                own = None if torch.is_grad_enabled() else _lib.linear_wgrad(g2, x2, want_gb and ctx.bias_dtype == torch.float32)
+                if own is not None:
+                    gw, gb = own
                 else:
-                    gw = (g2.t() @ x2).to(ctx.weight_dtype)
-            if want_gb and gb is None:
-                # torch's multi-block column reduction clears its scratch with a memset node, which does not survive
-                # HIP-graph replay; the library's two-stage sum has no such node
-                if g2.is_cuda and g2.shape[1] % 8 == 0:
-                    gb = _lib.colsum(g2.contiguous(), ctx.bias_dtype)
-                else:
-                    if g2.is_cuda and torch.cuda.is_current_stream_capturing():
-                        raise RuntimeError("dual_linear: the bias gradient of a layer whose output width is not a multiple of 8 falls back "
-                                           "to torch's column sum, which does not replay correctly from a captured graph")
-                    gb = g2.sum(0).to(ctx.bias_dtype)
-        finally:
-            if fork:
-                torch.cuda.set_stream(main)
+                    gw = torch.mm(g2.t(), x2, out_dtype=torch.float32)   # the GEMM stores its fp32 accumulators: no cast kernel
+            else:
+                gw = (g2.t() @ x2).to(ctx.weight_dtype)
+        if want_gb and gb is None:
+            # torch's multi-block column reduction clears its scratch with a memset node, which does not survive
+            # HIP-graph replay; the library's two-stage sum has no such node
+            if g2.is_cuda and g2.shape[1] % 8 == 0:
+                gb = _lib.colsum(g2.contiguous(), ctx.bias_dtype)
+            else:
+                if g2.is_cuda and torch.cuda.is_current_stream_capturing():
+                    raise RuntimeError("dual_linear: the bias gradient of a layer whose output width is not a multiple of 8 falls back "
+                                       "to torch's column sum, which does not replay correctly from a captured graph")
+                gb = g2.sum(0).to(ctx.bias_dtype)
         if want_gx:
             gx = (g2 @ w).reshape(x.shape).to(x.dtype)
-        if fork:
-            main.wait_stream(side)
-            for t in (gw, gb):   # allocated on the side stream, consumed (and later freed) on the main one
-                if t is not None:
-                    t.record_stream(main)
         return gx, None, gw, gb, None, None
 
 

@@ -27,9 +27,7 @@
 #include <ATen/functorch/DynamicLayer.h>
 #include <ATen/functorch/TensorWrapper.h>
 #include <ATen/hip/EmptyTensor.h>
-#include <c10/core/Event.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
-#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
@@ -804,20 +802,6 @@ py::object timestep_embedding(const Tensor& t_, int64_t dim, double max_period) 
 
 // ---- linear --------------------------------------------------------------------------------------------------------------
 
-// One extra stream per device for the weight-gradient half of a layer's backward (the one dmf_amd._lib.side_stream hands out).
-c10::Stream side_stream(const Tensor& t) {
-  static std::array<std::optional<c10::Stream>, 64> streams;
-  static std::mutex m;
-  std::lock_guard<std::mutex> lock(m);
-  auto& s = streams.at(t.get_device());
-  if (!s) {
-    py::gil_scoped_acquire gil;
-    const py::object st = g_lib.attr("side_stream")(t.get_device());
-    s = c10::Stream::unpack3(st.attr("stream_id").cast<int64_t>(), st.attr("device_index").cast<int>(), at::kCUDA);
-  }
-  return *s;
-}
-
 Tensor column_sum(const Tensor& x, at::ScalarType dt) {
   const int64_t rows = x.size(0), C = x.size(1);
   const Tensor out = empty({C}, dt, x), ws = workspace(dmf_block_workspace_floats(3, 1, (int)std::min<int64_t>(rows, INT32_MAX), (int)C), x);
@@ -843,51 +827,30 @@ Tensor weight_gradient(const Tensor& g, const Tensor& x, Tensor* gb) {
   return gw;
 }
 
-// DualLinearFunc.backward: the parameter gradients on the side stream next to the input gradient.
+// DualLinearFunc.backward, in one stream: the parameter gradients next to the input gradient in a second one slow each other down, and a fork
+// and join leave the GPU idle for 18 us a layer.  Three-block training steps, two streams -> one: C1152 M8192 6.05 -> 5.56 ms, M2048 3.9 -> 3.3,
+// C768 M16384 5.81 -> 5.30, M8192 4.0 -> 3.42, C1024 M8192 5.17 -> 4.71; replayed from a graph C1152 M8192 5.83 -> 5.73, C768 M8192 3.70 -> 3.50,
+// C384 M8192 2.19 -> 2.06.
 variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w, const Tensor& gy, at::ScalarType w_type, at::ScalarType b_type,
                               bool has_bias) {
   const Tensor g2 = gy.reshape({-1, gy.size(-1)}).to(w.scalar_type()), x2 = x.reshape({-1, x.size(-1)}).to(w.scalar_type());
-  const bool want_gx = node.wants(0), want_gw = node.wants(1), want_gb = has_bias && node.wants(2), fork = want_gx && (want_gw || want_gb);
+  const bool want_gx = node.wants(0), want_gw = node.wants(1), want_gb = has_bias && node.wants(2), fp32_gw = g2.scalar_type() != w_type && w_type == at::kFloat;
   Tensor gx, gw, gb;
   if (!KernelNode::plain_call({gy})) {   // differentiated again or mapped over: operators that can be
     if (want_gx) gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
     if (want_gw) {
-      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = at::mm(g2.t().to(at::kFloat), x2.to(at::kFloat));
+      if (fp32_gw) gw = at::mm(g2.t().to(at::kFloat), x2.to(at::kFloat));
       else gw = at::mm(g2.t(), x2).to(w_type);
     }
     if (want_gb) gb = g2.sum(at::IntArrayRef{0}, false, at::kFloat).to(b_type);
     return {gx, gw, gb};
   }
-  auto parameters = [&] {
-    if (want_gw) {
-      if (g2.scalar_type() != w_type && w_type == at::kFloat) gw = weight_gradient(g2, x2, want_gb && b_type == at::kFloat ? &gb : nullptr);
-      else gw = at::mm(g2.t(), x2).to(w_type);
-    }
-    if (want_gb && !gb.defined()) gb = column_sum(dense(g2), b_type);
-  };
-  if (fork) {
-    const c10::impl::VirtualGuardImpl impl(at::kCUDA);
-    const c10::Stream main = impl.getStream(g2.device()), side = side_stream(g2);
-    c10::Event forked(at::kCUDA), joined(at::kCUDA);
-    forked.record(main);
-    side.wait(forked);
-    impl.exchangeStream(side);
-    try {
-      parameters();
-    } catch (...) {
-      impl.exchangeStream(main);
-      throw;
-    }
-    joined.record(side);
-    impl.exchangeStream(main);
-    gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
-    main.wait(joined);
-    for (const Tensor* t : {&gw, &gb})   // allocated on the side stream, consumed (and later freed) on the main one
-      if (t->defined()) t->record_stream(main);
-  } else {
-    parameters();
-    if (want_gx) gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
+  if (want_gw) {
+    if (fp32_gw) gw = weight_gradient(g2, x2, want_gb && b_type == at::kFloat ? &gb : nullptr);
+    else gw = at::mm(g2.t(), x2).to(w_type);
   }
+  if (want_gb && !gb.defined()) gb = column_sum(dense(g2), b_type);
+  if (want_gx) gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
   return {gx, gw, gb};
 }
 
