@@ -144,6 +144,8 @@ def timestep_embedding(t: Tensor, dim: int, max_period: int = 10000) -> Tensor:
 class TimestepEmbedder(nn.Module):
     """Reference models/layers.py:59-71."""
 
+    fused = False   # (of modules pickled whole before they had the option)
+
     def __init__(self, hidden_size: int, emb_size: int = 256, block_ops: str = "torch"):
         super().__init__()
         self.emb_size = emb_size
