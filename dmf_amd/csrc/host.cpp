@@ -854,8 +854,10 @@ variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w
   return {gx, gw, gb};
 }
 
-// The casts in front of a product: those that are fp32 -> bf16 of dense arrays are one launch, made by run().
+// The casts in front of a product: those that are fp32 -> bf16 of dense arrays are one launch, made by run().  Until then their sources
+// are held: a copy that reshape made would go back to the allocator, and the next one over it.
 struct Casts {
+  Tensor held[4];
   const void* src[4];
   void* dst[4];
   int64_t n[4];
@@ -867,6 +869,7 @@ struct Casts {
         reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 || count == 4 || (like.defined() && like.device() != t.device()))
       return t.to(dt);
     like = empty(t.sizes(), dt, t);
+    held[count] = t;
     src[count] = ptr(t);
     dst[count] = mptr(like);
     n[count++] = t.numel();

@@ -11,7 +11,7 @@ import dmf_amd
 from dmf_amd import _lib, block_ops, harness
 from dmf_amd.dmft import DMFT
 from dmf_amd.flash_attention_hip_jvp import flash_attn_projection
-from dmf_amd.layers import DiTBlock, FinalLayer, frozen_low_precision_params, stacked_modulations
+from dmf_amd.layers import DiTBlock, FinalLayer, Linear, frozen_low_precision_params, stacked_modulations
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -422,3 +422,23 @@ def test_block_with_hooks_or_replaced_parts_is_not_one_call():
         assert blk._one_call(x, x) is None
         del module.forward
     assert blk._one_call(x, x) is not None
+
+
+@pytest.mark.parametrize("view", [lambda t: t[:, 1:], lambda t: t.transpose(0, 1), lambda t: t[..., :128]])
+@pytest.mark.parametrize("both", [True, False])
+def test_linear_under_autocast_on_rows_that_have_to_be_copied(view, both):
+    """fp32 tokens that are no rows in memory, primal and tangent (or the primal alone): the bits of the dense call, with the weights
+    cast per call or kept."""
+    width = view(torch.empty(3, 9, 192)).shape[-1]
+    x, tx = (view(torch.randn(3, 9, 192, device=DEV)) for _ in range(2))
+    if not both:
+        tx = tx.contiguous()
+    layer = Linear(width, 256, block_ops="hip").to(DEV).requires_grad_(False)
+    fns = [layer, lambda t: block_ops.linear_gelu_tanh(t, layer.weight, layer.bias, layer.lp_weight, layer.lp_bias)]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        for kept in (contextlib.nullcontext(), frozen_low_precision_params(layer)):
+            with kept:
+                for fn in fns:
+                    got, ref = (torch.func.jvp(fn, (a,), (b,)) for a, b in ((x, tx), (x.contiguous(), tx.contiguous())))
+                    assert all(torch.equal(g, r) for g, r in zip(got, ref))
+                    assert torch.equal(fn(x), ref[0])
