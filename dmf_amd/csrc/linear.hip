@@ -355,6 +355,20 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
 #pragma unroll
     for (int i = 0; i < decltype(rows)::value; ++i) landed_in(X[b][i]);
   };
+  // The operands that are read ahead of a tile's first chunk.  The compiler takes what an assembly read returns for there and may copy it
+  // before it is: at the branch into a half tile it did.  So nothing is under way where the control flow is more than the loop over a tile's
+  // steps; across that loop's back edge the reads stay in flight, and that no instruction touches their registers before the wait is
+  // checked on the built code.
+  auto settle = [&] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int b = 0; b < AHEAD; ++b) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) landed_in(W[b][i]);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) landed_in(X[b][i]);
+    }
+  };
   f32x16 acc[NT][MT];
 
   // One stage's products.  Between the last chunk's and the next stage's, the emptied slots are requested again: w's at once, x's over the three
@@ -417,6 +431,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
 #pragma unroll
     for (int j = 0; j < T::PX / 3; ++j) request_x(j);
   }
+  settle();
 
   // Output rows leave two accumulator tiles at a time through this wave's 4 KB of LDS (32 rows of 128 bytes, slot v of row r holding vector
   // v ^ r / 2 % 8), in whole 16-byte vectors; while one pass is on its way through LDS the next one is computed.
@@ -427,6 +442,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   const int half = (lane >> 2) & 1;
   auto finish = [&](uint32_t id, auto rows_) {
     constexpr int MA = decltype(rows_)::value;
+    settle();
     const Place at = place(id);
     // bias of columns 8 v + 4 g .. + 3: wave-uniform vectors of eight by scalar loads (vector loads would wait for the DMA in flight)
     typedef const __attribute__((address_space(4))) uint32_t* ScalarPtr;

@@ -12,14 +12,14 @@ import pytest
 from dmf_amd import _lib
 
 LLVM = "/opt/rocm/llvm/bin"
-TOOLS = [os.path.join(LLVM, t) for t in ("llvm-objcopy", "clang-offload-bundler", "llvm-readelf")]
+TOOLS = [os.path.join(LLVM, t) for t in ("llvm-objcopy", "clang-offload-bundler", "llvm-readelf", "llvm-objdump")]
 pytestmark = pytest.mark.skipif(not all(os.path.exists(t) for t in TOOLS), reason="ROCm LLVM tools not installed")
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 
 @pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
-    """{mangled kernel name: {vgpr_count, vgpr_spill_count, private_segment_fixed_size, group_segment_fixed_size}}"""
+def code_objects(tmp_path_factory):
+    """Paths of the device code objects of the built library."""
     lib = _lib.LIB_PATH
     if not os.path.exists(lib):
         pytest.skip("library not built")
@@ -29,17 +29,26 @@ def kernels(tmp_path_factory):
     data = fat.read_bytes()
     starts = [m.start() for m in re.finditer(re.escape(MAGIC), data)]
     assert starts, "no offload bundle in the library"
-    out = {}
+    objects = []
     for i, s in enumerate(starts):
         bundle, co = tmp / f"b{i}.bin", tmp / f"co{i}.elf"
         bundle.write_bytes(data[s:starts[i + 1] if i + 1 < len(starts) else len(data)])
         subprocess.run([TOOLS[1], "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={bundle}", f"--output={co}",
                         "--unbundle"], check=True)
-        notes = subprocess.run([TOOLS[2], "--notes", str(co)], check=True, capture_output=True, text=True).stdout
+        objects.append(str(co))
+    yield objects
+    shutil.rmtree(tmp, ignore_errors=True)
+
+
+@pytest.fixture(scope="module")
+def kernels(code_objects):
+    """{mangled kernel name: {vgpr_count, vgpr_spill_count, private_segment_fixed_size, group_segment_fixed_size}}"""
+    out = {}
+    for co in code_objects:
+        notes = subprocess.run([TOOLS[2], "--notes", co], check=True, capture_output=True, text=True).stdout
         for m in re.finditer(r"\.name:\s+(\S+)\n(.*?)\.wavefront_size", notes, re.S):
             fields = dict(re.findall(r"\.(\w+):\s+(\d+)", m.group(2)))
             out[m.group(1)] = {k: int(v) for k, v in fields.items()}
-    shutil.rmtree(tmp, ignore_errors=True)
     return out
 
 
@@ -111,3 +120,109 @@ def test_products_and_split_operand_kernels_stay_within_their_launch_bounds(kern
     for n in names:
         k = kernels[n]
         assert k["vgpr_count"] <= registers and k["vgpr_spill_count"] <= spills, (n, k)
+
+
+# ---- LDS reads written in assembly -------------------------------------------------------------------------------------------
+# The compiler takes the result of an assembly read for there at once; the hardware does not hold back an instruction that uses the register
+# before the read has returned.  What keeps them apart is a wait in the source, and that the compiler moves nothing in between: checked on
+# the code it made, over all paths.
+
+SCALAR = 1 << 1024   # (a scalar load in the queue: those return in any order)
+
+
+def _registers(text):
+    mask = 0
+    for kind, one, first, last in re.findall(r"\b([va])(?:(\d+)\b|\[(\d+):(\d+)\])", text):
+        for r in range(int(one or first), int(one or last) + 1):
+            mask |= 1 << (r + (0 if kind == "v" else 512))
+    return mask
+
+
+def _decode(lines):
+    """(operation, registers it names, branch target, lgkmcnt waited for, registers a queued read returns or None) of every instruction."""
+    code = [(int(m.group(3), 16), m.group(1), m.group(2)) for m in (re.match(r"\t(\S+)\s*(.*?)\s*// ([0-9A-F]+):", l) for l in lines) if m]
+    at, out = {a: i for i, (a, _, _) in enumerate(code)}, []
+    for address, op, args in code:
+        target = wait = queued = None
+        if op == "s_branch" or op.startswith("s_cbranch"):
+            offset = int(args.split()[0])
+            target = at[address + 4 + 4 * (offset - 65536 * (offset >= 32768))]
+        elif op == "s_waitcnt":
+            assert "cnt(" in args, args
+            m = re.search(r"lgkmcnt\((\d+)\)", args)
+            wait = int(m.group(1)) if m else None
+        elif op.startswith("ds_"):
+            queued = _registers(args.split(",")[0]) if any(s in op for s in ("read", "_rtn", "permute", "swizzle")) else 0
+        elif op.startswith(("s_load", "s_buffer_load", "s_memtime", "s_memrealtime")):
+            queued = SCALAR
+        assert not op.startswith(("flat_", "s_swappc", "s_setpc", "s_call")), op
+        out.append((op, _registers(args), target, wait, queued))
+    return out
+
+
+def _touched_in_flight(code):
+    """Indices of instructions that name a register an LDS read may still be about to write.  State at a place: what the last 16 requests
+    return (the counter holds no more), newest last, joined over the paths that lead there."""
+    entries = {0} | {t for _, _, t, _, _ in code if t is not None} | {i + 1 for i, c in enumerate(code) if c[2] is not None}
+    states, work, bad = {0: ()}, [0], set()
+
+    def join(i, queue):
+        old = states.get(i)
+        if old is not None:
+            n = max(len(old), len(queue))
+            queue = tuple(a | b for a, b in zip((0,) * (n - len(old)) + old, (0,) * (n - len(queue)) + queue))
+        if queue != old:
+            states[i] = queue
+            work.append(i)
+
+    while work:
+        i = work.pop()
+        queue, first = states[i], True
+        while first or i not in entries:
+            first = False
+            op, names, target, wait, queued = code[i]
+            pending = 0
+            for q in queue:
+                pending |= q
+            if names & pending:
+                bad.add(i)
+            if wait == 0:
+                queue = ()
+            elif wait is not None and not pending & SCALAR:
+                queue = queue[-wait:]
+            if queued is not None:
+                queue = (queue + (queued,))[-16:]
+            if target is not None:
+                join(target, queue)
+            if op in ("s_branch", "s_endpgm"):
+                break
+            i += 1
+        else:
+            join(i, queue)
+    return bad
+
+
+def test_the_check_sees_a_read_that_is_not_waited_for():
+    lines = lambda *ops: [f"\t{op} // {4 * i:012X}: 00000000" for i, op in enumerate(ops)]
+    read, use = "ds_read_b128 v[4:7], v0", "v_mov_b32_e32 v8, v5"
+    assert _touched_in_flight(_decode(lines(read, use, "s_endpgm"))) == {1}
+    assert not _touched_in_flight(_decode(lines(read, "s_waitcnt lgkmcnt(0)", use, "s_endpgm")))
+    assert _touched_in_flight(_decode(lines(read, "ds_write_b64 v1, v[2:3]", "s_waitcnt vmcnt(0) lgkmcnt(2)", use, "s_endpgm"))) == {3}
+    assert not _touched_in_flight(_decode(lines(read, "ds_write_b64 v1, v[2:3]", "s_waitcnt vmcnt(0) lgkmcnt(1)", use, "s_endpgm")))
+    # over a back edge: read at the end of one turn, waited for in the next one only behind the use
+    assert _touched_in_flight(_decode(lines(use, "s_waitcnt lgkmcnt(0)", read, "s_cbranch_scc1 65532", "s_endpgm"))) == {0}
+
+
+def test_no_register_is_touched_between_its_lds_read_and_the_wait(code_objects):
+    names, code = [], []
+    for co in code_objects:
+        for line in subprocess.run([TOOLS[3], "-d", co], check=True, capture_output=True, text=True).stdout.splitlines():
+            m = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+            if m:
+                names.append(m.group(1))
+                code.append([])
+            elif code:
+                code[-1].append(line)
+    assert any("linear_walk_kernel" in n for n in names)
+    for name, lines in zip(names, code):
+        assert not _touched_in_flight(_decode(lines)), name
