@@ -95,17 +95,25 @@ struct Arg {
   bool grad() const { return var.defined() && var.requires_grad(); }
 };
 
+// What the kernels can read by address: a view that stands for its buffer's negative (torch._neg_view, the imaginary part of a conjugate) and
+// a zero tensor without storage are made into ordinary ones.
+Tensor in_memory(const Tensor& t) {
+  if (!t.is_neg() && !t._is_zerotensor()) return t;
+  const Below below;
+  return t._is_zerotensor() ? at::zeros(t.sizes(), t.options()) : t.resolve_neg();
+}
+
 Arg unpack(const Tensor& x) {
   Arg a;
   if (!x.defined()) return a;
   const Tensor& t = x._fw_grad(0);
   if (t.defined()) {
     const Tensor tv = unwrap(t);
-    a.tan = data_of(tv);
+    a.tan = in_memory(data_of(tv));
     a.tan_grad = tv.requires_grad();
   }
   a.var = unwrap(x);
-  a.data = data_of(a.var);
+  a.data = in_memory(data_of(a.var));
   return a;
 }
 Arg unpack(const OptTensor& x) { return x.has_value() ? unpack(*x) : Arg{}; }
@@ -865,7 +873,7 @@ struct Casts {
   Tensor like;
   Tensor add(const Tensor& t, at::ScalarType dt) {
     if (t.scalar_type() == dt) return t;
-    if (dt != at::kBFloat16 || t.scalar_type() != at::kFloat || t._is_zerotensor() || !t.is_contiguous() || t.numel() < 8 || t.numel() % 8 ||
+    if (dt != at::kBFloat16 || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.numel() < 8 || t.numel() % 8 ||
         reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 || count == 4 || (like.defined() && like.device() != t.device()))
       return t.to(dt);
     like = empty(t.sizes(), dt, t);
@@ -1005,6 +1013,7 @@ py::object chunk_last(const Tensor& x_, int64_t n) {
   if (level == kUnsupported) return none();
   const Arg x = unpack(x_);
   if (!plain_gpu(x) || x.data.dim() < 1 || x.data.size(-1) % n || only_tangents_want(x)) return none();
+  if (!x.data.is_alias_of(x.var)) return none();   // (the chunks are views of x)
   std::vector<Tensor> parts, tparts;
   const int64_t w = x.data.size(-1) / n;
   {

@@ -11,7 +11,7 @@ import dmf_amd
 from dmf_amd import _lib, block_ops, harness
 from dmf_amd.dmft import DMFT
 from dmf_amd.flash_attention_hip_jvp import flash_attn_projection
-from dmf_amd.layers import DiTBlock, FinalLayer, Linear, frozen_low_precision_params, stacked_modulations
+from dmf_amd.layers import DiTBlock, FinalLayer, Linear, TimestepEmbedder, frozen_low_precision_params, stacked_modulations
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -442,3 +442,20 @@ def test_linear_under_autocast_on_rows_that_have_to_be_copied(view, both):
                     got, ref = (torch.func.jvp(fn, (a,), (b,)) for a, b in ((x, tx), (x.contiguous(), tx.contiguous())))
                     assert all(torch.equal(g, r) for g, r in zip(got, ref))
                     assert torch.equal(fn(x), ref[0])
+
+
+def test_views_that_stand_for_the_negative_of_their_buffer():
+    """torch._neg_view of fp32 operands: the values of the negated tensor, under autocast (one cast for all operands) and without."""
+    x, t = torch.randn(3, 8, 128, device=DEV), torch.rand(16, device=DEV)
+    layer, emb = Linear(128, 256, block_ops="hip").to(DEV), TimestepEmbedder(128, block_ops="hip").to(DEV)
+    fns = [(layer, x), (lambda a: block_ops.linear_gelu_tanh(a, layer.weight, layer.bias), x), (emb, t), (block_ops.gelu_tanh, x),
+           (lambda a: block_ops.chunk_last(a, 2)[1], x)]
+    for autocast in (True, False):
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            for fn, a in fns:
+                neg = torch._neg_view(a)
+                assert neg.is_neg() and torch.equal(fn(neg), fn(-a))
+                assert all(torch.equal(g, r) for g, r in zip(torch.func.jvp(fn, (neg,), (neg,)), torch.func.jvp(fn, (-a,), (-a,))))
+    part = block_ops.chunk_last(torch._neg_view(x), 2)[0]
+    x[0, 0, 0] = 5.0
+    assert part[0, 0, 0] == -5.0
