@@ -308,20 +308,26 @@ class FinalLayer(nn.Module):
         return self.linear(modulate(self.norm_final(x), shift, scale))
 
 
-def _quiet(module: nn.Module, cls: type) -> bool:
-    """Calling the module is calling ``cls.forward``: no subclass, no replaced method, no hook of any direction."""
-    return (type(module) is cls and "forward" not in module.__dict__
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks))
+# what the classes' methods are, to tell a method that was replaced on the class from this file's own
+_OWN = {cls: cls.forward for cls in (nn.Sequential, SiLU, Linear, Attention, Mlp)} | {cls: cls.modulation for cls in (DiTBlock, FinalLayer)}
 
 
 def _plain(module: nn.Module, cls: type) -> bool:
-    return type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
+    """Calling the module is calling ``cls.forward`` as it stands here: no subclass, no method replaced on the object or on the class, no
+    forward hook, not compiled."""
+    return (type(module) is cls and cls.forward is _OWN[cls] and "forward" not in module.__dict__ and module._compiled_call_impl is None
+            and not module._forward_hooks and not module._forward_pre_hooks)
+
+
+def _quiet(module: nn.Module, cls: type) -> bool:
+    """``_plain``, and nothing watches its backward pass."""
+    return _plain(module, cls) and not module._backward_hooks and not module._backward_pre_hooks
 
 
 def _projection(owner: nn.Module, cls: type):
     """The adaLN projection of a block or final layer that computes it the way this file does: no subclass, no hook, no replaced
     method on the path from the conditioning vector to the chunks.  None otherwise."""
-    if type(owner).modulation is not cls.modulation or "modulation" in owner.__dict__ or not owner.fused:
+    if type(owner).modulation is not _OWN[cls] or "modulation" in owner.__dict__ or not owner.fused:
         return None
     seq = owner.adaLN_modulation
     if not _plain(seq, nn.Sequential) or len(seq._modules) != 2:

@@ -11,7 +11,7 @@ import dmf_amd
 from dmf_amd import _lib, block_ops, harness
 from dmf_amd.dmft import DMFT
 from dmf_amd.flash_attention_hip_jvp import flash_attn_projection
-from dmf_amd.layers import DiTBlock, FinalLayer, Linear, TimestepEmbedder, frozen_low_precision_params, stacked_modulations
+from dmf_amd.layers import Attention, DiTBlock, FinalLayer, Linear, Mlp, TimestepEmbedder, frozen_low_precision_params, stacked_modulations
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -421,7 +421,36 @@ def test_block_with_hooks_or_replaced_parts_is_not_one_call():
         module.forward = type(module).forward.__get__(module)
         assert blk._one_call(x, x) is None
         del module.forward
+        module.compile()   # (nothing is compiled before the first call)
+        assert blk._one_call(x, x) is None
+        module._compiled_call_impl = None
     assert blk._one_call(x, x) is not None
+
+
+@pytest.mark.parametrize("cls", [Attention, Mlp, Linear])
+def test_block_honours_a_forward_replaced_on_a_class(cls, monkeypatch):
+    blk = DiTBlock(128, 2, attn_func="hip", block_ops="hip").to(DEV).requires_grad_(False)
+    x, mods = torch.randn(2, 24, 128, device=DEV), [torch.randn(2, 1, 128, device=DEV) for _ in range(8)]
+    call, calls, forward = lambda: blk.forward_chained(x, x, mods[:6], *mods[6:], 1e-6), [], cls.forward
+    ref = call()
+    monkeypatch.setattr(cls, "forward", lambda self, *a: calls.append(self) or forward(self, *a))
+    got = call()
+    assert calls and all(torch.equal(g, r) for g, r in zip(got, ref))
+
+
+def test_stacked_modulations_honour_replaced_and_compiled_parts(monkeypatch):
+    blk, final = DiTBlock(128, 2, attn_func="hip", block_ops="hip").to(DEV, torch.bfloat16), FinalLayer(128, 2, 4, block_ops="hip").to(DEV, torch.bfloat16)
+    blk.requires_grad_(False), final.requires_grad_(False)
+    c = torch.randn(2, 1, 128, device=DEV).bfloat16()
+    ref, calls = stacked_modulations([blk], [c], final, c), []
+    flat = lambda out: [*out[0][0], *out[1]]
+    for owner, name in ((Linear, "forward"), (DiTBlock, "modulation"), (FinalLayer, "modulation")):
+        method = getattr(owner, name)
+        with monkeypatch.context() as m:
+            m.setattr(owner, name, lambda self, *a: calls.append(owner) or method(self, *a))
+            got = stacked_modulations([blk], [c], final, c)
+        # (bf16 results of sums in another order: a rounding each, 2^-8 of the value; sums near zero differ by 128 terms' fp32 roundings)
+        assert owner in calls and all(torch.allclose(g, r, rtol=2 ** -7, atol=1e-3) for g, r in zip(flat(got), flat(ref)))
 
 
 @pytest.mark.parametrize("view", [lambda t: t[:, 1:], lambda t: t.transpose(0, 1), lambda t: t[..., :128]])
