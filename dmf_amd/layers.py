@@ -252,10 +252,11 @@ class DiTBlock(nn.Module):
         x = x + gate_mlp * self.mlp(modulate(self.norm2(x), shift_mlp, scale_mlp))
         return x
 
-    def _one_call(self, x: Tensor, z: Tensor):
+    def _one_call(self, x: Tensor, z: Tensor, *mods: Tensor):
         """What the native host path needs to run the block in one call: heads, the four linear layers' tensors, the q / k norms.  None
-        where a module on the way is not this file's own, has a hook or a replaced forward, or anything watches the calls."""
-        if not _lib.native(x, z) or torch.nn.modules.module._has_any_global_hook():
+        where a module on the way is not this file's own, has a hook or a replaced forward, or anything watches the calls, be it the class
+        of an operand."""
+        if not _lib.native(x, z, *mods) or torch.nn.modules.module._has_any_global_hook():
             return None
         attn, mlp = self.attn, self.mlp
         if not (_quiet(attn, Attention) and attn.packed and _quiet(mlp, Mlp)):
@@ -278,7 +279,7 @@ class DiTBlock(nn.Module):
         block's msa pair, or the final layer's).  Returns ``(x_out, z_next)``; same
         values as ``forward``."""
         _, _, gate_msa, shift_mlp, scale_mlp, gate_mlp = mods
-        layers = self._one_call(x, z)
+        layers = self._one_call(x, z, gate_msa, shift_mlp, scale_mlp, gate_mlp, next_shift, next_scale)
         if layers is not None:
             out = _lib.host().block(x, z, gate_msa, shift_mlp, scale_mlp, gate_mlp, next_shift, next_scale, self.norm2.eps, next_eps, *layers)
             if out is not None:

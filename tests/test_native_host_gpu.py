@@ -427,6 +427,28 @@ def test_block_with_hooks_or_replaced_parts_is_not_one_call():
     assert blk._one_call(x, x) is not None
 
 
+def test_block_with_modulations_of_a_class_of_their_own_is_not_one_call():
+    """Gates, shifts and scales whose class has a __torch_function__: it sees the operators, as it did one by one."""
+    class Watching(torch.Tensor):
+        seen = []
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            cls.seen.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    blk = DiTBlock(128, 2, attn_func="hip", block_ops="hip").to(DEV).requires_grad_(False)
+    x, mods = torch.randn(2, 24, 128, device=DEV), [torch.randn(2, 1, 128, device=DEV) for _ in range(8)]
+    ref = blk.forward_chained(x, x, mods[:6], *mods[6:], 1e-6)
+    assert blk._one_call(x, x, *mods[2:]) is not None
+    for i in range(2, 8):
+        own = [m.as_subclass(Watching) if k == i else m for k, m in enumerate(mods)]
+        assert blk._one_call(x, x, *own[2:]) is None
+        Watching.seen.clear()
+        got = blk.forward_chained(x, x, own[:6], *own[6:], 1e-6)
+        assert Watching.seen and all(torch.equal(g.as_subclass(torch.Tensor), r) for g, r in zip(got, ref))
+
+
 @pytest.mark.parametrize("cls", [Attention, Mlp, Linear])
 def test_block_honours_a_forward_replaced_on_a_class(cls, monkeypatch):
     blk = DiTBlock(128, 2, attn_func="hip", block_ops="hip").to(DEV).requires_grad_(False)
