@@ -301,8 +301,8 @@ def linear_gelu_tanh(x, weight, bias, w_lp=None, b_lp=None):
     activation -- and its derivative on the tangent -- rides in the product's epilogue
     (the pre-activation never reaches HBM); otherwise the pre-activation is needed for
     the backward pass and this is ``dual_linear`` followed by ``gelu_tanh``."""
-    if bias is not None and not (torch.is_grad_enabled() and weight.requires_grad) and _lib.native(x, weight, bias):
-        out = _lib.host().linear_gelu(x, weight, bias, w_lp, b_lp)
+    if _lib.native(x, weight, bias):
+        out = _lib.host().linear_gelu_tanh(x, weight, bias, w_lp, b_lp)
         if out is not None:
             return out
     if torch.is_grad_enabled() or bias is None or not x.is_cuda or fwAD.unpack_dual(x).tangent is not None:

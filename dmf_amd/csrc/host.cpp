@@ -1007,6 +1007,22 @@ py::object linear_gelu(const Tensor& x_, const Tensor& weight_, const Tensor& bi
   return py::cast(finish(y, ty, nullptr, level));
 }
 
+// gelu_tanh(linear(x)), one kernel or two.  Without history to build and yet not for the kernel above: none, the general route has a library
+// call with the activation in it.
+py::object linear_gelu_tanh(const Tensor& x, const Tensor& weight, const OptTensor& bias, const OptTensor& w_lp, const OptTensor& b_lp) {
+  if (current_level() == kUnsupported) return none();
+  const bool grad = c10::GradMode::is_enabled();
+  if (bias && !(grad && weight.requires_grad())) {
+    py::object out = linear_gelu(x, weight, *bias, w_lp, b_lp);
+    if (!out.is_none()) return out;
+  }
+  if (bias && !grad) return none();
+  const py::object h = linear(x, weight, bias, w_lp, b_lp);
+  if (h.is_none()) return none();
+  py::object out = activation(h.cast<Tensor>(), Act::gelu);
+  return out.is_none() ? py::object(py::module_::import("dmf_amd.block_ops").attr("gelu_tanh")(h)) : out;
+}
+
 // x.chunk(n, -1) of a modulation tensor, tangent included
 py::object chunk_last(const Tensor& x_, int64_t n) {
   const int64_t level = current_level();
@@ -1077,17 +1093,11 @@ py::object block(const Tensor& x, const Tensor& z, const Tensor& gate_msa, const
     if (out.is_none()) out = ops("residual_ln_modulate")(x, gate, h, shift, scale, eps);
     return py::tuple(std::move(out));
   };
-  const auto mlp_in = [&](const py::object& in) {   // (as block_ops.linear_gelu_tanh)
+  const auto mlp_in = [&](const py::object& in) {
     const auto& [w, b, w_lp, b_lp] = fc1;
-    const bool grad = c10::GradMode::is_enabled();
-    if (b && !(grad && w.requires_grad())) {
-      py::object out = linear_gelu(in.cast<Tensor>(), w, *b, w_lp, b_lp);
-      if (!out.is_none()) return out;
-    }
-    if (b && !grad) return py::object(ops("linear_gelu_tanh")(in, w, *b, w_lp, b_lp));
-    const py::object h = project(in, fc1);
-    py::object out = activation(h.cast<Tensor>(), Act::gelu);
-    return out.is_none() ? py::object(ops("gelu_tanh")(h)) : out;
+    const Tensor t = in.cast<Tensor>();
+    py::object out = linear_gelu_tanh(t, w, b, w_lp, b_lp);
+    return out.is_none() ? py::object(ops("linear_gelu_tanh")(t, w, b, w_lp, b_lp)) : out;
   };
   py::object h = project(py::cast(z), qkv);
   h = attend(h);
@@ -1207,7 +1217,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("gelu_tanh", [](const Tensor& x) { return activation(x, Act::gelu); });
   m.def("silu", [](const Tensor& x) { return activation(x, Act::silu); });
   m.def("linear", &linear);
-  m.def("linear_gelu", &linear_gelu);
+  m.def("linear_gelu_tanh", &linear_gelu_tanh);
   m.def("chunk_last", &chunk_last);
   m.def("modulations", &modulations);
   m.def("block", &block);

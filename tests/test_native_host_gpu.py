@@ -371,14 +371,15 @@ def test_stacked_modulations_leave_to_the_blocks():
     assert tries(c) == [True] and tries(c.requires_grad_()) == [False]
 
 
+@pytest.mark.parametrize("C,H,L", [(128, 2, 24), (1152, 16, 40), (384, 6, 333)])
 @pytest.mark.parametrize("dtype,qk_norm,autocast", [(torch.float32, False, True), (torch.float32, True, True), (torch.float32, True, False),
                                                    (torch.bfloat16, False, False)])
-def test_block_in_one_call(dtype, qk_norm, autocast):
+def test_block_in_one_call(dtype, qk_norm, autocast, C, H, L):
     """A block as one native call and as its modules one by one: the same bits in every way it is differentiated, with frozen weights too."""
     torch.manual_seed(3)
-    blk = DiTBlock(128, 2, qk_norm=qk_norm, attn_func="hip", block_ops="hip").to(DEV, dtype)
+    blk = DiTBlock(C, H, qk_norm=qk_norm, attn_func="hip", block_ops="hip").to(DEV, dtype)
     rnd = lambda *s: torch.randn(*s, device=DEV).to(dtype)
-    x, z, mods, nxt = rnd(2, 24, 128), rnd(2, 24, 128), [rnd(2, 1, 128) for _ in range(6)], [rnd(2, 1, 128) for _ in range(2)]
+    x, z, mods, nxt = rnd(2, L, C), rnd(2, L, C), [rnd(2, 1, C) for _ in range(6)], [rnd(2, 1, C) for _ in range(2)]
     params = list(blk.parameters())[:-2]   # (the modulation's own layer is not part of it)
 
     def every_mode():
