@@ -316,13 +316,16 @@ _OWN = {cls: cls.forward for cls in (nn.Sequential, SiLU, Linear, Attention, Mlp
 def _plain(module: nn.Module, cls: type) -> bool:
     """Calling the module is calling ``cls.forward`` as it stands here: no subclass, no method replaced on the object or on the class, no
     forward hook, not compiled."""
-    return (type(module) is cls and cls.forward is _OWN[cls] and "forward" not in module.__dict__ and module._compiled_call_impl is None
-            and not module._forward_hooks and not module._forward_pre_hooks)
+    own = module.__dict__
+    return (type(module) is cls and cls.forward is _OWN[cls] and "forward" not in own and module._compiled_call_impl is None
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"]))
 
 
 def _quiet(module: nn.Module, cls: type) -> bool:
     """``_plain``, and nothing watches its backward pass."""
-    return _plain(module, cls) and not module._backward_hooks and not module._backward_pre_hooks
+    own = module.__dict__
+    return (type(module) is cls and cls.forward is _OWN[cls] and "forward" not in own and module._compiled_call_impl is None
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]))
 
 
 def _projection(owner: nn.Module, cls: type):
