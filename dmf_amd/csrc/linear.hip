@@ -199,7 +199,8 @@ static int launch_linear(LinearParams& p, bool jvp, hipStream_t stream) {
 // tile's first stages arrive during the last ones of the tile before and its stores drain behind the next one's products: 113 us, 1026 TFLOP/s; C768
 // M16384 K 4C 153 -> 125, gelu pair N 4C 195 -> 162; C1152 M8192 N 3C 126 -> 115, K 4C 170 -> 148, gelu pair 176 -> 163.  Without its DMA the loop runs at
 // 1560 TFLOP/s: what is left is the waves' wait at the CU's one address unit, four requests at a time (letting the waves take turns by branches cost
-// more than it gave: 8192 cubed 819 -> 927 us), and a tile's end (3 us of 19 at 12 steps).
+// more than it gave: 8192 cubed 819 -> 927 us), and a tile's end (3 us of 19 at 12 steps; the 6 us a tile of the estimate below are what it takes
+// beyond its steps at the pace of deep products).
 // Stages are 64 contraction elements, whole 128-byte lines (stages of 32 with twice the depth: 8192 x 3 unchanged, but 12 % more time in light
 // grids, where each half line is a request of its own); three of x and two of w fill the LDS, x being the operand that comes from HBM.  Slot v of
 // row r holds vector v ^ r / 2 % 8: 16 rows read at one vector meet all sixteen 16-byte bank groups.  While the products of one 16-deep chunk issue,
@@ -560,14 +561,23 @@ static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
   return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
 }
 
-// Tile policy: the shortest of the estimates, in 10 ns, of six kernels.  Fitted to 268 products of the models' widths (384, 768, 1024, 1152), 512
-// to 32768 rows, single and in pairs, with and without gelu; standard error 8 to 11 %, and the tile taken is within 1 % of the fastest one in the
-// mean.  (Refitted for the 128 x 96 tile alone, 110 products of which it takes 20.)  linear_kernel: a K step (64) and a work-group's start and end with one, two, three work-groups on a CU; linear_walk_kernel: a step of a
-// whole and of half a tile, a tile's end, and the launch's.
+// Tile policy: the shortest of the estimates, in 10 ns, of six kernels.  linear_kernel: a K step (64) and a work-group's start and end with one,
+// two, three work-groups on a CU, more of them never taking less; linear_walk_kernel: a step and what a tile takes beyond its steps at that
+// pace, of whole and of half a tile, and the launch's.  Fitted to 1440 products of
+// widths 384 to 1280, 64 to 32768 rows, single and in pairs, with and without gelu, seven tenths of them; all of them and the fit's aim are in
+// profiles/linear_tiles.txt.  Tiles within 1.3 of the fastest one are met to 4 (128 x 96) to 11 % (64 x 64); the tile taken is 0.24 % slower than
+// the fastest in the mean (0.25 % where the fit did not look), 5 % in one of a hundred.  128 x 192 is all but never that tile; it is here
+// for the rows of more than 65536 elements that the walking kernel does not take.
 struct LinTile { int bm, bn, per_cu, a[3], b[3]; };
-constexpr LinTile kLinTiles[3] = {{128, 192, 2, {76, 121, 0}, {508, 750, 0}}, {128, 64, 3, {50, 60, 85}, {337, 437, 340}}, {64, 64, 2, {15, 37, 0}, {480, 170, 0}}};
+constexpr LinTile kLinTiles[3] = {{128, 192, 2, {82, 113, 0}, {541, 761, 0}}, {128, 64, 3, {48, 68, 80}, {262, 364, 466}}, {64, 64, 2, {23, 39, 0}, {279, 263, 0}}};
+constexpr bool never_shorter_with_more(const LinTile& t) {
+  for (int o = 1; o < t.per_cu; ++o)
+    if (t.a[o] < t.a[o - 1] || t.a[o] + t.b[o] < t.a[o - 1] + t.b[o - 1]) return false;
+  return true;
+}
+static_assert(never_shorter_with_more(kLinTiles[0]) && never_shorter_with_more(kLinTiles[1]) && never_shorter_with_more(kLinTiles[2]));
 struct LinWalk { int bm, bn, a, b, a_half, b_half, launch; };
-constexpr LinWalk kLinWalks[2] = {{256, 192, 100, 700, 52, 540, 40}, {256, 128, 76, 460, 43, 430, 80}};
+constexpr LinWalk kLinWalks[2] = {{256, 192, 94, 607, 59, 433, 136}, {256, 128, 73, 386, 45, 413, 135}};
 
 // A gelu pair holds an element of x and its tangent in one wave, half of the rows of each: it has as many work-groups as a single product of twice
 // the rows, takes the tiles with two row tiles per wave, and whole ones.
@@ -599,7 +609,7 @@ static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
   // 128 x 96, where all tiles run at once: an L2 shared by more than half of the CUs lengthens the step
   if (!both && N <= 65536 && K <= 65536) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 95) / 96) * (jvp ? 2 : 1);
-    if (tiles <= cus) take(5, 480 + (30 * cus + 20 * std::max<int64_t>(0, tiles - cus / 2)) * steps / cus);
+    if (tiles <= cus) take(5, 534 + (31 * cus + 14 * std::max<int64_t>(0, tiles - cus / 2)) * steps / cus);
   }
   // (the walking kernel's row offsets within a tile are 32-bit)
   for (int t = 0; t < 2 && N <= 65536 && K <= 65536; ++t) {
