@@ -639,23 +639,32 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
 
 }  // namespace dmf
 
-// Which calls these kernels are the faster ones for (us, library -> here; C: model width, M rows):
-//   pairs: C768 M16384 N 3C 137 -> 113, N C 48 -> 40, K 4C 129 -> 125; C1152 M8192 161 -> 115, 65 -> 43, N 4C 169 -> 149, K 4C 167 -> 148;
-//     M4096 84 -> 66, 40 -> 24, K 4C 98 -> 73;
-//   single: C768 M2048 N 3C 20 -> 12.3, M4096 N 3C 20.8 -> 19.1; C1152 M8192 N 3C 83 -> 63, K 4C 80 -> 75, M16384 K 4C 157 -> 148;
-//     K 4C: M1024 C768 22 -> 13, M2048 C768 20.7 -> 19.6 (C384 22.7 -> 8.1), M3000 C768 23.7 -> 21.2, M4096 C768 26.5 -> 24.0,
-//     M2048 C1152 32.0 -> 28.6, M8192 C768 37.3 -> 36.9;
-//   the library keeps single products with few columns for their depth up to four million results where the 128 x 96 tiles need a second round
-//   (K 4C: C768 M4500 28.3 against 29.1, M5000 30.4 against 35.7; C1024 M3072 30.0 against 31.7), those that spread a short K over a large result (N 4C M16384: C768 pairs 137 against
-//   144, 32768 rows 130 against 136 single), rows of 2 or 8 KB on large results (C1024: M16384 K 4C 183 against 234, N C 60 against 63,
-//   M8192 N 4C 106 against 122) and outputs narrower than a tile;
+// Which calls these kernels are the faster ones for (us on the GPU, library -> here; C: model width, M rows; called from the host a library
+// product takes 18 us at least, one of these 5):
+//   pairs: C768 M16384 N 3C 137 -> 106, N C 45 -> 38, K 4C 131 -> 124; C1152 M8192 158 -> 113, 62 -> 42, N 4C 169 -> 148, K 4C 165 -> 149;
+//     M4096 81 -> 62, 37 -> 24, K 4C 94 -> 73;
+//   single: C768 M1024 N 3C 11.5 -> 9.4, M2048 15.6 -> 12.7, M4096 18.5 -> 18.8, N C 11.8 -> 9.7; C1152 M8192 N 3C 79 -> 64, K 4C 80 -> 73;
+//     K 4C: M1024 C768 15.1 -> 13.5, M2048 C384 9.9 -> 8.5, C1152 31.8 -> 29.4, M3000 C768 23.3 -> 21.4, M4096 25.3 -> 23.6, M8192 36.4 -> 37.1.
+// The library's time moves by a fifth to either side with its own choice of tile, so that no line is sharp.  It keeps
+//   single products deeper than they are wide (K 4C) whose 128 x 96 tiles need up to a third of a second round, 4 % faster in the mean of 48 measured
+//     (M4500 C768 26.5 against 29.1, M3072 C1024 30.1 against 32.4, M3000 C1152 36.0 against 38.7; one round, M4096 C768, 25.3 against
+//     23.6; from four thirds on even in the mean, up to a tenth either way; K up to 2304 even);
+//   those that spread a short K over a large result (N 4C: C768 M16384 pairs 131 against 138, M32768 single 128 against 140), rows of 2 or 8 KB on
+//     large results (C1024: M16384 K 4C 92 against 116, N C 28.9 against 32.8, M8192 N 4C 56 against 67);
+//   and outputs narrower than a tile.
+// Deep products of few rows are a trade: on the GPU alone, as replayed from a graph, the library's are faster (K 4C: M64 C768 7.4 against 12.6, M256
+// 8.7 against 12.6, M512 11.5 against 12.1, M2048 18.2 against 19.7), called from the host slower where that is what bounds the calls (18.3
+// against 12.1 up to M512; the library taken for M2197 C768, two blocks sampled by a host that does not run ahead: 1.68 -> 1.73 ms).  They are taken.
 //   pairs with gelu (library pair and activation kernel; this kernel's pair and the activation kernel -> here), N 4C, wins from one row up:
-//     M16 C384 10.4; 7.7 -> 5.3, C768 11.3; 8.1 -> 7.1, C1152 12.7; 9.2 -> 8.9;  M512 C768 23.4; 15.5 -> 10.6, C1152 34.0; 24.1 -> 18.3;
-//     M4096 C768 61.7; 58.2 -> 40.3, C1152 131; 104 -> 80;  M8192 C384 63.8; 43.6 -> 30.1, C1024 152; 182 -> 142, C1152 212; 212 -> 163.
+//     M16 C384 10.4; 7.7 -> 5.3, C768 11.3; 8.1 -> 7.1, C1152 12.7; 9.2 -> 8.9;  M512 C768 23.4; 15.5 -> 12.0, C1152 34.0; 24.1 -> 18.2;
+//     M4096 C768 61.7; 58.2 -> 40.7, C1152 131; 104 -> 82;  M8192 C384 63.8; 43.6 -> 28.6, C1024 152; 182 -> 138, C1152 212; 212 -> 159.
 extern "C" int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu) {
   if (M < 1 || N < 64 || N % 8 || K < 64 || K % 64 || M * K > (int64_t)1 << 30 || (int64_t)N * K > (int64_t)1 << 30 || M * N > (int64_t)1 << 30) return 0;
   if (jvp && gelu) return 1;
-  if (!jvp && K >= 2 * N && K > 2048 && M * N > 2000000 && M * N < 4000000 && ((M + 127) / 128) * ((N + 95) / 96) > dmf::compute_units()) return 0;
+  if (!jvp && K > 2048 && K >= 2 * N) {
+    const int64_t cus = dmf::compute_units(), tiles = ((M + 127) / 128) * ((N + 95) / 96);
+    if (tiles > cus && 3 * tiles <= 4 * cus) return 0;
+  }
   if (K >= 1024 && (K & (K - 1)) == 0 && (M >= 16384 || (N >= 4 * K && M >= 4096))) return 0;
   if (M * N > 40000000 && N > 3 * K && N > 2048 && (jvp || K < 1024)) return 0;
   return 1;

@@ -384,3 +384,13 @@ def test_operators_do_without_the_native_host_path(monkeypatch, built_for):
         assert not _lib.native(on_gpu)
     with pytest.raises(RuntimeError, match="dmf_amd.build"):
         _lib.host()
+
+
+@pytest.mark.parametrize("C", [640, 768, 896, 1024, 1152, 1280])
+def test_deep_products_go_to_the_library_by_rounds(C):
+    """Single products four times as deep as wide: the library's where 128 x 96 tiles need up to a third of a second round on 256 CUs, whatever
+    the number of results."""
+    for M in range(64, 9000, 64):
+        for rows in (M, M + 1):
+            tiles = -(-rows // 128) * -(-C // 96)
+            assert _lib.load().dmf_linear_plan(rows, C, 4 * C, 0, 0) == (not 256 < tiles <= 341), rows
