@@ -64,6 +64,7 @@ FUSED_SIGNATURES = {
     "dmf_modulation_fwd": (c_int, [_P] * 5 + [_I] * 6 + [_P]),
     "dmf_linear_plan": (c_int, [_L] + [_I] * 4),
     "dmf_linear_fwd": (c_int, [_P] * 6 + [_I] * 4 + [_P]),
+    "dmf_linear_fwd_plan": (c_int, [_L] + [_I] * 4 + [ctypes.c_char_p, _I]),
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
     "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
     "dmf_linear_wgrad": (c_int, [_P] * 5 + [_I] * 3 + [_P]),

@@ -5,6 +5,7 @@
 // The library ran the two products of a layer one after the other (two partly empty last rounds), in tiles that fit these widths
 // badly, and spent 18 us of host time on each.  Here both are one grid; 192 columns divide most layer widths of the models.
 #include <algorithm>
+#include <cstdio>
 #include <type_traits>
 #include <utility>
 #include "attn_common.h"
@@ -668,6 +669,19 @@ extern "C" int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu) {
   if (K >= 1024 && (K & (K - 1)) == 0 && (M >= 16384 || (N >= 4 * K && M >= 4096))) return 0;
   if (M * N > 40000000 && N > 3 * K && N > 2048 && (jvp || K < 1024)) return 0;
   return 1;
+}
+
+extern "C" int dmf_linear_fwd_plan(int64_t M, int N, int K, int jvp, int gelu, char* buf, int buflen) {
+  if (M < 1 || M > INT32_MAX || N < 8 || N % 8 || K < 64 || K % 64 || M * K > (int64_t)1 << 30 || (int64_t)N * K > (int64_t)1 << 30 || M * N > (int64_t)1 << 30)
+    return DMF_ATTN_ESHAPE;
+  if (buf == nullptr || buflen < 1) return DMF_ATTN_ENULL;
+  const int mode = !gelu ? dmf::kLinPlain : jvp ? dmf::kLinGeluJvp : dmf::kLinGelu;
+  const char* form[6] = {"linear_kernel<128, 192, 2, %d>", "linear_kernel<128, 64, 2, %d>", "linear_kernel<64, 64, 4, %d>",
+                         "linear_walk_kernel<dmf::WalkTile<4, 3, 2, 3, 2>, %d>", "linear_walk_kernel<dmf::WalkTile<4, 2, 2, 3, 3>, %d>",
+                         "linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>, %d>"};
+  const int n = snprintf(buf, (size_t)buflen, "dmf::");
+  if (n < buflen) snprintf(buf + n, (size_t)(buflen - n), form[dmf::linear_tile(M, N, K, jvp != 0, gelu != 0)], mode);
+  return DMF_ATTN_OK;
 }
 
 extern "C" int dmf_linear_fwd(const void* x, const void* tx, const void* w, const void* bias, void* y, void* ty, int M, int N, int K, int gelu, void* stream) {

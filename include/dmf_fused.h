@@ -41,9 +41,11 @@ DMF_ATTN_API int dmf_modulation_fwd(const void* const* s, const void* const* w, 
  * y = x w^T + bias (gelu: with the tanh form of gelu applied), bf16 with fp32 accumulation: x (M, K), w (N, K), bias (N) or NULL,
  * y (M, N), all dense; tx / ty (both or neither): ty = tx w^T besides, in the same grid (gelu: times the activation's derivative).
  * K a multiple of 64, N of 8, at most 2^30 elements in x, w and y; 16-byte aligned, bias 8-byte.  dmf_linear_plan: 1 where this
- * kernel is the better choice (and covers the shape), 0 where a library product is; host-only.
+ * kernel is the better choice (and covers the shape), 0 where a library product is; host-only.  dmf_linear_fwd_plan: the name of the kernel
+ * that dmf_linear_fwd launches for the shape on the current device, as profilers print it; host-only.
  */
 DMF_ATTN_API int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu);
+DMF_ATTN_API int dmf_linear_fwd_plan(int64_t M, int N, int K, int jvp, int gelu, char* buf, int buflen);
 DMF_ATTN_API int dmf_linear_fwd(const void* x, const void* tx, const void* w, const void* bias, void* y, void* ty, int M, int N, int K,
                         int gelu, void* stream);
 

@@ -122,6 +122,16 @@ def test_products_and_split_operand_kernels_stay_within_their_launch_bounds(kern
         assert k["vgpr_count"] <= registers and k["vgpr_spill_count"] <= spills, (n, k)
 
 
+def test_every_product_kernel_is_launched_by_a_test(kernels):
+    """The kernels of dmf_linear_fwd, by their template arguments, against those that the sizes of the GPU tests reach on 256 CUs (what a
+    process without a GPU plans for)."""
+    from test_linear_gpu import REACHED, planned
+    numbers = lambda pattern, name: tuple(int(n) for n in re.findall(pattern, name))
+    built = {numbers(r"Li(\d+)E", n) for n in kernels if re.search(r"linear_(walk_)?kernelI", n)}
+    reached = {numbers(r"\b(\d+)\b", planned(*size, *mode)) for _, size, modes in REACHED for mode in modes}
+    assert len(built) == 16 and reached == built
+
+
 # ---- LDS reads written in assembly -------------------------------------------------------------------------------------------
 # The compiler takes the result of an assembly read for there at once; the hardware does not hold back an instruction that uses the register
 # before the read has returned.  What keeps them apart is a wait in the source, and that the compiler moves nothing in between: checked on

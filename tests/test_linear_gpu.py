@@ -1,4 +1,6 @@
 """The package's own product kernel (dmf_linear_fwd) against fp32 products of the same bf16 operands."""
+import ctypes
+
 import pytest
 import torch
 
@@ -35,7 +37,7 @@ def _check(got, ref):
     assert ((got.float() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all()
 
 
-# the four tiles (64 x 64; 128 x 64; 128 x 128; 128 x 192) and their edges: one row, a row past a tile, columns that fill none, one step
+# edges of whatever tile is taken: one row, a row past a tile, columns that fill none, one step (which kernel runs: REACHED, below)
 SIZES = [(1, 8, 64), (63, 64, 64), (65, 72, 128), (129, 200, 192), (333, 1152, 384), (4096, 768, 768), (4097, 712, 640), (2048, 2304, 768),
          (2000, 3456, 128), (8192, 2304, 768), (16384, 2304, 64), (16389, 2296, 320), (256, 768, 3072)]
 
@@ -139,8 +141,8 @@ def test_weight_gradient_refuses():
     assert lib.dmf_linear_wgrad_workspace_floats(64, 60, 64) == -1
 
 
-# the kernel whose work-groups walk through the tiles (256 x 192, 256 x 128; with tangents and gelu 128 rows of each): whole rounds and half
-# tiles behind them, only half tiles, a row and a column block that fill neither, one step per tile and fewer steps than stages; outputs whole
+# sizes that the kernel whose work-groups walk through the tiles takes (256 x 192, 256 x 128; with tangents and gelu 128 rows of each): whole rounds and
+# half tiles behind them, only half tiles, a row and a column block that fill neither, one step per tile and fewer steps than stages; outputs whole
 WALK = [(2049, 2296, 768), (8193, 1152, 1152), (4100, 1016, 1024), (12345, 1016, 192), (16384, 2304, 64), (2300, 3064, 448)]
 
 
@@ -161,8 +163,8 @@ def test_products_of_many_tiles(M, N, K):
     _check(ty, tact)
 
 
-# the same kernel's 128 x 96 tiles, up to one per CU: a row past a tile, a last column block of 8 and of 88 columns, fewer steps than stages' ring
-# and many; single products, and pairs of half the rows
+# products of about one tile of 128 x 96 per CU and its neighbours in size, where several kernels are close: a row past a tile, a last column block of
+# 8 and of 88 columns, few steps and many; single products, and pairs of half the rows
 ONE_ROUND = [(2433, 776, 448), (2561, 1144, 576), (1025, 2296, 448), (2047, 1528, 768), (897, 3064, 768), (4096, 768, 3072)]
 
 
@@ -178,3 +180,52 @@ def test_products_of_one_round(M, N, K):
         _check(ty, tref[:half])
     act = torch.nn.functional.gelu(ref, approximate="tanh")
     assert (_call(x, None, w, b, 1)[0].float() - act).norm() <= TOL * act.norm()
+
+
+# Every kernel in every mode, with what dmf_linear_fwd_plan says for 256 CUs asserted: rows and columns that fill no tile, more than one round
+# where the kernel is taken there, half tiles and whole ones, one step and many, rows of more than 65536 elements
+PLAIN, PAIR, GELU, GELU_PAIR = MODES = [(0, 0), (1, 0), (0, 1), (1, 1)]   # (tangents, gelu)
+REACHED = [("linear_kernel<128, 192, 2", (130, 65656, 64), MODES), ("linear_kernel<128, 192, 2", (21778, 264, 128), [PLAIN, GELU]),
+           ("linear_kernel<128, 64, 2", (16795, 200, 64), MODES), ("linear_kernel<128, 64, 2", (21851, 392, 128), [PLAIN, GELU]),
+           ("linear_kernel<128, 64, 2", (4097, 712, 640), [PLAIN, GELU]), ("linear_kernel<128, 64, 2", (33, 72, 64), [GELU_PAIR]),
+           ("linear_kernel<64, 64, 4", (33, 72, 64), [PLAIN, PAIR, GELU]), ("linear_kernel<64, 64, 4", (2049, 776, 3072), [PLAIN, GELU]),
+           ("linear_kernel<64, 64, 4", (33, 65680, 128), [PAIR]),
+           ("linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>", (19121, 72, 576), [PLAIN, GELU]),
+           ("linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>", (8200, 72, 640), [PAIR]),
+           ("linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>", (4095, 760, 3072), [PLAIN, GELU]),
+           ("linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>", (2497, 1144, 1152), [PLAIN, GELU]),
+           ("linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>", (1024, 1528, 768), [PAIR]),
+           ("linear_walk_kernel<dmf::WalkTile<4, 2, 2, 3, 3>", (23318, 392, 192), MODES),
+           ("linear_walk_kernel<dmf::WalkTile<4, 2, 2, 3, 3>", (24656, 200, 64), MODES),
+           ("linear_walk_kernel<dmf::WalkTile<4, 2, 2, 3, 3>", (4000, 1016, 1152), MODES),
+           ("linear_walk_kernel<dmf::WalkTile<4, 3, 2, 3, 2>", (26350, 520, 128), MODES),
+           ("linear_walk_kernel<dmf::WalkTile<4, 3, 2, 3, 2>", (2049, 2296, 768), MODES),
+           ("linear_walk_kernel<dmf::WalkTile<4, 3, 2, 3, 2>", (7321, 1144, 1152), MODES)]
+
+
+def planned(M, N, K, jvp, gelu):
+    name = ctypes.create_string_buffer(128)
+    assert _lib.load().dmf_linear_fwd_plan(M, N, K, jvp, gelu, name, len(name)) == 0
+    return name.value.decode()
+
+
+@pytest.mark.parametrize("kernel,size,modes", REACHED)
+def test_every_kernel(kernel, size, modes):
+    M, N, K = size
+    x, tx, w, b = _operands(M, N, K)
+    ref, tref = torch.nn.functional.linear(x.float(), w.float(), b.float()), tx.float() @ w.float().t()
+    act, tact = torch.func.jvp(lambda t: torch.nn.functional.gelu(t, approximate="tanh"), (ref.double(),), (tref.double(),))
+    for jvp, gelu in modes:
+        assert planned(M, N, K, jvp, gelu) == f"dmf::{kernel}, {gelu + (jvp and gelu)}>"
+        y, ty = _call(x, tx if jvp else None, w, b, gelu)
+        for got, exp in ((y, act if gelu else ref), (ty, tact if gelu else tref)):
+            if got is not None:
+                _check(got, exp)
+
+
+def test_the_plan_refuses_what_the_entry_refuses():
+    plan, name = _lib.load().dmf_linear_fwd_plan, ctypes.create_string_buffer(4)
+    for size in ((64, 64, 32), (64, 60, 64), (0, 64, 64), (2 ** 25, 64, 64)):
+        assert plan(*size, 0, 0, name, len(name)) == -3
+    assert plan(64, 64, 64, 0, 0, None, 0) == -5
+    assert plan(64, 64, 64, 0, 0, name, len(name)) == 0 and name.value == b"dmf"   # (cut to the buffer)
