@@ -169,6 +169,9 @@ class SiluFunc(torch.autograd.Function):
         if gy is None:
             return None, None, None
         (x,) = ctx.saved_tensors
+        if torch.is_grad_enabled():   # differentiated again: operators that can be
+            s = torch.sigmoid(x)
+            return gy.to(x.dtype) * (s * (1 + x * (1 - s))), None, None
         return _lib.silu_bwd(gy, x), None, None
 
 
@@ -255,13 +258,16 @@ class DualLinearFunc(torch.autograd.Function):
         want_gx, want_gw = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
         want_gb = ctx.bias_dtype is not None and ctx.needs_input_grad[3]
         gx = gw = gb = None
+        again = torch.is_grad_enabled()   # to be differentiated again: operators that can be
         # (in one stream: next to each other in two, the products slow one another down and each fork and join idles the GPU)
         if want_gw:
             x2 = x.reshape(-1, x.shape[-1]).to(w.dtype)
             if g2.is_cuda and g2.dtype != ctx.weight_dtype and ctx.weight_dtype == torch.float32:
-                own = None if torch.is_grad_enabled() else _lib.linear_wgrad(g2, x2, want_gb and ctx.bias_dtype == torch.float32)
+                own = None if again else _lib.linear_wgrad(g2, x2, want_gb and ctx.bias_dtype == torch.float32)
                 if own is not None:
                     gw, gb = own
+                elif again:
+                    gw = g2.t().float() @ x2.float()
                 else:
                     gw = torch.mm(g2.t(), x2, out_dtype=torch.float32)   # the GEMM stores its fp32 accumulators: no cast kernel
             else:
@@ -269,10 +275,11 @@ class DualLinearFunc(torch.autograd.Function):
         if want_gb and gb is None:
             # torch's multi-block column reduction clears its scratch with a memset node, which does not survive
             # HIP-graph replay; the library's two-stage sum has no such node
-            if g2.is_cuda and g2.shape[1] % 8 == 0:
+            capturing = g2.is_cuda and torch.cuda.is_current_stream_capturing()
+            if g2.is_cuda and g2.shape[1] % 8 == 0 and (capturing or not again):
                 gb = _lib.colsum(g2.contiguous(), ctx.bias_dtype)
             else:
-                if g2.is_cuda and torch.cuda.is_current_stream_capturing():
+                if capturing:
                     raise RuntimeError("dual_linear: the bias gradient of a layer whose output width is not a multiple of 8 falls back "
                                        "to torch's column sum, which does not replay correctly from a captured graph")
                 gb = g2.sum(0).to(ctx.bias_dtype)

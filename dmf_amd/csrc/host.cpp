@@ -767,19 +767,27 @@ py::object activation(const Tensor& x_, Act act) {
   }
   std::shared_ptr<KernelNode> node;
   if (any_grad(x)) {
-    node = make_node(act == Act::gelu ? "GeluTanhBackward" : "SiluBackward", {x}, {xd});
-    node->fn = [act](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
-      const Tensor& x = sv[0];
-      const Tensor gx = dense_like(x);
-      if (act == Act::gelu) {
-        const Tensor gy = dense(g[0].to(x.scalar_type()));
+    if (act == Act::gelu) {
+      node = make_node("GeluTanhBackward", {x}, {xd});
+      node->fn = [](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+        const Tensor& x = sv[0];
+        const Tensor gx = dense_like(x), gy = dense(g[0].to(x.scalar_type()));
         check(dmf_gelu_tanh_bwd(ptr(gy), ptr(x), mptr(gx), x.numel(), code_of(x), stream_of(x)), "dmf_gelu_tanh_bwd");
-      } else {
-        const Tensor gy = dense(g[0]);
+        return {gx};
+      };
+    } else {
+      node = make_node("SiluBackward", {x}, {x.var});   // (the variable itself, for create_graph=True)
+      node->torch_ops = true;
+      node->fn = [](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
+        if (!KernelNode::plain_call({g[0]})) {
+          const Tensor s = at::sigmoid(sv[0]);
+          return {g[0].to(sv[0].scalar_type()) * (s * (1 + sv[0] * (1 - s)))};
+        }
+        const Tensor x = dense(in_memory(sv[0])), gx = dense_like(x), gy = dense(g[0]);
         check(dmf_silu_bwd(ptr(gy), ptr(x), mptr(gx), x.numel(), code_of(x), code_of(gy), stream_of(x)), "dmf_silu_bwd");
-      }
-      return {gx};
-    };
+        return {gx};
+      };
+    }
   }
   return py::cast(finish(y, ty, node, level));
 }

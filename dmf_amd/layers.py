@@ -141,6 +141,17 @@ def timestep_embedding(t: Tensor, dim: int, max_period: int = 10000) -> Tensor:
     return emb
 
 
+class _TimestepSiLU(SiLU):
+    """``SiLU`` that leaves to torch what its kernel does not take (CPU tensors, other types, sizes no multiple of 8), as the embedder's MLP always
+    could."""
+
+    def forward(self, x: Tensor) -> Tensor:
+        types = {x.dtype, torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype}
+        if x.is_cuda and x.numel() and x.numel() % 8 == 0 and types <= {torch.float32, torch.bfloat16}:
+            return super().forward(x)
+        return torch.nn.functional.silu(x)
+
+
 class TimestepEmbedder(nn.Module):
     """Reference models/layers.py:59-71."""
 
@@ -150,7 +161,7 @@ class TimestepEmbedder(nn.Module):
         super().__init__()
         self.emb_size = emb_size
         self.fused = _check_block_ops(block_ops)
-        self.mlp = nn.Sequential(Linear(emb_size, hidden_size, block_ops=block_ops), SiLU(block_ops),
+        self.mlp = nn.Sequential(Linear(emb_size, hidden_size, block_ops=block_ops), _TimestepSiLU(block_ops),
                                  Linear(hidden_size, hidden_size, block_ops=block_ops))
 
     def forward(self, t: Tensor) -> Tensor:

@@ -404,6 +404,36 @@ def test_timestep_embedder_of_a_single_time():
     assert torch.equal(emb(t), emb(t[None]))
 
 
+@pytest.mark.parametrize("native", [True, False])
+def test_timestep_embedder_takes_what_the_plain_one_takes(native, monkeypatch):
+    """Types, devices and batches its kernels have no form for: the plain embedder's values.  Differentiated twice: those of fp64."""
+    from dmf_amd import _lib
+    from dmf_amd.layers import TimestepEmbedder
+    if not native:
+        monkeypatch.setattr(_lib, "native", lambda *t: False)
+    # (60: rows that are no multiple of eight values)
+    for dtype, device, width, n in ((torch.float16, DEV, 64, 4), (torch.float64, DEV, 64, 4), (torch.float32, "cpu", 64, 4), (torch.float32, DEV, 60, 3),
+                                    (torch.bfloat16, "cpu", 64, 4)):
+        emb, plain = (TimestepEmbedder(width, block_ops=b).to(device, dtype) for b in ("hip", "torch"))
+        plain.load_state_dict(emb.state_dict())
+        t = torch.rand(n, device=device).to(dtype)
+        tol = 1e-5 if dtype == torch.float32 else 1e-12 if dtype == torch.float64 else 6e-3
+        for got, ref in zip(torch.func.jvp(emb, (t,), (t,)), torch.func.jvp(plain, (t,), (t,))):
+            assert got.dtype == ref.dtype and ao.rel_l2(got.double().cpu(), ref.double().cpu()) <= tol
+    emb, plain = TimestepEmbedder(64, block_ops="hip").to(DEV), TimestepEmbedder(64).to(DEV).double()
+    plain.load_state_dict(emb.state_dict())
+    t = torch.rand(5, device=DEV)
+
+    def second(model, t):
+        leaves = [t.requires_grad_(), *model.parameters()]
+        first = torch.autograd.grad(model(t).square().sum(), leaves, create_graph=True)
+        return torch.autograd.grad(sum(g.square().sum() for g in first), leaves)
+
+    # (sums of fp32 products and the expressions' fp32 angles: 1e-5 of a gradient, twice)
+    for got, ref in zip(second(emb, t.clone()), second(plain, t.double())):
+        assert ao.rel_l2(got.double().cpu(), ref.cpu()) <= 4e-5
+
+
 def test_timestep_embedding_refuses():
     from dmf_amd import _lib
     call, p = _lib.load().dmf_timestep_embedding_fwd, torch.zeros(8, device=DEV).data_ptr()
