@@ -97,10 +97,13 @@ struct Arg {
 
 // What the kernels can read by address: a view that stands for its buffer's negative (torch._neg_view, the imaginary part of a conjugate) and
 // a zero tensor without storage are made into ordinary ones.
-Tensor in_memory(Tensor t) {
-  if (!t.is_neg() && !t._is_zerotensor()) return t;
+C10_NOINLINE Tensor made_ordinary(const Tensor& t) {
   const Below below;
   return t._is_zerotensor() ? at::zeros(t.sizes(), t.options()) : t.resolve_neg();
+}
+inline Tensor in_memory(Tensor t) {
+  if (C10_UNLIKELY(t.is_neg() || t._is_zerotensor())) return made_ordinary(t);
+  return t;
 }
 
 Arg unpack(const Tensor& x) {
