@@ -65,6 +65,8 @@ FUSED_SIGNATURES = {
     "dmf_linear_plan": (c_int, [_L] + [_I] * 4),
     "dmf_linear_fwd": (c_int, [_P] * 6 + [_I] * 4 + [_P]),
     "dmf_linear_fwd_plan": (c_int, [_L] + [_I] * 4 + [ctypes.c_char_p, _I]),
+    "dmf_linear_dgrad_plan": (c_int, [_L] + [_I] * 2),
+    "dmf_linear_dgrad": (c_int, [_P] * 3 + [_I] * 3 + [_P]),
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
     "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
     "dmf_linear_wgrad": (c_int, [_P] * 5 + [_I] * 3 + [_P]),
@@ -702,6 +704,23 @@ def linear_wgrad(g, x, bias: bool = False):
         ws = _empty((need,), torch.float32, g.device) if need else None
         _check(load().dmf_linear_wgrad(_ptr(g), _ptr(x), _ptr(gw), _ptr(gb), _ptr(ws), M, N, K, _stream(g)), "dmf_linear_wgrad")
     return gw, gb
+
+
+def linear_dgrad(g, w):
+    """``g w`` in bf16 for (M, N) g and (N, K) w by the package's own kernel; None where a library product is the better choice or the operands
+    are not plain dense bf16 tensors on the GPU."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous()
+                   or t.is_neg() or t._is_zerotensor() or t.data_ptr() % 16 for t in (g, w))
+            or torch._C._functorch.peek_interpreter_stack() is not None):
+        return None
+    (M, N), K = g.shape, w.shape[1]
+    if max(M, N, K) > 0x7fffffff or w.shape[0] != N or w.device != g.device or not load().dmf_linear_dgrad_plan(M, N, K):
+        return None
+    with torch.cuda.device(g.device):
+        gx = _empty((M, K), g.dtype, g.device)
+        _check(load().dmf_linear_dgrad(_ptr(g), _ptr(w), _ptr(gx), M, N, K, _stream(g)), "dmf_linear_dgrad")
+    return gx
 
 
 def colsum(x, out_dtype=None):

@@ -284,7 +284,8 @@ class DualLinearFunc(torch.autograd.Function):
                                        "to torch's column sum, which does not replay correctly from a captured graph")
                 gb = g2.sum(0).to(ctx.bias_dtype)
         if want_gx:
-            gx = (g2 @ w).reshape(x.shape).to(x.dtype)
+            gx = None if again else _lib.linear_dgrad(g2, w)
+            gx = (g2 @ w if gx is None else gx).reshape(x.shape).to(x.dtype)
         return gx, None, gw, gb, None, None
 
 

@@ -828,12 +828,28 @@ Tensor column_sum(const Tensor& x, at::ScalarType dt) {
   return out;
 }
 
+bool readable16(const Tensor& t) {
+  return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+}
+
+// g w: the package's own kernel where it reads the operands as they are and is the faster one, else a library product
+Tensor input_gradient(const Tensor& g, const Tensor& w) {
+  // (w comes out of a saved variable, whose hooks may hand back whatever a product takes)
+  const auto ordinary = [](const Tensor& t) {
+    return t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && !t.is_neg() && !t._is_zerotensor() && !t.key_set().has(c10::DispatchKey::Python);
+  };
+  const int64_t M = g.size(0), N = g.size(1), K = w.dim() == 2 ? w.size(1) : 0;
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || w.dim() != 2 || w.size(0) != N || !dmf_linear_dgrad_plan(M, (int)N, (int)K) || !ordinary(g) || !ordinary(w) ||
+      w.device() != g.device() || !readable16(g) || !readable16(w))
+    return at::mm(g, w);
+  const Tensor gx = empty({M, K}, at::kBFloat16, g);
+  check(dmf_linear_dgrad(ptr(g), ptr(w), mptr(gx), (int)M, (int)N, (int)K, stream_of(g)), "dmf_linear_dgrad");
+  return gx;
+}
+
 // g^T x in fp32 and, with `gb`, the column sums of g: the package's own kernel where it reads the operands as they are, else a library
 // product that stores its accumulators (and no sums).
 Tensor weight_gradient(const Tensor& g, const Tensor& x, Tensor* gb) {
-  const auto readable16 = [](const Tensor& t) {
-    return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
-  };
   const int64_t M = g.size(0), N = g.size(1), K = x.size(1);
   if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !readable16(g) || !readable16(x) || !dmf_linear_wgrad_plan(M, (int)N, (int)K))
     return at::mm(g.t(), x, at::kFloat);
@@ -869,7 +885,7 @@ variable_list linear_backward(KernelNode& node, const Tensor& x, const Tensor& w
     else gw = at::mm(g2.t(), x2).to(w_type);
   }
   if (want_gb && !gb.defined()) gb = column_sum(dense(g2), b_type);
-  if (want_gx) gx = at::mm(g2, w).reshape(x.sizes()).to(x.scalar_type());
+  if (want_gx) gx = input_gradient(g2, w).reshape(x.sizes()).to(x.scalar_type());
   return {gx, gw, gb};
 }
 
@@ -931,9 +947,6 @@ bool linear_ok(const Arg& x, const Arg& weight, const Arg& bias) {
 // The package's own product kernel (dmf_linear_fwd) where it reads the operands as they are and is the faster one: y, and ty with a
 // tangent.  False: nothing done.
 bool own_linear(const Tensor& x2, const Tensor& tx2, const Tensor& w, const Tensor& b, bool gelu, Tensor& y, Tensor& ty) {
-  const auto readable16 = [](const Tensor& t) {
-    return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
-  };
   const int64_t M = x2.size(0), N = w.size(0), K = w.size(1);
   if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !dmf_linear_plan(M, (int)N, (int)K, tx2.defined(), gelu) || !readable16(x2) || !readable16(w) ||
       (tx2.defined() && !readable16(tx2)) || (b.defined() && (!readable16(b) || b.numel() != N)))

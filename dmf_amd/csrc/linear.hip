@@ -227,6 +227,10 @@ __device__ __forceinline__ void lds_write64(uint32_t addr, u32x2 v) { asm volati
 // (after a wait: keeps uses of what has been read behind it)
 __device__ __forceinline__ void landed_in(u32x4& v) { asm volatile("" : "+v"(v)); }
 
+__device__ __forceinline__ void landed_in(TrPair& v) { asm volatile("" : "+v"(v.lo), "+v"(v.hi)); }
+__device__ __forceinline__ bf16x8 as_operand(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
+__device__ __forceinline__ bf16x8 as_operand(const TrPair& v) { return __builtin_bit_cast(bf16x8, tr_operand(v).v); }
+
 template <class F, int... I>
 __device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f) {
   (f(std::integral_constant<int, I>{}), ...);
@@ -250,7 +254,7 @@ struct WalkTile {
 
 constexpr int kNonTemporal = 2;   // (buffer instructions' aux bits)
 
-template <class T, int MODE>
+template <class T, int MODE, bool COLS = false>
 __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   constexpr int MT = T::MT, NT = T::NT, BM = T::BM, BN = T::BN;
   constexpr bool BOTH = MODE == kLinGeluJvp;
@@ -297,6 +301,17 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   for (int j = 0; j < (T::PX > T::PW ? T::PX : T::PW); ++j)
     voff[j] = (32 * j + 8 * wave + drow) * kb + (((lane & 7) ^ ((4 * (wave & 1) + (drow >> 1)) & 7)) * 16);
   // the stages being requested, of x (with tx) and of w: tile, step, slot
+  // COLS: w is (K, N) and a stage 64 of its rows, in panels of 64 columns (128-byte lines) of 8 KB each; a request is 8 rows of one panel.  The 64-byte
+  // halves of rows 4 i + 2 and 4 i + 3 are exchanged: 32 lanes of a transposed read take 64 bytes of four consecutive rows, and meet all 64 banks.
+  const uint32_t nb = (uint32_t)p.N * 2;
+  uint32_t wvoff[COLS ? T::PW : 1];
+  if constexpr (COLS) {
+#pragma unroll
+    for (int j = 0; j < T::PW; ++j) {
+      const int b = 4 * j + wave;
+      wvoff[j] = (8 * (b & 7) + drow) * nb + (b >> 3) * 128 + (((lane & 7) ^ ((drow >> 1 & 1) * 4)) * 16);
+    }
+  }
   struct Cursor { uint32_t nth, slot; int step; };
   Cursor cx{0, 0, 0}, cw{0, 0, 0};
   __amdgpu_buffer_rsrc_t rx, rtx, rw;
@@ -307,7 +322,9 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   };
   auto aim_w = [&](uint32_t id) {
     const Place t = place(id);
-    rw = make_rows_rsrc(p.w + (int64_t)t.n0 * p.K, kb, min(BN, p.N - t.n0), (int)kb);
+    // (COLS: columns past the last are those of the next row, or zeros behind the last one, and their results are not stored)
+    if constexpr (COLS) rw = make_rows_rsrc(p.w + t.n0, nb, p.K, (int)(nb - t.n0 * 2));
+    else rw = make_rows_rsrc(p.w + (int64_t)t.n0 * p.K, kb, min(BN, p.N - t.n0), (int)kb);
   };
   auto request_x = [&](int j) {   // a wave's j-th KB of the stage
     char* dst = smem + cx.slot * T::XS + (4 * j + wave) * 1024;
@@ -316,7 +333,8 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   };
   auto request_w = [&](int j) {
     char* dst = smem + T::NSX * T::XS + cw.slot * T::WS + (4 * j + wave) * 1024;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)dst, 16, voff[j], cw.step * 128, 0, 0);
+    if constexpr (COLS) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)dst, 16, wvoff[j], cw.step * 64 * nb, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)dst, 16, voff[j], cw.step * 128, 0, 0);
   };
   // (past the last tile's last step the requests go on -- bytes of other rows, or zeros -- so that the number in flight is constant; nothing
   //  reads them, and the kernel's end waits for them)
@@ -328,6 +346,8 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
         ++c.nth;
         c.step = 0;
         aim(next);
+      } else if constexpr (COLS) {
+        --c.step;   // (rows of w past its last one would be addressed: the last step's again)
       }
     }
   };
@@ -340,18 +360,31 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     xaddr[c] = lds_addr(smem) + (wm * 32 + c32) * 128 + k;
     waddr[c] = lds_addr(smem) + T::NSX * T::XS + (wn * 32 * NT + c32) * 128 + k;
   }
+  // COLS: of column group i, rows 8 g .. + 3 of a chunk's 16 (the other four: + 512), so that a lane's slots are those of its rows of x
+  static_assert(!COLS || NT <= 4);
+  if constexpr (COLS) {
+    const uint32_t i16 = lane & 15, in_panel = (8 * g + (i16 >> 2)) * 128 + ((lane >> 4) & 1) * 32 + (i16 & 3) * 8, swap = (i16 >> 3) & 1;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const uint32_t c = wn * NT + i;
+      waddr[i] = lds_addr(smem) + T::NSX * T::XS + (c >> 1) * 8192 + in_panel + ((c & 1) ^ swap) * 64;
+    }
+  }
+  constexpr int WREADS = COLS ? 2 : 1;   // LDS reads of an operand of w
   constexpr int AHEAD = T::AHEAD, BUFS = 2 * AHEAD;
-  u32x4 X[BUFS][MT], W[BUFS][NT];
+  u32x4 X[BUFS][MT];
+  std::conditional_t<COLS, TrPair, u32x4> W[BUFS][NT];
   uint32_t xslot = 0, wslot = 0;   // of the stage being read
   auto read = [&](auto cc, auto ii) {   // operand ii of chunk cc
     constexpr int c = decltype(cc)::value, i = decltype(ii)::value, b = c % BUFS;
-    if constexpr (i < NT) W[b][i] = lds_read128_issue<i * 4096>(waddr[c] + wslot * T::WS);
+    if constexpr (i < NT && COLS) W[b][i] = lds_tr16_issue<c * 2048, c * 2048 + 512>(waddr[i] + wslot * T::WS);
+    else if constexpr (i < NT) W[b][i] = lds_read128_issue<i * 4096>(waddr[c] + wslot * T::WS);
     else X[b][i - NT] = lds_read128_issue<((i - NT) % MX * 32 * T::WM + (i - NT) / MX * ROWS) * 128>(xaddr[c] + xslot * T::XS);
   };
   auto landed = [&](auto cc, auto rows) {   // chunk cc's operands; where stages change, all that are read
     constexpr int c = decltype(cc)::value, b = c % BUFS;
     if constexpr (AHEAD == 1 || c == T::LAST + 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MT + NT) : "memory");
+    else asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MT + NT * WREADS) : "memory");
 #pragma unroll
     for (int i = 0; i < NT; ++i) landed_in(W[b][i]);
 #pragma unroll
@@ -391,7 +424,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       }
       for_each(std::make_integer_sequence<int, NM>{}, [&](auto ii) {
         constexpr int i = decltype(ii)::value, n = i / MA, m = i % MA;
-        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, W[c % BUFS][n]), __builtin_bit_cast(bf16x8, X[c % BUFS][m]),
+        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_operand(W[c % BUFS][n]), as_operand(X[c % BUFS][m]),
                                                             FIRST && c == 0 ? f32x16{0} : acc[n][m], 0, 0, 0);
         constexpr int SLOTS = NM < R ? NM : R, r0 = i < SLOTS ? i * R / SLOTS : R, r1 = i < SLOTS ? (i + 1) * R / SLOTS : R;
         for_each(std::make_integer_sequence<int, r1 - r0>{}, [&](auto rr) {
@@ -437,7 +470,6 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
 
   // Output rows leave two accumulator tiles at a time through this wave's 4 KB of LDS (32 rows of 128 bytes, slot v of row r holding vector
   // v ^ r / 2 % 8), in whole 16-byte vectors; while one pass is on its way through LDS the next one is computed.
-  const uint32_t nb = (uint32_t)p.N * 2;
   const uint32_t own = lds_addr(smem) + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
   const uint32_t put = own + c32 * 128 + ((c32 >> 1) & 7) * 16 + g * 8;
   const uint32_t get = own + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 4)) * 16);   // rows + 8 i: slot ^ 4 i % 8
@@ -562,6 +594,26 @@ static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
   return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
 }
 
+// The input gradient gx = g W: the same walk with w read by columns, contracted over its rows as they lie in memory.  The library's products ran at
+// 560 to 910 TFLOP/s here (C1152 M8192: 3C -> C 84.6 us, C -> C 38.7, 4C -> C 108, C -> 4C 97.5); these at 850 to 1080 (63.4, 27.0, 83.7, 81.1), bounded like
+// the forward's by the address unit and the tiles' ends: transposed reads of w take as many bytes out of LDS as rows of it.
+template <class T>
+__global__ __launch_bounds__(256, 1) void linear_dgrad_kernel(const LinearParams p) {
+  linear_walk<T, kLinPlain, true>(p);
+}
+
+template <class T>
+static int launch_dgrad(LinearParams& p, hipStream_t stream) {
+  auto kern = linear_dgrad_kernel<T>;
+  static bool lds_ok[64] = {};
+  if (!ensure_dynamic_lds(kern, T::LDS, lds_ok)) return -7;
+  p.mtiles = (p.M + T::BM - 1) / T::BM;
+  p.ntiles = (p.N + T::BN - 1) / T::BN;
+  const int64_t tiles = (int64_t)p.mtiles * p.ntiles, cus = compute_units();
+  const int64_t grid = tiles >= cus ? cus : T::MT % 2 == 0 && 2 * tiles <= cus ? 2 * tiles : tiles;
+  return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
+}
+
 // Tile policy: the shortest of the estimates, in 10 ns, of six kernels.  linear_kernel: a K step (64) and a work-group's start and end with one,
 // two, three work-groups on a CU, more of them never taking less; linear_walk_kernel: a step and what a tile takes beyond its steps at that
 // pace, of whole and of half a tile, and the launch's.  Fitted to 1440 products of
@@ -579,6 +631,11 @@ constexpr bool never_shorter_with_more(const LinTile& t) {
 static_assert(never_shorter_with_more(kLinTiles[0]) && never_shorter_with_more(kLinTiles[1]) && never_shorter_with_more(kLinTiles[2]));
 struct LinWalk { int bm, bn, a, b, a_half, b_half, launch; };
 constexpr LinWalk kLinWalks[2] = {{256, 192, 94, 607, 59, 433, 136}, {256, 128, 73, 386, 45, 413, 135}};
+
+static int64_t walk_cost(const LinWalk& c, int64_t M, int64_t N, int64_t steps, int products, bool halves) {
+  const int64_t cus = compute_units(), tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * products, rest = tiles % cus;
+  return c.launch + tiles / cus * (c.a * steps + c.b) + (rest == 0 ? 0 : halves && 2 * rest <= cus ? c.a_half * steps + c.b_half : c.a * steps + c.b);
+}
 
 // A gelu pair holds an element of x and its tangent in one wave, half of the rows of each: it has as many work-groups as a single product of twice
 // the rows, takes the tiles with two row tiles per wave, and whole ones.
@@ -613,12 +670,7 @@ static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
     if (tiles <= cus) take(5, 534 + (31 * cus + 14 * std::max<int64_t>(0, tiles - cus / 2)) * steps / cus);
   }
   // (the walking kernel's row offsets within a tile are 32-bit)
-  for (int t = 0; t < 2 && N <= 65536 && K <= 65536; ++t) {
-    const LinWalk& c = kLinWalks[t];
-    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * (jvp ? 2 : 1), rest = tiles % cus;
-    const bool half = !both && 2 * rest <= cus;
-    take(3 + t, c.launch + tiles / cus * (c.a * steps + c.b) + (rest == 0 ? 0 : half ? c.a_half * steps + c.b_half : c.a * steps + c.b));
-  }
+  for (int t = 0; t < 2 && N <= 65536 && K <= 65536; ++t) take(3 + t, walk_cost(kLinWalks[t], M, N, steps, jvp ? 2 : 1, !both));
   return best;
 }
 
@@ -704,6 +756,45 @@ extern "C" int dmf_linear_fwd(const void* x, const void* tx, const void* w, cons
   const int tile = dmf::linear_tile(M, N, K, jvp, gelu != 0);
   if (jvp && gelu) return dmf::launch_linear_tile<dmf::kLinGeluJvp>(tile, p, true, stm);
   return gelu ? dmf::launch_linear_tile<dmf::kLinGelu>(tile, p, false, stm) : dmf::launch_linear_tile<dmf::kLinPlain>(tile, p, jvp, stm);
+}
+
+static bool dgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
+  constexpr int64_t most = (int64_t)1 << 30;   // (and rows within a tile are addressed in 32 bits)
+  return M >= 1 && M <= INT32_MAX && N >= 64 && N % 64 == 0 && K >= 8 && K % 8 == 0 && N <= 65536 && K <= 65536 && M * N <= most && N * K <= most && M * K <= most;
+}
+
+// Which input gradients the walking kernel is the faster one for, N -> K (us on the GPU, library -> here; 318 products of widths 384 to 1152, 64 to 32768
+// rows; the 193 it takes need 0.88 of the library's time in the mean, and 5 us of host time where that takes 18):
+//   from 3072 rows on (2048 where a row of tiles is not mostly idle or cut): C768 M4096 3C -> C 29.9 -> 23.1, M16384 62.8 -> 55.0; C1152 M16384 157 -> 118;
+//     C384 M16384 26.4 -> 19.7; but C384 M2048 10.8 against 12.9, C1024 M2048 26.4 against 28.5, C768 M1536 17.6 against 21.5;
+//   C -> 4C from 768 rows on: C768 M1024 14.4 -> 11.3, C1152 24.7 -> 16.3; not with one to 4/3 rounds of 256 x 192 tiles: C768 M5120 28.2 against 30.6,
+//     C1024 M3072 28.5 against 32.6;
+//   widths that 192 columns do not divide lose in many rows: C1024 M12288 3C -> C 71.6 against 81.5, M16384 89.4 against 94.6 (M8192 59.0 -> 49.6).
+extern "C" int dmf_linear_dgrad_plan(int64_t M, int N, int K) {
+  if (!dgrad_shape_ok(M, N, K) || M < 768) return 0;
+  if (K >= 3 * (int64_t)N) {
+    const int64_t cus = dmf::compute_units(), tiles = ((M + 255) / 256) * ((K + 191) / 192);
+    return tiles <= cus || 3 * tiles > 4 * cus;
+  }
+  if (M < 3072 && (M < 2048 || K < 512 || K % 192 != 0)) return 0;
+  return K % 192 == 0 || M < 10240;
+}
+
+extern "C" int dmf_linear_dgrad(const void* g, const void* w, void* gx, int M, int N, int K, void* stream) {
+  if (g == nullptr || w == nullptr || gx == nullptr) return DMF_ATTN_ENULL;
+  if (!dgrad_shape_ok(M, N, K)) return DMF_ATTN_ESHAPE;
+  for (const void* q : {g, w, (const void*)gx})
+    if (reinterpret_cast<uintptr_t>(q) % 16) return DMF_ATTN_EALIGN;
+  dmf::LinearParams p{};
+  p.x[0] = static_cast<const __bf16*>(g);
+  p.w = static_cast<const __bf16*>(w);
+  p.y[0] = static_cast<__bf16*>(gx);
+  p.M = M; p.N = K; p.K = N;   // (of the product: columns of the result, depth)
+  auto stm = static_cast<hipStream_t>(stream);
+  // (the forward's estimates: on the products above the tile they choose takes 0.4 % more than the faster of the two in the mean)
+  return dmf::walk_cost(dmf::kLinWalks[0], M, K, N / dmf::kLinK, 1, true) <= dmf::walk_cost(dmf::kLinWalks[1], M, K, N / dmf::kLinK, 1, true)
+             ? dmf::launch_dgrad<dmf::WalkTile<4, 3, 2, 3, 2>>(p, stm)
+             : dmf::launch_dgrad<dmf::WalkTile<4, 2, 2, 3, 3>>(p, stm);
 }
 
 namespace dmf {

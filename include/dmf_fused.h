@@ -50,6 +50,13 @@ DMF_ATTN_API int dmf_linear_fwd(const void* x, const void* tx, const void* w, co
                         int gelu, void* stream);
 
 /*
+ * gx = g w, the gradient of a linear layer's input: g (M, N), w (N, K), gx (M, K), bf16 and dense, fp32 accumulation.  N a multiple of 64, K
+ * of 8, both up to 65536, at most 2^30 elements in each; 16-byte aligned.  dmf_linear_dgrad_plan: as dmf_linear_plan.
+ */
+DMF_ATTN_API int dmf_linear_dgrad_plan(int64_t M, int N, int K);
+DMF_ATTN_API int dmf_linear_dgrad(const void* g, const void* w, void* gx, int M, int N, int K, void* stream);
+
+/*
  * gw = g^T x, contracted over the M rows: g (M, N), x (M, K), bf16 and dense, gw (N, K) fp32, fp32 accumulation in a fixed order;
  * gbias (N, fp32) or NULL: the column sums of g besides.
  * N and K multiples of 8, fewer than 2^30 elements in each; 16-byte aligned.  workspace: dmf_linear_wgrad_workspace_floats(M, N, K)

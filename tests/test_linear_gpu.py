@@ -91,6 +91,62 @@ def test_layers_take_it_for_what_it_covers(dual):
                 assert g.shape == e.shape and (g.float() - e).norm() <= 2 * TOL * e.norm(), (i, fn)
 
 
+# ---- input gradient (dmf_linear_dgrad), N -> K: one row, rows and columns that fill no tile, one step per tile and fewer than stages, whole rounds with
+# half tiles behind them, only half tiles, either tile width; exact operands and fp32 sums, so that the bound is the result's rounding
+DGRAD = [(1, 64, 8), (63, 64, 64), (129, 192, 200), (4097, 640, 712), (2049, 768, 2296), (8193, 1152, 1152), (4100, 1024, 1016), (12345, 192, 1016),
+         (16389, 64, 2304), (2300, 448, 3064), (256, 3072, 768), (8192, 4608, 1152)]
+
+
+@pytest.mark.parametrize("M,N,K", DGRAD)
+def test_input_gradient(M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    # (what lies behind the last row of either operand would show if it were summed)
+    g, w = torch.randn(M + 64, N, generator=gen, device=DEV).bfloat16(), (torch.randn(N + 64, K, generator=gen, device=DEV) * N ** -0.5).bfloat16()
+    g[M:], w[N:] = 1e4, 1e4
+    ref, lib = g[:M].float() @ w[:N].float(), _lib.load()
+    for _ in range(2):
+        gx = torch.full((M + 1, K), 7.0, device=DEV, dtype=torch.bfloat16)
+        assert lib.dmf_linear_dgrad(g.data_ptr(), w.data_ptr(), gx.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+        _check(gx[:M], ref)
+        assert (gx[M] == 7.0).all()
+
+
+def test_input_gradient_routes():
+    """A layer's input gradient, native and Python route, for dense, strided and negated gradients and with a saved weight that a hook hands back
+    in another layout: the product of the bf16 operands; the general form where it is differentiated again."""
+    M, N, K = 3072, 384, 768
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV).bfloat16()
+    x, w, dense = r(M, K), (r(N, K) * N ** -0.5).requires_grad_(), r(M, N)
+    assert _lib.load().dmf_linear_dgrad_plan(M, N, K) == 1
+    own = _lib.linear_dgrad(dense, w.detach())
+    _check(own, dense.float() @ w.detach().float())
+    for other in (dense[:, ::2], dense.float(), torch._neg_view(dense), r(N, M).t()):
+        assert _lib.linear_dgrad(other, w.detach()) is None
+    for gy in (dense, r(N, M).t(), torch._neg_view(dense), dense[:1].expand(M, N)):
+        ref = gy.float() @ w.detach().float()
+        a = x.clone().requires_grad_()
+        _check(torch.autograd.grad(block_ops.dual_linear(a, w), a, gy)[0], ref)
+        y, *_ = block_ops.DualLinearFunc.apply(a, None, w, None, None, None)
+        _check(torch.autograd.grad(y, a, gy)[0], ref)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.t().contiguous(), lambda t: t.t()):
+            y = block_ops.dual_linear(a, w)
+        _check(torch.autograd.grad(y, a, gy)[0], ref)
+    a, gy = x.clone().requires_grad_(), dense.clone().requires_grad_()
+    gx = torch.autograd.grad(block_ops.dual_linear(a, w), a, gy, create_graph=True)[0]
+    _check(torch.autograd.grad(gx, gy, x)[0], x.float() @ w.detach().float().t())
+
+
+def test_input_gradient_refuses():
+    g, w, lib = torch.randn(64, 64, device=DEV).bfloat16(), torch.randn(64, 64, device=DEV).bfloat16(), _lib.load()
+    gx = torch.empty(64, 64, device=DEV, dtype=torch.bfloat16)
+    call = lambda g, w, o, M, N, K: lib.dmf_linear_dgrad(g, w, o, M, N, K, None)
+    p, q, o = g.data_ptr(), w.data_ptr(), gx.data_ptr()
+    for size in ((0, 64, 64), (64, 32, 64), (64, 64, 12), (64, 64, 65544), (1 << 25, 64, 8)):
+        assert call(p, q, o, *size) == -3 and lib.dmf_linear_dgrad_plan(*size) == 0
+    assert call(None, q, o, 64, 64, 64) == -5 and call(p + 2, q, o, 64, 64, 64) == -6
+
+
 # ---- weight gradient (dmf_linear_wgrad): products exact in fp32, sums in fp32 -- M terms in some order, error below sqrt(M) 2^-24 of the
 # sum of magnitudes on random data; 2e-6 covers M = 16389 (7.6e-6 of a worst single element, checked against the largest)
 WGRAD = [(1, 8, 8), (63, 64, 64), (64, 128, 192), (65, 136, 200), (129, 120, 184), (333, 1152, 1152), (2048, 384, 1536), (4097, 712, 328),
