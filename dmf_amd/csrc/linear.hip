@@ -939,6 +939,173 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
   }
 }
 
+// Much work: the walking forward kernel's tile, stages and order of reads, products and requests (see linear_walk), of 256 columns of g against 192 of x,
+// a work-group per CU.  Both operands lie in 64-column panels of 64 rows and are read by columns.  A step of 6.3 MFLOP takes 0.8 to 1.2 us, by how many
+// CUs take part (two of linear_wgrad_kernel's, the same work, 1.25); start, end and launch 12 us where that takes 9.  With the partial sums' kernel, M 8192:
+// 4608 x 1152 109 -> 100 us, 3072 x 768 59.6 -> 54.7, 3072 x 1024 79.5 -> 71.5, 1152 x 1152 42.5 -> 40.5; M 16384: 4608 x 1152 207 -> 178.
+// The two waves that hold the same columns of g sum two chunks of a step each for the bias (two thirds of the room between a chunk's products).
+struct WgradWide : WalkTile<4, 3, 2, 3, 2> { static constexpr int STAGES = NSX * XS + NSW * WS; };
+
+__global__ __launch_bounds__(256, 1) void linear_wgrad_wide_kernel(const WgradParams p) {
+  using T = WgradWide;
+  constexpr int MT = T::MT, NT = T::NT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5, i16 = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / T::WN, wn = wave % T::WN;
+  // as in linear_wgrad_kernel: the tiles of one split are neighbours, in bands of six k tiles
+  const uint32_t per = (uint32_t)p.ntiles * p.ktiles, id = xcd_remap(blockIdx.x, gridDim.x), split = id / per, tile = id - split * per;
+  const uint32_t band = tile / (6 * p.ntiles), in = tile - band * 6 * p.ntiles, wide = min((uint32_t)p.ktiles - 6 * band, 6u);
+  const int n0 = (int)(in / wide) * T::BM, k0 = (int)(6 * band + in % wide) * T::BN;
+  const int first = (int)split * p.per, steps = min(p.per, (p.M + 63) / 64 - first);   // (at least one: no split is empty)
+
+  const uint32_t gb = (uint32_t)p.N * 2, xb = (uint32_t)p.K * 2;
+  const __amdgpu_buffer_rsrc_t rg = make_rows_rsrc(p.g + n0, gb, p.M, (int)(gb - n0 * 2));
+  const __amdgpu_buffer_rsrc_t rx = make_rows_rsrc(p.x + k0, xb, p.M, (int)(xb - k0 * 2));
+  uint32_t gvoff[T::PX], xvoff[T::PW];   // a wave's j-th KB of a stage: 8 rows of a panel
+#pragma unroll
+  for (int j = 0; j < T::PX; ++j) {
+    const int b = 4 * j + wave;
+    const uint32_t row = 8 * (b & 7) + (lane >> 3), col = (b >> 3) * 128 + ((lane & 7) ^ (((lane >> 4) & 1) * 4)) * 16;
+    gvoff[j] = row * gb + col;
+    if (j < T::PW) xvoff[j] = row * xb + col;
+  }
+  // steps being requested, and the slots they go to (past the last step: that one again; nothing reads it)
+  int sg = 0, sx = 0;
+  uint32_t gto = 0, xto = 0;
+  auto request_g = [&](int j) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)(smem + gto * T::XS + (4 * j + wave) * 1024), 16, gvoff[j],
+                                             (uint32_t)(first + sg) * 64 * gb, 0, 0);
+  };
+  auto request_x = [&](int j) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(smem + T::NSX * T::XS + xto * T::WS + (4 * j + wave) * 1024), 16,
+                                             xvoff[j], (uint32_t)(first + sx) * 64 * xb, 0, 0);
+  };
+  auto advance_g = [&] { gto = gto + 1 == T::NSX ? 0 : gto + 1; sg = min(sg + 1, steps - 1); };
+  auto advance_x = [&] { xto = xto + 1 == T::NSW ? 0 : xto + 1; sx = min(sx + 1, steps - 1); };
+
+  const uint32_t in_panel = (8 * g + (i16 >> 2)) * 128 + ((lane >> 4) & 1) * 32 + (i16 & 3) * 8, swap = (i16 >> 3) & 1;
+  const uint32_t gaddr = lds_addr(smem) + in_panel + (wm ^ swap) * 64;   // column group 2 m + wm: half wm of panel m
+  uint32_t xaddr[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) xaddr[n] = lds_addr(smem) + T::NSX * T::XS + ((wn * NT + n) >> 1) * 8192 + in_panel + (((wn * NT + n) & 1) ^ swap) * 64;
+  TrPair G[2][MT], X[2][NT];
+  uint32_t gslot = 0, xslot = 0;   // of the stage being read
+  auto read = [&](auto cc, auto ii) {   // operand ii of chunk cc
+    constexpr int c = decltype(cc)::value, i = decltype(ii)::value, b = c % 2;
+    if constexpr (i < NT) X[b][i] = lds_tr16_issue<c * 2048, c * 2048 + 512>(xaddr[i] + xslot * T::WS);
+    else G[b][i - NT] = lds_tr16_issue<(i - NT) * 8192 + c * 2048, (i - NT) * 8192 + c * 2048 + 512>(gaddr + gslot * T::XS);
+  };
+  auto landed = [&](auto bb) {
+    constexpr int b = decltype(bb)::value;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NT; ++i) landed_in(X[b][i]);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) landed_in(G[b][i]);
+  };
+  f32x16 acc[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = f32x16{0};
+  float total[MT] = {};
+  auto stage = [&](auto sums_) {   // sums_: 0, 1: of chunks 0 and 1, or 2 and 3; 2: none
+    float part[MT] = {};
+    for_each(std::make_integer_sequence<int, 4>{}, [&](auto cc) {
+      constexpr int c = decltype(cc)::value, NM = MT * NT, R = MT + NT;
+      landed(std::integral_constant<int, c % 2>{});
+      if constexpr (c == 3) {
+        wait_vm<T::BEHIND>();
+        asm volatile("s_barrier" ::: "memory");   // the next stage is in LDS and everybody has taken its operands of this one
+        gslot = gslot + 1 == T::NSX ? 0 : gslot + 1;
+        xslot = xslot + 1 == T::NSW ? 0 : xslot + 1;
+      }
+      for_each(std::make_integer_sequence<int, NM>{}, [&](auto ii) {
+        constexpr int i = decltype(ii)::value, n = i / MT, m = i % MT;
+        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_operand(X[c % 2][n]), as_operand(G[c % 2][m]), acc[n][m], 0, 0, 0);
+        if constexpr (i < R) read(std::integral_constant<int, (c + 1) % 4>{}, ii);
+        if constexpr (c == 3) {
+#pragma unroll
+          for (int j = i * T::PW / NM; j < (i + 1) * T::PW / NM; ++j) request_x(j);
+        } else {
+          constexpr int at = c * NM + i;
+#pragma unroll
+          for (int j = at * T::PX / (3 * NM); j < (at + 1) * T::PX / (3 * NM); ++j) request_g(j);
+        }
+        if constexpr (decltype(sums_)::value == c / 2 && i >= NM - MT) {
+          constexpr int k = i - (NM - MT);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t pair = tr_operand(G[c % 2][k]).v[e];
+            part[k] += __uint_as_float(pair << 16) + __uint_as_float(pair & 0xffff0000u);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (c == 3) advance_x();
+      if constexpr (c == 2) advance_g();
+    });
+    if constexpr (decltype(sums_)::value < 2) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) total[m] += part[m];
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < T::NSW; ++s) {
+#pragma unroll
+    for (int j = 0; j < T::PW; ++j) request_x(j);
+    advance_x();
+    if (s < T::NSX - 1) {
+#pragma unroll
+      for (int j = 0; j < T::PX; ++j) request_g(j);
+      advance_g();
+    }
+  }
+  wait_vm<(T::NSW - 1) * T::PW + (T::NSX - 2) * T::PX>();
+  asm volatile("s_barrier" ::: "memory");
+  const bool sums = p.bias != nullptr && k0 == 0;
+  auto run = [&](auto sums_) {
+    for_each(std::make_integer_sequence<int, MT + NT>{}, [&](auto ii) { read(std::integral_constant<int, 0>{}, ii); });
+    for (int s = 0; s < steps; ++s) stage(sums_);
+    landed(std::integral_constant<int, 0>{});   // (of a stage past the last: nothing may be under way where control flow meets)
+  };
+  if (!sums) run(std::integral_constant<int, 2>{});
+  else if (wn == 0) run(std::integral_constant<int, 0>{});
+  else run(std::integral_constant<int, 1>{});
+  wait_vm<0>();   // (no DMA may outlive the work-group's LDS)
+
+  if (sums) {   // of both waves, and of the halves of a wave, which hold different rows
+    asm volatile("s_barrier" ::: "memory");
+    float* both = reinterpret_cast<float*>(smem) + wm * MT * 64;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      if (wn == 1) both[m * 64 + lane] = total[m];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int row = n0 + 64 * m + 32 * wm + c32;
+      float t = total[m] + both[m * 64 + lane];
+      t += __shfl_xor(t, 32);
+      if (wn == 0 && g == 0 && row < p.N) p.bias[(int64_t)split * p.N + row] = t;
+    }
+  }
+  float* out = p.out + (int64_t)split * p.N * p.K;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = n0 + 64 * m + 32 * wm + c32;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int col = k0 + 96 * wn + 32 * n + 8 * q + 4 * g;
+        const f32x16& a = acc[n][m];
+        if (row < p.N && col < p.K)
+          *reinterpret_cast<f32x4*>(out + (int64_t)row * p.K + col) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+      }
+  }
+}
+
 // out = the sum of `splits` arrays of 4 n4 floats, in order; behind them, arrays of 4 b4 floats into bias
 struct SumSplitsParams { const f32x4* part; f32x4 *out, *bias; int64_t n4, b4; int splits; };
 __global__ __launch_bounds__(256) void sum_splits_kernel(const SumSplitsParams p) {
@@ -978,6 +1145,27 @@ static int wgrad_splits(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+// Splits for linear_wgrad_wide_kernel, 0 where linear_wgrad_kernel is the better one: below 8 G multiply-adds, measured on 160 products (3072 x 768: M 3072 -5 %,
+// 768 x 768: M 12288 +2 %, M 16384 -2 %; 1152 x 1152: M 4096 +6 %, M 6144 -11 %).  Estimates fitted to those, in 10 ns; all work-groups at once; chains
+// of sums no longer than that kernel's.
+static int wgrad_wide_splits(int64_t M, int64_t N, int64_t K) {
+  if (M * N < 8000000000 / K) return 0;
+  const int64_t cus = compute_units(), tiles = ((N + WgradWide::BM - 1) / WgradWide::BM) * ((K + WgradWide::BN - 1) / WgradWide::BN), total = (M + 63) / 64;
+  int best = 0;
+  int64_t cost_best = INT64_MAX;
+  for (int64_t s = wgrad_splits(M, N, K); s <= 64 && s <= total && tiles * s <= cus; ++s) {
+    const int64_t per = (total + s - 1) / s;
+    if ((s - 1) * per >= total) continue;   // (a split would be empty)
+    int64_t cost = per * (77 * cus + 46 * tiles * s) / cus + 173 * tiles * s / cus;
+    if (s > 1) cost += N * K * 4 * (2 * s + 1) / 152000 + 396;
+    if (cost < cost_best) {
+      cost_best = cost;
+      best = (int)s;
+    }
+  }
+  return best;
+}
+
 static bool wgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 8 || N % 8 || K < 8 || K % 8 || M * K >= (int64_t)1 << 30 || N * K >= (int64_t)1 << 30 || M * N >= (int64_t)1 << 30) return false;
   // rows up to the end of the last step are addressed too, in 32 bits: wrapped around, one past the last would be read, not be zero
@@ -988,7 +1176,7 @@ static bool wgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
 
 extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
   if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return -1;
-  const int s = dmf::wgrad_splits(M, N, K);
+  const int wide = dmf::wgrad_wide_splits(M, N, K), s = wide ? wide : dmf::wgrad_splits(M, N, K);
   return s > 1 ? (int64_t)s * N * (K + 1) : 0;
 }
 
@@ -997,24 +1185,23 @@ extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
 //   9.3 .. 12.4 -> 6.3 .. 7.1, 4608 x 768 12.5 .. 15.3 -> 8.0 .. 8.8, 6912 x 1152 16.3 .. 22.0 -> 12.3 .. 14.1;  M 512: 768 x 768 15.2 -> 12.4,
 //   4608 x 1152 27.1 -> 15.5;  M 1000: 768 x 768 20.5 -> 15.9, 4608 x 1152 38.9 -> 23.3;  M 1472: 3072 x 768 30.5 -> 27.7, 3456 x 1152 32.8 -> 29.0;
 //   M 2048: 1536 x 384 20.0 -> 18.4, but 2304 x 768 21 against 23, 3456 x 1152 28 against 34;
-//   M 4096: 3072 x 768 42 -> 36, 1152 x 1152 33 -> 25, but 3456 x 1152 46 against 51;  M 8192: 3456 x 1152 83 -> 81, 4608 x 1152 119 -> 101,
-//   1152 x 4608 118 -> 97, 1152 x 1152 61 -> 36, 768 x 768 48 -> 24;  M 16384: 3072 x 768 172 -> 94, 4608 x 1152 327 -> 183 (948 TFLOP/s);
-//   widths that 192 columns do not divide lose on large results: 4096 x 1024 M 8192 86 against 89.  The largest result
-//   measured is 6912 x 1152 (8 M elements); beyond it the library's products are kept.
+//   M 4096: 3072 x 768 44 -> 37, 1152 x 1152 35 -> 30, 3072 x 1024 47 -> 46, 4608 x 1152 67 -> 62, but 3456 x 1152 50 against 53, 4096 x 1024 50 against 55;
+//   M 6144: 3456 x 1152 69 against 71, 4608 x 1152 97 -> 81, 4096 x 1024 77 -> 75, 1024 x 4096 80 -> 76 (and no column sum beside it);
+//   M 8192: 3456 x 1152 99 -> 85, 4608 x 1152 125 -> 100, 4096 x 1024 106 -> 92, 1152 x 1152 64 -> 41, 768 x 768 51 -> 27;  M 16384: 3072 x 768 177 ->
+//   91, 4608 x 1152 335 -> 178 (975 TFLOP/s).  The largest result measured is 6912 x 1152 (8 M elements); beyond it the library's products are kept.
 extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return 0;
   const int64_t result = (int64_t)N * K;
   if (result > 8000000) return 0;
   if (M < 1536) return 1;
   if (M < 4096) return result <= 600000;
-  if (M < 8192) return result <= 2400000;
-  return K % dmf::kWgK == 0 || result <= 3200000;
+  return M >= 6144 || result <= 3200000 || (result >= 5000000 && K % dmf::kWgK == 0);
 }
 
 extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream) {
   if (g == nullptr || x == nullptr || gw == nullptr) return DMF_ATTN_ENULL;
   if (!dmf::wgrad_shape_ok(M, N, K)) return DMF_ATTN_ESHAPE;
-  const int splits = dmf::wgrad_splits(M, N, K);
+  const int wide = dmf::wgrad_wide_splits(M, N, K), splits = wide ? wide : dmf::wgrad_splits(M, N, K);
   if (splits > 1 && workspace == nullptr) return DMF_ATTN_ENULL;
   for (const void* q : {g, x, (const void*)gw, (const void*)gbias, (const void*)workspace})
     if (reinterpret_cast<uintptr_t>(q) % 16) return DMF_ATTN_EALIGN;
@@ -1024,14 +1211,19 @@ extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* 
   p.out = splits > 1 ? workspace : gw;
   p.bias = gbias == nullptr ? nullptr : splits > 1 ? workspace + (int64_t)splits * N * K : gbias;
   p.M = M; p.N = N; p.K = K;
-  p.ntiles = (N + dmf::kWgN - 1) / dmf::kWgN;
+  const int columns = wide ? dmf::WgradWide::BM : dmf::kWgN;
+  p.ntiles = (N + columns - 1) / columns;
   p.ktiles = (K + dmf::kWgK - 1) / dmf::kWgK;
   p.splits = splits;
   p.per = ((M + 63) / 64 + splits - 1) / splits;
-  static bool lds_ok[64] = {};
-  if (!dmf::ensure_dynamic_lds(dmf::linear_wgrad_kernel, 2 * dmf::kWgStage, lds_ok)) return -7;
+  static bool lds_ok[64] = {}, lds_ok_wide[64] = {};
+  if (!(wide ? dmf::ensure_dynamic_lds(dmf::linear_wgrad_wide_kernel, dmf::WgradWide::STAGES, lds_ok_wide)
+             : dmf::ensure_dynamic_lds(dmf::linear_wgrad_kernel, 2 * dmf::kWgStage, lds_ok)))
+    return -7;
   auto stm = static_cast<hipStream_t>(stream);
-  const int rc = dmf::launch_kernel(dmf::linear_wgrad_kernel, dim3((uint32_t)p.ntiles * p.ktiles * splits), dim3(256), 2 * dmf::kWgStage, stm, p);
+  const dim3 grid((uint32_t)p.ntiles * p.ktiles * splits);
+  const int rc = wide ? dmf::launch_kernel(dmf::linear_wgrad_wide_kernel, grid, dim3(256), dmf::WgradWide::STAGES, stm, p)
+                      : dmf::launch_kernel(dmf::linear_wgrad_kernel, grid, dim3(256), 2 * dmf::kWgStage, stm, p);
   if (rc != 0 || splits == 1) return rc;
   const int64_t n4 = (int64_t)N * K / 4, b4 = gbias == nullptr ? 0 : N / 4;
   const dmf::SumSplitsParams q{reinterpret_cast<const f32x4*>(workspace), reinterpret_cast<f32x4*>(gw), reinterpret_cast<f32x4*>(gbias), n4, b4, splits};

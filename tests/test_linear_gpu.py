@@ -153,7 +153,11 @@ WGRAD = [(1, 8, 8), (63, 64, 64), (64, 128, 192), (65, 136, 200), (129, 120, 184
          (8192, 1152, 1152), (8192, 3456, 1152), (4096, 4608, 1152), (4096, 1152, 4608), (16389, 768, 768), (32768, 96, 200), (20001, 384, 384)]
 
 
-@pytest.mark.parametrize("M,N,K", WGRAD)
+# (those of 8 G multiply-adds and more go through linear_wgrad_wide_kernel: columns that fill no tile on either side, rows that fill no step, one tile)
+WGRAD_WIDE = [(6145, 1288, 1032), (4097, 712, 2800), (250001, 184, 200), (16389, 264, 1944), (8192, 4608, 1152), (6144, 1152, 4608)]
+
+
+@pytest.mark.parametrize("M,N,K", WGRAD + WGRAD_WIDE)
 def test_weight_gradient(M, N, K):
     gen = torch.Generator(device=DEV).manual_seed(M + N + K)
     # (rows past the last hold values that would show if they were summed)
