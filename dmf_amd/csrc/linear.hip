@@ -31,10 +31,17 @@ constexpr int kLinK = 64;   // contraction elements per step: one 128-byte line 
 // holds both sums of an element.
 enum LinMode { kLinPlain, kLinGelu, kLinGeluJvp };
 
-// sigma = 1 / (1 + exp(-2 u)), u = sqrt(2 / pi) (v + 0.044715 v^3): gelu(v) = 0.5 v (1 + tanh u) = v sigma
+// sigma = 1 / (1 + exp(-2 u)), u = sqrt(2 / pi) (v + 0.044715 v^3): gelu(v) = 0.5 v (1 + tanh u) = v sigma.  The epilogues' arithmetic is not covered by
+// products (a quarter of a gelu pair's time): the constants are multiplied out, sigma is four operations, an exp2 and a reciprocal
+// (with the bias in LDS, pairs N 4C: C768 M16384 165 -> 155 us, C1152 M8192 167 -> 157; the errors against fp64 stay the same to seven digits).
+constexpr double kGelu2u = 1.5957691216057308, kGeluCubic = 0.044715;   // 2 u = kGelu2u v (1 + kGeluCubic v^2)
 __device__ __forceinline__ float gelu_sigma(float v) {
-  const float u2 = 1.5957691216057308f * v * fmaf(0.044715f, v * v, 1.f);
-  return __builtin_amdgcn_rcpf(1.f + fast_exp2(-kLog2e * u2));
+  constexpr double log2e = 1.4426950408889634;
+  return __builtin_amdgcn_rcpf(1.f + fast_exp2(v * fmaf((float)(-log2e * kGelu2u * kGeluCubic), v * v, (float)(-log2e * kGelu2u))));
+}
+// d gelu = sigma (1 + v (1 - sigma) d(2 u))
+__device__ __forceinline__ float gelu_slope(float v, float sigma) {
+  return sigma * fmaf(fmaf(-v, sigma, v), fmaf((float)(3 * kGelu2u * kGeluCubic), v * v, (float)kGelu2u), 1.f);
 }
 
 template <int BM, int BN, int NST, int MODE>
@@ -156,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(const LinearParams p) {
           if constexpr (BOTH) {
             const float x = acc[n][0][4 * q + e] + b[e], sg = gelu_sigma(x);
             if (m == 0) v[e] = x * sg;
-            else v[e] *= sg * fmaf(x * (1.f - sg), 1.5957691216057308f * fmaf(3.f * 0.044715f, x * x, 1.f), 1.f);
+            else v[e] *= gelu_slope(x, sg);
           }
         }
         const int row = wm * WROWS + MROWS * m + c32;
@@ -216,6 +223,13 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+template <int OFF>
+__device__ __forceinline__ u32x2 lds_read64_issue(uint32_t lane_addr) {
+  u32x2 r;
+  asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(r) : "v"(lane_addr), "n"(OFF));
+  return r;
+}
+
 // one element of a product's sums
 __device__ __forceinline__ float sum(float a) {
   float v;
@@ -226,6 +240,7 @@ __device__ __forceinline__ void lds_write64(uint32_t addr, u32x2 v) { asm volati
 
 // (after a wait: keeps uses of what has been read behind it)
 __device__ __forceinline__ void landed_in(u32x4& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void landed_in(u32x2& v) { asm volatile("" : "+v"(v)); }
 
 __device__ __forceinline__ void landed_in(TrPair& v) { asm volatile("" : "+v"(v.lo), "+v"(v.hi)); }
 __device__ __forceinline__ bf16x8 as_operand(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
@@ -246,7 +261,7 @@ struct WalkTile {
   // requests of a wave that may be in flight behind the stage that is waited for
   static constexpr int BEHIND = NSX > NSW ? (NSW - 2) * (PX + PW) + PX : (NSW - 2) * (PX + PW);
   static constexpr int BEFORE = NSX > NSW ? NSW - 2 : NSW - 3;   // last stage of a tile whose last chunk waits for requests from before the stores
-  static_assert(NSW >= 2 && (NSX == NSW || NSX == NSW + 1) && LDS <= 160 * 1024 && (MT % 2 == 0 || MT == 1 && NT == 3) && BEHIND + STORES <= 63);
+  static_assert(NSW >= 2 && (NSX == NSW || NSX == NSW + 1) && LDS <= 160 * 1024 && (MT % 2 == 0 || MT == 1 && NT == 3) && BEHIND + STORES + 1 <= 63);
   // two accumulator tiles leave together, side by side where the row allows: a pass' tile h (0, 1)
   static constexpr int row_of(int pass, int h) { return MT == 1 ? 0 : NT == 3 ? 2 * (pass / 3) + (pass % 3 == 2 ? h : pass % 3) : pass / (NT / 2); }
   static constexpr int col_of(int pass, int h) { return MT == 1 ? 2 * pass + h : NT == 3 ? (pass % 3 == 2 ? 2 : h) : 2 * (pass % (NT / 2)) + h; }
@@ -257,7 +272,7 @@ constexpr int kNonTemporal = 2;   // (buffer instructions' aux bits)
 template <class T, int MODE, bool COLS = false>
 __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   constexpr int MT = T::MT, NT = T::NT, BM = T::BM, BN = T::BN;
-  constexpr bool BOTH = MODE == kLinGeluJvp;
+  constexpr bool BOTH = MODE == kLinGeluJvp, BIAS = !COLS;
   static_assert(!BOTH || MT % 2 == 0, "as many row tiles of x as of tx");
   constexpr int ROWS = BOTH ? BM / 2 : BM, MX = BOTH ? MT / 2 : MT;   // of y: a tile's rows, a wave's row tiles (WM * 32 rows apart)
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -416,7 +431,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       constexpr int c = decltype(cc)::value, NEXT = (c + AHEAD) % 4, NM = MA * NT, R = MA + NT, CHANGE = T::LAST + 1;
       landed(cc, rows_);
       if constexpr (c == CHANGE) {
-        if (stores) wait_vm<T::BEHIND + T::STORES>();
+        if (stores) wait_vm<T::BEHIND + T::STORES + BIAS>();
         else wait_vm<T::BEHIND>();
         asm volatile("s_barrier" ::: "memory");   // the next stage is in LDS and everybody has taken its operands of this one
         xslot = xslot + 1 == T::NSX ? 0 : xslot + 1;
@@ -478,23 +493,22 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     constexpr int MA = decltype(rows_)::value;
     settle();
     const Place at = place(id);
-    // bias of columns 8 v + 4 g .. + 3: wave-uniform vectors of eight by scalar loads (vector loads would wait for the DMA in flight)
-    typedef const __attribute__((address_space(4))) uint32_t* ScalarPtr;
-    const bool biased = p.bias != nullptr && !at.second;
-    const __bf16* bias = biased ? p.bias : p.w;   // (something readable)
-    const uint32_t keep = biased ? ~0u : 0u;
-    u32x2 braw[NT * 4];
-    for_each(std::make_integer_sequence<int, NT * 4>{}, [&](auto vv) {
-      constexpr int v = decltype(vv)::value;
-      const ScalarPtr s = (ScalarPtr)(uintptr_t)(bias + min(at.n0 + wn * 32 * NT + v * 8, p.N - 8));
-      uint32_t w0 = s[0], w1 = s[1], w2 = s[2], w3 = s[3];
-      asm("" : "+s"(w0), "+s"(w1), "+s"(w2), "+s"(w3));   // (or the selection is made of addresses, and the loads are vector loads)
-      braw[v] = u32x2{(g ? w2 : w0) & keep, (g ? w3 : w1) & keep};
-    });
+    u32x2 braw[BIAS ? NT * 4 : 1];   // bias of columns 8 v + 4 g .. + 3
+    if constexpr (BIAS) {
+      if (steps < T::BEFORE + 2) wait_vm<T::PX + T::PW>();   // (else the tile's last stage has waited for it)
+      for_each(std::make_integer_sequence<int, NT * 4>{}, [&](auto vv) {
+        braw[decltype(vv)::value] = lds_read64_issue<decltype(vv)::value * 16>(own + wn * 64 * NT + g * 8);
+      });
+    }
     // (sums are taken out of their registers one quad at a time: left to itself the compiler copies all of them at once, and spills; the wait
     //  states between the last product and the first of these reads are written out, as it does not look into assembly)
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+    if constexpr (BIAS) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int v = 0; v < NT * 4; ++v) landed_in(braw[v]);
+    }
     const int ncols = min(BN, p.N - at.n0);
     __amdgpu_buffer_rsrc_t ry[2];
     for (int h = 0; h < (BOTH ? 2 : 1); ++h)
@@ -519,7 +533,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       constexpr int pass = decltype(pp)::value;
       for_each(std::make_integer_sequence<int, pass_col(pass, 1) < NT ? 8 : 4>{}, [&](auto vv) {   // (a last tile by itself: half the rows' bytes)
         constexpr int v = decltype(vv)::value, h = v / 4, m = pass_row(pass, h), n = pass_col(pass, h), q = v % 4;
-        const u32x2 raw = braw[4 * n + q];
+        const u32x2 raw = braw[BIAS ? 4 * n + q : 0];
         const float bb[4] = {__uint_as_float(raw[0] << 16), __uint_as_float(raw[0] & 0xffff0000u), __uint_as_float(raw[1] << 16),
                              __uint_as_float(raw[1] & 0xffff0000u)};
         float o[4];
@@ -529,11 +543,11 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
           if constexpr (BOTH && pass % 2) {
             o[e] *= slope[h][4 * q + e];
           } else {
-            o[e] += bb[e];
+            if constexpr (BIAS) o[e] += bb[e];
             if constexpr (MODE != kLinPlain) {
               const float x = o[e], sg = gelu_sigma(x);
               o[e] = x * sg;
-              if constexpr (BOTH) slope[h][4 * q + e] = sg * fmaf(x * (1.f - sg), 1.5957691216057308f * fmaf(3.f * 0.044715f, x * x, 1.f), 1.f);
+              if constexpr (BOTH) slope[h][4 * q + e] = gelu_slope(x, sg);
             }
           }
         });
@@ -555,12 +569,23 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     asm volatile("s_nop 1" ::: "memory");   // (before assembly may write these registers again)
   };
 
+  // A tile's bias waits, from before the tile's first stage on, where its results will pass through: the KB from its first column on, zeros past the last
+  // one and for tangents.  (Scalar loads at the tile's end left everything waiting for them: pairs C768 M16384 N 3C 119 -> 113 us,
+  // C1152 M8192 N 4C 154 -> 149; 128 x 96 tiles, C768 M4096 N C 10.1 -> 9.4.)
+  auto request_bias = [&](uint32_t id) {
+    const Place t = place(id);
+    const __amdgpu_buffer_rsrc_t rb = make_rows_rsrc(p.bias + t.n0, 0, 1, p.bias != nullptr && !t.second ? (p.N - t.n0) * 2 : 0);
+    char* dst = smem + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)dst, 16, lane * 16, 0, 0, 0);
+  };
+
   using Whole = std::integral_constant<int, MT>;
   using Half = std::integral_constant<int, HALVES ? MT / 2 : MT>;
   for (uint32_t n = 0;; ++n) {
     const uint32_t id = nth_tile(n);
     if (id == END) break;
     const bool stores = n > 0 && T::BEFORE >= 0;
+    if constexpr (BIAS) request_bias(id);
     if (!HALVES || id % 4 == 0) {
       stage(std::true_type{}, Whole{}, stores);
       for (int t = 1; t < steps; ++t) stage(std::false_type{}, Whole{}, stores && t <= T::BEFORE);
