@@ -254,13 +254,18 @@ __device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f
 template <int MT_, int NT_, int WM_, int NSX_, int NSW_>
 struct WalkTile {
   static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = 4 / WM, NSX = NSX_, NSW = NSW_, BM = 32 * MT * WM, BN = 32 * NT * WN;
-  static constexpr int XS = BM * 128, WS = BN * 128, LDS = NSX * XS + NSW * WS + 4 * 4096;
+  static constexpr int XS = BM * 128, WS = BN * 128;
+  // results pass through 4 KB of LDS per wave, its own or, where the stages take everything, the KBs of the next emptied slot of x that the wave
+  // itself will request into
+  static constexpr bool IN_SLOT = NSX * XS + NSW * WS + 4 * 4096 > 160 * 1024;
+  static constexpr int LDS = NSX * XS + NSW * WS + (IN_SLOT ? 0 : 4 * 4096);
   static constexpr int PX = XS / 4096, PW = WS / 4096, STORES = (MT * NT + 1) / 2 * 4;
   // chunks whose operands are read ahead: with one row tile the products of one chunk are too short to hide its reads
   static constexpr int AHEAD = MT == 1 ? 2 : 1, LAST = 3 - AHEAD;   // LAST: the chunk before the one that changes stages
   // requests of a wave that may be in flight behind the stage that is waited for
   static constexpr int BEHIND = NSX > NSW ? (NSW - 2) * (PX + PW) + PX : (NSW - 2) * (PX + PW);
   static constexpr int BEFORE = NSX > NSW ? NSW - 2 : NSW - 3;   // last stage of a tile whose last chunk waits for requests from before the stores
+  static_assert(!IN_SLOT || NSX > NSW && XS >= 16 * 1024);   // (the slot is requested into behind the tile's end)
   static_assert(NSW >= 2 && (NSX == NSW || NSX == NSW + 1) && LDS <= 160 * 1024 && (MT % 2 == 0 || MT == 1 && NT == 3) && BEHIND + STORES + 1 <= 63);
   // two accumulator tiles leave together, side by side where the row allows: a pass' tile h (0, 1)
   static constexpr int row_of(int pass, int h) { return MT == 1 ? 0 : NT == 3 ? 2 * (pass / 3) + (pass % 3 == 2 ? h : pass % 3) : pass / (NT / 2); }
@@ -485,19 +490,31 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
 
   // Output rows leave two accumulator tiles at a time through this wave's 4 KB of LDS (32 rows of 128 bytes, slot v of row r holding vector
   // v ^ r / 2 % 8), in whole 16-byte vectors; while one pass is on its way through LDS the next one is computed.
-  const uint32_t own = lds_addr(smem) + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
-  const uint32_t put = own + c32 * 128 + ((c32 >> 1) & 7) * 16 + g * 8;
-  const uint32_t get = own + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 4)) * 16);   // rows + 8 i: slot ^ 4 i % 8
+  constexpr int GROUP = T::IN_SLOT ? 4096 : 1024;   // between groups of eight rows
+  uint32_t own, put, get;   // get: rows + 8 i: slot ^ 4 i % 8
+  auto pass_through = [&](uint32_t base) {
+    own = base;
+    put = own + (c32 >> 3) * GROUP + (c32 & 7) * 128 + ((c32 >> 1) & 7) * 16 + g * 8;
+    get = own + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 4)) * 16);
+  };
+  if constexpr (!T::IN_SLOT) pass_through(lds_addr(smem) + T::NSX * T::XS + T::NSW * T::WS + wave * 4096);
+  uint32_t bias2 = 0;
   const int half = (lane >> 2) & 1;
   auto finish = [&](uint32_t id, auto rows_) {
     constexpr int MA = decltype(rows_)::value;
     settle();
+    if constexpr (T::IN_SLOT) pass_through(lds_addr(smem) + cx.slot * T::XS + wave * 1024);
     const Place at = place(id);
     u32x2 braw[BIAS ? NT * 4 : 1];   // bias of columns 8 v + 4 g .. + 3
     if constexpr (BIAS) {
-      if (steps < T::BEFORE + 2) wait_vm<T::PX + T::PW>();   // (else the tile's last stage has waited for it)
+      if constexpr (T::IN_SLOT) {
+        wait_vm<T::PX + T::PW>();   // (as many requests are behind it at least, and no more in flight here)
+        asm volatile("ds_write_b32 %0, %1" ::"v"(own + lane * 4), "v"(bias2) : "memory");
+      } else if (steps < T::BEFORE + 2) {
+        wait_vm<T::PX + T::PW>();   // (else the tile's last stage has waited for it)
+      }
       for_each(std::make_integer_sequence<int, NT * 4>{}, [&](auto vv) {
-        braw[decltype(vv)::value] = lds_read64_issue<decltype(vv)::value * 16>(own + wn * 64 * NT + g * 8);
+        braw[decltype(vv)::value] = lds_read64_issue<decltype(vv)::value * 16>(own + (T::IN_SLOT ? 0 : wn * 64 * NT) + g * 8);
       });
     }
     // (sums are taken out of their registers one quad at a time: left to itself the compiler copies all of them at once, and spills; the wait
@@ -560,7 +577,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       }
       for_each(std::make_integer_sequence<int, 4>{}, [&](auto ii) {
         constexpr int i = decltype(ii)::value;
-        out[pass & 1][i] = lds_read128_issue<i * 1024>(i & 1 ? get ^ 64 : get);
+        out[pass & 1][i] = lds_read128_issue<i * GROUP>(i & 1 ? get ^ 64 : get);
       });
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -569,14 +586,21 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     asm volatile("s_nop 1" ::: "memory");   // (before assembly may write these registers again)
   };
 
-  // A tile's bias waits, from before the tile's first stage on, where its results will pass through: the KB from its first column on, zeros past the last
-  // one and for tangents.  (Scalar loads at the tile's end left everything waiting for them: pairs C768 M16384 N 3C 119 -> 113 us,
-  // C1152 M8192 N 4C 154 -> 149; 128 x 96 tiles, C768 M4096 N C 10.1 -> 9.4.)
+  // A tile's bias is requested before its first stage (scalar loads at the tile's end left everything waiting for them: pairs C768 M16384 N 3C 119 ->
+  // 113 us, C1152 M8192 N 4C 154 -> 149; 128 x 96 tiles, C768 M4096 N C 10.1 -> 9.4): the KB from the tile's first column on, zeros past the last one and
+  // for tangents, to where the results will pass through.  Without LDS for it, this wave's columns into a register, two per lane; in assembly, as
+  // the compiler would wait for all requests in flight at its use, and that nothing touches it before its wait is checked on the built code.
   auto request_bias = [&](uint32_t id) {
     const Place t = place(id);
-    const __amdgpu_buffer_rsrc_t rb = make_rows_rsrc(p.bias + t.n0, 0, 1, p.bias != nullptr && !t.second ? (p.N - t.n0) * 2 : 0);
-    char* dst = smem + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)dst, 16, lane * 16, 0, 0, 0);
+    const int bytes = p.bias != nullptr && !t.second ? (p.N - t.n0) * 2 : 0;
+    if constexpr (T::IN_SLOT) {
+      const u32x4 rb = rows_rsrc_words(p.bias + t.n0, 0, 1, bytes);
+      asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, %2, 0 offen" : "=v"(bias2) : "v"((wn * 32 * NT + 2 * lane) * 2), "s"(rb) : "memory");
+    } else {
+      const __amdgpu_buffer_rsrc_t rb = make_rows_rsrc(p.bias + t.n0, 0, 1, bytes);
+      char* dst = smem + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)dst, 16, lane * 16, 0, 0, 0);
+    }
   };
 
   using Whole = std::integral_constant<int, MT>;
@@ -606,10 +630,21 @@ __global__ __launch_bounds__(256, 1) void linear_walk_kernel(const LinearParams 
   linear_walk<T, MODE>(p);
 }
 
+// 256 x 256: an eighth fewer bytes and LDS reads per product than 256 x 192, all of the accumulation registers and of the LDS (results pass through
+// the slot that is to be requested into next).  Where the rounds are as full: pairs C768 M16384 N 4C 144 -> 136 us, N 3C 111 -> 107, with gelu 157 ->
+// 148; C1024 M8192 N 4C 128 -> 115, M16384 K 4C 234 -> 209; 8192 cubed 867 -> 798 (1378 TFLOP/s).
+using WalkWide = WalkTile<4, 4, 2, 3, 2>;
+template <int MODE>
+__global__ __launch_bounds__(256, 1) void linear_walk_wide_kernel(const LinearParams p) {
+  linear_walk<WalkWide, MODE>(p);
+}
+
 template <class T, int MODE>
 static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
   constexpr int rows = MODE == kLinGeluJvp ? T::BM / 2 : T::BM;
-  auto kern = linear_walk_kernel<T, MODE>;
+  void (*kern)(LinearParams);
+  if constexpr (std::is_same_v<T, WalkWide>) kern = linear_walk_wide_kernel<MODE>;
+  else kern = linear_walk_kernel<T, MODE>;
   static bool lds_ok[64] = {};
   if (!ensure_dynamic_lds(kern, T::LDS, lds_ok)) return -7;
   p.mtiles = (p.M + rows - 1) / rows;
@@ -639,13 +674,14 @@ static int launch_dgrad(LinearParams& p, hipStream_t stream) {
   return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
 }
 
-// Tile policy: the shortest of the estimates, in 10 ns, of six kernels.  linear_kernel: a K step (64) and a work-group's start and end with one,
+// Tile policy: the shortest of the estimates, in 10 ns, of seven kernels.  linear_kernel: a K step (64) and a work-group's start and end with one,
 // two, three work-groups on a CU, more of them never taking less; linear_walk_kernel: a step and what a tile takes beyond its steps at that
 // pace, of whole and of half a tile, and the launch's.  Fitted to 1440 products of
 // widths 384 to 1280, 64 to 32768 rows, single and in pairs, with and without gelu, seven tenths of them; all of them and the fit's aim are in
 // profiles/linear_tiles.txt.  Tiles within 1.3 of the fastest one are met to 4 (128 x 96) to 11 % (64 x 64); the tile taken is 0.24 % slower than
 // the fastest in the mean (0.25 % where the fit did not look), 5 % in one of a hundred.  128 x 192 is all but never that tile; it is here
-// for the rows of more than 65536 elements that the walking kernel does not take.
+// for the rows of more than 65536 elements that the walking kernel does not take.  The estimate of 256 x 256 is set on 175 further products of up to
+// 16384 rows (117 of at least one round), so that the choice among the three walking tiles is 0.1 % slower than the fastest of them in the mean.
 struct LinTile { int bm, bn, per_cu, a[3], b[3]; };
 constexpr LinTile kLinTiles[3] = {{128, 192, 2, {82, 113, 0}, {541, 761, 0}}, {128, 64, 3, {48, 68, 80}, {262, 364, 466}}, {64, 64, 2, {23, 39, 0}, {279, 263, 0}}};
 constexpr bool never_shorter_with_more(const LinTile& t) {
@@ -655,7 +691,7 @@ constexpr bool never_shorter_with_more(const LinTile& t) {
 }
 static_assert(never_shorter_with_more(kLinTiles[0]) && never_shorter_with_more(kLinTiles[1]) && never_shorter_with_more(kLinTiles[2]));
 struct LinWalk { int bm, bn, a, b, a_half, b_half, launch; };
-constexpr LinWalk kLinWalks[2] = {{256, 192, 94, 607, 59, 433, 136}, {256, 128, 73, 386, 45, 413, 135}};
+constexpr LinWalk kLinWalks[3] = {{256, 192, 94, 607, 59, 433, 136}, {256, 128, 73, 386, 45, 413, 135}, {256, 256, 116, 800, 64, 640, 136}};
 
 static int64_t walk_cost(const LinWalk& c, int64_t M, int64_t N, int64_t steps, int products, bool halves) {
   const int64_t cus = compute_units(), tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * products, rest = tiles % cus;
@@ -696,6 +732,9 @@ static int linear_tile(int64_t M, int N, int K, bool jvp, bool gelu) {
   }
   // (the walking kernel's row offsets within a tile are 32-bit)
   for (int t = 0; t < 2 && N <= 65536 && K <= 65536; ++t) take(3 + t, walk_cost(kLinWalks[t], M, N, steps, jvp ? 2 : 1, !both));
+  // 256 x 256 from nearly a round on (M12288 C1152 K 4C, 240 tiles, 131 -> 106 us; half tiles alone are no use: M3072 pair 67 against 74)
+  if (N <= 65536 && K <= 65536 && 8 * ((M + 255) / 256) * ((N + 255) / 256) * (jvp ? 2 : 1) >= 7 * cus)
+    take(6, walk_cost(kLinWalks[2], M, N, steps, jvp ? 2 : 1, !both));
   return best;
 }
 
@@ -709,6 +748,7 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
     case 5:
       if constexpr (MODE != kLinGeluJvp) return launch_walk<WalkTile<1, 3, 4, 5, 5>, MODE>(p, jvp, stream);
       break;
+    case 6: return launch_walk<WalkWide, MODE>(p, jvp, stream);
     default: break;
   }
   if constexpr (MODE == kLinGeluJvp) return DMF_ATTN_ESHAPE;   // (linear_tile does not answer this)
@@ -753,9 +793,9 @@ extern "C" int dmf_linear_fwd_plan(int64_t M, int N, int K, int jvp, int gelu, c
     return DMF_ATTN_ESHAPE;
   if (buf == nullptr || buflen < 1) return DMF_ATTN_ENULL;
   const int mode = !gelu ? dmf::kLinPlain : jvp ? dmf::kLinGeluJvp : dmf::kLinGelu;
-  const char* form[6] = {"linear_kernel<128, 192, 2, %d>", "linear_kernel<128, 64, 2, %d>", "linear_kernel<64, 64, 4, %d>",
+  const char* form[7] = {"linear_kernel<128, 192, 2, %d>", "linear_kernel<128, 64, 2, %d>", "linear_kernel<64, 64, 4, %d>",
                          "linear_walk_kernel<dmf::WalkTile<4, 3, 2, 3, 2>, %d>", "linear_walk_kernel<dmf::WalkTile<4, 2, 2, 3, 3>, %d>",
-                         "linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>, %d>"};
+                         "linear_walk_kernel<dmf::WalkTile<1, 3, 4, 5, 5>, %d>", "linear_walk_wide_kernel<%d>"};
   const int n = snprintf(buf, (size_t)buflen, "dmf::");
   if (n < buflen) snprintf(buf + n, (size_t)(buflen - n), form[dmf::linear_tile(M, N, K, jvp != 0, gelu != 0)], mode);
   return DMF_ATTN_OK;

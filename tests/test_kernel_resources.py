@@ -106,6 +106,7 @@ def test_lds_budgets(kernels):
 BUDGETS = [
     (r"13linear_kernelI", 256, 0), (r"18linear_walk_kernelI", 512, 0), (r"19linear_wgrad_kernelE", 256, 0), (r"17modulation_kernelI", 512, 0),
     (r"19linear_dgrad_kernelI", 512, 0), (r"24linear_wgrad_wide_kernelE", 512, 0),
+    (r"23linear_walk_wide_kernelI", 512, 0),
     (r"21attn_fwd_small_kernelIDF16_Li(64|72|80|96)ELb0E", 256, 0), (r"21attn_fwd_small_kernelIDF16bLi(64|72|80|96)ELb0ELb0E", 256, 0),
     (r"21attn_fwd_small_kernelI", 512, 0),
     (r"20attn_fwd_wide_kernelIDF16_Li(72|80)ELb0E", 128, 4), (r"20attn_fwd_wide_kernelI(DF16_Li(72|80)|fLi(32|64))ELb1E", 256, 0),
@@ -149,30 +150,38 @@ def _registers(text):
     return mask
 
 
-def _decode(lines):
-    """(operation, registers it names, branch target, lgkmcnt waited for, registers a queued read returns or None) of every instruction."""
+def _decode(lines, counter="lgkmcnt"):
+    """(operation, registers it names, branch target, count of `counter` waited for, registers a queued read returns or None) of every
+    instruction.  vmcnt: loads from memory, and those into LDS and stores, which return nothing; loads return in order, so that one may name
+    the register that another is about to write as its own result."""
     code = [(int(m.group(3), 16), m.group(1), m.group(2)) for m in (re.match(r"\t(\S+)\s*(.*?)\s*// ([0-9A-F]+):", l) for l in lines) if m]
     at, out = {a: i for i, (a, _, _) in enumerate(code)}, []
     for address, op, args in code:
         target = wait = queued = None
+        names = _registers(args)
         if op == "s_branch" or op.startswith("s_cbranch"):
             offset = int(args.split()[0])
             target = at[address + 4 + 4 * (offset - 65536 * (offset >= 32768))]
         elif op == "s_waitcnt":
             assert "cnt(" in args, args
-            m = re.search(r"lgkmcnt\((\d+)\)", args)
+            m = re.search(counter + r"\((\d+)\)", args)
             wait = int(m.group(1)) if m else None
+        elif counter == "vmcnt":
+            if op.startswith(("buffer_load", "buffer_store", "global_load", "global_store", "scratch_load", "scratch_store", "global_atomic", "buffer_atomic")):
+                queued = 0
+                if "load" in op and not re.search(r"\blds\b", args) and "_lds_" not in op:
+                    queued, names = _registers(args.split(",")[0]), _registers(args.split(",", 1)[1])
         elif op.startswith("ds_"):
             queued = _registers(args.split(",")[0]) if any(s in op for s in ("read", "_rtn", "permute", "swizzle")) else 0
         elif op.startswith(("s_load", "s_buffer_load", "s_memtime", "s_memrealtime")):
             queued = SCALAR
         assert not op.startswith(("flat_", "s_swappc", "s_setpc", "s_call")), op
-        out.append((op, _registers(args), target, wait, queued))
+        out.append((op, names, target, wait, queued))
     return out
 
 
-def _touched_in_flight(code):
-    """Indices of instructions that name a register an LDS read may still be about to write.  State at a place: what the last 16 requests
+def _touched_in_flight(code, most=16):
+    """Indices of instructions that name a register a read may still be about to write.  State at a place: what the last `most` requests
     return (the counter holds no more), newest last, joined over the paths that lead there."""
     entries = {0} | {t for _, _, t, _, _ in code if t is not None} | {i + 1 for i, c in enumerate(code) if c[2] is not None}
     states, work, bad = {0: ()}, [0], set()
@@ -202,7 +211,7 @@ def _touched_in_flight(code):
             elif wait is not None and not pending & SCALAR:
                 queue = queue[-wait:]
             if queued is not None:
-                queue = (queue + (queued,))[-16:]
+                queue = (queue + (queued,))[-most:]
             if target is not None:
                 join(target, queue)
             if op in ("s_branch", "s_endpgm"):
@@ -222,6 +231,26 @@ def test_the_check_sees_a_read_that_is_not_waited_for():
     assert not _touched_in_flight(_decode(lines(read, "ds_write_b64 v1, v[2:3]", "s_waitcnt vmcnt(0) lgkmcnt(1)", use, "s_endpgm")))
     # over a back edge: read at the end of one turn, waited for in the next one only behind the use
     assert _touched_in_flight(_decode(lines(use, "s_waitcnt lgkmcnt(0)", read, "s_cbranch_scc1 65532", "s_endpgm"))) == {0}
+
+
+def test_no_register_is_touched_between_a_product_kernels_load_and_the_wait(code_objects):
+    """The bias of a walking kernel's tile is loaded in assembly and waited for by counting the requests behind it: as for the LDS reads below."""
+    lines = lambda *ops: [f"\t{op} // {4 * i:012X}: 00000000" for i, op in enumerate(ops)]
+    load, use, dma = "buffer_load_dword v5, v0, s[0:3], 0 offen", "v_mov_b32_e32 v8, v5", "buffer_load_dwordx4 v1, s[0:3], 0 offen lds"
+    assert _touched_in_flight(_decode(lines(load, dma, "s_waitcnt vmcnt(2)", use, "s_endpgm"), "vmcnt"), 64) == {3}
+    assert not _touched_in_flight(_decode(lines(load, dma, "s_waitcnt vmcnt(1)", use, "s_endpgm"), "vmcnt"), 64)
+    checked = 0
+    for co in code_objects:
+        name, code = "", {}
+        for line in subprocess.run([TOOLS[3], "-d", co], check=True, capture_output=True, text=True).stdout.splitlines():
+            m = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+            name = m.group(1) if m else name
+            code.setdefault(name, []).append(line)
+        for name, lines in code.items():
+            if re.search(r"linear_(walk|walk_wide|dgrad|wgrad_wide)_kernel", name):
+                checked += 1
+                assert not _touched_in_flight(_decode(lines, "vmcnt"), 64), name
+    assert checked >= 14
 
 
 def test_no_register_is_touched_between_its_lds_read_and_the_wait(code_objects):

@@ -283,6 +283,29 @@ def test_every_kernel(kernel, size, modes):
                 _check(got, exp)
 
 
+# 256 x 256 tiles, whose results pass through a slot of the stages: rows and columns that fill no tile, one step and two, whole and half tiles behind
+# the rounds, no bias and one with its last columns past the tile
+WIDE = [((16129, 1016, 64), MODES), ((16129, 2040, 128), MODES), ((8193, 3064, 768), [PLAIN, PAIR, GELU]), ((16300, 2040, 1152), MODES),
+        ((21000, 1016, 192), [PAIR, GELU_PAIR]), ((57345, 248, 64), MODES)]
+
+
+@pytest.mark.parametrize("size,modes", WIDE)
+def test_products_of_the_widest_tiles(size, modes):
+    M, N, K = size
+    x, tx, w, b = _operands(M, N, K)
+    ref, tref = torch.nn.functional.linear(x.float(), w.float(), b.float()), tx.float() @ w.float().t()
+    act, tact = torch.func.jvp(lambda t: torch.nn.functional.gelu(t, approximate="tanh"), (ref.double(),), (tref.double(),))
+    for jvp, gelu in modes:
+        assert planned(M, N, K, jvp, gelu) == f"dmf::linear_walk_wide_kernel<{gelu + (jvp and gelu)}>"
+        for _ in range(2):
+            y, ty = _call(x, tx if jvp else None, w, b, gelu)
+            for got, exp in ((y, act if gelu else ref), (ty, tact if gelu else tref)):
+                if got is not None:
+                    _check(got, exp)
+        if not gelu:
+            _check(_call(x, tx if jvp else None, w, None, 0)[0], ref - b.float())
+
+
 def test_the_plan_refuses_what_the_entry_refuses():
     plan, name = _lib.load().dmf_linear_fwd_plan, ctypes.create_string_buffer(4)
     for size in ((64, 64, 32), (64, 60, 64), (0, 64, 64), (2 ** 25, 64, 64)):
