@@ -461,13 +461,16 @@ constexpr float kSplitLazyLog2 = 6.0f;   // the running maximum is raised when e
 // requested and committed a phase apart (half as many loads in flight), the planes of dQ in LDS; and with twice as many rows to a
 // tile the splitting of fp32 elements, a third of the vector instructions, is shared by twice as many waves -- with tangents four
 // of them bring the primal tile of a pair and four the tangent's.  us (4 -> 8 waves): fp16 + tangents B8 H16 N1024 D72 311 -> 188,
-// fp32 + tangents B4 H16 N1024 D64 267 -> 233, fp16 B8 H16 N1024 D72 97 -> 78 (four waves per SIMD instead of three).
+// fp32 + tangents B4 H16 N1024 D64 267 -> 233, fp16 B8 H16 N1024 D72 97 -> 78 (four waves per SIMD instead of three).  Without tangents two stages fit
+// beside one another even so, and K and V come together, one barrier a step instead of two; with products ahead of the other waves' vector
+// instructions (s_setprio) 72.3 -> 69.7 (of which 1 the barrier), B64 N256 50.4 -> 47.3, B4 N2048 137 -> 133, two thirds of a round B12 N1024 115 -> 116;
+// with tangents the priority changes nothing (fp32 B16 H12 N256 D64 153 -> 153).
 template <typename T, int D, bool JVP, int NW>
 struct SplitFwdPlan {
   using C = SplitCfg<T, D, NW>;
-  static constexpr bool WIDE = NW == 8, PAIR = JVP && WIDE;
+  static constexpr bool WIDE = NW == 8, PAIR = JVP && WIDE, PHASED = PAIR;   // PHASED: one stage, K and V a phase apart
   static constexpr int NT = JVP ? 4 : 2, STAGE = NT * C::TILE;
-  static constexpr int STAGES = !WIDE && 2 * STAGE <= 160 * 1024 ? 2 : 1;
+  static constexpr int STAGES = !PHASED && 2 * STAGE <= (WIDE ? 80 : 160) * 1024 ? 2 : 1;
   static constexpr bool DQ_LDS = PAIR && (sizeof(T) == 4 || D > 64);
   static constexpr int DQ_OFF = STAGES * STAGE, DQ_BYTES = DQ_LDS ? NW * C::NCHUNK * SplitType<T>::NI * 64 * 16 : 0;
   static constexpr int BYTES = DQ_OFF + DQ_BYTES > C::STAGE_ROWS_BYTES ? DQ_OFF + DQ_BYTES : C::STAGE_ROWS_BYTES;
@@ -565,15 +568,16 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
 
   const int ntiles = (p.Lkv + 31) / 32;
   commit_k(0);
-  if constexpr (!Plan::WIDE) commit_v(0);
+  if constexpr (!Plan::PHASED) commit_v(0);
   for (int it = 0; it < ntiles; ++it) {
     __syncthreads();   // the tile (wide: its K half) is in LDS; wide: every wave is done with V of the tile before
-    if constexpr (Plan::WIDE) commit_v(it);
+    if constexpr (Plan::PHASED) commit_v(it);
     if (it + 1 < ntiles) {   // in flight during the math
       load_k(it + 1);
-      if constexpr (!Plan::WIDE) load_v(it + 1);
+      if constexpr (!Plan::PHASED) load_v(it + 1);
     }
     const char *Kt = tile(it, 0), *Vt = tile(it, 1), *dKt = tile(it, 2), *dVt = tile(it, 3);
+    if constexpr (Plan::WIDE && !JVP) __builtin_amdgcn_s_setprio(1);
     f32x16 S = {0}, dS = {0};
 #pragma unroll
     for (int c = 0; c < NCHUNK; ++c) {
@@ -595,6 +599,7 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
         }
       }
     }
+    if constexpr (Plan::WIDE && !JVP) __builtin_amdgcn_s_setprio(0);
     if ((it + 1) * 32 > p.Lkv) {
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -633,13 +638,14 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     }
     WOperand<T> we;
     we.template form<true>(E);
-    if constexpr (Plan::WIDE) {
+    if constexpr (Plan::PHASED) {
       __syncthreads();   // V is in LDS; every wave is done with K
       if (it + 1 < ntiles) {
         commit_k(it + 1);
         load_v(it + 1);
       }
     }
+    if constexpr (Plan::WIDE && !JVP) __builtin_amdgcn_s_setprio(1);
     if constexpr (JVP) {
       gs.update(G, dO);
       if constexpr (F16) G *= gs.mul;
@@ -651,7 +657,8 @@ __device__ __forceinline__ void split_fwd_body(const FwdParams& p) {
     } else {
       contract_rows<T, D, NW>(Vt, lane, O, we);
     }
-    if constexpr (!Plan::WIDE) {
+    if constexpr (Plan::WIDE && !JVP) __builtin_amdgcn_s_setprio(0);
+    if constexpr (!Plan::PHASED) {
       if constexpr (Plan::STAGES == 1) __syncthreads();   // every wave is done with the stage
       if (it + 1 < ntiles) {
         commit_k(it + 1);
