@@ -65,6 +65,8 @@ FUSED_SIGNATURES = {
     "dmf_linear_plan": (c_int, [_L] + [_I] * 4),
     "dmf_linear_fwd": (c_int, [_P] * 6 + [_I] * 4 + [_P]),
     "dmf_linear_fwd_plan": (c_int, [_L] + [_I] * 4 + [ctypes.c_char_p, _I]),
+    "dmf_linear_gelu_plan": (c_int, [_L] + [_I] * 2),
+    "dmf_linear_gelu_fwd": (c_int, [_P] * 7 + [_I] * 3 + [_P]),
     "dmf_linear_dgrad_plan": (c_int, [_L] + [_I] * 2),
     "dmf_linear_dgrad": (c_int, [_P] * 3 + [_I] * 3 + [_P]),
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),

@@ -1031,6 +1031,55 @@ py::object linear_gelu(const Tensor& x_, const Tensor& weight_, const Tensor& bi
   return py::cast(finish(y, ty, nullptr, level));
 }
 
+// gelu_tanh(linear(x)) with a tangent and a backward pass to come: one kernel, which keeps the pre-activation besides, and one node that does what the
+// two operators' nodes do in turn.
+py::object linear_gelu_kept(const Tensor& x_, const Tensor& weight_, const OptTensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
+  const int64_t level = current_level();
+  if (level == kUnsupported) return none();
+  const Arg x = unpack(x_), weight = unpack(weight_), bias = unpack(bias_);
+  if (!linear_ok(x, weight, bias) || !x.tan.defined() || !any_grad(x, weight, bias)) return none();
+  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+  const at::ScalarType dt = autocast_type(x.data);
+  const int64_t K = x.data.size(-1), M = x.data.numel() / K, N = weight.data.size(0);
+  const auto dense16 = [](const Tensor& t) { return !t.defined() || (t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0); };
+  if (dt != at::kBFloat16 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !dmf_linear_gelu_plan(M, (int)N, (int)K) || !dense16(x.data) ||
+      !dense16(x.tan) || !dense16(weight.data) || !dense16(bias.data) || (bias.defined() && (bias.data.numel() != N || bias.data.dim() != 1)))
+    return none();
+  c10::OptionalDeviceGuard device(x.data.device());
+  Tensor h, y, ty;
+  LinearOperands o;
+  {
+    Below below;
+    Casts casts;
+    o = linear_operands(autocast, dt, weight, bias, w_lp, b_lp, casts);
+    if (!o.ok || o.w.scalar_type() != dt || !dense16(o.w) || o.w.sizes() != weight.data.sizes() || o.w.device() != x.data.device() ||
+        (bias.defined() && (!o.b.defined() || o.b.scalar_type() != dt || !dense16(o.b) || o.b.sizes() != bias.data.sizes() || o.b.device() != x.data.device())))
+      return none();   // (nothing has been launched: the casts wait for run())
+    auto sizes = x.data.sizes().vec();
+    sizes.back() = N;
+    const Tensor x2 = casts.add(x.data, dt), tx2 = casts.add(x.tan, dt);
+    casts.run();
+    h = empty(sizes, dt, x.data);
+    y = empty(sizes, dt, x.data);
+    ty = empty(sizes, dt, x.data);
+    check(dmf_linear_gelu_fwd(ptr(x2), ptr(tx2), ptr(o.w), ptr(o.b), mptr(h), mptr(y), mptr(ty), (int)M, (int)N, (int)K, stream_of(x.data)), "dmf_linear_gelu_fwd");
+  }
+  std::shared_ptr<KernelNode> node = make_node("LinearGeluTanhBackward", {x, weight, bias}, {x.var, o.w.is_same(weight.data) ? weight.var : o.w, h});
+  node->torch_ops = true;
+  node->fn = [wt = weight.data.scalar_type(), has_bias = bias.defined(), bt = bias.defined() ? bias.data.scalar_type() : at::kFloat](
+                 KernelNode& node, const std::vector<Tensor>& sv, const variable_list& g) {
+    Tensor gh;
+    {
+      const Below below;   // (the activation's gradient is a constant where it is differentiated again)
+      const Tensor h = dense(in_memory(sv[2])), gy = dense(g[0].to(h.scalar_type()));
+      gh = dense_like(h);
+      check(dmf_gelu_tanh_bwd(ptr(gy), ptr(h), mptr(gh), h.numel(), code_of(h), stream_of(h)), "dmf_gelu_tanh_bwd");
+    }
+    return linear_backward(node, sv[0], sv[1], gh, wt, bt, has_bias);
+  };
+  return py::cast(finish(y, ty, node, level));
+}
+
 // gelu_tanh(linear(x)), one kernel or two.  Without history to build and yet not for the kernel above: none, the general route has a library
 // call with the activation in it.
 py::object linear_gelu_tanh(const Tensor& x, const Tensor& weight, const OptTensor& bias, const OptTensor& w_lp, const OptTensor& b_lp) {
@@ -1041,6 +1090,8 @@ py::object linear_gelu_tanh(const Tensor& x, const Tensor& weight, const OptTens
     if (!out.is_none()) return out;
   }
   if (bias && !grad) return none();
+  py::object kept = linear_gelu_kept(x, weight, bias, w_lp, b_lp);
+  if (!kept.is_none()) return kept;
   const py::object h = linear(x, weight, bias, w_lp, b_lp);
   if (h.is_none()) return none();
   py::object out = activation(h.cast<Tensor>(), Act::gelu);

@@ -16,7 +16,7 @@ namespace dmf {
 
 struct LinearParams {
   const __bf16 *x[2], *w, *bias;   // x[1]: the tangent's rows (second half of the grid), no bias
-  __bf16* y[2];
+  __bf16 *y[2], *pre;              // pre: the pre-activation x w^T + bias as well (kLinGeluJvpPre)
   int M, N, K, mtiles, ntiles;
 };
 
@@ -29,7 +29,8 @@ constexpr int kLinK = 64;   // contraction elements per step: one 128-byte line 
 // cover each other's reads.
 // MODE: plain; gelu; or gelu with its tangent, where the BM rows of a work-group are BM / 2 of x and the same ones of tx, so that a wave
 // holds both sums of an element.
-enum LinMode { kLinPlain, kLinGelu, kLinGeluJvp };
+// kLinGeluJvpPre (walking kernel): that, and the pre-activation for a backward pass.
+enum LinMode { kLinPlain, kLinGelu, kLinGeluJvp, kLinGeluJvpPre };
 
 // sigma = 1 / (1 + exp(-2 u)), u = sqrt(2 / pi) (v + 0.044715 v^3): gelu(v) = 0.5 v (1 + tanh u) = v sigma.  The epilogues' arithmetic is not covered by
 // products (a quarter of a gelu pair's time): the constants are multiplied out, sigma is four operations, an exp2 and a reciprocal
@@ -277,7 +278,9 @@ constexpr int kNonTemporal = 2;   // (buffer instructions' aux bits)
 template <class T, int MODE, bool COLS = false>
 __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   constexpr int MT = T::MT, NT = T::NT, BM = T::BM, BN = T::BN;
-  constexpr bool BOTH = MODE == kLinGeluJvp, BIAS = !COLS;
+  constexpr bool BOTH = MODE >= kLinGeluJvp, BIAS = !COLS;
+  constexpr int KINDS = MODE == kLinGeluJvpPre ? 3 : BOTH ? 2 : 1, STORES = BOTH ? T::STORES / 2 * KINDS : T::STORES;   // of results of an element of x
+  static_assert(T::BEHIND + STORES + 1 <= 63, "vmcnt immediate");
   static_assert(!BOTH || MT % 2 == 0, "as many row tiles of x as of tx");
   constexpr int ROWS = BOTH ? BM / 2 : BM, MX = BOTH ? MT / 2 : MT;   // of y: a tile's rows, a wave's row tiles (WM * 32 rows apart)
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -436,7 +439,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       constexpr int c = decltype(cc)::value, NEXT = (c + AHEAD) % 4, NM = MA * NT, R = MA + NT, CHANGE = T::LAST + 1;
       landed(cc, rows_);
       if constexpr (c == CHANGE) {
-        if (stores) wait_vm<T::BEHIND + T::STORES + BIAS>();
+        if (stores) wait_vm<T::BEHIND + STORES + BIAS>();
         else wait_vm<T::BEHIND>();
         asm volatile("s_barrier" ::: "memory");   // the next stage is in LDS and everybody has taken its operands of this one
         xslot = xslot + 1 == T::NSX ? 0 : xslot + 1;
@@ -527,25 +530,30 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
       for (int v = 0; v < NT * 4; ++v) landed_in(braw[v]);
     }
     const int ncols = min(BN, p.N - at.n0);
-    __amdgpu_buffer_rsrc_t ry[2];
-    for (int h = 0; h < (BOTH ? 2 : 1); ++h)
-      ry[h] = make_rows_rsrc(p.y[BOTH ? h : at.second] + (int64_t)at.m0 * p.N + at.n0, nb, at.rows, at.rows > 0 ? ncols * 2 : (int)nb);
-    constexpr int PASSES = (MA * NT + 1) / 2;   // with tangents: of x, then of tx, by turns
+    __amdgpu_buffer_rsrc_t ry[KINDS];
+#pragma unroll
+    for (int h = 0; h < KINDS; ++h) {
+      __bf16* y = MODE == kLinGeluJvpPre && h == 0 ? p.pre : p.y[BOTH ? h - (KINDS - 2) : at.second];
+      ry[h] = make_rows_rsrc(y + (int64_t)at.m0 * p.N + at.n0, nb, at.rows, at.rows > 0 ? ncols * 2 : (int)nb);
+    }
+    // with tangents: of x (first as it is, with kLinGeluJvpPre), then of tx, by turns
+    constexpr int PASSES = (MA * NT + 1) / 2 * KINDS / (BOTH ? 2 : 1);
     u32x4 out[2][4];
-    auto pass_row = [](int pass, int h) constexpr { return T::row_of(BOTH ? pass / 2 : pass, h) + (BOTH && pass % 2 ? MX : 0); };
-    auto pass_col = [](int pass, int h) constexpr { return T::col_of(BOTH ? pass / 2 : pass, h); };
+    auto pass_row = [](int pass, int h) constexpr { return T::row_of(pass / KINDS, h) + (BOTH && pass % KINDS == KINDS - 1 ? MX : 0); };
+    auto pass_col = [](int pass, int h) constexpr { return T::col_of(pass / KINDS, h); };
     auto store = [&](auto pp) {
       constexpr int pass = decltype(pp)::value, m0 = pass_row(pass, 0), m1 = pass_row(pass, 1), n0 = pass_col(pass, 0), n1 = pass_col(pass, 1);
       static_assert(m0 / MX == m1 / MX, "both of x, or both of tx");
+      constexpr int kind = BOTH ? pass % KINDS : 0;
       const int tile = half ? n1 : n0, col = (wn * NT + tile) * 32 + (lane & 3) * 8, row = ((half ? m1 % MX : m0 % MX) * T::WM + wm) * 32 + (lane >> 3);
       const uint32_t off = (row * nb + col * 2) | (col < ncols && tile < NT ? 0u : 0x80000000u);   // (past the end: dropped)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         landed_in(out[pass & 1][i]);
-        __builtin_amdgcn_raw_buffer_store_b128(out[pass & 1][i], ry[m0 / MX], off, 8 * i * nb, kNonTemporal);
+        __builtin_amdgcn_raw_buffer_store_b128(out[pass & 1][i], ry[kind], off, 8 * i * nb, kNonTemporal);
       }
     };
-    float slope[BOTH ? 2 : 1][16];   // d gelu of the pass' elements, for their tangents
+    float slope[BOTH ? 2 : 1][16];   // d gelu of the pass' elements, for their tangents; before that, with kLinGeluJvpPre, the elements
     for_each(std::make_integer_sequence<int, PASSES>{}, [&](auto pp) {
       constexpr int pass = decltype(pp)::value;
       for_each(std::make_integer_sequence<int, pass_col(pass, 1) < NT ? 8 : 4>{}, [&](auto vv) {   // (a last tile by itself: half the rows' bytes)
@@ -556,12 +564,16 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
         float o[4];
         for_each(std::make_integer_sequence<int, 4>{}, [&](auto ee) {
           constexpr int e = decltype(ee)::value;
-          o[e] = sum(acc[n][m][4 * q + e]);
-          if constexpr (BOTH && pass % 2) {
+          constexpr int kind = pass % KINDS;
+          if constexpr (MODE == kLinGeluJvpPre && kind == 1) o[e] = slope[h][4 * q + e];
+          else o[e] = sum(acc[n][m][4 * q + e]);
+          if constexpr (BOTH && kind == KINDS - 1) {
             o[e] *= slope[h][4 * q + e];
           } else {
-            if constexpr (BIAS) o[e] += bb[e];
-            if constexpr (MODE != kLinPlain) {
+            if constexpr (BIAS && kind == 0) o[e] += bb[e];
+            if constexpr (MODE == kLinGeluJvpPre && kind == 0) {
+              slope[h][4 * q + e] = o[e];
+            } else if constexpr (MODE != kLinPlain) {
               const float x = o[e], sg = gelu_sigma(x);
               o[e] = x * sg;
               if constexpr (BOTH) slope[h][4 * q + e] = gelu_slope(x, sg);
@@ -639,18 +651,26 @@ __global__ __launch_bounds__(256, 1) void linear_walk_wide_kernel(const LinearPa
   linear_walk<WalkWide, MODE>(p);
 }
 
+// The MLP's first half where a backward pass follows: pre-activation, activation and its tangent from one product pair, where an activation kernel (50 us at
+// 8192 x 4608) read the pre-activations of both back.  XL/2-width training step, four blocks, 6.74 -> 6.64 ms.
+template <class T>
+__global__ __launch_bounds__(256, 1) void linear_walk_pre_kernel(const LinearParams p) {
+  linear_walk<T, kLinGeluJvpPre>(p);
+}
+
 template <class T, int MODE>
 static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
-  constexpr int rows = MODE == kLinGeluJvp ? T::BM / 2 : T::BM;
+  constexpr int rows = MODE >= kLinGeluJvp ? T::BM / 2 : T::BM;
   void (*kern)(LinearParams);
-  if constexpr (std::is_same_v<T, WalkWide>) kern = linear_walk_wide_kernel<MODE>;
+  if constexpr (MODE == kLinGeluJvpPre) kern = linear_walk_pre_kernel<T>;
+  else if constexpr (std::is_same_v<T, WalkWide>) kern = linear_walk_wide_kernel<MODE>;
   else kern = linear_walk_kernel<T, MODE>;
   static bool lds_ok[64] = {};
   if (!ensure_dynamic_lds(kern, T::LDS, lds_ok)) return -7;
   p.mtiles = (p.M + rows - 1) / rows;
   p.ntiles = (p.N + T::BN - 1) / T::BN;
   const int64_t tiles = (int64_t)p.mtiles * p.ntiles * (jvp && MODE == kLinPlain ? 2 : 1);
-  const int64_t cus = compute_units(), grid = tiles >= cus ? cus : MODE != kLinGeluJvp && T::MT % 2 == 0 && 2 * tiles <= cus ? 2 * tiles : tiles;
+  const int64_t cus = compute_units(), grid = tiles >= cus ? cus : MODE < kLinGeluJvp && T::MT % 2 == 0 && 2 * tiles <= cus ? 2 * tiles : tiles;
   return launch_kernel(kern, dim3((uint32_t)grid), dim3(256), T::LDS, stream, p);
 }
 
@@ -786,6 +806,33 @@ extern "C" int dmf_linear_plan(int64_t M, int N, int K, int jvp, int gelu) {
   if (K >= 1024 && (K & (K - 1)) == 0 && (M >= 16384 || (N >= 4 * K && M >= 4096))) return 0;
   if (M * N > 40000000 && N > 3 * K && N > 2048 && (jvp || K < 1024)) return 0;
   return 1;
+}
+
+extern "C" int dmf_linear_gelu_plan(int64_t M, int N, int K) {
+  if (!dmf_linear_plan(M, N, K, 1, 1) || N > 65536 || K > 65536) return 0;
+  const int tile = dmf::linear_tile(M, N, K, true, true);
+  return tile == 3 || tile == 4 || tile == 6;
+}
+
+extern "C" int dmf_linear_gelu_fwd(const void* x, const void* tx, const void* w, const void* bias, void* pre, void* y, void* ty, int M, int N, int K, void* stream) {
+  if (x == nullptr || tx == nullptr || w == nullptr || pre == nullptr || y == nullptr || ty == nullptr) return DMF_ATTN_ENULL;
+  if (!dmf_linear_gelu_plan(M, N, K)) return DMF_ATTN_ESHAPE;
+  for (const void* q : {x, tx, w, bias, (const void*)pre, (const void*)y, (const void*)ty})
+    if (reinterpret_cast<uintptr_t>(q) % (q == bias ? 8 : 16)) return DMF_ATTN_EALIGN;
+  dmf::LinearParams p{};
+  p.x[0] = static_cast<const __bf16*>(x);
+  p.x[1] = static_cast<const __bf16*>(tx);
+  p.w = static_cast<const __bf16*>(w);
+  p.bias = static_cast<const __bf16*>(bias);
+  p.y[0] = static_cast<__bf16*>(y);
+  p.y[1] = static_cast<__bf16*>(ty);
+  p.pre = static_cast<__bf16*>(pre);
+  p.M = M; p.N = N; p.K = K;
+  auto stm = static_cast<hipStream_t>(stream);
+  const int tile = dmf::linear_tile(M, N, K, true, true);
+  return tile == 3   ? dmf::launch_walk<dmf::WalkTile<4, 3, 2, 3, 2>, dmf::kLinGeluJvpPre>(p, true, stm)
+         : tile == 4 ? dmf::launch_walk<dmf::WalkTile<4, 2, 2, 3, 3>, dmf::kLinGeluJvpPre>(p, true, stm)
+                     : dmf::launch_walk<dmf::WalkWide, dmf::kLinGeluJvpPre>(p, true, stm);
 }
 
 extern "C" int dmf_linear_fwd_plan(int64_t M, int N, int K, int jvp, int gelu, char* buf, int buflen) {

@@ -50,6 +50,14 @@ DMF_ATTN_API int dmf_linear_fwd(const void* x, const void* tx, const void* w, co
                         int gelu, void* stream);
 
 /*
+ * The first half of an MLP whose backward pass follows: pre = x w^T + bias, y = gelu(pre) and ty, the tangent of y along tx, activated from the fp32 sums
+ * (of which pre is the rounding).  Types, sizes and alignment of dmf_linear_fwd; the shapes for which dmf_linear_gelu_plan says 1, DMF_ATTN_ESHAPE
+ * otherwise (dmf_linear_fwd and dmf_gelu_tanh_fwd do those).
+ */
+DMF_ATTN_API int dmf_linear_gelu_plan(int64_t M, int N, int K);
+DMF_ATTN_API int dmf_linear_gelu_fwd(const void* x, const void* tx, const void* w, const void* bias, void* pre, void* y, void* ty, int M, int N, int K, void* stream);
+
+/*
  * gx = g w, the gradient of a linear layer's input: g (M, N), w (N, K), gx (M, K), bf16 and dense, fp32 accumulation.  N a multiple of 64, K
  * of 8, both up to 65536, at most 2^30 elements in each; 16-byte aligned.  dmf_linear_dgrad_plan: as dmf_linear_plan.
  */

@@ -106,7 +106,7 @@ def test_lds_budgets(kernels):
 BUDGETS = [
     (r"13linear_kernelI", 256, 0), (r"18linear_walk_kernelI", 512, 0), (r"19linear_wgrad_kernelE", 256, 0), (r"17modulation_kernelI", 512, 0),
     (r"19linear_dgrad_kernelI", 512, 0), (r"24linear_wgrad_wide_kernelE", 512, 0),
-    (r"23linear_walk_wide_kernelI", 512, 0),
+    (r"23linear_walk_wide_kernelI", 512, 0), (r"22linear_walk_pre_kernelI", 512, 0),
     (r"21attn_fwd_small_kernelIDF16_Li(64|72|80|96)ELb0E", 256, 0), (r"21attn_fwd_small_kernelIDF16bLi(64|72|80|96)ELb0ELb0E", 256, 0),
     (r"21attn_fwd_small_kernelI", 512, 0),
     (r"20attn_fwd_wide_kernelIDF16_Li(72|80)ELb0E", 128, 4), (r"20attn_fwd_wide_kernelI(DF16_Li(72|80)|fLi(32|64))ELb1E", 256, 0),
@@ -247,10 +247,10 @@ def test_no_register_is_touched_between_a_product_kernels_load_and_the_wait(code
             name = m.group(1) if m else name
             code.setdefault(name, []).append(line)
         for name, lines in code.items():
-            if re.search(r"linear_(walk|walk_wide|dgrad|wgrad_wide)_kernel", name):
+            if re.search(r"linear_(walk|walk_wide|walk_pre|dgrad|wgrad_wide)_kernel", name):
                 checked += 1
                 assert not _touched_in_flight(_decode(lines, "vmcnt"), 64), name
-    assert checked >= 14
+    assert checked >= 17
 
 
 def test_no_register_is_touched_between_its_lds_read_and_the_wait(code_objects):

@@ -306,6 +306,65 @@ def test_products_of_the_widest_tiles(size, modes):
             _check(_call(x, tx if jvp else None, w, None, 0)[0], ref - b.float())
 
 
+# the MLP's first half with its pre-activation kept, in each of the three tiles: rows and columns that fill none, one step, two and many
+KEPT = [(2049, 2296, 704), (8193, 4088, 128), (16129, 1016, 64), (16300, 2040, 1152), (4000, 1016, 1152), (2300, 3064, 448)]
+
+
+@pytest.mark.parametrize("M,N,K", KEPT)
+def test_products_that_keep_their_pre_activation(M, N, K):
+    x, tx, w, b = _operands(M, N, K)
+    lib, p = _lib.load(), lambda t: None if t is None else t.data_ptr()
+    assert lib.dmf_linear_gelu_plan(M, N, K) == 1
+    tref = tx.float() @ w.float().t()
+    for bias in (b, None):
+        ref = torch.nn.functional.linear(x.float(), w.float(), None if bias is None else bias.float())
+        act, tact = torch.func.jvp(lambda t: torch.nn.functional.gelu(t, approximate="tanh"), (ref.double(),), (tref.double(),))
+        for _ in range(2):
+            out = [torch.full((M + 1, N), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(3)]
+            assert lib.dmf_linear_gelu_fwd(p(x), p(tx), p(w), p(bias), *map(p, out), M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+            for got, exp in zip(out, (ref, act, tact)):
+                _check(got[:M], exp)
+                assert (got[M] == 7.0).all()
+
+
+def test_the_kept_form_refuses():
+    lib, t = _lib.load(), torch.zeros(4096, 64, device=DEV, dtype=torch.bfloat16)
+    p = t.data_ptr()
+    assert lib.dmf_linear_gelu_plan(64, 64, 64) == 0 and lib.dmf_linear_gelu_fwd(p, p, p, None, p, p, p, 64, 64, 64, None) == -3
+    assert lib.dmf_linear_gelu_fwd(p, None, p, None, p, p, p, 2049, 2296, 704, None) == -5
+    assert lib.dmf_linear_gelu_fwd(p + 2, p, p, None, p, p, p, 2049, 2296, 704, None) == -6
+
+
+def test_mlp_first_half_with_a_backward_pass():
+    """linear_gelu_tanh at a dual level with gradients: one node, whose gradients are those of the two operators' (the same kernels on the same
+    pre-activation, rounded where theirs is), for every choice of what asks for one, under autocast and in bf16, and differentiated again as far as theirs."""
+    import torch.autograd.forward_ad as fwAD
+    M, N, K = 2049, 2296, 704
+    x, tx, w, b = _operands(M, N, K)
+    gy = torch.randn(M, N, device=DEV).bfloat16()
+    for autocast in (True, False):
+        wt, bias = (w.float(), b.float()) if autocast else (w, b)
+        for ask in ((1, 1, 1), (1, 0, 0), (0, 1, 0), (0, 0, 1)):
+            leaves = [t.detach().clone().requires_grad_(bool(a)) for t, a in zip((x, wt, bias), ask)]
+            wanted = [t for t in leaves if t.requires_grad]
+            res = []
+            for fn in (block_ops.linear_gelu_tanh, lambda *a: block_ops.gelu_tanh(block_ops.dual_linear(*a))):
+                with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast), fwAD.dual_level():
+                    y, ty = fwAD.unpack_dual(fn(fwAD.make_dual(leaves[0], tx), *leaves[1:]))
+                res.append((y.detach(), ty.detach(), *torch.autograd.grad(y, wanted, gy)))
+                if fn is block_ops.linear_gelu_tanh:
+                    assert y.grad_fn.next_functions[0][0].name() == "LinearGeluTanhBackward"   # (behind unpack_dual's view)
+            for got, exp in zip(*res):
+                assert got.dtype == exp.dtype and got.shape == exp.shape and (got.float() - exp.float()).norm() <= 2 ** -7 * exp.float().norm()
+            for got, exp in zip(res[0][2:], res[1][2:]):
+                assert torch.equal(got, exp)
+    a, wt = x.clone().requires_grad_(), w.clone().requires_grad_()
+    with fwAD.dual_level():
+        y = fwAD.unpack_dual(block_ops.linear_gelu_tanh(fwAD.make_dual(a, tx), wt, b))[0]
+    gx = torch.autograd.grad(y, a, gy, create_graph=True)[0]
+    assert torch.autograd.grad(gx, wt, x)[0].shape == wt.shape
+
+
 def test_the_plan_refuses_what_the_entry_refuses():
     plan, name = _lib.load().dmf_linear_fwd_plan, ctypes.create_string_buffer(4)
     for size in ((64, 64, 32), (64, 60, 64), (0, 64, 64), (2 ** 25, 64, 64)):
