@@ -929,6 +929,24 @@ struct WgradParams {
 };
 constexpr int kWgN = 128, kWgK = 192, kWgStage = (kWgN + kWgK) * 128;
 
+// 32 x 32 sums out of a wave's registers through 4 KB of LDS of its own, in whole lines of 128 bytes per row; vector v of row r lies in slot v ^ r % 8.
+// Stored from the registers as they are, 32 bytes of each row at a time, a tile's end took 2 to 3 us more (wide kernel with the partial sums', M 8192:
+// 4608 x 1152 100.4 -> 97.0 us, 1152 x 1152 40.3 -> 38.0, 3072 x 768 53.4 -> 50.9, past the caches 97.3, 39.2, 51.5; linear_wgrad_kernel: 6912 x 1152 M 32 12.9
+// -> 9.8, 3456 x 1152 M 512 15.6 -> 14.6, 768 x 768 M 4096 24.4 -> 23.9).
+__device__ __forceinline__ void store_sums(char* own, const f32x16& a, float* out, int row0, int col0, int N, int K, int lane) {
+  const int c32 = lane & 31, g = lane >> 5, col = col0 + (lane & 7) * 4;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *reinterpret_cast<f32x4*>(own + c32 * 128 + (((2 * q + g) ^ (c32 & 7)) * 16)) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (no other wave is waited for)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 8 * i + (lane >> 3), row = row0 + r;
+    const f32x4 v = *reinterpret_cast<const f32x4*>(own + r * 128 + (((lane & 7) ^ (lane >> 3)) * 16));
+    if (row < N && col < K) *reinterpret_cast<f32x4*>(out + (int64_t)row * K + col) = v;
+  }
+}
+
 __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5, i16 = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1030,7 +1048,8 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
       }
     }
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // (no DMA may outlive the work-group's LDS)
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // (no DMA may be on its way into what follows)
+  __syncthreads();
   float* out = p.out + (int64_t)split * p.N * p.K;
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
@@ -1040,14 +1059,7 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
       if (g == 0 && row < p.N) p.bias[(int64_t)split * p.N + row] = both;
     }
 #pragma unroll
-    for (int n = 0; n < 3; ++n)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int col = k0 + 96 * wn + 32 * n + 8 * q + 4 * g;
-        const f32x16& a = acc[n][m];
-        if (row < p.N && col < p.K)
-          *reinterpret_cast<f32x4*>(out + (int64_t)row * p.K + col) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
-      }
+    for (int n = 0; n < 3; ++n) store_sums(smem + wave * 8192 + ((3 * m + n) & 1) * 4096, acc[n][m], out, n0 + 64 * wm + 32 * m, k0 + 96 * wn + 32 * n, p.N, p.K, lane);
   }
 }
 
@@ -1202,19 +1214,12 @@ __global__ __launch_bounds__(256, 1) void linear_wgrad_wide_kernel(const WgradPa
       if (wn == 0 && g == 0 && row < p.N) p.bias[(int64_t)split * p.N + row] = t;
     }
   }
+  __syncthreads();
   float* out = p.out + (int64_t)split * p.N * p.K;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    const int row = n0 + 64 * m + 32 * wm + c32;
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int col = k0 + 96 * wn + 32 * n + 8 * q + 4 * g;
-        const f32x16& a = acc[n][m];
-        if (row < p.N && col < p.K)
-          *reinterpret_cast<f32x4*>(out + (int64_t)row * p.K + col) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
-      }
+    for (int n = 0; n < NT; ++n) store_sums(smem + wave * 8192 + ((m * NT + n) & 1) * 4096, acc[n][m], out, n0 + 64 * m + 32 * wm, k0 + 96 * wn + 32 * n, p.N, p.K, lane);
   }
 }
 
