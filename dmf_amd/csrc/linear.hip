@@ -1065,8 +1065,9 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
 
 // Much work: the walking forward kernel's tile, stages and order of reads, products and requests (see linear_walk), of 256 columns of g against 192 of x,
 // a work-group per CU.  Both operands lie in 64-column panels of 64 rows and are read by columns.  A step of 6.3 MFLOP takes 0.8 to 1.2 us, by how many
-// CUs take part (two of linear_wgrad_kernel's, the same work, 1.25); start, end and launch 12 us where that takes 9.  With the partial sums' kernel, M 8192:
-// 4608 x 1152 109 -> 100 us, 3072 x 768 59.6 -> 54.7, 3072 x 1024 79.5 -> 71.5, 1152 x 1152 42.5 -> 40.5; M 16384: 4608 x 1152 207 -> 178.
+// CUs take part (two of linear_wgrad_kernel's, the same work, 1.25); start, end and launch 12 us where that takes 9 (both 2 less since the
+// sums leave by store_sums).  With the partial sums' kernel, both before that, M 8192: 4608 x 1152 109 -> 100 us (98 now), 3072 x 768 59.6 -> 54.7 (51),
+// 3072 x 1024 79.5 -> 71.5 (68), 1152 x 1152 42.5 -> 40.5 (38); M 16384: 4608 x 1152 207 -> 178.
 // The two waves that hold the same columns of g sum two chunks of a step each for the bias (two thirds of the room between a chunk's products).
 struct WgradWide : WalkTile<4, 3, 2, 3, 2> { static constexpr int STAGES = NSX * XS + NSW * WS; };
 
@@ -1304,7 +1305,7 @@ extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
 //   M 2048: 1536 x 384 20.0 -> 18.4, but 2304 x 768 21 against 23, 3456 x 1152 28 against 34;
 //   M 4096: 3072 x 768 44 -> 37, 1152 x 1152 35 -> 30, 3072 x 1024 47 -> 46, 4608 x 1152 67 -> 62, but 3456 x 1152 50 against 53, 4096 x 1024 50 against 55;
 //   M 6144: 3456 x 1152 69 against 71, 4608 x 1152 97 -> 81, 4096 x 1024 77 -> 75, 1024 x 4096 80 -> 76 (and no column sum beside it);
-//   M 8192: 3456 x 1152 99 -> 85, 4608 x 1152 125 -> 100, 4096 x 1024 106 -> 92, 1152 x 1152 64 -> 41, 768 x 768 51 -> 27;  M 16384: 3072 x 768 177 ->
+//   M 8192: 3456 x 1152 99 -> 80, 4608 x 1152 125 -> 98, 4096 x 1024 106 -> 88, 1152 x 1152 64 -> 38, 768 x 768 51 -> 26;  M 16384: 3072 x 768 177 ->
 //   91, 4608 x 1152 335 -> 178 (975 TFLOP/s).  The largest result measured is 6912 x 1152 (8 M elements); beyond it the library's products are kept.
 extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return 0;
