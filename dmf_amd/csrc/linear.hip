@@ -881,14 +881,16 @@ static bool dgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
 //     C384 M16384 26.4 -> 19.7; but C384 M2048 10.8 against 12.9, C1024 M2048 26.4 against 28.5, C768 M1536 17.6 against 21.5;
 //   C -> 4C from 768 rows on: C768 M1024 14.4 -> 11.3, C1152 24.7 -> 16.3; not with one to 4/3 rounds of 256 x 192 tiles: C768 M5120 28.2 against 30.6,
 //     C1024 M3072 28.5 against 32.6;
-//   widths that 192 columns do not divide lose in many rows: C1024 M12288 3C -> C 71.6 against 81.5, M16384 89.4 against 94.6 (M8192 59.0 -> 49.6).
+//   widths that 192 columns do not divide lose in many rows: C1024 M12288 3C -> C 71.6 against 81.5, M16384 89.4 against 94.6 (M8192 59.0 -> 49.6);
+//   outputs narrower than a tile lose, M8192 1152 -> 64 9.3 against 11.7, and up to 6144 rows narrow ones that fill none: M3072 3072 -> 320 18.9 against 25.7.
 extern "C" int dmf_linear_dgrad_plan(int64_t M, int N, int K) {
-  if (!dgrad_shape_ok(M, N, K) || M < 768) return 0;
+  if (!dgrad_shape_ok(M, N, K) || M < 768 || K < 192) return 0;
   if (K >= 3 * (int64_t)N) {
     const int64_t cus = dmf::compute_units(), tiles = ((M + 255) / 256) * ((K + 191) / 192);
     return tiles <= cus || 3 * tiles > 4 * cus;
   }
   if (M < 3072 && (M < 2048 || K < 512 || K % 192 != 0)) return 0;
+  if (M < 6144 && K < 512 && K % 192 != 0) return 0;
   return K % 192 == 0 || M < 10240;
 }
 

@@ -394,3 +394,19 @@ def test_deep_products_go_to_the_library_by_rounds(C):
         for rows in (M, M + 1):
             tiles = -(-rows // 128) * -(-C // 96)
             assert _lib.load().dmf_linear_plan(rows, C, 4 * C, 0, 0) == (not 256 < tiles <= 341), rows
+
+
+@pytest.mark.parametrize("N,K", [(1152, 64), (3072, 320), (2304, 768), (768, 3072), (3072, 1024)])
+def test_input_gradients_keep_the_library_where_it_is_faster(N, K):
+    """Narrow outputs, few rows, one to 4/3 rounds of 256 x 192 tiles behind a short depth, many rows of a width that 192 columns do not divide (256 CUs)."""
+    for M in range(64, 20000, 96):
+        tiles = -(-M // 256) * -(-K // 192)
+        if K < 192 or M < 768:
+            own = False
+        elif K >= 3 * N:
+            own = not 256 < tiles <= 341
+        elif K % 192 == 0:
+            own = M >= (2048 if K >= 512 else 3072)
+        else:
+            own = (3072 if K >= 512 else 6144) <= M < 10240
+        assert _lib.load().dmf_linear_dgrad_plan(M, N, K) == own, M
