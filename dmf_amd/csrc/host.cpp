@@ -1035,15 +1035,15 @@ py::object linear_gelu(const Tensor& x_, const Tensor& weight_, const Tensor& bi
 // two operators' nodes do in turn.
 py::object linear_gelu_kept(const Tensor& x_, const Tensor& weight_, const OptTensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
   const int64_t level = current_level();
-  if (level == kUnsupported) return none();
+  if (level == kUnsupported || x_.dim() < 2 || weight_.dim() != 2 || x_.numel() == 0) return none();
+  const int64_t K = x_.size(-1), M = x_.numel() / K, N = weight_.size(0);
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !dmf_linear_gelu_plan(M, (int)N, (int)K)) return none();   // (first: small calls are the host's time)
   const Arg x = unpack(x_), weight = unpack(weight_), bias = unpack(bias_);
-  if (!linear_ok(x, weight, bias) || !x.tan.defined() || !any_grad(x, weight, bias)) return none();
+  if (!linear_ok(x, weight, bias) || !x.tan.defined() || !any_grad(x, weight, bias) || x.data.numel() != M * K || weight.data.size(0) != N) return none();
   const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
   const at::ScalarType dt = autocast_type(x.data);
-  const int64_t K = x.data.size(-1), M = x.data.numel() / K, N = weight.data.size(0);
   const auto dense16 = [](const Tensor& t) { return !t.defined() || (t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0); };
-  if (dt != at::kBFloat16 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !dmf_linear_gelu_plan(M, (int)N, (int)K) || !dense16(x.data) ||
-      !dense16(x.tan) || !dense16(weight.data) || !dense16(bias.data) || (bias.defined() && (bias.data.numel() != N || bias.data.dim() != 1)))
+  if (dt != at::kBFloat16 || !dense16(x.data) || !dense16(x.tan) || !dense16(weight.data) || !dense16(bias.data) || (bias.defined() && (bias.data.numel() != N || bias.data.dim() != 1)))
     return none();
   c10::OptionalDeviceGuard device(x.data.device());
   Tensor h, y, ty;
