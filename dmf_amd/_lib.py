@@ -71,6 +71,7 @@ FUSED_SIGNATURES = {
     "dmf_linear_dgrad": (c_int, [_P] * 3 + [_I] * 3 + [_P]),
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
     "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
+    "dmf_linear_wgrad_sums_plan": (c_int, [_L] + [_I] * 2),
     "dmf_linear_wgrad": (c_int, [_P] * 5 + [_I] * 3 + [_P]),
     "dmf_cast_bf16": (c_int, [_P] * 3 + [_I, _P]),
     "dmf_timestep_embedding_fwd": (c_int, [_P] * 4 + [_L, _I, _F, _I, _P]),
@@ -697,7 +698,8 @@ def linear_wgrad(g, x, bias: bool = False):
                    for t in (g, x)) or torch._C._functorch.peek_interpreter_stack() is not None):
         return None
     (M, N), K = g.shape, x.shape[1]
-    if max(M, N, K) > 0x7fffffff or not load().dmf_linear_wgrad_plan(M, N, K):
+    plan = load().dmf_linear_wgrad_sums_plan if bias else load().dmf_linear_wgrad_plan
+    if max(M, N, K) > 0x7fffffff or not plan(M, N, K):
         return None
     with torch.cuda.device(g.device):
         gw = _empty((N, K), torch.float32, g.device)

@@ -851,7 +851,8 @@ Tensor input_gradient(const Tensor& g, const Tensor& w) {
 // product that stores its accumulators (and no sums).
 Tensor weight_gradient(const Tensor& g, const Tensor& x, Tensor* gb) {
   const int64_t M = g.size(0), N = g.size(1), K = x.size(1);
-  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !readable16(g) || !readable16(x) || !dmf_linear_wgrad_plan(M, (int)N, (int)K))
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !readable16(g) || !readable16(x) ||
+      !(gb ? dmf_linear_wgrad_sums_plan(M, (int)N, (int)K) : dmf_linear_wgrad_plan(M, (int)N, (int)K)))
     return at::mm(g.t(), x, at::kFloat);
   const int64_t need = dmf_linear_wgrad_workspace_floats(M, (int)N, (int)K);
   if (gb) *gb = empty({N}, at::kFloat, x);

@@ -1318,6 +1318,11 @@ extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   return M >= 6144 || result <= 3200000 || (result >= 5000000 && K % dmf::kWgK == 0);
 }
 
+// ... and with the column sums, where the library's product has a column sum beside it (two launches, 8 to 11 us): on every result of the models (us, library
+// and column sum -> here): M 1536: 2304 x 768 27.8 -> 23.5, 3072 x 1024 32.5 -> 29.8;  M 2048: 3072 x 768 36.5 -> 29.0, 3072 x 1024 36.9 -> 36.5, 1152 x 1152 32.2 ->
+// 24.4, 4608 x 1152 48.5 -> 39.3;  M 4096: 3456 x 1152 60.7 -> 49.9, 4096 x 1024 59.6 -> 53.6;  M 5120: 3456 x 1152 71.0 -> 57.0, 1024 x 4096 68.6 -> 63.5.
+extern "C" int dmf_linear_wgrad_sums_plan(int64_t M, int N, int K) { return M <= INT32_MAX && dmf::wgrad_shape_ok(M, N, K) && (int64_t)N * K <= 8000000; }
+
 extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream) {
   if (g == nullptr || x == nullptr || gw == nullptr) return DMF_ATTN_ENULL;
   if (!dmf::wgrad_shape_ok(M, N, K)) return DMF_ATTN_ESHAPE;

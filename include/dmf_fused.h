@@ -68,10 +68,12 @@ DMF_ATTN_API int dmf_linear_dgrad(const void* g, const void* w, void* gx, int M,
  * gw = g^T x, contracted over the M rows: g (M, N), x (M, K), bf16 and dense, gw (N, K) fp32, fp32 accumulation in a fixed order;
  * gbias (N, fp32) or NULL: the column sums of g besides.
  * N and K multiples of 8, fewer than 2^30 elements in each; 16-byte aligned.  workspace: dmf_linear_wgrad_workspace_floats(M, N, K)
- * floats (0: none is needed and NULL will do; -1: shape not covered), not cleared.  dmf_linear_wgrad_plan: as dmf_linear_plan.
+ * floats (0: none is needed and NULL will do; -1: shape not covered), not cleared.  dmf_linear_wgrad_plan: as dmf_linear_plan;
+ * dmf_linear_wgrad_sums_plan: the same for calls that want the column sums, which a library product does not give.
  */
 DMF_ATTN_API int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K);
 DMF_ATTN_API int dmf_linear_wgrad_plan(int64_t M, int N, int K);
+DMF_ATTN_API int dmf_linear_wgrad_sums_plan(int64_t M, int N, int K);
 DMF_ATTN_API int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream);
 
 /*

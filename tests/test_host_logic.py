@@ -396,6 +396,18 @@ def test_deep_products_go_to_the_library_by_rounds(C):
             assert _lib.load().dmf_linear_plan(rows, C, 4 * C, 0, 0) == (not 256 < tiles <= 341), rows
 
 
+def test_weight_gradients_with_column_sums_are_the_packages():
+    """Wherever the product alone is, and on every result of the models between, where it is the library's; not on what the kernel does not cover."""
+    lib = _lib.load()
+    for C in (384, 768, 1024, 1152):
+        for N, K in ((3 * C, C), (C, C), (4 * C, C), (C, 4 * C), (6 * C, C)):
+            for M in (1, 100, 1536, 2048, 3333, 4096, 5120, 8192, 32768):
+                assert lib.dmf_linear_wgrad_sums_plan(M, N, K) == 1
+    assert not lib.dmf_linear_wgrad_plan(2048, 3456, 1152)
+    for size in ((64, 60, 64), (0, 64, 64), (2048, 8192, 1024), (3, 8, 1 << 25)):
+        assert not lib.dmf_linear_wgrad_sums_plan(*size)
+
+
 @pytest.mark.parametrize("N,K", [(1152, 64), (3072, 320), (2304, 768), (768, 3072), (3072, 1024)])
 def test_input_gradients_keep_the_library_where_it_is_faster(N, K):
     """Narrow outputs, few rows, one to 4/3 rounds of 256 x 192 tiles behind a short depth, many rows of a width that 192 columns do not divide (256 CUs)."""
