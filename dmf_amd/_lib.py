@@ -170,6 +170,18 @@ def _raw(t):
     return t
 
 
+def ordinary(t):
+    """``t``; what stands for something else than its buffer holds -- a view of the negative (torch._neg_view), zeros without storage -- made
+    into an ordinary tensor, which a kernel can read by address."""
+    if not (t.is_neg() or t._is_zerotensor()):
+        return t
+    return torch.zeros(t.shape, dtype=t.dtype, device=t.device) if t._is_zerotensor() else t.resolve_neg()
+
+
+def _in_memory(t):
+    return None if t is None else _raw(ordinary(_raw(t)))
+
+
 def _apply(fn_cls, args):
     """``fn_cls.apply(*args)`` minus what ``torch.autograd.Function.apply`` does in Python
     before handing over to the C++ node constructor: binding the arguments against
@@ -251,7 +263,7 @@ def _empty(shape, dtype, device) -> torch.Tensor:
 def _prep(t: torch.Tensor) -> torch.Tensor:
     """Kernels need unit last-dim stride and 16-byte aligned rows; views into a
     packed qkv buffer already satisfy this and are passed through untouched."""
-    t = _raw(t)
+    t = _in_memory(t)
     eb = t.element_size()
     ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((s * eb) % 16 == 0 for s in t.stride()[:-1])
     if ok:
@@ -346,7 +358,7 @@ def fwd_qnorm(q, k, v, tq, tk, tv, q_gain, eps: float, scale: float, need_lse: b
     else:
         _check_inputs(q, k, v)
         q, k, v = map(_prep, (q, k, v))
-    gain = _raw(q_gain)
+    gain = _in_memory(q_gain)
     if gain.dim() != 1 or gain.shape[0] != q.shape[-1] or gain.device != q.device:
         raise ValueError("fwd_qnorm: q_gain must be a (D) tensor on the device of q")
     if q.dtype != torch.bfloat16:
@@ -389,7 +401,7 @@ def fwd_qknorm(q, k, v, tq, tk, tv, q_gain, k_gain, eps: float, scale: float, ne
         if gn is None and name == "k_gain":   # k is already normalised
             gains.append(None)
             continue
-        gn = _raw(gn)
+        gn = _in_memory(gn)
         if gn.dim() != 1 or gn.shape[0] != q.shape[-1] or gn.device != q.device:
             raise ValueError(f"fwd_qknorm: {name} must be a (D) tensor on the device of q")
         gains.append(_raw(gn.float().contiguous()))   # exact for a bf16 gain (a model cast to bf16 as a whole)
@@ -458,7 +470,7 @@ def bwd_qknorm(dout, q_hat, k_hat, v, o, lse, q, k, q_gain, k_gain, eps: float, 
     dout, q_hat, k_hat, v, o, q, k = map(_prep, (dout, q_hat, k_hat, v, o, q, k))
     if q.dtype != torch.bfloat16:
         return None
-    gains = [_raw(_raw(g).float().contiguous()) for g in (q_gain, k_gain)]
+    gains = [_raw(_in_memory(g).float().contiguous()) for g in (q_gain, k_gain)]
     lse = _raw(_raw(lse).contiguous())
     dq, dk, dv = map(_raw, out)
     _check_inputs(q, dq, dk, dv)
@@ -489,7 +501,7 @@ def _dense(t):
     """Contiguous, functorch-unwrapped (None passes through)."""
     if t is None:
         return None
-    t = _raw(t)
+    t = _in_memory(t)
     return t if t.is_contiguous() else _raw(t.contiguous())
 
 
@@ -499,7 +511,7 @@ def _mod(t, B: int, C: int):
     are passed through without a copy."""
     if t is None:
         return None, 0
-    t = _raw(t)
+    t = _in_memory(t)
     if t.numel() != B * C or t.shape[0] != B or t.shape[-1] != C:
         raise ValueError(f"expected a (B, C) or (B, 1, C) modulation tensor with B={B}, C={C}, got {tuple(t.shape)}")
     eb = t.element_size()
@@ -677,7 +689,7 @@ def linear_fwd(x, tx, w, bias, gelu: bool = False):
     if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0
             or len(_interpreters()) > 1
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous()
-                   for t in present) or any(t.data_ptr() % 16 for t in present)):
+                   or t.is_neg() or t._is_zerotensor() for t in present) or any(t.data_ptr() % 16 for t in present)):
         return None
     M, K, N = x.shape[0], x.shape[1], w.shape[0]
     if w.dim() != 2 or w.shape[1] != K or (bias is not None and bias.shape != (N,)) or max(M, N, K) > 0x7fffffff or not load().dmf_linear_plan(
@@ -694,8 +706,8 @@ def linear_wgrad(g, x, bias: bool = False):
     """``(g^T x, column sums of g or None)`` in fp32 for (M, N) g and (M, K) x by the package's own kernel; None where a library product is the better choice or
     the operands are not plain dense bf16 tensors on the GPU."""
     if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
-            or any(type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16
-                   for t in (g, x)) or torch._C._functorch.peek_interpreter_stack() is not None):
+            or any(type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.bfloat16 or not t.is_contiguous() or t.is_neg() or t._is_zerotensor()
+                   or t.data_ptr() % 16 for t in (g, x)) or torch._C._functorch.peek_interpreter_stack() is not None):
         return None
     (M, N), K = g.shape, x.shape[1]
     plan = load().dmf_linear_wgrad_sums_plan if bias else load().dmf_linear_wgrad_plan

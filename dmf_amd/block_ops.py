@@ -253,8 +253,8 @@ class DualLinearFunc(torch.autograd.Function):
         _primal_only(gty)
         if gy is None:
             return (None,) * 6
-        x, w = ctx.saved_tensors
-        g2 = gy.reshape(-1, gy.shape[-1]).to(w.dtype)
+        x, w = map(_lib.ordinary, ctx.saved_tensors)
+        g2 = _lib.ordinary(gy).reshape(-1, gy.shape[-1]).to(w.dtype)
         want_gx, want_gw = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
         want_gb = ctx.bias_dtype is not None and ctx.needs_input_grad[3]
         gx = gw = gb = None

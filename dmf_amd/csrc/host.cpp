@@ -102,7 +102,7 @@ C10_NOINLINE Tensor made_ordinary(const Tensor& t) {
   return t._is_zerotensor() ? at::zeros(t.sizes(), t.options()) : t.resolve_neg();
 }
 inline Tensor in_memory(Tensor t) {
-  if (C10_UNLIKELY(t.is_neg() || t._is_zerotensor())) return made_ordinary(t);
+  if (C10_UNLIKELY(t.defined() && (t.is_neg() || t._is_zerotensor()))) return made_ordinary(t);
   return t;
 }
 
@@ -206,7 +206,11 @@ struct KernelNode : Node {
     const auto first = std::find_if(primal.begin(), primal.end(), [](const Tensor& g) { return g.defined(); });
     c10::OptionalDeviceGuard device(first->device());
     std::optional<Below> below;
-    if (!torch_ops || plain_call(primal)) below.emplace();
+    if (!torch_ops || plain_call(primal)) {   // the kernels' route: read by address
+      below.emplace();
+      for (Tensor& t : s) t = in_memory(std::move(t));
+      for (Tensor& t : primal) t = in_memory(std::move(t));
+    }
     variable_list out = fn(*this, s, primal);
     out.resize(n);
     return out;
@@ -786,7 +790,7 @@ py::object activation(const Tensor& x_, Act act) {
           const Tensor s = at::sigmoid(sv[0]);
           return {g[0].to(sv[0].scalar_type()) * (s * (1 + sv[0] * (1 - s)))};
         }
-        const Tensor x = dense(in_memory(sv[0])), gx = dense_like(x), gy = dense(g[0]);
+        const Tensor x = dense(sv[0]), gx = dense_like(x), gy = dense(g[0]);
         check(dmf_silu_bwd(ptr(gy), ptr(x), mptr(gx), x.numel(), code_of(x), code_of(gy), stream_of(x)), "dmf_silu_bwd");
         return {gx};
       };

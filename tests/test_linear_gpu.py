@@ -191,6 +191,48 @@ def test_weight_gradient_routes():
     assert _lib.linear_wgrad(dense[:, ::2], x) is None and _lib.linear_wgrad(dense.float(), x.float()) is None
 
 
+@pytest.mark.parametrize("M,N,K", [(130, 256, 128), (3072, 384, 768), (2048, 1152, 1152)])
+def test_gradients_that_stand_for_something_else(M, N, K):
+    """Gradients, inputs and saved tensors that are views of their buffer's negative, or zeros without storage: every gradient of a layer and of a
+    layer with its activation is that of the ordinary tensor, to the bit, on the native and on the Python route."""
+    import torch.autograd.forward_ad as fwAD
+    x, tx, w, b = _operands(M, N, K)
+    dense = torch.randn(M, N, device=DEV).bfloat16()
+    zero = torch._efficientzerotensor((M, N), dtype=torch.bfloat16, device=DEV)
+    assert zero._is_zerotensor() and torch._neg_view(dense).is_neg()
+
+    def grads(layer, gy, x, hooks=None):
+        leaves = [x.detach().requires_grad_() if not x.is_neg() else x, w.float().requires_grad_(), b.float().requires_grad_()]
+        wanted = leaves[not leaves[0].requires_grad:]
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            if hooks:
+                with torch.autograd.graph.saved_tensors_hooks(*hooks):
+                    y = layer(*leaves)
+            else:
+                y = layer(*leaves)
+        return torch.autograd.grad(y, wanted, gy)
+
+    def kept(x, w, b):
+        with fwAD.dual_level():
+            return fwAD.unpack_dual(block_ops.linear_gelu_tanh(fwAD.make_dual(x, tx), w, b))[0]
+
+    def python(x, w, b):
+        return block_ops.DualLinearFunc.apply(x, None, w, b, None, None)[0]
+
+    negated = (lambda t: torch.neg(t), lambda t: torch._neg_view(t))
+    for layer in (block_ops.dual_linear, python, lambda *a: block_ops.gelu_tanh(block_ops.dual_linear(*a)), kept):
+        plain, at_zero = grads(layer, dense, x), grads(layer, zero, x)
+        for got, exp in zip(grads(layer, torch._neg_view(-dense), x), plain):
+            assert torch.equal(got, exp)
+        assert all(bool((g == 0).all()) for g in at_zero)
+        for got, exp in zip(grads(layer, dense, torch._neg_view(-x)), plain[1:]):
+            assert torch.equal(got, exp)
+        for got, exp in zip(grads(layer, dense, x, negated), plain):
+            assert torch.equal(got, exp)
+    assert _lib.linear_wgrad(torch._neg_view(dense), x) is None and _lib.linear_wgrad(dense, torch._neg_view(x)) is None
+    assert _lib.linear_fwd(torch._neg_view(x), None, w, b) is None
+
+
 def test_weight_gradient_refuses():
     g, x = torch.randn(64, 64, device=DEV).bfloat16(), torch.randn(64, 64, device=DEV).bfloat16()
     out, lib = torch.empty(64, 64, device=DEV), _lib.load()

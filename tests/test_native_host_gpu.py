@@ -511,3 +511,23 @@ def test_views_that_stand_for_the_negative_of_their_buffer():
     part = block_ops.chunk_last(torch._neg_view(x), 2)[0]
     x[0, 0, 0] = 5.0
     assert part[0, 0, 0] == -5.0
+
+
+def test_gradients_that_stand_for_the_negative_of_their_buffer():
+    """A torch._neg_view as an incoming gradient, and zeros without storage: the gradients of the ordinary tensors, on the native and on the Python
+    route of every operator."""
+    r = lambda *s: torch.randn(*s, device=DEV)
+    cases = [_attn_case(k, torch.bfloat16) for k in ("separate", "packed", "qknorm")]
+    cases += [(block_ops.ln_modulate, [r(2, 16, 64), r(2, 64), r(2, 64)]), (block_ops.gate_residual, [r(2, 16, 64), r(2, 64), r(2, 16, 64)]),
+              (block_ops.gelu_tanh, [r(3, 64)]), (block_ops.silu, [r(3, 64)]), (block_ops.rms_norm, [r(2, 16, 2, 64), r(64)]),
+              (lambda *a: torch.cat(block_ops.residual_ln_modulate(*a)), [r(2, 16, 64), r(2, 64), r(2, 16, 64), r(2, 64), r(2, 64)])]
+    for fn, args in cases:
+        def grads(gy):
+            leaves = [a.detach().clone().requires_grad_() for a in args]
+            return torch.autograd.grad(fn(*leaves), leaves, gy)
+        gy = torch.randn_like(fn(*args))
+        zero = torch._efficientzerotensor(gy.shape, dtype=gy.dtype, device=DEV)
+        for route in (lambda f: f(), _general):
+            plain = route(lambda: grads(gy))
+            assert all(torch.equal(g, e) for g, e in zip(route(lambda: grads(torch._neg_view(-gy))), plain))
+            assert not any(bool(g.any()) for g in route(lambda: grads(zero)))
