@@ -205,6 +205,8 @@ struct KernelNode : Node {
     if (!any) return variable_list(n);
     const auto first = std::find_if(primal.begin(), primal.end(), [](const Tensor& g) { return g.defined(); });
     c10::OptionalDeviceGuard device(first->device());
+    // (operands have their types; under autocast torch's rule for gelu's second derivative gives a tangent of another type than its primal's)
+    c10::impl::ExcludeDispatchKeyGuard no_autocast{c10::autocast_dispatch_keyset};
     std::optional<Below> below;
     if (!torch_ops || plain_call(primal)) {   // the kernels' route: read by address
       below.emplace();
@@ -1037,7 +1039,7 @@ py::object linear_gelu(const Tensor& x_, const Tensor& weight_, const Tensor& bi
 }
 
 // gelu_tanh(linear(x)) with a tangent and a backward pass to come: one kernel, which keeps the pre-activation besides, and one node that does what the
-// two operators' nodes do in turn.
+// two operators' nodes do in turn, and is differentiated again as torch's operators are.
 py::object linear_gelu_kept(const Tensor& x_, const Tensor& weight_, const OptTensor& bias_, const OptTensor& w_lp, const OptTensor& b_lp) {
   const int64_t level = current_level();
   if (level == kUnsupported || x_.dim() < 2 || weight_.dim() != 2 || x_.numel() == 0) return none();
@@ -1069,16 +1071,21 @@ py::object linear_gelu_kept(const Tensor& x_, const Tensor& weight_, const OptTe
     ty = empty(sizes, dt, x.data);
     check(dmf_linear_gelu_fwd(ptr(x2), ptr(tx2), ptr(o.w), ptr(o.b), mptr(h), mptr(y), mptr(ty), (int)M, (int)N, (int)K, stream_of(x.data)), "dmf_linear_gelu_fwd");
   }
-  std::shared_ptr<KernelNode> node = make_node("LinearGeluTanhBackward", {x, weight, bias}, {x.var, o.w.is_same(weight.data) ? weight.var : o.w, h});
+  // (variables and copies as DualLinearBackward has them)
+  std::shared_ptr<KernelNode> node = make_node("LinearGeluTanhBackward", {x, weight, bias},
+                                               {x.var, o.w.is_same(weight.data) ? weight.var : o.w, h, bias.defined() && o.b.is_same(bias.data) ? bias.var : o.b});
   node->torch_ops = true;
   node->fn = [wt = weight.data.scalar_type(), has_bias = bias.defined(), bt = bias.defined() ? bias.data.scalar_type() : at::kFloat](
                  KernelNode& node, const std::vector<Tensor>& sv, const variable_list& g) {
+    const Tensor &w = sv[1], &b = sv[3];
     Tensor gh;
-    {
-      const Below below;   // (the activation's gradient is a constant where it is differentiated again)
-      const Tensor h = dense(in_memory(sv[2])), gy = dense(g[0].to(h.scalar_type()));
+    if (KernelNode::plain_call({g[0]})) {
+      const Tensor h = dense(sv[2]), gy = dense(g[0].to(h.scalar_type()));
       gh = dense_like(h);
       check(dmf_gelu_tanh_bwd(ptr(gy), ptr(h), mptr(gh), h.numel(), code_of(h), stream_of(h)), "dmf_gelu_tanh_bwd");
+    } else {   // differentiated again or mapped over: the pre-activation once more, as a function of the variables
+      const Tensor x2 = sv[0].reshape({-1, sv[0].size(-1)}).to(w.scalar_type()), pre = b.defined() ? at::addmm(b, x2, w.t()) : at::mm(x2, w.t());
+      gh = at::gelu_backward(g[0].to(pre.scalar_type()), pre.view(sv[2].sizes()), "tanh");
     }
     return linear_backward(node, sv[0], sv[1], gh, wt, bt, has_bias);
   };

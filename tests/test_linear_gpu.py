@@ -407,6 +407,47 @@ def test_mlp_first_half_with_a_backward_pass():
     assert torch.autograd.grad(gx, wt, x)[0].shape == wt.shape
 
 
+@pytest.mark.parametrize("case", ["second", "over_reverse"])
+@pytest.mark.parametrize("autocast", [True, False])
+@pytest.mark.parametrize("M,N,K", [(2049, 2296, 704), (2048, 8192, 1024)])
+def test_mlp_first_half_differentiated_again(case, autocast, M, N, K):
+    """The gradients of the kept form differentiated once more (create_graph=True), and with an incoming gradient that carries a tangent
+    (forward over reverse), against the same expressions of torch's operators in fp64 on the same operands.  The weight's copy under autocast is a
+    constant where a gradient is differentiated again.  A result is the sum of at most four products of at most five bf16 factors each, every one
+    of them rounded once more (2^-9): 2^-9 times 6, and a factor 2 for terms that cancel."""
+    import torch.autograd.forward_ad as fwAD
+    tol = 12 * 2 ** -9
+    gen = torch.Generator(device=DEV).manual_seed(11)
+    x, tx, w, b = _operands(M, N, K)
+    gy, tgy = ((torch.randn(M, N, generator=gen, device=DEV) * M ** -0.5).bfloat16() for _ in range(2))
+    vx, vw = torch.randn(M, K, generator=gen, device=DEV).bfloat16(), (torch.randn(N, K, generator=gen, device=DEV) * K ** -0.5).bfloat16()
+    assert _lib.load().dmf_linear_gelu_plan(M, N, K) == 1
+
+    def run(fn, dt, pdt, constant_copy):
+        leaves = [x.to(dt).requires_grad_(), w.to(pdt).requires_grad_(), b.to(pdt).requires_grad_()]
+        g = gy.to(dt).requires_grad_(case == "second")
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast and dt != torch.float64), fwAD.dual_level():
+            y = fn(fwAD.make_dual(leaves[0], tx.to(dt)), *leaves[1:])
+            if case == "over_reverse":
+                # (the tangent of x as well as of the gradient)
+                grads = torch.autograd.grad(y, leaves, fwAD.make_dual(g, tgy.to(dt)))
+                return [fwAD.unpack_dual(t).tangent for t in grads]
+            y = fwAD.unpack_dual(y)[0]
+        gx, gw = torch.autograd.grad(y, leaves[:2], g, create_graph=True)
+        # (a second gradient for x and for what came in; the parameters' too where they are not copied)
+        first = (gx * vx.to(gx.dtype)).float().sum() if dt != torch.float64 else (gx * vx.double()).sum()
+        second = (gw * vw.to(gw.dtype)).float().sum() if dt != torch.float64 else (gw * vw.double()).sum()
+        wanted = [leaves[0], g] + ([] if constant_copy else leaves[1:])
+        return [*torch.autograd.grad(first, wanted, retain_graph=True), *torch.autograd.grad(second, wanted)]
+
+    got = run(block_ops.linear_gelu_tanh, torch.bfloat16, torch.float32 if autocast else torch.bfloat16, autocast)
+    exp = run(lambda x, w, b: torch.nn.functional.gelu(torch.nn.functional.linear(x, w, b), approximate="tanh"), torch.float64, torch.float64, autocast)
+    assert len(got) == len(exp)
+    for i, (a, e) in enumerate(zip(got, exp)):
+        assert a is not None and a.shape == e.shape, i
+        assert (a.double() - e).norm() <= tol * e.norm(), (i, float((a.double() - e).norm() / e.norm()))
+
+
 def test_the_plan_refuses_what_the_entry_refuses():
     plan, name = _lib.load().dmf_linear_fwd_plan, ctypes.create_string_buffer(4)
     for size in ((64, 64, 32), (64, 60, 64), (0, 64, 64), (2 ** 25, 64, 64)):
