@@ -50,6 +50,11 @@ def _primal_only(*tangent_cotangents):
             "with block_ops='torch'")
 
 
+def _again(g) -> bool:
+    """True where a gradient is to be differentiated again (create_graph=True) or carries a tangent: what can be made of torch's operators is."""
+    return torch.is_grad_enabled() or fwAD.unpack_dual(g).tangent is not None
+
+
 def _like(g, ref):
     """Gradient of a (B, C) modulation operand reshaped to the operand's shape."""
     return g.reshape(ref)
@@ -148,6 +153,8 @@ class GeluTanhFunc(torch.autograd.Function):
         if gy is None:
             return None, None
         (x,) = ctx.saved_tensors
+        if _again(gy):
+            return torch.ops.aten.gelu_backward(gy.to(x.dtype), x, approximate="tanh"), None
         return _lib.gelu_tanh_bwd(gy.to(x.dtype), x), None
 
 
@@ -169,7 +176,7 @@ class SiluFunc(torch.autograd.Function):
         if gy is None:
             return None, None, None
         (x,) = ctx.saved_tensors
-        if torch.is_grad_enabled():   # differentiated again: operators that can be
+        if _again(gy):
             s = torch.sigmoid(x)
             return gy.to(x.dtype) * (s * (1 + x * (1 - s))), None, None
         return _lib.silu_bwd(gy, x), None, None

@@ -777,15 +777,16 @@ py::object activation(const Tensor& x_, Act act) {
   std::shared_ptr<KernelNode> node;
   if (any_grad(x)) {
     if (act == Act::gelu) {
-      node = make_node("GeluTanhBackward", {x}, {xd});
+      node = make_node("GeluTanhBackward", {x}, {x.var});   // (the variable itself, for create_graph=True)
+      node->torch_ops = true;
       node->fn = [](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
-        const Tensor& x = sv[0];
-        const Tensor gx = dense_like(x), gy = dense(g[0].to(x.scalar_type()));
+        if (!KernelNode::plain_call({g[0]})) return {at::gelu_backward(g[0].to(sv[0].scalar_type()), sv[0], "tanh")};
+        const Tensor x = dense(sv[0]), gx = dense_like(x), gy = dense(g[0].to(x.scalar_type()));
         check(dmf_gelu_tanh_bwd(ptr(gy), ptr(x), mptr(gx), x.numel(), code_of(x), stream_of(x)), "dmf_gelu_tanh_bwd");
         return {gx};
       };
     } else {
-      node = make_node("SiluBackward", {x}, {x.var});   // (the variable itself, for create_graph=True)
+      node = make_node("SiluBackward", {x}, {x.var});
       node->torch_ops = true;
       node->fn = [](KernelNode&, const std::vector<Tensor>& sv, const variable_list& g) -> variable_list {
         if (!KernelNode::plain_call({g[0]})) {

@@ -206,6 +206,36 @@ def test_linear_and_chunk_stay_twice_differentiable():
             assert (got[i] - exp).norm() <= 1e-5 * exp.norm()
 
 
+@pytest.mark.parametrize("route", [lambda f: f(), _general], ids=["native", "python"])
+@pytest.mark.parametrize("case", ["second", "over_reverse"])
+@pytest.mark.parametrize("op", ["gelu_tanh", "silu"])
+def test_operators_differentiated_again(op, case, route):
+    """Gradients of create_graph=True differentiated once more, and gradients that carry a tangent (forward over reverse), against torch's operators in
+    fp64: elementwise in fp32 and products of up to 64 terms.  The layer has the size from which its input gradient is the package's own (M 3072, bf16):
+    2^-9 of each of the at most three factors that are rounded."""
+    bf16 = op == "dual_linear"
+    g = torch.Generator(device=DEV).manual_seed(12)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16 if bf16 else torch.float32)
+    args = [r(3072, 192), r(64, 192)] if bf16 else [2 * r(24, 64)]
+    gy, tgy = r(3072, 64) if bf16 else r(24, 64), r(3072, 64) if bf16 else r(24, 64)
+    probes = [r(*a.shape) for a in args]
+    assert not bf16 or _lib.load().dmf_linear_dgrad_plan(3072, 64, 192) == 1
+
+    def run(fn, dt):
+        leaves, up = [a.to(dt).requires_grad_() for a in args], gy.to(dt)
+        if case == "over_reverse":
+            with fwAD.dual_level():
+                return [fwAD.unpack_dual(t).tangent for t in torch.autograd.grad(fn(*leaves), leaves, fwAD.make_dual(up, tgy.to(dt)))]
+        up.requires_grad_()
+        grads = torch.autograd.grad(fn(*leaves), leaves, up, create_graph=True)
+        return torch.autograd.grad(sum((a * p.to(dt)).sum(dtype=torch.float32 if bf16 and dt != torch.float64 else dt) for a, p in zip(grads, probes)), [*leaves, up])
+
+    ref = {"gelu_tanh": lambda x: torch.nn.functional.gelu(x, approximate="tanh"), "silu": lambda x: x * torch.sigmoid(x), "dual_linear": torch.nn.functional.linear}[op]
+    got, exp = route(lambda: run(getattr(block_ops, op), args[0].dtype)), run(ref, torch.float64)
+    for a, e in zip(got, exp):
+        assert a is not None and (a.double() - e).norm() <= (3 * 2 ** -9 if bf16 else 1e-5) * e.norm()
+
+
 def test_graphs_that_never_run_backward_are_freed():
     """A gradient-enabled call whose results are dropped without a backward pass leaves nothing behind: a node that holds its own output
     would keep the graph above it."""
