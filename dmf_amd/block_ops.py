@@ -265,7 +265,7 @@ class DualLinearFunc(torch.autograd.Function):
         want_gx, want_gw = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
         want_gb = ctx.bias_dtype is not None and ctx.needs_input_grad[3]
         gx = gw = gb = None
-        again = torch.is_grad_enabled()   # to be differentiated again: operators that can be
+        again = _again(gy)
         # (in one stream: next to each other in two, the products slow one another down and each fork and join idles the GPU)
         if want_gw:
             x2 = x.reshape(-1, x.shape[-1]).to(w.dtype)

@@ -208,7 +208,7 @@ def test_linear_and_chunk_stay_twice_differentiable():
 
 @pytest.mark.parametrize("route", [lambda f: f(), _general], ids=["native", "python"])
 @pytest.mark.parametrize("case", ["second", "over_reverse"])
-@pytest.mark.parametrize("op", ["gelu_tanh", "silu"])
+@pytest.mark.parametrize("op", ["gelu_tanh", "silu", "dual_linear"])
 def test_operators_differentiated_again(op, case, route):
     """Gradients of create_graph=True differentiated once more, and gradients that carry a tangent (forward over reverse), against torch's operators in
     fp64: elementwise in fp32 and products of up to 64 terms.  The layer has the size from which its input gradient is the package's own (M 3072, bf16):
