@@ -711,7 +711,7 @@ def linear_wgrad(g, x, bias: bool = False):
         return None
     (M, N), K = g.shape, x.shape[1]
     plan = load().dmf_linear_wgrad_sums_plan if bias else load().dmf_linear_wgrad_plan
-    if max(M, N, K) > 0x7fffffff or not plan(M, N, K):
+    if max(M, N, K) > 0x7fffffff or x.shape[0] != M or x.device != g.device or not plan(M, N, K):
         return None
     with torch.cuda.device(g.device):
         gw = _empty((N, K), torch.float32, g.device)

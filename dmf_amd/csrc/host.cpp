@@ -23,6 +23,7 @@
 #include <torch/version.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/functorch/DynamicLayer.h>
 #include <ATen/functorch/TensorWrapper.h>
@@ -177,6 +178,13 @@ struct KernelNode : Node {
   using Fn = std::function<variable_list(KernelNode&, const std::vector<Tensor>&, const variable_list&)>;
   const char* label;
   std::vector<SavedVariable> saved;
+  struct Form {
+    bool defined;
+    at::DimVector sizes, strides;
+    at::ScalarType type;
+    at::Device device;
+  };
+  std::vector<Form> forms;   // of `saved`, where saved-tensor hooks may hand back something else
   Fn fn;
   bool dual = false, refuse_tangent_gradient = true;
   bool torch_ops = false;   // fn can be made of differentiable, batchable calls (see plain_call)
@@ -191,6 +199,7 @@ struct KernelNode : Node {
     std::vector<Tensor> s;
     s.reserve(saved.size());
     for (auto& v : saved) s.push_back(v.unpack(shared_from_this()));
+    for (size_t i = 0; i < forms.size(); ++i) as_saved(s[i], forms[i]);
     const size_t n = num_outputs();
     variable_list primal;
     bool any = false;
@@ -216,6 +225,16 @@ struct KernelNode : Node {
     variable_list out = fn(*this, s, primal);
     out.resize(n);
     return out;
+  }
+  // The kernels read by address, in sizes and types of the call: what a hook hands back has to be of the device and the sizes of what it was
+  // given; type and strides may differ (torch_ops: fn sees to them).
+  void as_saved(Tensor& t, const Form& f) const {
+    if (!f.defined) return;
+    TORCH_CHECK(t.defined() && t.layout() == at::kStrided && t.device() == f.device && t.sizes() == at::IntArrayRef(f.sizes), label,
+                ": a saved-tensor hook handed back something else than it was given, a tensor of sizes ", at::IntArrayRef(f.sizes), " on ", f.device);
+    if (torch_ops) return;
+    if (t.scalar_type() != f.type) t = t.to(f.type);
+    if (t.strides() != at::IntArrayRef(f.strides)) t = t.contiguous();
   }
   // False under create_graph=True, for batched gradients and for gradients that carry a tangent (forward over reverse at a dual
   // level): there, what consists of torch operators stays differentiable and mapped, as autograd.Function's backward is.
@@ -243,6 +262,11 @@ std::shared_ptr<KernelNode> make_node(const char* name, std::initializer_list<Ar
   node->set_next_edges(std::move(edges));
   node->saved.reserve(save.size());
   for (const Tensor& t : save) node->saved.emplace_back(t, false);
+  if (at::SavedTensorDefaultHooks::get_hooks()) {
+    for (const Tensor& t : save)
+      node->forms.push_back(t.defined() ? KernelNode::Form{true, at::DimVector(t.sizes()), at::DimVector(t.strides()), t.scalar_type(), t.device()}
+                                        : KernelNode::Form{false, {}, {}, at::kFloat, at::kCPU});
+  }
   return node;
 }
 
@@ -835,19 +859,21 @@ Tensor column_sum(const Tensor& x, at::ScalarType dt) {
   return out;
 }
 
+// An operand of a layer's backward pass that a kernel may read: it comes out of a saved variable, whose hooks may hand back whatever a product takes
+bool addressable(const Tensor& t, const Tensor& like) {
+  return t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && t.device() == like.device() && !t.is_neg() && !t._is_zerotensor() &&
+         !t.key_set().has(c10::DispatchKey::Python);
+}
+
 bool readable16(const Tensor& t) {
   return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
 }
 
 // g w: the package's own kernel where it reads the operands as they are and is the faster one, else a library product
 Tensor input_gradient(const Tensor& g, const Tensor& w) {
-  // (w comes out of a saved variable, whose hooks may hand back whatever a product takes)
-  const auto ordinary = [](const Tensor& t) {
-    return t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && !t.is_neg() && !t._is_zerotensor() && !t.key_set().has(c10::DispatchKey::Python);
-  };
   const int64_t M = g.size(0), N = g.size(1), K = w.dim() == 2 ? w.size(1) : 0;
-  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || w.dim() != 2 || w.size(0) != N || !dmf_linear_dgrad_plan(M, (int)N, (int)K) || !ordinary(g) || !ordinary(w) ||
-      w.device() != g.device() || !readable16(g) || !readable16(w))
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || w.dim() != 2 || w.size(0) != N || !dmf_linear_dgrad_plan(M, (int)N, (int)K) || !addressable(g, g) ||
+      !addressable(w, g) || !readable16(g) || !readable16(w))
     return at::mm(g, w);
   const Tensor gx = empty({M, K}, at::kBFloat16, g);
   check(dmf_linear_dgrad(ptr(g), ptr(w), mptr(gx), (int)M, (int)N, (int)K, stream_of(g)), "dmf_linear_dgrad");
@@ -858,7 +884,7 @@ Tensor input_gradient(const Tensor& g, const Tensor& w) {
 // product that stores its accumulators (and no sums).
 Tensor weight_gradient(const Tensor& g, const Tensor& x, Tensor* gb) {
   const int64_t M = g.size(0), N = g.size(1), K = x.size(1);
-  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !readable16(g) || !readable16(x) ||
+  if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || x.size(0) != M || !addressable(g, g) || !addressable(x, g) || !readable16(g) || !readable16(x) ||
       !(gb ? dmf_linear_wgrad_sums_plan(M, (int)N, (int)K) : dmf_linear_wgrad_plan(M, (int)N, (int)K)))
     return at::mm(g.t(), x, at::kFloat);
   const int64_t need = dmf_linear_wgrad_workspace_floats(M, (int)N, (int)K);

@@ -561,3 +561,28 @@ def test_gradients_that_stand_for_the_negative_of_their_buffer():
             plain = route(lambda: grads(gy))
             assert all(torch.equal(g, e) for g, e in zip(route(lambda: grads(torch._neg_view(-gy))), plain))
             assert not any(bool(g.any()) for g in route(lambda: grads(zero)))
+
+
+def test_what_saved_tensor_hooks_hand_back():
+    """Other strides are read (or copied) and another type is cast; what is not of the saved tensor's device and sizes is refused: nothing is read past its
+    end, or through a host address."""
+    r = lambda *s: torch.randn(*s, device=DEV)
+    cases = [_attn_case(k, torch.bfloat16) for k in ("separate", "packed", "qknorm")]
+    cases += [(block_ops.ln_modulate, [r(2, 16, 64), r(2, 64), r(2, 64)]), (block_ops.gate_residual, [r(2, 16, 64), r(2, 64), r(2, 16, 64)]),
+              (block_ops.gelu_tanh, [r(3, 64)]), (block_ops.silu, [r(3, 64)]), (block_ops.dual_linear, [r(3, 64), r(32, 64), r(32)])]
+    for fn, args in cases:
+        def grads(pack, unpack):
+            leaves = [a.detach().clone().requires_grad_() for a in args]
+            with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+                y = fn(*leaves)
+            return torch.autograd.grad(y, leaves, torch.linspace(-1, 1, y.numel(), device=DEV).reshape(y.shape).to(y.dtype))
+        same = lambda t: t
+        plain = grads(same, same)
+        for got, exp in zip(grads(lambda t: t.mT.contiguous() if t.dim() > 1 else t, lambda t: t.mT if t.dim() > 1 else t), plain):
+            assert (got - exp).norm() <= 2 ** -8 * exp.norm()   # (the same kernels; a layer's products in another layout)
+        assert all(torch.equal(g, e) for g, e in zip(grads(lambda t: t.cpu(), lambda t: t.to(DEV)), plain))
+        if fn not in (block_ops.gelu_tanh, block_ops.silu, block_ops.dual_linear):   # (these compute in the type that they get)
+            assert all(torch.equal(g, e) for g, e in zip(grads(same, lambda t: t.double()), plain))
+        for unpack in (lambda t: t.cpu(), lambda t: t[:1] if t.dim() > 1 else t[:-8]):
+            with pytest.raises(RuntimeError, match="hook handed back"):
+                grads(same, unpack)
