@@ -384,7 +384,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     waddr[c] = lds_addr(smem) + T::NSX * T::XS + (wn * 32 * NT + c32) * 128 + k;
   }
   // COLS: of column group i, rows 8 g .. + 3 of a chunk's 16 (the other four: + 512), so that a lane's slots are those of its rows of x
-  static_assert(!COLS || NT <= 4);
+  static_assert(NT <= 4);   // (of the bias too: two columns per lane)
   if constexpr (COLS) {
     const uint32_t i16 = lane & 15, in_panel = (8 * g + (i16 >> 2)) * 128 + ((lane >> 4) & 1) * 32 + (i16 & 3) * 8, swap = (i16 >> 3) & 1;
 #pragma unroll
@@ -517,7 +517,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
         wait_vm<T::PX + T::PW>();   // (else the tile's last stage has waited for it)
       }
       for_each(std::make_integer_sequence<int, NT * 4>{}, [&](auto vv) {
-        braw[decltype(vv)::value] = lds_read64_issue<decltype(vv)::value * 16>(own + (T::IN_SLOT ? 0 : wn * 64 * NT) + g * 8);
+        braw[decltype(vv)::value] = lds_read64_issue<decltype(vv)::value * 16>(own + g * 8);
       });
     }
     // (sums are taken out of their registers one quad at a time: left to itself the compiler copies all of them at once, and spills; the wait
@@ -599,9 +599,9 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
   };
 
   // A tile's bias is requested before its first stage (scalar loads at the tile's end left everything waiting for them: pairs C768 M16384 N 3C 119 ->
-  // 113 us, C1152 M8192 N 4C 154 -> 149; 128 x 96 tiles, C768 M4096 N C 10.1 -> 9.4): the KB from the tile's first column on, zeros past the last one and
-  // for tangents, to where the results will pass through.  Without LDS for it, this wave's columns into a register, two per lane; in assembly, as
-  // the compiler would wait for all requests in flight at its use, and that nothing touches it before its wait is checked on the built code.
+  // 113 us, C1152 M8192 N 4C 154 -> 149; 128 x 96 tiles, C768 M4096 N C 10.1 -> 9.4): this wave's columns, two per lane (by dwords, as a bias is 8-byte
+  // aligned), zeros past the last one and for tangents, to where the results will pass through.  Without LDS for it, into a register; in assembly,
+  // as the compiler would wait for all requests in flight at its use, and that nothing touches it before its wait is checked on the built code.
   auto request_bias = [&](uint32_t id) {
     const Place t = place(id);
     const int bytes = p.bias != nullptr && !t.second ? (p.N - t.n0) * 2 : 0;
@@ -611,7 +611,7 @@ __device__ __forceinline__ void linear_walk(const LinearParams& p) {
     } else {
       const __amdgpu_buffer_rsrc_t rb = make_rows_rsrc(p.bias + t.n0, 0, 1, bytes);
       char* dst = smem + T::NSX * T::XS + T::NSW * T::WS + wave * 4096;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)dst, 16, lane * 16, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)dst, 4, (wn * 32 * NT + 2 * lane) * 2, 0, 0, 0);
     }
   };
 

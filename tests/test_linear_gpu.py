@@ -348,6 +348,31 @@ def test_products_of_the_widest_tiles(size, modes):
             _check(_call(x, tx if jvp else None, w, None, 0)[0], ref - b.float())
 
 
+# (one of each kernel; a walking kernel's with more columns than one wave's)
+UNALIGNED = ["linear_kernel<128, 64", "linear_kernel<64, 64", "WalkTile<1, 3", "WalkTile<4, 2", "WalkTile<4, 3"]
+
+
+@pytest.mark.parametrize("kernel,size", [(k, next(s for n, s, m in REACHED if k in n and PLAIN in m)) for k in UNALIGNED] + [("wide", WIDE[1][0])])
+def test_bias_aligned_to_eight_bytes(kernel, size):
+    """The least alignment that the entry takes, with values around the bias that would show."""
+    M, N, K = size
+    x, tx, w, b = _operands(M, N, K)
+    around = torch.full((N + 8,), 1e4, device=DEV, dtype=torch.bfloat16)
+    bias = around[4:N + 4]
+    bias.copy_(b)
+    assert bias.data_ptr() % 16 == 8 and kernel in planned(M, N, K, 0, 0)
+    assert torch.equal(_call(x, None, w, bias, 0)[0], _call(x, None, w, b, 0)[0])
+    for gelu in (0, 1):
+        for got, exp in zip(_call(x, tx, w, bias, gelu), _call(x, tx, w, b, gelu)):
+            assert torch.equal(got, exp)
+    if _lib.load().dmf_linear_gelu_plan(M, N, K):
+        outs = [[torch.empty(M, N, device=DEV, dtype=torch.bfloat16) for _ in range(3)] for _ in range(2)]
+        for o, bb in zip(outs, (bias, b)):
+            assert _lib.load().dmf_linear_gelu_fwd(x.data_ptr(), tx.data_ptr(), w.data_ptr(), bb.data_ptr(), *(t.data_ptr() for t in o), M, N, K,
+                                                   torch.cuda.current_stream().cuda_stream) == 0
+        assert all(torch.equal(*t) for t in zip(*outs))
+
+
 # the MLP's first half with its pre-activation kept, in each of the three tiles: rows and columns that fill none, one step, two and many
 KEPT = [(2049, 2296, 704), (8193, 4088, 128), (16129, 1016, 64), (16300, 2040, 1152), (4000, 1016, 1152), (2300, 3064, 448)]
 
