@@ -72,6 +72,7 @@ FUSED_SIGNATURES = {
     "dmf_linear_wgrad_workspace_floats": (c_int64, [_L] + [_I] * 2),
     "dmf_linear_wgrad_plan": (c_int, [_L] + [_I] * 2),
     "dmf_linear_wgrad_sums_plan": (c_int, [_L] + [_I] * 2),
+    "dmf_linear_train_plan": (c_int, [_I, _L, _I, _I, ctypes.c_char_p, _I]),
     "dmf_linear_wgrad": (c_int, [_P] * 5 + [_I] * 3 + [_P]),
     "dmf_cast_bf16": (c_int, [_P] * 3 + [_I, _P]),
     "dmf_timestep_embedding_fwd": (c_int, [_P] * 4 + [_L, _I, _F, _I, _P]),

@@ -894,6 +894,11 @@ extern "C" int dmf_linear_dgrad_plan(int64_t M, int N, int K) {
   return K % 192 == 0 || M < 10240;
 }
 
+// (the forward's estimates, by linear_tile's numbers: on the products above the tile they choose takes 0.4 % more than the faster of the two in the mean)
+static int dgrad_tile(int64_t M, int N, int K) {
+  return dmf::walk_cost(dmf::kLinWalks[0], M, K, N / dmf::kLinK, 1, true) <= dmf::walk_cost(dmf::kLinWalks[1], M, K, N / dmf::kLinK, 1, true) ? 3 : 4;
+}
+
 extern "C" int dmf_linear_dgrad(const void* g, const void* w, void* gx, int M, int N, int K, void* stream) {
   if (g == nullptr || w == nullptr || gx == nullptr) return DMF_ATTN_ENULL;
   if (!dgrad_shape_ok(M, N, K)) return DMF_ATTN_ESHAPE;
@@ -905,10 +910,7 @@ extern "C" int dmf_linear_dgrad(const void* g, const void* w, void* gx, int M, i
   p.y[0] = static_cast<__bf16*>(gx);
   p.M = M; p.N = K; p.K = N;   // (of the product: columns of the result, depth)
   auto stm = static_cast<hipStream_t>(stream);
-  // (the forward's estimates: on the products above the tile they choose takes 0.4 % more than the faster of the two in the mean)
-  return dmf::walk_cost(dmf::kLinWalks[0], M, K, N / dmf::kLinK, 1, true) <= dmf::walk_cost(dmf::kLinWalks[1], M, K, N / dmf::kLinK, 1, true)
-             ? dmf::launch_dgrad<dmf::WalkTile<4, 3, 2, 3, 2>>(p, stm)
-             : dmf::launch_dgrad<dmf::WalkTile<4, 2, 2, 3, 3>>(p, stm);
+  return dgrad_tile(M, N, K) == 3 ? dmf::launch_dgrad<dmf::WalkTile<4, 3, 2, 3, 2>>(p, stm) : dmf::launch_dgrad<dmf::WalkTile<4, 2, 2, 3, 3>>(p, stm);
 }
 
 namespace dmf {
@@ -1325,6 +1327,20 @@ extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
 // and column sum -> here): M 1536: 2304 x 768 27.8 -> 23.5, 3072 x 1024 32.5 -> 29.8;  M 2048: 3072 x 768 36.5 -> 29.0, 3072 x 1024 36.9 -> 36.5, 1152 x 1152 32.2 ->
 // 24.4, 4608 x 1152 48.5 -> 39.3;  M 4096: 3456 x 1152 60.7 -> 49.9, 4096 x 1024 59.6 -> 53.6;  M 5120: 3456 x 1152 71.0 -> 57.0, 1024 x 4096 68.6 -> 63.5.
 extern "C" int dmf_linear_wgrad_sums_plan(int64_t M, int N, int K) { return M <= INT32_MAX && dmf::wgrad_shape_ok(M, N, K) && (int64_t)N * K <= 8000000; }
+
+extern "C" int dmf_linear_train_plan(int which, int64_t M, int N, int K, char* buf, int buflen) {
+  const bool ok = which == 0 ? M <= INT32_MAX && dmf_linear_gelu_plan(M, N, K) : which == 1 ? dgrad_shape_ok(M, N, K) : which == 2 && M <= INT32_MAX && dmf::wgrad_shape_ok(M, N, K);
+  if (!ok) return DMF_ATTN_ESHAPE;
+  if (buf == nullptr || buflen < 1) return DMF_ATTN_ENULL;
+  if (which == 2) {
+    const int wide = dmf::wgrad_wide_splits(M, N, K);
+    snprintf(buf, (size_t)buflen, "dmf::linear_wgrad_%skernel, %d splits", wide ? "wide_" : "", wide ? wide : dmf::wgrad_splits(M, N, K));
+    return DMF_ATTN_OK;
+  }
+  const char* tile[7] = {"", "", "", "4, 3, 2, 3, 2", "4, 2, 2, 3, 3", "", "4, 4, 2, 3, 2"};
+  snprintf(buf, (size_t)buflen, "dmf::linear_%s_kernel<dmf::WalkTile<%s> >", which ? "dgrad" : "walk_pre", tile[which ? dgrad_tile(M, N, K) : dmf::linear_tile(M, N, K, true, true)]);
+  return DMF_ATTN_OK;
+}
 
 extern "C" int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream) {
   if (g == nullptr || x == nullptr || gw == nullptr) return DMF_ATTN_ENULL;

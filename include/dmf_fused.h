@@ -74,6 +74,8 @@ DMF_ATTN_API int dmf_linear_dgrad(const void* g, const void* w, void* gx, int M,
 DMF_ATTN_API int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K);
 DMF_ATTN_API int dmf_linear_wgrad_plan(int64_t M, int N, int K);
 DMF_ATTN_API int dmf_linear_wgrad_sums_plan(int64_t M, int N, int K);
+/* As dmf_linear_fwd_plan, for a layer's training: which 0 dmf_linear_gelu_fwd, 1 dmf_linear_dgrad, 2 dmf_linear_wgrad (with its splits of the rows). */
+DMF_ATTN_API int dmf_linear_train_plan(int which, int64_t M, int N, int K, char* buf, int buflen);
 DMF_ATTN_API int dmf_linear_wgrad(const void* g, const void* x, float* gw, float* gbias, float* workspace, int M, int N, int K, void* stream);
 
 /*

@@ -93,12 +93,13 @@ def test_layers_take_it_for_what_it_covers(dual):
 
 # ---- input gradient (dmf_linear_dgrad), N -> K: one row, rows and columns that fill no tile, one step per tile and fewer than stages, whole rounds with
 # half tiles behind them, only half tiles, either tile width; exact operands and fp32 sums, so that the bound is the result's rounding
-DGRAD = [(1, 64, 8), (63, 64, 64), (129, 192, 200), (4097, 640, 712), (2049, 768, 2296), (8193, 1152, 1152), (4100, 1024, 1016), (12345, 192, 1016),
-         (16389, 64, 2304), (2300, 448, 3064), (256, 3072, 768), (8192, 4608, 1152)]
+DGRAD = {"4, 2, 2, 3, 3": [(1, 64, 8), (63, 64, 64), (129, 192, 200), (4097, 640, 712), (12345, 192, 1016), (16389, 64, 2304), (2300, 448, 3064), (256, 3072, 768)],
+         "4, 3, 2, 3, 2": [(2049, 768, 2296), (8193, 1152, 1152), (4100, 1024, 1016), (8192, 4608, 1152)]}
 
 
-@pytest.mark.parametrize("M,N,K", DGRAD)
-def test_input_gradient(M, N, K):
+@pytest.mark.parametrize("M,N,K,tile", [(*size, tile) for tile, sizes in DGRAD.items() for size in sizes])
+def test_input_gradient(M, N, K, tile):
+    assert trained(1, M, N, K) == f"dmf::linear_dgrad_kernel<dmf::WalkTile<{tile}> >"
     gen = torch.Generator(device=DEV).manual_seed(M + N + K)
     # (what lies behind the last row of either operand would show if it were summed)
     g, w = torch.randn(M + 64, N, generator=gen, device=DEV).bfloat16(), (torch.randn(N + 64, K, generator=gen, device=DEV) * N ** -0.5).bfloat16()
@@ -150,15 +151,23 @@ def test_input_gradient_refuses():
 # ---- weight gradient (dmf_linear_wgrad): products exact in fp32, sums in fp32 -- M terms in some order, error below sqrt(M) 2^-24 of the
 # sum of magnitudes on random data; 2e-6 covers M = 16389 (7.6e-6 of a worst single element, checked against the largest)
 WGRAD = [(1, 8, 8), (63, 64, 64), (64, 128, 192), (65, 136, 200), (129, 120, 184), (333, 1152, 1152), (2048, 384, 1536), (4097, 712, 328),
-         (8192, 1152, 1152), (8192, 3456, 1152), (4096, 4608, 1152), (4096, 1152, 4608), (16389, 768, 768), (32768, 96, 200), (20001, 384, 384)]
+         (32768, 96, 200), (20001, 384, 384), (16389, 264, 1944)]
+# linear_wgrad_wide_kernel: columns that fill no tile on either side, rows that fill no step, one tile, one split (whose sums go straight out)
+WGRAD_WIDE = [(6145, 1288, 1032), (4097, 712, 2800), (250001, 184, 200), (8193, 520, 1944), (641, 4088, 3064), (8192, 4608, 1152), (6144, 1152, 4608),
+              (8192, 1152, 1152), (8192, 3456, 1152), (4096, 4608, 1152), (4096, 1152, 4608), (16389, 768, 768)]
 
 
-# (those of 8 G multiply-adds and more go through linear_wgrad_wide_kernel: columns that fill no tile on either side, rows that fill no step, one tile)
-WGRAD_WIDE = [(6145, 1288, 1032), (4097, 712, 2800), (250001, 184, 200), (16389, 264, 1944), (8192, 4608, 1152), (6144, 1152, 4608)]
+def trained(which, M, N, K):
+    """What dmf_linear_train_plan calls the kernel, for 256 CUs: which 0 the kept form, 1 the input gradient, 2 the weight gradient."""
+    name = ctypes.create_string_buffer(128)
+    assert _lib.load().dmf_linear_train_plan(which, M, N, K, name, len(name)) == 0
+    return name.value.decode()
 
 
 @pytest.mark.parametrize("M,N,K", WGRAD + WGRAD_WIDE)
 def test_weight_gradient(M, N, K):
+    assert ("linear_wgrad_wide_kernel, " if (M, N, K) in WGRAD_WIDE else "linear_wgrad_kernel, ") in trained(2, M, N, K)
+    assert ((M, N, K) == (641, 4088, 3064)) <= trained(2, M, N, K).endswith(" 1 splits")
     gen = torch.Generator(device=DEV).manual_seed(M + N + K)
     # (rows past the last hold values that would show if they were summed)
     g, x = (torch.randn(M + 64, C, generator=gen, device=DEV).bfloat16() for C in (N, K))
@@ -374,11 +383,13 @@ def test_bias_aligned_to_eight_bytes(kernel, size):
 
 
 # the MLP's first half with its pre-activation kept, in each of the three tiles: rows and columns that fill none, one step, two and many
-KEPT = [(2049, 2296, 704), (8193, 4088, 128), (16129, 1016, 64), (16300, 2040, 1152), (4000, 1016, 1152), (2300, 3064, 448)]
+KEPT = {"4, 3, 2, 3, 2": [(2049, 2296, 704), (8193, 4088, 128)], "4, 4, 2, 3, 2": [(16129, 1016, 64), (16300, 2040, 1152)],
+        "4, 2, 2, 3, 3": [(4000, 1016, 1152), (2300, 3064, 448)]}
 
 
-@pytest.mark.parametrize("M,N,K", KEPT)
-def test_products_that_keep_their_pre_activation(M, N, K):
+@pytest.mark.parametrize("M,N,K,tile", [(*size, tile) for tile, sizes in KEPT.items() for size in sizes])
+def test_products_that_keep_their_pre_activation(M, N, K, tile):
+    assert trained(0, M, N, K) == f"dmf::linear_walk_pre_kernel<dmf::WalkTile<{tile}> >"
     x, tx, w, b = _operands(M, N, K)
     lib, p = _lib.load(), lambda t: None if t is None else t.data_ptr()
     assert lib.dmf_linear_gelu_plan(M, N, K) == 1
@@ -429,7 +440,7 @@ def test_mlp_first_half_with_a_backward_pass():
     with fwAD.dual_level():
         y = fwAD.unpack_dual(block_ops.linear_gelu_tanh(fwAD.make_dual(a, tx), wt, b))[0]
     gx = torch.autograd.grad(y, a, gy, create_graph=True)[0]
-    assert torch.autograd.grad(gx, wt, x)[0].shape == wt.shape
+    assert torch.autograd.grad(gx, wt, x)[0].shape == wt.shape   # (values: test_mlp_first_half_differentiated_again)
 
 
 @pytest.mark.parametrize("case", ["second", "over_reverse"])
@@ -471,6 +482,14 @@ def test_mlp_first_half_differentiated_again(case, autocast, M, N, K):
     for i, (a, e) in enumerate(zip(got, exp)):
         assert a is not None and a.shape == e.shape, i
         assert (a.double() - e).norm() <= tol * e.norm(), (i, float((a.double() - e).norm() / e.norm()))
+
+
+def test_the_training_plan_refuses_what_the_entries_refuse():
+    plan, name = _lib.load().dmf_linear_train_plan, ctypes.create_string_buffer(4)
+    for which, size in ((0, (64, 64, 64)), (0, (2 ** 31, 2296, 704)), (1, (64, 32, 64)), (1, (1 << 25, 64, 8)), (2, (64, 60, 64)), (2, (2 ** 31, 64, 64)), (3, (64, 64, 64))):
+        assert plan(which, *size, name, len(name)) == -3
+    assert plan(2, 64, 64, 64, None, 0) == -5
+    assert plan(2, 64, 64, 64, name, len(name)) == 0 and name.value == b"dmf"   # (cut to the buffer)
 
 
 def test_the_plan_refuses_what_the_entry_refuses():
