@@ -642,9 +642,9 @@ __global__ __launch_bounds__(256, 1) void linear_walk_kernel(const LinearParams 
   linear_walk<T, MODE>(p);
 }
 
-// 256 x 256: an eighth fewer bytes and LDS reads per product than 256 x 192, all of the accumulation registers and of the LDS (results pass through
-// the slot that is to be requested into next).  Where the rounds are as full: pairs C768 M16384 N 4C 144 -> 136 us, N 3C 111 -> 107, with gelu 157 ->
-// 148; C1024 M8192 N 4C 128 -> 115, M16384 K 4C 234 -> 209; 8192 cubed 867 -> 798 (1378 TFLOP/s).
+// 256 x 256: a seventh fewer bytes and LDS reads per product than 256 x 192, all of the accumulation registers and of the LDS (results pass through
+// the slot that is to be requested into next).  Where the rounds are as full: pairs C768 M16384 N 3C 114 -> 107 us, N 4C with gelu 162 -> 149; C1152 M8192
+// N 4C 148 -> 143; C1024 M8192 N 4C with gelu 140 -> 123; single C1152 M12288 K 4C 124 -> 105; 8192 cubed 867 -> 798 (1378 TFLOP/s).
 using WalkWide = WalkTile<4, 4, 2, 3, 2>;
 template <int MODE>
 __global__ __launch_bounds__(256, 1) void linear_walk_wide_kernel(const LinearParams p) {
@@ -675,7 +675,7 @@ static int launch_walk(LinearParams& p, bool jvp, hipStream_t stream) {
 }
 
 // The input gradient gx = g W: the same walk with w read by columns, contracted over its rows as they lie in memory.  The library's products ran at
-// 560 to 910 TFLOP/s here (C1152 M8192: 3C -> C 84.6 us, C -> C 38.7, 4C -> C 108, C -> 4C 97.5); these at 850 to 1080 (63.4, 27.0, 83.7, 81.1), bounded like
+// 560 to 910 TFLOP/s here (C1152 M8192: 3C -> C 84.6 us, C -> C 38.7, 4C -> C 108, C -> 4C 97.5); these at 800 to 1170 (57 to 63, 24 to 27, 74 to 84, 78 to 81, by the card), bounded like
 // the forward's by the address unit and the tiles' ends: transposed reads of w take as many bytes out of LDS as rows of it.
 template <class T>
 __global__ __launch_bounds__(256, 1) void linear_dgrad_kernel(const LinearParams p) {
@@ -697,11 +697,11 @@ static int launch_dgrad(LinearParams& p, hipStream_t stream) {
 // Tile policy: the shortest of the estimates, in 10 ns, of seven kernels.  linear_kernel: a K step (64) and a work-group's start and end with one,
 // two, three work-groups on a CU, more of them never taking less; linear_walk_kernel: a step and what a tile takes beyond its steps at that
 // pace, of whole and of half a tile, and the launch's.  Fitted to 1440 products of
-// widths 384 to 1280, 64 to 32768 rows, single and in pairs, with and without gelu, seven tenths of them; all of them and the fit's aim are in
-// profiles/linear_tiles.txt.  Tiles within 1.3 of the fastest one are met to 4 (128 x 96) to 11 % (64 x 64); the tile taken is 0.24 % slower than
-// the fastest in the mean (0.25 % where the fit did not look), 5 % in one of a hundred.  128 x 192 is all but never that tile; it is here
-// for the rows of more than 65536 elements that the walking kernel does not take.  The estimate of 256 x 256 is set on 175 further products of up to
-// 16384 rows (117 of at least one round), so that the choice among the three walking tiles is 0.1 % slower than the fastest of them in the mean.
+// widths 384 to 1280, 64 to 32768 rows, single and in pairs, with and without gelu, seven tenths of them, before there was 256 x 256 and before the walking
+// kernels' tiles ended as they do now; all of them, measured since, and the fit's aim are in profiles/linear_tiles.txt.  Tiles within 1.3 of the fastest
+// one are met to 5 (128 x 96) to 9 % (64 x 64); the tile taken is 0.87 % slower than the fastest in the mean, 15 % in one of a hundred.  128 x 192 is all but
+// never that tile; it is here for the rows of more than 65536 elements that the walking kernel does not take.  The estimate of 256 x 256 was set by hand on
+// 175 products of up to 16384 rows; where it takes a product from another tile (710 of 2110) it needs 0.94 of that one's time, 1.06 at most.
 struct LinTile { int bm, bn, per_cu, a[3], b[3]; };
 constexpr LinTile kLinTiles[3] = {{128, 192, 2, {82, 113, 0}, {541, 761, 0}}, {128, 64, 3, {48, 68, 80}, {262, 364, 466}}, {64, 64, 2, {23, 39, 0}, {279, 263, 0}}};
 constexpr bool never_shorter_with_more(const LinTile& t) {
@@ -777,21 +777,21 @@ static int launch_linear_tile(int tile, LinearParams& p, bool jvp, hipStream_t s
 
 }  // namespace dmf
 
-// Which calls these kernels are the faster ones for (us on the GPU, library -> here; C: model width, M rows; called from the host a library
-// product takes 18 us at least, one of these 5):
-//   pairs: C768 M16384 N 3C 137 -> 106, N C 45 -> 38, K 4C 131 -> 124; C1152 M8192 158 -> 113, 62 -> 42, N 4C 169 -> 148, K 4C 165 -> 149;
-//     M4096 81 -> 62, 37 -> 24, K 4C 94 -> 73;
-//   single: C768 M1024 N 3C 11.5 -> 9.4, M2048 15.6 -> 12.7, M4096 18.5 -> 18.8, N C 11.8 -> 9.7; C1152 M8192 N 3C 79 -> 64, K 4C 80 -> 73;
-//     K 4C: M1024 C768 15.1 -> 13.5, M2048 C384 9.9 -> 8.5, C1152 31.8 -> 29.4, M3000 C768 23.3 -> 21.4, M4096 25.3 -> 23.6, M8192 36.4 -> 37.1.
+// Which calls these kernels are the faster ones for (us on the GPU, library -> here, all in profiles/linear_tiles.txt; C: model width, M rows; called from
+// the host a library product takes 18 us at least, one of these 5):
+//   pairs: C768 M16384 N 3C 139 -> 107, N C 48 -> 42, K 4C 134 -> 131; C1152 M8192 160 -> 112, 64 -> 44, N 4C 174 -> 143, K 4C 169 -> 149;
+//     M4096 83 -> 60, 40 -> 25, K 4C 93 -> 75;
+//   single: C768 M1024 N 3C 11.6 -> 9.0, M2048 16.4 -> 12.7, M4096 19.7 -> 19.0, N C 12.0 -> 10.7; C1152 M8192 N 3C 80 -> 61, K 4C 80 -> 73;
+//     K 4C: M1024 C768 15.2 -> 13.4, M2048 C384 9.9 -> 8.6, C1152 32.5 -> 28.2, M3000 C768 24.0 -> 20.8, M4096 26.8 -> 25.0, M8192 38.2 -> 37.7.
 // The library's time moves by a fifth to either side with its own choice of tile, so that no line is sharp.  It keeps
-//   single products deeper than they are wide (K 4C) whose 128 x 96 tiles need up to a third of a second round, 4 % faster in the mean of 48 measured
-//     (M4500 C768 26.5 against 29.1, M3072 C1024 30.1 against 32.4, M3000 C1152 36.0 against 38.7; one round, M4096 C768, 25.3 against
-//     23.6; from four thirds on even in the mean, up to a tenth either way; K up to 2304 even);
-//   those that spread a short K over a large result (N 4C: C768 M16384 pairs 131 against 138, M32768 single 128 against 140), rows of 2 or 8 KB on
-//     large results (C1024: M16384 K 4C 92 against 116, N C 28.9 against 32.8, M8192 N 4C 56 against 67);
+//   single products deeper than they are wide (K 4C) whose 128 x 96 tiles need up to a third of a second round (M4500 C768 28.0 against 29.8, M3072 C1024 30.0
+//     against 32.1, M3000 C1152 37.1 against 38.5; one round, M4096 C768, 26.8 against 25.0; from four thirds on even in the mean);
+//   those that spread a short K over a large result (N 4C: C768 M16384 pairs 135 against 136, M32768 single 132 against 137), rows of 2 or 8 KB on
+//     large results (C1024: M16384 K 4C 94 against 105, N C 29.9 against 32.2, M8192 N 4C 56 against 60);
 //   and outputs narrower than a tile.
-// Deep products of few rows are a trade: on the GPU alone, as replayed from a graph, the library's are faster (K 4C: M64 C768 7.4 against 12.6, M256
-// 8.7 against 12.6, M512 11.5 against 12.1, M2048 18.2 against 19.7), called from the host slower where that is what bounds the calls (18.3
+// These lines were drawn before 256 x 256 tiles: the 287 products that they leave to the library would take 0.95 of its time here, in the mean.
+// Deep products of few rows are a trade: on the GPU alone, as replayed from a graph, the library's are faster (K 4C: M64 C768 10.2 against 12.5, M256
+// 9.3 against 13.1, M512 12.9 against 12.8, M2048 18.9 against 20.5), called from the host slower where that is what bounds the calls (18.3
 // against 12.1 up to M512; the library taken for M2197 C768, two blocks sampled by a host that does not run ahead: 1.68 -> 1.73 ms).  They are taken.
 //   pairs with gelu (library pair and activation kernel; this kernel's pair and the activation kernel -> here), N 4C, wins from one row up:
 //     M16 C384 10.4; 7.7 -> 5.3, C768 11.3; 8.1 -> 7.1, C1152 12.7; 9.2 -> 8.9;  M512 C768 23.4; 15.5 -> 12.0, C1152 34.0; 24.1 -> 18.2;
@@ -875,19 +875,26 @@ static bool dgrad_shape_ok(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && M <= INT32_MAX && N >= 64 && N % 64 == 0 && K >= 8 && K % 8 == 0 && N <= 65536 && K <= 65536 && M * N <= most && N * K <= most && M * K <= most;
 }
 
-// Which input gradients the walking kernel is the faster one for, N -> K (us on the GPU, library -> here; 318 products of widths 384 to 1152, 64 to 32768
-// rows; the 193 it takes need 0.88 of the library's time in the mean, and 5 us of host time where that takes 18):
-//   from 3072 rows on (2048 where a row of tiles is not mostly idle or cut): C768 M4096 3C -> C 29.9 -> 23.1, M16384 62.8 -> 55.0; C1152 M16384 157 -> 118;
-//     C384 M16384 26.4 -> 19.7; but C384 M2048 10.8 against 12.9, C1024 M2048 26.4 against 28.5, C768 M1536 17.6 against 21.5;
-//   C -> 4C from 768 rows on: C768 M1024 14.4 -> 11.3, C1152 24.7 -> 16.3; not with one to 4/3 rounds of 256 x 192 tiles: C768 M5120 28.2 against 30.6,
-//     C1024 M3072 28.5 against 32.6;
-//   widths that 192 columns do not divide lose in many rows: C1024 M12288 3C -> C 71.6 against 81.5, M16384 89.4 against 94.6 (M8192 59.0 -> 49.6);
-//   outputs narrower than a tile lose, M8192 1152 -> 64 9.3 against 11.7, and up to 6144 rows narrow ones that fill none: M3072 3072 -> 320 18.9 against 25.7.
+// Which input gradients the walking kernel is the faster one for, N -> K (us on the GPU, library -> here, of the 389 products of
+// profiles/linear_train_products.txt, widths 384 to 1152, 64 to 46080 rows; the 250 it takes need 0.84 of the library's time in the mean, and 5 us of
+// host time where that takes 18):
+//   from 3072 rows on (2048 where a row of tiles is not mostly idle or cut): C768 M4096 3C -> C 26.8 -> 21.5, M16384 53.9 -> 48.8; C1152 M16384 150 -> 114;
+//     C384 M16384 22.9 -> 19.5; but C384 M2048 10.6 against 13.0, C1024 M2048 25.3 against 27.5, C768 M1536 17.5 against 20.5;
+//   C -> 4C from 768 rows on: C768 M1024 13.8 -> 11.4, C1152 23.7 -> 15.1; not with one to 4/3 rounds of 256 x 192 tiles: C768 M5120 28.2 against 30.6,
+//     C1024 M3072 28.5 against 32.6, on another card 28.1 against 27.1 and 28.9 against 28.6;
+//   deep ones of a width that 256 columns divide lose with one to 4/3 rounds: C768 M19200 3C -> C 62.0 against 64.1, 4C -> C 77.7 against 80.9, M21120
+//     63.7 against 65.8 (C1152 M13482 170 -> 95, C384 M38400 45 -> 38; C768 M22080 83 -> 71);
+//   widths that 192 columns do not divide lose in many rows: C1024 M12288 3C -> C 64.8 against 70.4, M16384 80.7 against 85.9 (M8192 49.9 -> 44.7);
+//   outputs narrower than a tile lose, M8192 1152 -> 64 9.1 against 11.5, and up to 6144 rows narrow ones that fill none: M3072 3072 -> 320 18.5 against 25.5.
 extern "C" int dmf_linear_dgrad_plan(int64_t M, int N, int K) {
   if (!dgrad_shape_ok(M, N, K) || M < 768 || K < 192) return 0;
   if (K >= 3 * (int64_t)N) {
     const int64_t cus = dmf::compute_units(), tiles = ((M + 255) / 256) * ((K + 191) / 192);
     return tiles <= cus || 3 * tiles > 4 * cus;
+  }
+  if (K % 256 == 0 && N >= 3 * (int64_t)K) {
+    const int64_t cus = dmf::compute_units(), tiles = ((M + 255) / 256) * ((K + 191) / 192);
+    if (tiles > cus && 3 * tiles <= 4 * cus) return 0;
   }
   if (M < 3072 && (M < 2048 || K < 512 || K % 192 != 0)) return 0;
   if (M < 6144 && K < 512 && K % 192 != 0) return 0;
@@ -1070,8 +1077,8 @@ __global__ __launch_bounds__(256, 2) void linear_wgrad_kernel(const WgradParams 
 // Much work: the walking forward kernel's tile, stages and order of reads, products and requests (see linear_walk), of 256 columns of g against 192 of x,
 // a work-group per CU.  Both operands lie in 64-column panels of 64 rows and are read by columns.  A step of 6.3 MFLOP takes 0.8 to 1.2 us, by how many
 // CUs take part (two of linear_wgrad_kernel's, the same work, 1.25); start, end and launch 12 us where that takes 9 (both 2 less since the
-// sums leave by store_sums).  With the partial sums' kernel, both before that, M 8192: 4608 x 1152 109 -> 100 us (98 now), 3072 x 768 59.6 -> 54.7 (51),
-// 3072 x 1024 79.5 -> 71.5 (68), 1152 x 1152 42.5 -> 40.5 (38); M 16384: 4608 x 1152 207 -> 178.
+// sums leave by store_sums).  With column sums and the partial sums' kernel, M 8192: 4608 x 1152 109 -> 93 us, 3456 x 1152 81 -> 74, 3072 x 768 52.7 -> 50.6,
+// 3072 x 1024 78 -> 67, 1152 x 1152 39.1 -> 37.6; M 16384: 4608 x 1152 191 -> 168.
 // The two waves that hold the same columns of g sum two chunks of a step each for the bias (two thirds of the room between a chunk's products).
 struct WgradWide : WalkTile<4, 3, 2, 3, 2> { static constexpr int STAGES = NSX * XS + NSW * WS; };
 
@@ -1270,9 +1277,10 @@ static int wgrad_splits(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-// Splits for linear_wgrad_wide_kernel, 0 where linear_wgrad_kernel is the better one: below 8 G multiply-adds, measured on 160 products (3072 x 768: M 3072 -5 %,
-// 768 x 768: M 12288 +2 %, M 16384 -2 %; 1152 x 1152: M 4096 +6 %, M 6144 -11 %).  Estimates fitted to those, in 10 ns; all work-groups at once; chains
-// of sums no longer than that kernel's.
+// Splits for linear_wgrad_wide_kernel, 0 where linear_wgrad_kernel is the better one: below 8 G multiply-adds (profiles/linear_train_products.txt, with column
+// sums, there against here: 768 x 768 M 12288 31.4 against 29.9 us, M 16384 36.7 -> 34.7; 1152 x 1152 M 6144 35.1 -> 32.9; 2304 x 768 M 5120 33.3 -> 34.8, M 6144 36.5 ->
+// 37.0, M 8192 44.3 -> 43.9; the kernel taken is 0.5 % slower than the faster in the mean).  Estimates fitted to 160 such products, in 10 ns; all work-groups at
+// once; chains of sums no longer than that kernel's.
 static int wgrad_wide_splits(int64_t M, int64_t N, int64_t K) {
   if (M * N < 8000000000 / K) return 0;
   const int64_t cus = compute_units(), tiles = ((N + WgradWide::BM - 1) / WgradWide::BM) * ((K + WgradWide::BN - 1) / WgradWide::BN), total = (M + 63) / 64;
@@ -1305,15 +1313,16 @@ extern "C" int64_t dmf_linear_wgrad_workspace_floats(int64_t M, int N, int K) {
   return s > 1 ? (int64_t)s * N * (K + 1) : 0;
 }
 
-// Which weight gradients this kernel is the faster one for (us, library -> here; the library's launch alone takes 20 us of host time):
-//   up to M 1472 on every result of the models (column sums included on both sides): M 1 .. 128, the adaLN layers' batches: 2304 x 384
-//   9.3 .. 12.4 -> 6.3 .. 7.1, 4608 x 768 12.5 .. 15.3 -> 8.0 .. 8.8, 6912 x 1152 16.3 .. 22.0 -> 12.3 .. 14.1;  M 512: 768 x 768 15.2 -> 12.4,
-//   4608 x 1152 27.1 -> 15.5;  M 1000: 768 x 768 20.5 -> 15.9, 4608 x 1152 38.9 -> 23.3;  M 1472: 3072 x 768 30.5 -> 27.7, 3456 x 1152 32.8 -> 29.0;
-//   M 2048: 1536 x 384 20.0 -> 18.4, but 2304 x 768 21 against 23, 3456 x 1152 28 against 34;
-//   M 4096: 3072 x 768 44 -> 37, 1152 x 1152 35 -> 30, 3072 x 1024 47 -> 46, 4608 x 1152 67 -> 62, but 3456 x 1152 50 against 53, 4096 x 1024 50 against 55;
-//   M 6144: 3456 x 1152 69 against 71, 4608 x 1152 97 -> 81, 4096 x 1024 77 -> 75, 1024 x 4096 80 -> 76 (and no column sum beside it);
-//   M 8192: 3456 x 1152 99 -> 80, 4608 x 1152 125 -> 98, 4096 x 1024 106 -> 88, 1152 x 1152 64 -> 38, 768 x 768 51 -> 26;  M 16384: 3072 x 768 177 ->
-//   91, 4608 x 1152 335 -> 178 (975 TFLOP/s).  The largest result measured is 6912 x 1152 (8 M elements); beyond it the library's products are kept.
+// Which weight gradients without column sums these kernels are the faster ones for (us, library -> here, of profiles/linear_train_products.txt; the library's
+// launch alone takes 20 us of host time): those of layers without a bias, which the models do not have.
+//   up to M 1472 on every result of the models with a column sum beside the library's (next rule); without one the GPU alone takes 5 to 30 % more here
+//   for 768 x 768 and smaller (M 512 8.7 against 10.6, M 1000 13.8 against 14.7), which the host's share outweighs, and less for large results
+//   (4608 x 1152 M 512 17.1 -> 13.3, M 1000 28.4 -> 19.6);
+//   M 2048: 1152 x 1152 21 against 23, 2304 x 768 20.5 against 22.9, 3456 x 1152 28 against 34;
+//   M 4096: 3072 x 768 43 -> 34, 1152 x 1152 34 -> 25, 3072 x 1024 43 -> 42, 4608 x 1152 60 -> 53, but 3456 x 1152 45 against 46, 4096 x 1024 45 against 47;
+//   M 6144: 3456 x 1152 63 -> 57, 4608 x 1152 86 -> 69, 4096 x 1024 64 -> 62, 1024 x 4096 64 -> 60;
+//   M 8192: 3456 x 1152 83 -> 69, 4608 x 1152 112 -> 85, 4096 x 1024 84 -> 76, 1152 x 1152 61 -> 36, 768 x 768 49 -> 23;  M 16384: 3072 x 768 147 ->
+//   82, 4608 x 1152 320 -> 158 (1100 TFLOP/s).  The largest result measured is 6912 x 1152 (8 M elements); beyond it the library's products are kept.
 extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   if (M > INT32_MAX || !dmf::wgrad_shape_ok(M, N, K)) return 0;
   const int64_t result = (int64_t)N * K;
@@ -1323,9 +1332,10 @@ extern "C" int dmf_linear_wgrad_plan(int64_t M, int N, int K) {
   return M >= 6144 || result <= 3200000 || (result >= 5000000 && K % dmf::kWgK == 0);
 }
 
-// ... and with the column sums, where the library's product has a column sum beside it (two launches, 8 to 11 us): on every result of the models (us, library
-// and column sum -> here): M 1536: 2304 x 768 27.8 -> 23.5, 3072 x 1024 32.5 -> 29.8;  M 2048: 3072 x 768 36.5 -> 29.0, 3072 x 1024 36.9 -> 36.5, 1152 x 1152 32.2 ->
-// 24.4, 4608 x 1152 48.5 -> 39.3;  M 4096: 3456 x 1152 60.7 -> 49.9, 4096 x 1024 59.6 -> 53.6;  M 5120: 3456 x 1152 71.0 -> 57.0, 1024 x 4096 68.6 -> 63.5.
+// ... and with the column sums, where the library's product has a column sum beside it (two launches, 8 to 11 us): on every result of the models, 0.62 of the
+// library's time in the mean of 320 (us, library and column sum -> here): M 1: 768 x 768 9.3 -> 5.7;  M 256: 4608 x 768 19.8 -> 10.3, 6912 x 1152 24.1 -> 13.4;  M 512:
+// 768 x 768 15.6 -> 12.3;  M 1536: 2304 x 768 27.2 -> 23.3, 3072 x 1024 31.5 -> 29.0;  M 2048: 3072 x 768 36.0 -> 28.4, 3072 x 1024 36.4 -> 36.3, 1152 x 1152 31.3 ->
+// 23.4, 4608 x 1152 45.3 -> 38.4;  M 4096: 3456 x 1152 54.8 -> 47.6, 4096 x 1024 56.3 -> 51.6;  M 5120: 3456 x 1152 64.5 -> 53.7, 1024 x 4096 63.7 -> 57.8.
 extern "C" int dmf_linear_wgrad_sums_plan(int64_t M, int N, int K) { return M <= INT32_MAX && dmf::wgrad_shape_ok(M, N, K) && (int64_t)N * K <= 8000000; }
 
 extern "C" int dmf_linear_train_plan(int which, int64_t M, int N, int K, char* buf, int buflen) {

@@ -4,6 +4,7 @@ launched on those paths), and the autograd / forward-AD protocol of the Python
 operator behaves like the reference's (models/flash_attention_2_jvp.py:177-319)
 when the three kernel calls are replaced by stand-ins defined in this file."""
 import ctypes
+import math
 import os
 import re
 
@@ -408,17 +409,41 @@ def test_weight_gradients_with_column_sums_are_the_packages():
         assert not lib.dmf_linear_wgrad_sums_plan(*size)
 
 
-@pytest.mark.parametrize("N,K", [(1152, 64), (3072, 320), (2304, 768), (768, 3072), (3072, 1024)])
-def test_input_gradients_keep_the_library_where_it_is_faster(N, K):
-    """Narrow outputs, few rows, one to 4/3 rounds of 256 x 192 tiles behind a short depth, many rows of a width that 192 columns do not divide (256 CUs)."""
-    for M in range(64, 20000, 96):
-        tiles = -(-M // 256) * -(-K // 192)
-        if K < 192 or M < 768:
-            own = False
-        elif K >= 3 * N:
-            own = not 256 < tiles <= 341
-        elif K % 192 == 0:
-            own = M >= (2048 if K >= 512 else 3072)
-        else:
-            own = (3072 if K >= 512 else 6144) <= M < 10240
-        assert _lib.load().dmf_linear_dgrad_plan(M, N, K) == own, M
+MEASURED = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles", "linear_train_products.txt")
+
+
+def _measured(columns):
+    with open(MEASURED) as f:
+        rows = [[None if c == "-" else float(c) for c in line.split()] for line in f if line[:1].isdigit()]
+    return [(*map(int, r[:3]), *r[3:]) for r in rows if len(r) == columns]
+
+
+def _mean(ratios):
+    return math.exp(sum(map(math.log, ratios)) / len(ratios))
+
+
+def test_input_gradients_go_where_they_were_measured_to_be_faster():
+    """dmf_linear_dgrad_plan against the measured products of profiles/linear_train_products.txt (256 CUs, 1 % between two measurements in the mean, a tenth
+    at most): what goes to the kernel is not slower there than in the library, what goes to the library not slower than in the kernel as a whole."""
+    own, other = [], []
+    for M, N, K, t192, t128, library in _measured(6):
+        name = ctypes.create_string_buffer(128)
+        assert _lib.load().dmf_linear_train_plan(1, M, N, K, name, len(name)) == 0
+        taken = t192 if b"WalkTile<4, 3, 2, 3, 2>" in name.value else t128
+        (own if _lib.load().dmf_linear_dgrad_plan(M, N, K) else other).append(taken / library)
+        assert taken <= 1.2 * min(t192, t128), (M, N, K)
+    assert len(own) > 200 and len(other) > 100
+    assert max(own) <= 1.1 and _mean(own) <= 0.86 and _mean(other) >= 1.1
+
+
+def test_weight_gradients_go_where_they_were_measured_to_be_faster():
+    """The kernel that a weight gradient with column sums takes, against the other one and against the library and a column sum."""
+    kernels, library = [], []
+    for M, N, K, _, narrow, _, wide, _, other in _measured(9):
+        name = ctypes.create_string_buffer(128)
+        assert _lib.load().dmf_linear_train_plan(2, M, N, K, name, len(name)) == 0 and _lib.load().dmf_linear_wgrad_sums_plan(M, N, K)
+        taken = wide if b"wide" in name.value else narrow
+        kernels.append(taken / min(narrow, wide or narrow))
+        library.append(taken / other)
+    assert len(kernels) == 320 and max(kernels) <= 1.2 and _mean(kernels) <= 1.01
+    assert max(library) <= 1.1 and _mean(library) <= 0.65
