@@ -109,7 +109,7 @@ BUDGETS = [
     (r"23linear_walk_wide_kernelI", 512, 0), (r"22linear_walk_pre_kernelI", 512, 0),
     (r"21attn_fwd_small_kernelIDF16_Li(64|72|80|96)ELb0E", 256, 0), (r"21attn_fwd_small_kernelIDF16bLi(64|72|80|96)ELb0ELb0E", 256, 0),
     (r"21attn_fwd_small_kernelI", 512, 0),
-    (r"20attn_fwd_wide_kernelIDF16_Li(72|80)ELb0E", 128, 4), (r"20attn_fwd_wide_kernelI(DF16_Li(72|80)|fLi(32|64))ELb1E", 256, 0),
+    (r"20attn_fwd_wide_kernelIDF16_Li(72|80)ELb0E", 128, 1), (r"20attn_fwd_wide_kernelI(DF16_Li(72|80)|fLi(32|64))ELb1E", 256, 0),
     (r"18attn_bwd_dq_kernelI(f|DF16_)Li64E", 256, 0), (r"19attn_bwd_dkv_kernelIDF16_Li(64|72|80)E", 256, 0), (r"19attn_bwd_dkv_kernelIfLi64E", 256, 12),
     (r"18attn_bwd_dq_kernelI(f|DF16_)Li72E", 512, 0), (r"19attn_bwd_dkv_kernelIfLi72E", 512, 0),
 ]
