@@ -306,6 +306,13 @@ def _check_inputs(ref: torch.Tensor, *others: torch.Tensor) -> None:
             raise ValueError("all attention operands must share device and dtype")
 
 
+def _extent(what: str, device, *operands) -> None:
+    """Backward operands come from saved tensors, whose hooks may hand back anything: the kernels read each (tensor, elements) by address."""
+    for t, n in operands:
+        if t is not None and (t.numel() != n or t.device != device):
+            raise ValueError(f"{what}: an operand has {t.numel()} elements on {t.device}, where the call needs {n} on {device}")
+
+
 def fwd_jvp(q, k, v, tq, tk, tv, scale: float, need_dlse: bool = False, dtype_code=None):
     """Fused forward + JVP.  Returns (o, to, lse) -- or (o, to, lse, dlse) with
     ``need_dlse`` -- o/to contiguous (B, Lq, H, D), lse/dlse (B, H, Lq) fp32.
@@ -435,9 +442,12 @@ def bwd(dout, q, k, v, o, lse, scale: float, out=None, dtype_code=None):
     of one packed (B, L, 3, H, D) gradient buffer), which the kernels fill in place."""
     _check_inputs(q, k, v, o, dout)
     dout, q, k, v, o = map(_prep, (dout, q, k, v, o))
-    lse = _raw(_raw(lse).contiguous())
+    lse = _raw(_raw(lse).float().contiguous())
     B, Lq, H, D = q.shape
     Lkv = k.shape[1]
+    if dout.shape != q.shape or o.shape != q.shape or k.shape != (B, Lkv, H, D) or v.shape != k.shape:
+        raise ValueError("bwd: operands of different shapes")
+    _extent("bwd", q.device, (lse, B * H * Lq))
     if out is None:
         dq = _empty((B, Lq, H, D), q.dtype, q.device)
         dk = _empty((B, Lkv, H, D), q.dtype, q.device)
@@ -472,11 +482,14 @@ def bwd_qknorm(dout, q_hat, k_hat, v, o, lse, q, k, q_gain, k_gain, eps: float, 
     if q.dtype != torch.bfloat16:
         return None
     gains = [_raw(_in_memory(g).float().contiguous()) for g in (q_gain, k_gain)]
-    lse = _raw(_raw(lse).contiguous())
+    lse = _raw(_raw(lse).float().contiguous())
     dq, dk, dv = map(_raw, out)
     _check_inputs(q, dq, dk, dv)
     B, Lq, H, D = q.shape
     Lkv = k.shape[1]
+    if any(t.shape != q.shape for t in (dout, q_hat, o, dq)) or any(t.shape != (B, Lkv, H, D) for t in (k, k_hat, v, dk, dv)):
+        raise ValueError("bwd_qknorm: operands of different shapes")
+    _extent("bwd_qknorm", q.device, (lse, B * H * Lq), *((g, D) for g in gains))
     delta = _empty((B, H, Lq), torch.float32, q.device)
     ws = _empty((int(load().dmf_attn_bwd_qknorm_workspace_floats(B, H, Lq, Lkv, D)),), torch.float32, q.device)
     dgains = [_empty((D,), torch.float32, q.device) for _ in range(2)]
@@ -566,6 +579,7 @@ def ln_modulate_bwd(gy, x, scale, eps: float = 1e-6, gres=None):
     _same_dtype("ln_modulate_bwd x", x, gres)
     gy, x, gres = _dense(gy), _dense(x), _dense(gres)
     scale, ss = _mod(scale, B, C)
+    _extent("ln_modulate_bwd", x.device, (gy, B * L * C), (gres, B * L * C), (scale, B * C))
     gx = _empty((B, L, C), x.dtype, x.device)
     gshift = _empty((B, C), scale.dtype, x.device)
     gscale = _empty((B, C), scale.dtype, x.device)
@@ -603,6 +617,7 @@ def gate_residual_bwd(gy, gate, h):
     B, L, C = _blc(h)
     gy, h = _dense(gy), _dense(h)
     gate, gs = _mod(gate, B, C)
+    _extent("gate_residual_bwd", h.device, (gy, B * L * C), (gate, B * C))
     gh = _empty((B, L, C), h.dtype, h.device)
     ggate = _empty((B, C), gate.dtype, h.device)
     ws = _workspace(1, B, L, C, h.device)
@@ -631,6 +646,7 @@ def gelu_tanh_fwd(x, tx=None):
 def gelu_tanh_bwd(gy, x):
     _same_dtype("gelu_tanh_bwd", x, gy)
     gy, x = _dense(gy), _dense(x)
+    _extent("gelu_tanh_bwd", gy.device, (x, gy.numel()))
     gx = _empty(x.shape, x.dtype, x.device)
     with _on(x.device):
         rc = load().dmf_gelu_tanh_bwd(gy.data_ptr(), x.data_ptr(), gx.data_ptr(), x.numel(), _dtype_code(x), _stream(x))
@@ -662,6 +678,7 @@ def rmsnorm_bwd(gy, x, gain, eps: float = 1e-6, out=None):
     _check_inputs(x, gy)
     x, gy, gain = _prep(x), _dense(gy), _dense(gain)
     B, L, H, D = x.shape
+    _extent("rmsnorm_bwd", x.device, (gy, x.numel()), (gain, D))
     if out is None:
         gx = _empty((B, L, H, D), x.dtype, x.device)
     else:
@@ -774,6 +791,7 @@ def silu_fwd(x, tx=None, out_dtype=None):
 
 def silu_bwd(gy, x):
     gy, x = _dense(gy), _dense(x)
+    _extent("silu_bwd", gy.device, (x, gy.numel()))
     gx = _empty(x.shape, x.dtype, x.device)
     with _on(x.device):
         rc = load().dmf_silu_bwd(gy.data_ptr(), x.data_ptr(), gx.data_ptr(), x.numel(), _dtype_code(x), _dtype_code(gy), _stream(x))

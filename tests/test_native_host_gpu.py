@@ -586,3 +586,6 @@ def test_what_saved_tensor_hooks_hand_back():
         for unpack in (lambda t: t.cpu(), lambda t: t[:1] if t.dim() > 1 else t[:-8]):
             with pytest.raises(RuntimeError, match="hook handed back"):
                 grads(same, unpack)
+            with pytest.raises((RuntimeError, ValueError)):
+                _general(lambda: grads(same, unpack))
+        assert all(torch.equal(g, e) for g, e in zip(_general(lambda: grads(lambda t: t.cpu(), lambda t: t.to(DEV))), _general(lambda: grads(same, same))))
